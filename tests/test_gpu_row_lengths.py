@@ -1,0 +1,40 @@
+"""Row operations at the row lengths where their launches change: rows of a block's registers (multiples of the block's
+chunks, one more, one less, no multiple of four), rows shared by several blocks, and rows no block holds."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def close(a, b, rtol, atol):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    bad = np.abs(a - b) > atol + rtol * np.abs(b)
+    assert not bad.any(), f"{bad.sum()} of {bad.size} differ; max abs err {np.abs(a - b).max():.3e}"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from caten_amd import _lib, ops as o
+    _lib.init(0)
+    return o
+
+
+@pytest.mark.parametrize("rows,n", [(3, 3), (3, 4), (5, 5), (2, 255), (2, 257), (2, 1023), (7, 1025), (2, 2047), (2, 2049), (2, 4097),
+                                    (3, 8190), (2, 8193), (2, 16386), (2, 32769), (49, 32769), (2, 53248), (2, 53251), (2, 65536), (1, 65541)])
+def test_rows_of_any_length(ops, oracle, rows, n):
+    rng = np.random.default_rng(n)
+    x = rng.normal(0.3, 1, (rows, n)).astype(np.float32)
+    g, b = rng.normal(1, 0.02, n).astype(np.float32), rng.normal(0, 0.02, n).astype(np.float32)
+    close(ops.softmax(x), oracle.softmax(x), 1e-4, 1e-7)
+    close(ops.layernorm(x, g, b), oracle.layernorm(x, g, b), 1e-4, 3e-5)
+    close(ops.rmsnorm(x, g), oracle.rmsnorm(x, g), 1e-4, 1e-5)
+    close(ops.layernorm_softmax(x, g, b), oracle.softmax(oracle.layernorm(x, g, b)), 1e-4, 1e-7)
+
+
+@pytest.mark.parametrize("rows,n", [(3, 1), (3, 3), (5, 5), (4, 1023), (4, 1025), (2, 4099), (2, 8191), (16, 8192), (17, 16385), (3, 50257)])
+def test_argmax_of_any_length(ops, rows, n):
+    rng = np.random.default_rng(n)
+    x = rng.integers(0, max(2, n // 3), (rows, n)).astype(np.float32)  # many ties: the lowest index counts
+    x[0, n - 1] = n  # the last element, which a row that is no multiple of four reads through an overlapping piece
+    for _ in range(2):  # the counters behind a row's last part are back at zero
+        assert np.array_equal(np.atleast_1d(ops.argmax(x)).ravel(), x.argmax(-1))
