@@ -334,16 +334,15 @@ int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, in
   return 0;
 }
 
-// Rows of any length from 4 up to 4 NT VPL floats, at any alignment: one block per row, the row in its registers (read
-// once, written once).  Chunk c of four floats starts at min(4c, n - 4): the last one of a row that is no multiple of
-// four overlaps its neighbour, whose share it leaves out of the sums and stores a second time with the same values.
-// (The loads are 16 bytes at 4-byte alignment.)  What this replaces read the row three to four times, a float per lane:
-// softmax of one row of 50 257 floats 70 -> 6 us, RMSNorm of (5402, 7011) 111 -> 63 us (4.8 TB/s).
+// Softmax of rows of any length from 4 up to 4 NT VPL floats (LayerNorm -> softmax likewise), at any alignment: one block
+// per row, the row in its registers (read once, written once).  Chunk c of four floats starts at min(4c, n - 4): the last
+// one of a row that is no multiple of four overlaps its neighbour, whose share it leaves out of the sums and stores a second
+// time with the same values.  (The loads are 16 bytes at 4-byte alignment.)  What this replaces read the row three to five
+// times, a float per lane: (5402, 7011) 102 -> 51 us, 5.9 TB/s.
 typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
 template <int MODE, int NT, int VPL>
 __global__ __launch_bounds__(NT) void k_rowop_block(RowArgs a) {
   constexpr int NW = NT / 64;
-  constexpr bool NORM = MODE != ROW_SOFTMAX;
   __shared__ float red[4][NW];
   const int tid = threadIdx.x, n = a.n, nc = (n + 3) >> 2;
   const float *xr = a.x + (int64_t)blockIdx.x * n;
@@ -365,18 +364,14 @@ __global__ __launch_bounds__(NT) void k_rowop_block(RowArgs a) {
     for (int w = 1; w < NW; w++) s = mx ? fmaxf(s, red[slot][w]) : s + red[slot][w];
     return s;
   };
-  if (NORM) {
+  if (MODE == ROW_LN_SOFTMAX) {
     const float inv_n = 1.0f / (float)n;
-    float mean = 0.0f;
-    if (MODE != ROW_RMSNORM) {
-      float s = 0.0f;
+    float s = 0.0f, q = 0.0f;
 #pragma unroll
-      for (int j = 0; j < VPL; j++)
+    for (int j = 0; j < VPL; j++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) s += counts(j, e) ? v[j][e] : 0.0f;
-      mean = block(0, s, false) * inv_n;
-    }
-    float q = 0.0f;
+      for (int e = 0; e < 4; e++) s += counts(j, e) ? v[j][e] : 0.0f;
+    const float mean = block(0, s, false) * inv_n;
 #pragma unroll
     for (int j = 0; j < VPL; j++)
 #pragma unroll
@@ -398,30 +393,81 @@ __global__ __launch_bounds__(NT) void k_rowop_block(RowArgs a) {
       v[j][3] = v[j][3] * rstd * g.w + b.w;
     }
   }
-  if (MODE == ROW_SOFTMAX || MODE == ROW_LN_SOFTMAX) {
-    float m = -INFINITY;  // (a maximum may count an element twice)
-#pragma unroll
-    for (int j = 0; j < VPL; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) m = fmaxf(m, v[j][e]);
-    m = block(2, m, true);
-    float s = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPL; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[j][e] = ct_exp(v[j][e] - m);
-        s += counts(j, e) ? v[j][e] : 0.0f;
-      }
-    const float inv = 1.0f / block(3, s, false);
-#pragma unroll
-    for (int j = 0; j < VPL; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[j][e] *= inv;
-  }
+  float m = -INFINITY;  // (a maximum may count an element twice)
 #pragma unroll
   for (int j = 0; j < VPL; j++)
-    if (tid + NT * j < nc) *(f4_any *)(yr + min(4 * (tid + NT * j), n - 4)) = f4_any{v[j][0], v[j][1], v[j][2], v[j][3]};
+#pragma unroll
+    for (int e = 0; e < 4; e++) m = fmaxf(m, v[j][e]);
+  m = block(2, m, true);
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < VPL; j++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      v[j][e] = ct_exp(v[j][e] - m);
+      s += counts(j, e) ? v[j][e] : 0.0f;
+    }
+  const float inv = 1.0f / block(3, s, false);
+#pragma unroll
+  for (int j = 0; j < VPL; j++)
+    if (tid + NT * j < nc)
+      *(f4_any *)(yr + min(4 * (tid + NT * j), n - 4)) = f4_any{v[j][0] * inv, v[j][1] * inv, v[j][2] * inv, v[j][3] * inv};
+}
+
+// LayerNorm / RMSNorm of rows of up to 256 VPL floats: a block per row, thread t holds elements t, t + 256, ... and sums
+// them in that order -- the sums of the kernel below bit for bit (a session over Q8_0 cache rows turns a last bit into a
+// quantisation step), with all of a row's requests in flight at once and the row read once instead of three times:
+// RMSNorm of (5402, 7011) 85 -> 57 us, LayerNorm 125 -> 59, 5.2 TB/s.
+template <int MODE, int VPL>
+__global__ __launch_bounds__(256) void k_norm_block(RowArgs a) {
+  __shared__ float red[2][4];
+  const int tid = threadIdx.x, n = a.n;
+  const float *__restrict__ xr = a.x + (int64_t)blockIdx.x * n;
+  float *__restrict__ yr = a.y + (int64_t)blockIdx.x * n;
+  float v[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; j++) v[j] = xr[min(tid + 256 * j, n - 1)];
+  __builtin_amdgcn_sched_barrier(0);  // all of them before the first use; elements past the end are selected away, not branched over
+  auto block_sum = [&](int slot, float s) {
+    s = wave_sum(s);
+    if ((tid & 63) == 0) red[slot][tid >> 6] = s;
+    __syncthreads();
+    return red[slot][0] + red[slot][1] + red[slot][2] + red[slot][3];
+  };
+  float mean = 0.0f;
+  if (MODE != ROW_RMSNORM) {
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPL; j++) s = tid + 256 * j < n ? s + v[j] : s;
+    mean = block_sum(0, s) / (float)n;
+  }
+  float q = 0.0f;
+#pragma unroll
+  for (int j = 0; j < VPL; j++) {
+    const float d = v[j] - mean;
+    q = tid + 256 * j < n ? fmaf(d, d, q) : q;
+  }
+  const float rstd = 1.0f / sqrtf(block_sum(1, q) / (float)n + a.eps);
+  const float *gp = a.g ? a.g : xr, *bp = a.b ? a.b : xr;  // xr: unused stand-in, so that no request sits behind a branch
+  constexpr int P = VPL < 8 ? VPL : 8;
+#pragma unroll
+  for (int j0 = 0; j0 < VPL; j0 += P) {
+    float gm[P], bt[P];
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      const int i = min(tid + 256 * (j0 + j), n - 1);
+      gm[j] = gp[i];
+      bt[j] = bp[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      float t = (v[j0 + j] - mean) * rstd;
+      t = a.g ? t * gm[j] : t;
+      t = a.b ? t + bt[j] : t;
+      if (tid + 256 * (j0 + j) < n) yr[tid + 256 * (j0 + j)] = t;
+    }
+  }
 }
 
 // Softmax of rows too long for a block's registers, or so few that a block per row leaves the chip idle: gridDim.x
@@ -554,6 +600,18 @@ static int launch_rowop(RowArgs a) {
     if (e != hipSuccess) return fail((int)e, "row op: launch -> %s", hipGetErrorString(e));
     return rc;
   }
+  if constexpr (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM) {
+#define NORM_BLOCK(VPL) hipLaunchKernelGGL((k_norm_block<MODE, VPL>), grid, dim3(256), 0, st, a)
+    if (a.n <= 1024) NORM_BLOCK(4);
+    else if (a.n <= 2048) NORM_BLOCK(8);
+    else if (a.n <= 4096) NORM_BLOCK(16);
+    else if (a.n <= 8192) NORM_BLOCK(32);
+    else if (a.n <= 16384) NORM_BLOCK(64);
+    else hipLaunchKernelGGL((k_rowop_generic<MODE>), grid, dim3(256), 0, st, a);
+#undef NORM_BLOCK
+    CTHIP_LAUNCH_CHECK();
+    return 0;
+  } else {
 #define ROW_BLOCK(NT, VPL) hipLaunchKernelGGL((k_rowop_block<MODE, NT, VPL>), grid, dim3(NT), 0, st, a)
   if (a.n < 4 || nc > 16384) hipLaunchKernelGGL((k_rowop_generic<MODE>), grid, dim3(256), 0, st, a);
   else if (nc <= 64) ROW_BLOCK(64, 1);
@@ -566,9 +624,11 @@ static int launch_rowop(RowArgs a) {
   else if (nc <= 13312) ROW_BLOCK(1024, 13);
   else ROW_BLOCK(1024, 16);
 #undef ROW_BLOCK
-  CTHIP_LAUNCH_CHECK();
-  return 0;
+    CTHIP_LAUNCH_CHECK();
+    return 0;
+  }
 }
+
 
 // ------------------------------------------------------------------ elementwise
 // A block owns UNARY_PER_BLOCK consecutive elements; a thread takes UNARY_VEC-wide pieces 256 pieces apart, all of
@@ -1038,7 +1098,7 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
     } else {
       // device-scope stores: written through to memory, no cache to flush (a fence here would write back and
       // invalidate the whole L2 of the XCD under every other workgroup's key reads: measured 2x slower than no split)
-      float *mine = sp_part + ((int64_t)h * gridDim.z + blockIdx.z) * (DH + 2);
+      float *mine = sp_part + ((int64_t)(i * H + h) * gridDim.z + blockIdx.z) * (DH + 2);
       __hip_atomic_store(mine + tid, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (tid == 0) {
         __hip_atomic_store(mine + DH, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1052,13 +1112,13 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
     // range's triple with device-scope loads (which do not look into a cache that could hold an older launch's).
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) ticket = __hip_atomic_fetch_add(sp_count + h, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) ticket = __hip_atomic_fetch_add(sp_count + i * H + h, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (ticket != nranges - 1) return;  // (uniform)
     if (tid < DH) {
-      out[((int64_t)i * H + h) * DH + tid] = attn_split_merge(sp_part + (int64_t)h * gridDim.z * (DH + 2), nranges, DH, tid);
+      out[((int64_t)i * H + h) * DH + tid] = attn_split_merge(sp_part + (int64_t)(i * H + h) * gridDim.z * (DH + 2), nranges, DH, tid);
     }
-    if (tid == 0) __hip_atomic_store(sp_count + h, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the next launch counts again
+    if (tid == 0) __hip_atomic_store(sp_count + i * H + h, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the next launch counts again
   }
 }
 
@@ -1587,8 +1647,8 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
   float *nop = nullptr;
   int *noc = nullptr;
   if (split && split->ranges > kAttnSplitMaxRanges) return fail(CTHIP_E_BAD_ARG, "attention: %d key ranges per head (at most %d)", split->ranges, kAttnSplitMaxRanges);
-  if (S == 1 && split && split->ranges > 1) {  // one row over a context that may be long: the keys shared by several workgroups
-    dim3 grid(H, 1, split->ranges), block(1024);
+  if (split && split->ranges > 1) {  // a row (or a few) over a context that may be long: the keys shared by several workgroups
+    dim3 grid(H, S, split->ranges), block(1024);
     switch (Dh) {
       case 32: hipLaunchKernelGGL((k_attn_cached<32, false, true>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
       case 64: hipLaunchKernelGGL((k_attn_cached<64, false, true>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
