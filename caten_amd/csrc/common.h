@@ -202,8 +202,8 @@ int gemv_rows_per_wave(int type, int64_t cols);
 bool gemv_pair_swiglu_ok(int type, int64_t rows, int64_t cols);
 // out[i] = silu(in[2i]) * in[2i+1], i < n (gate / up columns interleaved)
 int launch_swiglu_pairs(float *out, const float *in, int64_t n);
-// One query row over a long context: `ranges` workgroups per head share the keys (k_attn_cached, SPLIT).  part holds
-// H x ranges x (head_dim + 2) floats, count H zeroed ints (each launch leaves them zeroed again).
+// A query row over a long context: `ranges` workgroups per head share the keys (k_attn_cached, SPLIT).  For S rows (fewer
+// than 16) part holds S x H x ranges x (head_dim + 2) floats, count S x H zeroed ints (each launch leaves them zeroed again).
 struct AttnSplit {
   int ranges;
   float *part;
@@ -251,6 +251,10 @@ constexpr int kActSwigluPairs = 64;
 // route: non-null = y is ignored, the columns go where the route says; K is not split then.
 int launch_linear_gemm(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual,
                        int act, int precision, GemmDeferred *defer = nullptr, const GemmRoute *route = nullptr);
+// the same for 2 .. 32 rows, prologue included (linear_rows.hip); call only where linear_rows_pays
+bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b);
+int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
+                       int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route = nullptr);
 bool reduce_norm_supported(int n, int nparts);
 // C (m, n) = sum_z ws[z] + bias + residual for partial tiles handed over through GemmDeferred
 int launch_splitk_reduce(float *C, float *ws, int ksplit, int m, int n, const float *bias, const float *residual);

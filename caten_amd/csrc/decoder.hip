@@ -17,10 +17,10 @@
 // kernel, GQA attention and a fused gate|up matrix whose SwiGLU is the prologue of
 // the down projection.
 //
-// The reference pushes a whole prompt through one forward (s > 1).  Prompts of 8 or more rows
-// run as one batch (MFMA GEMMs over the rows, see prefill()); shorter ones are fed row by row
-// through the decode step (causal attention makes that the same function).  Either way only the
-// last row runs lm_head and argmax.
+// The reference pushes a whole prompt through one forward (s > 1).  Prompts run as one batch (see
+// prefill(): MFMA GEMMs over 8 rows and more, fp32-grade Linears over fewer); two rows over
+// three-launch layers are fed row by row through the decode step (causal attention makes that the
+// same function).  Either way only the last row runs lm_head and argmax.
 #include <stdlib.h>
 #include <string.h>
 
@@ -51,6 +51,7 @@ static size_t raw_nbytes(int type, int64_t n) {
 }
 
 static const int kStepsPerGraph = 8;
+static const int kAttnCachedRows = 15;  // most query rows of a launch that shares keys between workgroups
 
 struct Layer {
   // GPT-2
@@ -376,7 +377,7 @@ static int finalize(Decoder *d) {
     if (state().attn_split > 1) ranges = state().attn_split;  // (a given number of ranges)
     if (ranges > 1 && state().attn_split) {
       TRY(dev_alloc(d, (void **)&d->att_split.part, sizeof(float) * (size_t)c.n_heads * ranges * (Dh + 2)));
-      TRY(dev_alloc(d, (void **)&d->att_split.count, sizeof(int) * (size_t)c.n_heads));  // zero-filled
+      TRY(dev_alloc(d, (void **)&d->att_split.count, sizeof(int) * (size_t)c.n_heads * kAttnCachedRows));  // zero-filled
       d->att_split.ranges = ranges;
     }
   }
@@ -864,10 +865,43 @@ static int queue_head(Decoder *d) {
   return launch_gemv(d->lm_head, o, 1);
 }
 
-// A prompt of s >= kPrefillMin rows as one batch (the reference's forward with s > 1): every Linear is
-// an MFMA GEMM over the s rows (weights dequantised while staged), attention runs all s query rows
-// against the cache under the causal mask; only the last row goes through lm_head.
-static const int kPrefillMin = 8;
+// Rows from which a prompt is one batch.  A batch has seven launches a layer or so whatever its rows are, a row through the
+// decode step has three or five: a 7B shape's three rows took 5.0 ms one by one and 2.9 ms as a batch.
+// (Over Q8_0 cache rows a row of a batch attends to its batch's rows before they are quantised, a row through the decode
+// step after; fewer than eight keep the latter.)
+static int prefill_min(const Decoder *d) { return d->kvq ? 8 : d->fused || d->fused_gqa || d->flow ? 3 : 2; }
+
+// One Linear of a prompt batch.  Eight rows and more: launch_linear_gemm.  Fewer keep what the decode step gives them,
+// fp32-grade products: all rows in one pass over the weights where that is the faster launch, else the single-row kernels.
+static int prompt_linear(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual, int act, int precision,
+                         GemmDeferred *defer = nullptr, const GemmRoute *route = nullptr) {
+  if (linear_rows_pays(w, x, w->cols, m, precision, nullptr, nullptr))
+    return launch_linear_rows(y, w, x, w->cols, m, bias, residual, act, CTHIP_PRO_NONE, nullptr, nullptr, 0.0f, precision, route);
+  if (m >= 8) return launch_linear_gemm(y, w, x, m, bias, residual, act, precision, defer, route);
+  GemvArgs a = {};
+  a.x = x;
+  a.x_stride = w->cols;
+  a.bias = bias;
+  a.residual = residual;
+  a.act = act == kActSwigluPairs ? CTHIP_ACT_NONE : act;
+  a.pair_swiglu = act == kActSwigluPairs;
+  a.y = y;
+  a.y_stride = act == kActSwigluPairs ? w->rows / 2 : w->rows;
+  if (route) {  // query rows, then the cache rows of keys and values
+    a.y = route->dst[0];
+    a.y_stride = route->ld[0];
+    a.y1 = route->dst[1];
+    a.y2 = route->dst[2];
+    a.split1 = route->c0[1];
+    a.split2 = route->c0[2];
+    a.pos_stride = route->ld[1];
+  }
+  return launch_gemv(w, a, m);
+}
+
+// A prompt of several rows as one batch (the reference's forward with s > 1): every Linear is one launch over the s
+// rows (weights dequantised while staged), attention runs all s query rows against the cache under the causal mask; only
+// the last row goes through lm_head.
 static int prefill(Decoder *d, const int *ids, int s, int n) {
   const cthip_decoder_config &c = d->cfg;
   const bool gpt2 = c.arch == CTHIP_ARCH_GPT2;
@@ -877,6 +911,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   int rc = 0;
   float *X = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *Hb = nullptr, *G = nullptr, *KF = nullptr, *VF = nullptr;
   int *ids_dev = nullptr;
+  AttnSplit split = {1, nullptr, nullptr};
   std::vector<void *> tmp;
   auto alloc = [&](void **p, size_t bytes) {
     int r = alloc_scratch(p, bytes);  // every temporary below is fully written before it is read
@@ -898,6 +933,11 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     TRY(alloc((void **)&KF, sizeof(float) * (size_t)(n + s) * KD));
     TRY(alloc((void **)&VF, sizeof(float) * (size_t)(n + s) * KD));
   }
+  if (s <= kAttnCachedRows && n + s >= 512 && d->att_split.ranges > 1) {  // few rows over a long context: keys shared as in a decode step
+    split.ranges = d->att_split.ranges / s < 2 ? 2 : d->att_split.ranges / s;
+    split.count = d->att_split.count;
+    TRY(alloc((void **)&split.part, sizeof(float) * (size_t)s * c.n_heads * split.ranges * (Dh + 2)));
+  }
   TRY(alloc((void **)&ids_dev, sizeof(int) * (size_t)s));
   TRY(cthip_h2d(ids_dev, ids, sizeof(int) * (size_t)s));
   {
@@ -916,7 +956,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     auto linear_residual_norm = [&](const WMat *w, const float *in, const float *bias, const float *g, const float *b) {
       GemmDeferred df;
       const bool fuse = g != nullptr && reduce_norm_supported(D, 1);
-      int r = launch_linear_gemm(X, w, in, s, bias, X, CTHIP_ACT_NONE, prec, fuse ? &df : nullptr);
+      int r = prompt_linear(X, w, in, s, bias, X, CTHIP_ACT_NONE, prec, fuse ? &df : nullptr);
       if (r) return r;
       if (df.ws) {
         if (reduce_norm_supported(D, df.ksplit)) {
@@ -938,38 +978,38 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         // batch's rows [n, n + s) join them (rotated where the model rotates) and are quantised into the cache
         TRY(launch_kvq_dequant(KF, L.kq, L.kdq, n, KD));
         TRY(launch_kvq_dequant(VF, L.vq, L.vdq, n, KD));
-        TRY(launch_linear_gemm(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
+        TRY(prompt_linear(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
         TRY(launch_qkv_split(Q, KF, VF, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
         TRY(launch_kvq_append(L.kq, L.kdq, KF + (int64_t)n * KD, KD, s, n, nullptr, KD));
         TRY(launch_kvq_append(L.vq, L.vdq, VF + (int64_t)n * KD, KD, s, n, nullptr, KD));
-        TRY(launch_attn(ATT, Q, KF, VF, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh));
+        TRY(launch_attn(ATT, Q, KF, VF, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, &split));
       } else if (d->kvp) {
         // attention of a prompt batch runs on dense rows: the cached rows [0, n) are gathered out of their pages, the
         // batch's rows [n, n + s) join them (rotated where the model rotates) and are copied into their pages
         TRY(launch_kvp_gather(KF, L.k_pages, n, KD));
         TRY(launch_kvp_gather(VF, L.v_pages, n, KD));
-        TRY(launch_linear_gemm(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
+        TRY(prompt_linear(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
         TRY(launch_qkv_split(Q, KF, VF, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
         TRY(launch_kvp_append(L.k_pages, L.v_pages, KF + (int64_t)n * KD, VF + (int64_t)n * KD, KD, s, n, nullptr, KD));
-        TRY(launch_attn(ATT, Q, KF, VF, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh));
+        TRY(launch_attn(ATT, Q, KF, VF, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, &split));
       } else {
       if (gpt2 && D % 128 == 0 && KD % 128 == 0) {
         // no rotation: the thirds of the fused projection go straight to the query rows and the cache rows
         const GemmRoute rt = {{Q, L.k_cache + (int64_t)n * KD, L.v_cache + (int64_t)n * KD}, {0, D, D + KD}, {D, KD, KD}};
-        TRY(launch_linear_gemm(nullptr, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec, nullptr, &rt));
+        TRY(prompt_linear(nullptr, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec, nullptr, &rt));
       } else {
-        TRY(launch_linear_gemm(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
+        TRY(prompt_linear(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
         TRY(launch_qkv_split(Q, L.k_cache, L.v_cache, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
       }
-      TRY(launch_attn(ATT, Q, L.k_cache, L.v_cache, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh));
+      TRY(launch_attn(ATT, Q, L.k_cache, L.v_cache, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, &split));
       }
       TRY(linear_residual_norm(L.proj, ATT, L.proj_b, L.ln2_g, L.ln2_b));
       const float *hin = Hb;
       if (!gpt2 && L.fc_pairs && (2 * F) % 4 == 0) {  // SwiGLU in the epilogue of the gate|up launch
-        TRY(launch_linear_gemm(G, L.fc, XN, s, L.fc_b, nullptr, kActSwigluPairs, prec));
+        TRY(prompt_linear(G, L.fc, XN, s, L.fc_b, nullptr, kActSwigluPairs, prec));
         hin = G;
       } else {
-        TRY(launch_linear_gemm(Hb, L.fc, XN, s, L.fc_b, nullptr, gpt2 ? CTHIP_ACT_GELU : CTHIP_ACT_NONE, prec));
+        TRY(prompt_linear(Hb, L.fc, XN, s, L.fc_b, nullptr, gpt2 ? CTHIP_ACT_GELU : CTHIP_ACT_NONE, prec));
         if (!gpt2) {
           if (L.fc_pairs) TRY(launch_swiglu_pairs(G, Hb, (int64_t)s * F));
           else TRY(launch_prologue(G, Hb, F, CTHIP_PRO_SWIGLU, nullptr, nullptr, 0.0f, 2 * (int64_t)F, s));
@@ -1136,7 +1176,7 @@ int cthip_decoder_forward(void *dec, const float *tokens, int s, int n, int64_t 
     const float tf = tokens[i];
     ids[i] = (tf >= 0.0f && tf < (float)c.vocab && (float)(int)tf == tf) ? (int)tf : -1;
   }
-  if (s >= kPrefillMin && state().prefill_gemm) {
+  if (s >= prefill_min(d) && state().prefill_gemm) {
     if ((rc = prefill(d, ids.data(), s, n))) return rc;
   } else {
     for (int i = 0; i < s; i++) {

@@ -20,7 +20,6 @@
 // wavefront visits, so the steady state touches nothing but weights.  Partial
 // sums are combined with DPP/shuffle steps inside the group and the group's
 // first lane applies the epilogue.
-#include <stdlib.h>
 #include <string.h>
 
 #include <vector>
@@ -353,6 +352,8 @@ __global__ __launch_bounds__(256) void k_swiglu_rows(float *__restrict__ out, co
 int launch_prologue(float *out, const float *x, int cols, int pro, const float *g, const float *b, float eps,
                     int64_t x_stride, int m) {
   if (m == 0) return 0;
+  if (m >= 8 && x_stride == cols && pro == CTHIP_PRO_LAYERNORM) return cthip_layernorm(out, x, g, b, eps, m, cols);
+  if (m >= 8 && x_stride == cols && pro == CTHIP_PRO_RMSNORM && !b) return cthip_rmsnorm(out, x, g, eps, m, cols);
   if (pro == CTHIP_PRO_SWIGLU)
     hipLaunchKernelGGL(k_swiglu_rows, dim3((unsigned)((cols + 1023) / 1024), (unsigned)m), dim3(256), 0, state().stream, out, x, cols, x_stride);
   else
@@ -709,6 +710,9 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
   if (m == 0) return 0;
   if (m > 65535) return fail(CTHIP_E_BAD_ARG, "cthip_linear: m = %d exceeds 65535", m);
   const WMat *w = (const WMat *)wmat;
+  const int64_t x_stride = prologue == CTHIP_PRO_SWIGLU ? 2 * w->cols : w->cols;
+  if (linear_rows_pays(w, x, x_stride, m, state().gemm_precision, norm_g, norm_b))
+    return launch_linear_rows(y, w, x, x_stride, m, bias, residual, act, prologue, norm_g, norm_b, eps, state().gemm_precision);
   if (m >= 8) {
     // several input rows: the MFMA tile path reads the weights once instead of once per row
     const float *xin = x;

@@ -1,0 +1,612 @@
+// Linear over a few rows (2 .. 32: a handful of sequences decoded together, a short prompt, the next turn of a
+// conversation) on packed weights.  What such a launch cannot do without is ONE read of the weights; a
+// single-row kernel per row reads them once for each, and a GEMM tile of 64 rows spends its time converting operands it
+// uses once.
+//
+// A wavefront owns NS x 16 weight rows and multiplies them with all input rows on the matrix cores
+// (v_mfma_f32_16x16x32).  Its weights come straight from memory into a ring of its own in LDS, whole cache lines of a row
+// at a time, PD units (4 - 8 KB) in flight per wavefront and no barrier in the loop.  The input rows, split into 16-bit
+// terms by a small launch in front (k_rows_planes, which also applies the norm or SwiGLU), wait in LDS for the workgroup's
+// share of k.  (Every workgroup splitting its own share of the rows saved that launch and cost 5 us per workgroup.)
+//
+// Terms are fp16 where the weights are: a quantised weight is an integer times its block's scale and an fp16 weight is what
+// it is, so the weight operand is exact and costs little more than one vector instruction a pair (Q8_0), or none (fp16).  The
+// inputs are scaled by a power of two per row (their largest below 2^15; undone at the end), so that two terms
+// hold 22 bits of every value that matters and three hold all 24.  A block's scale is applied to its partial sum.  fp32
+// weights are split like the inputs, into bf16 terms, which have their range.
+// Terms per input: three for fewer than 8 rows (what the single-row kernels give), else what "gemm_precision" says.
+//
+// K is shared among as many workgroups as fill the chip; a share leaves its partial sums in memory and draws a ticket, the
+// last one of a column group adds them in share order and stores the result (bias, activation, residual, routes).
+#include <type_traits>
+
+#include "common.h"
+#include "planes.h"
+
+namespace cthip {
+
+struct RowsGemmArgs {
+  const unsigned char *A;    // planes of the input rows: [M][nkb][NPA][32], nkb = whole units (zeros past K)
+  const float *rscale;       // per input row: what undoes its scaling (null for bf16 terms)
+  int nkb;
+  const unsigned char *W;    // N rows of packed weights, wpitch = wbytes apart
+  const unsigned short *wd;  // scales, dpitch apart
+  int wbytes, dpitch;
+  int kblocks, kper;         // blocks of 32 k per weight row, per workgroup (whole units)
+  float *parts;              // [column groups][shares][M][columns of a group]; null: one share
+  PlaneGemmArgs e;           // M, N and what happens to the result
+};
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+// two bytes of v as fp16 integers less `bias`: 0x64 in front of a byte is 1024 + byte
+__device__ __forceinline__ unsigned half2_of_bytes(unsigned v, unsigned sel, float bias) {
+  const v2h x = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, v, sel));
+  const _Float16 b = (_Float16)(-1024.0f - bias);
+  return __builtin_bit_cast(unsigned, x + v2h{b, b});
+}
+template <bool SIGNED>  // 8 int8 -> fp16 (SIGNED), or 8 nibbles (a byte each) - 8
+__device__ __forceinline__ v8h h_of_bytes(unsigned a, unsigned b) {
+  constexpr float bias = SIGNED ? 128.0f : 8.0f;
+  if (SIGNED) a ^= 0x80808080u, b ^= 0x80808080u;
+  return __builtin_bit_cast(v8h, make_uint4(half2_of_bytes(a, 0x04010400u, bias), half2_of_bytes(a, 0x04030402u, bias),
+                                            half2_of_bytes(b, 0x04010400u, bias), half2_of_bytes(b, 0x04030402u, bias)));
+}
+// 8 floats -> NP fp16 terms (of values below 2^15), each of what the terms before it miss
+template <int NP>
+__device__ __forceinline__ void split8_half(const float *v, uint4 *pl) {
+  float r[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) r[e] = v[e];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    v8h h;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      h[e] = (_Float16)r[e];
+      r[e] -= (float)h[e];
+    }
+    pl[p] = __builtin_bit_cast(uint4, h);
+  }
+}
+typedef float v4f __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4f mma_rows(v8h a, v8h b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ v4f mma_rows(v8bf a, v8bf b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+enum { RW_Q8 = 1, RW_Q4 = 2, RW_F16 = 3, RW_F32 = 4 };
+
+constexpr int kRowsMax = 32, kRowsGroups = 4096;  // input rows, column groups
+__device__ int g_rows_tickets[kRowsGroups];  // zero between launches
+
+// Bytes of a weight row in a unit, and blocks of 32 k: whole cache lines.  (Requests that cover 32 bytes of a row each, as
+// operand registers would ask for them, are bound by the tag lookups of the compute unit's cache: 2.4 TB/s of Q8_0 and
+// 1.5 TB/s of Q4_0 weights, most of it for the scales.)
+template <int SRC>
+struct RowsUnit {
+  static constexpr int BLOCKS = SRC == RW_Q8 ? 4 : SRC == RW_Q4 ? 8 : 2;
+  static constexpr int BYTES = SRC == RW_F32 ? 256 : 128;
+};
+
+// A wavefront: NS x 16 weight rows against MB x 16 input rows, v_mfma_f32_16x16x32 (lane l: row l % 16 of its operand, k =
+// 8 (l / 16) .. + 7 of the block; result row 4 (l / 16) + r, column l % 16).  WIDE_D: a row's scales start at a multiple of four bytes, two of them are fetched as one dword
+template <int SRC, int NPA, int MB, int NS, int NW, int PD, bool WIDE_D>
+__global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
+  constexpr bool QUANT = SRC == RW_Q8 || SRC == RW_Q4;
+  constexpr int NPB = SRC == RW_F32 ? NPA : 1;
+  constexpr int UB = RowsUnit<SRC>::BLOCKS, CPW = RowsUnit<SRC>::BYTES / 16;  // blocks, 16-byte chunks of a row per unit
+  constexpr int NR = 16 * NS;                                                     // weight rows of a wavefront
+  constexpr int IW = NR * CPW / 64, ID = !QUANT ? 0 : NR * UB / (WIDE_D ? 2 : 1) / 64;  // load instructions per unit: weights, scales
+  constexpr int WBYTES = NR * CPW * 16, SLOT = WBYTES + ID * 256;
+  constexpr int NT = NR * NW, T = 64 * NW;  // columns of a workgroup, threads
+  constexpr bool HALF = SRC != RW_F32;
+  typedef typename std::conditional<HALF, v8h, v8bf>::type op_t;  // one matrix operand
+  extern __shared__ __align__(16) unsigned char smem[];
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;
+  const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = (blockIdx.x * NW + wave) * NR;
+  const int M = a.e.M, N = a.e.N;
+  const int kb0 = blockIdx.y * a.kper, units = (min(a.kblocks - kb0, a.kper) + UB - 1) / UB, kbs = units * UB;  // blocks of this share
+
+  // ---- this wavefront's ring: unit u in slot u % PD, row r's chunk c at r * CPW + (c ^ (r & 7)) ----
+  const unsigned ring = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * (PD * SLOT));
+  const unsigned char *wbase = uniform(a.W + (int64_t)min(n0, N - 1) * a.wbytes);
+  const unsigned char *dbase = QUANT ? uniform((const unsigned char *)(a.wd + (int64_t)min(n0, N - 1) * a.dpitch)) : nullptr;
+  const int last = N - 1 - min(n0, N - 1);  // rows past the end repeat the last one
+  int wrow[IW], wch[IW];
+#pragma unroll
+  for (int j = 0; j < IW; j++) {
+    const int s = j * 64 + lane, r = s / CPW;
+    wrow[j] = min(r, last) * a.wbytes;
+    wch[j] = ((s % CPW) ^ (r & 7)) * 16;
+  }
+  auto request = [&](int u) __attribute__((always_inline)) {
+    const unsigned slot = ring + (unsigned)(u % PD) * SLOT;
+    u = min(u, units - 1);  // past the end: the last unit again (never read), so that the counts stay the same
+    const int at = (kb0 / UB + u) * (CPW * 16);
+    // chunks past the end of a row repeat its last one (and meet zeros of the input)
+#pragma unroll
+    for (int j = 0; j < IW; j++) dma16(wbase, (unsigned)(wrow[j] + min(at + wch[j], a.wbytes - 16)), slot + j * 1024);
+#pragma unroll
+    for (int j = 0; j < ID; j++) {  // scale (pair) i of row r at dword i * NR + r
+      const int s = j * 64 + lane, r = min(s % NR, last) * a.dpitch, kb = kb0 + u * UB;
+      if (WIDE_D) dma4(dbase, 2u * (unsigned)(r + min(kb + 2 * (s / NR), a.kblocks - 2)), slot + WBYTES + j * 256);
+      else dma2(dbase, 2u * (unsigned)(r + min(kb + s / NR, a.kblocks - 1)), slot + WBYTES + j * 256);
+    }
+  };
+  // ---- the share of the input rows -> LDS behind the rings: row r's chunk c (16 bytes) at r * cpr + (c ^ (r & 7)) ----
+  __shared__ int s_ticket;
+  const unsigned char *As = smem + NW * PD * SLOT;
+  const int cpr = kbs * 4 * NPA;
+  for (int r = wave; r < M; r += NW) {
+    const unsigned char *src = uniform(a.A + ((int64_t)r * a.nkb + kb0) * (64 * NPA));
+    for (int c0 = 0; c0 < cpr; c0 += 64)
+      if (c0 + lane < cpr)
+        dma16(src, (unsigned)((c0 + lane) ^ (r & 7)) * 16u, __builtin_amdgcn_readfirstlane(lds0 + NW * PD * SLOT + (unsigned)(r * cpr + c0) * 16u));
+  }
+#pragma unroll
+  for (int p = 0; p < PD; p++) request(p);
+  wait_barrier<PD *(IW + ID)>();  // the rows are there, the weights on their way
+
+  v4f acc[MB][NS];
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NS; j++) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  // Chunk of an input row's share: 4 (NPA kb + q) + grp for block kb, term q.  Its place differs from it in the low three
+  // bits only, which take two values a lane (blocks come in pairs: 8 NPA chunks).
+  const unsigned char *arow[MB][2];
+#pragma unroll
+  for (int i = 0; i < MB; i++) {
+    const int r = min(16 * i + col, M - 1);
+#pragma unroll
+    for (int t = 0; t < 2; t++) arow[i][t] = As + (r * cpr + ((4 * t + grp) ^ (r & 7))) * 16;
+  }
+  const unsigned char *wown = smem + wave * (PD * SLOT);
+  auto pair = [&](const unsigned char *slot, int bp, int kb) __attribute__((always_inline)) {  // blocks 2 bp, 2 bp + 1 of the unit = kb, kb + 1 of the share
+    // All operand reads of the pair first, then (behind a scheduling fence) the conversions, which hide them: left alone
+    // the compiler reads each operand right before its matrix instruction and waits out an LDS round trip every time.
+    constexpr int NV = SRC == RW_F32 ? 2 : 1;
+    uint4 w[NS][2][NV];
+    unsigned dv[NS][2];
+#pragma unroll
+    for (int j = 0; j < NS; j++) {
+      const int r = 16 * j + col;
+      auto at = [&](int ch) { return slot + (r * CPW + (ch ^ (r & 7))) * 16; };
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        if constexpr (SRC == RW_Q8) {
+          const uint2 t = *(const uint2 *)(at(2 * (2 * bp + b) + (grp >> 1)) + 8 * (grp & 1));
+          w[j][b][0].x = t.x, w[j][b][0].y = t.y;
+        } else if constexpr (SRC == RW_Q4) {
+          const uint2 t = *(const uint2 *)(at(2 * bp + b) + 8 * (grp & 1));
+          w[j][b][0].x = t.x, w[j][b][0].y = t.y;
+        } else if constexpr (SRC == RW_F16) {
+          w[j][b][0] = *(const uint4 *)at(4 * b + grp);
+        } else {
+          w[j][b][0] = *(const uint4 *)at(8 * b + 2 * grp);
+          w[j][b][NV - 1] = *(const uint4 *)at(8 * b + 2 * grp + 1);
+        }
+      }
+      if constexpr (QUANT) {
+        const unsigned *D = (const unsigned *)(slot + WBYTES);
+        if (WIDE_D) dv[j][0] = D[bp * NR + r];
+        else dv[j][0] = D[2 * bp * NR + r], dv[j][1] = D[(2 * bp + 1) * NR + r];
+      }
+    }
+    op_t af[MB][2][NPA];
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int q = 0; q < NPA; q++) {
+          const int c4 = NPA * b + q;  // in units of four chunks
+          af[i][b][q] = __builtin_bit_cast(op_t, *(const uint4 *)(arow[i][c4 & 1] + kb * (NPA * 64) + (c4 >> 1) * 128));
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    op_t bf[NS][2][NPB];
+#pragma unroll
+    for (int j = 0; j < NS; j++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        const uint4 v = w[j][b][0];
+        if constexpr (SRC == RW_Q8) {
+          bf[j][b][0] = h_of_bytes<true>(v.x, v.y);
+        } else if constexpr (SRC == RW_Q4) {  // k 0..15 of a block are the low nibbles of its bytes, 16..31 the high ones
+          bf[j][b][0] = h_of_bytes<false>((v.x >> (4 * (grp >> 1))) & 0x0f0f0f0fu, (v.y >> (4 * (grp >> 1))) & 0x0f0f0f0fu);
+        } else if constexpr (SRC == RW_F16) {
+          bf[j][b][0] = __builtin_bit_cast(v8h, v);
+        } else {
+          const uint4 u = w[j][b][NV - 1];
+          const float x[8] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w),
+                              __uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)};
+          uint4 pl[NPB];
+          split8_planes<NPB>(x, pl);
+#pragma unroll
+          for (int q = 0; q < NPB; q++) bf[j][b][q] = __builtin_bit_cast(op_t, pl[q]);
+        }
+      }
+    // a block's (quantised) or the pair's sum by itself: it is scaled before it is added, and one chain of matrix
+    // instructions over thousands of k would round five times as much
+    if constexpr (QUANT) {
+      float dd[NS][2];
+#pragma unroll
+      for (int j = 0; j < NS; j++) {
+        dd[j][0] = half_bits_to_float((unsigned short)(dv[j][0] & 0xffff));
+        dd[j][1] = half_bits_to_float((unsigned short)(WIDE_D ? dv[j][0] >> 16 : dv[j][1]));
+        asm("" : "+v"(dd[j][0]), "+v"(dd[j][1]));  // as floats: a multiply-add that converts its fp16 operand runs at half rate
+      }
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        v4f tmp[NS][2];
+#pragma unroll
+        for (int q = NPA - 1; q >= 0; q--)
+#pragma unroll
+          for (int j = 0; j < NS; j++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) tmp[j][b] = mma_rows(af[i][b][q], bf[j][b][0], q == NPA - 1 ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : tmp[j][b]);
+#pragma unroll
+        for (int j = 0; j < NS; j++)
+#pragma unroll
+          for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(dd[j][b], tmp[j][b][r], acc[i][j][r]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        v4f tmp[NS];
+#pragma unroll
+        for (int j = 0; j < NS; j++) tmp[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+          for (int t = NPA - 1; t >= 0; t--)  // pairs of terms above 2^-8(terms) of the leading product, smallest first
+#pragma unroll
+            for (int q = 0; q <= t; q++)
+              if (t - q < NPB)
+#pragma unroll
+                for (int j = 0; j < NS; j++) tmp[j] = mma_rows(af[i][b][q], bf[j][b][t - q], tmp[j]);
+#pragma unroll
+        for (int j = 0; j < NS; j++) acc[i][j] += tmp[j];
+      }
+    }
+  };
+  // Unit u has landed when at most the requests of the PD - 1 units behind it are outstanding.  Its slot is asked for again
+  // when its last reads are done: no other wavefront looks into this ring, so there is no barrier.
+  for (int u = 0; u < units; u++) {
+    wait_loads<(PD - 1) * (IW + ID)>();
+    const unsigned char *slot = wown + (u % PD) * SLOT;
+#pragma unroll
+    for (int bp = 0; bp < UB / 2; bp++) pair(slot, bp, u * UB + 2 * bp);
+    wait_lds();
+    request(u + PD);
+  }
+  wait_barrier<0>();  // (the last requests have landed: the memory is free for other things)
+
+  // ---- the result: this share's partial sums, and behind the group's last ticket their sum ----
+  const bool shares = a.parts != nullptr;
+  float *mine = shares ? a.parts + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * M * NT : (float *)smem;
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NS; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int m = 16 * i + 4 * grp + r;
+        if (m >= M) continue;
+        float *o = mine + m * NT + wave * NR + 16 * j + col;
+        const float v = HALF ? acc[i][j][r] * a.rscale[m] : acc[i][j][r];
+        if (shares) __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *o = v;
+      }
+  if (shares) {
+    // a share's sums are device-scope stores that have reached memory before its ticket is drawn (a fence would write
+    // back and invalidate the whole L2 of the XCD); the counters are left at zero for the next launch
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) s_ticket = __hip_atomic_fetch_add(g_rows_tickets + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_ticket != (int)gridDim.y - 1) return;
+    if (tid == 0) __hip_atomic_store(g_rows_tickets + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    __syncthreads();
+  }
+  const float *all = shares ? a.parts + (int64_t)blockIdx.x * gridDim.y * M * NT : (const float *)smem;
+  for (int f = tid; f < M * (NT / 4); f += T) {
+    const int m = f / (NT / 4), c = 4 * (f % (NT / 4));
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (shares) {
+      for (int z0 = 0; z0 < (int)gridDim.y; z0 += 8) {  // eight shares requested together, added in order
+        unsigned long long t[8][2];
+#pragma unroll
+        for (int z = 0; z < 8; z++) {
+          const unsigned long long *src = (const unsigned long long *)(all + ((int64_t)min(z0 + z, (int)gridDim.y - 1) * M + m) * NT + c);
+          t[z][0] = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          t[z][1] = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int z = 0; z < 8; z++)
+          if (z0 + z < (int)gridDim.y) {
+            v.x += __uint_as_float((unsigned)t[z][0]), v.y += __uint_as_float((unsigned)(t[z][0] >> 32));
+            v.z += __uint_as_float((unsigned)t[z][1]), v.w += __uint_as_float((unsigned)(t[z][1] >> 32));
+          }
+      }
+    } else {
+      v = *(const float4 *)(all + m * NT + c);
+    }
+    plane_gemm_store(a.e, m, blockIdx.x * NT + c, v);
+  }
+}
+
+// ---- input rows -> planes, with what the Linear has in front ----
+// One block per row, held in registers (VPL pieces of 8 floats per thread).  HALF: fp16 terms of the row times a power of
+// two, which rscale undoes; else bf16 terms.  kbp: blocks of 32 k per row of planes (zeros past K).
+struct RowsPlanesArgs {
+  uint4 *out;
+  float *rscale;
+  const float *x;
+  int64_t stride;
+  int K, kbp;
+  const float *g, *b;
+  float eps;
+};
+template <int PRO, int NP, bool HALF, int VPL>
+__global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
+  __shared__ float red[3][4];
+  const int tid = threadIdx.x, K = a.K, nc = (K + 7) >> 3;
+  const float *xr = a.x + blockIdx.x * a.stride;
+  constexpr bool NORM = PRO == CTHIP_PRO_LAYERNORM || PRO == CTHIP_PRO_RMSNORM;
+  float v[VPL][8];
+  auto ld8 = [&](const float *p, int j, float *o) __attribute__((always_inline)) {  // K % 4 == 0: four floats are inside the row or past it
+    const int k = 8 * (tid + 256 * j);
+    const float4 t0 = *(const float4 *)(p + min(k, K - 4)), t1 = *(const float4 *)(p + min(k + 4, K - 4));
+    o[0] = t0.x, o[1] = t0.y, o[2] = t0.z, o[3] = t0.w, o[4] = t1.x, o[5] = t1.y, o[6] = t1.z, o[7] = t1.w;
+  };
+  auto in = [&](int j, int e) { return 8 * (tid + 256 * j) + e < K; };
+#pragma unroll
+  for (int j = 0; j < VPL; j++) ld8(xr, j, v[j]);
+  if (PRO == CTHIP_PRO_SWIGLU) {
+#pragma unroll
+    for (int j = 0; j < VPL; j++) {
+      float u[8];
+      ld8(xr + K, j, u);
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[j][e] = ct_silu(v[j][e]) * u[e];
+    }
+  }
+  auto block_sum = [&](int slot, float s) {
+    s = wave_sum(s);
+    if ((tid & 63) == 0) red[slot][tid >> 6] = s;
+    __syncthreads();
+    return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
+  };
+  if (NORM) {
+    const float inv_n = 1.0f / (float)K;
+    float mean = 0.0f, q = 0.0f;
+    if (PRO == CTHIP_PRO_LAYERNORM) {
+      float s = 0.0f;
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) s += in(j, e) ? v[j][e] : 0.0f;
+      mean = block_sum(0, s) * inv_n;
+    }
+#pragma unroll
+    for (int j = 0; j < VPL; j++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        v[j][e] -= mean;
+        q += in(j, e) ? v[j][e] * v[j][e] : 0.0f;
+      }
+    const float rstd = 1.0f / sqrtf(block_sum(1, q) * inv_n + a.eps);
+#pragma unroll
+    for (int j = 0; j < VPL; j++) {
+      float g[8], b[8];
+      if (a.g) ld8(a.g, j, g);
+      if (a.b) ld8(a.b, j, b);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        v[j][e] *= rstd;
+        if (a.g) v[j][e] *= g[e];
+        if (a.b) v[j][e] += b[e];
+      }
+    }
+  }
+  float up = 1.0f;
+  if (HALF) {
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPL; j++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) m = fmaxf(m, in(j, e) ? fabsf(v[j][e]) : 0.0f);
+    m = wave_max(m);
+    if ((tid & 63) == 0) red[2][tid >> 6] = m;
+    __syncthreads();
+    const unsigned mb = __float_as_uint(fmaxf(fmaxf(red[2][0], red[2][1]), fmaxf(red[2][2], red[2][3])));
+    // 2^(14 - exponent of the largest value): it lands in [2^14, 2^15).  Exponents kept where both powers are normal
+    const int ex = mb == 0 ? 141 : min(max((int)(mb >> 23), 16), 250);
+    up = __uint_as_float((unsigned)(268 - ex) << 23);
+    if (tid == 0) a.rscale[blockIdx.x] = __uint_as_float((unsigned)(ex - 14) << 23);
+  }
+#pragma unroll
+  for (int j = 0; j < VPL; j++) {
+    const int c = tid + 256 * j;
+    if (c >= 4 * a.kbp) continue;
+    float t[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] * up : 0.0f;
+    uint4 pl[NP];
+    if (HALF) split8_half<NP>(t, pl);
+    else split8_planes<NP>(t, pl);
+#pragma unroll
+    for (int q = 0; q < NP; q++) a.out[((int64_t)blockIdx.x * a.kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
+  }
+}
+constexpr int kRowsPlanesMaxK = 8 * 256 * 16;  // widest row the largest instantiation holds
+
+// One launch: how many workgroups share K.  Every compute unit holds `resident` workgroups (LDS) at a time; a round of
+// them costs its units at the rate of the compute unit (about 0.85 us per 16 KB of weights and workgroup, 30 % more per
+// further 16 input rows) and about 1.5 us of its own, a share costs its partial sums.
+template <int SRC, int NPA, int MB, bool WIDE_D>
+static int rows_launch(RowsGemmArgs a) {
+  constexpr int NS = 2, NW = 4 * MB, PD = 2, NT = 16 * NS * NW, T = 64 * NW, UB = RowsUnit<SRC>::BLOCKS;
+  constexpr int SLOT = 16 * NS * RowsUnit<SRC>::BYTES + (SRC == RW_Q8 || SRC == RW_Q4 ? 16 * NS * UB / (WIDE_D ? 2 : 1) / 64 * 256 : 0);
+  const int M = a.e.M, N = a.e.N, cus = state().compute_units;
+  const int groups = (N + NT - 1) / NT, units = (a.kblocks + UB - 1) / UB;
+  double best = 0;
+  int best_per = 0;
+  size_t best_lds = 0;
+  for (int ks = 1; ks <= 32 && ks <= units; ks++) {
+    const int per = (units + ks - 1) / ks;
+    if ((units + per - 1) / per != ks || (ks > 1 && groups > kRowsGroups)) continue;
+    size_t lds = (size_t)NW * PD * SLOT + (size_t)M * per * UB * 64 * NPA;
+    if (lds < (size_t)M * NT * 4) lds = (size_t)M * NT * 4;
+    if (lds > 156 * 1024) continue;
+    const int resident = lds <= 78 * 1024 ? 2 : 1;
+    const double tu = 0.85 * RowsUnit<SRC>::BYTES / 128 * NW / 4 * (1 + 0.3 * (MB - 1));
+    const int64_t wgs = (int64_t)groups * ks;
+    const int64_t full = wgs / (cus * resident), left = wgs - full * cus * resident;
+    double t = full * (resident * per * tu + 1.5);
+    if (left) t += (left > cus ? 2 : 1) * per * tu + 1.5;
+    t += ks > 1 ? 1.0 + (double)ks * M * N * 8 / 4e6 : 0.0;
+    if (best_per == 0 || t < best) best = t, best_per = per, best_lds = lds;
+  }
+  if (best_per == 0) return fail(CTHIP_E_STATE, "linear rows: no share of (%d, %d, %d blocks) fits", M, N, a.kblocks);
+  a.kper = best_per * UB;
+  const int ks = (units + best_per - 1) / best_per;
+  a.parts = nullptr;
+  int rc = 0;
+  if (ks > 1 && (rc = alloc_scratch((void **)&a.parts, sizeof(float) * (size_t)groups * ks * M * NT))) return rc;
+  static bool big_lds = false;
+  auto fn = k_linear_rows<SRC, NPA, MB, NS, NW, PD, WIDE_D>;
+  if (!big_lds) {
+    CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 157 * 1024));
+    big_lds = true;
+  }
+  hipLaunchKernelGGL(fn, dim3(groups, ks), dim3(T), best_lds, state().stream, a);
+  const hipError_t e = hipGetLastError();
+  if (a.parts) rc = cthip_free(a.parts);  // stream-ordered: handed out again only to later work on this stream
+  if (e != hipSuccess) return fail((int)e, "linear rows: launch -> %s", hipGetErrorString(e));
+  return rc;
+}
+
+template <int PRO, int NP, bool HALF>
+static void rows_planes_launch(const RowsPlanesArgs &a, int m) {
+  const int pieces = (a.kbp * 4 + 255) / 256;
+  const dim3 grid(m), block(256);
+#define RP(V) hipLaunchKernelGGL((k_rows_planes<PRO, NP, HALF, V>), grid, block, 0, state().stream, a)
+  if (pieces <= 1) RP(1);
+  else if (pieces <= 2) RP(2);
+  else if (pieces <= 4) RP(4);
+  else if (pieces <= 8) RP(8);
+  else RP(16);
+#undef RP
+}
+
+// Whether this is the launch to take: the operands are laid out for it, and it is the faster one.
+// Fewer than 8 rows: against the single-row kernels, one pass over the weights per row.  They cost about 3 us + m weights
+// at 4.3 (quantised), 2.7 (fp16) or 2.0 (fp32) per ns, the two launches here 9.5 us + the weights once at 3.2 / 2.3 / 1.15.
+//   us, m = 3 / 5 / 7:  4096 x 4096 Q8_0 17 / 20 / 29 -> 12 / 14 / 14;  22016 x 4096 Q8_0 52 / 80 / 110 -> 31 / 39 / 41;
+//   4096 x 11008 Q4_0 m = 5 50 -> 22;  768 x 3072 stays there at 5 / 6 / 9 (12 .. 15 here)
+// 8 rows and more: against a GEMM tile of 64 rows, which is as fast on small matrices and where the tile fills up:
+//   22016 x 4096 m = 12 / 24: Q8_0 52 / 55 -> 42 / 54, Q4_0 53 / 53 -> 36 / 55, fp16 78 / 78 -> 53 / 61, fp32 103 / 107 -> 109 / 111;
+//   11264 x 2048 m = 12: 19, 20, 27 -> 17, 17, 19;  4096 x 4096 m = 12: 14, 14, 18 -> 15, 15, 18
+bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b) {
+  if (m < 2 || m > kRowsMax || (m >= 8 && precision == GEMM_FP32)) return false;
+  if (w->cols % (w->type == CTHIP_F16 ? 8 : 4) || w->cols < 64 || w->cols > kRowsPlanesMaxK - 256) return false;  // whole 16-byte pieces
+  auto al = [](const void *p) { return (uintptr_t)p % 16 == 0; };
+  if (x_stride % 4 || !al(x) || !al(g) || !al(b)) return false;
+  const double weights = (double)w->rows * w->cols * 1e-3;
+  const bool quant = w->type == CTHIP_Q8_0 || w->type == CTHIP_Q4_0;
+  if (m < 8) {
+    const double each = quant ? 4.3 : w->type == CTHIP_F16 ? 2.7 : 2.0, once = quant ? 3.2 : w->type == CTHIP_F16 ? 2.3 : 1.15;
+    return 3000 + m * weights / each > 9500 + weights / once;
+  }
+  if (w->type == CTHIP_F32) return false;
+  return m <= 16 ? weights >= (quant ? 22e3 : 20e3) : w->type == CTHIP_F16 && weights >= 60e3;
+}
+
+// y (m, rows) = act(prologue(x) @ W^T + bias) + residual for a few rows; act may be kActSwigluPairs, route as for
+// launch_linear_gemm.  Call only where linear_rows_pays.
+int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
+                       int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route) {
+  const int terms = m < 8 ? 3 : precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1;
+  const bool half = w->type != CTHIP_F32;
+  const int ub = w->type == CTHIP_Q8_0 ? RowsUnit<RW_Q8>::BLOCKS : w->type == CTHIP_Q4_0 ? RowsUnit<RW_Q4>::BLOCKS : RowsUnit<RW_F16>::BLOCKS;
+  RowsGemmArgs a = {};
+  a.kblocks = (int)((w->cols + 31) / 32);
+  a.nkb = (a.kblocks + ub - 1) / ub * ub;
+  a.W = (const unsigned char *)w->q;
+  a.wd = (const unsigned short *)w->d;
+  a.dpitch = (int)(w->cols / 32);
+  a.wbytes = (int)(w->type == CTHIP_Q8_0 ? w->cols : w->type == CTHIP_Q4_0 ? w->cols / 2 : w->type == CTHIP_F16 ? 2 * w->cols : 4 * w->cols);
+  a.e.C = y;
+  a.e.M = m;
+  a.e.N = (int)w->rows;
+  a.e.bias = bias;
+  a.e.residual = residual;
+  a.e.act = act;
+  if (act == kActSwigluPairs) {
+    if (a.e.N % 4 || residual || route) return fail(CTHIP_E_BAD_ARG, "launch_linear_rows: paired SwiGLU epilogue with %d rows, a residual or a route", a.e.N);
+    a.e.act = CTHIP_ACT_NONE;
+    a.e.pairs = 1;
+  }
+  if (route) {
+    a.e.routed = 1;
+    a.e.route = *route;
+  }
+  unsigned char *planes = nullptr;
+  const size_t plane_bytes = (size_t)m * a.nkb * 64 * terms;
+  int rc = alloc_scratch((void **)&planes, plane_bytes + sizeof(float) * kRowsMax);  // fully written by the first launch
+  if (rc) return rc;
+  a.A = planes;
+  float *rscale = (float *)(planes + plane_bytes);
+  a.rscale = half ? rscale : nullptr;
+  const RowsPlanesArgs pa = {(uint4 *)planes, rscale, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
+#define RP3(PRO, HALF)                                           \
+  do {                                                           \
+    if (terms == 3) rows_planes_launch<PRO, 3, HALF>(pa, m);     \
+    else if (terms == 2) rows_planes_launch<PRO, 2, HALF>(pa, m); \
+    else rows_planes_launch<PRO, 1, HALF>(pa, m);                \
+  } while (0)
+#define RP2(HALF)                                        \
+  switch (pro) {                                         \
+    case CTHIP_PRO_LAYERNORM: RP3(CTHIP_PRO_LAYERNORM, HALF); break; \
+    case CTHIP_PRO_RMSNORM: RP3(CTHIP_PRO_RMSNORM, HALF); break;     \
+    case CTHIP_PRO_SWIGLU: RP3(CTHIP_PRO_SWIGLU, HALF); break;       \
+    default: RP3(CTHIP_PRO_NONE, HALF); break;           \
+  }
+  if (half) {
+    RP2(true)
+  } else {
+    RP2(false)
+  }
+#undef RP2
+#undef RP3
+  const bool wide = a.dpitch % 2 == 0;
+#define RL4(SRC, NPA, WD)                                  \
+  do {                                                     \
+    if (m <= 16) rc = rows_launch<SRC, NPA, 1, WD>(a);     \
+    else rc = rows_launch<SRC, NPA, 2, WD>(a);             \
+  } while (0)
+#define RL3(SRC, WD)                      \
+  do {                                    \
+    if (terms == 3) RL4(SRC, 3, WD);      \
+    else if (terms == 2) RL4(SRC, 2, WD); \
+    else RL4(SRC, 1, WD);                 \
+  } while (0)
+  if (w->type == CTHIP_Q8_0 && wide) RL3(RW_Q8, true);
+  else if (w->type == CTHIP_Q8_0) RL3(RW_Q8, false);
+  else if (w->type == CTHIP_Q4_0 && wide) RL3(RW_Q4, true);
+  else if (w->type == CTHIP_Q4_0) RL3(RW_Q4, false);
+  else if (w->type == CTHIP_F16) RL3(RW_F16, false);
+  else RL3(RW_F32, false);
+#undef RL3
+#undef RL4
+  const int rf = cthip_free(planes);  // stream-ordered: handed out again only to later work on this stream
+  return rc ? rc : rf;
+}
+
+}  // namespace cthip

@@ -1,0 +1,175 @@
+// GEMM operands in memory as bf16 terms (gemm_planes.hip): layout and the epilogue shared by its instantiations.
+#pragma once
+#include "common.h"
+
+namespace cthip {
+
+enum { PL_PLANES = 0, PL_Q8 = 1, PL_Q4 = 2, PL_INT = 3 };
+
+struct PlaneGemmArgs {
+  float *C;
+  const unsigned char *A, *B;
+  const unsigned short *bd;  // scales of raw quants
+  int apitch, bpitch;        // bytes between rows
+  int dpitch;                // scales between rows
+  int M, N, nkb;             // nkb: blocks of 32 k
+  int kper;                  // blocks per workgroup along gridDim.y (split K)
+  const float *bias, *residual;
+  int act;
+  float *ws;                 // split K: raw partial tiles ws[z][M][N]; null: C is complete
+  int tm, tn, rx, rm, rn;    // tile -> workgroup mapping, one region of tiles per XCD (see GemmArgs)
+  int pairs;                 // columns (2j, 2j + 1) are (gate, up): C (M, N / 2) gets silu(gate) * up
+  int routed;
+  GemmRoute route;
+  unsigned short *planes;    // non-null: the result goes out as planes of two terms instead of C
+  int pkb;                   // blocks of 32 columns per row of `planes`
+};
+
+#if defined(__HIPCC__)
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf_pl __attribute__((ext_vector_type(2)));
+typedef float v2f_pl __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned pack_bf16_pl(float x0, float x1) {  // one v_cvt_pk_bf16_f32, round to nearest even
+  const v2f_pl v = {x0, x1};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, v2bf_pl));
+}
+template <int NP>
+__device__ __forceinline__ void split4_planes(float r0, float r1, float r2, float r3, uint2 *pl) {
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    pl[p].x = pack_bf16_pl(r0, r1);
+    pl[p].y = pack_bf16_pl(r2, r3);
+    if (p + 1 < NP) {  // exact: the difference of a float and its own leading bits
+      r0 -= __uint_as_float(pl[p].x << 16);
+      r1 -= __uint_as_float(pl[p].x & 0xffff0000u);
+      r2 -= __uint_as_float(pl[p].y << 16);
+      r3 -= __uint_as_float(pl[p].y & 0xffff0000u);
+    }
+  }
+}
+template <int NP>
+__device__ __forceinline__ void split8_planes(const float *v, uint4 *pl) {
+  uint2 a[NP], b[NP];
+  split4_planes<NP>(v[0], v[1], v[2], v[3], a);
+  split4_planes<NP>(v[4], v[5], v[6], v[7], b);
+#pragma unroll
+  for (int p = 0; p < NP; p++) pl[p] = make_uint4(a[p].x, a[p].y, b[p].x, b[p].y);
+}
+// four consecutive columns col .. col + 3 (col a multiple of 4) of a row as two-term planes
+__device__ __forceinline__ void store_planes4(unsigned short *planes, int64_t row, int pkb, int col, const float *v) {
+  uint2 pl[2];
+  split4_planes<2>(v[0], v[1], v[2], v[3], pl);
+  unsigned short *p = planes + (row * pkb + (col >> 5)) * 64 + (col & 31);
+  *(uint2 *)p = pl[0];
+  *(uint2 *)(p + 32) = pl[1];
+}
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// 16 bytes per lane from sbase + voff straight into LDS at lds + 16 * lane.  Written out because the compiler, which
+// cannot tell the buffers of a ring apart, waits for ALL such loads before every LDS read; the kernel below counts
+// them itself (the reads it protects lie behind the same asm's "memory" clobber).
+__device__ __forceinline__ void dma16(const void *sbase, unsigned voff, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory");
+}
+// 2 bytes per lane, zero-extended to the dword at lds + 4 * lane
+__device__ __forceinline__ void dma2(const void *sbase, unsigned voff, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_ushort %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory");
+}
+// 4 bytes per lane
+__device__ __forceinline__ void dma4(const void *sbase, unsigned voff, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory");
+}
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ const unsigned char *uniform(const unsigned char *p) {
+  const uint64_t v = (uint64_t)p;
+  return (const unsigned char *)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)v));
+}
+// all but the youngest N of this wavefront's loads have landed, its LDS reads are done, and so are everybody else's
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // ... of this wavefront only
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ unsigned pack_int_bf16(float x0, float x1) {
+  return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);  // high halves of both
+}
+// 8 int8 -> 8 bf16, exact
+__device__ __forceinline__ v8bf bf_of_q8(unsigned a, unsigned b) {
+  return __builtin_bit_cast(v8bf, make_uint4(pack_int_bf16(sbyte0_f32(a), sbyte1_f32(a)), pack_int_bf16(sbyte2_f32(a), sbyte3_f32(a)),
+                                             pack_int_bf16(sbyte0_f32(b), sbyte1_f32(b)), pack_int_bf16(sbyte2_f32(b), sbyte3_f32(b))));
+}
+// 8 nibbles (one per byte of a and b, 0..15) -> nibble - 8 as bf16, exact
+__device__ __forceinline__ v8bf bf_of_q4(unsigned a, unsigned b) {
+  a = (a + 0x78787878u) ^ 0x80808080u;  // per byte: nibble - 8 as int8 (no carry leaves a byte)
+  b = (b + 0x78787878u) ^ 0x80808080u;
+  return bf_of_q8(a, b);
+}
+
+// columns col .. col + 3 of one row of a finished tile: bias, activation, residual, and where they go
+__device__ __forceinline__ void plane_gemm_store(const PlaneGemmArgs &a, int row, int col, float4 v4) {
+  const int N = a.N;
+  if (row >= a.M || col >= N) return;
+  float v[4] = {v4.x, v4.y, v4.z, v4.w};
+  if (a.ws) {
+    float *o = a.ws + ((int64_t)blockIdx.y * a.M + row) * N + col;
+    if ((N & 3) == 0) *(float4 *)o = v4;
+    else
+      for (int t = 0; t < 4 && col + t < N; t++) o[t] = v[t];
+    return;
+  }
+  if ((N & 3) == 0) {
+    if (a.bias) {
+      const float4 bb = *(const float4 *)(a.bias + col);
+      v[0] += bb.x, v[1] += bb.y, v[2] += bb.z, v[3] += bb.w;
+    }
+    if (a.pairs) {
+      v[0] = apply_act(CTHIP_ACT_SILU, v[0]) * v[1], v[1] = apply_act(CTHIP_ACT_SILU, v[2]) * v[3];
+      if (a.planes) {  // two columns of the result: neighbours in both terms
+        const unsigned h = pack_bf16_pl(v[0], v[1]);
+        const unsigned l = pack_bf16_pl(v[0] - __uint_as_float(h << 16), v[1] - __uint_as_float(h & 0xffff0000u));
+        unsigned short *p = a.planes + ((int64_t)row * a.pkb + (col >> 6)) * 64 + ((col >> 1) & 31);
+        *(unsigned *)p = h;
+        *(unsigned *)(p + 32) = l;
+      } else {
+        *(float2 *)(a.C + (int64_t)row * (N >> 1) + (col >> 1)) = make_float2(v[0], v[1]);
+      }
+      return;
+    }
+    if (a.act != CTHIP_ACT_NONE)
+#pragma unroll
+      for (int t = 0; t < 4; t++) v[t] = apply_act(a.act, v[t]);
+    if (a.residual) {
+      const float4 rr = *(const float4 *)(a.residual + (int64_t)row * N + col);
+      v[0] += rr.x, v[1] += rr.y, v[2] += rr.z, v[3] += rr.w;
+    }
+    if (a.planes) {
+      store_planes4(a.planes, row, a.pkb, col, v);
+      return;
+    }
+    float *dst = a.C;
+    int ldd = N, cbase = 0;
+    if (a.routed) {
+      // (selected, not indexed: an index would put the arguments into scratch memory)
+      const bool p2 = col >= a.route.c0[2], p1 = col >= a.route.c0[1];
+      dst = p2 ? a.route.dst[2] : p1 ? a.route.dst[1] : a.route.dst[0];
+      ldd = p2 ? a.route.ld[2] : p1 ? a.route.ld[1] : a.route.ld[0];
+      cbase = p2 ? a.route.c0[2] : p1 ? a.route.c0[1] : 0;
+    }
+    *(float4 *)(dst + (int64_t)row * ldd + (col - cbase)) = make_float4(v[0], v[1], v[2], v[3]);
+    return;
+  }
+  for (int t = 0; t < 4 && col + t < N; t++) {
+    float x = apply_act(a.act, v[t] + (a.bias ? a.bias[col + t] : 0.0f));
+    if (a.residual) x += a.residual[(int64_t)row * N + col + t];
+    a.C[(int64_t)row * N + col + t] = x;
+  }
+}
+#endif
+
+}  // namespace cthip

@@ -1,0 +1,76 @@
+"""Linears over 2 .. 32 rows in one pass over the weights (csrc/linear_rows.hip) at the shapes where it takes over: column
+groups and units of k that the matrix does not fill, rows of an odd number of blocks (scales fetched one by one), widths
+that are no multiple of a block, every prologue and terms per input, the largest and smallest row counts of its tiles."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from caten_amd import _lib, ops as o
+    _lib.init(0)
+    return o
+
+
+def packed(kind, a):
+    from caten_amd.llm import Tensor
+    return Tensor.from_f32(a, kind).raw
+
+
+def norm(x, g, b, kind):
+    if kind == "layernorm":
+        x = x - x.mean(-1, keepdims=True)
+    x = x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-5) * g
+    return x + b if kind == "layernorm" else x
+
+
+@pytest.mark.parametrize("kind,rows,cols,m", [
+    ("q8_0", 2611, 2080, 7), ("q8_0", 12000, 2048, 3), ("q8_0", 9001, 2560, 8), ("q8_0", 9001, 2560, 16),
+    ("q4_0", 2611, 2080, 7), ("q4_0", 2600, 11008, 2), ("q4_0", 9001, 2560, 9), ("q4_0", 700, 11008, 6),
+    ("f16", 2603, 2056, 7), ("f16", 4099, 5000, 5), ("f16", 9001, 2560, 16), ("f16", 15001, 4104, 17), ("f16", 15001, 4104, 32),
+    ("f32", 2603, 2052, 7), ("f32", 1501, 4100, 4)])
+@pytest.mark.parametrize("prologue", [None, "layernorm", "rmsnorm", "swiglu"])
+def test_linear_rows(ops, kind, rows, cols, m, prologue):
+    rng = np.random.default_rng(rows + m)
+    w = ops.WeightMatrix(kind, packed(kind, rng.normal(0, 0.05, (rows, cols)).astype(np.float32)), rows, cols)
+    x = rng.normal(0, 1, (m, cols * (2 if prologue == "swiglu" else 1))).astype(np.float32)
+    x[:, 3] *= 300.0  # one input far above the others of its row
+    g, b = rng.normal(1, 0.05, cols).astype(np.float32), rng.normal(0, 0.05, cols).astype(np.float32)
+    bias, res = rng.normal(0, 1, rows).astype(np.float32), rng.normal(0, 1, (m, rows)).astype(np.float32)
+    at = np.unique(np.r_[0:40, rows - 40:rows, rng.integers(0, rows, 100)])  # output columns that are checked
+    x64 = x.astype(np.float64)
+    if prologue == "swiglu":
+        x64 = x64[:, :cols] / (1 + np.exp(-x64[:, :cols])) * x64[:, cols:]
+    elif prologue:
+        x64 = norm(x64, g, b, prologue)
+    want = np.maximum(x64 @ w.dequantize()[at].astype(np.float64).T + bias[at], 0.0) + res[:, at]
+    kw = dict(norm_g=g, norm_b=b if prologue == "layernorm" else None) if prologue in ("layernorm", "rmsnorm") else {}
+    for _ in range(2):  # the shares' counters are back at zero
+        got = ops.linear(x, w, bias, res, act="relu", prologue=prologue, **kw)[:, at]
+        rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert rel < (1e-6 if m < 8 else 1e-5), rel
+    w.free()
+
+
+@pytest.mark.parametrize("rows", [2, 3, 7])
+def test_short_prompt_equals_its_rows_one_by_one(ops, rows):
+    from caten_amd import _lib, llm, synth
+    cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], max_seq=700)
+    model = llm.make_llama(cfg, llm.llama_state_dict(synth.llama_weights(cfg, seed=3), "q8_0"))
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], 640 + rows, seed=3)]
+    lib = _lib.load()
+    model.forward(ids[:640], 640, 0)
+    got = [model.forward(ids[n:n + rows], rows, n, return_logits=True) for n in (5, 640)]  # a short and a long context
+    try:
+        _lib.check(lib.cthip_set_option(b"prefill_gemm", 0))
+        model.forward(ids[5:5 + rows], rows, 5)
+        model.forward(ids[5:640], 635, 5)
+        want = [model.forward(ids[n:n + rows], rows, n, return_logits=True) for n in (5, 640)]
+    finally:
+        _lib.check(lib.cthip_set_option(b"prefill_gemm", 1))
+    for (t0, l0), (t1, l1) in zip(got, want):
+        assert t0 == t1
+        assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
+    model.close()
