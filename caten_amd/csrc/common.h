@@ -255,6 +255,10 @@ int launch_linear_gemm(float *y, const WMat *w, const float *x, int m, const flo
 bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b);
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route = nullptr);
+// matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
+bool matmul_planes_pay(int M, int N, int K, int precision);
+int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N, int K, int act, const float *bias, const float *residual, int precision,
+                         bool *done);
 bool reduce_norm_supported(int n, int nparts);
 // C (m, n) = sum_z ws[z] + bias + residual for partial tiles handed over through GemmDeferred
 int launch_splitk_reduce(float *C, float *ws, int ksplit, int m, int n, const float *bias, const float *residual);

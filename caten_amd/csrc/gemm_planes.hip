@@ -1,0 +1,492 @@
+// MFMA GEMM over operands that lie in memory as bf16 terms ("planes"), for products large enough to fill the chip:
+// prompts, Linears over many rows and big matmuls.  The small ones stay with matmul.hip.
+//
+// matmul.hip converts fp32 operands on their way into LDS, once per tile: every tile of a row of tiles repeats the
+// conversion of the same rows, a third of a workgroup's wavefronts do nothing else, and a 64 x 64 (64 x 128) tile asks the
+// caches for 64 bytes per matrix instruction.  Here an operand is split ONCE (by k_planes_rows / k_planes_cols or by
+// the kernel that produces it) and the GEMM kernel only moves and multiplies: global memory -> LDS by the load path that
+// bypasses registers, LDS -> operand registers, matrix cores.
+//
+// Layout of a plane operand: row-major, a row is a sequence of blocks of 32 consecutive k, a block is NP runs of 32
+// bf16 (term 0 = bf16(x), term p = bf16 of what terms 0..p-1 miss).  A K-step of a row is one contiguous piece of NP * 64
+// bytes: whole cache lines for NP = 2.
+#include "common.h"
+#include "planes.h"
+
+namespace cthip {
+
+// 16-byte chunk c of row r of an LDS tile with CPR chunks per row is kept at chunk r * CPR + (c ^ swz<CPR>(r)): eight
+// consecutive rows then read (or are written) eight different 16-byte columns of the banks.
+template <int CPR>
+__device__ __forceinline__ int swz(int r) {
+  return CPR % 8 == 0 ? (r & 7) : CPR % 4 == 0 ? ((r >> 1) & 3) : CPR % 2 == 0 ? ((r >> 2) & 1) : 0;
+}
+
+// SRC: how B lies in memory: PL_PLANES, or PL_INT, one plane of the integers of a quantised matrix (exact in bf16) with an
+// fp16 scale per block of 32, which is applied to the block's partial sum (acc += d * sum a q).
+// MB x NB blocks of 32 x 32 per wavefront, WM x WN wavefronts, NBUF LDS buffers; a step is a block of 32 k.
+//
+// What bounds it: the matrix cores ask LDS for an operand per instruction and block edge, so a wavefront's piece wants to be
+// large (64 x 64: 16 reads for 24 instructions at two terms); two workgroups of four wavefronts per compute unit fill each
+// other's waits.  4096^3, two terms: 371 TFLOP/s of results = 1.1 PFLOP/s of matrix instructions (the library's bf16 product
+// of this size reaches 1.2 - 1.5 on the card), against 180 with the operands converted per tile.
+template <int NPA, int SRC, int NPB, int MB, int NB, int WM, int WN, int NBUF>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a) {
+  constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN;
+  constexpr int CA = 4 * NPA, CB = 4 * NPB;  // chunks per row and step
+  constexpr int ABYTES = BM * CA * 16, BBYTES = BN * CB * 16, SBYTES = SRC == PL_PLANES ? 0 : BN * 4;
+  constexpr int BUF = ABYTES + BBYTES + SBYTES;
+  constexpr int IA = (BM * CA / 64 + NW - 1) / NW, IB = (BN * CB / 64 + NW - 1) / NW;  // load instructions per wavefront and step
+  constexpr int IS = SRC == PL_PLANES ? 0 : (BN / 64 + NW - 1) / NW;
+  constexpr int LOADS = IA + IB + IS;
+  static_assert(BM * CA % 64 == 0 && BN * CB % 64 == 0, "whole load instructions");
+  extern __shared__ __align__(16) unsigned char smem[];
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  if (local >= a.rm * a.rn) return;
+  const int mi = (xcd % a.rx) * a.rm + local % a.rm, ni = (xcd / a.rx) * a.rn + local / a.rm;
+  if (mi >= a.tm || ni >= a.tn) return;  // the regions overhang a grid they do not divide
+  const int m0 = mi * BM, n0 = ni * BN;
+  const int kb0 = blockIdx.y * a.kper, kb1 = min(a.nkb, kb0 + a.kper);  // this workgroup's blocks of 32 k
+  const int nsteps = kb1 - kb0;
+
+  // where this lane's pieces of a step lie, as offsets from the step's bases; rows past the end repeat the last one
+  unsigned avo[IA], bvo[IB], svo[IS > 0 ? IS : 1];
+#pragma unroll
+  for (int j = 0; j < IA; j++) {
+    const int s = ((j * NW + wave) * 64 + lane) % (BM * CA), r = s / CA, c = (s % CA) ^ swz<CA>(r);
+    avo[j] = (unsigned)(min(r, a.M - 1 - m0) * a.apitch + c * 16);
+  }
+#pragma unroll
+  for (int j = 0; j < IB; j++) {
+    const int s = ((j * NW + wave) * 64 + lane) % (BN * CB), r = s / CB, c = (s % CB) ^ swz<CB>(r);
+    bvo[j] = (unsigned)(min(r, a.N - 1 - n0) * a.bpitch + c * 16);
+  }
+#pragma unroll
+  for (int j = 0; j < IS; j++) {
+    const int s = ((j * NW + wave) * 64 + lane) % BN;
+    svo[j] = (unsigned)(min(s, a.N - 1 - n0) * a.dpitch) * 2u;
+  }
+  const unsigned char *ab = a.A + (int64_t)m0 * a.apitch + (int64_t)kb0 * (64 * NPA);
+  const unsigned char *bb = a.B + (int64_t)n0 * a.bpitch + (int64_t)kb0 * (CB * 16);
+  const unsigned char *sb = SRC == PL_PLANES ? nullptr : (const unsigned char *)(a.bd + (int64_t)n0 * a.dpitch + kb0);
+  auto issue = [&](int step, int buf) __attribute__((always_inline)) {
+    step = min(step, nsteps - 1);  // past the end: the last step again, so that the counts stay the same
+    const unsigned base = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)buf * BUF);
+    const unsigned char *as = uniform(ab + (int64_t)step * (CA * 16)), *bs = uniform(bb + (int64_t)step * (CB * 16));
+#pragma unroll
+    for (int j = 0; j < IA; j++) dma16(as, avo[j], base + ((j * NW + wave) * 1024) % ABYTES);
+#pragma unroll
+    for (int j = 0; j < IB; j++) dma16(bs, bvo[j], base + ABYTES + ((j * NW + wave) * 1024) % BBYTES);
+#pragma unroll
+    for (int j = 0; j < IS; j++) dma2(uniform(sb + (int64_t)step * 2), svo[j], base + ABYTES + BBYTES + ((j * NW + wave) * 256) % (SBYTES ? SBYTES : 1));
+  };
+
+  v16f acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][b][r] = 0.0f;
+
+  const int half = lane >> 5, col = lane & 31;
+  // k of the matrix instructions of a block: slice s, lane half h take k = 16 h + 8 s .. +7 (the same for A and B)
+  auto mul = [&](int buf) __attribute__((always_inline)) {
+    const unsigned char *At = smem + buf * BUF, *Bt = At + ABYTES;
+    const int ra = 32 * MB * wm + col, rb = 32 * NB * wn + col;
+    auto lda = [&](int i, int ch) { return *(const uint4 *)(At + ((ra + 32 * i) * CA + (ch ^ swz<CA>(ra))) * 16); };
+    auto ldb = [&](int b, int ch) { return *(const uint4 *)(Bt + ((rb + 32 * b) * CB + (ch ^ swz<CB>(rb))) * 16); };
+    // The operands of a slice are read before the slice in front of it is multiplied, behind a scheduling fence: left alone
+    // the compiler puts every LDS read right in front of its use, and each pair of matrix instructions waits out an LDS
+    // round trip.
+    v8bf af[2][MB][NPA], bf[2][NB][NPB];
+    auto ld = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int p = 0; p < NPB; p++) bf[s][b][p] = __builtin_bit_cast(v8bf, ldb(b, p * 4 + 2 * half + s));
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int p = 0; p < NPA; p++) af[s][i][p] = __builtin_bit_cast(v8bf, lda(i, p * 4 + 2 * half + s));
+    };
+    ld(0);
+    ld(1);
+    if constexpr (SRC == PL_PLANES) {
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        __builtin_amdgcn_sched_barrier(0);
+        // every pair of terms whose product is above 2^-8(terms) of the leading one, smallest first
+#pragma unroll
+        for (int t = (NPA > NPB ? NPA : NPB) - 1; t >= 0; t--)
+#pragma unroll
+          for (int p = 0; p <= t; p++)
+            if (p < NPA && t - p < NPB)
+#pragma unroll
+              for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s][i][p], bf[s][b][t - p], acc[i][b], 0, 0, 0);
+      }
+    } else {
+      float d[NB];
+#pragma unroll
+      for (int b = 0; b < NB; b++) d[b] = half_bits_to_float((unsigned short)((const unsigned *)(Bt + BBYTES))[rb + 32 * b]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < NB; b++) asm("" : "+v"(d[b]));  // as a float: a multiply-add that converts its fp16 operand runs at half rate
+      // the partial sums of column block b - 1 are scaled under the matrix instructions of column block b
+      v16f tmp[2][MB];
+#pragma unroll
+      for (int b = 0; b <= NB; b++) {
+        if (b < NB) {
+#pragma unroll
+          for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) tmp[b & 1][i][r] = 0.0f;
+#pragma unroll
+          for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int p = NPA - 1; p >= 0; p--)
+#pragma unroll
+              for (int i = 0; i < MB; i++) tmp[b & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s][i][p], bf[s][b][0], tmp[b & 1][i], 0, 0, 0);
+        }
+        if (b > 0)
+#pragma unroll
+          for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][b - 1][r] = fmaf(d[b - 1], tmp[(b - 1) & 1][i][r], acc[i][b - 1][r]);
+      }
+    }
+  };
+
+  if (nsteps > 0) {
+#pragma unroll
+    for (int s = 0; s < NBUF - 1; s++) issue(s, s);
+    int buf = 0;
+    for (int i = 0; i < nsteps; i++) {
+      wait_barrier<LOADS *(NBUF - 2)>();  // step i has landed; nobody reads the buffer of step i - 1 any more
+      issue(i + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
+      mul(buf);
+      buf = buf + 1 == NBUF ? 0 : buf + 1;
+    }
+  }
+  wait_barrier<0>();
+
+  // ---- acc[i][b][r] is row 8 (r / 4) + 4 half + r % 4, column `col` of its block.  A wavefront turns its blocks around
+  // in a piece of LDS of its own (no barrier) and stores rows of 32 NB columns, 16 bytes per lane.
+  constexpr int LDC = 32 * NB + 4, C4 = 8 * NB;
+  float *Cs = (float *)smem + wave * 32 * LDC;
+#pragma unroll
+  for (int i = 0; i < MB; i++) {
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) Cs[(8 * (r >> 2) + 4 * half + (r & 3)) * LDC + 32 * b + col] = acc[i][b][r];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll 2  // (a body small enough that the loop over i is unrolled for certain: acc has to stay in registers)
+    for (int u = 0; u < 32 * C4 / 64; u++) {
+      const int f = lane + 64 * u, lr = f / C4, c4 = f % C4;
+      const float4 v = *(const float4 *)(Cs + lr * LDC + 4 * c4);
+      plane_gemm_store(a, m0 + 32 * (MB * wm + i) + lr, n0 + 32 * NB * wn + 4 * c4, v);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// ---- operands -> planes ----
+// fp32 / fp16 rows (R, K) with pitch ld: a thread takes 8 consecutive k.  kbp: blocks of a plane row (k past K are zeros)
+template <int NP, typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_planes_rows(uint4 *__restrict__ out, const T *__restrict__ x, int64_t R, int K, int64_t ld, int kbp) {
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int per = kbp * 4;
+  if (u >= R * per) return;
+  const int64_t row = u / per;
+  const int c = (int)(u - row * per), k = 8 * c;
+  float v[8];
+  const T *p = x + row * ld + k;
+  if (VEC) {
+    if (k < K) {
+      if constexpr (sizeof(T) == 4) {
+        const float4 t0 = *(const float4 *)p, t1 = *(const float4 *)(p + 4);
+        v[0] = t0.x, v[1] = t0.y, v[2] = t0.z, v[3] = t0.w, v[4] = t1.x, v[5] = t1.y, v[6] = t1.z, v[7] = t1.w;
+      } else {
+        const uint4 t = *(const uint4 *)p;
+        const unsigned w[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[2 * j] = half_bits_to_float((unsigned short)(w[j] & 0xffff)), v[2 * j + 1] = half_bits_to_float((unsigned short)(w[j] >> 16));
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] = 0.0f;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = k + j < K ? (float)p[j] : 0.0f;
+  }
+  uint4 pl[NP];
+  split8_planes<NP>(v, pl);
+#pragma unroll
+  for (int q = 0; q < NP; q++) out[(row * kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
+}
+
+// (K, N) row-major -> planes of its columns (N rows of K): a workgroup turns 64 k x 64 n around in LDS
+template <int NP, bool VEC>
+__global__ __launch_bounds__(256) void k_planes_cols(uint4 *__restrict__ out, const float *__restrict__ x, int K, int N, int kbp) {
+  __shared__ float T[64][65];
+  const int k0 = blockIdx.y * 64, n0 = blockIdx.x * 64, tid = threadIdx.x;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int k = k0 + (tid >> 4) + 16 * j, n = n0 + 4 * (tid & 15);
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (k < K) {
+      const float *p = x + (int64_t)k * N + n;
+      if (VEC) {
+        if (n < N) v = *(const float4 *)p;
+      } else {
+        if (n < N) v.x = p[0];
+        if (n + 1 < N) v.y = p[1];
+        if (n + 2 < N) v.z = p[2];
+        if (n + 3 < N) v.w = p[3];
+      }
+    }
+    float *t = &T[(tid >> 4) + 16 * j][4 * (tid & 15)];
+    t[0] = v.x, t[1] = v.y, t[2] = v.z, t[3] = v.w;
+  }
+  __syncthreads();
+  const int n = tid >> 2;
+  if (n0 + n >= N) return;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int c = 2 * (tid & 3) + j;  // chunk of 8 k within the 64
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = T[8 * c + e][n];
+    uint4 pl[NP];
+    split8_planes<NP>(v, pl);
+    if (k0 / 32 + (c >> 2) < kbp)
+#pragma unroll
+      for (int q = 0; q < NP; q++) out[((int64_t)(n0 + n) * kbp + k0 / 32 + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
+  }
+}
+
+// quant plane of a Q8_0 / Q4_0 matrix -> one plane of its integers: a thread takes 8 consecutive k
+template <bool Q4>
+__global__ __launch_bounds__(256) void k_planes_int(uint4 *__restrict__ out, const unsigned char *__restrict__ q, int64_t n8) {
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;  // rows are whole blocks: the planes are as contiguous as the quants
+  if (u >= n8) return;
+  unsigned a, b;
+  if (Q4) {
+    const uint2 t = *(const uint2 *)(q + (u >> 2) * 16 + 8 * (u & 1));
+    const int sh = (u & 2) ? 4 : 0;  // k 0..15 of a block are the low nibbles of its bytes, 16..31 the high ones
+    a = (((t.x >> sh) & 0x0f0f0f0fu) + 0x78787878u) ^ 0x80808080u;  // per byte: nibble - 8 as int8 (no carry leaves a byte)
+    b = (((t.y >> sh) & 0x0f0f0f0fu) + 0x78787878u) ^ 0x80808080u;
+  } else {
+    const uint2 t = *(const uint2 *)(q + u * 8);
+    a = t.x, b = t.y;
+  }
+  out[u] = __builtin_bit_cast(uint4, bf_of_q8(a, b));
+}
+
+template <int NPA, int SRC, int NPB, int MB, int NB, int WM, int WN, int NBUF>
+static int planes_launch(PlaneGemmArgs a) {
+  constexpr int BM = 32 * MB * WM, BN = 32 * NB * WN;
+  constexpr size_t buf = (size_t)BM * 64 * NPA + (size_t)BN * 64 * NPB + (SRC == PL_PLANES ? 0 : BN * 4);
+  constexpr size_t turn = (size_t)WM * WN * 32 * (32 * NB + 4) * 4;
+  constexpr size_t lds = NBUF * buf > turn ? NBUF * buf : turn;
+  static_assert(lds <= 160 * 1024, "LDS");
+  a.tm = (a.M + BM - 1) / BM;
+  a.tn = (a.N + BN - 1) / BN;
+  // one region of tiles per XCD: the split with the fewest tiles per XCD, then the least operand bytes per L2
+  double best = -1.0;
+  for (int rx = 1; rx <= 8; rx *= 2) {
+    const int ry = 8 / rx, rm = (a.tm + rx - 1) / rx, rn = (a.tn + ry - 1) / ry;
+    const double score = (double)rm * rn * 1e6 + (double)rm * BM * NPA + (double)rn * BN * NPB;
+    if (best < 0 || score < best) best = score, a.rx = rx, a.rm = rm, a.rn = rn;
+  }
+  a.kper = a.nkb;
+  auto fn = k_gemm_planes<NPA, SRC, NPB, MB, NB, WM, WN, NBUF>;
+  static bool big_lds = false;
+  if (!big_lds && lds > 64 * 1024) {
+    CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    big_lds = true;
+  }
+  hipLaunchKernelGGL(fn, dim3(8u * a.rm * a.rn), dim3(64 * WM * WN), lds, state().stream, a);
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+
+// Which tile: the one whose rounds over the chip cost least.  A compute unit holds `resident` workgroups; alone a workgroup
+// reaches `one`, together they reach `all` (TFLOP/s of results, measured at 1024^3, 2000^3 and 4096^3; one term runs at 2.4 times
+// the rate of two).
+struct PlaneTile {
+  int bm, bn, resident;
+  double one, all;
+};
+static double plane_tile_us(const PlaneTile &t, const PlaneGemmArgs &a, int cus) {
+  const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn), slots = (int64_t)cus * t.resident;
+  const double work = 2.0 * t.bm * t.bn * 32.0 * a.nkb * cus * 1e-6;  // MFLOP of a tile on every compute unit
+  const int64_t full = tiles / slots, left = tiles - full * slots;
+  double us = full * work * t.resident / t.all;
+  const int64_t per = (left + cus - 1) / cus;
+  if (per) us += work * per / (per == 1 || t.resident == 1 ? t.one : t.one + (t.all - t.one) * (per - 1) / (t.resident - 1));
+  return us;
+}
+
+// A x B^T for operands in planes.  terms: of A; a.bd non-null: B is one plane of integers with scales, else terms_b planes.
+// Returns the estimated microseconds instead when `estimate` is set.
+static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *estimate) {
+  const int cus = state().compute_units;
+  const bool q = a.bd != nullptr;
+  static const PlaneTile plane[] = {{64, 64, 2, 190, 267}, {128, 64, 3, 205, 320}, {128, 128, 2, 300, 345}, {128, 128, 2, 258, 371}, {256, 256, 1, 366, 366}};
+  static const PlaneTile plane6[] = {{64, 64, 3, 110, 160}, {128, 64, 2, 110, 170}, {128, 256, 1, 205, 205}};
+  static const PlaneTile ints[] = {{64, 64, 2, 190, 267}, {128, 64, 3, 205, 330}, {128, 128, 2, 320, 360}, {128, 128, 2, 280, 422}};
+  const PlaneTile *tiles = q ? ints : terms == 3 ? plane6 : plane;
+  const int n = q ? 4 : terms == 3 ? 3 : 5;
+  int pick = 0;
+  double us = 1e30;
+  for (int i = 0; i < n; i++) {
+    const double t = plane_tile_us(tiles[i], a, cus);
+    if (t < us) us = t, pick = i;
+  }
+  if (estimate) {
+    *estimate = q ? us * terms / 2.0 + 4.0 : terms == 1 ? us * 0.42 + 10.0 : us + 4.0;
+    return 0;
+  }
+#define T(NPA, SRC, NPB, MB, NB, WM, WN) return planes_launch<NPA, SRC, NPB, MB, NB, WM, WN, 2>(a)
+#define TILES(NPA)                                  \
+  switch (pick) {                                   \
+    case 0: T(NPA, PL_PLANES, NPA, 1, 1, 2, 2);     \
+    case 1: T(NPA, PL_PLANES, NPA, 2, 1, 2, 2);     \
+    case 2: T(NPA, PL_PLANES, NPA, 2, 1, 2, 4);     \
+    case 3: T(NPA, PL_PLANES, NPA, 2, 2, 2, 2);     \
+    case 4: T(NPA, PL_PLANES, NPA, 4, 2, 2, 4);     \
+  }
+#define QTILES(NPA)                                 \
+  switch (pick) {                                   \
+    case 0: T(NPA, PL_INT, 1, 1, 1, 2, 2);          \
+    case 1: T(NPA, PL_INT, 1, 2, 1, 2, 2);          \
+    case 2: T(NPA, PL_INT, 1, 1, 2, 4, 2);          \
+    case 3: T(NPA, PL_INT, 1, 2, 2, 2, 2);          \
+  }
+  if (q) {
+    if (terms == 3) QTILES(3)
+    else if (terms == 2) QTILES(2)
+    else QTILES(1)
+  } else if (terms == 3) {
+    switch (pick) {
+      case 0: T(3, PL_PLANES, 3, 1, 1, 2, 2);
+      case 1: T(3, PL_PLANES, 3, 2, 1, 2, 2);
+      case 2: T(3, PL_PLANES, 3, 2, 2, 2, 4);
+    }
+  } else if (terms == 2) {
+    TILES(2)
+  } else {
+    TILES(1)
+  }
+#undef T
+#undef QTILES
+#undef TILES
+  return fail(CTHIP_E_STATE, "gemm planes: no tile (%d terms)", terms);
+}
+
+template <typename T>
+static int planes_rows(unsigned char *out, const T *x, int64_t rows, int K, int64_t ld, int terms) {
+  const int kbp = (K + 31) / 32;
+  const int64_t blocks = (rows * kbp * 4 + 255) / 256;
+  if (blocks > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "gemm planes: operand too large");
+  const bool vec = K % 8 == 0 && ld % 8 == 0 && (uintptr_t)x % 16 == 0;
+#define PR(NP)                                                                                                                             \
+  do {                                                                                                                                     \
+    if (vec) hipLaunchKernelGGL((k_planes_rows<NP, T, true>), dim3((unsigned)blocks), dim3(256), 0, state().stream, (uint4 *)out, x, rows, K, ld, kbp); \
+    else hipLaunchKernelGGL((k_planes_rows<NP, T, false>), dim3((unsigned)blocks), dim3(256), 0, state().stream, (uint4 *)out, x, rows, K, ld, kbp);    \
+  } while (0)
+  if (terms == 3) PR(3);
+  else if (terms == 2) PR(2);
+  else PR(1);
+#undef PR
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+
+static void planes_operands(PlaneGemmArgs &a, int K, int terms, int terms_b) {
+  a.nkb = (K + 31) / 32;
+  a.apitch = a.nkb * 64 * terms;
+  a.bpitch = a.nkb * 64 * terms_b;
+}
+static int plane_terms(int precision) { return precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1; }
+
+// Whether a product (M, N, K) is faster through planes: two passes over the operands (about 4.2 TB/s; none for operands that
+// lie in planes already) and a denser GEMM, against `other` microseconds.
+static bool planes_pay(int M, int N, int K, int terms, int terms_b, bool ints, double pass_bytes, double other) {
+  if ((int64_t)((K + 31) / 32) * 64 * 3 * 256 >= (1ll << 31)) return false;  // 32-bit offsets within a tile's rows
+  PlaneGemmArgs a = {};
+  a.M = M, a.N = N;
+  planes_operands(a, K, terms, terms_b);
+  static const unsigned short dummy = 0;
+  a.bd = ints ? &dummy : nullptr;
+  double us = 0;
+  planes_gemm(a, terms, terms_b, &us);
+  us += pass_bytes > 0 ? pass_bytes / 4.2e6 + 6.0 : 0.0;
+  return us < other;
+}
+
+// C = act(A . B + bias) + residual with B (K, N) row-major.  *done stays false, and the caller takes the other path, where the
+// results do not lie on 16 bytes or there is no memory for the terms.
+int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N, int K, int act, const float *bias, const float *residual, int precision,
+                         bool *done) {
+  if (N % 4 == 0 && (((uintptr_t)C | (uintptr_t)bias | (uintptr_t)residual) & 15)) return 0;
+  const int terms = plane_terms(precision);
+  PlaneGemmArgs a = {};
+  a.C = C;
+  a.M = M, a.N = N;
+  a.act = act;
+  a.bias = bias, a.residual = residual;
+  planes_operands(a, K, terms, terms);
+  unsigned char *pa = nullptr;
+  const size_t abytes = (size_t)M * a.apitch, bbytes = (size_t)N * a.bpitch;
+  int rc = alloc_scratch((void **)&pa, abytes + bbytes + 256);  // fully written by the two passes
+  if (rc) return 0;
+  *done = true;
+  unsigned char *pb = pa + (abytes + 255) / 256 * 256;
+  rc = planes_rows<float>(pa, A, M, K, K, terms);
+  if (!rc) {
+    const dim3 grid((N + 63) / 64, (K + 63) / 64);
+    const bool vec = N % 4 == 0 && (uintptr_t)B % 16 == 0;
+#define PC(NP)                                                                                                             \
+  do {                                                                                                                     \
+    if (vec) hipLaunchKernelGGL((k_planes_cols<NP, true>), grid, dim3(256), 0, state().stream, (uint4 *)pb, B, K, N, a.nkb); \
+    else hipLaunchKernelGGL((k_planes_cols<NP, false>), grid, dim3(256), 0, state().stream, (uint4 *)pb, B, K, N, a.nkb);    \
+  } while (0)
+    if (terms == 3) PC(3);
+    else if (terms == 2) PC(2);
+    else PC(1);
+#undef PC
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = fail((int)e, "gemm planes: launch -> %s", hipGetErrorString(e));
+  }
+  a.A = pa, a.B = pb;
+  if (!rc) rc = planes_gemm(a, terms, terms, nullptr);
+  const int rf = cthip_free(pa);  // stream-ordered: handed out again only to later work on this stream
+  return rc ? rc : rf;
+}
+// What the same product takes with its operands converted per 64 x 64 tile (launch_gemm): one workgroup per compute unit at a
+// time, 8 / 12.5 / 17.5 us per 1000 k at one / two / three terms, 29 where rows are not whole 16-byte pieces, short grids
+// split over K.  Within 15 % of the measured times from 500^3 to 4096^3.
+static double tiles64_us(int M, int N, int K, int terms, bool aligned) {
+  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64), cus = state().compute_units;
+  int64_t ks = (tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles;
+  ks = ks < K / 192 ? ks : K / 192;
+  ks = ks < 1 ? 1 : ks > 16 ? 16 : ks;
+  const double c = !aligned ? 29.0 : terms == 3 ? 17.5 : terms == 2 ? 12.5 : 8.0;
+  return 2.0 + (ks > 1 ? 5.0 : 0.0) + (double)((tiles * ks + cus - 1) / cus) * (1.0 + c * K / ks * 1e-3);
+}
+bool matmul_planes_pay(int M, int N, int K, int precision) {
+  if (precision == GEMM_FP32 || M < 64 || N < 64 || K < 64) return false;
+  const int terms = plane_terms(precision);
+  return planes_pay(M, N, K, terms, terms, false, ((double)M + N) * K * (4 + 2 * terms), tiles64_us(M, N, K, terms, K % 4 == 0 && N % 4 == 0));
+}
+
+}  // namespace cthip

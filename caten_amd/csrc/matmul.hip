@@ -1343,6 +1343,11 @@ int matmul_routed(float *C, const float *A, const float *B, int M, int N, int K,
     a.wtype = CTHIP_F32;
     return launch_gemm(a, B_WMAT, GEMM_BF16X6, nullptr, 0, nullptr);
   }
+  if (matmul_planes_pay(M, N, K, GEMM_BF16X6)) {
+    bool done = false;
+    const int rc = launch_matmul_planes(C, A, B, M, N, K, act, bias, residual, GEMM_BF16X6, &done);
+    if (done) return rc;
+  }
   a.B = B;
   return launch_gemm(a, B_ROWMAJOR, GEMM_BF16X6, nullptr, 0, nullptr);
 }
@@ -1365,6 +1370,11 @@ static int matmul_entry(float *C, const float *A, const float *B, int M, int N, 
   a.N = N;
   a.K = K;
   a.act = act;
+  if (!noalloc && matmul_planes_pay(M, N, K, precision)) {
+    bool done = false;
+    const int rc = launch_matmul_planes(C, A, B, M, N, K, act, nullptr, nullptr, precision, &done);
+    if (done) return rc;
+  }
   if (!noalloc) return launch_gemm(a, B_ROWMAJOR, precision, nullptr, 0, nullptr);
   float *ws = g_scratch_ptr[state().device];
   if (!ws) return fail(CTHIP_E_STATE, "cthip_matmul_noalloc: no scratch address for device %d", state().device);

@@ -4,7 +4,7 @@
 
 namespace cthip {
 
-enum { PL_PLANES = 0, PL_Q8 = 1, PL_Q4 = 2, PL_INT = 3 };
+enum { PL_PLANES = 0, PL_INT = 1 };
 
 struct PlaneGemmArgs {
   float *C;
@@ -104,13 +104,6 @@ __device__ __forceinline__ v8bf bf_of_q8(unsigned a, unsigned b) {
   return __builtin_bit_cast(v8bf, make_uint4(pack_int_bf16(sbyte0_f32(a), sbyte1_f32(a)), pack_int_bf16(sbyte2_f32(a), sbyte3_f32(a)),
                                              pack_int_bf16(sbyte0_f32(b), sbyte1_f32(b)), pack_int_bf16(sbyte2_f32(b), sbyte3_f32(b))));
 }
-// 8 nibbles (one per byte of a and b, 0..15) -> nibble - 8 as bf16, exact
-__device__ __forceinline__ v8bf bf_of_q4(unsigned a, unsigned b) {
-  a = (a + 0x78787878u) ^ 0x80808080u;  // per byte: nibble - 8 as int8 (no carry leaves a byte)
-  b = (b + 0x78787878u) ^ 0x80808080u;
-  return bf_of_q8(a, b);
-}
-
 // columns col .. col + 3 of one row of a finished tile: bias, activation, residual, and where they go
 __device__ __forceinline__ void plane_gemm_store(const PlaneGemmArgs &a, int row, int col, float4 v4) {
   const int N = a.N;
