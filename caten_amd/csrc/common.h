@@ -86,6 +86,9 @@ struct WMat {
   // valid for exactly these gamma / beta / bias vectors
   const float *fold_g = nullptr, *fold_b = nullptr, *fold_bias = nullptr;
   float *fold_s = nullptr, *fold_c = nullptr;
+  // the matrix as bf16 terms, made by the first Linear over many rows that wants them (gemm_planes.hip)
+  void *planes = nullptr;
+  int64_t planes_bytes = 0;
 };
 // gfx950: 256 MB of Infinity Cache in front of HBM
 static const int64_t kInfinityCacheBytes = 256ll << 20;
@@ -256,6 +259,15 @@ bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, in
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route = nullptr);
 // matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
+// A Linear over many rows through the same kernel: x as fp32 rows or already as planes of plane_terms(precision) terms, the
+// result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, double extra_us = 0.0);
+bool linear_planes_ready(const WMat *w, int m, int precision, double extra_us);  // x in planes certainly runs
+int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
+                         int precision, const GemmRoute *route, unsigned char *planes_out, bool *done);
+bool rows_planes_supported(int K);
+int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps);
+void wmat_drop_planes(WMat *w);
 bool matmul_planes_pay(int M, int N, int K, int precision);
 int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N, int K, int act, const float *bias, const float *residual, int precision,
                          bool *done);

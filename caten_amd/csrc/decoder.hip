@@ -911,7 +911,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   int rc = 0;
   float *X = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *Hb = nullptr, *G = nullptr, *KF = nullptr, *VF = nullptr;
   int *ids_dev = nullptr;
-  AttnSplit split = {1, nullptr, nullptr};
+  AttnSplit split = {1, nullptr, nullptr}, last_split = {1, nullptr, nullptr};
   std::vector<void *> tmp;
   auto alloc = [&](void **p, size_t bytes) {
     int r = alloc_scratch(p, bytes);  // every temporary below is fully written before it is read
@@ -933,10 +933,13 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     TRY(alloc((void **)&KF, sizeof(float) * (size_t)(n + s) * KD));
     TRY(alloc((void **)&VF, sizeof(float) * (size_t)(n + s) * KD));
   }
-  if (s <= kAttnCachedRows && n + s >= 512 && d->att_split.ranges > 1) {  // few rows over a long context: keys shared as in a decode step
-    split.ranges = d->att_split.ranges / s < 2 ? 2 : d->att_split.ranges / s;
-    split.count = d->att_split.count;
-    TRY(alloc((void **)&split.part, sizeof(float) * (size_t)s * c.n_heads * split.ranges * (Dh + 2)));
+  if (n + s >= 512 && d->att_split.ranges > 1) {  // few rows over a long context: keys shared as in a decode step
+    last_split = d->att_split;
+    if (s <= kAttnCachedRows) {
+      split.ranges = d->att_split.ranges / s < 2 ? 2 : d->att_split.ranges / s;
+      split.count = d->att_split.count;
+      TRY(alloc((void **)&split.part, sizeof(float) * (size_t)s * c.n_heads * split.ranges * (Dh + 2)));
+    }
   }
   TRY(alloc((void **)&ids_dev, sizeof(int) * (size_t)s));
   TRY(cthip_h2d(ids_dev, ids, sizeof(int) * (size_t)s));
@@ -946,78 +949,110 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   }
   TRY(launch_embedding(X, d->wte, nullptr, ids_dev, s, V, D, gpt2 ? d->wpe : nullptr, d->tokpos + 1, c.max_seq));
   {
+    // Rows a layer works on: all of them, but for the last layer only the last one once its keys and values are stored (no
+    // other row of its output is read).
+    int R = s;
+    float *Xr = X;
     // A row-split Linear (attention projection, second MLP Linear) whose reduction axis was shared among several
     // workgroups per tile leaves partial tiles; what follows it is the residual add and the next norm, so one pass
     // over the rows does all three (launch_reduce_norm) instead of a reduction launch and a norm launch.
-    auto norm = [&](float *y, const float *x, const float *g, const float *b) {
-      return gpt2 ? cthip_layernorm(y, x, g, b, c.eps, s, D) : cthip_rmsnorm(y, x, g, c.eps, s, D);
+    // Many rows: a Linear takes its input as two bf16 terms (gemm_planes.hip) and what produces that input writes it so;
+    // a row of terms is as long as the fp32 row whose buffer it takes.  (A session with a quantised cache keeps the
+    // order of summation of the tiles: a rounding step of a cached value is a hundred times what a sum is off by.)
+    const bool planes = !d->kvq && prec == GEMM_BF16X3_DEFAULT && s >= 64 && rows_planes_supported(D) && F % 32 == 0;
+    // (before: the Linear in front of the norm that feeds w.  Its split reduction goes into that norm's launch where the norm
+    // writes fp32 rows: 7 us over two launches)
+    auto in_planes = [&](const WMat *w, const WMat *before) {
+      return planes && w && linear_planes_ready(w, R, prec, before && reduce_norm_supported(D, 1) && !linear_planes_pays(before, R, prec, false) ? 7.0 : 0.0);
     };
-    // X += W.in + bias, then XN = norm(X) with (g, b); g == nullptr: no norm follows (after the last layer)
-    auto linear_residual_norm = [&](const WMat *w, const float *in, const float *bias, const float *g, const float *b) {
+    // y = norm(x), as terms where the Linear behind it takes them
+    auto norm = [&](float *y, const float *x, const float *g, const float *b, bool terms) {
+      if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps);
+      return gpt2 ? cthip_layernorm(y, x, g, b, c.eps, R, D) : cthip_rmsnorm(y, x, g, c.eps, R, D);
+    };
+    // y = W.in + ..., in and y as terms where in_terms / out_terms
+    auto linear = [&](float *y, const WMat *w, const float *in, bool in_terms, const float *bias, const float *residual, int act, const GemmRoute *route,
+                      bool out_terms, GemmDeferred *defer = nullptr) {
+      if (in_terms || (planes && linear_planes_pays(w, R, prec, false))) {
+        bool taken = false;
+        const int r = launch_linear_planes(out_terms ? nullptr : y, w, in_terms ? nullptr : in, in_terms ? (const unsigned char *)in : nullptr, R, bias,
+                                           residual, act, prec, route, out_terms ? (unsigned char *)y : nullptr, &taken);
+        if (taken) return r;
+        if (in_terms || out_terms) return fail(CTHIP_E_STATE, "prompt: a Linear of %lld x %lld over %d rows cannot take its input as terms", (long long)w->rows, (long long)w->cols, R);
+      }
+      return prompt_linear(y, w, in, R, bias, residual, act, prec, defer, route);
+    };
+    // Xr += W.in + bias, then XN = norm(Xr) with (g, b), as terms or not; g == nullptr: no norm follows (after the last layer)
+    auto linear_residual_norm = [&](const WMat *w, const float *in, bool in_terms, const float *bias, const float *g, const float *b, bool out_terms) {
       GemmDeferred df;
-      const bool fuse = g != nullptr && reduce_norm_supported(D, 1);
-      int r = prompt_linear(X, w, in, s, bias, X, CTHIP_ACT_NONE, prec, fuse ? &df : nullptr);
+      const bool fuse = g != nullptr && reduce_norm_supported(D, 1) && !out_terms;
+      int r = linear(Xr, w, in, in_terms, bias, Xr, CTHIP_ACT_NONE, nullptr, false, fuse ? &df : nullptr);
       if (r) return r;
       if (df.ws) {
         if (reduce_norm_supported(D, df.ksplit)) {
-          r = launch_reduce_norm(XN, X, df.ws, df.ksplit, (int64_t)s * D, bias, X, g, b, c.eps, s, D, !gpt2);
+          r = launch_reduce_norm(XN, Xr, df.ws, df.ksplit, (int64_t)R * D, bias, Xr, g, b, c.eps, R, D, !gpt2);
         } else {  // too many shares of too wide a row to hold at once: reduce, then normalise
-          r = launch_splitk_reduce(X, df.ws, df.ksplit, s, D, bias, X);
-          if (!r) r = norm(XN, X, g, b);
+          r = launch_splitk_reduce(Xr, df.ws, df.ksplit, R, D, bias, Xr);
+          if (!r) r = norm(XN, Xr, g, b, out_terms);
         }
         const int r2 = cthip_free(df.ws);  // stream-ordered: reused only by later work on this stream
         return r ? r : r2;
       }
-      return g ? norm(XN, X, g, b) : 0;
+      return g ? norm(XN, Xr, g, b, out_terms) : 0;
     };
-    TRY(norm(XN, X, d->layers[0].ln1_g, d->layers[0].ln1_b));
+    bool xt = in_planes(d->layers[0].attn, nullptr);
+    TRY(norm(XN, X, d->layers[0].ln1_g, d->layers[0].ln1_b, xt));
     for (int l = 0; l < c.n_layers; l++) {
       Layer &L = d->layers[l];
+      const bool last = l + 1 == c.n_layers;
+      const float *K = L.k_cache, *V = L.v_cache;  // what attention reads
       if (d->kvq) {
         // attention of a prompt batch runs on fp32 rows: the cached rows [0, n) are widened into a temporary, the
         // batch's rows [n, n + s) join them (rotated where the model rotates) and are quantised into the cache
         TRY(launch_kvq_dequant(KF, L.kq, L.kdq, n, KD));
         TRY(launch_kvq_dequant(VF, L.vq, L.vdq, n, KD));
-        TRY(prompt_linear(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
+        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, false));
         TRY(launch_qkv_split(Q, KF, VF, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
         TRY(launch_kvq_append(L.kq, L.kdq, KF + (int64_t)n * KD, KD, s, n, nullptr, KD));
         TRY(launch_kvq_append(L.vq, L.vdq, VF + (int64_t)n * KD, KD, s, n, nullptr, KD));
-        TRY(launch_attn(ATT, Q, KF, VF, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, &split));
+        K = KF, V = VF;
       } else if (d->kvp) {
         // attention of a prompt batch runs on dense rows: the cached rows [0, n) are gathered out of their pages, the
         // batch's rows [n, n + s) join them (rotated where the model rotates) and are copied into their pages
         TRY(launch_kvp_gather(KF, L.k_pages, n, KD));
         TRY(launch_kvp_gather(VF, L.v_pages, n, KD));
-        TRY(prompt_linear(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
+        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, false));
         TRY(launch_qkv_split(Q, KF, VF, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
         TRY(launch_kvp_append(L.k_pages, L.v_pages, KF + (int64_t)n * KD, VF + (int64_t)n * KD, KD, s, n, nullptr, KD));
-        TRY(launch_attn(ATT, Q, KF, VF, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, &split));
+        K = KF, V = VF;
       } else {
       if (gpt2 && D % 128 == 0 && KD % 128 == 0) {
         // no rotation: the thirds of the fused projection go straight to the query rows and the cache rows
         const GemmRoute rt = {{Q, L.k_cache + (int64_t)n * KD, L.v_cache + (int64_t)n * KD}, {0, D, D + KD}, {D, KD, KD}};
-        TRY(prompt_linear(nullptr, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec, nullptr, &rt));
+        TRY(linear(nullptr, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, &rt, false));
       } else {
-        TRY(prompt_linear(QKV, L.attn, XN, s, L.attn_b, nullptr, CTHIP_ACT_NONE, prec));
+        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, false));
         TRY(launch_qkv_split(Q, L.k_cache, L.v_cache, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
       }
-      TRY(launch_attn(ATT, Q, L.k_cache, L.v_cache, s, n, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, &split));
       }
-      TRY(linear_residual_norm(L.proj, ATT, L.proj_b, L.ln2_g, L.ln2_b));
+      if (last) R = 1, Xr = X + (int64_t)(s - 1) * D;
+      TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
+      const bool ft = in_planes(L.fc, L.proj), gt = ft && (gpt2 || L.fc_pairs) && in_planes(L.fc2, nullptr);
+      TRY(linear_residual_norm(L.proj, ATT, false, L.proj_b, L.ln2_g, L.ln2_b, ft));
       const float *hin = Hb;
       if (!gpt2 && L.fc_pairs && (2 * F) % 4 == 0) {  // SwiGLU in the epilogue of the gate|up launch
-        TRY(prompt_linear(G, L.fc, XN, s, L.fc_b, nullptr, kActSwigluPairs, prec));
+        TRY(linear(G, L.fc, XN, ft, L.fc_b, nullptr, kActSwigluPairs, nullptr, gt));
         hin = G;
       } else {
-        TRY(prompt_linear(Hb, L.fc, XN, s, L.fc_b, nullptr, gpt2 ? CTHIP_ACT_GELU : CTHIP_ACT_NONE, prec));
+        TRY(linear(Hb, L.fc, XN, ft, L.fc_b, nullptr, gpt2 ? CTHIP_ACT_GELU : CTHIP_ACT_NONE, nullptr, gt));
         if (!gpt2) {
-          if (L.fc_pairs) TRY(launch_swiglu_pairs(G, Hb, (int64_t)s * F));
-          else TRY(launch_prologue(G, Hb, F, CTHIP_PRO_SWIGLU, nullptr, nullptr, 0.0f, 2 * (int64_t)F, s));
+          if (L.fc_pairs) TRY(launch_swiglu_pairs(G, Hb, (int64_t)R * F));
+          else TRY(launch_prologue(G, Hb, F, CTHIP_PRO_SWIGLU, nullptr, nullptr, 0.0f, 2 * (int64_t)F, R));
           hin = G;
         }
       }
-      const bool last = l + 1 == c.n_layers;
-      TRY(linear_residual_norm(L.fc2, hin, L.fc2_b, last ? nullptr : d->layers[l + 1].ln1_g, last ? nullptr : d->layers[l + 1].ln1_b));
+      xt = !last && in_planes(d->layers[l + 1].attn, L.fc2);
+      TRY(linear_residual_norm(L.fc2, hin, gt, L.fc2_b, last ? nullptr : d->layers[l + 1].ln1_g, last ? nullptr : d->layers[l + 1].ln1_b, xt));
     }
   }
   // the last row continues through the decode-step head

@@ -10,6 +10,8 @@
 // Layout of a plane operand: row-major, a row is a sequence of blocks of 32 consecutive k, a block is NP runs of 32
 // bf16 (term 0 = bf16(x), term p = bf16 of what terms 0..p-1 miss).  A K-step of a row is one contiguous piece of NP * 64
 // bytes: whole cache lines for NP = 2.
+#include <mutex>
+
 #include "common.h"
 #include "planes.h"
 
@@ -28,8 +30,11 @@ __device__ __forceinline__ int swz(int r) {
 //
 // What bounds it: the matrix cores ask LDS for an operand per instruction and block edge, so a wavefront's piece wants to be
 // large (64 x 64: 16 reads for 24 instructions at two terms); two workgroups of four wavefronts per compute unit fill each
-// other's waits.  4096^3, two terms: 371 TFLOP/s of results = 1.1 PFLOP/s of matrix instructions (the library's bf16 product
-// of this size reaches 1.2 - 1.5 on the card), against 180 with the operands converted per tile.
+// other's waits (reading a step's operands under the step before it instead, two sets of registers, measured the same or
+// slower; so did deeper rings than the launcher's).  4096^3, two terms: 310 us without the passes in front = 440 TFLOP/s of
+// results, 1.3 PFLOP/s of matrix instructions (the library's bf16 product reaches 1.2 - 1.5 on the card), against 180 with
+// the operands converted per tile.  Integers need two products instead of three but 16 multiply-adds per lane and block for
+// the scales: 1900 x 11264 x 2048 240 us (two per tile before: 340), 1900 x 2048 x 5632 128 us (149).
 template <int NPA, int SRC, int NPB, int MB, int NB, int WM, int WN, int NBUF>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN;
@@ -44,10 +49,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  if (local >= a.rm * a.rn) return;
-  const int mi = (xcd % a.rx) * a.rm + local % a.rm, ni = (xcd / a.rx) * a.rn + local / a.rm;
-  if (mi >= a.tm || ni >= a.tn) return;  // the regions overhang a grid they do not divide
+  // tiles in bands of `band` rows of tiles, column by column within a band; each XCD takes an equal run of that order
+  const int tile = (blockIdx.x & 7) * a.chunk + (blockIdx.x >> 3);
+  if (tile >= a.tm * a.tn) return;
+  const int b0 = tile / (a.band * a.tn), inb = tile - b0 * a.band * a.tn, height = min(a.band, a.tm - b0 * a.band);
+  const int mi = b0 * a.band + inb % height, ni = inb / height;
   const int m0 = mi * BM, n0 = ni * BN;
   const int kb0 = blockIdx.y * a.kper, kb1 = min(a.nkb, kb0 + a.kper);  // this workgroup's blocks of 32 k
   const int nsteps = kb1 - kb0;
@@ -94,6 +100,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
 
   const int half = lane >> 5, col = lane & 31;
   // k of the matrix instructions of a block: slice s, lane half h take k = 16 h + 8 s .. +7 (the same for A and B)
+  v16f tmp[2][SRC == PL_INT ? MB : 1] = {};  // PL_INT: partial sums of a block of 32 k, unscaled
+  float dlast = 0.0f;
   auto mul = [&](int buf) __attribute__((always_inline)) {
     const unsigned char *At = smem + buf * BUF, *Bt = At + ABYTES;
     const int ra = 32 * MB * wm + col, rb = 32 * NB * wn + col;
@@ -137,28 +145,41 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int b = 0; b < NB; b++) asm("" : "+v"(d[b]));  // as a float: a multiply-add that converts its fp16 operand runs at half rate
-      // the partial sums of column block b - 1 are scaled under the matrix instructions of column block b
-      v16f tmp[2][MB];
+      // The partial sums of one column block are scaled under the matrix instructions of the next one (of the next step's
+      // first one for the last), a few multiply-adds behind each, which run while it occupies the matrix core.  An odd NB
+      // carries nothing into the next step: its buffers would change places.
 #pragma unroll
-      for (int b = 0; b <= NB; b++) {
-        if (b < NB) {
+      for (int b = 0; b < NB; b++) {
+        const int pb = (b + NB - 1) % NB;
+        const float dp = b ? d[b - 1] : dlast;
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) tmp[b & 1][i][r] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+          for (int p = NPA - 1; p >= 0; p--)
+#pragma unroll
+            for (int i = 0; i < MB; i++) tmp[b & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s][i][p], bf[s][b][0], tmp[b & 1][i], 0, 0, 0);
+        if (b > 0 || NB % 2 == 0)
 #pragma unroll
           for (int i = 0; i < MB; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) tmp[b & 1][i][r] = 0.0f;
+            for (int r = 0; r < 16; r++) acc[i][pb][r] = fmaf(dp, tmp[(b & 1) ^ 1][i][r], acc[i][pb][r]);
 #pragma unroll
-          for (int s = 0; s < 2; s++)
-#pragma unroll
-            for (int p = NPA - 1; p >= 0; p--)
-#pragma unroll
-              for (int i = 0; i < MB; i++) tmp[b & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s][i][p], bf[s][b][0], tmp[b & 1][i], 0, 0, 0);
+        for (int q = 0; q < 2 * NPA * MB; q++) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 8 / NPA, 0);
         }
-        if (b > 0)
-#pragma unroll
-          for (int i = 0; i < MB; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][b - 1][r] = fmaf(d[b - 1], tmp[(b - 1) & 1][i][r], acc[i][b - 1][r]);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      dlast = d[NB - 1];
+      if (NB % 2)
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[i][NB - 1][r] = fmaf(dlast, tmp[0][i][r], acc[i][NB - 1][r]);
     }
   };
 
@@ -174,6 +195,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
     }
   }
   wait_barrier<0>();
+  if (SRC == PL_INT && NB % 2 == 0)
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][NB - 1][r] = fmaf(dlast, tmp[1][SRC == PL_INT ? i : 0][r], acc[i][NB - 1][r]);
 
   // ---- acc[i][b][r] is row 8 (r / 4) + 4 half + r % 4, column `col` of its block.  A wavefront turns its blocks around
   // in a piece of LDS of its own (no barrier) and stores rows of 32 NB columns, 16 bytes per lane.
@@ -299,12 +325,12 @@ static int planes_launch(PlaneGemmArgs a) {
   static_assert(lds <= 160 * 1024, "LDS");
   a.tm = (a.M + BM - 1) / BM;
   a.tn = (a.N + BN - 1) / BN;
-  // one region of tiles per XCD: the split with the fewest tiles per XCD, then the least operand bytes per L2
+  a.chunk = (a.tm * a.tn + 7) / 8;
   double best = -1.0;
-  for (int rx = 1; rx <= 8; rx *= 2) {
-    const int ry = 8 / rx, rm = (a.tm + rx - 1) / rx, rn = (a.tn + ry - 1) / ry;
-    const double score = (double)rm * rn * 1e6 + (double)rm * BM * NPA + (double)rn * BN * NPB;
-    if (best < 0 || score < best) best = score, a.rx = rx, a.rm = rm, a.rn = rn;
+  for (int bands = 1; bands <= 8 && bands <= a.tm; bands++) {  // the band height for the least operand bytes per L2
+    const int h = (a.tm + bands - 1) / bands;
+    const double score = (double)h * BM * NPA + ((double)a.chunk / h + 1.0) * BN * NPB;
+    if (best < 0 || score < best) best = score, a.band = h;
   }
   a.kper = a.nkb;
   auto fn = k_gemm_planes<NPA, SRC, NPB, MB, NB, WM, WN, NBUF>;
@@ -313,7 +339,7 @@ static int planes_launch(PlaneGemmArgs a) {
     CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     big_lds = true;
   }
-  hipLaunchKernelGGL(fn, dim3(8u * a.rm * a.rn), dim3(64 * WM * WN), lds, state().stream, a);
+  hipLaunchKernelGGL(fn, dim3(8u * a.chunk), dim3(64 * WM * WN), lds, state().stream, a);
   CTHIP_LAUNCH_CHECK();
   return 0;
 }
@@ -329,9 +355,13 @@ static double plane_tile_us(const PlaneTile &t, const PlaneGemmArgs &a, int cus)
   const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn), slots = (int64_t)cus * t.resident;
   const double work = 2.0 * t.bm * t.bn * 32.0 * a.nkb * cus * 1e-6;  // MFLOP of a tile on every compute unit
   const int64_t full = tiles / slots, left = tiles - full * slots;
-  double us = full * work * t.resident / t.all;
-  const int64_t per = (left + cus - 1) / cus;
-  if (per) us += work * per / (per == 1 || t.resident == 1 ? t.one : t.one + (t.all - t.one) * (per - 1) / (t.resident - 1));
+  double us = 2.0 + full * work * t.resident / t.all;
+  if (left <= cus) {
+    if (left) us += work / t.one;
+  } else {  // between one tile per compute unit and a full round, steeper at the start: the shared units wait for both
+    const double one = work / t.one, all = work * t.resident / t.all;
+    us += one + (all - one) * (0.4 + 0.6 * (double)(left - cus) / (double)(slots - cus));
+  }
   return us;
 }
 
@@ -342,9 +372,9 @@ static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *e
   const bool q = a.bd != nullptr;
   static const PlaneTile plane[] = {{64, 64, 2, 190, 267}, {128, 64, 3, 205, 320}, {128, 128, 2, 300, 345}, {128, 128, 2, 258, 371}, {256, 256, 1, 366, 366}};
   static const PlaneTile plane6[] = {{64, 64, 3, 110, 160}, {128, 64, 2, 110, 170}, {128, 256, 1, 205, 205}};
-  static const PlaneTile ints[] = {{64, 64, 2, 190, 267}, {128, 64, 3, 205, 330}, {128, 128, 2, 320, 360}, {128, 128, 2, 280, 422}};
+  static const PlaneTile ints[] = {{64, 64, 4, 240, 245}, {128, 128, 2, 370, 400}, {128, 192, 2, 368, 430}};
   const PlaneTile *tiles = q ? ints : terms == 3 ? plane6 : plane;
-  const int n = q ? 4 : terms == 3 ? 3 : 5;
+  const int n = q || terms == 3 ? 3 : 5;
   int pick = 0;
   double us = 1e30;
   for (int i = 0; i < n; i++) {
@@ -352,10 +382,11 @@ static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *e
     if (t < us) us = t, pick = i;
   }
   if (estimate) {
-    *estimate = q ? us * terms / 2.0 + 4.0 : terms == 1 ? us * 0.42 + 10.0 : us + 4.0;
+    *estimate = q ? us * terms / 2.0 + 4.0 : terms == 1 ? us * 0.42 + 10.0 : us + 2.0;
     return 0;
   }
 #define T(NPA, SRC, NPB, MB, NB, WM, WN) return planes_launch<NPA, SRC, NPB, MB, NB, WM, WN, 2>(a)
+#define T3(NPA, SRC, NPB, MB, NB, WM, WN) return planes_launch<NPA, SRC, NPB, MB, NB, WM, WN, 3>(a)
 #define TILES(NPA)                                  \
   switch (pick) {                                   \
     case 0: T(NPA, PL_PLANES, NPA, 1, 1, 2, 2);     \
@@ -364,17 +395,21 @@ static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *e
     case 3: T(NPA, PL_PLANES, NPA, 2, 2, 2, 2);     \
     case 4: T(NPA, PL_PLANES, NPA, 4, 2, 2, 4);     \
   }
-#define QTILES(NPA)                                 \
-  switch (pick) {                                   \
-    case 0: T(NPA, PL_INT, 1, 1, 1, 2, 2);          \
-    case 1: T(NPA, PL_INT, 1, 2, 1, 2, 2);          \
-    case 2: T(NPA, PL_INT, 1, 1, 2, 4, 2);          \
-    case 3: T(NPA, PL_INT, 1, 2, 2, 2, 2);          \
+#define QTILES(NPA)                                    \
+  switch (pick) {                                      \
+    case 0: T3(NPA, PL_INT, 1, 1, 1, 2, 2);            \
+    case 1: T3(NPA, PL_INT, 1, 2, 2, 2, 2);            \
+    case 2: T(NPA, PL_INT, 1, 2, 3, 2, 2);             \
   }
   if (q) {
-    if (terms == 3) QTILES(3)
-    else if (terms == 2) QTILES(2)
+    if (terms == 2) QTILES(2)
     else QTILES(1)
+  } else if (terms == 3 && terms_b == 2) {
+    switch (pick) {
+      case 0: T(3, PL_PLANES, 2, 1, 1, 2, 2);
+      case 1: T(3, PL_PLANES, 2, 2, 1, 2, 2);
+      case 2: T(3, PL_PLANES, 2, 2, 2, 2, 4);
+    }
   } else if (terms == 3) {
     switch (pick) {
       case 0: T(3, PL_PLANES, 3, 1, 1, 2, 2);
@@ -387,6 +422,7 @@ static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *e
     TILES(1)
   }
 #undef T
+#undef T3
 #undef QTILES
 #undef TILES
   return fail(CTHIP_E_STATE, "gemm planes: no tile (%d terms)", terms);
@@ -429,8 +465,8 @@ static bool planes_pay(int M, int N, int K, int terms, int terms_b, bool ints, d
   a.bd = ints ? &dummy : nullptr;
   double us = 0;
   planes_gemm(a, terms, terms_b, &us);
-  us += pass_bytes > 0 ? pass_bytes / 4.2e6 + 6.0 : 0.0;
-  return us < other;
+  us += pass_bytes > 0 ? pass_bytes / 4.2e6 + 5.0 : 0.0;
+  return us * 1.04 < other;
 }
 
 // C = act(A . B + bias) + residual with B (K, N) row-major.  *done stays false, and the caller takes the other path, where the
@@ -474,7 +510,8 @@ int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N,
 }
 // What the same product takes with its operands converted per 64 x 64 tile (launch_gemm): one workgroup per compute unit at a
 // time, 8 / 12.5 / 17.5 us per 1000 k at one / two / three terms, 29 where rows are not whole 16-byte pieces, short grids
-// split over K.  Within 15 % of the measured times from 500^3 to 4096^3.
+// split over K.  Within 15 % of the measured times from 500^3 to 4096^3,
+// and the rule asks for 4 %.
 static double tiles64_us(int M, int N, int K, int terms, bool aligned) {
   const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64), cus = state().compute_units;
   int64_t ks = (tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles;
@@ -487,6 +524,144 @@ bool matmul_planes_pay(int M, int N, int K, int precision) {
   if (precision == GEMM_FP32 || M < 64 || N < 64 || K < 64) return false;
   const int terms = plane_terms(precision);
   return planes_pay(M, N, K, terms, terms, false, ((double)M + N) * K * (4 + 2 * terms), tiles64_us(M, N, K, terms, K % 4 == 0 && N % 4 == 0));
+}
+
+// ---- Linears over many rows ----
+// A weight matrix as planes: one of integers for a quantised matrix (2 bytes per weight), two exact terms for fp16 (4).
+// The first Linear that wants them makes them and they stay with the matrix, up to kWeightPlanesMax for all matrices together
+// (what a 16-bit model of 16e9 weights takes, a ninth of the card); past that, for fp32 matrices and for a single term of
+// an fp16 one they are made again by every call, 3 - 8 bytes of traffic per weight.
+static const int64_t kWeightPlanesMax = 32ll << 30;
+static std::mutex g_weight_planes_mu;
+static int64_t g_weight_planes_bytes = 0;
+
+static bool is_quant(const WMat *w) { return w->type == CTHIP_Q8_0 || w->type == CTHIP_Q4_0; }
+static int weight_terms(const WMat *w, int terms) { return is_quant(w) ? 1 : w->type == CTHIP_F16 && terms > 2 ? 2 : terms; }
+static int64_t weight_plane_bytes(const WMat *w, int terms_b) { return w->rows * ((w->cols + 31) / 32) * 64 * terms_b; }
+static bool weight_planes_stay(const WMat *w, int terms_b) { return is_quant(w) || (w->type == CTHIP_F16 && terms_b == 2); }
+
+static int make_weight_planes(unsigned char *out, const WMat *w, int terms_b) {
+  const int K = (int)w->cols;
+  if (w->type == CTHIP_F16) return planes_rows<_Float16>(out, (const _Float16 *)w->q, w->rows, K, K, terms_b);
+  if (w->type == CTHIP_F32) return planes_rows<float>(out, (const float *)w->q, w->rows, K, K, terms_b);
+  const int64_t n8 = w->rows * K / 8;
+  if ((n8 + 255) / 256 > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "gemm planes: operand too large");
+  const dim3 grid((unsigned)((n8 + 255) / 256));
+  if (w->type == CTHIP_Q4_0) hipLaunchKernelGGL(k_planes_int<true>, grid, dim3(256), 0, state().stream, (uint4 *)out, (const unsigned char *)w->q, n8);
+  else hipLaunchKernelGGL(k_planes_int<false>, grid, dim3(256), 0, state().stream, (uint4 *)out, (const unsigned char *)w->q, n8);
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+// *temp: the caller frees the planes after its launch.  null: no memory for them.
+static const unsigned char *weight_planes(const WMat *w, int terms_b, bool *temp) {
+  std::lock_guard<std::mutex> lk(g_weight_planes_mu);
+  *temp = false;
+  const int64_t bytes = weight_plane_bytes(w, terms_b);
+  const bool stay = weight_planes_stay(w, terms_b);
+  if (stay && w->planes) return (const unsigned char *)w->planes;
+  unsigned char *p = nullptr;
+  if (bytes > kWeightPlanesMax || alloc_scratch((void **)&p, (size_t)bytes)) return nullptr;
+  if (make_weight_planes(p, w, terms_b)) {
+    cthip_free(p);
+    return nullptr;
+  }
+  if (stay && g_weight_planes_bytes + bytes <= kWeightPlanesMax) {
+    WMat *m = const_cast<WMat *>(w);
+    m->planes = p;
+    m->planes_bytes = bytes;
+    g_weight_planes_bytes += bytes;
+  } else {
+    *temp = true;
+  }
+  return p;
+}
+void wmat_drop_planes(WMat *w) {
+  std::lock_guard<std::mutex> lk(g_weight_planes_mu);
+  if (!w->planes) return;
+  cthip_free(w->planes);
+  g_weight_planes_bytes -= w->planes_bytes;
+  w->planes = nullptr;
+}
+
+// What launch_gemm takes: 64 x 128 tiles of a quantised matrix, one workgroup per compute unit.
+static double linear_tiles_us(const WMat *w, int m, int terms) {
+  const int N = (int)w->rows, K = (int)w->cols;
+  if (!is_quant(w)) return tiles64_us(m, N, K, terms, true) * (w->type == CTHIP_F16 ? 0.87 : 1.0);
+  const int64_t tiles = (int64_t)((m + 63) / 64) * ((N + 127) / 128), cus = state().compute_units;
+  int64_t ks = cus / tiles;
+  ks = ks < K / 192 ? ks : K / 192;
+  ks = ks < 1 ? 1 : ks > 16 ? 16 : ks;
+  const double c = terms == 2 ? 13.2 : 10.0;
+  return 2.0 + (ks > 1 ? 5.0 : 0.0) + (double)((tiles * ks + cus - 1) / cus) * (1.0 + c * K / ks * 1e-3);
+}
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, double extra_us) {
+  if (precision == GEMM_FP32 || m < 64 || w->rows < 64 || w->cols < 64 || (!is_quant(w) && w->cols % 16)) return false;
+  // (three terms against integers: registers for one 32-column block less per wavefront, no faster than the tiles)
+  if (is_quant(w) && precision == GEMM_BF16X6) return false;
+  const int terms = plane_terms(precision), terms_b = weight_terms(w, terms);
+  double bytes = 0.0;
+  if (!weight_planes_stay(w, terms_b)) bytes = (double)w->rows * w->cols * (w->type == CTHIP_F16 ? 2.0 : 4.0) + weight_plane_bytes(w, terms_b);
+  if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
+  return planes_pay(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes, linear_tiles_us(w, m, terms) - extra_us);
+}
+// ... and nothing can be in the way of it: the matrix has its planes (made here if need be)
+bool linear_planes_ready(const WMat *w, int m, int precision, double extra_us) {
+  if (!linear_planes_pays(w, m, precision, true, extra_us)) return false;
+  const int terms_b = weight_terms(w, plane_terms(precision));
+  if (!weight_planes_stay(w, terms_b)) return false;
+  bool temp = false;
+  const unsigned char *p = weight_planes(w, terms_b, &temp);
+  if (temp) cthip_free(const_cast<unsigned char *>(p));
+  return p && !temp;
+}
+int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
+                         int precision, const GemmRoute *route, unsigned char *planes_out, bool *done) {
+  const int K = (int)w->cols, terms = plane_terms(precision), terms_b = weight_terms(w, terms);
+  PlaneGemmArgs a = {};
+  a.C = y;
+  a.M = m, a.N = (int)w->rows;
+  a.bias = bias, a.residual = residual;
+  a.act = act;
+  uintptr_t at = (uintptr_t)y | (uintptr_t)bias | (uintptr_t)residual;
+  if (act == kActSwigluPairs) {
+    if (a.N % 4 || residual || route) return 0;
+    a.act = CTHIP_ACT_NONE;
+    a.pairs = 1;
+  }
+  if (route) {
+    for (int i = 0; i < 3; i++)
+      if (route->c0[i] != INT_MAX) at |= (uintptr_t)route->dst[i] | (route->c0[i] % 4 || route->ld[i] % 4 ? 1 : 0);
+    if (route->c0[0] != 0 || residual || a.N % 4) return 0;
+    a.routed = 1;
+    a.route = *route;
+  }
+  if (a.N % 4 == 0 && (at & 15)) return 0;
+  if (planes_out) {
+    const int width = a.pairs ? a.N / 2 : a.N;
+    if (terms != 2 || a.N % 4 || width % 32) return 0;
+    a.planes = (unsigned short *)planes_out;
+    a.pkb = width / 32;
+  }
+  planes_operands(a, K, terms, terms_b);
+  if (is_quant(w)) {
+    a.bd = (const unsigned short *)w->d;
+    a.dpitch = a.nkb;
+  }
+  unsigned char *tmp = nullptr;
+  if (!xplanes && alloc_scratch((void **)&tmp, (size_t)m * a.apitch)) return 0;  // fully written by the pass in front
+  bool temp_b = false;
+  const unsigned char *pb = weight_planes(w, terms_b, &temp_b);
+  if (!pb) {
+    cthip_free(tmp);
+    return 0;
+  }
+  *done = true;
+  int rc = xplanes ? 0 : planes_rows<float>(tmp, x, m, K, K, terms);
+  a.A = xplanes ? xplanes : tmp, a.B = pb;
+  if (!rc) rc = planes_gemm(a, terms, terms_b, nullptr);
+  cthip_free(tmp);  // stream-ordered: handed out again only to later work on this stream
+  if (temp_b) cthip_free(const_cast<unsigned char *>(pb));
+  return rc;
 }
 
 }  // namespace cthip

@@ -653,6 +653,7 @@ int cthip_wmat_destroy(void *wmat) {
   cthip_free(w->d);
   if (w->fold_s) cthip_free(w->fold_s);
   if (w->fold_c) cthip_free(w->fold_c);
+  wmat_drop_planes(w);
   delete w;
   return 0;
 }
@@ -728,7 +729,11 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
       }
       xin = tmp;
     }
-    rc = launch_linear_gemm(y, w, xin, m, bias, residual, act, state().gemm_precision);
+    bool done = false;
+    rc = 0;
+    if (linear_planes_pays(w, m, state().gemm_precision, false))
+      rc = launch_linear_planes(y, w, xin, nullptr, m, bias, residual, act, state().gemm_precision, nullptr, nullptr, &done);
+    if (!done) rc = launch_linear_gemm(y, w, xin, m, bias, residual, act, state().gemm_precision);
     if (tmp) cthip_free(tmp);
     return rc;
   }

@@ -528,6 +528,17 @@ bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, in
   return m <= 16 ? weights >= (quant ? 22e3 : 20e3) : w->type == CTHIP_F16 && weights >= 60e3;
 }
 
+// rows with what a Linear has in front of it as bf16 planes for gemm_planes.hip (x on 16 bytes, K % 32 == 0)
+bool rows_planes_supported(int K) { return K % 32 == 0 && K <= kRowsPlanesMaxK; }
+int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps) {
+  const RowsPlanesArgs pa = {(uint4 *)planes, nullptr, x, K, K, K / 32, g, b, eps};
+  if (pro == CTHIP_PRO_LAYERNORM) rows_planes_launch<CTHIP_PRO_LAYERNORM, 2, false>(pa, m);
+  else if (pro == CTHIP_PRO_RMSNORM) rows_planes_launch<CTHIP_PRO_RMSNORM, 2, false>(pa, m);
+  else rows_planes_launch<CTHIP_PRO_NONE, 2, false>(pa, m);
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+
 // y (m, rows) = act(prologue(x) @ W^T + bias) + residual for a few rows; act may be kActSwigluPairs, route as for
 // launch_linear_gemm.  Call only where linear_rows_pays.
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,

@@ -9,7 +9,7 @@ enum { PL_PLANES = 0, PL_INT = 1 };
 struct PlaneGemmArgs {
   float *C;
   const unsigned char *A, *B;
-  const unsigned short *bd;  // scales of raw quants
+  const unsigned short *bd;  // scales of quants
   int apitch, bpitch;        // bytes between rows
   int dpitch;                // scales between rows
   int M, N, nkb;             // nkb: blocks of 32 k
@@ -17,7 +17,7 @@ struct PlaneGemmArgs {
   const float *bias, *residual;
   int act;
   float *ws;                 // split K: raw partial tiles ws[z][M][N]; null: C is complete
-  int tm, tn, rx, rm, rn;    // tile -> workgroup mapping, one region of tiles per XCD (see GemmArgs)
+  int tm, tn, band, chunk;   // tile -> workgroup mapping
   int pairs;                 // columns (2j, 2j + 1) are (gate, up): C (M, N / 2) gets silu(gate) * up
   int routed;
   GemmRoute route;

@@ -1,5 +1,6 @@
 """Products over operands split into bf16 terms once (csrc/gemm_planes.hip), at sizes where each of its tiles is chosen:
-edges that no tile divides, a last block of k that is part empty, rows that are no multiple of 16 bytes."""
+edges that no tile divides, a last block of k that is part empty, rows that are no multiple of 16 bytes; the Linears and
+prompts that take it."""
 import numpy as np
 import pytest
 
@@ -27,3 +28,45 @@ def test_matmul_planes(ops, m, n, k, precision, tol):
     assert np.all(np.abs(got[rows] - want) <= tol * (np.abs(a[rows]) @ np.abs(b)))
     relu = ops.matmul(a, b, relu=True, precision=precision)
     assert np.array_equal(relu, np.maximum(got, 0.0))
+
+
+@pytest.mark.parametrize("kind,rows,cols,m", [("q8_0", 11270, 2080, 391), ("q8_0", 5001, 2048, 1543), ("q4_0", 11270, 2080, 800), ("q4_0", 4096, 11008, 777),
+                                              ("f16", 4100, 1008, 777), ("f16", 1601, 6400, 1030), ("f32", 6402, 1600, 517)])
+@pytest.mark.parametrize("prologue", [None, "rmsnorm"])
+def test_linear_planes(ops, kind, rows, cols, m, prologue):
+    from caten_amd.llm import Tensor
+    rng = np.random.default_rng(rows + m)
+    w = ops.WeightMatrix(kind, Tensor.from_f32(rng.normal(0, 0.05, (rows, cols)).astype(np.float32), kind).raw, rows, cols)
+    x = rng.normal(0, 1, (m, cols)).astype(np.float32)
+    x[:, 3] *= 100.0
+    g = rng.normal(1, 0.05, cols).astype(np.float32)
+    bias, res = rng.normal(0, 1, rows).astype(np.float32), rng.normal(0, 1, (m, rows)).astype(np.float32)
+    at, rs = np.unique(np.r_[0:40, rows - 40:rows, rng.integers(0, rows, 100)]), np.unique(np.r_[0:9, m - 9:m, rng.integers(0, m, 40)])
+    x64 = x[rs].astype(np.float64)
+    if prologue:
+        x64 = x64 / np.sqrt((x64 * x64).mean(-1, keepdims=True) + 1e-5) * g
+    want = np.maximum(x64 @ w.dequantize()[at].astype(np.float64).T + bias[at], 0.0) + res[rs][:, at]
+    for _ in range(2):  # with the matrix's terms made, and as they are kept
+        got = ops.linear(x, w, bias, res, act="relu", prologue=prologue, **(dict(norm_g=g) if prologue else {}))[np.ix_(rs, at)]
+        assert np.linalg.norm(got - want) < 1e-5 * np.linalg.norm(want)
+    w.free()
+
+
+@pytest.mark.parametrize("arch,kind,rows", [("llama", "q8_0", 1501), ("llama", "q4_0", 1100), ("llama", "f16", 900), ("gpt2", "f16", 777), ("gpt2", "q8_0", 1900)])
+def test_long_prompt_equals_short_pieces(ops, arch, kind, rows):
+    from caten_amd import llm, synth
+    if arch == "llama":
+        cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=1024, n_heads=16, n_kv_heads=4, ffn=5632, n_layers=3, vocab=500, max_seq=2048)
+        model = llm.make_llama(cfg, llm.llama_state_dict(synth.llama_weights(cfg, seed=3), kind))
+    else:
+        cfg = dict(synth.GPT2_CONFIGS["gpt2"], dim=1024, n_heads=16, n_layers=3, vocab=500, max_seq=2048)
+        model = llm.make_gpt2(cfg, llm.gpt2_state_dict(synth.gpt2_weights(cfg, seed=3), kind))
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], rows + 1, seed=3)]
+    got = [model.forward(ids[:rows], rows, 0, return_logits=True), model.forward(ids[rows:], 1, rows, return_logits=True)]
+    for n in range(0, rows, 63):
+        want = [model.forward(ids[n:min(n + 63, rows)], min(63, rows - n), n, return_logits=True)]
+    want.append(model.forward(ids[rows:], 1, rows, return_logits=True))
+    for (t0, l0), (t1, l1) in zip(got, want):
+        assert t0 == t1
+        assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
+    model.close()
