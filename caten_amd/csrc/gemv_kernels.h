@@ -212,6 +212,8 @@ __device__ __forceinline__ void coop_prologue(const GemvArgs &a, const float *__
                                       (v.z - mean) * rstd * gg.z + bb.z, (v.w - mean) * rstd * gg.w + bb.w);
     }
   __syncthreads();
+  if (a.norm_out && blockIdx.x == 0)
+    for (int i = tid; i < n4; i += nthr) ((float4 *)(a.norm_out + (int64_t)blockIdx.y * a.cols))[i] = ((const float4 *)xs)[i];
 }
 
 // Folded norm with a staged input: the workgroup writes gamma * x into LDS once and reduces the
@@ -480,6 +482,7 @@ __device__ __forceinline__ void gemv_ring(const GemvArgs &a, float *xs_lds, floa
           const float4 bt = a.norm_b ? sb[k] : make_float4(0.f, 0.f, 0.f, 0.f);
           ((float4 *)xs_lds)[i] = make_float4((v.x - mu) * rstd * gm.x + bt.x, (v.y - mu) * rstd * gm.y + bt.y,
                                               (v.z - mu) * rstd * gm.z + bt.z, (v.w - mu) * rstd * gm.w + bt.w);
+          if (a.norm_out && blockIdx.x == 0) ((float4 *)(a.norm_out + (int64_t)blockIdx.y * a.cols))[i] = ((const float4 *)xs_lds)[i];
         }
       }
       mu = 0.0f;
@@ -794,6 +797,7 @@ struct GemvVariant {
   gemv_fn fn[2];       // looping launches: [0] cached weights, [1] streamed (non-temporal) weights
   gemv_fn fn_epi[2];   // the same with per-row epilogue operands (bias, residual, fold term) travelling in the ring
   gemv_fn fn_direct[2];  // looping, no epilogue operands, a LayerNorm applied to the staged input
+  gemv_fn fn_direct_epi[2];  // both: fp32 rows behind a LayerNorm whose result is kept; null elsewhere
   gemv_fn fn_small[2]; // one tile per wavefront: latency-bound launches
   gemv_fn fn_pair[2];  // looping, one row per wavefront, (gate, up) row pairs in neighbouring ring slots with SwiGLU as the epilogue; null where the shape has none
 };
@@ -802,10 +806,16 @@ constexpr gemv_fn gemv_pair_fn() {
   if constexpr (G == 64 && PD_OF_T(T, KC) >= 2 && PD_OF_T(T, KC) % 2 == 0) return k_gemv<T, G, KC, PD_OF_T(T, KC), NT, false, false, true>;
   else return nullptr;
 }
+template <int T, int G, int KC, bool NT>
+constexpr gemv_fn gemv_direct_epi_fn() {
+  if constexpr (T == CTHIP_F32 && PD_OF_T(T, KC) > 1) return k_gemv<T, G, KC, PD_OF_T(T, KC), NT, true, true>;
+  else return nullptr;
+}
 #define V(T, G, KC)                                                                           \
   {T, G, KC, {k_gemv<T, G, KC, PD_OF_T(T, KC), false>, k_gemv<T, G, KC, PD_OF_T(T, KC), true>},         \
    {k_gemv<T, G, KC, PD_OF_T(T, KC), false, PD_OF_T(T, KC) != 1>, k_gemv<T, G, KC, PD_OF_T(T, KC), true, PD_OF_T(T, KC) != 1>}, \
    {k_gemv<T, G, KC, PD_OF_T(T, KC), false, false, PD_OF_T(T, KC) != 1>, k_gemv<T, G, KC, PD_OF_T(T, KC), true, false, PD_OF_T(T, KC) != 1>}, \
+   {gemv_direct_epi_fn<T, G, KC, false>(), gemv_direct_epi_fn<T, G, KC, true>()},                         \
    {k_gemv<T, G, KC, 1, false>, k_gemv<T, G, KC, 1, true>},                                              \
    {gemv_pair_fn<T, G, KC, false>(), gemv_pair_fn<T, G, KC, true>()}},
 // defined in gemv_q8.hip, gemv_q4.hip, gemv_f32.hip, gemv_f16.hip

@@ -381,6 +381,10 @@ static bool gemv_prefers_wide(const GemvVariant *v, int type, int64_t rows) {
   const int opt = state().gemv_wide;
   return opt && (!v || heavy || opt >= 2);
 }
+bool gemv_norm_out_ok(const WMat *w) {
+  const GemvVariant *v = pick_variant(w->type, (int)w->cols);
+  return v && !gemv_prefers_wide(v, w->type, w->rows);
+}
 bool gemv_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
   if (rows <= 0 || (rows & 1) || cols <= 0 || cols > 0x7fffffff) return false;
   const GemvVariant *v = pick_variant(type, (int)cols);
@@ -449,6 +453,14 @@ static int launch_variant(const GemvVariant *v, const WMat *w, GemvArgs a, int m
     const bool pair1 = a.pair_swiglu && v->G > 32;
     if (pair1 && (p.kernel != GEMV_K_LOOP || !v->fn_pair[0]))
       return fail(CTHIP_E_UNSUPPORTED, "gemv: the paired SwiGLU epilogue over (%d, %d) needs a looping launch with an even ring and no per-row operands", a.rows, a.cols);
+    // a norm kept for the caller (graph_ops.hip) in front of a few thousand rows: a row per wavefront, every workgroup
+    // normalising for itself, is done before a looping launch has its second tile
+    if (a.norm_out && p.kernel != GEMV_K_SMALL && p.stage && a.rows <= 16 * s.compute_units && v->G == 64) {
+      p.kernel = GEMV_K_SMALL;
+      p.grid_x = (unsigned)(a.rows + 3) / 4;
+      p.block = 256;
+      p.nwaves = (int)p.grid_x * 4;
+    }
     a.stage_x = p.stage ? 1 : 0;
     if (p.unfold) {
       a.fold_s = nullptr;
@@ -460,7 +472,7 @@ static int launch_variant(const GemvVariant *v, const WMat *w, GemvArgs a, int m
     // the looping kernel with per-row operands in its ring dereferences one of them unconditionally
     if (p.kernel == GEMV_K_LOOP_EPI && !a.bias && !a.residual && !a.fold_s)
       return fail(CTHIP_E_STATE, "gemv: a launch with epilogue operands in its ring has none");
-    const gemv_fn fn = pair1 ? v->fn_pair[nt] : p.kernel == GEMV_K_SMALL ? v->fn_small[nt] : p.kernel == GEMV_K_LOOP_EPI ? v->fn_epi[nt]
+    const gemv_fn fn = pair1 ? v->fn_pair[nt] : p.kernel == GEMV_K_SMALL ? v->fn_small[nt] : p.kernel == GEMV_K_LOOP_EPI ? (a.norm_out && !a.fold_s && v->fn_direct_epi[nt] ? v->fn_direct_epi[nt] : v->fn_epi[nt])
                      : p.kernel == GEMV_K_LOOP_DIRECT ? v->fn_direct[nt] : v->fn[nt];
     hipLaunchKernelGGL(fn, dim3(p.grid_x, p.grid_y), dim3(p.block), p.lds, s.stream, a);
     CTHIP_LAUNCH_CHECK();

@@ -44,6 +44,7 @@
 #include <vector>
 
 #include "common.h"
+#include "graph_ops.h"
 
 namespace cthip {
 
@@ -537,7 +538,7 @@ static bool affine_n(const Sx &index, const std::vector<std::string> &idx, std::
   return v == want;
 }
 
-enum RouteKind { R_NONE = 0, R_MATMUL, R_EMBEDDING, R_ARGMAX, R_SOFTMAX, R_LAYERNORM, R_RMSNORM };
+enum RouteKind { R_NONE = 0, R_MATMUL, R_EMBEDDING, R_ARGMAX, R_SOFTMAX, R_LAYERNORM, R_RMSNORM, R_COPY };
 struct Route {
   RouteKind kind = R_NONE;
   int out = -1, a = -1, b = -1, bias = -1;  // argument positions
@@ -569,6 +570,8 @@ struct Program {
   hipFunction_t fn = nullptr;
   // what the matmul route derived from the shape arguments at the last launch: the layers of a model share one program
   // and launch it with the same shapes, so the index expressions are evaluated once per set of values
+  std::vector<char> arg_code;   // per argument: p pointer, f floating point, else the integer type
+  std::vector<int> scalar_pos;  // positions of the integers
   std::vector<long long> memo_key, memo_ext;
   bool memo_ok = false;
   AffineN memo_aff[5];
@@ -778,6 +781,27 @@ static bool match_matmul(const Item &it, Route &r) {
   if (r.out == r.a || r.out == r.b) return false;
   if (!probe_matmul_epilogue(it, st.rhs, acc, r)) return false;
   r.kind = R_MATMUL;
+  return true;
+}
+
+// for ...: for ...: [for ...:] out[..] = in[..]
+static bool match_copy(const Item &it, Route &r) {
+  const std::vector<BpNode> &b = it.body;
+  const int n = (int)b.size(), P = (n - 1) / 2;
+  if (n % 2 == 0 || P < 1 || P > 3) return false;
+  for (int q = 0; q < P; q++) {
+    if (b[q].t != BpNode::FOR || b[n - 1 - q].t != BpNode::ENDFOR || b[q].grid_rank >= 0) return false;
+    const Sx *ub = upper_bound(b[q]);
+    if (!ub || !is_zero(b[q].upfrom)) return false;
+    r.lidx.push_back(b[q].idx);
+    r.lbound.push_back(*ub);
+  }
+  const BpNode &st = b[P];
+  if (st.t != BpNode::EXPR || st.declare || st.writes.size() != 1 || !is_global_aref(it, st.writes[0], r.out) || !is_global_aref(it, st.rhs, r.a)) return false;
+  if (r.out == r.a || it.globals[r.out].type != "output") return false;
+  r.out_idx = st.writes[0].v[2];
+  r.a_idx = st.rhs.v[2];
+  r.kind = R_COPY;
   return true;
 }
 
@@ -1699,21 +1723,33 @@ int launch_embedding(float *out, const float *W, const float *idx_f, const int *
                      const float *W2, const int *pos, int max_pos);
 int launch_embedding_rows(float *out, const float *W, long long first, long long step, int ntok, int vocab, int dim, const float *addend);
 
-static bool launch_route(Program &pg, void **args, const std::map<std::string, long long> &env, int &rc) {
+// The by-value integer arguments of a launch: as numbers at once, under their names when an expression has to be evaluated.
+struct ScalarArgs {
+  const Item &it;
+  const std::vector<int> &pos;  // their argument positions
+  std::vector<long long> val;
+  mutable std::map<std::string, long long> named;
+  const std::map<std::string, long long> &env() const {
+    if (named.empty())
+      for (size_t k = 0; k < pos.size(); k++) named[it.globals[pos[k]].id] = val[k];
+    return named;
+  }
+};
+static bool launch_route(Program &pg, void **args, const ScalarArgs &sc, int &rc) {
   Route &r = pg.route;
   rc = 0;
+  // what the index expressions give is kept with the scalars it was derived from (softmax and the norms: memo_ext = rows, width)
+  const bool memo = pg.memo_ok && sc.val == pg.memo_key;
   auto ptr = [&](int pos) { return *(void **)args[pos]; };
-  auto bound = [&](int q, long long &v) { return eval_int(r.bound[q], env, v) && v >= 0 && v <= 0x7fffffff; };
+  auto bound = [&](int q, long long &v) { return eval_int(r.bound[q], sc.env(), v) && v >= 0 && v <= 0x7fffffff; };
   auto aligned = [](const float *p) { return ((uintptr_t)p % 16) == 0; };
   if (r.kind == R_MATMUL) {
     const int nl = (int)r.lidx.size(), P = nl - 1;  // loops: batch..., i, j, then k
     const int ii = P - 2, jj = P - 1, kk = P;
-    std::vector<long long> key;
-    key.reserve(env.size());
-    for (const auto &kv : env) key.push_back(kv.second);
-    if (!pg.memo_ok || key != pg.memo_key) {
+    if (!memo) {
+      const std::map<std::string, long long> &env = sc.env();
       pg.memo_ok = false;
-      pg.memo_key = key;
+      pg.memo_key = sc.val;
       pg.memo_ext.assign(nl, 0);
       for (int q = 0; q < nl; q++)
         if (!eval_int(r.lbound[q], env, pg.memo_ext[q]) || pg.memo_ext[q] < 0 || pg.memo_ext[q] > 0x7fffffff) return false;
@@ -1757,7 +1793,15 @@ static bool launch_route(Program &pg, void **args, const std::map<std::string, l
       else dense = false;
     }
     if (dense) {
-      rc = matmul_routed(C, A, B, (int)M, (int)N, (int)K, r.act, bias, resid, b_nk);
+      if (b_nk) {
+        GraphOp op = {};
+        op.kind = GraphOp::LINEAR;
+        op.out = C, op.x = A, op.w = B, op.bias = bias, op.resid = resid;
+        op.rows = M, op.cols = (int)N, op.n = (int)K, op.act = r.act;
+        rc = graph_op(op);
+      } else if (!(rc = graph_ops_flush())) {
+        rc = matmul_routed(C, A, B, (int)M, (int)N, (int)K, r.act, bias, resid, false);
+      }
       pg.last_route = b_nk ? "cthip_linear" : "cthip_matmul";
       return true;
     }
@@ -1798,41 +1842,87 @@ static bool launch_route(Program &pg, void **args, const std::map<std::string, l
       }
     }
     if (K == 0 || !bmm_variant(g)) return false;
-    rc = launch_bmm(g);
+    GraphOp op = {};
+    op.kind = GraphOp::BMM;
+    op.bmm = g;
+    rc = graph_op(op);
     pg.last_route = "cthip_bmm";
     return true;
   }
-  if (r.kind == R_EMBEDDING) {
-    long long T, D, V;
-    if (!bound(0, T) || !bound(1, D) || !bound(2, V)) return false;
-    Affine ao, aw, ai;
-    if (!affine_of(r.out_idx, r.idx, 3, env, ao) || !affine_of(r.a_idx, r.idx, 3, env, aw) || !affine_of(r.b_idx, r.idx, 3, env, ai)) return false;
-    if (ao.base || ao.c[0] != D || ao.c[1] != 1 || ao.c[2]) return false;  // out (T, D)
-    if (aw.base || aw.c[0] || aw.c[1] != 1 || aw.c[2] != D) return false;  // W (V, D)
-    Affine av;
-    if (!affine_of(r.bias_idx, r.idx, 3, env, av) || av.base || av.c[0] || av.c[1] || av.c[2] != 1) return false;  // compared with v itself
-    const float *addend = nullptr;
-    if (r.extra[0] >= 0) {  // + other[t, d]
-      Affine ae;
-      if (!affine_of(r.extra_idx[0], r.idx, 3, env, ae) || ae.base || ae.c[0] != D || ae.c[1] != 1 || ae.c[2]) return false;
-      addend = (const float *)ptr(r.extra[0]);
+  if ((r.kind == R_EMBEDDING || r.kind == R_ARGMAX || r.kind == R_RMSNORM) && (rc = graph_ops_flush())) return true;
+  if (r.kind == R_COPY) {
+    if (!graph_ops_collecting()) return false;  // by itself the rendered kernel is as good
+    const int nl = (int)r.lidx.size();
+    if (!memo) {
+      const std::map<std::string, long long> &env = sc.env();
+      pg.memo_ok = false;
+      pg.memo_key = sc.val;
+      pg.memo_ext.assign(nl, 0);
+      for (int q = 0; q < nl; q++)
+        if (!eval_int(r.lbound[q], env, pg.memo_ext[q]) || pg.memo_ext[q] < 0 || pg.memo_ext[q] > 0x7fffffff) return false;
+      if (!affine_n(r.out_idx, r.lidx, env, pg.memo_aff[0]) || !affine_n(r.a_idx, r.lidx, env, pg.memo_aff[1])) return false;
+      pg.memo_ok = true;
     }
+    const AffineN &o = pg.memo_aff[0], &i = pg.memo_aff[1];
+    if (o.base < 0 || i.base < 0) return false;
+    GraphOp op = {};
+    op.kind = GraphOp::COPY;
+    op.copy.out = (float *)ptr(r.out) + o.base;
+    op.copy.in = (const float *)ptr(r.a) + i.base;
+    double count = 1.0;
+    for (int q = 0; q < 3; q++) {
+      const int at = q - (3 - nl);  // loops are the last axes
+      op.copy.ext[q] = at < 0 ? 1 : (int)pg.memo_ext[at];
+      op.copy.os[q] = at < 0 ? 0 : o.c[at];
+      op.copy.is[q] = at < 0 ? 0 : i.c[at];
+      if (op.copy.os[q] < 0 || op.copy.is[q] < 0) return false;
+      count *= op.copy.ext[q];
+    }
+    if (count == 0.0) return true;
+    if (count > 64e6) return false;
+    rc = graph_op(op);
+    pg.last_route = "rendered";  // (the item has no kernel of its own: it is copied along with others)
+    return true;
+  }
+  if (r.kind == R_EMBEDDING) {
+    if (!memo) {  // memo_ext: tokens, width, rows of the table, and for rows by position the first one and the step
+      const std::map<std::string, long long> &env = sc.env();
+      pg.memo_ok = false;
+      long long T, D, V;
+      if (!bound(0, T) || !bound(1, D) || !bound(2, V)) return false;
+      Affine ao, aw, ai;
+      if (!affine_of(r.out_idx, r.idx, 3, env, ao) || !affine_of(r.a_idx, r.idx, 3, env, aw) || !affine_of(r.b_idx, r.idx, 3, env, ai)) return false;
+      if (ao.base || ao.c[0] != D || ao.c[1] != 1 || ao.c[2]) return false;  // out (T, D)
+      if (aw.base || aw.c[0] || aw.c[1] != 1 || aw.c[2] != D) return false;  // W (V, D)
+      Affine av;
+      if (!affine_of(r.bias_idx, r.idx, 3, env, av) || av.base || av.c[0] || av.c[1] || av.c[2] != 1) return false;  // compared with v itself
+      if (r.extra[0] >= 0) {  // + other[t, d]
+        Affine ae;
+        if (!affine_of(r.extra_idx[0], r.idx, 3, env, ae) || ae.base || ae.c[0] != D || ae.c[1] != 1 || ae.c[2]) return false;
+      }
+      if (r.b < 0) {
+        if (ai.c[1] || ai.c[2]) return false;
+      } else if (r.extra[0] >= 0 || ai.base || ai.c[0] != 1 || ai.c[1] || ai.c[2]) {  // idx (T)
+        return false;
+      }
+      pg.memo_key = sc.val;
+      pg.memo_ext = {T, D, V, ai.base, ai.c[0]};
+      pg.memo_ok = true;
+    }
+    const long long T = pg.memo_ext[0], D = pg.memo_ext[1], V = pg.memo_ext[2];
+    if (T == 0 || D == 0) return true;
     if (r.b < 0) {
       // rows first, first + step, ...: token position t selects row (first + step * t)
-      if (ai.c[1] || ai.c[2]) return false;
-      if (T == 0 || D == 0) return true;
-      rc = launch_embedding_rows((float *)ptr(r.out), (const float *)ptr(r.a), ai.base, ai.c[0], (int)T, (int)V, (int)D, addend);
-      pg.last_route = "cthip_embedding";
-      return true;
+      const float *addend = r.extra[0] >= 0 ? (const float *)ptr(r.extra[0]) : nullptr;
+      rc = launch_embedding_rows((float *)ptr(r.out), (const float *)ptr(r.a), pg.memo_ext[3], pg.memo_ext[4], (int)T, (int)V, (int)D, addend);
+    } else {
+      rc = cthip_embedding((float *)ptr(r.out), (const float *)ptr(r.a), (const float *)ptr(r.b), (int)T, (int)V, (int)D);
     }
-    if (addend) return false;
-    if (ai.base || ai.c[0] != 1 || ai.c[1] || ai.c[2]) return false;       // idx (T)
-    if (T == 0 || D == 0) return true;
-    rc = cthip_embedding((float *)ptr(r.out), (const float *)ptr(r.a), (const float *)ptr(r.b), (int)T, (int)V, (int)D);
     pg.last_route = "cthip_embedding";
     return true;
   }
   if (r.kind == R_ARGMAX) {
+    const std::map<std::string, long long> &env = sc.env();
     long long Rn, N;
     if (!bound(0, Rn) || !bound(1, N) || N < 1) return false;
     Affine ax, ao;
@@ -1859,29 +1949,54 @@ static bool launch_route(Program &pg, void **args, const std::map<std::string, l
     return true;
   }
   if (r.kind == R_SOFTMAX) {
-    long long Rn, N;
-    if (!bound(0, Rn) || !bound(1, N) || N < 1) return false;
-    Affine ax, ao;
-    if (!affine_of(r.a_idx, r.idx, 2, env, ax) || ax.base || ax.c[0] != N || ax.c[1] != 1) return false;
-    if (!affine_of(r.out_idx, r.idx, 2, env, ao) || ao.base || ao.c[0] != N || ao.c[1] != 1) return false;
+    if (!memo) {
+      const std::map<std::string, long long> &env = sc.env();
+      pg.memo_ok = false;
+      long long Rn, N;
+      if (!bound(0, Rn) || !bound(1, N) || N < 1) return false;
+      Affine ax, ao;
+      if (!affine_of(r.a_idx, r.idx, 2, env, ax) || ax.base || ax.c[0] != N || ax.c[1] != 1) return false;
+      if (!affine_of(r.out_idx, r.idx, 2, env, ao) || ao.base || ao.c[0] != N || ao.c[1] != 1) return false;
+      pg.memo_key = sc.val;
+      pg.memo_ext = {Rn, N};
+      pg.memo_ok = true;
+    }
+    const long long Rn = pg.memo_ext[0], N = pg.memo_ext[1];
     if (Rn == 0) return true;
-    rc = cthip_softmax((float *)ptr(r.out), (const float *)ptr(r.a), Rn, (int)N);
+    GraphOp op = {};
+    op.kind = GraphOp::SOFTMAX;
+    op.out = (float *)ptr(r.out), op.x = (const float *)ptr(r.a);
+    op.rows = Rn, op.n = (int)N;
+    rc = graph_op(op);
     pg.last_route = "cthip_softmax";
     return true;
   }
   if (r.kind == R_LAYERNORM || r.kind == R_RMSNORM) {
-    long long Rn, N;
-    if (!bound(0, Rn) || !bound(1, N) || N < 1) return false;
-    Affine ax, ao, ag;
-    if (!affine_of(r.a_idx, r.idx, 2, env, ax) || ax.base || ax.c[0] != N || ax.c[1] != 1) return false;
-    if (!affine_of(r.out_idx, r.idx, 2, env, ao) || ao.base || ao.c[0] != N || ao.c[1] != 1) return false;
-    // gamma / beta are read by column, whatever the row
-    if (r.b >= 0 && (!affine_of(r.b_idx, r.idx, 2, env, ag) || ag.base || ag.c[0] != 0 || ag.c[1] != 1)) return false;
-    if (r.bias >= 0 && (!affine_of(r.bias_idx, r.idx, 2, env, ag) || ag.base || ag.c[0] != 0 || ag.c[1] != 1)) return false;
+    if (!memo) {
+      const std::map<std::string, long long> &env = sc.env();
+      pg.memo_ok = false;
+      long long Rn, N;
+      if (!bound(0, Rn) || !bound(1, N) || N < 1) return false;
+      Affine ax, ao, ag;
+      if (!affine_of(r.a_idx, r.idx, 2, env, ax) || ax.base || ax.c[0] != N || ax.c[1] != 1) return false;
+      if (!affine_of(r.out_idx, r.idx, 2, env, ao) || ao.base || ao.c[0] != N || ao.c[1] != 1) return false;
+      // gamma / beta are read by column, whatever the row
+      if (r.b >= 0 && (!affine_of(r.b_idx, r.idx, 2, env, ag) || ag.base || ag.c[0] != 0 || ag.c[1] != 1)) return false;
+      if (r.bias >= 0 && (!affine_of(r.bias_idx, r.idx, 2, env, ag) || ag.base || ag.c[0] != 0 || ag.c[1] != 1)) return false;
+      pg.memo_key = sc.val;
+      pg.memo_ext = {Rn, N};
+      pg.memo_ok = true;
+    }
+    const long long Rn = pg.memo_ext[0], N = pg.memo_ext[1];
     if (Rn == 0) return true;
     const float *g = r.b >= 0 ? (const float *)ptr(r.b) : nullptr, *bt = r.bias >= 0 ? (const float *)ptr(r.bias) : nullptr;
     if (r.kind == R_LAYERNORM) {
-      rc = cthip_layernorm((float *)ptr(r.out), (const float *)ptr(r.a), g, bt, (float)r.eps, Rn, (int)N);
+      GraphOp op = {};
+      op.kind = GraphOp::LAYERNORM;
+      op.out = (float *)ptr(r.out), op.x = (const float *)ptr(r.a), op.g = g, op.b = bt;
+      op.eps = (float)r.eps;
+      op.rows = Rn, op.n = (int)N;
+      rc = graph_op(op);
       pg.last_route = "cthip_layernorm";
     } else {
       rc = cthip_rmsnorm((float *)ptr(r.out), (const float *)ptr(r.a), g, (float)r.eps, Rn, (int)N);
@@ -1923,6 +2038,7 @@ int cthip_program_create(void **program, const char *blueprint) {
   else if ((r = Route(), match_softmax(pg->item, r))) pg->route = r, pg->route_name = "softmax";
   else if ((r = Route(), match_layernorm(pg->item, r))) pg->route = r, pg->route_name = "layernorm";
   else if ((r = Route(), match_rmsnorm(pg->item, r))) pg->route = r, pg->route_name = "rmsnorm";
+  else if ((r = Route(), match_copy(pg->item, r))) pg->route = r;
   *program = pg;
   return 0;
 }
@@ -1955,30 +2071,44 @@ int cthip_program_launch(void *program, void **args, int nargs) {
   const Item &it = pg->item;
   if (nargs != (int)it.globals.size())
     return fail(CTHIP_E_BAD_ARG, "HIP: %s takes %zu arguments, got %d", it.name.c_str(), it.globals.size(), nargs);
-  std::map<std::string, long long> env;
-  for (int k = 0; k < nargs; k++) {
-    const Global &g = it.globals[k];
-    if (!args[k]) return fail(CTHIP_E_BAD_ARG, "HIP: %s: argument %s is null", it.name.c_str(), g.id.c_str());
-    if (g.pointer) {
-      if (!*(void **)args[k]) return fail(CTHIP_E_BAD_ARG, "HIP: please transfer the buffer %s to the device first", g.id.c_str());
-      continue;
+  if ((int)pg->arg_code.size() != nargs) {
+    pg->scalar_pos.clear();
+    for (int k = 0; k < nargs; k++) {
+      const Global &g = it.globals[k];
+      const int code = g.pointer ? 'p' : g.dtype == "int64" || g.dtype == "uint64" ? 'q' : g.dtype == "int32" ? 'i' : g.dtype == "uint32" ? 'I'
+                     : g.dtype == "int16" ? 'h' : g.dtype == "uint16" ? 'H' : g.dtype == "int8" ? 'b' : g.dtype == "uint8" || g.dtype == "bool" ? 'B' : 'f';
+      pg->arg_code.push_back((char)code);
+      if (code != 'p' && code != 'f') pg->scalar_pos.push_back(k);  // floating-point scalars do not size anything
     }
-    long long v = 0;
-    if (g.dtype == "int64" || g.dtype == "uint64") v = *(long long *)args[k];
-    else if (g.dtype == "int32") v = *(int *)args[k];
-    else if (g.dtype == "uint32") v = *(unsigned *)args[k];
-    else if (g.dtype == "int16") v = *(short *)args[k];
-    else if (g.dtype == "uint16") v = *(unsigned short *)args[k];
-    else if (g.dtype == "int8") v = *(signed char *)args[k];
-    else if (g.dtype == "uint8" || g.dtype == "bool") v = *(unsigned char *)args[k];
-    else continue;  // floating-point scalars do not size anything
-    env[g.id] = v;
+  }
+  ScalarArgs sc = {it, pg->scalar_pos, {}, {}};
+  sc.val.reserve(pg->scalar_pos.size());
+  for (int k = 0; k < nargs; k++) {
+    if (!args[k]) return fail(CTHIP_E_BAD_ARG, "HIP: %s: argument %s is null", it.name.c_str(), it.globals[k].id.c_str());
+    switch (pg->arg_code[k]) {
+      case 'p':
+        if (!*(void **)args[k]) return fail(CTHIP_E_BAD_ARG, "HIP: please transfer the buffer %s to the device first", it.globals[k].id.c_str());
+        break;
+      case 'q': sc.val.push_back(*(long long *)args[k]); break;
+      case 'i': sc.val.push_back(*(int *)args[k]); break;
+      case 'I': sc.val.push_back(*(unsigned *)args[k]); break;
+      case 'h': sc.val.push_back(*(short *)args[k]); break;
+      case 'H': sc.val.push_back(*(unsigned short *)args[k]); break;
+      case 'b': sc.val.push_back(*(signed char *)args[k]); break;
+      case 'B': sc.val.push_back(*(unsigned char *)args[k]); break;
+      default: break;
+    }
   }
   if (pg->route.kind != R_NONE && state().render_routes) {
     int rc = 0;
-    if (launch_route(*pg, args, env, rc)) return rc;
+    if (launch_route(*pg, args, sc, rc)) return rc;
+  }
+  {
+    const int rc = graph_ops_flush();
+    if (rc) return rc;
   }
   if (!pg->fn) return fail(CTHIP_E_STATE, "HIP: %s has not been bound to a compiled module (cthip_program_bind)", it.name.c_str());
+  const std::map<std::string, long long> &env = sc.env();
   long long total = 1;
   for (const Sx &b : pg->grid_bounds) {
     long long v;

@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "common.h"
+#include "graph_ops.h"
 
 namespace cthip {
 
@@ -462,8 +463,10 @@ int cthip_vm_run(void *vm) {
     }
     if (v->profile && v->runs++)  // (the first forward opens everything)
       v->open_ns += std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now() - t0).count();
+    GraphCollector collector;  // neighbours that can share a launch do (graph_ops.hip)
     for (size_t k = 0; k < v->nodes.size() && !rc; k++)
       if (v->nodes[k].type == VM_NODE_KERNEL) rc = vm_kernel(*v, (int)k, v->nodes[k]);
+    if (!rc) rc = graph_ops_flush();
     return rc;
   }
   for (size_t k = 0; k < v->nodes.size() && !rc; k++) {
