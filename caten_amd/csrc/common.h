@@ -151,7 +151,6 @@ struct GemvArgs {
   const float *residual;
   const float *norm_g;
   const float *norm_b;
-  float *norm_out;  // a LayerNorm applied in front of the product (no fold): where the normalised rows are kept as well, or null
   // LayerNorm folded through the product (see k_gemv): fold_s[r] = sum_k W[r,k]*gamma[k]; the caller
   // passes sum_k W[r,k]*beta[k] + b[r] as `bias`.  Null = normalise the input first.
   const float *fold_s;
@@ -189,6 +188,7 @@ struct GemvArgs {
   float *nx_out;
   const float *nx_wte, *nx_wpe;
   int nx_dim, nx_vocab, nx_max_pos;
+  float *norm_out;  // a LayerNorm applied in front of the product (no fold): where the normalised rows are kept as well, or null
 };
 // most wavefronts any GEMV launch uses (sizes the am_val / am_idx scratch)
 constexpr int kGemvMaxWaves = 16384;
@@ -199,7 +199,7 @@ int launch_gemv_wide(const WMat *w, GemvArgs a, int m);
 int wmat_create_impl(WMat **out, int type, const void *raw, int64_t rows, int64_t cols);
 // true when a register-resident GEMV variant covers the matrix (no temporary is allocated at launch)
 bool gemv_is_direct(const WMat *w);
-bool gemv_norm_out_ok(const WMat *w);  // the single-row launch over this matrix honours norm_out
+bool gemv_norm_out_ok(const WMat *w);  // the single-row launch over this matrix honours norm_out (given a bias or a residual)
 // rows a wavefront of the register-resident variant for (type, cols) produces per pass; 0 = no such variant
 int gemv_rows_per_wave(int type, int64_t cols);
 // true when the single-row launch over a (rows, cols) matrix whose rows are gate / up rows in turn holds a row pair

@@ -212,8 +212,6 @@ __device__ __forceinline__ void coop_prologue(const GemvArgs &a, const float *__
                                       (v.z - mean) * rstd * gg.z + bb.z, (v.w - mean) * rstd * gg.w + bb.w);
     }
   __syncthreads();
-  if (a.norm_out && blockIdx.x == 0)
-    for (int i = tid; i < n4; i += nthr) ((float4 *)(a.norm_out + (int64_t)blockIdx.y * a.cols))[i] = ((const float4 *)xs)[i];
 }
 
 // Folded norm with a staged input: the workgroup writes gamma * x into LDS once and reduces the
@@ -482,7 +480,7 @@ __device__ __forceinline__ void gemv_ring(const GemvArgs &a, float *xs_lds, floa
           const float4 bt = a.norm_b ? sb[k] : make_float4(0.f, 0.f, 0.f, 0.f);
           ((float4 *)xs_lds)[i] = make_float4((v.x - mu) * rstd * gm.x + bt.x, (v.y - mu) * rstd * gm.y + bt.y,
                                               (v.z - mu) * rstd * gm.z + bt.z, (v.w - mu) * rstd * gm.w + bt.w);
-          if (a.norm_out && blockIdx.x == 0) ((float4 *)(a.norm_out + (int64_t)blockIdx.y * a.cols))[i] = ((const float4 *)xs_lds)[i];
+          if (EPI && a.norm_out && blockIdx.x == 0) ((float4 *)(a.norm_out + (int64_t)blockIdx.y * a.cols))[i] = ((const float4 *)xs_lds)[i];
         }
       }
       mu = 0.0f;
@@ -694,7 +692,11 @@ __global__ __launch_bounds__(256) void k_gemv(GemvArgs a) {
   const float pivot = (folded && a.pro == CTHIP_PRO_LAYERNORM) ? x[0] : 0.0f;
   if (coop) {
     if (folded) coop_fold(a, x, xs_lds, red, pivot, bs1, bs2);
-    else coop_prologue(a, x, xs_lds, red, a.pro != CTHIP_PRO_NONE);
+    else {
+      coop_prologue(a, x, xs_lds, red, a.pro != CTHIP_PRO_NONE);
+      if (a.norm_out && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < a.cols >> 2; i += blockDim.x) ((float4 *)(a.norm_out + (int64_t)m * a.cols))[i] = ((const float4 *)xs_lds)[i];
+    }
   }
   const float *__restrict__ xsrc = coop ? xs_lds : x;
 #pragma unroll

@@ -7,7 +7,8 @@
 //   * scores -> softmax -> values [-> copy of the result]: a workgroup takes one row of one batch through all of them;
 //   * a LayerNorm and the Linear over few rows that reads it: the Linear's workgroups normalise the row themselves.
 // Every operation's result is still written where its own launch would have written it: a fused launch leaves the same
-// buffers behind.  Anything else runs as before, in order.  GPT-2 small, 12 steps from a 16-token prompt: 7.35 -> 4.9 ms.
+// buffers behind.  Anything else runs as before, in order.  GPT-2 small, 12 steps from a 16-token prompt: 7.3 -> 6.1 ms, the host
+// 520 -> 250 us a step; what is left is the device's: 62 launches that are each a few round trips to memory.
 #include <stdint.h>
 #include <string.h>
 
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(256) void k_copies(CopyBatch cb) {
 }
 
 // One row of one batch: scores (bmm.hip's KC layout), softmax, values (NC layout), copy.  Sums as in k_bmm.  The row's scores stay in
-// LDS; a 12-head step at position 30: 6 us instead of four launches of 2.6 - 4.8.
+// LDS; a 12-head step at position 30: 9 us instead of six launches of 2.6 - 4.8, every one of them behind the host.
 struct GraphAttn {
   BmmArgs s, v;
   float *probs;
@@ -337,7 +338,7 @@ static int run_attention(const GraphOp *ops, int left, int &rc) {
 static bool run_norm_linear(const GraphOp *ops, int left, int &rc) {
   if (left < 2 || ops[0].kind != GraphOp::LAYERNORM || ops[1].kind != GraphOp::LINEAR) return false;
   const GraphOp &n = ops[0], &l = ops[1];
-  if (l.x != n.out || l.rows != n.rows || l.n != n.n || l.rows < 1 || l.rows > 2 || n.n % 4 || n.n > 4096) return false;
+  if (l.x != n.out || l.rows != n.rows || l.n != n.n || l.rows < 1 || l.rows > 2 || n.n % 4 || n.n > 4096 || (!l.bias && !l.resid)) return false;
   WMat w = {};
   w.type = CTHIP_F32;
   w.rows = l.cols;
