@@ -227,6 +227,9 @@ __device__ __forceinline__ int attn_head_of_block(int b, int H, int Hkv) {
 #endif
 int launch_attn(float *out, const float *q, const float *kc, const float *vc, int S, int start_pos, const int *pos,
                 int max_T, int H, int Hkv, int Dh, const AttnSplit *split = nullptr);
+// attention of many prompt rows with keys and values split once (attn_planes.hip); out as fp32 rows or as rows of two terms
+bool attn_planes_pays(int S, int start, int H, int Hkv, int DH);
+int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH);
 int launch_embedding(float *out, const float *W, const float *idx_f, const int *idx_i, int ntok, int vocab, int dim,
                      const float *W2, const int *pos, int max_pos);
 int launch_argmax(int64_t *out, const float *x, int64_t rows, int n, int *tok_out, int *pos, int64_t *history,

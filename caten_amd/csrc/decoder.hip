@@ -1036,9 +1036,11 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       }
       }
       if (last) R = 1, Xr = X + (int64_t)(s - 1) * D;
-      TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
+      const bool at = !last && planes && attn_planes_pays(R, n, c.n_heads, c.n_kv_heads, Dh), att = at && in_planes(L.proj, nullptr);
+      if (at) TRY(launch_attn_planes(att ? nullptr : ATT, att ? ATT : nullptr, Q, K, V, R, n, c.n_heads, c.n_kv_heads, Dh));
+      else TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
       const bool ft = in_planes(L.fc, L.proj), gt = ft && (gpt2 || L.fc_pairs) && in_planes(L.fc2, nullptr);
-      TRY(linear_residual_norm(L.proj, ATT, false, L.proj_b, L.ln2_g, L.ln2_b, ft));
+      TRY(linear_residual_norm(L.proj, ATT, att, L.proj_b, L.ln2_g, L.ln2_b, ft));
       const float *hin = Hb;
       if (!gpt2 && L.fc_pairs && (2 * F) % 4 == 0) {  // SwiGLU in the epilogue of the gate|up launch
         TRY(linear(G, L.fc, XN, ft, L.fc_b, nullptr, kActSwigluPairs, nullptr, gt));

@@ -70,3 +70,23 @@ def test_long_prompt_equals_short_pieces(ops, arch, kind, rows):
         assert t0 == t1
         assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
     model.close()
+
+
+@pytest.mark.parametrize("heads,kv_heads,first,rows", [(32, 4, 0, 1333), (32, 8, 37, 1500), (16, 16, 0, 2000), (16, 4, 3, 1999)])
+def test_long_prompt_attention_equals_short_pieces(ops, heads, kv_heads, first, rows):
+    """csrc/attn_planes.hip: grouped and single heads of 64 and 128, cached rows that are no multiple of a key tile in front."""
+    from caten_amd import llm, synth
+    cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=2048, n_heads=heads, n_kv_heads=kv_heads, ffn=512, n_layers=2, vocab=500, max_seq=2048)
+    model = llm.make_llama(cfg, llm.llama_state_dict(synth.llama_weights(cfg, seed=4), "q8_0"))
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], first + rows + 1, seed=4)]
+    n = first + rows
+    if first:
+        model.forward(ids[:first], first, 0)
+    got = [model.forward(ids[first:n], rows, first, return_logits=True), model.forward(ids[n:], 1, n, return_logits=True)]
+    for at in range(0, n, 63):
+        want = [model.forward(ids[at:min(at + 63, n)], min(63, n - at), at, return_logits=True)]
+    want.append(model.forward(ids[n:], 1, n, return_logits=True))
+    for (t0, l0), (t1, l1) in zip(got, want):
+        assert t0 == t1
+        assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
+    model.close()
