@@ -266,8 +266,8 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
 // matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
 // A Linear over many rows through the same kernel: x as fp32 rows or already as planes of plane_terms(precision) terms, the
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
-bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, double extra_us = 0.0);
-bool linear_planes_ready(const WMat *w, int m, int precision, double extra_us);  // x in planes certainly runs
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in);
+bool linear_planes_ready(const WMat *w, int m, int precision);  // x in planes certainly runs
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
                          int precision, const GemmRoute *route, unsigned char *planes_out, bool *done);
 bool rows_planes_supported(int K);
@@ -280,7 +280,7 @@ bool reduce_norm_supported(int n, int nparts);
 // C (m, n) = sum_z ws[z] + bias + residual for partial tiles handed over through GemmDeferred
 int launch_splitk_reduce(float *C, float *ws, int ksplit, int m, int n, const float *bias, const float *residual);
 int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, int64_t part_stride, const float *bias,
-                       const float *resid, const float *g, const float *b, float eps, int64_t rows, int n, bool rms);
+                       const float *resid, const float *g, const float *b, float eps, int64_t rows, int n, bool rms, bool terms = false);
 // takes the device address of the static split-K scratch of cthip_matmul_noalloc (once per device, that device current)
 int matmul_scratch_init(int device);
 // gate|up rows (m, 2*cols) -> silu(gate)*up (m, cols), or a norm, as a launch of its own

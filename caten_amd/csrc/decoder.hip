@@ -960,11 +960,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // a row of terms is as long as the fp32 row whose buffer it takes.  (A session with a quantised cache keeps the
     // order of summation of the tiles: a rounding step of a cached value is a hundred times what a sum is off by.)
     const bool planes = !d->kvq && prec == GEMM_BF16X3_DEFAULT && s >= 64 && rows_planes_supported(D) && F % 32 == 0;
-    // (before: the Linear in front of the norm that feeds w.  Its split reduction goes into that norm's launch where the norm
-    // writes fp32 rows: 7 us over two launches)
-    auto in_planes = [&](const WMat *w, const WMat *before) {
-      return planes && w && linear_planes_ready(w, R, prec, before && reduce_norm_supported(D, 1) && !linear_planes_pays(before, R, prec, false) ? 7.0 : 0.0);
-    };
+    auto in_planes = [&](const WMat *w) { return planes && w && linear_planes_ready(w, R, prec); };
     // y = norm(x), as terms where the Linear behind it takes them
     auto norm = [&](float *y, const float *x, const float *g, const float *b, bool terms) {
       if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps);
@@ -985,12 +981,12 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // Xr += W.in + bias, then XN = norm(Xr) with (g, b), as terms or not; g == nullptr: no norm follows (after the last layer)
     auto linear_residual_norm = [&](const WMat *w, const float *in, bool in_terms, const float *bias, const float *g, const float *b, bool out_terms) {
       GemmDeferred df;
-      const bool fuse = g != nullptr && reduce_norm_supported(D, 1) && !out_terms;
+      const bool fuse = g != nullptr && reduce_norm_supported(D, 1);
       int r = linear(Xr, w, in, in_terms, bias, Xr, CTHIP_ACT_NONE, nullptr, false, fuse ? &df : nullptr);
       if (r) return r;
       if (df.ws) {
         if (reduce_norm_supported(D, df.ksplit)) {
-          r = launch_reduce_norm(XN, Xr, df.ws, df.ksplit, (int64_t)R * D, bias, Xr, g, b, c.eps, R, D, !gpt2);
+          r = launch_reduce_norm(XN, Xr, df.ws, df.ksplit, (int64_t)R * D, bias, Xr, g, b, c.eps, R, D, !gpt2, out_terms);
         } else {  // too many shares of too wide a row to hold at once: reduce, then normalise
           r = launch_splitk_reduce(Xr, df.ws, df.ksplit, R, D, bias, Xr);
           if (!r) r = norm(XN, Xr, g, b, out_terms);
@@ -1000,7 +996,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       }
       return g ? norm(XN, Xr, g, b, out_terms) : 0;
     };
-    bool xt = in_planes(d->layers[0].attn, nullptr);
+    bool xt = in_planes(d->layers[0].attn);
     TRY(norm(XN, X, d->layers[0].ln1_g, d->layers[0].ln1_b, xt));
     for (int l = 0; l < c.n_layers; l++) {
       Layer &L = d->layers[l];
@@ -1036,10 +1032,10 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       }
       }
       if (last) R = 1, Xr = X + (int64_t)(s - 1) * D;
-      const bool at = !last && planes && attn_planes_pays(R, n, c.n_heads, c.n_kv_heads, Dh), att = at && in_planes(L.proj, nullptr);
+      const bool at = !last && planes && attn_planes_pays(R, n, c.n_heads, c.n_kv_heads, Dh), att = at && in_planes(L.proj);
       if (at) TRY(launch_attn_planes(att ? nullptr : ATT, att ? ATT : nullptr, Q, K, V, R, n, c.n_heads, c.n_kv_heads, Dh));
       else TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
-      const bool ft = in_planes(L.fc, L.proj), gt = ft && (gpt2 || L.fc_pairs) && in_planes(L.fc2, nullptr);
+      const bool ft = in_planes(L.fc), gt = ft && (gpt2 || L.fc_pairs) && in_planes(L.fc2);
       TRY(linear_residual_norm(L.proj, ATT, att, L.proj_b, L.ln2_g, L.ln2_b, ft));
       const float *hin = Hb;
       if (!gpt2 && L.fc_pairs && (2 * F) % 4 == 0) {  // SwiGLU in the epilogue of the gate|up launch
@@ -1053,7 +1049,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
           hin = G;
         }
       }
-      xt = !last && in_planes(d->layers[l + 1].attn, L.fc2);
+      xt = !last && in_planes(d->layers[l + 1].attn);
       TRY(linear_residual_norm(L.fc2, hin, gt, L.fc2_b, last ? nullptr : d->layers[l + 1].ln1_g, last ? nullptr : d->layers[l + 1].ln1_b, xt));
     }
   }

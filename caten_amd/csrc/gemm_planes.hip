@@ -594,7 +594,7 @@ static double linear_tiles_us(const WMat *w, int m, int terms) {
   const double c = terms == 2 ? 13.2 : 10.0;
   return 2.0 + (ks > 1 ? 5.0 : 0.0) + (double)((tiles * ks + cus - 1) / cus) * (1.0 + c * K / ks * 1e-3);
 }
-bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, double extra_us) {
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   if (precision == GEMM_FP32 || m < 64 || w->rows < 64 || w->cols < 64 || (!is_quant(w) && w->cols % 16)) return false;
   // (three terms against integers: registers for one 32-column block less per wavefront, no faster than the tiles)
   if (is_quant(w) && precision == GEMM_BF16X6) return false;
@@ -602,11 +602,11 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, dou
   double bytes = 0.0;
   if (!weight_planes_stay(w, terms_b)) bytes = (double)w->rows * w->cols * (w->type == CTHIP_F16 ? 2.0 : 4.0) + weight_plane_bytes(w, terms_b);
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
-  return planes_pay(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes, linear_tiles_us(w, m, terms) - extra_us);
+  return planes_pay(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes, linear_tiles_us(w, m, terms));
 }
 // ... and nothing can be in the way of it: the matrix has its planes (made here if need be)
-bool linear_planes_ready(const WMat *w, int m, int precision, double extra_us) {
-  if (!linear_planes_pays(w, m, precision, true, extra_us)) return false;
+bool linear_planes_ready(const WMat *w, int m, int precision) {
+  if (!linear_planes_pays(w, m, precision, true)) return false;
   const int terms_b = weight_terms(w, plane_terms(precision));
   if (!weight_planes_stay(w, terms_b)) return false;
   bool temp = false;

@@ -133,7 +133,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &a, const float *Cs, i
   const bool plain = a.ksplit > 1;
   float *dst = plain ? a.ws + (int64_t)blockIdx.y * M * N : a.C;
   int ldd = N, cbase = 0;  // row pitch of the destination and the column its first element stands for
-  if (a.routed) {
+  if (a.routed && !plain) {
     const int part = n0 >= a.route.c0[2] ? 2 : n0 >= a.route.c0[1] ? 1 : 0;  // uniform over the workgroup
     dst = a.route.dst[part], ldd = a.route.ld[part], cbase = a.route.c0[part];
   }
@@ -1069,6 +1069,7 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
 }
 
 // C = act(sum_z ws[z] + bias) + residual, z in ascending order (the result does not depend on timing)
+template <bool ROUTED>
 __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs a) {
   const int64_t n = (int64_t)a.M * a.N;
   // Up to eight partials, bias and residual are requested together, none behind a branch (absent ones re-read
@@ -1089,7 +1090,12 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs a) {
     if (a.bias) v += bv;
     v = apply_act(a.act, v);
     if (a.residual) v += rv;
-    a.C[i] = v;
+    if (ROUTED) {
+      const int row = (int)(i / a.N), col = (int)(i % a.N), part = col >= a.route.c0[2] ? 2 : col >= a.route.c0[1] ? 1 : 0;
+      a.route.dst[part][(int64_t)row * a.route.ld[part] + (col - a.route.c0[part])] = v;
+    } else {
+      a.C[i] = v;
+    }
   }
 }
 
@@ -1159,7 +1165,9 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
     int ks = quant ? (int)(cus / tiles) : (int)((tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles);
     if (ks > nsteps / 3) ks = nsteps / 3;
     if (ks > 16) ks = 16;
-    if (a.routed || a.pairs) ks = 1;  // routed / paired tiles are stored by the workgroup that computed them
+    if (a.pairs) ks = 1;  // paired tiles are stored by the workgroup that computed them
+    // routed ones go through the reduction where it shortens every workgroup's chain by more than its launch takes (500 k: 6 us)
+    if (a.routed && ks > 1 && a.K - a.K / ks < 500) ks = 1;
     if (ks > 1) {
       const int steps_per = (nsteps + ks - 1) / ks;
       a.kper = steps_per * 64;
@@ -1251,7 +1259,8 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
   if (a.ksplit > 1) {
     int64_t blocks = ((int64_t)a.M * a.N + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)blocks), dim3(256), 0, st, a);
+    if (a.routed) hipLaunchKernelGGL(k_splitk_reduce<true>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(k_splitk_reduce<false>, dim3((unsigned)blocks), dim3(256), 0, st, a);
     le = hipGetLastError();
     int rc = static_ws ? 0 : cthip_free(a.ws);  // stream-ordered: the block is reused only by later work on the same stream
     if (le != hipSuccess) return fail((int)le, "gemm: launch -> %s", hipGetErrorString(le));
@@ -1273,7 +1282,7 @@ int launch_splitk_reduce(float *C, float *ws, int ksplit, int m, int n, const fl
   a.act = CTHIP_ACT_NONE;
   int64_t blocks = ((int64_t)m * n + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)blocks), dim3(256), 0, state().stream, a);
+  hipLaunchKernelGGL(k_splitk_reduce<false>, dim3((unsigned)blocks), dim3(256), 0, state().stream, a);
   CTHIP_LAUNCH_CHECK();
   return 0;
 }
