@@ -30,8 +30,10 @@ struct State {
   // 2 .. 16 = that many, 0 = one workgroup per head
   int attn_split = 1;
   // option "attn_long_from": the position from which sessions with a three-launch layer give the attention a launch
-  // of its own (keys shared by several workgroups, then the projection): four launches per layer; 0 = never
-  int attn_long_from = 896;
+  // of its own (keys shared by several workgroups, then the projection): four launches per layer; 0 = never.  The
+  // line lies where they cross: 12 heads of 64 at positions 600 / 760, us per step: 214 / 229 as three launches, 220 / 223
+  // as four; 32 heads over 4: 601 / 625 against 618 / 617.
+  int attn_long_from = 704;
   // decoder sessions read these when they first run
   int decoder_graph = 1;  // option "decoder_graph": 0 = the step's launches are issued one by one (kernel tracing)
   int prefill_gemm = 1;   // option "prefill_gemm": 0 = prompts are fed row by row through the decode step
@@ -215,6 +217,8 @@ struct AttnSplit {
   int *count;
 };
 constexpr int kAttnSplitMaxRanges = 16;
+constexpr int kAttnSplitTile = 256;  // keys of a tile of the split attention launches over heads of 64 elements
+int launch_attn_parts(const float *q, const float *kc, const float *vc, const int *pos, int H, int Hkv, int Dh, const AttnSplit &split);
 #ifdef __HIPCC__
 // Which head a workgroup of a decode attention launch takes.  Workgroups are dealt to the eight XCDs in turn (XCD =
 // linear workgroup id mod 8, blockIdx.x running fastest).  With H a multiple of 8, head (b mod 8) * (H / 8) + b / 8
@@ -360,6 +364,11 @@ __device__ __forceinline__ float half_bits_to_float(unsigned short h) {
 // api/high-level-ops.lisp:112-117): exp(x) = exp2(x * 1/ln2); sigmoid = recip(1 + exp2(-x/ln2));
 // tanh(y) = 2*sigmoid(2y) - 1.
 __device__ __forceinline__ float ct_exp(float x) { return exp2f(x * 1.442695f); }
+// keys per range where at most nz workgroups share T keys in whole tiles
+__device__ __forceinline__ int attn_split_keys(int T, int nz, int tile) {
+  const int tiles = (T + tile - 1) / tile;
+  return ((tiles + nz - 1) / nz) * tile;
+}
 // The workgroup that drew a head's last ticket adds the ranges' triples up, in range order: `all` holds nranges
 // records of dh unnormalised outputs, the running maximum and the running sum.  The loads are device-scope (they do
 // not look into a cache that could hold an older launch's values) and ALL of them are requested before the first is
@@ -385,6 +394,36 @@ __device__ __forceinline__ float attn_split_merge(const float *all, int nranges,
       const float e = ct_exp(mv[r] - M);
       o = fmaf(e, ov[r], o);
       L = fmaf(e, lv[r], L);
+    }
+  }
+  return o / L;
+}
+// The same sum, the same bits, in the launch after: `all` holds one head's `ranges` records, of which the first
+// `nranges` are this step's.  One wavefront, every lane its output column.  The records are asked for before the
+// number in use is known (it hangs on the position's own load), each range's weight is worked out by one lane.
+// (the caller asks with attn_parts_load before it waits for anything else)
+struct AttnParts {
+  float o[kAttnSplitMaxRanges];
+  float2 ml;
+};
+__device__ __forceinline__ AttnParts attn_parts_load(const float *all, int ranges, int dh, int lane) {
+  AttnParts p;
+  p.ml = *(const float2 *)(all + (lane < ranges ? lane : ranges - 1) * (dh + 2) + dh);
+#pragma unroll
+  for (int r = 0; r < kAttnSplitMaxRanges; r++) p.o[r] = all[(r < ranges ? r : ranges - 1) * (dh + 2) + lane];
+  return p;
+}
+__device__ __forceinline__ float attn_parts_merge(const AttnParts &p, int nranges, int lane) {
+  const float m = lane < nranges ? p.ml.x : -INFINITY;
+  const float M = wave_max(m);
+  const float e = ct_exp(m - M);
+  float o = 0.0f, L = 0.0f;
+#pragma unroll
+  for (int r = 0; r < kAttnSplitMaxRanges; r++) {
+    if (r < nranges) {
+      const float er = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), r));
+      o = fmaf(er, p.o[r], o);
+      L = fmaf(er, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.ml.y), r)), L);
     }
   }
   return o / L;

@@ -60,7 +60,8 @@ struct DecAttnArgs {
   float *part;               // out: fp32 [H][D], head h's share of the projection
   void *zero;                // cleared here: the MLP accumulators
   int64_t zero_n16;          // ... in 16-byte units
-  const float *att_in;       // null, or the heads' attention outputs [H][Dh] from a launch of its own: projection only
+  const float *parts;        // null, or the heads' attention from a launch of its own, `ranges` records per head: projection only
+  int ranges;                // ... at most: how many are in use follows from the position (attn_split_keys)
 };
 
 // the same launch over a cache kept as Q8_0 rows (kvq.hip): the step's new key / value row arrives as fp32 (k then v,
@@ -277,7 +278,8 @@ struct GqaAttnArgs {
   void *zero;                // cleared here: the MLP launch's accumulators
   int64_t zero_n16;
   int D, KD;
-  const float *att_in;       // null, or the heads' attention outputs [H][Dh] from a launch of its own: projection only
+  const float *parts;        // null, or the heads' attention from a launch of its own, `ranges` records per head: projection only
+  int ranges;                // ... at most: how many are in use follows from the position (attn_split_keys)
 };
 
 struct GqaMlpArgs {

@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void k_dec_qkv(DecQkvArgs a) {
 // holds four passes of K and V in registers, per-wavefront online softmax, one meeting in LDS.  The head's
 // slab of the projection (D rows x DH columns, contiguous after the re-layout) does not depend on anything
 // computed here and is requested first, so it arrives while the keys are being processed.
-template <int TYPE, int DH, int JR, bool ATT_IN>
+template <int TYPE, int DH, int JR, bool PARTS>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_dec_attn_proj(DecAttnArgs a) {
   constexpr int LPK = DH / 4, KPW = 64 / LPK, KPT = 4, NW = 16, TILE = NW * KPW * KPT;
@@ -204,10 +204,16 @@ void k_dec_attn_proj(DecAttnArgs a) {
     const int64_t nthr = (int64_t)H * gridDim.y * 1024;
     for (int64_t k = ((int64_t)blockIdx.y * H + h) * 1024 + tid; k < a.zero_n16; k += nthr) z[k] = zz;
   };
-  if constexpr (ATT_IN) {
+  if constexpr (PARTS) {
     clear_accumulators();
     // the head's attention was computed by a launch of its own (long contexts: its keys shared by several workgroups)
-    if (tid < DH) oh[tid] = a.att_in[h * DH + tid];
+    // and left as one record per range, added up here
+    static_assert(DH == 64, "a wavefront of output columns");
+    if (wv == 0) {
+      const AttnParts p = attn_parts_load(a.parts + (int64_t)h * a.ranges * (DH + 2), a.ranges, DH, lane);
+      const int T = a.pos[0] + 1, per = attn_split_keys(T, a.ranges, kAttnSplitTile);
+      oh[lane] = attn_parts_merge(p, (T + per - 1) / per, lane);
+    }
     __syncthreads();
   } else {
     const int T = a.pos[0] + 1;
@@ -805,7 +811,7 @@ int launch_dec_attn_proj(const DecAttnArgs &a, int type, int H, int D, int repli
   const int rpp = 1024 / (64 / xpc), jr = (D / replicas + rpp - 1) / rpp;
   if (jr > 4) return fail(CTHIP_E_BAD_ARG, "decoder: fused attention launch needs %d passes over its slab", jr);
 #define GO_T(T)                                                                                     \
-  if (a.att_in) {                                                                                   \
+  if (a.parts) {                                                                                   \
     switch (jr) {                                                                                   \
       case 1: hipLaunchKernelGGL((k_dec_attn_proj<T, 64, 1, true>), grid, block, 0, st, a); break;  \
       case 2: hipLaunchKernelGGL((k_dec_attn_proj<T, 64, 2, true>), grid, block, 0, st, a); break;  \

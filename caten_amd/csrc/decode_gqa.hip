@@ -188,7 +188,7 @@ __global__ __launch_bounds__(NT) void k_gqa_qkv(GqaQkvArgs a) {
 // Attention as in k_dec_attn_proj; the key / value rows are those of the head's group.  The head's slab of wo
 // (D rows x two Q4_0 blocks) is requested first.  gridDim.y workgroups per head repeat the attention and share
 // the slab's rows.
-template <int JR, bool ATT_IN>
+template <int JR, bool PARTS>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_gqa_attn_proj(GqaAttnArgs a) {
   constexpr int DH = 64, LPK = DH / 4, KPW = 64 / LPK, KPT = 4, NW = 16, TILE = NW * KPW * KPT;
@@ -218,9 +218,15 @@ void k_gqa_attn_proj(GqaAttnArgs a) {
     const int64_t nthr = (int64_t)H * gridDim.y * 1024;
     for (int64_t k = ((int64_t)blockIdx.y * H + h) * 1024 + tid; k < a.zero_n16; k += nthr) z[k] = zz;
   }
-  if constexpr (ATT_IN) {
+  if constexpr (PARTS) {
     // the head's attention was computed by a launch of its own (long contexts: its keys shared by several workgroups)
-    if (tid < DH) oh[tid] = a.att_in[h * DH + tid];
+    // and left as one record per range, added up here
+    static_assert(DH == 64, "a wavefront of output columns");
+    if (wv == 0) {
+      const AttnParts p = attn_parts_load(a.parts + (int64_t)h * a.ranges * (DH + 2), a.ranges, DH, lane);
+      const int T = a.pos[0] + 1, per = attn_split_keys(T, a.ranges, kAttnSplitTile);
+      oh[lane] = attn_parts_merge(p, (T + per - 1) / per, lane);
+    }
     __syncthreads();
   } else {
     const int T = a.pos[0] + 1;
@@ -483,7 +489,7 @@ int launch_gqa_attn_proj(const GqaAttnArgs &a, int H, int HKV, int replicas) {
   dim3 grid(H, replicas), block(1024);
   hipStream_t st = state().stream;
   const int jr = (D / replicas + 511) / 512;
-  if (a.att_in) {
+  if (a.parts) {
     switch (jr) {
       case 1: hipLaunchKernelGGL((k_gqa_attn_proj<1, true>), grid, block, 0, st, a); break;
       case 2: hipLaunchKernelGGL((k_gqa_attn_proj<2, true>), grid, block, 0, st, a); break;

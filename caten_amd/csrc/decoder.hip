@@ -635,16 +635,19 @@ static int queue_step(Decoder *d, bool with_head, bool embed) {
         a8.zero_n16 = aa.zero_n16;
         if (skip & 2) {
         } else if (d->long_mode) {  // rotation (none here), quantisation, append and attention, then the projection
-          TRY(launch_attn_q8_step(d->att, d->q, d->kv_tmp, L.kq, L.kdq, L.vq, L.vdq, pos, c.n_heads, c.n_kv_heads, Dh, 0.0f, &d->att_split));
-          aa.att_in = d->att;
+          AttnSplit parts = {d->att_split.ranges, d->att_split.part, nullptr};
+          TRY(launch_attn_q8_step(nullptr, d->q, d->kv_tmp, L.kq, L.kdq, L.vq, L.vdq, pos, c.n_heads, c.n_kv_heads, Dh, 0.0f, &parts));
+          aa.parts = parts.part;
+          aa.ranges = parts.ranges;
           TRY(launch_dec_attn_proj(aa, L.attn->type, c.n_heads, D, replicas));
         } else {
           TRY(launch_dec_attn_proj_q8(a8, L.attn->type, c.n_heads, D, replicas));
         }
       } else if (!(skip & 2)) {
         if (d->long_mode) {
-          TRY(launch_attn(d->att, d->q, L.k_cache, L.v_cache, 1, 0, pos, c.max_seq, c.n_heads, c.n_kv_heads, Dh, &d->att_split));
-          aa.att_in = d->att;
+          TRY(launch_attn_parts(d->q, L.k_cache, L.v_cache, pos, c.n_heads, c.n_kv_heads, Dh, d->att_split));
+          aa.parts = d->att_split.part;
+          aa.ranges = d->att_split.ranges;
         }
         TRY(launch_dec_attn_proj(aa, L.attn->type, c.n_heads, D, replicas));
       }
@@ -718,8 +721,9 @@ static int queue_step(Decoder *d, bool with_head, bool embed) {
       aa.D = D;
       aa.KD = KD;
       if (d->long_mode) {
-        TRY(launch_attn(d->att, d->q, L.k_cache, L.v_cache, 1, 0, pos, c.max_seq, c.n_heads, c.n_kv_heads, Dh, &d->att_split));
-        aa.att_in = d->att;
+        TRY(launch_attn_parts(d->q, L.k_cache, L.v_cache, pos, c.n_heads, c.n_kv_heads, Dh, d->att_split));
+        aa.parts = d->att_split.part;
+        aa.ranges = d->att_split.ranges;
       }
       TRY(launch_gqa_attn_proj(aa, c.n_heads, c.n_kv_heads, replicas));
       GqaMlpArgs ma = {};

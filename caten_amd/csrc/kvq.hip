@@ -171,7 +171,8 @@ __global__ __launch_bounds__(256) void k_attn_cached_q8(float *__restrict__ out,
 // quantises the new key and value as k_kvq_append does (the planes get the same bits), uses them as key T - 1 and,
 // in the first query head of each key / value head, stores them into the planes.  A head's keys are shared by
 // gridDim.z workgroups as in k_attn_cached's SPLIT form (ranges of whole tiles, device-scope stores of the
-// (max, sum, output) triples, a ticket per range, the last one adds them up in range order).
+// (max, sum, output) triples, a ticket per range, the last one adds them up in range order).  Without `out` the
+// triples are the launch's result, as in its kSplitParts form.
 template <int DH>
 __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, const float *__restrict__ qv, const float *__restrict__ newkv,
                                                       signed char *__restrict__ kq, unsigned short *__restrict__ kd,
@@ -179,6 +180,7 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
                                                       const int *__restrict__ pos, int H, int Hkv, float log2_base, int rope,
                                                       float *__restrict__ sp_part, int *__restrict__ sp_count) {
   constexpr int LPK = DH / 16, KPW = 64 / LPK, KPT = 4, NW = 4, TILE = NW * KPW * KPT;
+  static_assert(DH != 64 || TILE == kAttnSplitTile, "attn_parts_merge's ranges");
   __shared__ float part[NW][DH];
   __shared__ float pm[NW], pl[NW];
   __shared__ float ang_s[DH / 2], ang_c[DH / 2];
@@ -187,8 +189,7 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
   const int T = pos[0] + 1;
   int k0 = 0, k1 = T, nranges = 1;
   {
-    const int nz = (int)gridDim.z, tiles = (T + TILE - 1) / TILE;
-    const int per = ((tiles + nz - 1) / nz) * TILE;  // keys per range
+    const int per = attn_split_keys(T, (int)gridDim.z, TILE);
     nranges = (T + per - 1) / per;
     k0 = (int)blockIdx.z * per;
     if (k0 >= T) return;  // (uniform) no range for this workgroup
@@ -367,7 +368,11 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
       o = fmaf(e, part[w][tid], o);
       L = fmaf(e, pl[w], L);
     }
-    if (nranges == 1) {
+    if (!out) {
+      float *mine = sp_part + ((int64_t)h * gridDim.z + blockIdx.z) * (DH + 2);
+      mine[tid] = o;
+      if (tid == 0) *(float2 *)(mine + DH) = make_float2(M, L);
+    } else if (nranges == 1) {
       out[(int64_t)h * DH + tid] = o / L;
     } else {
       float *mine = sp_part + ((int64_t)h * gridDim.z + blockIdx.z) * (DH + 2);
@@ -378,7 +383,7 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
       }
     }
   }
-  if (nranges > 1) {
+  if (out && nranges > 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's device-scope stores have reached memory
     __syncthreads();
     if (tid == 0) ticket = __hip_atomic_fetch_add(sp_count + h, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -433,6 +438,7 @@ int launch_attn_q8_step(float *out, const float *q, const float *newkv, void *kq
   if (Hkv <= 0 || H % Hkv) return fail(CTHIP_E_BAD_ARG, "quantised KV cache: %d query heads over %d key / value heads", H, Hkv);
   if (split && split->ranges > kAttnSplitMaxRanges) return fail(CTHIP_E_BAD_ARG, "quantised KV cache: %d key ranges per head (at most %d)", split->ranges, kAttnSplitMaxRanges);
   const bool shared = split && split->ranges > 1;
+  if (!out && !shared) return fail(CTHIP_E_BAD_ARG, "quantised KV cache: an attention step without an output");
   dim3 grid((unsigned)H, 1, shared ? (unsigned)split->ranges : 1u), block(256);
   hipStream_t st = state().stream;
   const int rope = rope_base > 0.0f ? 1 : 0;

@@ -914,7 +914,14 @@ __global__ __launch_bounds__(256) void k_qkv_split(float *__restrict__ q, float 
 // adds the ranges up.  The grid is fixed when the step is captured while the position is device data, so how many
 // ranges are in use is decided here: workgroups past the last range leave at once, and a context of one tile is
 // one range whose workgroup writes the output itself, without a ticket.
-template <int DH, bool APPEND, bool SPLIT>
+//
+// SPLIT == kSplitParts: the ranges' triples are what the launch leaves, one range or many, and the launch that needs the
+// heads' outputs adds them up (attn_parts_merge).  The tickets cost a chain of three round trips to memory behind the
+// last key -- the stores' acknowledgement, the counter, the other ranges' triples -- where the next launch has one in
+// its prologue, beside its weights (32 query / 4 key-value heads, Q4_0 layers of width 2048, position 1500: 30.0 -> 28.3 us
+// per layer).
+enum { kSplitNone = 0, kSplitMerged = 1, kSplitParts = 2 };
+template <int DH, bool APPEND, int SPLIT>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
                                                       float *__restrict__ kc, float *__restrict__ vc,
@@ -926,6 +933,7 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
   constexpr int KPT = 4;           // passes held in registers
   constexpr int NW = 16;
   constexpr int TILE = NW * KPW * KPT;
+  static_assert(DH != 64 || TILE == kAttnSplitTile, "attn_parts_merge's ranges");
   __shared__ float part[NW][DH];
   __shared__ float pm[NW], pl[NW];
   __shared__ int ticket;
@@ -934,8 +942,7 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
   // this workgroup's keys [k0, k1): everything, or one of `nranges` ranges of whole tiles
   int k0 = 0, k1 = T, nranges = 1;
   if (SPLIT) {
-    const int nz = (int)gridDim.z, tiles = (T + TILE - 1) / TILE;
-    const int per = ((tiles + nz - 1) / nz) * TILE;  // keys per range
+    const int per = attn_split_keys(T, (int)gridDim.z, TILE);
     nranges = (T + per - 1) / per;
     k0 = (int)blockIdx.z * per;
     if (k0 >= T) return;  // (uniform) no range for this workgroup
@@ -1098,7 +1105,11 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
       o = fmaf(e, part[w][tid], o);
       L = fmaf(e, pl[w], L);
     }
-    if (!SPLIT || nranges == 1) {
+    if (SPLIT == kSplitParts) {  // read by the next launch
+      float *mine = sp_part + ((int64_t)(i * H + h) * gridDim.z + blockIdx.z) * (DH + 2);
+      mine[tid] = o;
+      if (tid == 0) *(float2 *)(mine + DH) = make_float2(M, L);
+    } else if (SPLIT == kSplitNone || nranges == 1) {
       out[((int64_t)i * H + h) * DH + tid] = o / L;
     } else {
       // device-scope stores: written through to memory, no cache to flush (a fence here would write back and
@@ -1111,7 +1122,7 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
       }
     }
   }
-  if (SPLIT && nranges > 1) {
+  if (SPLIT == kSplitMerged && nranges > 1) {
     // a thread's stores have reached memory when the memory counter is back at zero; after the barrier that holds
     // for the whole workgroup, and only then is its ticket drawn.  The workgroup with the last ticket reads every
     // range's triple with device-scope loads (which do not look into a cache that could hold an older launch's).
@@ -1609,6 +1620,20 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma_bf(float *__restrict__ ou
   }
 }
 
+// one decode row over a context shared by split.ranges workgroups per head, the ranges' triples left in split.part for
+// attn_parts_merge in the launch that follows
+int launch_attn_parts(const float *q, const float *kc, const float *vc, const int *pos, int H, int Hkv, int Dh, const AttnSplit &split) {
+  if (Dh != 64 || !pos || split.ranges < 1 || split.ranges > kAttnSplitMaxRanges)
+    return fail(CTHIP_E_BAD_ARG, "attention: parts of %d key ranges, head_dim %d", split.ranges, Dh);
+  float *noo = nullptr;
+  const float *nokv = nullptr;
+  int *noc = nullptr;
+  hipLaunchKernelGGL((k_attn_cached<64, false, kSplitParts>), dim3(H, 1, split.ranges), dim3(1024), 0, state().stream, noo, q,
+                     const_cast<float *>(kc), const_cast<float *>(vc), 0, pos, H, Hkv, nokv, 0.0f, split.part, noc);
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+
 int launch_attn(float *out, const float *q, const float *kc, const float *vc, int S, int start_pos, const int *pos,
                 int max_T, int H, int Hkv, int Dh, const AttnSplit *split) {
   if (S == 0) return 0;
@@ -1655,9 +1680,9 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
   if (split && split->ranges > 1) {  // a row (or a few) over a context that may be long: the keys shared by several workgroups
     dim3 grid(H, S, split->ranges), block(1024);
     switch (Dh) {
-      case 32: hipLaunchKernelGGL((k_attn_cached<32, false, true>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
-      case 64: hipLaunchKernelGGL((k_attn_cached<64, false, true>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
-      case 128: hipLaunchKernelGGL((k_attn_cached<128, false, true>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
+      case 32: hipLaunchKernelGGL((k_attn_cached<32, false, kSplitMerged>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
+      case 64: hipLaunchKernelGGL((k_attn_cached<64, false, kSplitMerged>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
+      case 128: hipLaunchKernelGGL((k_attn_cached<128, false, kSplitMerged>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, split->part, split->count); break;
       default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
     }
     CTHIP_LAUNCH_CHECK();
@@ -1665,9 +1690,9 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
   }
   dim3 grid(H, S), block(1024);
   switch (Dh) {
-    case 32: hipLaunchKernelGGL((k_attn_cached<32, false, false>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, nop, noc); break;
-    case 64: hipLaunchKernelGGL((k_attn_cached<64, false, false>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, nop, noc); break;
-    case 128: hipLaunchKernelGGL((k_attn_cached<128, false, false>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, nop, noc); break;
+    case 32: hipLaunchKernelGGL((k_attn_cached<32, false, kSplitNone>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, nop, noc); break;
+    case 64: hipLaunchKernelGGL((k_attn_cached<64, false, kSplitNone>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, nop, noc); break;
+    case 128: hipLaunchKernelGGL((k_attn_cached<128, false, kSplitNone>), grid, block, 0, st, out, q, kcw, vcw, start_pos, pos, H, Hkv, nokv, 0.0f, nop, noc); break;
     default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
   }
   CTHIP_LAUNCH_CHECK();
@@ -1683,9 +1708,9 @@ int launch_attn_rope_append(float *out, const float *q, float *kc, float *vc, co
   if (split && split->ranges > 1) {
     dim3 grid(H, 1, split->ranges), block(1024);
     switch (Dh) {
-      case 32: hipLaunchKernelGGL((k_attn_cached<32, true, true>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, split->part, split->count); break;
-      case 64: hipLaunchKernelGGL((k_attn_cached<64, true, true>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, split->part, split->count); break;
-      case 128: hipLaunchKernelGGL((k_attn_cached<128, true, true>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, split->part, split->count); break;
+      case 32: hipLaunchKernelGGL((k_attn_cached<32, true, kSplitMerged>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, split->part, split->count); break;
+      case 64: hipLaunchKernelGGL((k_attn_cached<64, true, kSplitMerged>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, split->part, split->count); break;
+      case 128: hipLaunchKernelGGL((k_attn_cached<128, true, kSplitMerged>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, split->part, split->count); break;
       default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
     }
     CTHIP_LAUNCH_CHECK();
@@ -1695,9 +1720,9 @@ int launch_attn_rope_append(float *out, const float *q, float *kc, float *vc, co
   float *nop = nullptr;
   int *noc = nullptr;
   switch (Dh) {
-    case 32: hipLaunchKernelGGL((k_attn_cached<32, true, false>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, nop, noc); break;
-    case 64: hipLaunchKernelGGL((k_attn_cached<64, true, false>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, nop, noc); break;
-    case 128: hipLaunchKernelGGL((k_attn_cached<128, true, false>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, nop, noc); break;
+    case 32: hipLaunchKernelGGL((k_attn_cached<32, true, kSplitNone>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, nop, noc); break;
+    case 64: hipLaunchKernelGGL((k_attn_cached<64, true, kSplitNone>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, nop, noc); break;
+    case 128: hipLaunchKernelGGL((k_attn_cached<128, true, kSplitNone>), grid, block, 0, st, out, q, kc, vc, 0, pos, H, Hkv, newkv, lb, nop, noc); break;
     default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
   }
   CTHIP_LAUNCH_CHECK();

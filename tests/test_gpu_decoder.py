@@ -251,6 +251,40 @@ def test_three_launch_layer_with_the_attention_as_a_launch_of_its_own(arch, plen
         assert any(not np.array_equal(a, b) for a, b in zip(runs[0][1][-8:], runs[1][1][-8:]))
 
 
+@pytest.mark.parametrize("arch,plen,split,kv", [("llama", 252, 1, 0), ("llama", 508, 2, 0), ("llama", 764, 3, 0), ("gpt2", 508, 16, 0),
+                                                ("gpt2", 764, 2, 1)])
+def test_key_ranges_added_up_by_the_projection_launch(arch, plen, split, kv):
+    """Positions on both sides of a tile of 256 keys, where the number of ranges in use changes, with fewer, as many and
+    more ranges than tiles (option attn_split): the projection launch adds the ranges' records up; tokens of the
+    three-launch layer that repeats the attention, logits inside the fp32 band."""
+    print(f"case: key ranges added up by the projection launch, {arch} prompt {plen} split {split} kv_cache {kv}", flush=True)
+    from caten_amd import _lib, synth, llm
+    lib = _lib.load()
+    if arch == "gpt2":
+        cfg = dict(synth.GPT2_CONFIGS["gpt2-mini"], max_seq=1024)
+        sd, make = llm.gpt2_state_dict(synth.gpt2_weights(cfg, seed=37), "q8_0"), llm.make_gpt2
+    else:
+        cfg = dict(synth.LLAMA_CONFIGS["llama-1.1b"], n_layers=2, max_seq=1024, vocab=2000)
+        sd, make = llm.llama_state_dict(synth.llama_weights(cfg, seed=37), "q4_0"), llm.make_llama
+    prompt = synth.prompt(cfg["vocab"], plen, seed=37)
+    runs = []
+    try:
+        _lib.check(lib.cthip_set_option(b"kv_cache", kv))
+        _lib.check(lib.cthip_set_option(b"attn_split", split))
+        for long_from in (64, 0):
+            _lib.check(lib.cthip_set_option(b"attn_long_from", long_from))
+            model = make(cfg, sd)
+            runs.append(llm.gpt2_generate(model, prompt, 9, on_device=False, keep_logits=True))
+            model.close()
+    finally:
+        _lib.check(lib.cthip_set_option(b"attn_long_from", 704))
+        _lib.check(lib.cthip_set_option(b"attn_split", 1))
+        _lib.check(lib.cthip_set_option(b"kv_cache", 0))
+    assert runs[0][0] == runs[1][0]
+    for a, b in zip(runs[0][1], runs[1][1]):
+        close(a, b)
+
+
 @pytest.mark.parametrize("plen", [3, 40])
 def test_three_launch_grouped_query_layer_equals_five_launch_layer(plen):
     """The same for RMSNorm / RoPE / grouped-query / SwiGLU layers with Q4_0 weights at the width the three-launch
