@@ -476,7 +476,8 @@ __global__ __launch_bounds__(256) void k_norm_block(RowArgs a) {
 }
 
 // Softmax of rows too long for a block's registers, or so few that a block per row leaves the chip idle: gridDim.x
-// pieces per row each leave (maximum, sum of exponentials) ...
+// pieces per row each leave (maximum, sum of exponentials).  A piece of nothing but -inf (a masked stretch) has no finite
+// maximum to subtract: it leaves a sum of 0 (of NaN if there is one in it), which its row's maximum then scales by 0 ...
 __global__ __launch_bounds__(256) void k_softmax_part(float2 *__restrict__ part, const float *__restrict__ x, int n, int per) {
   __shared__ float red[2][4];
   const int tid = threadIdx.x, lo = blockIdx.x * per, hi = min(n, lo + per);
@@ -487,8 +488,9 @@ __global__ __launch_bounds__(256) void k_softmax_part(float2 *__restrict__ part,
   if ((tid & 63) == 0) red[0][tid >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+  const float base = m == -INFINITY ? 0.0f : m;
   float s = 0.0f;
-  for (int i = lo + tid; i < hi; i += 256) s += ct_exp(xr[i] - m);
+  for (int i = lo + tid; i < hi; i += 256) s += ct_exp(xr[i] - base);
   s = wave_sum(s);
   if ((tid & 63) == 0) red[1][tid >> 6] = s;
   __syncthreads();

@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 def close(a, b, rtol, atol):
     a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
-    bad = np.abs(a - b) > atol + rtol * np.abs(b)
+    bad = ~(np.abs(a - b) <= atol + rtol * np.abs(b))  # (a NaN is a difference)
     assert not bad.any(), f"{bad.sum()} of {bad.size} differ; max abs err {np.abs(a - b).max():.3e}"
 
 
@@ -29,6 +29,30 @@ def test_rows_of_any_length(ops, oracle, rows, n):
     close(ops.layernorm(x, g, b), oracle.layernorm(x, g, b), 1e-4, 3e-5)
     close(ops.rmsnorm(x, g), oracle.rmsnorm(x, g), 1e-4, 1e-5)
     close(ops.layernorm_softmax(x, g, b), oracle.softmax(oracle.layernorm(x, g, b)), 1e-4, 1e-7)
+
+
+@pytest.mark.parametrize("rows,n", [(3, 1025), (2, 8193), (1, 32769), (3, 50257), (49, 32769), (1, 65541), (2, 70001)])
+@pytest.mark.parametrize("masked", [-np.inf, np.finfo(np.float32).min])
+def test_softmax_of_masked_rows(ops, oracle, rows, n, masked):
+    """A row of which a sampler keeps a few values: whole stretches of it, and whole pieces where a row is shared, are masked.
+    Rows without a probability distribution stay what they are: NaN."""
+    rng = np.random.default_rng(n)
+    x = np.full((rows, n), masked, np.float32)
+    for r in range(rows):
+        x[r, rng.choice(n // 2, 40, replace=False) + (n // 2 if r % 2 else 0)] = rng.normal(0, 3, 40)
+    with np.errstate(over="ignore"):
+        want = oracle.softmax(x)
+    assert np.isfinite(want).all()
+    close(ops.softmax(x), want, 1e-4, 1e-7)
+    for bad in (np.inf, np.nan):
+        y = x.copy()
+        y[0, n - 1] = bad
+        got = ops.softmax(y)
+        assert np.isnan(got[0]).all()
+        close(got[1:], want[1:], 1e-4, 1e-7)
+    y = x.copy()
+    y[0] = -np.inf
+    assert np.isnan(ops.softmax(y)[0]).all()
 
 
 @pytest.mark.parametrize("rows,n", [(3, 1), (3, 3), (5, 5), (4, 1023), (4, 1025), (2, 4099), (2, 8191), (16, 8192), (17, 16385), (3, 50257)])
