@@ -81,22 +81,27 @@ __device__ int g_rows_tickets[kRowsGroups];  // zero between launches
 // Bytes of a weight row in a unit, and blocks of 32 k: whole cache lines.  (Requests that cover 32 bytes of a row each, as
 // operand registers would ask for them, are bound by the tag lookups of the compute unit's cache: 2.4 TB/s of Q8_0 and
 // 1.5 TB/s of Q4_0 weights, most of it for the scales.)
-template <int SRC>
-struct RowsUnit {
-  static constexpr int BLOCKS = SRC == RW_Q8 ? 4 : SRC == RW_Q4 ? 8 : 2;
-  static constexpr int BYTES = SRC == RW_F32 ? 256 : 128;
-};
+constexpr int rows_unit_blocks(int src) { return src == RW_Q8 ? 4 : src == RW_Q4 ? 8 : 2; }
+constexpr int rows_unit_bytes(int src) { return src == RW_F32 ? 256 : 128; }
+constexpr bool rows_quant(int src) { return src == RW_Q8 || src == RW_Q4; }
+// What the launcher instantiates: 16 NS weight rows a wavefront, 4 MB wavefronts, rings of PD units
+constexpr int kRowsNS = 2, kRowsPD = 2;
+constexpr int rows_columns(int mb) { return 16 * kRowsNS * 4 * mb; }  // of the result, per workgroup
+constexpr int rows_slot(int src, bool wide_d) {  // bytes of a unit in a ring: weights, scales (whole load instructions)
+  return 16 * kRowsNS * rows_unit_bytes(src) + (rows_quant(src) ? 16 * kRowsNS * rows_unit_blocks(src) / (wide_d ? 2 : 1) / 64 * 256 : 0);
+}
 
 // A wavefront: NS x 16 weight rows against MB x 16 input rows, v_mfma_f32_16x16x32 (lane l: row l % 16 of its operand, k =
 // 8 (l / 16) .. + 7 of the block; result row 4 (l / 16) + r, column l % 16).  WIDE_D: a row's scales start at a multiple of four bytes, two of them are fetched as one dword
 template <int SRC, int NPA, int MB, int NS, int NW, int PD, bool WIDE_D>
 __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
-  constexpr bool QUANT = SRC == RW_Q8 || SRC == RW_Q4;
+  constexpr bool QUANT = rows_quant(SRC);
   constexpr int NPB = SRC == RW_F32 ? NPA : 1;
-  constexpr int UB = RowsUnit<SRC>::BLOCKS, CPW = RowsUnit<SRC>::BYTES / 16;  // blocks, 16-byte chunks of a row per unit
+  constexpr int UB = rows_unit_blocks(SRC), CPW = rows_unit_bytes(SRC) / 16;  // blocks, 16-byte chunks of a row per unit
   constexpr int NR = 16 * NS;                                                     // weight rows of a wavefront
   constexpr int IW = NR * CPW / 64, ID = !QUANT ? 0 : NR * UB / (WIDE_D ? 2 : 1) / 64;  // load instructions per unit: weights, scales
   constexpr int WBYTES = NR * CPW * 16, SLOT = WBYTES + ID * 256;
+  static_assert(NS == kRowsNS && PD == kRowsPD && SLOT == rows_slot(SRC, WIDE_D), "the LDS that rows_share counts");
   constexpr int NT = NR * NW, T = 64 * NW;  // columns of a workgroup, threads
   constexpr bool HALF = SRC != RW_F32;
   typedef typename std::conditional<HALF, v8h, v8bf>::type op_t;  // one matrix operand
@@ -446,36 +451,45 @@ __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
 }
 constexpr int kRowsPlanesMaxK = 8 * 256 * 16;  // widest row the largest instantiation holds
 
-// One launch: how many workgroups share K.  Every compute unit holds `resident` workgroups (LDS) at a time; a round of
-// them costs its units at the rate of the compute unit (about 0.85 us per 16 KB of weights and workgroup, 30 % more per
-// further 16 input rows) and about 1.5 us of its own, a share costs its partial sums.
-template <int SRC, int NPA, int MB, bool WIDE_D>
-static int rows_launch(RowsGemmArgs a) {
-  constexpr int NS = 2, NW = 4 * MB, PD = 2, NT = 16 * NS * NW, T = 64 * NW, UB = RowsUnit<SRC>::BLOCKS;
-  constexpr int SLOT = 16 * NS * RowsUnit<SRC>::BYTES + (SRC == RW_Q8 || SRC == RW_Q4 ? 16 * NS * UB / (WIDE_D ? 2 : 1) / 64 * 256 : 0);
-  const int M = a.e.M, N = a.e.N, cus = state().compute_units;
-  const int groups = (N + NT - 1) / NT, units = (a.kblocks + UB - 1) / UB;
-  double best = 0;
-  int best_per = 0;
-  size_t best_lds = 0;
+// How many workgroups share K, as units per share, and the LDS such a workgroup asks for.  Every compute unit holds `resident`
+// workgroups (LDS) at a time; a round of them costs its units at the rate of the compute unit (about 0.85 us per 16 KB of weights
+// and workgroup, 30 % more per further 16 input rows) and about 1.5 us of its own, a share costs its partial sums.
+// At most 32 shares, one where there are more column groups than tickets: wide rows then fit no workgroup (per = 0).
+struct RowsShare {
+  int per = 0;
+  size_t lds = 0;
+};
+static RowsShare rows_share(int src, int terms, int mb, bool wide_d, int M, int N, int kblocks) {
+  const int ub = rows_unit_blocks(src), nt = rows_columns(mb), cus = state().compute_units;
+  const int groups = (N + nt - 1) / nt, units = (kblocks + ub - 1) / ub;
+  RowsShare best;
+  double best_us = 0;
   for (int ks = 1; ks <= 32 && ks <= units; ks++) {
     const int per = (units + ks - 1) / ks;
     if ((units + per - 1) / per != ks || (ks > 1 && groups > kRowsGroups)) continue;
-    size_t lds = (size_t)NW * PD * SLOT + (size_t)M * per * UB * 64 * NPA;
-    if (lds < (size_t)M * NT * 4) lds = (size_t)M * NT * 4;
+    size_t lds = (size_t)4 * mb * kRowsPD * rows_slot(src, wide_d) + (size_t)M * per * ub * 64 * terms;
+    if (lds < (size_t)M * nt * 4) lds = (size_t)M * nt * 4;
     if (lds > 156 * 1024) continue;
     const int resident = lds <= 78 * 1024 ? 2 : 1;
-    const double tu = 0.85 * RowsUnit<SRC>::BYTES / 128 * NW / 4 * (1 + 0.3 * (MB - 1));
+    const double tu = 0.85 * rows_unit_bytes(src) / 128 * mb * (1 + 0.3 * (mb - 1));
     const int64_t wgs = (int64_t)groups * ks;
     const int64_t full = wgs / (cus * resident), left = wgs - full * cus * resident;
     double t = full * (resident * per * tu + 1.5);
     if (left) t += (left > cus ? 2 : 1) * per * tu + 1.5;
     t += ks > 1 ? 1.0 + (double)ks * M * N * 8 / 4e6 : 0.0;
-    if (best_per == 0 || t < best) best = t, best_per = per, best_lds = lds;
+    if (best.per == 0 || t < best_us) best_us = t, best.per = per, best.lds = lds;
   }
-  if (best_per == 0) return fail(CTHIP_E_STATE, "linear rows: no share of (%d, %d, %d blocks) fits", M, N, a.kblocks);
-  a.kper = best_per * UB;
-  const int ks = (units + best_per - 1) / best_per;
+  return best;
+}
+
+template <int SRC, int NPA, int MB, bool WIDE_D>
+static int rows_launch(RowsGemmArgs a) {
+  constexpr int NS = kRowsNS, NW = 4 * MB, PD = kRowsPD, NT = rows_columns(MB), T = 64 * NW, UB = rows_unit_blocks(SRC);
+  const int M = a.e.M, N = a.e.N, groups = (N + NT - 1) / NT, units = (a.kblocks + UB - 1) / UB;
+  const RowsShare share = rows_share(SRC, NPA, MB, WIDE_D, M, N, a.kblocks);
+  if (share.per == 0) return fail(CTHIP_E_STATE, "linear rows: no share of (%d, %d, %d blocks) fits", M, N, a.kblocks);
+  a.kper = share.per * UB;
+  const int ks = (units + share.per - 1) / share.per;
   a.parts = nullptr;
   int rc = 0;
   if (ks > 1 && (rc = alloc_scratch((void **)&a.parts, sizeof(float) * (size_t)groups * ks * M * NT))) return rc;
@@ -485,7 +499,7 @@ static int rows_launch(RowsGemmArgs a) {
     CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 157 * 1024));
     big_lds = true;
   }
-  hipLaunchKernelGGL(fn, dim3(groups, ks), dim3(T), best_lds, state().stream, a);
+  hipLaunchKernelGGL(fn, dim3(groups, ks), dim3(T), share.lds, state().stream, a);
   const hipError_t e = hipGetLastError();
   if (a.parts) rc = cthip_free(a.parts);  // stream-ordered: handed out again only to later work on this stream
   if (e != hipSuccess) return fail((int)e, "linear rows: launch -> %s", hipGetErrorString(e));
@@ -505,7 +519,11 @@ static void rows_planes_launch(const RowsPlanesArgs &a, int m) {
 #undef RP
 }
 
-// Whether this is the launch to take: the operands are laid out for it, and it is the faster one.
+static int rows_source(const WMat *w) { return w->type == CTHIP_Q8_0 ? RW_Q8 : w->type == CTHIP_Q4_0 ? RW_Q4 : w->type == CTHIP_F16 ? RW_F16 : RW_F32; }
+static int rows_terms(int m, int precision) { return m < 8 || precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1; }
+static bool rows_wide_scales(const WMat *w) { return w->cols / 32 % 2 == 0 && rows_quant(rows_source(w)); }
+
+// Whether this is the launch to take: the operands are laid out for it, a share of it fits a workgroup, and it is the faster one.
 // Fewer than 8 rows: against the single-row kernels, one pass over the weights per row.  They cost about 3 us + m weights
 // at 4.3 (quantised), 2.7 (fp16) or 2.0 (fp32) per ns, the two launches here 9.5 us + the weights once at 3.2 / 2.3 / 1.15.
 //   us, m = 3 / 5 / 7:  4096 x 4096 Q8_0 17 / 20 / 29 -> 12 / 14 / 14;  22016 x 4096 Q8_0 52 / 80 / 110 -> 31 / 39 / 41;
@@ -522,10 +540,11 @@ bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, in
   const bool quant = w->type == CTHIP_Q8_0 || w->type == CTHIP_Q4_0;
   if (m < 8) {
     const double each = quant ? 4.3 : w->type == CTHIP_F16 ? 2.7 : 2.0, once = quant ? 3.2 : w->type == CTHIP_F16 ? 2.3 : 1.15;
-    return 3000 + m * weights / each > 9500 + weights / once;
+    if (3000 + m * weights / each <= 9500 + weights / once) return false;
+  } else if (w->type == CTHIP_F32 || (m <= 16 ? weights < (quant ? 22e3 : 20e3) : quant || weights < 60e3)) {
+    return false;
   }
-  if (w->type == CTHIP_F32) return false;
-  return m <= 16 ? weights >= (quant ? 22e3 : 20e3) : w->type == CTHIP_F16 && weights >= 60e3;
+  return rows_share(rows_source(w), rows_terms(m, precision), m <= 16 ? 1 : 2, rows_wide_scales(w), m, (int)w->rows, (int)((w->cols + 31) / 32)).per > 0;
 }
 
 // rows with what a Linear has in front of it as bf16 planes for gemm_planes.hip (x on 16 bytes, K % 32 == 0)
@@ -543,9 +562,9 @@ int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, cons
 // launch_linear_gemm.  Call only where linear_rows_pays.
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route) {
-  const int terms = m < 8 ? 3 : precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1;
+  const int terms = rows_terms(m, precision);
   const bool half = w->type != CTHIP_F32;
-  const int ub = w->type == CTHIP_Q8_0 ? RowsUnit<RW_Q8>::BLOCKS : w->type == CTHIP_Q4_0 ? RowsUnit<RW_Q4>::BLOCKS : RowsUnit<RW_F16>::BLOCKS;
+  const int ub = rows_unit_blocks(rows_source(w));
   RowsGemmArgs a = {};
   a.kblocks = (int)((w->cols + 31) / 32);
   a.nkb = (a.kblocks + ub - 1) / ub * ub;
@@ -596,7 +615,7 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
   }
 #undef RP2
 #undef RP3
-  const bool wide = a.dpitch % 2 == 0;
+  const bool wide = rows_wide_scales(w);
 #define RL4(SRC, NPA, WD)                                  \
   do {                                                     \
     if (m <= 16) rc = rows_launch<SRC, NPA, 1, WD>(a);     \

@@ -54,6 +54,33 @@ def test_linear_rows(ops, kind, rows, cols, m, prologue):
     w.free()
 
 
+@pytest.mark.parametrize("kind,rows,cols,m,precision", [
+    ("f16", 2100, 28672, 27, 2), ("f16", 2100, 28672, 32, 2), ("f16", 2100, 28672, 18, 3), ("f16", 2100, 28672, 32, 3), ("f16", 2050, 29568, 25, 2),
+    ("f16", 2500, 24576, 31, 2), ("q4_0", 4098 * 128, 2240, 16, 2), ("f16", 2100, 28672, 17, 2), ("f16", 2100, 28672, 16, 2), ("q8_0", 1700, 28672, 16, 3)])
+def test_wide_rows_and_many_columns(ops, oracle, kind, rows, cols, m, precision):
+    """Matrices whose rows no share of a workgroup's memory holds, whether for their width or because more column groups than
+    tickets allow one share only: another launch takes them.  The last three are of this kernel's."""
+    from caten_amd import _lib
+    lib = _lib.init(0)
+    rng = np.random.default_rng(rows + m)
+    base = min(rows, 4098)
+    raw = packed(kind, rng.normal(0, 0.05, (base, cols)).astype(np.float32))
+    w = ops.WeightMatrix(kind, np.tile(np.ascontiguousarray(raw).view(np.uint8).ravel(), rows // base), rows, cols)
+    x = rng.normal(0, 1, (m, cols)).astype(np.float32)
+    at = np.unique(np.r_[0:40, base - 40:base, rng.integers(0, base, 100)])
+    dense = ops.WeightMatrix(kind, raw, base, cols)
+    want = x.astype(np.float64) @ dense.dequantize()[at].astype(np.float64).T
+    dense.free()
+    try:
+        _lib.check(lib.cthip_set_option(b"gemm_precision", precision))
+        got = ops.linear(x, w)
+    finally:
+        _lib.check(lib.cthip_set_option(b"gemm_precision", 2))
+    for first in {0, rows - base}:
+        assert np.linalg.norm(got[:, first + at] - want) < 1e-5 * np.linalg.norm(want)
+    w.free()
+
+
 @pytest.mark.parametrize("rows", [2, 3, 7])
 def test_short_prompt_equals_its_rows_one_by_one(ops, rows):
     from caten_amd import _lib, llm, synth
