@@ -50,6 +50,8 @@ struct State {
 State &state();
 // cthip_alloc without the zero fill, for temporaries that are fully written before they are read
 int alloc_scratch(void **out, size_t bytes);
+// the same for what is only kept to be faster: refused rather than taking the last memory from others
+int alloc_spare(void **out, size_t bytes);
 bool device_readable(const void *p);
 void set_error(const char *fmt, ...);
 int fail(int code, const char *fmt, ...);
@@ -91,6 +93,7 @@ struct WMat {
   // the matrix as bf16 terms, made by the first Linear over many rows that wants them (gemm_planes.hip)
   void *planes = nullptr;
   int64_t planes_bytes = 0;
+  int planes_users = 0;  // launches being put together from them; they are not given back meanwhile
 };
 // gfx950: 256 MB of Infinity Cache in front of HBM
 static const int64_t kInfinityCacheBytes = 256ll << 20;
@@ -271,7 +274,13 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
 // A Linear over many rows through the same kernel: x as fp32 rows or already as planes of plane_terms(precision) terms, the
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
 bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in);
-bool linear_planes_ready(const WMat *w, int m, int precision);  // x in planes certainly runs
+// x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
+bool linear_planes_ready(const WMat *w, int m, int precision);
+void weight_planes_release(const WMat *w);
+// The terms of all matrices together are kept up to this many bytes.  They are given back where memory is short, by
+// cthip_cache_trim and by a lower limit; weight_planes_drop returns whether there were any.
+void weight_planes_limit(int64_t bytes);
+bool weight_planes_drop();
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
                          int precision, const GemmRoute *route, unsigned char *planes_out, bool *done);
 bool rows_planes_supported(int K);

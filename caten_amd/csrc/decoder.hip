@@ -21,6 +21,7 @@
 // prefill(): MFMA GEMMs over 8 rows and more, fp32-grade Linears over fewer); two rows over
 // three-launch layers are fed row by row through the decode step (causal attention makes that the
 // same function).  Either way only the last row runs lm_head and argmax.
+#include <algorithm>
 #include <stdlib.h>
 #include <string.h>
 
@@ -917,6 +918,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   int *ids_dev = nullptr;
   AttnSplit split = {1, nullptr, nullptr}, last_split = {1, nullptr, nullptr};
   std::vector<void *> tmp;
+  std::vector<const WMat *> held;  // matrices whose terms a Linear further down counts on
   auto alloc = [&](void **p, size_t bytes) {
     int r = alloc_scratch(p, bytes);  // every temporary below is fully written before it is read
     if (r == 0) tmp.push_back(*p);
@@ -964,7 +966,11 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // a row of terms is as long as the fp32 row whose buffer it takes.  (A session with a quantised cache keeps the
     // order of summation of the tiles: a rounding step of a cached value is a hundred times what a sum is off by.)
     const bool planes = !d->kvq && prec == GEMM_BF16X3_DEFAULT && s >= 64 && rows_planes_supported(D) && F % 32 == 0;
-    auto in_planes = [&](const WMat *w) { return planes && w && linear_planes_ready(w, R, prec); };
+    auto in_planes = [&](const WMat *w) {
+      if (!planes || !w || !linear_planes_ready(w, R, prec)) return false;
+      held.push_back(w);
+      return true;
+    };
     // y = norm(x), as terms where the Linear behind it takes them
     auto norm = [&](float *y, const float *x, const float *g, const float *b, bool terms) {
       if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps);
@@ -977,6 +983,10 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         bool taken = false;
         const int r = launch_linear_planes(out_terms ? nullptr : y, w, in_terms ? nullptr : in, in_terms ? (const unsigned char *)in : nullptr, R, bias,
                                            residual, act, prec, route, out_terms ? (unsigned char *)y : nullptr, &taken);
+        if (in_terms) {  // no more than a layer's matrices are held at a time
+          held.erase(std::find(held.begin(), held.end(), w));
+          weight_planes_release(w);
+        }
         if (taken) return r;
         if (in_terms || out_terms) return fail(CTHIP_E_STATE, "prompt: a Linear of %lld x %lld over %d rows cannot take its input as terms", (long long)w->rows, (long long)w->cols, R);
       }
@@ -1066,6 +1076,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   TRY(queue_head(d));
 #undef TRY
 done:
+  for (const WMat *w : held) weight_planes_release(w);
   for (void *p : tmp) cthip_free(p);
   return rc;
 }

@@ -11,6 +11,7 @@
 // bf16 (term 0 = bf16(x), term p = bf16 of what terms 0..p-1 miss).  A K-step of a row is one contiguous piece of NP * 64
 // bytes: whole cache lines for NP = 2.
 #include <mutex>
+#include <unordered_set>
 
 #include "common.h"
 #include "planes.h"
@@ -528,12 +529,13 @@ bool matmul_planes_pay(int M, int N, int K, int precision) {
 
 // ---- Linears over many rows ----
 // A weight matrix as planes: one of integers for a quantised matrix (2 bytes per weight), two exact terms for fp16 (4).
-// The first Linear that wants them makes them and they stay with the matrix, up to kWeightPlanesMax for all matrices together
-// (what a 16-bit model of 16e9 weights takes, a ninth of the card); past that, for fp32 matrices and for a single term of
-// an fp16 one they are made again by every call, 3 - 8 bytes of traffic per weight.
-static const int64_t kWeightPlanesMax = 32ll << 30;
-static std::mutex g_weight_planes_mu;
-static int64_t g_weight_planes_bytes = 0;
+// The first Linear that wants them makes them and they stay with the matrix, up to a limit for all matrices together
+// (option "weight_planes"; what a 16-bit model of 16e9 weights takes, a ninth of the card), as long as a sixteenth of the card
+// stays free; they go with the matrix, when an allocation fails, with cthip_cache_trim and with a lower limit.  Past that, for
+// fp32 matrices and for a single term of an fp16 one they are made again by every call, 3 - 8 bytes of traffic per weight.
+static std::mutex g_planes_mu;  // guards the fields planes* of every matrix, and:
+static int64_t g_planes_limit = 32ll << 30, g_planes_bytes = 0;
+static std::unordered_set<WMat *> g_planes_of;
 
 static bool is_quant(const WMat *w) { return w->type == CTHIP_Q8_0 || w->type == CTHIP_Q4_0; }
 static int weight_terms(const WMat *w, int terms) { return is_quant(w) ? 1 : w->type == CTHIP_F16 && terms > 2 ? 2 : terms; }
@@ -552,35 +554,72 @@ static int make_weight_planes(unsigned char *out, const WMat *w, int terms_b) {
   CTHIP_LAUNCH_CHECK();
   return 0;
 }
-// *temp: the caller frees the planes after its launch.  null: no memory for them.
+// The terms for one launch, null where there is no memory for them.  *temp: the caller frees them after its launch, else it
+// calls weight_planes_release.
 static const unsigned char *weight_planes(const WMat *w, int terms_b, bool *temp) {
-  std::lock_guard<std::mutex> lk(g_weight_planes_mu);
+  std::lock_guard<std::mutex> lk(g_planes_mu);
+  WMat *m = const_cast<WMat *>(w);
   *temp = false;
   const int64_t bytes = weight_plane_bytes(w, terms_b);
   const bool stay = weight_planes_stay(w, terms_b);
-  if (stay && w->planes) return (const unsigned char *)w->planes;
+  if (stay && w->planes) {
+    m->planes_users++;
+    return (const unsigned char *)w->planes;
+  }
   unsigned char *p = nullptr;
-  if (bytes > kWeightPlanesMax || alloc_scratch((void **)&p, (size_t)bytes)) return nullptr;
+  if (alloc_spare((void **)&p, (size_t)bytes)) return nullptr;
   if (make_weight_planes(p, w, terms_b)) {
     cthip_free(p);
     return nullptr;
   }
-  if (stay && g_weight_planes_bytes + bytes <= kWeightPlanesMax) {
-    WMat *m = const_cast<WMat *>(w);
+  if (stay && g_planes_bytes + bytes <= g_planes_limit) {
     m->planes = p;
     m->planes_bytes = bytes;
-    g_weight_planes_bytes += bytes;
+    m->planes_users = 1;
+    g_planes_bytes += bytes;
+    g_planes_of.insert(m);
   } else {
     *temp = true;
   }
   return p;
 }
-void wmat_drop_planes(WMat *w) {
-  std::lock_guard<std::mutex> lk(g_weight_planes_mu);
-  if (!w->planes) return;
+void weight_planes_release(const WMat *w) {
+  std::lock_guard<std::mutex> lk(g_planes_mu);
+  const_cast<WMat *>(w)->planes_users--;
+}
+static void planes_give_back(WMat *w) {  // (stream-ordered: the block goes to later work on this stream only)
   cthip_free(w->planes);
-  g_weight_planes_bytes -= w->planes_bytes;
+  g_planes_bytes -= w->planes_bytes;
   w->planes = nullptr;
+}
+void wmat_drop_planes(WMat *w) {
+  std::lock_guard<std::mutex> lk(g_planes_mu);
+  if (!w->planes) return;
+  planes_give_back(w);
+  g_planes_of.erase(w);
+}
+bool weight_planes_drop() {
+  std::lock_guard<std::mutex> lk(g_planes_mu);
+  bool any = false;
+  for (auto it = g_planes_of.begin(); it != g_planes_of.end();) {
+    if ((*it)->planes_users) {
+      ++it;
+      continue;
+    }
+    planes_give_back(*it);
+    it = g_planes_of.erase(it);
+    any = true;
+  }
+  return any;
+}
+void weight_planes_limit(int64_t bytes) {
+  bool over;
+  {
+    std::lock_guard<std::mutex> lk(g_planes_mu);
+    g_planes_limit = bytes;
+    over = g_planes_bytes > bytes;
+  }
+  if (over) weight_planes_drop();
 }
 
 // What launch_gemm takes: 64 x 128 tiles of a quantised matrix, one workgroup per compute unit.
@@ -604,7 +643,7 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
   return planes_pay(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes, linear_tiles_us(w, m, terms));
 }
-// ... and nothing can be in the way of it: the matrix has its planes (made here if need be)
+// ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {
   if (!linear_planes_pays(w, m, precision, true)) return false;
   const int terms_b = weight_terms(w, plane_terms(precision));
@@ -661,6 +700,7 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
   if (!rc) rc = planes_gemm(a, terms, terms_b, nullptr);
   cthip_free(tmp);  // stream-ordered: handed out again only to later work on this stream
   if (temp_b) cthip_free(const_cast<unsigned char *>(pb));
+  else weight_planes_release(w);
   return rc;
 }
 

@@ -815,6 +815,11 @@ int cthip_set_option(const char *name, int value) {
     state().kv_cache = value;
     return 0;
   }
+  if (!strcmp(name, "weight_planes")) {
+    if (value < 0) return fail(CTHIP_E_BAD_ARG, "cthip_set_option: weight_planes is a limit in MiB");
+    weight_planes_limit((int64_t)value << 20);
+    return 0;
+  }
   if (!strcmp(name, "decode_skip")) {
     if (value < 0 || value > 31) return fail(CTHIP_E_BAD_ARG, "cthip_set_option: decode_skip is a mask of 5 bits");
     state().decode_skip = value;

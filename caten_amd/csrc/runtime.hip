@@ -188,9 +188,28 @@ bool cthip::device_readable(const void *p) {
   return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged || attr.type == hipMemoryTypeHost;
 }
 
-// a block of the caching allocator with whatever its last owner left in it (temporaries that are
-// fully written before they are read); released with cthip_free like any other block
-int cthip::alloc_scratch(void **out, size_t bytes) {
+// gives the cached blocks back to the driver (queued work may still read them: the stream is waited for)
+static int trim_blocks() {
+  CTHIP_CHECK(hipStreamSynchronize(state().stream));
+  Allocator &a = allocator();
+  std::lock_guard<std::mutex> lk(a.mu);
+  for (auto &kv : a.cache)
+    for (void *p : kv.second) (void)hipFree(p);
+  a.cache.clear();
+  a.cached_bytes = 0;
+  return 0;
+}
+
+// hipMalloc; an error is not left behind for the next launch check to report
+static hipError_t driver_alloc(void **p, size_t cls) {
+  const hipError_t e = hipMalloc(p, cls);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
+// needed: when the driver has no memory left, give back what is only kept to be faster (cached blocks, then the weights'
+// terms of gemm_planes.hip) and try again.  Otherwise a block is taken only where that leaves a sixteenth of the card free.
+static int take_block(void **out, size_t bytes, bool needed) {
   CTHIP_REQUIRE_INIT();
   CTHIP_ARG(out != nullptr);
   size_t cls = size_class(bytes);
@@ -206,11 +225,21 @@ int cthip::alloc_scratch(void **out, size_t bytes) {
     }
   }
   if (!p) {
-    hipError_t e = hipMalloc(&p, cls);
-    if (e != hipSuccess) {  // give cached blocks back to the driver and retry once
-      (void)hipGetLastError();
-      cthip_cache_trim();
-      e = hipMalloc(&p, cls);
+    hipError_t e = hipErrorOutOfMemory;
+    if (needed) {
+      e = driver_alloc(&p, cls);
+      if (e != hipSuccess) {
+        trim_blocks();
+        e = driver_alloc(&p, cls);
+      }
+      if (e != hipSuccess && weight_planes_drop()) {
+        trim_blocks();
+        e = driver_alloc(&p, cls);
+      }
+    } else {
+      size_t free_bytes = 0, total = 0;
+      if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) (void)hipGetLastError();
+      else if (free_bytes >= cls + total / 16) e = driver_alloc(&p, cls);
     }
     if (e != hipSuccess) return fail((int)e, "cthip_alloc: hipMalloc(%zu) -> %s", cls, hipGetErrorString(e));
     std::lock_guard<std::mutex> lk(a.mu);
@@ -224,6 +253,11 @@ int cthip::alloc_scratch(void **out, size_t bytes) {
   *out = p;
   return 0;
 }
+
+// a block of the caching allocator with whatever its last owner left in it (temporaries that are
+// fully written before they are read); released with cthip_free like any other block
+int cthip::alloc_scratch(void **out, size_t bytes) { return take_block(out, bytes, true); }
+int cthip::alloc_spare(void **out, size_t bytes) { return take_block(out, bytes, false); }
 
 extern "C" {
 
@@ -252,14 +286,8 @@ int cthip_free(void *p) {
 
 int cthip_cache_trim(void) {
   CTHIP_REQUIRE_INIT();
-  CTHIP_CHECK(hipStreamSynchronize(state().stream));
-  Allocator &a = allocator();
-  std::lock_guard<std::mutex> lk(a.mu);
-  for (auto &kv : a.cache)
-    for (void *p : kv.second) (void)hipFree(p);
-  a.cache.clear();
-  a.cached_bytes = 0;
-  return 0;
+  weight_planes_drop();
+  return trim_blocks();
 }
 
 int cthip_cache_stats(size_t *live_bytes, size_t *cached_bytes, size_t *driver_allocs) {

@@ -66,7 +66,8 @@ int cthip_device_info(char *name, int name_cap, int *compute_units, int *wave_si
 int cthip_alloc(void **out, size_t bytes);
 /* close-buffer (buffer.lisp:81): returns the block to the cache. NULL is a no-op. */
 int cthip_free(void *p);
-/* Releases all cached (unused) blocks back to the driver. */
+/* Releases all cached (unused) blocks back to the driver, and what is kept of weights only to be faster
+ * (option "weight_planes"). */
 int cthip_cache_trim(void);
 int cthip_cache_stats(size_t *live_bytes, size_t *cached_bytes, size_t *driver_allocs);
 
@@ -272,6 +273,13 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  *   2 = fp32 rows in pages of cthip_kv_page_rows() rows per layer, opened when the position first reaches them
  *   (a session then holds the rows it has used instead of max_seq rows); such a session runs one launch per
  *   Linear; tokens and logits are those of the dense cache.
+ * "weight_planes": MiB (default 32768).  A Linear over 64 rows and more, a long prompt's among them, may take its
+ *   weights as bf16 terms; a quantised matrix (2 bytes per weight, beside its 1.06 or 0.56) and an fp16 one (4 bytes)
+ *   keep theirs from the first such call on, up to this limit for all matrices of the process together and as long as
+ *   a sixteenth of the device memory stays free: a 7B model of 4 bits holds 4 GB before its first long prompt and 17 behind it.
+ *   They are given back when a matrix is destroyed, by cthip_cache_trim, by an allocation here that finds no memory,
+ *   and by a lower limit; 0 = none are kept.  Results do not depend on it where the same launch is chosen; past the
+ *   limit the terms are made by every call that still pays with them.
  * "decode_skip": knock-out timing of the three-launch decode step -- a mask of launches a session created
  *   afterwards leaves out (1 qkv, 2 attention + projection, 4 MLP, 8 the sum in front of lm_head,
  *   16 lm_head + argmax).  Tokens and logits of such a session are meaningless; 0 (default) = none.

@@ -1,6 +1,8 @@
 """Products over operands split into bf16 terms once (csrc/gemm_planes.hip), at sizes where each of its tiles is chosen:
 edges that no tile divides, a last block of k that is part empty, rows that are no multiple of 16 bytes; the Linears and
 prompts that take it."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -90,3 +92,61 @@ def test_long_prompt_attention_equals_short_pieces(ops, heads, kv_heads, first, 
         assert t0 == t1
         assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
     model.close()
+
+
+def allocated(lib):
+    """bytes in use, blocks asked of the driver so far"""
+    from caten_amd import _lib
+    live, cached, drv = C.c_size_t(), C.c_size_t(), C.c_size_t()
+    _lib.check(lib.cthip_cache_stats(C.byref(live), C.byref(cached), C.byref(drv)))
+    return live.value, drv.value
+
+
+def matrix(ops, kind, rows, cols, seed):
+    from caten_amd.llm import Tensor
+    rng = np.random.default_rng(seed)
+    return ops.WeightMatrix(kind, Tensor.from_f32(rng.normal(0, 0.05, (rows, cols)).astype(np.float32), kind).raw, rows, cols)
+
+
+def test_weight_terms_are_bounded_and_given_back(ops):
+    """Option "weight_planes" bounds what matrices keep; cthip_cache_trim, a lower limit, an allocation that finds no memory and the
+    end of a matrix give it back, and the next call makes the terms again with the same result."""
+    from caten_amd import HipError, _lib
+    lib = _lib.init(0)
+    a, b = matrix(ops, "q8_0", 5001, 2048, 1), matrix(ops, "q8_0", 11270, 2080, 2)
+    a_bytes, b_bytes = 5001 * 64 * 64, 11270 * 65 * 64  # 20.5 + 46.9 MB
+    x, y = (np.random.default_rng(3).normal(0, 1, (3000, n)).astype(np.float32) for n in (2048, 2080))  # rows that pay for the terms at every call
+    try:
+        _lib.check(lib.cthip_set_option(b"weight_planes", 0))
+        none = allocated(lib)[0]
+        ra, rb = ops.linear(x, a), ops.linear(y, b)
+        assert allocated(lib)[0] == none
+        _lib.check(lib.cthip_set_option(b"weight_planes", 64))  # room for one of them
+        same = lambda: np.array_equal(ops.linear(x, a), ra) and np.array_equal(ops.linear(y, b), rb)
+        assert same()
+        kept = allocated(lib)[0] - none
+        assert a_bytes <= kept < b_bytes
+        assert same() and allocated(lib)[0] - none == kept
+        _lib.check(lib.cthip_cache_trim())
+        assert allocated(lib)[0] == none
+        assert same() and allocated(lib)[0] - none == kept
+        p = C.c_void_p()
+        with pytest.raises(HipError, match="hipMalloc"):
+            _lib.check(lib.cthip_alloc(C.byref(p), 1 << 50))
+        assert allocated(lib)[0] == none
+        assert same() and allocated(lib)[0] - none == kept  # (and the failed call's error is not found by a later launch)
+        _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
+        assert same() and a_bytes + b_bytes <= allocated(lib)[0] - none
+        _lib.check(lib.cthip_set_option(b"weight_planes", 8))
+        assert allocated(lib)[0] == none
+        assert same() and allocated(lib)[0] == none
+        _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
+        assert same()
+        both = allocated(lib)[0]
+        a.free()
+        assert allocated(lib)[0] <= both - a_bytes - 5001 * 2048
+        with pytest.raises(HipError, match="weight_planes"):
+            _lib.check(lib.cthip_set_option(b"weight_planes", -1))
+    finally:
+        _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
+    b.free()
