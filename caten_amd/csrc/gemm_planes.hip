@@ -554,33 +554,41 @@ static int make_weight_planes(unsigned char *out, const WMat *w, int terms_b) {
   CTHIP_LAUNCH_CHECK();
   return 0;
 }
-// The terms for one launch, null where there is no memory for them.  *temp: the caller frees them after its launch, else it
-// calls weight_planes_release.
+// Whether they are there or the next call's stay (with g_planes_mu held)
+static bool weight_planes_room(const WMat *w, int terms_b) {
+  return weight_planes_stay(w, terms_b) && (w->planes || g_planes_bytes + weight_plane_bytes(w, terms_b) <= g_planes_limit);
+}
+static bool weight_planes_kept(const WMat *w, int terms_b) {
+  std::lock_guard<std::mutex> lk(g_planes_mu);
+  return weight_planes_room(w, terms_b);
+}
+// The terms for one launch, null where there is no memory for them (or for terms that stay, where temp is null).  *temp:
+// the caller frees them after its launch, else it calls weight_planes_release.
 static const unsigned char *weight_planes(const WMat *w, int terms_b, bool *temp) {
   std::lock_guard<std::mutex> lk(g_planes_mu);
   WMat *m = const_cast<WMat *>(w);
-  *temp = false;
   const int64_t bytes = weight_plane_bytes(w, terms_b);
-  const bool stay = weight_planes_stay(w, terms_b);
+  const bool stay = weight_planes_room(w, terms_b);
   if (stay && w->planes) {
     m->planes_users++;
+    if (temp) *temp = false;
     return (const unsigned char *)w->planes;
   }
+  if (!stay && !temp) return nullptr;
   unsigned char *p = nullptr;
   if (alloc_spare((void **)&p, (size_t)bytes)) return nullptr;
   if (make_weight_planes(p, w, terms_b)) {
     cthip_free(p);
     return nullptr;
   }
-  if (stay && g_planes_bytes + bytes <= g_planes_limit) {
+  if (stay) {
     m->planes = p;
     m->planes_bytes = bytes;
     m->planes_users = 1;
     g_planes_bytes += bytes;
     g_planes_of.insert(m);
-  } else {
-    *temp = true;
   }
+  if (temp) *temp = !stay;
   return p;
 }
 void weight_planes_release(const WMat *w) {
@@ -639,19 +647,13 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   if (is_quant(w) && precision == GEMM_BF16X6) return false;
   const int terms = plane_terms(precision), terms_b = weight_terms(w, terms);
   double bytes = 0.0;
-  if (!weight_planes_stay(w, terms_b)) bytes = (double)w->rows * w->cols * (w->type == CTHIP_F16 ? 2.0 : 4.0) + weight_plane_bytes(w, terms_b);
+  if (!weight_planes_kept(w, terms_b)) bytes = (double)w->q_bytes + weight_plane_bytes(w, terms_b);
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
   return planes_pay(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes, linear_tiles_us(w, m, terms));
 }
 // ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {
-  if (!linear_planes_pays(w, m, precision, true)) return false;
-  const int terms_b = weight_terms(w, plane_terms(precision));
-  if (!weight_planes_stay(w, terms_b)) return false;
-  bool temp = false;
-  const unsigned char *p = weight_planes(w, terms_b, &temp);
-  if (temp) cthip_free(const_cast<unsigned char *>(p));
-  return p && !temp;
+  return linear_planes_pays(w, m, precision, true) && weight_planes(w, weight_terms(w, plane_terms(precision)), nullptr);
 }
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
                          int precision, const GemmRoute *route, unsigned char *planes_out, bool *done) {

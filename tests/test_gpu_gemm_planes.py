@@ -95,11 +95,11 @@ def test_long_prompt_attention_equals_short_pieces(ops, heads, kv_heads, first, 
 
 
 def allocated(lib):
-    """bytes in use, blocks asked of the driver so far"""
+    """bytes in use, bytes taken from the driver"""
     from caten_amd import _lib
     live, cached, drv = C.c_size_t(), C.c_size_t(), C.c_size_t()
     _lib.check(lib.cthip_cache_stats(C.byref(live), C.byref(cached), C.byref(drv)))
-    return live.value, drv.value
+    return live.value, live.value + cached.value
 
 
 def matrix(ops, kind, rows, cols, seed):
@@ -150,3 +150,31 @@ def test_weight_terms_are_bounded_and_given_back(ops):
     finally:
         _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
     b.free()
+
+
+@pytest.mark.parametrize("kind,rows", [("q4_0", 200), ("q8_0", 200), ("f16", 260)])
+def test_prompt_without_room_for_weight_terms(ops, kind, rows):
+    """Past the limit a Linear takes terms only where making them at every call pays, and none are made to be thrown away: at
+    these rows the gate|up matrix is faster with kept terms and slower with its own."""
+    from caten_amd import _lib, llm, synth
+    lib = _lib.init(0)
+    cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=2048, n_heads=32, n_kv_heads=4, ffn=5632, n_layers=2, vocab=500, max_seq=1024)
+    model = llm.make_llama(cfg, llm.llama_state_dict(synth.llama_weights(cfg, seed=5), kind))
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], rows, seed=5)]
+    model.forward(ids[:8], 8, 0)
+    try:
+        _lib.check(lib.cthip_set_option(b"weight_planes", 0))
+        _lib.check(lib.cthip_cache_trim())
+        before = allocated(lib)[1]
+        t0, l0 = model.forward(ids, rows, 0, return_logits=True)
+        taken = allocated(lib)[1] - before
+        terms = 11264 * 2048 * (4 if kind == "f16" else 2)  # of the gate|up matrix
+        assert taken < terms, (taken, terms)
+    finally:
+        _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
+    live = allocated(lib)[0]
+    t1, l1 = model.forward(ids, rows, 0, return_logits=True)
+    assert allocated(lib)[0] - live >= terms
+    assert t0 == t1
+    assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
+    model.close()
