@@ -9,17 +9,16 @@
 // terms by a small launch in front (k_rows_planes, which also applies the norm or SwiGLU), wait in LDS for the workgroup's
 // share of k.  (Every workgroup splitting its own share of the rows saved that launch and cost 5 us per workgroup.)
 //
-// Terms are fp16 where the weights are: a quantised weight is an integer times its block's scale and an fp16 weight is what
-// it is, so the weight operand is exact and costs little more than one vector instruction a pair (Q8_0), or none (fp16).  The
-// inputs are scaled by a power of two per row (their largest below 2^15; undone at the end), so that two terms
-// hold 22 bits of every value that matters and three hold all 24.  A block's scale is applied to its partial sum.  fp32
-// weights are split like the inputs, into bf16 terms, which have their range.
-// Terms per input: three for fewer than 8 rows (what the single-row kernels give), else what "gemm_precision" says.
+// Terms are bf16: they have the range of a float, so that an input keeps its bits whatever the largest of its row is (a row of a
+// model with outlier channels spans more than the 2^39 of scaled fp16 terms).  Three of them hold all 24 bits.  A quantised
+// weight is an integer, exact in bf16, times its block's scale, which is applied to the block's partial sum; an fp16 weight
+// is two terms, exact; an fp32 weight three.  Products of terms below 2^-24 of the leading one are left out.
+// An infinity or a NaN stands in the last term, which meets the leading term of a weight only (infinity times a lower
+// term of zero would be NaN): it comes out as it does of fp32 products.
+// Three terms per input, two where "gemm_precision" asks for operands rounded to bf16.
 //
 // K is shared among as many workgroups as fill the chip; a share leaves its partial sums in memory and draws a ticket, the
 // last one of a column group adds them in share order and stores the result (bias, activation, residual, routes).
-#include <type_traits>
-
 #include "common.h"
 #include "planes.h"
 
@@ -27,7 +26,6 @@ namespace cthip {
 
 struct RowsGemmArgs {
   const unsigned char *A;    // planes of the input rows: [M][nkb][NPA][32], nkb = whole units (zeros past K)
-  const float *rscale;       // per input row: what undoes its scaling (null for bf16 terms)
   int nkb;
   const unsigned char *W;    // N rows of packed weights, wpitch = wbytes apart
   const unsigned short *wd;  // scales, dpitch apart
@@ -37,40 +35,33 @@ struct RowsGemmArgs {
   PlaneGemmArgs e;           // M, N and what happens to the result
 };
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-// two bytes of v as fp16 integers less `bias`: 0x64 in front of a byte is 1024 + byte
-__device__ __forceinline__ unsigned half2_of_bytes(unsigned v, unsigned sel, float bias) {
-  const v2h x = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, v, sel));
-  const _Float16 b = (_Float16)(-1024.0f - bias);
-  return __builtin_bit_cast(unsigned, x + v2h{b, b});
+template <bool SIGNED>  // 8 int8 -> bf16 (SIGNED), or 8 nibbles (a byte each) - 8
+__device__ __forceinline__ v8bf bf_of_bytes(unsigned a, unsigned b) {
+  if (!SIGNED) a = (a + 0x78787878u) ^ 0x80808080u, b = (b + 0x78787878u) ^ 0x80808080u;  // per byte: nibble - 8 as int8 (no carry leaves a byte)
+  return bf_of_q8(a, b);
 }
-template <bool SIGNED>  // 8 int8 -> fp16 (SIGNED), or 8 nibbles (a byte each) - 8
-__device__ __forceinline__ v8h h_of_bytes(unsigned a, unsigned b) {
-  constexpr float bias = SIGNED ? 128.0f : 8.0f;
-  if (SIGNED) a ^= 0x80808080u, b ^= 0x80808080u;
-  return __builtin_bit_cast(v8h, make_uint4(half2_of_bytes(a, 0x04010400u, bias), half2_of_bytes(a, 0x04030402u, bias),
-                                            half2_of_bytes(b, 0x04010400u, bias), half2_of_bytes(b, 0x04030402u, bias)));
-}
-// 8 floats -> NP fp16 terms (of values below 2^15), each of what the terms before it miss
+// 8 floats -> NP terms, each of what the terms before it miss
 template <int NP>
-__device__ __forceinline__ void split8_half(const float *v, uint4 *pl) {
-  float r[8];
+__device__ __forceinline__ void split8_rows(const float *v, uint4 *pl) {
+  constexpr float kLargest = 3.38953139e38f;  // of bf16: what a float above it has more goes to the next term
+  float r[8], t[8];
 #pragma unroll
-  for (int e = 0; e < 8; e++) r[e] = v[e];
+  for (int e = 0; e < 8; e++) r[e] = fabsf(v[e]) < INFINITY ? v[e] : 0.0f;
 #pragma unroll
   for (int p = 0; p < NP; p++) {
-    v8h h;
+    unsigned w[4];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      h[e] = (_Float16)r[e];
-      r[e] -= (float)h[e];
+    for (int e = 0; e < 8; e++) t[e] = p == 0 ? fminf(fmaxf(r[e], -kLargest), kLargest) : p + 1 == NP && !(fabsf(v[e]) < INFINITY) ? v[e] : r[e];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      w[e] = pack_bf16_pl(t[2 * e], t[2 * e + 1]);
+      r[2 * e] -= __uint_as_float(w[e] << 16);  // exact: the difference of a float and its own leading bits
+      r[2 * e + 1] -= __uint_as_float(w[e] & 0xffff0000u);
     }
-    pl[p] = __builtin_bit_cast(uint4, h);
+    pl[p] = make_uint4(w[0], w[1], w[2], w[3]);
   }
 }
 typedef float v4f __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ v4f mma_rows(v8h a, v8h b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ v4f mma_rows(v8bf a, v8bf b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 enum { RW_Q8 = 1, RW_Q4 = 2, RW_F16 = 3, RW_F32 = 4 };
@@ -96,15 +87,13 @@ constexpr int rows_slot(int src, bool wide_d) {  // bytes of a unit in a ring: w
 template <int SRC, int NPA, int MB, int NS, int NW, int PD, bool WIDE_D>
 __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
   constexpr bool QUANT = rows_quant(SRC);
-  constexpr int NPB = SRC == RW_F32 ? NPA : 1;
+  constexpr int NPB = QUANT ? 1 : SRC == RW_F16 ? 2 : NPA;
   constexpr int UB = rows_unit_blocks(SRC), CPW = rows_unit_bytes(SRC) / 16;  // blocks, 16-byte chunks of a row per unit
   constexpr int NR = 16 * NS;                                                     // weight rows of a wavefront
   constexpr int IW = NR * CPW / 64, ID = !QUANT ? 0 : NR * UB / (WIDE_D ? 2 : 1) / 64;  // load instructions per unit: weights, scales
   constexpr int WBYTES = NR * CPW * 16, SLOT = WBYTES + ID * 256;
   static_assert(NS == kRowsNS && PD == kRowsPD && SLOT == rows_slot(SRC, WIDE_D), "the LDS that rows_share counts");
   constexpr int NT = NR * NW, T = 64 * NW;  // columns of a workgroup, threads
-  constexpr bool HALF = SRC != RW_F32;
-  typedef typename std::conditional<HALF, v8h, v8bf>::type op_t;  // one matrix operand
   extern __shared__ __align__(16) unsigned char smem[];
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;
   const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, col = lane & 15;
@@ -199,7 +188,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
         else dv[j][0] = D[2 * bp * NR + r], dv[j][1] = D[(2 * bp + 1) * NR + r];
       }
     }
-    op_t af[MB][2][NPA];
+    v8bf af[MB][2][NPA];
 #pragma unroll
     for (int i = 0; i < MB; i++)
 #pragma unroll
@@ -207,29 +196,35 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
 #pragma unroll
         for (int q = 0; q < NPA; q++) {
           const int c4 = NPA * b + q;  // in units of four chunks
-          af[i][b][q] = __builtin_bit_cast(op_t, *(const uint4 *)(arow[i][c4 & 1] + kb * (NPA * 64) + (c4 >> 1) * 128));
+          af[i][b][q] = __builtin_bit_cast(v8bf, *(const uint4 *)(arow[i][c4 & 1] + kb * (NPA * 64) + (c4 >> 1) * 128));
         }
     __builtin_amdgcn_sched_barrier(0);
-    op_t bf[NS][2][NPB];
+    v8bf bf[NS][2][NPB];
 #pragma unroll
     for (int j = 0; j < NS; j++)
 #pragma unroll
       for (int b = 0; b < 2; b++) {
         const uint4 v = w[j][b][0];
         if constexpr (SRC == RW_Q8) {
-          bf[j][b][0] = h_of_bytes<true>(v.x, v.y);
+          bf[j][b][0] = bf_of_bytes<true>(v.x, v.y);
         } else if constexpr (SRC == RW_Q4) {  // k 0..15 of a block are the low nibbles of its bytes, 16..31 the high ones
-          bf[j][b][0] = h_of_bytes<false>((v.x >> (4 * (grp >> 1))) & 0x0f0f0f0fu, (v.y >> (4 * (grp >> 1))) & 0x0f0f0f0fu);
-        } else if constexpr (SRC == RW_F16) {
-          bf[j][b][0] = __builtin_bit_cast(v8h, v);
+          bf[j][b][0] = bf_of_bytes<false>((v.x >> (4 * (grp >> 1))) & 0x0f0f0f0fu, (v.y >> (4 * (grp >> 1))) & 0x0f0f0f0fu);
         } else {
-          const uint4 u = w[j][b][NV - 1];
-          const float x[8] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w),
-                              __uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)};
+          float x[8];
+          if constexpr (SRC == RW_F16) {
+            const unsigned h[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[2 * e] = half_bits_to_float((unsigned short)(h[e] & 0xffff)), x[2 * e + 1] = half_bits_to_float((unsigned short)(h[e] >> 16));
+          } else {
+            const uint4 u = w[j][b][NV - 1];
+            const unsigned f[8] = {v.x, v.y, v.z, v.w, u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = __uint_as_float(f[e]);
+          }
           uint4 pl[NPB];
           split8_planes<NPB>(x, pl);
 #pragma unroll
-          for (int q = 0; q < NPB; q++) bf[j][b][q] = __builtin_bit_cast(op_t, pl[q]);
+          for (int q = 0; q < NPB; q++) bf[j][b][q] = __builtin_bit_cast(v8bf, pl[q]);
         }
       }
     // a block's (quantised) or the pair's sum by itself: it is scaled before it is added, and one chain of matrix
@@ -264,13 +259,15 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
         v4f tmp[NS];
 #pragma unroll
         for (int j = 0; j < NS; j++) tmp[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        // pairs of terms above 2^-8(terms) of the leading product, the smallest first: only the two leading ones round at the
+        // size of the sum (fp16 weights, 5 rows of 4096: error 1.26e-7 -> 1.1e-7 of the result, block after block -> this)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int t = NPA - 1; t >= 0; t--)
 #pragma unroll
-          for (int t = NPA - 1; t >= 0; t--)  // pairs of terms above 2^-8(terms) of the leading product, smallest first
+          for (int q = 0; q <= t; q++)
+            if (t - q < NPB)
 #pragma unroll
-            for (int q = 0; q <= t; q++)
-              if (t - q < NPB)
+              for (int b = 0; b < 2; b++)
 #pragma unroll
                 for (int j = 0; j < NS; j++) tmp[j] = mma_rows(af[i][b][q], bf[j][b][t - q], tmp[j]);
 #pragma unroll
@@ -302,9 +299,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
         const int m = 16 * i + 4 * grp + r;
         if (m >= M) continue;
         float *o = mine + m * NT + wave * NR + 16 * j + col;
-        const float v = HALF ? acc[i][j][r] * a.rscale[m] : acc[i][j][r];
-        if (shares) __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else *o = v;
+        if (shares) __hip_atomic_store(o, acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *o = acc[i][j][r];
       }
   if (shares) {
     // a share's sums are device-scope stores that have reached memory before its ticket is drawn (a fence would write
@@ -346,21 +342,20 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
 }
 
 // ---- input rows -> planes, with what the Linear has in front ----
-// One block per row, held in registers (VPL pieces of 8 floats per thread).  HALF: fp16 terms of the row times a power of
-// two, which rscale undoes; else bf16 terms.  kbp: blocks of 32 k per row of planes (zeros past K).
+// One block per row, held in registers (VPL pieces of 8 floats per thread).  ROWS: terms for k_linear_rows, else for
+// gemm_planes.hip.  kbp: blocks of 32 k per row of planes (zeros past K).
 struct RowsPlanesArgs {
   uint4 *out;
-  float *rscale;
   const float *x;
   int64_t stride;
   int K, kbp;
   const float *g, *b;
   float eps;
 };
-template <int PRO, int NP, bool HALF, int VPL>
+template <int PRO, int NP, bool ROWS, int VPL>
 __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
-  __shared__ float red[3][4];
-  const int tid = threadIdx.x, K = a.K, nc = (K + 7) >> 3;
+  __shared__ float red[2][4];
+  const int tid = threadIdx.x, K = a.K;
   const float *xr = a.x + blockIdx.x * a.stride;
   constexpr bool NORM = PRO == CTHIP_PRO_LAYERNORM || PRO == CTHIP_PRO_RMSNORM;
   float v[VPL][8];
@@ -419,31 +414,15 @@ __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
       }
     }
   }
-  float up = 1.0f;
-  if (HALF) {
-    float m = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPL; j++)
-#pragma unroll
-      for (int e = 0; e < 8; e++) m = fmaxf(m, in(j, e) ? fabsf(v[j][e]) : 0.0f);
-    m = wave_max(m);
-    if ((tid & 63) == 0) red[2][tid >> 6] = m;
-    __syncthreads();
-    const unsigned mb = __float_as_uint(fmaxf(fmaxf(red[2][0], red[2][1]), fmaxf(red[2][2], red[2][3])));
-    // 2^(14 - exponent of the largest value): it lands in [2^14, 2^15).  Exponents kept where both powers are normal
-    const int ex = mb == 0 ? 141 : min(max((int)(mb >> 23), 16), 250);
-    up = __uint_as_float((unsigned)(268 - ex) << 23);
-    if (tid == 0) a.rscale[blockIdx.x] = __uint_as_float((unsigned)(ex - 14) << 23);
-  }
 #pragma unroll
   for (int j = 0; j < VPL; j++) {
     const int c = tid + 256 * j;
     if (c >= 4 * a.kbp) continue;
     float t[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] * up : 0.0f;
+    for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] : 0.0f;
     uint4 pl[NP];
-    if (HALF) split8_half<NP>(t, pl);
+    if (ROWS) split8_rows<NP>(t, pl);
     else split8_planes<NP>(t, pl);
 #pragma unroll
     for (int q = 0; q < NP; q++) a.out[((int64_t)blockIdx.x * a.kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
@@ -506,11 +485,11 @@ static int rows_launch(RowsGemmArgs a) {
   return rc;
 }
 
-template <int PRO, int NP, bool HALF>
+template <int PRO, int NP, bool ROWS>
 static void rows_planes_launch(const RowsPlanesArgs &a, int m) {
   const int pieces = (a.kbp * 4 + 255) / 256;
   const dim3 grid(m), block(256);
-#define RP(V) hipLaunchKernelGGL((k_rows_planes<PRO, NP, HALF, V>), grid, block, 0, state().stream, a)
+#define RP(V) hipLaunchKernelGGL((k_rows_planes<PRO, NP, ROWS, V>), grid, block, 0, state().stream, a)
   if (pieces <= 1) RP(1);
   else if (pieces <= 2) RP(2);
   else if (pieces <= 4) RP(4);
@@ -520,19 +499,22 @@ static void rows_planes_launch(const RowsPlanesArgs &a, int m) {
 }
 
 static int rows_source(const WMat *w) { return w->type == CTHIP_Q8_0 ? RW_Q8 : w->type == CTHIP_Q4_0 ? RW_Q4 : w->type == CTHIP_F16 ? RW_F16 : RW_F32; }
-static int rows_terms(int m, int precision) { return m < 8 || precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1; }
+// terms per input: all 24 bits, or 16 where operands rounded to bf16 are asked for
+static int rows_terms(int m, int precision) { return m >= 8 && precision == GEMM_BF16 ? 2 : 3; }
 static bool rows_wide_scales(const WMat *w) { return w->cols / 32 % 2 == 0 && rows_quant(rows_source(w)); }
 
 // Whether this is the launch to take: the operands are laid out for it, a share of it fits a workgroup, and it is the faster one.
 // Fewer than 8 rows: against the single-row kernels, one pass over the weights per row.  They cost about 3 us + m weights
 // at 4.3 (quantised), 2.7 (fp16) or 2.0 (fp32) per ns, the two launches here 9.5 us + the weights once at 3.2 / 2.3 / 1.15.
-//   us, m = 3 / 5 / 7:  4096 x 4096 Q8_0 17 / 20 / 29 -> 12 / 14 / 14;  22016 x 4096 Q8_0 52 / 80 / 110 -> 31 / 39 / 41;
-//   4096 x 11008 Q4_0 m = 5 50 -> 22;  768 x 3072 stays there at 5 / 6 / 9 (12 .. 15 here)
+//   us, m = 3 / 5 / 7, weights not in any cache:  22016 x 4096 Q8_0 49 / 73 / 98 -> 30 / 34 / 35, fp32 158 / 261 / 368 -> 86 / 89 / 103;
+//   4096 x 4096 Q8_0 m = 5 / 7 23 / 29 -> 12 / 12;  4096 x 11008 Q4_0 m = 5 44 -> 19;  768 x 3072 stays there at 5 / 7 (6 / 7; 11 here)
 // 8 rows and more: against a GEMM tile of 64 rows, which is as fast on small matrices and where the tile fills up:
-//   22016 x 4096 m = 12 / 24: Q8_0 52 / 55 -> 42 / 54, Q4_0 53 / 53 -> 36 / 55, fp16 78 / 78 -> 53 / 61, fp32 103 / 107 -> 109 / 111;
-//   11264 x 2048 m = 12: 19, 20, 27 -> 17, 17, 19;  4096 x 4096 m = 12: 14, 14, 18 -> 15, 15, 18
+//   22016 x 4096 m = 12: Q8_0 51 -> 37, Q4_0 52 -> 35, fp16 74 -> 49;  fp16 m = 24 / 32 74 / 74 -> 61 / 73;
+//   11264 x 2048 m = 12: Q8_0, Q4_0, fp16 20, 20, 26 -> 15, 15, 19;  4096 x 4096 m = 12: 15, 14, 18 -> 14, 14, 16.
+// Of 14 - 16 rows as long as 11008 a workgroup's memory holds a share too small for one round over the chip: Q8_0 m = 14 / 16
+// 25 / 26 -> 22 / 28; they are taken for their bits (the tiles' error is 2.4e-6 there, 1.3e-7 here).
 bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b) {
-  if (m < 2 || m > kRowsMax || (m >= 8 && precision == GEMM_FP32)) return false;
+  if (m < 2 || m > kRowsMax || precision == GEMM_FP32) return false;  // (fp32 operands asked for: the single-row kernels')
   if (w->cols % (w->type == CTHIP_F16 ? 8 : 4) || w->cols < 64 || w->cols > kRowsPlanesMaxK - 256) return false;  // whole 16-byte pieces
   auto al = [](const void *p) { return (uintptr_t)p % 16 == 0; };
   if (x_stride % 4 || !al(x) || !al(g) || !al(b)) return false;
@@ -550,7 +532,7 @@ bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, in
 // rows with what a Linear has in front of it as bf16 planes for gemm_planes.hip (x on 16 bytes, K % 32 == 0)
 bool rows_planes_supported(int K) { return K % 32 == 0 && K <= kRowsPlanesMaxK; }
 int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps) {
-  const RowsPlanesArgs pa = {(uint4 *)planes, nullptr, x, K, K, K / 32, g, b, eps};
+  const RowsPlanesArgs pa = {(uint4 *)planes, x, K, K, K / 32, g, b, eps};
   if (pro == CTHIP_PRO_LAYERNORM) rows_planes_launch<CTHIP_PRO_LAYERNORM, 2, false>(pa, m);
   else if (pro == CTHIP_PRO_RMSNORM) rows_planes_launch<CTHIP_PRO_RMSNORM, 2, false>(pa, m);
   else rows_planes_launch<CTHIP_PRO_NONE, 2, false>(pa, m);
@@ -563,7 +545,6 @@ int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, cons
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route) {
   const int terms = rows_terms(m, precision);
-  const bool half = w->type != CTHIP_F32;
   const int ub = rows_unit_blocks(rows_source(w));
   RowsGemmArgs a = {};
   a.kblocks = (int)((w->cols + 31) / 32);
@@ -588,53 +569,36 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
     a.e.route = *route;
   }
   unsigned char *planes = nullptr;
-  const size_t plane_bytes = (size_t)m * a.nkb * 64 * terms;
-  int rc = alloc_scratch((void **)&planes, plane_bytes + sizeof(float) * kRowsMax);  // fully written by the first launch
+  int rc = alloc_scratch((void **)&planes, (size_t)m * a.nkb * 64 * terms);  // fully written by the first launch
   if (rc) return rc;
   a.A = planes;
-  float *rscale = (float *)(planes + plane_bytes);
-  a.rscale = half ? rscale : nullptr;
-  const RowsPlanesArgs pa = {(uint4 *)planes, rscale, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
-#define RP3(PRO, HALF)                                           \
-  do {                                                           \
-    if (terms == 3) rows_planes_launch<PRO, 3, HALF>(pa, m);     \
-    else if (terms == 2) rows_planes_launch<PRO, 2, HALF>(pa, m); \
-    else rows_planes_launch<PRO, 1, HALF>(pa, m);                \
+  const RowsPlanesArgs pa = {(uint4 *)planes, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
+#define RP2(PRO)                                              \
+  do {                                                        \
+    if (terms == 3) rows_planes_launch<PRO, 3, true>(pa, m);  \
+    else rows_planes_launch<PRO, 2, true>(pa, m);             \
   } while (0)
-#define RP2(HALF)                                        \
-  switch (pro) {                                         \
-    case CTHIP_PRO_LAYERNORM: RP3(CTHIP_PRO_LAYERNORM, HALF); break; \
-    case CTHIP_PRO_RMSNORM: RP3(CTHIP_PRO_RMSNORM, HALF); break;     \
-    case CTHIP_PRO_SWIGLU: RP3(CTHIP_PRO_SWIGLU, HALF); break;       \
-    default: RP3(CTHIP_PRO_NONE, HALF); break;           \
-  }
-  if (half) {
-    RP2(true)
-  } else {
-    RP2(false)
+  switch (pro) {
+    case CTHIP_PRO_LAYERNORM: RP2(CTHIP_PRO_LAYERNORM); break;
+    case CTHIP_PRO_RMSNORM: RP2(CTHIP_PRO_RMSNORM); break;
+    case CTHIP_PRO_SWIGLU: RP2(CTHIP_PRO_SWIGLU); break;
+    default: RP2(CTHIP_PRO_NONE); break;
   }
 #undef RP2
-#undef RP3
   const bool wide = rows_wide_scales(w);
-#define RL4(SRC, NPA, WD)                                  \
-  do {                                                     \
-    if (m <= 16) rc = rows_launch<SRC, NPA, 1, WD>(a);     \
-    else rc = rows_launch<SRC, NPA, 2, WD>(a);             \
+#define RL(SRC, MB, WD)                                 \
+  do {                                                  \
+    if (terms == 3) rc = rows_launch<SRC, 3, MB, WD>(a); \
+    else rc = rows_launch<SRC, 2, MB, WD>(a);           \
   } while (0)
-#define RL3(SRC, WD)                      \
-  do {                                    \
-    if (terms == 3) RL4(SRC, 3, WD);      \
-    else if (terms == 2) RL4(SRC, 2, WD); \
-    else RL4(SRC, 1, WD);                 \
-  } while (0)
-  if (w->type == CTHIP_Q8_0 && wide) RL3(RW_Q8, true);
-  else if (w->type == CTHIP_Q8_0) RL3(RW_Q8, false);
-  else if (w->type == CTHIP_Q4_0 && wide) RL3(RW_Q4, true);
-  else if (w->type == CTHIP_Q4_0) RL3(RW_Q4, false);
-  else if (w->type == CTHIP_F16) RL3(RW_F16, false);
-  else RL3(RW_F32, false);
-#undef RL3
-#undef RL4
+  if (w->type == CTHIP_Q8_0 && wide) RL(RW_Q8, 1, true);
+  else if (w->type == CTHIP_Q8_0) RL(RW_Q8, 1, false);
+  else if (w->type == CTHIP_Q4_0 && wide) RL(RW_Q4, 1, true);
+  else if (w->type == CTHIP_Q4_0) RL(RW_Q4, 1, false);
+  else if (w->type == CTHIP_F32) rc = rows_launch<RW_F32, 3, 1, false>(a);
+  else if (m <= 16) RL(RW_F16, 1, false);
+  else RL(RW_F16, 2, false);
+#undef RL
   const int rf = cthip_free(planes);  // stream-ordered: handed out again only to later work on this stream
   return rc ? rc : rf;
 }

@@ -235,7 +235,8 @@ int cthip_wmat_fold_layernorm(void *wmat, const float *gamma, const float *beta,
  *   y[m,:] = act( prologue(x[m,:]) @ W^T + bias ) + residual[m,:]
  * x (m, cols) [(m, 2*cols) for SWIGLU], y/residual (m, rows), fp32, contiguous.
  * norm_g/norm_b/bias/residual may be NULL.  m == 1 is the dequant-in-register
- * GEMV of batch-1 decode; m >= 8 uses the MFMA tile path (weights dequantised while staged). */
+ * GEMV of batch-1 decode; m >= 8 uses the MFMA tile path (weights dequantised while staged); 2 to 32 rows over
+ * matrices where it is faster take one pass over the weights on matrix cores with all 24 bits of every input. */
 int cthip_linear(float *y, const void *wmat, const float *x, int m, const float *bias,
                  const float *residual, int act, int prologue, const float *norm_g,
                  const float *norm_b, float eps);
@@ -244,8 +245,9 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  * "gemm_precision": operand format of the MFMA launches behind cthip_linear with m >= 8 input rows and
  *   the decoder's prefill: 2 (default) = every operand split into two bf16 terms, three bf16 MFMAs
  *   per product, fp32 accumulation (2^-16 of a product is lost); 3 = three terms, six MFMAs per
- *   product: all 24 bits of an fp32 operand; 0 = fp32 MFMA operands; 1 = operands rounded to bf16
- *   (rtol/atol 1e-2).
+ *   product: all 24 bits of an fp32 operand; 0 = fp32 MFMA operands (fewer than 8 rows: fp32 vector
+ *   instructions); 1 = operands rounded to bf16 (rtol/atol 1e-2).  It is the least that is kept: launches over a few
+ *   rows hold more where that costs nothing.
  * "gemm_bf16": 1 = shorthand for gemm_precision 1, 0 = back to the default.
  * "gemv_stream_weights": whether the single-row Linear kernels request the weights with the non-temporal
  *   hint: -1 (default) = per matrix -- a matrix larger than the 256 MB Infinity Cache, and every matrix of a

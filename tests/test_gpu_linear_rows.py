@@ -54,6 +54,62 @@ def test_linear_rows(ops, kind, rows, cols, m, prologue):
     w.free()
 
 
+def tree_bound(cols):
+    """Additions behind one output value: terms of a block or two on the matrix cores, blocks, shares of k.  What any order of them in
+    fp32 may be off by, in units of the sum of the products' magnitudes."""
+    return (3 * 64 + cols / 32 + 32) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("kind,rows,cols,m", [("q8_0", 2611, 2080, 7), ("q8_0", 9001, 2560, 12), ("q4_0", 2611, 2080, 7), ("q4_0", 9001, 2560, 16), ("f16", 2603, 2056, 7),
+                                              ("f16", 9001, 2560, 11), ("f16", 15001, 4104, 23), ("f32", 2603, 2052, 5)])
+@pytest.mark.parametrize("outlier", [1e8, 2.0 ** 100])
+def test_inputs_of_any_magnitude(ops, kind, rows, cols, m, outlier):
+    """An input far above the others costs them no bits, column by column: where its weight is zero the result is what the
+    others give.  Nor does one row of inputs cost another."""
+    rng = np.random.default_rng(rows + m)
+    a = rng.normal(0, 0.05, (rows, cols)).astype(np.float32)
+    a[:, 5], a[:, cols - 7] = 0.0, 0.0
+    w = ops.WeightMatrix(kind, packed(kind, a), rows, cols)
+    x = (rng.normal(0, 1, (m, cols)) * 10.0 ** rng.uniform(-9, 0, (m, cols))).astype(np.float32)
+    x[:, 5], x[:, cols - 7] = outlier, -outlier
+    x[1] *= np.float32(2.0 ** -60)
+    x[1, 5], x[1, cols - 7] = 1.0, 2.0 ** -70
+    w64 = w.dequantize().astype(np.float64)
+    assert not w64[:, 5].any() and not w64[:, cols - 7].any()
+    got = ops.linear(x, w)
+    x64 = x.astype(np.float64)
+    assert np.all(np.abs(got - x64 @ w64.T) <= tree_bound(cols) * (np.abs(x64) @ np.abs(w64).T))
+    w.free()
+
+
+@pytest.mark.parametrize("kind,rows,cols,m", [("q8_0", 2611, 2080, 7), ("q8_0", 9001, 2560, 12), ("q4_0", 2611, 2080, 7), ("f16", 2603, 2056, 7),
+                                              ("f16", 15001, 4104, 23), ("f32", 2603, 2052, 5)])
+def test_inputs_that_are_not_finite_or_nearly_so(ops, kind, rows, cols, m):
+    """Infinities and NaN as in fp32 arithmetic (infinity of a weight's sign; NaN against a weight of zero or another
+    infinity), rows beside them untouched; the largest floats times weights below one half."""
+    rng = np.random.default_rng(rows + m)
+    a = rng.normal(0, 0.05, (rows, cols)).astype(np.float32)
+    a[::3, 40] = 0.0
+    w = ops.WeightMatrix(kind, packed(kind, a), rows, cols)
+    w64 = w.dequantize().astype(np.float64)
+    x = rng.normal(0, 1, (m, cols)).astype(np.float32)
+    top = np.finfo(np.float32).max if kind in ("f16", "f32") else np.float32(2.0 ** 119)  # (integers up to 127 come before their scale)
+    x[0, 40] = np.inf
+    x[1, 40], x[1, 41] = -np.inf, np.inf
+    x[2, 7] = np.nan
+    x[3] = 0.0
+    x[3, 11] = top
+    got = ops.linear(x, w)
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(x[r].astype(np.float64) * w64).sum(1) for r in range(m)])
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    bound = tree_bound(cols) * (np.abs(np.where(np.isfinite(x), x, 0).astype(np.float64)) @ np.abs(w64).T)
+    assert np.all(np.abs(got - want)[ok] <= bound[ok])
+    w.free()
+
+
 @pytest.mark.parametrize("kind,rows,cols,m,precision", [
     ("f16", 2100, 28672, 27, 2), ("f16", 2100, 28672, 32, 2), ("f16", 2100, 28672, 18, 3), ("f16", 2100, 28672, 32, 3), ("f16", 2050, 29568, 25, 2),
     ("f16", 2500, 24576, 31, 2), ("q4_0", 4098 * 128, 2240, 16, 2), ("f16", 2100, 28672, 17, 2), ("f16", 2100, 28672, 16, 2), ("q8_0", 1700, 28672, 16, 3)])
