@@ -157,3 +157,34 @@ def test_short_prompt_equals_its_rows_one_by_one(ops, rows):
         assert t0 == t1
         assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
     model.close()
+
+
+@pytest.mark.parametrize("arch,rows", [("gpt2", 8), ("gpt2", 12), ("llama", 12)])
+def test_sessions_hold_the_same_rows_whatever_their_cache(oracle, arch, rows):
+    """A prompt of a few rows takes the same launches over both kinds of cache (thirds routed to the cache rows, or stored and
+    split): layer 0's Q8_0 rows are the quantised fp32 rows of the other session bit for bit."""
+    from caten_amd import _lib, llm, synth
+    lib = _lib.init(0)
+    if arch == "gpt2":  # 8448 x 2816
+        cfg = dict(synth.GPT2_CONFIGS["gpt2-tiny"], dim=2816, n_heads=22, ffn=256, n_layers=1, vocab=300)
+        make, sd = llm.make_gpt2, llm.gpt2_state_dict(synth.gpt2_weights(cfg, seed=6), "q8_0")
+    else:  # 8448 x 2816 likewise
+        cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=2816, n_heads=22, n_kv_heads=22, ffn=256, n_layers=1, vocab=300)
+        make, sd = llm.make_llama, llm.llama_state_dict(synth.llama_weights(cfg, seed=6), "q8_0")
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], rows, seed=6)]
+    held = []
+    try:
+        for mode in (0, 1):
+            _lib.check(lib.cthip_set_option(b"kv_cache", mode))
+            model = make(cfg, sd)
+            model.forward(ids, rows, 0)
+            if mode == 0:
+                held += [oracle.quantize("q8_0", model.peek(f"{c}_cache.0")[:rows * 2816]) for c in "kv"]
+                held = [np.asarray(h).view(np.uint8).reshape(-1, 34) for h in held]
+            else:
+                for c, h in zip("kv", held):
+                    assert np.array_equal(model.peek(f"{c}_cache_q8.0").view(np.uint8)[:rows * 2816].reshape(-1, 32), h[:, 2:])
+                    assert np.array_equal(model.peek(f"{c}_cache_d.0").view(np.uint8)[:rows * 176].reshape(-1, 2), h[:, :2])
+            model.close()
+    finally:
+        _lib.check(lib.cthip_set_option(b"kv_cache", 0))
