@@ -56,8 +56,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
   const int b0 = tile / (a.band * a.tn), inb = tile - b0 * a.band * a.tn, height = min(a.band, a.tm - b0 * a.band);
   const int mi = b0 * a.band + inb % height, ni = inb / height;
   const int m0 = mi * BM, n0 = ni * BN;
-  const int kb0 = blockIdx.y * a.kper, kb1 = min(a.nkb, kb0 + a.kper);  // this workgroup's blocks of 32 k
-  const int nsteps = kb1 - kb0;
+  const int nsteps = a.nkb;
 
   // where this lane's pieces of a step lie, as offsets from the step's bases; rows past the end repeat the last one
   unsigned avo[IA], bvo[IB], svo[IS > 0 ? IS : 1];
@@ -76,9 +75,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
     const int s = ((j * NW + wave) * 64 + lane) % BN;
     svo[j] = (unsigned)(min(s, a.N - 1 - n0) * a.dpitch) * 2u;
   }
-  const unsigned char *ab = a.A + (int64_t)m0 * a.apitch + (int64_t)kb0 * (64 * NPA);
-  const unsigned char *bb = a.B + (int64_t)n0 * a.bpitch + (int64_t)kb0 * (CB * 16);
-  const unsigned char *sb = SRC == PL_PLANES ? nullptr : (const unsigned char *)(a.bd + (int64_t)n0 * a.dpitch + kb0);
+  const unsigned char *ab = a.A + (int64_t)m0 * a.apitch;
+  const unsigned char *bb = a.B + (int64_t)n0 * a.bpitch;
+  const unsigned char *sb = SRC == PL_PLANES ? nullptr : (const unsigned char *)(a.bd + (int64_t)n0 * a.dpitch);
   auto issue = [&](int step, int buf) __attribute__((always_inline)) {
     step = min(step, nsteps - 1);  // past the end: the last step again, so that the counts stay the same
     const unsigned base = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)buf * BUF);
@@ -333,7 +332,6 @@ static int planes_launch(PlaneGemmArgs a) {
     const double score = (double)h * BM * NPA + ((double)a.chunk / h + 1.0) * BN * NPB;
     if (best < 0 || score < best) best = score, a.band = h;
   }
-  a.kper = a.nkb;
   auto fn = k_gemm_planes<NPA, SRC, NPB, MB, NB, WM, WN, NBUF>;
   static bool big_lds = false;
   if (!big_lds && lds > 64 * 1024) {

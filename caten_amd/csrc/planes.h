@@ -13,10 +13,8 @@ struct PlaneGemmArgs {
   int apitch, bpitch;        // bytes between rows
   int dpitch;                // scales between rows
   int M, N, nkb;             // nkb: blocks of 32 k
-  int kper;                  // blocks per workgroup along gridDim.y (split K)
   const float *bias, *residual;
   int act;
-  float *ws;                 // split K: raw partial tiles ws[z][M][N]; null: C is complete
   int tm, tn, band, chunk;   // tile -> workgroup mapping
   int pairs;                 // columns (2j, 2j + 1) are (gate, up): C (M, N / 2) gets silu(gate) * up
   int routed;
@@ -109,13 +107,6 @@ __device__ __forceinline__ void plane_gemm_store(const PlaneGemmArgs &a, int row
   const int N = a.N;
   if (row >= a.M || col >= N) return;
   float v[4] = {v4.x, v4.y, v4.z, v4.w};
-  if (a.ws) {
-    float *o = a.ws + ((int64_t)blockIdx.y * a.M + row) * N + col;
-    if ((N & 3) == 0) *(float4 *)o = v4;
-    else
-      for (int t = 0; t < 4 && col + t < N; t++) o[t] = v[t];
-    return;
-  }
   if ((N & 3) == 0) {
     if (a.bias) {
       const float4 bb = *(const float4 *)(a.bias + col);
