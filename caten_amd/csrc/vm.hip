@@ -466,7 +466,8 @@ int cthip_vm_run(void *vm) {
     GraphCollector collector;  // neighbours that can share a launch do (graph_ops.hip)
     for (size_t k = 0; k < v->nodes.size() && !rc; k++)
       if (v->nodes[k].type == VM_NODE_KERNEL) rc = vm_kernel(*v, (int)k, v->nodes[k]);
-    if (!rc) rc = graph_ops_flush();
+    // after a failed node too: what the nodes before it asked for has run when the walk stops (the earlier failure counts)
+    if (const int first = graph_ops_flush()) rc = first;
     return rc;
   }
   for (size_t k = 0; k < v->nodes.size() && !rc; k++) {

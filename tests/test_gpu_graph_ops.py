@@ -27,9 +27,34 @@ def test_shared_launches_leave_the_same_buffers(name, lengths):
                 got, want = (np.asarray(transfer_into_array(m.vm.getvar(b)), np.float64) for m in models)
                 seen = np.isfinite(want)  # (a masked score is -inf in both)
                 assert got.shape == want.shape and np.array_equal(seen, np.isfinite(got)), (b, n)
-                err, ref = np.linalg.norm((got - want)[seen]), np.linalg.norm(want[seen])
+                err, ref = np.linalg.norm(got[seen] - want[seen]), np.linalg.norm(want[seen])
                 assert err <= 2e-5 * ref + 1e-12, (b, n, err, ref)
             n += s
     finally:
         for m in models:
             m.close()
+
+
+def test_a_failing_node_leaves_what_ran_before_it(oracle):
+    """The walk stops at a node whose argument was never set; the operations in front of it, queued to share launches, have run."""
+    import ctypes as C
+    from caten_amd import _lib, blueprints, ops
+    from caten_amd.renderer import item_sexp
+    lib = _lib.init(0)
+    x = np.random.default_rng(0).normal(0, 1, (5, 77)).astype(np.float32)
+    dx, dy, dz = ops.DeviceArray.from_numpy(x), ops.DeviceArray((5, 77)), ops.DeviceArray((5, 77))
+    program, vm = C.c_void_p(), C.c_void_p()
+    _lib.check(lib.cthip_program_create(C.byref(program), item_sexp(blueprints.softmax_rows()).encode()))
+    _lib.check(lib.cthip_vm_create(C.byref(vm), 5))
+    dtypes, none, one = (C.c_int * 4)(0, 5, 5, 0), (C.c_double * 4)(), (C.c_int * 1)(0)
+    for out, src in ((2, 0), (3, 2), (3, 4)):  # softmax of x, of that, and of a buffer nobody sets
+        reads = (C.c_longlong * 4)(out, 5, 77, src)
+        _lib.check(lib.cthip_vm_add_kernel(vm, program, 4, (C.c_int * 4)(2, 0, 0, 2), reads, none, dtypes, 1, one, (C.c_int * 1)(out)))
+    for slot, d in ((0, dx), (2, dy), (3, dz)):
+        _lib.check(lib.cthip_vm_set_buffer(vm, slot, d.ptr))
+    assert lib.cthip_vm_run(vm) == _lib.E_STATE and b"vm: node 2" in lib.cthip_last_error()
+    want = oracle.softmax(x)
+    assert np.allclose(dy.numpy(), want, rtol=1e-5, atol=1e-6)
+    assert np.allclose(dz.numpy(), oracle.softmax(want), rtol=1e-5, atol=1e-6)
+    _lib.check(lib.cthip_vm_destroy(vm))
+    _lib.check(lib.cthip_program_destroy(program))
