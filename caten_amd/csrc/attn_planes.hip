@@ -243,7 +243,7 @@ bool attn_planes_pays(int S, int start, int H, int Hkv, int DH) {
   const double each = 0.75 * tiles / (4.0 * state().compute_units), chain = 0.75 * longest;
   return 10.0 + f * (each > chain ? each : chain) < before;
 }
-int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH) {
+int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH, bool *done) {
   if ((DH != 64 && DH != 128) || S < 1 || Hkv < 1 || H % Hkv) return fail(CTHIP_E_UNSUPPORTED, "attention: %d rows, %d heads on %d of %d", S, H, Hkv, DH);
   AttnPlanesArgs a = {};
   a.out = out;
@@ -255,10 +255,11 @@ int launch_attn_planes(float *out, void *out_planes, const float *q, const float
   a.units = (S + 31) / 32 * group;
   constexpr int NW = 4;
   const int wgs = Hkv * ((a.units + NW - 1) / NW);
-    unsigned char *planes = nullptr;
+  unsigned char *planes = nullptr;
   const size_t bytes = (size_t)Hkv * a.nkb * 128 * DH;
-  int rc = alloc_scratch((void **)&planes, 2 * bytes + 2 * 128 * DH);  // fully written by the first launch
-  if (rc) return rc;
+  if (alloc_scratch((void **)&planes, 2 * bytes + 2 * 128 * DH)) return 0;  // fully written by the first launch
+  *done = true;
+  int rc = 0;
   a.kp = planes;
   a.vp = planes + bytes;  // (a tile behind either may be read, and is not looked at)
   const dim3 sgrid(a.nkb, Hkv);

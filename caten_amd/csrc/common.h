@@ -52,6 +52,9 @@ State &state();
 int alloc_scratch(void **out, size_t bytes);
 // the same for what is only kept to be faster: refused rather than taking the last memory from others
 int alloc_spare(void **out, size_t bytes);
+// Whether the library's stream is being captured into a graph: a launch that would take scratch takes its other path then (a
+// replay would find the block in other hands), and nothing that stays is made (the launches that fill it have not run).
+bool stream_capturing();
 bool device_readable(const void *p);
 void set_error(const char *fmt, ...);
 int fail(int code, const char *fmt, ...);
@@ -236,7 +239,8 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
                 int max_T, int H, int Hkv, int Dh, const AttnSplit *split = nullptr);
 // attention of many prompt rows with keys and values split once (attn_planes.hip); out as fp32 rows or as rows of two terms
 bool attn_planes_pays(int S, int start, int H, int Hkv, int DH);
-int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH);
+// (*done stays false where there is no memory for the terms)
+int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH, bool *done);
 int launch_embedding(float *out, const float *W, const float *idx_f, const int *idx_i, int ntok, int vocab, int dim,
                      const float *W2, const int *pos, int max_pos);
 int launch_argmax(int64_t *out, const float *x, int64_t rows, int n, int *tok_out, int *pos, int64_t *history,
@@ -266,10 +270,11 @@ constexpr int kActSwigluPairs = 64;
 // route: non-null = y is ignored, the columns go where the route says; K is not split then.
 int launch_linear_gemm(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual,
                        int act, int precision, GemmDeferred *defer = nullptr, const GemmRoute *route = nullptr);
-// the same for 2 .. 32 rows, prologue included (linear_rows.hip); call only where linear_rows_pays
+// the same for 2 .. 32 rows, prologue included (linear_rows.hip); call only where linear_rows_pays.  *done stays false, and the
+// caller takes the other path, where there is no scratch to be had.
 bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b);
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
-                       int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route = nullptr);
+                       int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route, bool *done);
 // matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
 // A Linear over many rows through the same kernel: x as fp32 rows or already as planes of plane_terms(precision) terms, the
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.

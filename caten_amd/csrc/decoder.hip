@@ -880,8 +880,11 @@ static int prefill_min(const Decoder *d) { return d->kvq ? 8 : d->fused || d->fu
 // fp32-grade products: all rows in one pass over the weights where that is the faster launch, else the single-row kernels.
 static int prompt_linear(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual, int act, int precision,
                          GemmDeferred *defer = nullptr, const GemmRoute *route = nullptr) {
-  if (linear_rows_pays(w, x, w->cols, m, precision, nullptr, nullptr))
-    return launch_linear_rows(y, w, x, w->cols, m, bias, residual, act, CTHIP_PRO_NONE, nullptr, nullptr, 0.0f, precision, route);
+  if (linear_rows_pays(w, x, w->cols, m, precision, nullptr, nullptr)) {
+    bool done = false;
+    const int rc = launch_linear_rows(y, w, x, w->cols, m, bias, residual, act, CTHIP_PRO_NONE, nullptr, nullptr, 0.0f, precision, route, &done);
+    if (rc || done) return rc;
+  }
   if (m >= 8) return launch_linear_gemm(y, w, x, m, bias, residual, act, precision, defer, route);
   GemvArgs a = {};
   a.x = x;
@@ -972,6 +975,10 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       held.push_back(w);
       return true;
     };
+    auto no_planes = [&](const WMat *w) {
+      held.erase(std::find(held.begin(), held.end(), w));
+      weight_planes_release(w);
+    };
     // y = norm(x), as terms where the Linear behind it takes them
     auto norm = [&](float *y, const float *x, const float *g, const float *b, bool terms) {
       if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps);
@@ -984,10 +991,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         bool taken = false;
         const int r = launch_linear_planes(out_terms ? nullptr : y, w, in_terms ? nullptr : in, in_terms ? (const unsigned char *)in : nullptr, R, bias,
                                            residual, act, prec, route, out_terms ? (unsigned char *)y : nullptr, &taken);
-        if (in_terms) {  // no more than a layer's matrices are held at a time
-          held.erase(std::find(held.begin(), held.end(), w));
-          weight_planes_release(w);
-        }
+        if (in_terms) no_planes(w);  // no more than a layer's matrices are held at a time
         if (taken) return r;
         if (in_terms || out_terms) return fail(CTHIP_E_STATE, "prompt: a Linear of %lld x %lld over %d rows cannot take its input as terms", (long long)w->rows, (long long)w->cols, R);
       }
@@ -1047,9 +1051,13 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       }
       }
       if (last) R = 1, Xr = X + (int64_t)(s - 1) * D;
-      const bool at = !last && planes && attn_planes_pays(R, n, c.n_heads, c.n_kv_heads, Dh), att = at && in_planes(L.proj);
-      if (at) TRY(launch_attn_planes(att ? nullptr : ATT, att ? ATT : nullptr, Q, K, V, R, n, c.n_heads, c.n_kv_heads, Dh));
-      else TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
+      bool att = false, attended = false;
+      if (!last && planes && attn_planes_pays(R, n, c.n_heads, c.n_kv_heads, Dh)) {
+        att = in_planes(L.proj);
+        TRY(launch_attn_planes(att ? nullptr : ATT, att ? ATT : nullptr, Q, K, V, R, n, c.n_heads, c.n_kv_heads, Dh, &attended));
+        if (att && !attended) att = false, no_planes(L.proj);
+      }
+      if (!attended) TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
       const bool ft = in_planes(L.fc), gt = ft && (gpt2 || L.fc_pairs) && in_planes(L.fc2);
       TRY(linear_residual_norm(L.proj, ATT, att, L.proj_b, L.ln2_g, L.ln2_b, ft));
       const float *hin = Hb;

@@ -482,9 +482,9 @@ int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N,
   planes_operands(a, K, terms, terms);
   unsigned char *pa = nullptr;
   const size_t abytes = (size_t)M * a.apitch, bbytes = (size_t)N * a.bpitch;
-  int rc = alloc_scratch((void **)&pa, abytes + bbytes + 256);  // fully written by the two passes
-  if (rc) return 0;
+  if (stream_capturing() || alloc_scratch((void **)&pa, abytes + bbytes + 256)) return 0;  // fully written by the two passes
   *done = true;
+  int rc = 0;
   unsigned char *pb = pa + (abytes + 255) / 256 * 256;
   rc = planes_rows<float>(pa, A, M, K, K, terms);
   if (!rc) {
@@ -687,7 +687,7 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
     a.dpitch = a.nkb;
   }
   unsigned char *tmp = nullptr;
-  if (!xplanes && alloc_scratch((void **)&tmp, (size_t)m * a.apitch)) return 0;  // fully written by the pass in front
+  if (stream_capturing() || (!xplanes && alloc_scratch((void **)&tmp, (size_t)m * a.apitch))) return 0;  // fully written by the pass in front
   bool temp_b = false;
   const unsigned char *pb = weight_planes(w, terms_b, &temp_b);
   if (!pb) {

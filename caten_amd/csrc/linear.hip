@@ -724,8 +724,11 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
   if (m > 65535) return fail(CTHIP_E_BAD_ARG, "cthip_linear: m = %d exceeds 65535", m);
   const WMat *w = (const WMat *)wmat;
   const int64_t x_stride = prologue == CTHIP_PRO_SWIGLU ? 2 * w->cols : w->cols;
-  if (linear_rows_pays(w, x, x_stride, m, state().gemm_precision, norm_g, norm_b))
-    return launch_linear_rows(y, w, x, x_stride, m, bias, residual, act, prologue, norm_g, norm_b, eps, state().gemm_precision);
+  if (linear_rows_pays(w, x, x_stride, m, state().gemm_precision, norm_g, norm_b)) {
+    bool done = false;
+    const int rc = launch_linear_rows(y, w, x, x_stride, m, bias, residual, act, prologue, norm_g, norm_b, eps, state().gemm_precision, nullptr, &done);
+    if (rc || done) return rc;
+  }
   if (m >= 8) {
     // several input rows: the MFMA tile path reads the weights once instead of once per row
     const float *xin = x;

@@ -462,7 +462,7 @@ static RowsShare rows_share(int src, int terms, int mb, bool wide_d, int M, int 
 }
 
 template <int SRC, int NPA, int MB, bool WIDE_D>
-static int rows_launch(RowsGemmArgs a) {
+static int rows_launch(RowsGemmArgs a, bool *done) {
   constexpr int NS = kRowsNS, NW = 4 * MB, PD = kRowsPD, NT = rows_columns(MB), T = 64 * NW, UB = rows_unit_blocks(SRC);
   const int M = a.e.M, N = a.e.N, groups = (N + NT - 1) / NT, units = (a.kblocks + UB - 1) / UB;
   const RowsShare share = rows_share(SRC, NPA, MB, WIDE_D, M, N, a.kblocks);
@@ -470,8 +470,8 @@ static int rows_launch(RowsGemmArgs a) {
   a.kper = share.per * UB;
   const int ks = (units + share.per - 1) / share.per;
   a.parts = nullptr;
-  int rc = 0;
-  if (ks > 1 && (rc = alloc_scratch((void **)&a.parts, sizeof(float) * (size_t)groups * ks * M * NT))) return rc;
+  if (ks > 1 && alloc_scratch((void **)&a.parts, sizeof(float) * (size_t)groups * ks * M * NT)) return 0;
+  *done = true;
   static bool big_lds = false;
   auto fn = k_linear_rows<SRC, NPA, MB, NS, NW, PD, WIDE_D>;
   if (!big_lds) {
@@ -480,7 +480,7 @@ static int rows_launch(RowsGemmArgs a) {
   }
   hipLaunchKernelGGL(fn, dim3(groups, ks), dim3(T), share.lds, state().stream, a);
   const hipError_t e = hipGetLastError();
-  if (a.parts) rc = cthip_free(a.parts);  // stream-ordered: handed out again only to later work on this stream
+  const int rc = a.parts ? cthip_free(a.parts) : 0;  // stream-ordered: handed out again only to later work on this stream
   if (e != hipSuccess) return fail((int)e, "linear rows: launch -> %s", hipGetErrorString(e));
   return rc;
 }
@@ -541,9 +541,9 @@ int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, cons
 }
 
 // y (m, rows) = act(prologue(x) @ W^T + bias) + residual for a few rows; act may be kActSwigluPairs, route as for
-// launch_linear_gemm.  Call only where linear_rows_pays.
+// launch_linear_gemm.  Call only where linear_rows_pays; *done stays false where there is no scratch to be had.
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
-                       int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route) {
+                       int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route, bool *done) {
   const int terms = rows_terms(m, precision);
   const int ub = rows_unit_blocks(rows_source(w));
   RowsGemmArgs a = {};
@@ -569,8 +569,8 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
     a.e.route = *route;
   }
   unsigned char *planes = nullptr;
-  int rc = alloc_scratch((void **)&planes, (size_t)m * a.nkb * 64 * terms);  // fully written by the first launch
-  if (rc) return rc;
+  if (stream_capturing() || alloc_scratch((void **)&planes, (size_t)m * a.nkb * 64 * terms)) return 0;  // fully written by the first launch
+  int rc = 0;
   a.A = planes;
   const RowsPlanesArgs pa = {(uint4 *)planes, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
 #define RP2(PRO)                                              \
@@ -588,14 +588,14 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
   const bool wide = rows_wide_scales(w);
 #define RL(SRC, MB, WD)                                 \
   do {                                                  \
-    if (terms == 3) rc = rows_launch<SRC, 3, MB, WD>(a); \
-    else rc = rows_launch<SRC, 2, MB, WD>(a);           \
+    if (terms == 3) rc = rows_launch<SRC, 3, MB, WD>(a, done); \
+    else rc = rows_launch<SRC, 2, MB, WD>(a, done);           \
   } while (0)
   if (w->type == CTHIP_Q8_0 && wide) RL(RW_Q8, 1, true);
   else if (w->type == CTHIP_Q8_0) RL(RW_Q8, 1, false);
   else if (w->type == CTHIP_Q4_0 && wide) RL(RW_Q4, 1, true);
   else if (w->type == CTHIP_Q4_0) RL(RW_Q4, 1, false);
-  else if (w->type == CTHIP_F32) rc = rows_launch<RW_F32, 3, 1, false>(a);
+  else if (w->type == CTHIP_F32) rc = rows_launch<RW_F32, 3, 1, false>(a, done);
   else if (m <= 16) RL(RW_F16, 1, false);
   else RL(RW_F16, 2, false);
 #undef RL

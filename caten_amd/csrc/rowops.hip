@@ -598,14 +598,14 @@ static int launch_rowop(RowArgs a) {
   if (split) {
     const int per = max(1024, (a.n + kSoftmaxParts - 1) / kSoftmaxParts), parts = (a.n + per - 1) / per;
     float2 *part = nullptr;
-    int rc = alloc_scratch((void **)&part, sizeof(float2) * (size_t)a.rows * parts);  // fully written by the first launch
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_softmax_part, dim3(parts, (unsigned)a.rows), dim3(256), 0, st, part, a.x, a.n, per);
-    hipLaunchKernelGGL(k_softmax_apply, dim3(parts, (unsigned)a.rows), dim3(256), 0, st, a.y, a.x, part, a.n, per);
-    const hipError_t e = hipGetLastError();
-    rc = cthip_free(part);  // stream-ordered: handed out again only to later work on this stream
-    if (e != hipSuccess) return fail((int)e, "row op: launch -> %s", hipGetErrorString(e));
-    return rc;
+    if (!stream_capturing() && !alloc_scratch((void **)&part, sizeof(float2) * (size_t)a.rows * parts)) {  // fully written by the first launch
+      hipLaunchKernelGGL(k_softmax_part, dim3(parts, (unsigned)a.rows), dim3(256), 0, st, part, a.x, a.n, per);
+      hipLaunchKernelGGL(k_softmax_apply, dim3(parts, (unsigned)a.rows), dim3(256), 0, st, a.y, a.x, part, a.n, per);
+      const hipError_t e = hipGetLastError();
+      const int rc = cthip_free(part);  // stream-ordered: handed out again only to later work on this stream
+      if (e != hipSuccess) return fail((int)e, "row op: launch -> %s", hipGetErrorString(e));
+      return rc;
+    }
   }
   if constexpr (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM) {
 #define NORM_BLOCK(VPL) hipLaunchKernelGGL((k_norm_block<MODE, VPL>), grid, dim3(256), 0, st, a)
@@ -1754,13 +1754,13 @@ int launch_argmax(int64_t *out, const float *x, int64_t rows, int n, int *tok_ou
   hipStream_t st = state().stream;
   if (rows <= kArgmaxPartRows && n >= 8192) {
     unsigned long long *parts = nullptr;
-    int rc = alloc_scratch((void **)&parts, (size_t)rows * kArgmaxParts * 8);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_argmax_parts, dim3((unsigned)rows, kArgmaxParts), dim3(256), 0, st, a, parts);
-    const hipError_t e = hipGetLastError();
-    rc = cthip_free(parts);  // stream-ordered: handed out again only to later work on this stream
-    if (e != hipSuccess) return fail((int)e, "argmax: launch -> %s", hipGetErrorString(e));
-    return rc;
+    if (!stream_capturing() && !alloc_scratch((void **)&parts, (size_t)rows * kArgmaxParts * 8)) {
+      hipLaunchKernelGGL(k_argmax_parts, dim3((unsigned)rows, kArgmaxParts), dim3(256), 0, st, a, parts);
+      const hipError_t e = hipGetLastError();
+      const int rc = cthip_free(parts);  // stream-ordered: handed out again only to later work on this stream
+      if (e != hipSuccess) return fail((int)e, "argmax: launch -> %s", hipGetErrorString(e));
+      return rc;
+    }
   }
   // threads for four 16-byte pieces each: more would have nothing to ask for
   const dim3 grid((unsigned)rows);

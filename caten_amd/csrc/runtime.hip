@@ -259,6 +259,12 @@ static int take_block(void **out, size_t bytes, bool needed) {
 int cthip::alloc_scratch(void **out, size_t bytes) { return take_block(out, bytes, true); }
 int cthip::alloc_spare(void **out, size_t bytes) { return take_block(out, bytes, false); }
 
+bool cthip::stream_capturing() {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(state().stream, &st) != hipSuccess) (void)hipGetLastError();
+  return st != hipStreamCaptureStatusNone;
+}
+
 extern "C" {
 
 int cthip_alloc(void **out, size_t bytes) {
