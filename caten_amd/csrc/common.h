@@ -267,7 +267,7 @@ struct GemmRoute {
 // act == kActSwigluPairs: the weight rows are (gate_j, up_j) pairs and y (m, rows / 2) gets silu(gate_j) * up_j
 // (SwiGLU, external/llm/layers.lisp:53-64, in the epilogue of the gate|up launch); K is not split then.
 constexpr int kActSwigluPairs = 64;
-// route: non-null = y is ignored, the columns go where the route says; K is not split then.
+// route: non-null = y is ignored, the columns go where the route says.
 int launch_linear_gemm(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual,
                        int act, int precision, GemmDeferred *defer = nullptr, const GemmRoute *route = nullptr);
 // the same for 2 .. 32 rows, prologue included (linear_rows.hip); call only where linear_rows_pays.  *done stays false, and the
@@ -275,8 +275,7 @@ int launch_linear_gemm(float *y, const WMat *w, const float *x, int m, const flo
 bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b);
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route, bool *done);
-// matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
-// A Linear over many rows through the same kernel: x as fp32 rows or already as planes of plane_terms(precision) terms, the
+// A Linear over many rows from operands in memory as bf16 terms (gemm_planes.hip): x as fp32 rows or already as planes of plane_terms(precision) terms, the
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
 bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in);
 // x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
@@ -291,6 +290,7 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
 bool rows_planes_supported(int K);
 int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps);
 void wmat_drop_planes(WMat *w);
+// matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
 bool matmul_planes_pay(int M, int N, int K, int precision);
 int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N, int K, int act, const float *bias, const float *residual, int precision,
                          bool *done);

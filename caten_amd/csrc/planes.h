@@ -83,12 +83,14 @@ __device__ __forceinline__ const unsigned char *uniform(const unsigned char *p) 
   const uint64_t v = (uint64_t)p;
   return (const unsigned char *)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)v));
 }
-// all but the youngest N of this wavefront's loads have landed, its LDS reads are done, and so are everybody else's
+// all but the youngest N of this wavefront's loads have landed
 template <int N>
-__device__ __forceinline__ void wait_loads() {  // ... of this wavefront only
+__device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// this wavefront's LDS reads are done
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// all but the youngest N of this wavefront's loads have landed, its LDS reads are done, and so are everybody else's
 template <int N>
 __device__ __forceinline__ void wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");

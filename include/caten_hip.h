@@ -263,7 +263,7 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  *   max_seq >= 512 share the keys of a head among (compute units / heads) workgroups, at most 16, in their decode
  *   attention (long contexts); 2 .. 16 = that many workgroups per head; 0 = one workgroup per head.  Same tokens;
  *   logits differ in summation order only.
- * "attn_long_from": a position (default 896; 0 = never).  Decoder sessions created afterwards whose layers run as
+ * "attn_long_from": a position (default 704; 0 = never).  Decoder sessions created afterwards whose layers run as
  *   three launches switch, from this position on (half as far again over Q8_0 cache rows), to four launches per layer: the attention as a
  *   launch of its own with a head's keys shared by several workgroups ("attn_split"), then the projection.  Same
  *   tokens; logits differ in summation order only.
