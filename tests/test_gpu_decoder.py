@@ -15,7 +15,7 @@ RTOL, ATOL = 1e-3, 1e-4
 def close(a, b, rtol=RTOL, atol=ATOL):
     a = np.asarray(a, np.float64)
     b = np.asarray(b, np.float64)
-    bad = np.abs(a - b) > atol + rtol * np.abs(b)
+    bad = ~(np.abs(a - b) <= atol + rtol * np.abs(b))  # (a NaN is a difference)
     assert not bad.any(), f"{bad.sum()} of {bad.size} differ; max abs err {np.abs(a - b).max():.3e}"
 
 

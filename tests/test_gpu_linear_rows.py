@@ -29,7 +29,7 @@ def norm(x, g, b, kind):
 @pytest.mark.parametrize("kind,rows,cols,m", [
     ("q8_0", 2611, 2080, 7), ("q8_0", 12000, 2048, 3), ("q8_0", 9001, 2560, 8), ("q8_0", 9001, 2560, 16),
     ("q4_0", 2611, 2080, 7), ("q4_0", 2600, 11008, 2), ("q4_0", 9001, 2560, 9), ("q4_0", 700, 11008, 6),
-    ("f16", 2603, 2056, 7), ("f16", 4099, 5000, 5), ("f16", 9001, 2560, 16), ("f16", 15001, 4104, 17), ("f16", 15001, 4104, 32),
+    ("f16", 2603, 2056, 7), ("f16", 4099, 5000, 5), ("f16", 9001, 2560, 16), ("f16", 15001, 4104, 17), ("f16", 15001, 4104, 32), ("f16", 11000, 5632, 24),
     ("f32", 2603, 2052, 7), ("f32", 1501, 4100, 4)])
 @pytest.mark.parametrize("prologue", [None, "layernorm", "rmsnorm", "swiglu"])
 def test_linear_rows(ops, kind, rows, cols, m, prologue):
@@ -137,11 +137,22 @@ def test_wide_rows_and_many_columns(ops, oracle, kind, rows, cols, m, precision)
     w.free()
 
 
-@pytest.mark.parametrize("rows", [2, 3, 7])
-def test_short_prompt_equals_its_rows_one_by_one(ops, rows):
+# dim, ffn, heads: but for the first three, matrices of each are large enough for the launch at the rows beside it
+SHORT = [("llama", "q8_0", 512, 1024, 8, 2), ("llama", "q8_0", 512, 1024, 8, 3), ("llama", "q8_0", 512, 1024, 8, 7), ("llama", "q8_0", 2048, 5632, 32, 3), ("llama", "q4_0", 2048, 5632, 32, 7), ("llama", "f32", 2048, 2048, 16, 4),
+         ("gpt2", "f16", 1152, 4608, 18, 6), ("gpt2", "f16", 1024, 4096, 16, 7), ("gpt2", "q8_0", 2816, 1024, 22, 12), ("llama", "q4_0", 2048, 5632, 32, 16),
+         ("llama", "f16", 2048, 14848, 32, 17), ("llama", "f16", 2048, 14848, 32, 32)]
+
+
+@pytest.mark.parametrize("arch,kind,dim,ffn,heads,rows", SHORT)
+def test_short_prompt_equals_its_rows_one_by_one(ops, arch, kind, dim, ffn, heads, rows):
+    """A prompt of a few rows (thirds of the fused projection stored and split, or routed to the cache rows) against the decode step."""
     from caten_amd import _lib, llm, synth
-    cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], max_seq=700)
-    model = llm.make_llama(cfg, llm.llama_state_dict(synth.llama_weights(cfg, seed=3), "q8_0"))
+    if arch == "llama":
+        cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=dim, ffn=ffn, n_heads=heads, n_kv_heads=heads // 4, n_layers=2 if ffn < 9000 else 1, vocab=1000, max_seq=700)
+        model = llm.make_llama(cfg, llm.llama_state_dict(synth.llama_weights(cfg, seed=3), kind))
+    else:
+        cfg = dict(synth.GPT2_CONFIGS["gpt2-tiny"], dim=dim, ffn=ffn, n_heads=heads, vocab=1000, max_seq=700)
+        model = llm.make_gpt2(cfg, llm.gpt2_state_dict(synth.gpt2_weights(cfg, seed=3), kind))
     ids = [float(t) for t in synth.prompt(cfg["vocab"], 640 + rows, seed=3)]
     lib = _lib.load()
     model.forward(ids[:640], 640, 0)

@@ -62,3 +62,32 @@ def test_argmax_of_any_length(ops, rows, n):
     x[0, n - 1] = n  # the last element, which a row that is no multiple of four reads through an overlapping piece
     for _ in range(2):  # the counters behind a row's last part are back at zero
         assert np.array_equal(np.atleast_1d(ops.argmax(x)).ravel(), x.argmax(-1))
+
+
+@pytest.mark.parametrize("rows,n", [(4, 3), (5, 1025), (6, 8191), (5, 8193), (4, 50257), (17, 16385)])
+def test_argmax_of_rows_that_are_not_finite(ops, rows, n):
+    """Masked stretches and infinities are ordinary values, a NaN is never chosen; the lowest index where nothing is larger."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(0, 1, (rows, n)).astype(np.float32)
+    x[0, n // 2:] = -np.inf
+    x[1] = -np.inf
+    x[2, [1, n - 1]] = np.inf
+    x[3, rng.random(n) < 0.7] = np.nan
+    x[3, 0] = -np.inf
+    if rows > 4:
+        x[4] = np.nan
+    want = np.where(np.isnan(x), -np.inf, x).argmax(-1)
+    assert np.array_equal(ops.argmax(x).ravel(), want)
+
+
+@pytest.mark.parametrize("rows,n", [(3, 1024), (3, 2051), (2, 8193), (2, 53251), (1, 70001)])
+def test_layernorm_softmax_of_rows_that_are_not_finite(ops, rows, n):
+    """A row with an infinity or a NaN has no mean: NaN throughout, and the rows beside it what they are alone."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(0.3, 1, (rows, n)).astype(np.float32)
+    alone = ops.layernorm_softmax(x)
+    for bad in (np.inf, -np.inf, np.nan):
+        y = x.copy()
+        y[0, n - 1] = bad
+        got = ops.layernorm_softmax(y)
+        assert np.isnan(got[0]).all() and np.array_equal(got[1:], alone[1:])

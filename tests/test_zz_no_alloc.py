@@ -43,7 +43,7 @@ def test_noalloc_matmul_equals_matmul_twice_in_a_row(precision):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
         assert delta == (0, 0, 0), f"the allocator moved during the call: {delta}"
         ref = np.maximum(A.astype(np.float64) @ B.astype(np.float64), 0.0)
-        bad = np.abs(got - ref) > ATOL + RTOL * np.abs(ref)
+        bad = ~(np.abs(got - ref) <= ATOL + RTOL * np.abs(ref))
         assert not bad.any()
 
 
