@@ -5,7 +5,7 @@
 // scalar variables (runtime.lisp:228-259), the scalar nodes `:Add :Mul :Neg :Idiv :Mod :Max` compute dynamic shapes
 // and strides (runtime.lisp:396-449), and `:JIT_KERNEL` launches one compiled Schedule-Item and returns the arguments
 // at its out-positions (source/codegen/runner.lisp:20-32).  The reference runs that walk in compiled Lisp; a host
-// that is slower per node than a launch (150 launches of a GPT-2 decode step leave the device idle between them)
+// that is slower per node than a launch (the 150 kernel nodes of a GPT-2 decode step leave the device idle between them)
 // hands the list over once -- slots instead of variable names, programs instead of callers -- and asks for a whole
 // forward with one call.  Node kinds beyond these three (views, custom ops) stay with the host's own walk.
 //
