@@ -14,7 +14,8 @@
 // weight is an integer, exact in bf16, times its block's scale, which is applied to the block's partial sum; an fp16 weight
 // is two terms, exact; an fp32 weight three.  Products of terms below 2^-24 of the leading one are left out.
 // An infinity or a NaN stands in the last term, which meets the leading term of a weight only (infinity times a lower
-// term of zero would be NaN): it comes out as it does of fp32 products.
+// term of zero would be NaN): it comes out as it does of fp32 products.  Matrix cores take a term below 2^-126 for zero: a
+// row of nothing above 2^-32 goes in times 2^64.
 // Three terms per input, two where "gemm_precision" asks for operands rounded to bf16.
 //
 // K is shared among as many workgroups as fill the chip; a share leaves its partial sums in memory and draws a ticket, the
@@ -26,6 +27,7 @@ namespace cthip {
 
 struct RowsGemmArgs {
   const unsigned char *A;    // planes of the input rows: [M][nkb][NPA][32], nkb = whole units (zeros past K)
+  const float *rscale;       // per input row: what undoes its power of two
   int nkb;
   const unsigned char *W;    // N rows of packed weights, wpitch = wbytes apart
   const unsigned short *wd;  // scales, dpitch apart
@@ -299,8 +301,9 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
         const int m = 16 * i + 4 * grp + r;
         if (m >= M) continue;
         float *o = mine + m * NT + wave * NR + 16 * j + col;
-        if (shares) __hip_atomic_store(o, acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else *o = acc[i][j][r];
+        const float v = acc[i][j][r] * a.rscale[m];
+        if (shares) __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *o = v;
       }
   if (shares) {
     // a share's sums are device-scope stores that have reached memory before its ticket is drawn (a fence would write
@@ -346,6 +349,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
 // gemm_planes.hip.  kbp: blocks of 32 k per row of planes (zeros past K).
 struct RowsPlanesArgs {
   uint4 *out;
+  float *rscale;  // ROWS: what undoes a row's power of two
   const float *x;
   int64_t stride;
   int K, kbp;
@@ -354,7 +358,7 @@ struct RowsPlanesArgs {
 };
 template <int PRO, int NP, bool ROWS, int VPL>
 __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
-  __shared__ float red[2][4];
+  __shared__ float red[3][4];
   const int tid = threadIdx.x, K = a.K;
   const float *xr = a.x + blockIdx.x * a.stride;
   constexpr bool NORM = PRO == CTHIP_PRO_LAYERNORM || PRO == CTHIP_PRO_RMSNORM;
@@ -414,13 +418,27 @@ __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
       }
     }
   }
+  float up = 1.0f;
+  if (ROWS) {
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPL; j++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) m = in(j, e) && fabsf(v[j][e]) < INFINITY ? fmaxf(m, fabsf(v[j][e])) : m;
+    m = wave_max(m);
+    if ((tid & 63) == 0) red[2][tid >> 6] = m;
+    __syncthreads();
+    const bool small = fmaxf(fmaxf(red[2][0], red[2][1]), fmaxf(red[2][2], red[2][3])) < 0x1p-32f;
+    up = small ? 0x1p64f : 1.0f;
+    if (tid == 0) a.rscale[blockIdx.x] = small ? 0x1p-64f : 1.0f;
+  }
 #pragma unroll
   for (int j = 0; j < VPL; j++) {
     const int c = tid + 256 * j;
     if (c >= 4 * a.kbp) continue;
     float t[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] : 0.0f;
+    for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] * up : 0.0f;
     uint4 pl[NP];
     if (ROWS) split8_rows<NP>(t, pl);
     else split8_planes<NP>(t, pl);
@@ -532,7 +550,7 @@ bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, in
 // rows with what a Linear has in front of it as bf16 planes for gemm_planes.hip (x on 16 bytes, K % 32 == 0)
 bool rows_planes_supported(int K) { return K % 32 == 0 && K <= kRowsPlanesMaxK; }
 int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps) {
-  const RowsPlanesArgs pa = {(uint4 *)planes, x, K, K, K / 32, g, b, eps};
+  const RowsPlanesArgs pa = {(uint4 *)planes, nullptr, x, K, K, K / 32, g, b, eps};
   if (pro == CTHIP_PRO_LAYERNORM) rows_planes_launch<CTHIP_PRO_LAYERNORM, 2, false>(pa, m);
   else if (pro == CTHIP_PRO_RMSNORM) rows_planes_launch<CTHIP_PRO_RMSNORM, 2, false>(pa, m);
   else rows_planes_launch<CTHIP_PRO_NONE, 2, false>(pa, m);
@@ -569,10 +587,13 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
     a.e.route = *route;
   }
   unsigned char *planes = nullptr;
-  if (stream_capturing() || alloc_scratch((void **)&planes, (size_t)m * a.nkb * 64 * terms)) return 0;  // fully written by the first launch
+  const size_t plane_bytes = (size_t)m * a.nkb * 64 * terms;
+  if (stream_capturing() || alloc_scratch((void **)&planes, plane_bytes + sizeof(float) * kRowsMax)) return 0;  // fully written by the first launch
+  float *rscale = (float *)(planes + plane_bytes);
+  a.rscale = rscale;
   int rc = 0;
   a.A = planes;
-  const RowsPlanesArgs pa = {(uint4 *)planes, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
+  const RowsPlanesArgs pa = {(uint4 *)planes, rscale, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
 #define RP2(PRO)                                              \
   do {                                                        \
     if (terms == 3) rows_planes_launch<PRO, 3, true>(pa, m);  \

@@ -74,6 +74,7 @@ def test_inputs_of_any_magnitude(ops, kind, rows, cols, m, outlier):
     x[:, 5], x[:, cols - 7] = outlier, -outlier
     x[1] *= np.float32(2.0 ** -60)
     x[1, 5], x[1, cols - 7] = 1.0, 2.0 ** -70
+    x[2] = rng.normal(0, 1, cols) * 2.0 ** -126  # subnormal numbers among them: a term of 16-bit hardware takes them for zero
     w64 = w.dequantize().astype(np.float64)
     assert not w64[:, 5].any() and not w64[:, cols - 7].any()
     got = ops.linear(x, w)
