@@ -132,6 +132,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
   };
   // ---- the share of the input rows -> LDS behind the rings: row r's chunk c (16 bytes) at r * cpr + (c ^ (r & 7)) ----
   __shared__ int s_ticket;
+  __shared__ float s_scale[64];  // of the rows (requested here: read from memory at the end it cost every launch 3 us)
+  if (wave == 0) dma4(a.rscale, (unsigned)lane * 4u, (unsigned)(size_t)(__attribute__((address_space(3))) float *)s_scale);
   const unsigned char *As = smem + NW * PD * SLOT;
   const int cpr = kbs * 4 * NPA;
   for (int r = wave; r < M; r += NW) {
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
         const int m = 16 * i + 4 * grp + r;
         if (m >= M) continue;
         float *o = mine + m * NT + wave * NR + 16 * j + col;
-        const float v = acc[i][j][r] * a.rscale[m];
+        const float v = acc[i][j][r] * s_scale[m];
         if (shares) __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else *o = v;
       }
@@ -347,6 +349,9 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
 // ---- input rows -> planes, with what the Linear has in front ----
 // One block per row, held in registers (VPL pieces of 8 floats per thread).  ROWS: terms for k_linear_rows, else for
 // gemm_planes.hip.  kbp: blocks of 32 k per row of planes (zeros past K).
+// A few rows are a few blocks on cold compute units: what bounds those is the fetch of their own unrolled code and one wavefront's
+// chain, so a block has as many threads as its row has pieces (up to 1024).  5 rows of 11008 with SwiGLU, 256 threads of 8 pieces -> 1024
+// of 2: 9.5 -> 6.4 us.
 struct RowsPlanesArgs {
   uint4 *out;
   float *rscale;  // ROWS: what undoes a row's power of two
@@ -356,19 +361,20 @@ struct RowsPlanesArgs {
   const float *g, *b;
   float eps;
 };
-template <int PRO, int NP, bool ROWS, int VPL>
-__global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
-  __shared__ float red[3][4];
+template <int PRO, int NP, bool ROWS, int NT, int VPL>
+__global__ __launch_bounds__(NT) void k_rows_planes(RowsPlanesArgs a) {
+  constexpr int NW = NT / 64;
+  __shared__ float red[3][NW];
   const int tid = threadIdx.x, K = a.K;
   const float *xr = a.x + blockIdx.x * a.stride;
   constexpr bool NORM = PRO == CTHIP_PRO_LAYERNORM || PRO == CTHIP_PRO_RMSNORM;
   float v[VPL][8];
   auto ld8 = [&](const float *p, int j, float *o) __attribute__((always_inline)) {  // K % 4 == 0: four floats are inside the row or past it
-    const int k = 8 * (tid + 256 * j);
+    const int k = 8 * (tid + NT * j);
     const float4 t0 = *(const float4 *)(p + min(k, K - 4)), t1 = *(const float4 *)(p + min(k + 4, K - 4));
     o[0] = t0.x, o[1] = t0.y, o[2] = t0.z, o[3] = t0.w, o[4] = t1.x, o[5] = t1.y, o[6] = t1.z, o[7] = t1.w;
   };
-  auto in = [&](int j, int e) { return 8 * (tid + 256 * j) + e < K; };
+  auto in = [&](int j, int e) { return 8 * (tid + NT * j) + e < K; };
 #pragma unroll
   for (int j = 0; j < VPL; j++) ld8(xr, j, v[j]);
   if (PRO == CTHIP_PRO_SWIGLU) {
@@ -384,7 +390,10 @@ __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
     s = wave_sum(s);
     if ((tid & 63) == 0) red[slot][tid >> 6] = s;
     __syncthreads();
-    return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
+    s = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w += 2) s += red[slot][w] + red[slot][w + 1];
+    return s;
   };
   if (NORM) {
     const float inv_n = 1.0f / (float)K;
@@ -418,8 +427,23 @@ __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
       }
     }
   }
-  float up = 1.0f;
-  if (ROWS) {
+  auto emit = [&](float up) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < VPL; j++) {
+      const int c = tid + NT * j;
+      if (c >= 4 * a.kbp) continue;
+      float t[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] * up : 0.0f;
+      uint4 pl[NP];
+      if (ROWS) split8_rows<NP>(t, pl);
+      else split8_planes<NP>(t, pl);
+#pragma unroll
+      for (int q = 0; q < NP; q++) a.out[((int64_t)blockIdx.x * a.kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
+    }
+  };
+  emit(1.0f);
+  if (ROWS) {  // behind the stores, which then need not wait for the whole row: one of small numbers is stored again
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < VPL; j++)
@@ -428,25 +452,14 @@ __global__ __launch_bounds__(256) void k_rows_planes(RowsPlanesArgs a) {
     m = wave_max(m);
     if ((tid & 63) == 0) red[2][tid >> 6] = m;
     __syncthreads();
-    const bool small = fmaxf(fmaxf(red[2][0], red[2][1]), fmaxf(red[2][2], red[2][3])) < 0x1p-32f;
-    up = small ? 0x1p64f : 1.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) m = fmaxf(m, red[2][w]);
+    const bool small = m < 0x1p-32f;
+    if (small) emit(0x1p64f);
     if (tid == 0) a.rscale[blockIdx.x] = small ? 0x1p-64f : 1.0f;
   }
-#pragma unroll
-  for (int j = 0; j < VPL; j++) {
-    const int c = tid + 256 * j;
-    if (c >= 4 * a.kbp) continue;
-    float t[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) t[e] = in(j, e) ? v[j][e] * up : 0.0f;
-    uint4 pl[NP];
-    if (ROWS) split8_rows<NP>(t, pl);
-    else split8_planes<NP>(t, pl);
-#pragma unroll
-    for (int q = 0; q < NP; q++) a.out[((int64_t)blockIdx.x * a.kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
-  }
 }
-constexpr int kRowsPlanesMaxK = 8 * 256 * 16;  // widest row the largest instantiation holds
+constexpr int kRowsPlanesMaxK = 8 * 1024 * 4;  // widest row the largest instantiation holds
 
 // How many workgroups share K, as units per share, and the LDS such a workgroup asks for.  Every compute unit holds `resident`
 // workgroups (LDS) at a time; a round of them costs its units at the rate of the compute unit (about 0.85 us per 16 KB of weights
@@ -505,14 +518,13 @@ static int rows_launch(RowsGemmArgs a, bool *done) {
 
 template <int PRO, int NP, bool ROWS>
 static void rows_planes_launch(const RowsPlanesArgs &a, int m) {
-  const int pieces = (a.kbp * 4 + 255) / 256;
-  const dim3 grid(m), block(256);
-#define RP(V) hipLaunchKernelGGL((k_rows_planes<PRO, NP, ROWS, V>), grid, block, 0, state().stream, a)
-  if (pieces <= 1) RP(1);
-  else if (pieces <= 2) RP(2);
-  else if (pieces <= 4) RP(4);
-  else if (pieces <= 8) RP(8);
-  else RP(16);
+  const int pieces = a.kbp * 4;
+#define RP(NT, V) hipLaunchKernelGGL((k_rows_planes<PRO, NP, ROWS, NT, V>), dim3(m), dim3(NT), 0, state().stream, a)
+  if (pieces <= 256) RP(256, 1);
+  else if (pieces <= 512) RP(512, 1);
+  else if (pieces <= 1024) RP(1024, 1);
+  else if (pieces <= 2048) RP(1024, 2);
+  else RP(1024, 4);
 #undef RP
 }
 
@@ -524,11 +536,11 @@ static bool rows_wide_scales(const WMat *w) { return w->cols / 32 % 2 == 0 && ro
 // Whether this is the launch to take: the operands are laid out for it, a share of it fits a workgroup, and it is the faster one.
 // Fewer than 8 rows: against the single-row kernels, one pass over the weights per row.  They cost about 3 us + m weights
 // at 4.3 (quantised), 2.7 (fp16) or 2.0 (fp32) per ns, the two launches here 9.5 us + the weights once at 3.2 / 2.3 / 1.15.
-//   us, m = 3 / 5 / 7, weights not in any cache:  22016 x 4096 Q8_0 49 / 73 / 98 -> 30 / 34 / 35, fp32 158 / 261 / 368 -> 86 / 89 / 103;
-//   4096 x 4096 Q8_0 m = 5 / 7 23 / 29 -> 12 / 12;  4096 x 11008 Q4_0 m = 5 44 -> 19;  768 x 3072 stays there at 5 / 7 (6 / 7; 11 here)
+//   us, m = 3 / 5 / 7, weights not in any cache:  22016 x 4096 Q8_0 49 / 73 / 98 -> 31 / 33 / 33, fp32 158 / 261 / 368 -> 86 / 89 / 103;
+//   4096 x 4096 Q8_0 m = 5 / 7 23 / 29 -> 13 / 13;  4096 x 11008 Q4_0 m = 5 44 -> 20;  768 x 3072 stays there at 5 / 7 (6 / 7; 11 here)
 // 8 rows and more: against a GEMM tile of 64 rows, which is as fast on small matrices and where the tile fills up:
-//   22016 x 4096 m = 12: Q8_0 51 -> 37, Q4_0 52 -> 35, fp16 74 -> 49;  fp16 m = 24 / 32 74 / 74 -> 61 / 73;
-//   11264 x 2048 m = 12: Q8_0, Q4_0, fp16 20, 20, 26 -> 15, 15, 19;  4096 x 4096 m = 12: 15, 14, 18 -> 14, 14, 16.
+//   22016 x 4096 m = 12: Q8_0 51 -> 38, Q4_0 52 -> 36, fp16 74 -> 49;  fp16 m = 24 / 32 74 / 74 -> 61 / 73;
+//   11264 x 2048 m = 12: Q8_0, Q4_0, fp16 20, 20, 26 -> 16, 16, 19;  4096 x 4096 m = 12: 15, 14, 18 -> 14, 14, 16.
 // Of 14 - 16 rows as long as 11008 a workgroup's memory holds a share too small for one round over the chip: Q8_0 m = 14 / 16
 // 25 / 26 -> 22 / 28; they are taken for their bits (the tiles' error is 2.4e-6 there, 1.3e-7 here).
 bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b) {
@@ -588,7 +600,7 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
   }
   unsigned char *planes = nullptr;
   const size_t plane_bytes = (size_t)m * a.nkb * 64 * terms;
-  if (stream_capturing() || alloc_scratch((void **)&planes, plane_bytes + sizeof(float) * kRowsMax)) return 0;  // fully written by the first launch
+  if (stream_capturing() || alloc_scratch((void **)&planes, plane_bytes + sizeof(float) * 64)) return 0;  // fully written by the first launch
   float *rscale = (float *)(planes + plane_bytes);
   a.rscale = rscale;
   int rc = 0;
