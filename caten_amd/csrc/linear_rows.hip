@@ -253,9 +253,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
 #pragma unroll
         for (int j = 0; j < NS; j++)
 #pragma unroll
-          for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(dd[j][b], tmp[j][b][r], acc[i][j][r]);
+          // the pair's two meet first: half the roundings at the size of the total (Q8_0, 4096 columns: error 1.17e-7 -> 1.10e-7)
+          for (int r = 0; r < 4; r++) acc[i][j][r] += fmaf(dd[j][0], tmp[j][0][r], dd[j][1] * tmp[j][1][r]);
       }
     } else {
 #pragma unroll
