@@ -91,7 +91,7 @@ __global__ __launch_bounds__(128 * NW) void k_attn_planes(AttnPlanesArgs a) {
     const int p = (wv * LD + j) * 64 + lane;  // chunk of the buffer: keys of both tiles, then values of both
     isv[j] = wv * LD + j >= 2 * KT / 1024;
     const int pk = isv[j] ? p - 2 * KT / 16 : p, cpr = isv[j] ? 8 : CK, r = pk / cpr, c = pk % cpr;
-    voff[j] = (unsigned)(r * cpr + (c ^ (r & 7))) * 16u;
+    voff[j] = (unsigned)(r * cpr + (c ^ (isv[j] ? (r >> 1) & 7 : r & 15))) * 16u;  // (which lanes a read serves together: swz in gemm_planes.hip)
   }
   const unsigned char *kbase = a.kp + (int64_t)hk * a.nkb * KT, *vbase = a.vp + (int64_t)hk * a.nkb * KT;
   auto issue = [&](int t, int buf) __attribute__((always_inline)) {
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(128 * NW) void k_attn_planes(AttnPlanesArgs a) {
     v16f s0, s1;
 #pragma unroll
     for (int r = 0; r < 16; r++) s0[r] = s1[r] = 0.0f;
-    auto kld = [&](int term, int s) { return __builtin_bit_cast(v8bf, *(const uint4 *)(Kt + (col * CK + ((term * (DH / 8) + 2 * s + half) ^ (col & 7))) * 16)); };
+    auto kld = [&](int term, int s) { return __builtin_bit_cast(v8bf, *(const uint4 *)(Kt + (col * CK + ((term * (DH / 8) + 2 * s + half) ^ (col & 15))) * 16)); };
 #pragma unroll
     for (int s = 0; s < NSL; s++) {
       const v8bf kh = kld(0, s), kl = kld(1, s);
@@ -181,8 +181,8 @@ __global__ __launch_bounds__(128 * NW) void k_attn_planes(AttnPlanesArgs a) {
 #pragma unroll
       for (int d = 0; d < DB; d++) {
         const int row = 32 * d + col;
-        const v8bf vh = __builtin_bit_cast(v8bf, *(const uint4 *)(Vt + (row * 8 + ((2 * t2 + half) ^ (row & 7))) * 16));
-        const v8bf vl = __builtin_bit_cast(v8bf, *(const uint4 *)(Vt + (row * 8 + ((4 + 2 * t2 + half) ^ (row & 7))) * 16));
+        const v8bf vh = __builtin_bit_cast(v8bf, *(const uint4 *)(Vt + (row * 8 + ((2 * t2 + half) ^ ((row >> 1) & 7))) * 16));
+        const v8bf vl = __builtin_bit_cast(v8bf, *(const uint4 *)(Vt + (row * 8 + ((4 + 2 * t2 + half) ^ ((row >> 1) & 7))) * 16));
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vl, ph, o[d], 0, 0, 0);
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, pw, o[d], 0, 0, 0);
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, ph, o[d], 0, 0, 0);

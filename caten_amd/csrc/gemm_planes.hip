@@ -18,11 +18,16 @@
 
 namespace cthip {
 
-// 16-byte chunk c of row r of an LDS tile with CPR chunks per row is kept at chunk r * CPR + (c ^ swz<CPR>(r)): eight
-// consecutive rows then read (or are written) eight different 16-byte columns of the banks.
-template <int CPR>
+// 16-byte chunk c of row r of an LDS tile with CPR chunks per row is kept at chunk r * CPR + (c ^ swz<CPR>(r)).  A 16-byte read
+// is served sixteen lanes at a time over 64 banks (256 bytes): of lanes 0 .. 31, each reading the same chunk of its own row,
+// {0-3, 12-15, 20-27} and then {4-11, 16-19, 28-31}, and the same of lanes 32 .. 63 (timed on the card).  With SPREAD the sixteen rows of
+// such a set lie in sixteen different columns of the banks; without, which is right for eight consecutive rows over 128 bytes, a read
+// takes twice its cycles.
+template <int CPR, bool SPREAD>
 __device__ __forceinline__ int swz(int r) {
-  return CPR % 8 == 0 ? (r & 7) : CPR % 4 == 0 ? ((r >> 1) & 3) : CPR % 2 == 0 ? ((r >> 2) & 1) : 0;
+  static_assert(CPR % 4 == 0, "whole blocks of 32 k");
+  if (SPREAD) return CPR % 8 == 0 ? ((r >> 1) & 7) : ((r >> 2) & 3);
+  return CPR % 8 == 0 ? (r & 7) : ((r >> 1) & 3);
 }
 
 // SRC: how B lies in memory: PL_PLANES, or PL_INT, one plane of the integers of a quantised matrix (exact in bf16) with an
@@ -32,14 +37,18 @@ __device__ __forceinline__ int swz(int r) {
 // What bounds it: the matrix cores ask LDS for an operand per instruction and block edge, so a wavefront's piece wants to be
 // large (64 x 64: 16 reads for 24 instructions at two terms); two workgroups of four wavefronts per compute unit fill each
 // other's waits (reading a step's operands under the step before it instead, two sets of registers, measured the same or
-// slower; so did deeper rings than the launcher's).  4096^3, two terms: 310 us without the passes in front = 440 TFLOP/s of
-// results, 1.3 PFLOP/s of matrix instructions (the library's bf16 product reaches 1.2 - 1.5 on the card), against 180 with
-// the operands converted per tile.  Integers need two products instead of three but 16 multiply-adds per lane and block for
-// the scales: 1900 x 11264 x 2048 240 us (two per tile before: 340), 1900 x 2048 x 5632 128 us (149).
+// slower; so did deeper rings than the launcher's).  4096^3, two terms: 284 us without the passes in front = 484 TFLOP/s of
+// results, 1.45 PFLOP/s of matrix instructions (the library's bf16 product reaches 1.2 - 1.5 on the card: the clock falls to 1.6 GHz under
+// them), against 180 with the operands converted per tile.  Integers need two products instead of three but 16 multiply-adds per lane and block for
+// the scales: 1900 x 11264 x 2048 194 us (operands converted per tile: 340), 1900 x 2048 x 5632 117 us (149).
 template <int NPA, int SRC, int NPB, int MB, int NB, int WM, int WN, int NBUF>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN;
   constexpr int CA = 4 * NPA, CB = 4 * NPB;  // chunks per row and step
+  // Reads without conflicts are the faster ones (4096^3, two terms, 256 x 256 tiles: 354 -> 346 us; 128 x 128 of eight wavefronts: 392 -> 376; integers,
+  // 1900 x 2048 x 5632: 126 -> 117) but in two tiles of four wavefronts, two workgroups to a compute unit, for a reason no counter shows: 64 x 64 a wavefront
+  // at two terms (4096^3 357 -> 390, 3000 x 4100 x 5000 391 -> 435) and 64 x 32 at three (700 x 4500 x 800 49.9 -> 51.1).
+  constexpr bool SPREAD = !(SRC == PL_PLANES && NW == 4 && MB == 2 && ((NPA == 2 && NB == 2) || (NPA == 3 && NB == 1)));
   constexpr int ABYTES = BM * CA * 16, BBYTES = BN * CB * 16, SBYTES = SRC == PL_PLANES ? 0 : BN * 4;
   constexpr int BUF = ABYTES + BBYTES + SBYTES;
   constexpr int IA = (BM * CA / 64 + NW - 1) / NW, IB = (BN * CB / 64 + NW - 1) / NW;  // load instructions per wavefront and step
@@ -62,12 +71,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
   unsigned avo[IA], bvo[IB], svo[IS > 0 ? IS : 1];
 #pragma unroll
   for (int j = 0; j < IA; j++) {
-    const int s = ((j * NW + wave) * 64 + lane) % (BM * CA), r = s / CA, c = (s % CA) ^ swz<CA>(r);
+    const int s = ((j * NW + wave) * 64 + lane) % (BM * CA), r = s / CA, c = (s % CA) ^ swz<CA, SPREAD>(r);
     avo[j] = (unsigned)(min(r, a.M - 1 - m0) * a.apitch + c * 16);
   }
 #pragma unroll
   for (int j = 0; j < IB; j++) {
-    const int s = ((j * NW + wave) * 64 + lane) % (BN * CB), r = s / CB, c = (s % CB) ^ swz<CB>(r);
+    const int s = ((j * NW + wave) * 64 + lane) % (BN * CB), r = s / CB, c = (s % CB) ^ swz<CB, SPREAD>(r);
     bvo[j] = (unsigned)(min(r, a.N - 1 - n0) * a.bpitch + c * 16);
   }
 #pragma unroll
@@ -105,8 +114,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
   auto mul = [&](int buf) __attribute__((always_inline)) {
     const unsigned char *At = smem + buf * BUF, *Bt = At + ABYTES;
     const int ra = 32 * MB * wm + col, rb = 32 * NB * wn + col;
-    auto lda = [&](int i, int ch) { return *(const uint4 *)(At + ((ra + 32 * i) * CA + (ch ^ swz<CA>(ra))) * 16); };
-    auto ldb = [&](int b, int ch) { return *(const uint4 *)(Bt + ((rb + 32 * b) * CB + (ch ^ swz<CB>(rb))) * 16); };
+    auto lda = [&](int i, int ch) { return *(const uint4 *)(At + ((ra + 32 * i) * CA + (ch ^ swz<CA, SPREAD>(ra))) * 16); };
+    auto ldb = [&](int b, int ch) { return *(const uint4 *)(Bt + ((rb + 32 * b) * CB + (ch ^ swz<CB, SPREAD>(rb))) * 16); };
     // The operands of a slice are read before the slice in front of it is multiplied, behind a scheduling fence: left alone
     // the compiler puts every LDS read right in front of its use, and each pair of matrix instructions waits out an LDS
     // round trip.
@@ -344,19 +353,20 @@ static int planes_launch(PlaneGemmArgs a) {
 }
 
 // Which tile: the one whose rounds over the chip cost least.  A compute unit holds `resident` workgroups; alone a workgroup
-// reaches `one`, together they reach `all` (TFLOP/s of results, measured at 1024^3, 2000^3 and 4096^3; one term runs at 2.4 times
-// the rate of two).
+// reaches `one`, together they reach `all` (TFLOP/s of results, measured at 1536^3, 2048^3 and 4096^3).
 struct PlaneTile {
   int bm, bn, resident;
   double one, all;
+  double idle = 1.0;  // share of a round's time that a single tile takes in the last one
 };
 static double plane_tile_us(const PlaneTile &t, const PlaneGemmArgs &a, int cus) {
   const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn), slots = (int64_t)cus * t.resident;
   const double work = 2.0 * t.bm * t.bn * 32.0 * a.nkb * cus * 1e-6;  // MFLOP of a tile on every compute unit
   const int64_t full = tiles / slots, left = tiles - full * slots;
   double us = 2.0 + full * work * t.resident / t.all;
-  if (left <= cus) {
-    if (left) us += work / t.one;
+  if (t.resident == 1) us += (double)a.M * a.N * 4e-7;  // nothing runs under the stores (4500 x 4500 x 600 at one term: 63 us in tiles of 128, 73 of 256)
+  if (left <= cus) {  // (large tiles are bound by power, the fewer of them the higher the clock; a few small ones start under the round before)
+    if (left) us += work / t.one * (full || t.resident == 1 ? t.idle + (1.0 - t.idle) * (double)left / cus : 1.0);
   } else {  // between one tile per compute unit and a full round, steeper at the start: the shared units wait for both
     const double one = work / t.one, all = work * t.resident / t.all;
     us += one + (all - one) * (0.4 + 0.6 * (double)(left - cus) / (double)(slots - cus));
@@ -369,10 +379,14 @@ static double plane_tile_us(const PlaneTile &t, const PlaneGemmArgs &a, int cus)
 static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *estimate) {
   const int cus = state().compute_units;
   const bool q = a.bd != nullptr;
-  static const PlaneTile plane[] = {{64, 64, 2, 190, 267}, {128, 64, 3, 205, 320}, {128, 128, 2, 300, 345}, {128, 128, 2, 258, 371}, {256, 256, 1, 366, 366}};
-  static const PlaneTile plane6[] = {{64, 64, 3, 110, 160}, {128, 64, 2, 110, 170}, {128, 256, 1, 205, 205}};
+  // one term: 4096^3 in tiles of 64 x 64 .. 256 x 256 337, 265, 209, 202, 160 us, 2048^3 56, 49, 45, 46, 72, 1536^3 34, 36, 37, 39, 61
+  static const PlaneTile plane1[] = {{64, 64, 2, 330, 480, 0.5}, {128, 64, 3, 400, 650}, {128, 128, 2, 600, 880}, {128, 128, 2, 600, 922}, {256, 256, 1, 1290, 1290, 0.76}};
+  // two: 4096^3 580, 428, 376, 357, 346 us, 2048^3 81, 70, 69, 77, 137, 1536^3 45, 47, 51, 55, 109
+  static const PlaneTile plane[] = {{64, 64, 2, 200, 275, 0.5}, {128, 64, 3, 230, 365}, {128, 128, 2, 353, 438}, {128, 128, 2, 307, 469}, {256, 256, 1, 490, 490, 0.76}};
+  // three: 3000 x 4100 x 5000 883, 795, 732, 4096^3 1026, 861, 655
+  static const PlaneTile plane6[] = {{64, 64, 3, 110, 160}, {128, 64, 2, 110, 170}, {128, 256, 1, 205, 205, 0.6}};
   static const PlaneTile ints[] = {{64, 64, 4, 240, 245}, {128, 128, 2, 370, 400}, {128, 192, 2, 368, 430}};
-  const PlaneTile *tiles = q ? ints : terms == 3 ? plane6 : plane;
+  const PlaneTile *tiles = q ? ints : terms == 3 ? plane6 : terms == 2 ? plane : plane1;
   const int n = q || terms == 3 ? 3 : 5;
   int pick = 0;
   double us = 1e30;
@@ -381,7 +395,7 @@ static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *e
     if (t < us) us = t, pick = i;
   }
   if (estimate) {
-    *estimate = q ? us * terms / 2.0 + 4.0 : terms == 1 ? us * 0.42 + 10.0 : us + 2.0;
+    *estimate = q ? us * terms / 2.0 + 4.0 : us + 2.0;
     return 0;
   }
 #define T(NPA, SRC, NPB, MB, NB, WM, WN) return planes_launch<NPA, SRC, NPB, MB, NB, WM, WN, 2>(a)

@@ -18,7 +18,8 @@ def ops():
 
 @pytest.mark.parametrize("precision,tol", [("bf16x6", 2.0 ** -20), ("bf16x3", 2.0 ** -15), ("bf16", 2.0 ** -7)])
 @pytest.mark.parametrize("m,n,k", [(73, 2786, 631), (131, 2895, 2001), (1803, 131, 640), (1501, 2767, 72), (2355, 1286, 90), (2562, 1165, 67),
-                                   (2722, 2401, 65), (4095, 3071, 129), (1500, 1500, 1500)])
+                                   (2722, 2401, 65), (4095, 3071, 129), (1500, 1500, 1500),
+                                   (3001, 4099, 1605)])
 def test_matmul_planes(ops, m, n, k, precision, tol):
     rng = np.random.default_rng(m + k)
     a, b = rng.normal(0, 1, (m, k)).astype(np.float32), rng.normal(0, 1, (k, n)).astype(np.float32)
