@@ -89,6 +89,7 @@ struct WMat {
   // the single-row kernels request this matrix with the non-temporal hint: set for a matrix that cannot stay in
   // the Infinity Cache between two uses (too large by itself, or one of a model's that together are too large)
   bool stream;
+  bool stream_far = false;  // ... by so much that next to nothing of the cache is lost to it
   // a LayerNorm folded through the product (cthip_wmat_fold_layernorm): fold_s = W.gamma, fold_c = W.beta + bias,
   // valid for exactly these gamma / beta / bias vectors
   const float *fold_g = nullptr, *fold_b = nullptr, *fold_bias = nullptr;
@@ -204,6 +205,9 @@ int launch_gemv(const WMat *w, GemvArgs a, int m);
 // the same Linear by the wide-row kernel (gemv_wide.hip: input vector in LDS); a.q / a.d / a.rows / a.cols are set here
 bool gemv_wide_supported(const WMat *w, const GemvArgs &a);
 int launch_gemv_wide(const WMat *w, GemvArgs a, int m);
+// the same by integer matrix instructions (gemv_int.hip)
+bool gemv_int_supported(const WMat *w, const GemvArgs &a);
+int launch_gemv_int(const WMat *w, GemvArgs a, int m, int *am_parts);  // am_parts: partial (value, row) pairs of the fused argmax
 int wmat_create_impl(WMat **out, int type, const void *raw, int64_t rows, int64_t cols);
 // true when a register-resident GEMV variant covers the matrix (no temporary is allocated at launch)
 bool gemv_is_direct(const WMat *w);

@@ -407,7 +407,10 @@ static int finalize(Decoder *d) {
     int64_t total = 0;
     for (WMat *w : ws) total += w ? w->q_bytes + w->d_bytes : 0;
     for (WMat *w : ws)
-      if (w) w->stream = total > kInfinityCacheBytes / 4 * 3;
+      if (w) {
+        w->stream = total > kInfinityCacheBytes / 4 * 3;
+        w->stream_far = total > 8 * kInfinityCacheBytes;
+      }
   }
   if (c.arch == CTHIP_ARCH_GPT2 && state().decode_flow && !d->kvq && !d->kvp) {
     bool ok = true;

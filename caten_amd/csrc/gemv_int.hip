@@ -1,0 +1,294 @@
+// Single-row Linear on 4-bit quantised rows, multiplied as integers on the matrix cores.
+//
+// The vector kernels (gemv_kernels.h, gemv_wide.hip) spend 2.4 - 7.8 vector instructions on a weight -- a conversion, a
+// multiply-add, their share of the prologue -- which at one wavefront per SIMD is as much time as the weights take to arrive.
+// Here the input vector is written as four signed base-256 digits per element (30 bits below the largest value of its chunk, the block of 32
+// that meets 16 bytes of weights, with a power of two for each), nibbles go to v_mfma_i32_16x16x64_i8 as bytes (one or two
+// bit operations per four of them), and the products and their sums over a chunk are exact integers:
+//   sum q x = 2^e (((i0 256 + i1) 256 + i2) 256 + i3),  i_r = sum over the chunk of q * digit r.
+// Digits are the rows of the first operand, weight rows the columns of the second: lane l holds 16 bytes of weight row l % 16, the (l / 16)-th chunk of
+// an instruction, and only rows 4 (l / 16) + r of that chunk's k carry digit r (the other twelve are zeros), so that lane l of the
+// result holds the four digit sums of its own row and chunk -- the chunk whose scale it has fetched.  25 vector instructions per
+// 2048 weights.  (8-bit rows arrive no faster than the vector kernels multiply them: 12288 x 4096 15.0 us this way, 14.4 theirs.)
+//
+// K is shared among the ks wavefronts of a workgroup (a unit of 128 bytes of each of 16 rows at a time, whole cache lines of
+// a row), rgp such sets work on neighbouring groups of 16 rows; a workgroup goes over its groups with PD units in flight per
+// wavefront and meets once, for the sums of them all.  What bounds it: the weights, behind 3.5 us of launch, the vector's way into LDS and the meeting at
+// the end (22016 x 4096, 50.7 MB: 13.2 us).  Errors against 64 bits, 4096 columns: 0.6 - 1.2e-7; the vector kernels, which take nibbles times
+// inputs less eight times the inputs' sum, 2 - 5e-7.
+#include "common.h"
+#include "gemv_kernels.h"
+#include "gemv_plan.h"
+
+namespace cthip {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// four consecutive k of a chunk (eight neighbouring lanes hold one): digit words of the four elements, and what undoes the
+// chunk's power of two.  A chunk with an infinity or a NaN keeps its sign there and nothing else: 2^e becomes infinity / NaN.
+__device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
+  unsigned m = 0;
+#pragma unroll
+  for (int e = 0; e < 4; e++) m = max(m, __float_as_uint(v[e]) & 0x7fffffffu);  // (as integers: a NaN is the largest)
+  m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xf, 0xf, true));   // quad_perm 1, 0, 3, 2
+  m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xf, 0xf, true));   // quad_perm 2, 3, 0, 1
+  m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));  // row_half_mirror
+  const unsigned E = max(m >> 23, 30u);  // nothing below the smallest normal number is kept
+  const bool finite = m < 0x7f800000u;
+  const float up = __uint_as_float((finite ? 283u - E : 0u) << 23);
+  unsigned t[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    int x = (int)rintf(v[e] * up);
+    if (!finite) x = (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u ? ((int)__float_as_uint(v[e]) < 0 ? -1 : 1) << 24 : 0;
+    t[e] = ((unsigned)x + 0x808080u) ^ 0x808080u;  // bytes: signed digits, the highest in byte 3
+  }
+  const unsigned a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
+  const unsigned b01 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u), b23 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+  w[0] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
+  w[1] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+  w[2] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+  w[3] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+  return m > 0x7f800000u ? __uint_as_float(0x7fc00000u) : finite ? __uint_as_float((E - 29u) << 23) : INFINITY;
+}
+
+struct GemvIntShape {
+  int upw, ks, rgp;        // units per wavefront and group; wavefronts sharing a group; groups a workgroup works on together
+  int inv_ks, inv_rows;    // 65536 / ks, 65536 / (16 rgp), rounded up: quotients of numbers below 1024
+};
+
+template <int PRO, bool NT>
+__global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) {
+  constexpr int PD = 2;              // units in flight per wavefront (four: no faster stream, 0.8 us more code to get through)
+  constexpr bool RMS = PRO == CTHIP_PRO_RMSNORM, LAYERNORM = PRO == CTHIP_PRO_LAYERNORM;
+  constexpr int CB = 128;            // bytes of digits per chunk: [half of its k][digit][16 bytes]
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, g = lane >> 4, i = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), sub = (wv * sh.inv_ks) >> 16, wk = wv - sub * sh.ks, nw = sh.ks * sh.rgp;
+  const int nchunks = a.cols >> 5, n4 = a.cols >> 2;
+  const int cpad = sh.ks * sh.upw * 8;  // chunks that the wavefronts go over: zeros past the row
+  // LDS: 256 bytes of zeros, digits, a scale per chunk, reductions, the groups' partial sums
+  unsigned char *dig = smem + 256;
+  float *sx = (float *)(dig + (size_t)cpad * CB), *red = sx + cpad, *ps = red + 32;
+  const int m = blockIdx.y;
+  const float *__restrict__ x = a.x + (int64_t)m * a.x_stride;
+  const int rows_sg = 16 * sh.rgp, nsg = (a.rows + rows_sg - 1) / rows_sg;
+  const int iters = (nsg - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int posv = a.pos ? a.pos[0] : 0;
+
+  // ---- the row this thread finishes (the plan: no more of them than threads), and what it needs for that ----
+  const int oj = (tid * sh.inv_rows) >> 16, oi = tid - oj * rows_sg, orow = ((int)blockIdx.x + oj * (int)gridDim.x) * rows_sg + oi;
+  const float *zf = (const float *)g_gemv_zeros;
+  const int orc = min(orow, a.rows - 1);
+  const float *pb = a.bias ? a.bias + orc : zf, *pr = a.residual ? a.residual + (int64_t)m * a.y_stride + orc : zf, *pf = a.fold_s ? a.fold_s + orc : zf;
+
+  // ---- the input vector is asked for, then the first units of weights ----
+  constexpr int SB = 3;
+  const float4 *x4 = (const float4 *)x;
+  const float4 *u4 = (RMS || LAYERNORM) && a.norm_g ? (const float4 *)a.norm_g : x4;
+  float4 xv[SB], uv[SB];
+  auto ask = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < SB; b++) {
+      const int k = min(i0 + nthr * b, n4 - 1);
+      xv[b] = x4[k];
+      if (RMS || LAYERNORM) uv[b] = u4[k];
+    }
+  };
+  ask(tid);
+  const float ob = *pb, orr = *pr, of = *pf;
+
+  const uint4 *__restrict__ qp = (const uint4 *)a.q;
+  uint4 wt[PD][2];
+  unsigned st[PD];  // the scales of both chunks
+  const int nu = iters * sh.upw;  // units of this wavefront
+  int rq_j = 0, rq_u = 0;         // the next one to ask for
+  auto request = [&](int p) __attribute__((always_inline)) {
+    const int row = min(((int)blockIdx.x + rq_j * (int)gridDim.x) * rows_sg + 16 * sub + i, a.rows - 1);
+    const bool past = rq_j >= iters;  // (uniform) nothing left: sixteen bytes that are there anyway, never used
+    // chunks 2g and 2g + 1 of the unit: both loads of a wavefront touch the same lines, the scales are one load
+    const int c0 = (wk * sh.upw + rq_u) * 8 + 2 * g;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int c = min(c0 + s, nchunks - 1);  // past the row: its last chunk again, against zeros
+      wt[p][s] = load_chunk<NT>(past ? (const uint4 *)g_gemv_zeros : qp + (int64_t)row * nchunks + c);
+    }
+    st[p] = *(past ? (const unsigned *)g_gemv_zeros : (const unsigned *)(a.d + (int64_t)row * nchunks + min(c0, nchunks - 2)));
+    if (++rq_u == sh.upw) rq_u = 0, rq_j++;
+  };
+#pragma unroll
+  for (int p = 0; p < PD; p++) request(p);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- digits ----
+  float s1 = 0.0f, mu = 0.0f, rstd = 1.0f;
+  if (tid < 64) ((unsigned *)smem)[tid] = 0u;
+  auto put = [&](int k, const unsigned *w, float down) __attribute__((always_inline)) {  // digits of k = 4 k .. + 3: [16 k][digit][16 bytes]
+    unsigned *o = (unsigned *)(dig + (size_t)(k >> 2) * 64) + (k & 3);
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[4 * r] = w[r];
+    if (k % 8 == 0) sx[k >> 3] = down;
+  };
+  for (int k = n4 + tid; k < cpad * 8; k += nthr) {  // past the row
+    const unsigned z[4] = {0u, 0u, 0u, 0u};
+    put(k, z, 0.0f);
+  }
+  for (int i0 = tid; i0 < n4; i0 += nthr * SB) {  // (a chunk's lanes stay together: n4 is a multiple of eight)
+    if (i0 != tid) ask(i0);
+#pragma unroll
+    for (int b = 0; b < SB; b++) {
+      const int k = i0 + nthr * b;
+      if (k >= n4) break;
+      float v[4] = {xv[b].x, xv[b].y, xv[b].z, xv[b].w};
+      const float u[4] = {uv[b].x, uv[b].y, uv[b].z, uv[b].w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        if (LAYERNORM) s1 += v[e];
+        if (RMS) s1 = fmaf(v[e], v[e], s1);
+        if ((RMS || LAYERNORM) && a.norm_g) v[e] *= u[e];
+      }
+      unsigned w[4];
+      const float down = int_digits(v, w);
+      put(k, w, down * 0.0625f);  // (nibbles are multiplied as 16 (n - 8))
+    }
+  }
+  if (RMS || LAYERNORM) {
+    s1 = wave_sum(s1);
+    if (lane == 0) red[wv] = s1;
+  }
+  __syncthreads();
+  auto of_all = [&](const float *p, int stride, int n) __attribute__((always_inline)) {  // p[0] + p[stride] + ..., n <= 16, all asked for together
+    float t[16], v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; w++) t[w] = p[min(w, n - 1) * stride];
+#pragma unroll
+    for (int w = 0; w < 16; w++) v += w < n ? t[w] : 0.0f;
+    return v;
+  };
+  if (LAYERNORM) {  // the deviations from the mean: the vector once more (it is in the caches; the weights are on their way)
+    mu = of_all(red, 1, nw) / (float)a.cols;
+    float q = 0.0f;
+    for (int k = tid; k < n4; k += nthr) {
+      const float4 t = x4[k];
+      const float d0 = t.x - mu, d1 = t.y - mu, d2 = t.z - mu, d3 = t.w - mu;
+      q = fmaf(d0, d0, fmaf(d1, d1, fmaf(d2, d2, fmaf(d3, d3, q))));
+    }
+    q = wave_sum(q);
+    if (lane == 0) red[16 + wv] = q;  // (read behind the barrier after the stream)
+  }
+
+  // ---- stream ----
+  const bool act = (i >> 2) == g;  // this lane's row of the first operand belongs to its own chunk of k
+  const unsigned char *dl = act ? dig + g * (2 * CB) + (i & 3) * 16 : smem + (lane < 32 ? 192 : 64);
+  const int dunit = act ? 8 * CB : 0, dchunk = act ? CB : 0, dhalf = act ? 64 : 0;
+  float acc = 0.0f;
+  auto consume = [&](int p, int unit) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const uint4 q = wt[p][s];
+      const unsigned char *da = dl + unit * dunit + s * dchunk;
+      v4i r = {0, 0, 0, 0};
+      const v4i a0 = *(const v4i *)da, a1 = *(const v4i *)(da + dhalf);
+      const unsigned dw[4] = {q.x, q.y, q.z, q.w};
+      v4i lo, hi;
+#pragma unroll
+      for (int t = 0; t < 4; t++) {  // 16 (n - 8): the nibble in the byte's upper half, its top bit turned
+        lo[t] = (int)(((dw[t] << 4) & 0xf0f0f0f0u) ^ 0x80808080u);
+        hi[t] = (int)((dw[t] & 0xf0f0f0f0u) ^ 0x80808080u);
+      }
+      r = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, lo, r, 0, 0, 0);
+      r = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, hi, r, 0, 0, 0);
+      const float f = fmaf((float)(r[0] * 256 + r[1]), 65536.0f, (float)(r[2] * 256 + r[3]));
+      const float d = half_bits_to_float((unsigned short)(s ? st[p] >> 16 : st[p])) * sx[unit * 8 + 2 * g + s];
+      acc = fmaf(d, f, acc);
+    }
+  };
+  int j = 0, u = 0;
+  auto step = [&](int p) __attribute__((always_inline)) {
+    consume(p, wk * sh.upw + u);
+    if (++u == sh.upw) {  // (uniform) the group's share is complete
+      u = 0;
+      acc += __shfl_xor(acc, 16, 64);
+      acc += __shfl_xor(acc, 32, 64);
+      if (lane < 16) ps[(j * nw + wv) * 16 + lane] = acc;
+      acc = 0.0f;
+      j++;
+    }
+  };
+  int t = 0;
+  for (; t + PD <= nu; t += PD) {
+#pragma unroll
+    for (int p = 0; p < PD; p++) {
+      step(p);
+      request(p);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < PD; p++)
+    if (t + p < nu) step(p);  // (uniform)
+  __syncthreads();
+
+  // ---- the sums of the wavefronts, in their order, and the epilogue ----
+  if (RMS || LAYERNORM) rstd = 1.0f / sqrtf(of_all(LAYERNORM ? red + 16 : red, 1, nw) / (float)a.cols + a.eps);
+  float best = -INFINITY;
+  int besti = 0x7fffffff;
+  if (oj < iters && orow < a.rows) {
+    const float *p = ps + ((size_t)oj * nw + (oi >> 4) * sh.ks) * 16 + (oi & 15);
+    float v = of_all(p, 16, sh.ks);
+    if (LAYERNORM) v -= mu * of;
+    if (RMS || LAYERNORM) v *= rstd;
+    if (a.pair_swiglu) {  // rows 2r, 2r + 1 are a (gate, up) pair, in neighbouring threads (rows are even)
+      const float full = v + ob, up = __shfl_xor(full, 1, 64);
+      if (!(oi & 1)) a.y[(int64_t)m * a.y_stride + (orow >> 1)] = ct_silu(full) * up;
+    } else {
+      best = gemv_store(a, m, orow, v, posv, ob, orr);
+      besti = orow;
+    }
+  }
+  if (a.am_val) {
+    __syncthreads();
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) argmax_merge(best, besti, __shfl_xor(best, o, 64), __shfl_xor(besti, o, 64));
+    if (lane == 0) red[wv] = best, ((int *)red)[16 + wv] = besti;
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < nw; w++) argmax_merge(best, besti, red[w], ((int *)red)[16 + w]);
+      a.am_val[blockIdx.x] = best;
+      a.am_idx[blockIdx.x] = besti;
+    }
+  }
+}
+
+bool gemv_int_supported(const WMat *w, const GemvArgs &a) {
+  if (a.norm_out || a.pro == CTHIP_PRO_SWIGLU || (a.pro == CTHIP_PRO_LAYERNORM && !a.fold_s) || (a.pro == CTHIP_PRO_RMSNORM && a.norm_b)) return false;
+  if (a.pair_swiglu && ((w->rows & 1) || a.am_val || a.residual || a.act != CTHIP_ACT_NONE || (a.split1 > 0 && a.split1 != (int)w->rows))) return false;
+  return gemv_int_plan(w->type, w->rows, w->cols, state().compute_units).ok;
+}
+
+int launch_gemv_int(const WMat *w, GemvArgs a, int m, int *am_parts) {
+  State &s = state();
+  const GemvIntPlan p = gemv_int_plan(w->type, w->rows, w->cols, s.compute_units);
+  if (!p.ok) return fail(CTHIP_E_UNSUPPORTED, "gemv: no integer launch for a (%lld, %lld) matrix of type %d", (long long)w->rows, (long long)w->cols, w->type);
+  a.q = w->q;
+  a.d = (const unsigned short *)w->d;
+  a.rows = (int)w->rows;
+  a.cols = (int)w->cols;
+  if (a.split1 <= 0) a.split1 = a.split2 = a.rows;
+  // A line asked for with the hint is fetched a second time for its second chunk, which costs 4 - 7 % of a stream; keeping the weights from
+  // pushing each other out of the cache is worth more until they are many times its size (us per step, with the hint / without: 36 layers of 1280, 0.46 GB 1040 / 1100;
+  // 48 of 1600, 0.87 GB 1560 / 1560; 32 of 4096, 3.7 GB 1617 / 1549).
+  const bool nt = s.gemv_stream < 0 ? w->stream && !w->stream_far : s.gemv_stream != 0;
+  typedef void (*int_fn)(GemvArgs, GemvIntShape);
+#define PICK(PRO) (nt ? k_gemv_int<PRO, true> : k_gemv_int<PRO, false>)
+  int_fn fn = a.pro == CTHIP_PRO_RMSNORM ? PICK(CTHIP_PRO_RMSNORM) : a.pro == CTHIP_PRO_LAYERNORM ? PICK(CTHIP_PRO_LAYERNORM) : PICK(CTHIP_PRO_NONE);
+#undef PICK
+  if (p.lds > 64 * 1024) {
+    CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvIntMaxLdsBytes));
+  }
+  hipLaunchKernelGGL(fn, dim3(p.grid, (unsigned)m), dim3(64 * p.ks * p.rgp), p.lds, s.stream, a, GemvIntShape{p.upw, p.ks, p.rgp, (65536 + p.ks - 1) / p.ks, (65536 + 16 * p.rgp - 1) / (16 * p.rgp)});
+  CTHIP_LAUNCH_CHECK();
+  *am_parts = (int)p.grid;
+  return 0;
+}
+
+}  // namespace cthip

@@ -223,6 +223,40 @@ inline GemvWidePlan gemv_wide_plan(int type, long long rows, long long cols, int
   return p;
 }
 
+// The integer kernel (gemv_int.hip): ks wavefronts share a group of 16 rows, each takes upw units (128 bytes) of every row; a
+// workgroup has rgp such sets and goes over its groups of 16 rgp rows grid apart.  lds: bytes (256 of zeros, digits and scales of the vector,
+// 32 words of reductions, the partial sums of every wavefront and group).
+// Eight wavefronts and two workgroups to a compute unit where there are groups enough for that and a row is not too long for them, else
+// sixteen (us, 16 / 8: 12288 x 4096 9.9 / 8.6, 22016 x 4096 14.6 / 13.3, 4096 x 4096 6.1 / 6.2, 4096 x 11008 10.0 / 10.9).
+struct GemvIntPlan {
+  bool ok = false;
+  int upw = 0, ks = 0, rgp = 0, iters = 0;
+  unsigned grid = 0;
+  size_t lds = 0;
+};
+constexpr size_t kGemvIntMaxLdsBytes = 156 * 1024;
+inline GemvIntPlan gemv_int_plan(int type, long long rows, long long cols, int compute_units) {
+  GemvIntPlan p;
+  // (pairs of scales are fetched as one dword)
+  if (type != CTHIP_Q4_0 || rows <= 0 || rows > 0x7fffffff - 1024 || cols < 64 || cols % 64 || cols > (1 << 20)) return p;
+  const long long groups = (rows + 15) / 16;
+  const int units = (int)((cols / 2 + 127) / 128), cap = units <= 16 && groups >= 2ll * compute_units ? 8 : 16;
+  p.upw = (units + cap - 1) / cap;
+  p.ks = (units + p.upw - 1) / p.upw;
+  if (p.ks < 4) return p;  // rows of less than 512 bytes
+  p.rgp = cap / p.ks;
+  while (p.rgp > 1 && groups / p.rgp < compute_units) p.rgp--;
+  const long long nsg = (groups + p.rgp - 1) / p.rgp, slots = (long long)compute_units * (16 / (p.ks * p.rgp));
+  p.grid = (unsigned)(nsg < slots ? nsg : slots);
+  const long long iters = (nsg + p.grid - 1) / p.grid;
+  if (iters * 16 > 64 * p.ks) return p;  // a thread per row of a workgroup
+  p.iters = (int)iters;
+  const size_t cpad = (size_t)p.ks * p.upw * 8;
+  p.lds = 256 + cpad * 132 + 32 * 4 + (size_t)iters * p.ks * p.rgp * 64;
+  p.ok = p.lds <= kGemvIntMaxLdsBytes;
+  return p;
+}
+
 // How the split-K reduction + norm pass (rowops.hip) lays a row out: `wide` = four wavefronts per row instead of
 // one; `vpl` = the float4-per-lane count of the kernel instantiation chosen (one of 1,2,3,4,6,8 narrow / 1,2,4,8
 // wide); `nz` = the share bucket.  ok is false when no instantiation covers the row.

@@ -381,12 +381,19 @@ static bool gemv_prefers_wide(const GemvVariant *v, int type, int64_t rows) {
   const int opt = state().gemv_wide;
   return opt && (!v || heavy || opt >= 2);
 }
+// The integer kernel (gemv_int.hip), us against what was there: 12288 x 4096 10.2 -> 8.6, 22016 x 4096 14.4 -> 13.2, 4096 x 4096 6.3 -> 6.1, 4096 x 11008 12.6 -> 10.1,
+// 32000 x 4096 18.4 -> 16.6, 50257 x 1280 14.4 -> 9.6, 5120 x 1280 5.5 -> 4.7, 2560 x 2048 5.2 -> 4.4.  With fewer rows its groups of 16 leave compute
+// units idle (2048 x 5632 6.5 -> 6.7, 1280 x 1280 3.7 -> 3.9), as between one and two rounds of long rows (5120 x 5120 8.4 -> 8.7).
+static bool gemv_prefers_int(int type, int64_t rows, int64_t cols) {
+  if (state().gemv_wide != 1 || !gemv_int_plan(type, rows, cols, state().compute_units).ok) return false;
+  const int64_t round = 16ll * state().compute_units;  // rows
+  return rows >= 2560 && cols <= 16384 && !(cols > 4096 && cols <= 6144 && rows > round && rows < 2 * round);
+}
 bool gemv_norm_out_ok(const WMat *w) {
   const GemvVariant *v = pick_variant(w->type, (int)w->cols);
   return v && !gemv_prefers_wide(v, w->type, w->rows);
 }
-bool gemv_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
-  if (rows <= 0 || (rows & 1) || cols <= 0 || cols > 0x7fffffff) return false;
+static bool vector_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
   const GemvVariant *v = pick_variant(type, (int)cols);
   const State &s = state();
   if (gemv_prefers_wide(v, type, rows)) {
@@ -398,6 +405,10 @@ bool gemv_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
   // one row per wavefront: the pair sits in neighbouring slots of the ring, which a looping launch with an even ring
   // has (enough rows for every wavefront to loop at any occupancy)
   return (gemv_ring_depth(type, v->KC) & 1) == 0 && rows >= 32ll * s.compute_units;
+}
+bool gemv_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
+  if (rows <= 0 || (rows & 1) || cols <= 0 || cols > 0x7fffffff) return false;
+  return gemv_prefers_int(type, rows, cols) || vector_pair_swiglu_ok(type, rows, cols);
 }
 int gemv_rows_per_wave(int type, int64_t cols) {
   const GemvVariant *v = cols <= 0x7fffffff ? pick_variant(type, (int)cols) : nullptr;
@@ -494,6 +505,15 @@ int launch_gemv(const WMat *w, GemvArgs a, int m) {
   a.ld_chunks = a.ld_scales = a.up_off = 0;
   if (a.split1 <= 0) a.split1 = a.split2 = a.rows;
   if (a.am_val && m != 1) return fail(CTHIP_E_BAD_ARG, "gemv: the fused argmax needs m == 1");
+  // (rows laid out in pairs for a launch that only the integer kernel is: it stays with it whatever the options say now)
+  if ((gemv_prefers_int(w->type, w->rows, w->cols) || (a.pair_swiglu && !vector_pair_swiglu_ok(w->type, w->rows, w->cols))) && gemv_int_supported(w, a)) {
+    int parts = 0;
+    const int rc = launch_gemv_int(w, a, m, &parts);
+    if (rc || !a.am_val) return rc;
+    hipLaunchKernelGGL(k_argmax_finish, dim3(1), dim3(256), 0, s.stream, a, parts);
+    CTHIP_LAUNCH_CHECK();
+    return 0;
+  }
   const GemvVariant *v = pick_variant(w->type, a.cols);
   if (gemv_prefers_wide(v, w->type, a.rows) && gemv_wide_supported(w, a)) return launch_gemv_wide(w, a, m);
   if (a.pair_swiglu && (!v || (a.rows & 1) || a.am_val || a.residual || a.split1 != a.rows))

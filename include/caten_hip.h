@@ -257,8 +257,9 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  *   held in registers; rows of up to 36 000 columns in any weight format, no LayerNorm prologue, no fused argmax): 0 = none
  *   (rows wider than the register-resident kernels cover go as column slices, one launch each), 1 (default) = the
  *   rows no register-resident kernel covers and those whose register-resident kernel runs one wavefront per SIMD
- *   (4-bit rows past 6144 columns, 8-bit rows past 4096), 2 = every launch it supports.  Results differ between the two kernel
- *   families only in summation order.
+ *   (4-bit rows past 6144 columns, 8-bit rows past 4096) but for 4-bit matrices of 2560 rows and more, which go
+ *   through integer matrix instructions (0 and 2 keep them out), 2 = every launch it supports.  Results differ between the kernel
+ *   families only in summation order and rounding.
  * "attn_split": 1 (default) = decoder sessions created afterwards that run one launch per Linear and have
  *   max_seq >= 512 share the keys of a head among (compute units / heads) workgroups, at most 16, in their decode
  *   attention (long contexts); 2 .. 16 = that many workgroups per head; 0 = one workgroup per head.  Same tokens;

@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <string>
+#include <vector>
 
 #include "../../caten_amd/csrc/gemv_plan.h"
 
@@ -291,6 +292,71 @@ static void walk_wide(int type, int rows, int cols, int m_rows, int pro, bool bi
       }
 }
 
+// the integer kernel (gemv_int.hip): the same walk over its plan
+static void walk_int(int type, int rows, int cols, int m_rows, int pro, bool bias, bool residual, bool fold, int cus) {
+  const GemvIntPlan p = gemv_int_plan(type, rows, cols, cus);
+  if (!p.ok) return;
+  char buf[256];
+  snprintf(buf, sizeof(buf), "int type %d (%d,%d) m %d pro %d bias %d resid %d fold %d", type, rows, cols, m_rows, pro, bias, residual, fold);
+  g_case = buf;
+  g_launches++;
+  const int nchunks = cols / 32, n4 = cols / 4, CB = 128, LC = 8;
+  const int cpad = p.ks * p.upw * 8, nw = p.ks * p.rgp, nthr = 64 * nw, rows_sg = 16 * p.rgp, nsg = (rows + rows_sg - 1) / rows_sg;
+  const int inv_ks = (65536 + p.ks - 1) / p.ks, inv_rows = (65536 + rows_sg - 1) / rows_sg;
+  const long long dig = 256, sx = dig + (long long)cpad * CB, red = sx + 4ll * cpad, ps = red + 128;
+  Region Q = {"quants", true, (long long)rows * nchunks * 16}, D = {"scales", true, (long long)rows * nchunks * 2}, X = {"x", true, 4ll * cols * m_rows},
+         NG = {"gamma", true, 4ll * cols}, B = {"bias", bias, 4ll * rows}, F = {"fold", fold, 4ll * rows}, R = {"residual", residual, 4ll * rows * m_rows},
+         Y = {"y", true, 4ll * rows * m_rows}, L = {"LDS", true, (long long)p.lds};
+  auto bad = [&](const char *what) { if (g_violations++ < 40) printf("VIOLATION %s: %s\n", g_case.c_str(), what); };
+  if (nthr > 1024 || nw > 16 || p.ks * p.upw * 128 < cols / 2 || p.lds > kGemvIntMaxLdsBytes || p.grid > (unsigned)nsg) bad("plan");
+  std::vector<char> done((size_t)rows * m_rows, 0);
+  for (int m = 0; m < m_rows; m++)
+    for (int bx = 0; bx < (int)p.grid; bx++) {
+      const int iters = (nsg - bx + (int)p.grid - 1) / (int)p.grid;
+      if (iters < 1 || iters > p.iters || iters * rows_sg > nthr) bad("iterations");
+      for (int tid = 0; tid < nthr; tid++) {
+        const int lane = tid & 63, wv = tid >> 6, g = lane >> 4, i = lane & 15, sub = (wv * inv_ks) >> 16, wk = wv - sub * p.ks;
+        if (sub != wv / p.ks || sub >= p.rgp) bad("wavefront's set");
+        const int oj = (tid * inv_rows) >> 16, oi = tid - oj * rows_sg, orow = (bx + oj * (int)p.grid) * rows_sg + oi, orc = orow < rows ? orow : rows - 1;
+        if (oj != tid / rows_sg) bad("finished row");
+        if (bias) touch(B, 4ll * orc, 4, "int bias");
+        if (residual) touch(R, 4 * ((long long)rows * m + orc), 4, "int residual");
+        if (fold) touch(F, 4ll * orc, 4, "int fold");
+        for (int k = tid; k < n4 + nthr * 3; k += nthr) {
+          const int kk = k < n4 ? k : n4 - 1;
+          touch(X, 4ll * cols * m + 16ll * kk, 16, "int input");
+          if (pro == CTHIP_PRO_RMSNORM || pro == CTHIP_PRO_LAYERNORM) touch(NG, 16ll * kk, 16, "int gamma");
+        }
+        for (int k = tid; k < cpad * LC; k += nthr) {  // digits of the row, and zeros past it
+          for (int r = 0; r < 4; r++) touch(L, dig + (long long)(k >> 2) * 64 + 4 * (k & 3) + 16 * r, 4, "int digits");
+          if (k % LC == 0) touch(L, sx + 4ll * (k / LC), 4, "int scale of a chunk");
+        }
+        touch(L, red + 4 * (16 + wv), 4, "int reductions");
+        for (int j = 0; j < iters; j++) {
+          const int row0 = (bx + j * (int)p.grid) * rows_sg + 16 * sub + i, row = row0 < rows ? row0 : rows - 1;
+          for (int u = 0; u < p.upw; u++) {
+            const int unit = wk * p.upw + u, c0 = unit * 8 + 2 * g;
+            for (int s = 0; s < 2; s++) {
+              touch(Q, ((long long)row * nchunks + (c0 + s < nchunks ? c0 + s : nchunks - 1)) * 16, 16, "int weights");
+              touch(L, sx + 4ll * (unit * 8 + 2 * g + s), 4, "int scale read");
+              if ((i >> 2) == g)
+                for (int h = 0; h < 2; h++) touch(L, dig + g * 2 * CB + (i & 3) * 16 + (long long)unit * 8 * CB + s * CB + h * 64, 16, "int digits read");
+            }
+            touch(D, 2 * ((long long)row * nchunks + (c0 < nchunks - 2 ? c0 : nchunks - 2)), 4, "int scale pair");
+          }
+          if (lane < 16) touch(L, ps + 4ll * ((j * nw + wv) * 16 + lane), 4, "int partial sums");
+        }
+        if (oj < iters && orow < rows) {
+          for (int w = 0; w < p.ks; w++) touch(L, ps + 4ll * ((oj * nw + (oi >> 4) * p.ks) * 16 + (oi & 15) + 16 * w), 4, "int sums read");
+          touch(Y, 4 * ((long long)rows * m + orow), 4, "int store");
+          if (done[(size_t)m * rows + orow]++) bad("a row is finished twice");
+        }
+      }
+    }
+  for (char d : done)
+    if (!d) { bad("a row is not finished"); break; }
+}
+
 // the split-K reduction + norm pass: whatever (row length, shares, rows) the launcher accepts, the instantiation it
 // picks covers the whole row (lanes x float4 per lane x 4 floats) and keeps its shares within the register budget
 static void check_reduce_norm_plans() {
@@ -419,6 +485,16 @@ int main(int argc, char **argv) {
       }
     }
   }
+  for (int type : {CTHIP_Q4_0})
+    for (int cols : {1024, 1088, 1280, 1600, 2048, 2112, 4096, 4160, 5632, 11008})
+      for (int rows : {1, 15, 16, 17, 515, 1280, 2563, 4100, 4112, 8194, 11264, 50257}) {
+        if ((long long)rows * cols > 3000000 && !(cols == 1024 && rows == 50257)) continue;
+        for (int pro : {(int)CTHIP_PRO_NONE, (int)CTHIP_PRO_LAYERNORM, (int)CTHIP_PRO_RMSNORM}) {
+          if (pro == CTHIP_PRO_RMSNORM && rows > 3000) continue;
+          walk_int(type, rows, cols, rows < 100 ? 3 : 1, pro, rows & 1, cols & 64, pro == CTHIP_PRO_LAYERNORM, 256);
+          if (rows < 1300) walk_int(type, rows, cols, 1, pro, true, true, false, 64);
+        }
+      }
   // the wide-row kernel on widths around its tile sizes, and rows fewer / more than wavefronts
   for (int type : {CTHIP_Q8_0, CTHIP_Q4_0, CTHIP_F16, CTHIP_F32})
     for (int cols : {64, 96, 2048, 2080, 4096, 5504, 6144, 8192, 8224, 11008})

@@ -1,0 +1,102 @@
+"""The single-row Linear by integer matrix instructions (csrc/gemv_int.hip): rows that are no multiple of 16, units of 128 bytes that
+end inside a row, one wavefront's share of several units, one to many groups a workgroup; every prologue and epilogue it
+carries; inputs of any magnitude; (gate, up) row pairs and the fused argmax through sessions."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from caten_amd import _lib, ops as o
+    _lib.init(0)
+    return o
+
+
+def matrix(ops, kind, rows, cols, seed):
+    from caten_amd.llm import Tensor
+    rng = np.random.default_rng(seed)
+    w = ops.WeightMatrix(kind, Tensor.from_f32(rng.normal(0, 0.05, (rows, cols)).astype(np.float32), kind).raw, rows, cols)
+    return w, w.dequantize().astype(np.float64), rng
+
+
+# Error of a sum of n products against 64 bits: the inputs' digits keep 2^-30 of their chunk's largest value, the scales and sums round in
+# fp32, 2^-24 a step over at most 16 wavefronts x 6 units x 2 chunks of a lane: bounded by 2^-17 of the sum of magnitudes, seen at 1e-7 of the result.
+def close(got, want, scale):
+    assert np.all(np.isfinite(got)) and np.all(np.abs(got - want) <= 2.0 ** -17 * scale + 1e-30)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("kind,rows,cols", [("q4_0", 2563, 1024), ("q4_0", 2575, 1088), ("q4_0", 4096, 4096), ("q4_0", 2560, 11008), ("q4_0", 8207, 4160), ("q4_0", 20011, 1600),
+                                            ("q4_0", 50257, 1280), ("q4_0", 2561, 1216), ("q4_0", 12288, 2048)])
+def test_linear(ops, kind, rows, cols):
+    w, wd, rng = matrix(ops, kind, rows, cols, rows + cols)
+    x = rng.normal(0.1, 1, cols).astype(np.float32)
+    x[5], x[64:96] = 60.0, 0.0  # a large input among small ones, a chunk of zeros
+    x[cols - 1] = 7.0           # next to the padding
+    b, r, g = rng.normal(0, 1, rows).astype(np.float32), rng.normal(0, 1, rows).astype(np.float32), rng.normal(1, 0.1, cols).astype(np.float32)
+    beta = rng.normal(0, 0.1, cols).astype(np.float32)
+    x64 = x.astype(np.float64)
+    aw = np.abs(wd)
+    close(ops.linear(x, w), wd @ x64, aw @ np.abs(x64))
+    close(ops.linear(x, w, b, r, act="relu"), np.maximum(wd @ x64 + b, 0) + r, aw @ np.abs(x64) + np.abs(b) + np.abs(r))
+    n = x64 / np.sqrt((x64 * x64).mean() + 1e-5) * g
+    close(ops.linear(x, w, None, r, prologue="rmsnorm", norm_g=g), wd @ n + r, aw @ np.abs(n) + np.abs(r))
+    if cols <= 4096:
+        w.fold_layernorm(g, beta, b)
+        n = (x64 - x64.mean()) / np.sqrt(x64.var() + 1e-5) * g
+        got = w.linear_folded(x)
+        want = wd @ (n + beta) + b
+        assert np.linalg.norm(got - want) <= 3e-6 * np.linalg.norm(want)  # (the mean's part is taken off behind the product)
+    w.free()
+
+
+@pytest.mark.parametrize("kind,rows,cols", [("q4_0", 2600, 1024)])
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
+def test_inputs_of_any_magnitude(ops, kind, rows, cols, scale):
+    w, wd, rng = matrix(ops, kind, rows, cols, 3)
+    x = (rng.normal(0, 1, cols) * scale).astype(np.float32)
+    x[:32] *= np.float32(1e-6)  # a chunk of its own magnitude
+    close(ops.linear(x, w), wd @ x.astype(np.float64), np.abs(wd) @ np.abs(x.astype(np.float64)))
+    w.free()
+
+
+@pytest.mark.parametrize("kind,rows,cols", [("q4_0", 2600, 1024)])
+def test_inputs_that_are_not_finite(ops, kind, rows, cols):
+    w, wd, rng = matrix(ops, kind, rows, cols, 4)
+    x = rng.normal(0, 1, cols).astype(np.float32)
+    x[40] = np.inf
+    got, with_weight = ops.linear(x, w), wd[:, 40] != 0
+    assert np.array_equal(got[with_weight], np.sign(wd[with_weight, 40]) * np.inf) and np.all(np.isnan(got[~with_weight]))
+    x[40] = np.nan
+    assert np.all(np.isnan(ops.linear(x, w)))
+    w.free()
+
+
+@pytest.mark.parametrize("arch,kind", [("llama", "q4_0"), ("gpt2", "q4_0")])
+def test_sessions_match_the_vector_kernels(ops, arch, kind):
+    from caten_amd import _lib, llm, synth
+    lib = _lib.load()
+    if arch == "llama":  # (dim 1024: no three-launch layer, 8192 gate|up rows in pairs)
+        cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=1024, n_heads=8, n_kv_heads=8, ffn=4096, n_layers=2, vocab=4099, max_seq=128)
+        sd = llm.llama_state_dict(synth.llama_weights(cfg, seed=5), kind)
+    else:                # (dim 1280: a launch per Linear, LayerNorm folded)
+        cfg = dict(synth.GPT2_CONFIGS["gpt2"], dim=1280, n_heads=20, n_layers=2, vocab=6500, max_seq=128)
+        sd = llm.gpt2_state_dict(synth.gpt2_weights(cfg, seed=5), kind)
+    prompt, runs = synth.prompt(cfg["vocab"], 9, seed=5), []
+    try:
+        for wide in (1, 0):
+            _lib.check(lib.cthip_set_option(b"gemv_wide", wide))
+            model = (llm.make_llama if arch == "llama" else llm.make_gpt2)(cfg, sd)
+            tokens, logits = llm.gpt2_generate(model, prompt, 10, on_device=False, keep_logits=True)
+            model.close()
+            model = (llm.make_llama if arch == "llama" else llm.make_gpt2)(cfg, sd)
+            assert llm.gpt2_generate(model, prompt, 10, on_device=True) == tokens
+            model.close()
+            runs.append((tokens, logits))
+    finally:
+        _lib.check(lib.cthip_set_option(b"gemv_wide", 1))
+    assert runs[0][0] == runs[1][0]
+    for a, b in zip(runs[0][1], runs[1][1]):
+        assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
