@@ -1140,133 +1140,7 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
   }
 }
 
-// sum over aligned groups of LPK lanes (8, 16 or 32), every lane gets the sum
-template <int LPK>
-__device__ __forceinline__ float lpk_sum(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror: 8 lanes
-  if (LPK >= 16) v += dpp_f<0x140>(v);  // row_mirror: 16 lanes
-  if (LPK >= 32) v += __shfl_xor(v, 16, 64);
-  return v;
-}
-
-// Prompt rows (s > 1): one 256-thread block per (head, group of R consecutive query rows).  The group
-// shares every K / V tile it loads, so the cache is read once per R rows instead of once per row; the
-// causal mask (layers.lisp:83) is applied per row.  Same lane layout and per-wavefront online softmax
-// as k_attn_cached, with R running (max, sum, output) triples.
-template <int DH, int R>
-__global__ __launch_bounds__(256) void k_attn_rows(float *__restrict__ out, const float *__restrict__ q,
-                                                   const float *__restrict__ kc, const float *__restrict__ vc, int S,
-                                                   int start_pos, const int *__restrict__ pos, int H, int Hkv) {
-  constexpr int LPK = DH / 4, KPW = 64 / LPK, KPT = 8, NW = 4, TILE = NW * KPW * KPT;
-  __shared__ float part[NW][R][DH];
-  __shared__ float pm[NW][R], pl[NW][R];
-  // the last groups see the most keys: they are dispatched first so the short ones fill the tail
-  const int h = blockIdx.x, i0 = (gridDim.y - 1 - blockIdx.y) * R;
-  const int base = start_pos + (pos ? pos[0] : 0);
-  const int nrows = min(R, S - i0);
-  const int Tmax = base + i0 + nrows;  // keys the last row of the group sees
-  const int hk = h / (H / Hkv);
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int g = lane / LPK, c = lane % LPK;
-  const unsigned kvs4 = (unsigned)(Hkv * DH / 4);
-  const float4 *__restrict__ kp = (const float4 *)(kc + (int64_t)hk * DH) + c;
-  const float4 *__restrict__ vp = (const float4 *)(vc + (int64_t)hk * DH) + c;
-  const float scale = 1.0f / sqrtf((float)DH);
-  float4 q4[R];
-  float m[R], l[R], acc[R][4];
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    const int row = min(i0 + r, S - 1);  // rows past the end repeat the last one and are not stored
-    q4[r] = *(const float4 *)(q + ((int64_t)row * H + h) * DH + 4 * c);
-    m[r] = -INFINITY;
-    l[r] = 0.0f;
-    acc[r][0] = acc[r][1] = acc[r][2] = acc[r][3] = 0.0f;
-  }
-  for (int t0 = 0; t0 < Tmax; t0 += TILE) {
-    if (t0 + wv * KPT * KPW >= Tmax) break;  // nothing left for this wavefront (uniform)
-    float4 kr[KPT], vr[KPT];
-#pragma unroll
-    for (int u = 0; u < KPT; u++) {
-      const int j = t0 + (wv * KPT + u) * KPW + g;
-      const unsigned jj = (unsigned)min(j, Tmax - 1);
-      kr[u] = kp[jj * kvs4];
-      vr[u] = vp[jj * kvs4];
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int Tr = base + min(i0 + r, S - 1) + 1;  // keys row r sees
-      float sc[KPT];
-      float tmax = -INFINITY;
-#pragma unroll
-      for (int u = 0; u < KPT; u++) {
-        float d = q4[r].x * kr[u].x;
-        d = fmaf(q4[r].y, kr[u].y, d);
-        d = fmaf(q4[r].z, kr[u].z, d);
-        d = fmaf(q4[r].w, kr[u].w, d);
-        d = lpk_sum<LPK>(d);
-        const bool ok = (t0 + (wv * KPT + u) * KPW + g) < Tr;
-        sc[u] = ok ? d * scale : -INFINITY;
-        tmax = fmaxf(tmax, sc[u]);
-      }
-#pragma unroll
-      for (int o = LPK; o < 64; o <<= 1) tmax = fmaxf(tmax, __shfl_xor(tmax, o, 64));
-      const float m_new = fmaxf(m[r], tmax);
-      const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;  // every key of this tile masked for row r so far
-      const float corr = ct_exp(m[r] - m_use);
-      float ps = 0.0f;
-#pragma unroll
-      for (int k2 = 0; k2 < 4; k2++) acc[r][k2] *= corr;
-#pragma unroll
-      for (int u = 0; u < KPT; u++) {
-        const float p = ct_exp(sc[u] - m_use);
-        ps += p;
-        acc[r][0] = fmaf(p, vr[u].x, acc[r][0]);
-        acc[r][1] = fmaf(p, vr[u].y, acc[r][1]);
-        acc[r][2] = fmaf(p, vr[u].z, acc[r][2]);
-        acc[r][3] = fmaf(p, vr[u].w, acc[r][3]);
-      }
-#pragma unroll
-      for (int o = LPK; o < 64; o <<= 1) ps += __shfl_xor(ps, o, 64);
-      l[r] = l[r] * corr + ps;
-      m[r] = m_new;
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-#pragma unroll
-    for (int o = LPK; o < 64; o <<= 1) {
-#pragma unroll
-      for (int k2 = 0; k2 < 4; k2++) acc[r][k2] += __shfl_xor(acc[r][k2], o, 64);
-    }
-    if (lane < LPK) {
-#pragma unroll
-      for (int k2 = 0; k2 < 4; k2++) part[wv][r][4 * lane + k2] = acc[r][k2];
-    }
-    if (lane == 0) {
-      pm[wv][r] = m[r];
-      pl[wv][r] = l[r];
-    }
-  }
-  __syncthreads();
-  for (int e = tid; e < nrows * DH; e += 256) {
-    const int r = e / DH, d = e % DH;
-    float M = pm[0][r];
-#pragma unroll
-    for (int w = 1; w < NW; w++) M = fmaxf(M, pm[w][r]);  // finite: key 0 is visible to every row
-    float o = 0.0f, L = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-      const float wgt = ct_exp(pm[w][r] - M);
-      o = fmaf(wgt, part[w][r][d], o);
-      L = fmaf(wgt, pl[w][r], L);
-    }
-    out[((int64_t)(i0 + r) * H + h) * DH + d] = o / L;
-  }
-}
-
-// Prompt rows on the matrix cores (s >= 32): one block per (head, 32 consecutive query rows); its
+// Prompt rows on the matrix cores (16 rows and more): one block per (head, 32 consecutive query rows); its
 // NW wavefronts take the 32-key tiles of the visible cache round-robin, each with its own online softmax
 // for all 32 rows, and meet once in LDS.  fp32 MFMA operands (v_mfma_f32_32x32x2_f32): the products are the
 // reference's fp32 products, only the summation order differs.
@@ -1357,12 +1231,22 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma(float *__restrict__ out, 
     }
     if (t + NW < ntiles) load_k(t + NW);
     __builtin_amdgcn_wave_barrier();
-    v16f_t sacc;
+    // Several chains of products: a single one over the head (and over the tiles, below) rounds at the size of its sum at every step.  Error against 64 bits,
+    // 17 rows, 700 keys of 64: 3.5e-7 -> 1.8e-7, what the kernel for fewer rows has.
+    constexpr int NC = DH >= 128 ? 8 : 4;
+    v16f_t sc[NC];
 #pragma unroll
-    for (int r = 0; r < 16; r++) sacc[r] = 0.0f;
+    for (int c = 0; c < NC; c++)
 #pragma unroll
-    for (int s = 0; s < NS; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(W[wv].Kt[half * NS + s][col], qreg[s], sacc, 0, 0, 0);
+      for (int r = 0; r < 16; r++) sc[c][r] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NS; s++) sc[s % NC] = __builtin_amdgcn_mfma_f32_32x32x2f32(W[wv].Kt[half * NS + s][col], qreg[s], sc[s % NC], 0, 0, 0);
     __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int w = NC / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int c = 0; c < w; c++) sc[c] += sc[c + w];
+    v16f_t sacc = sc[0];
     // sacc[r] = score of key kb + 8*(r/4) + 4*half + r%4 against query `col`
     float tmax = -INFINITY;
 #pragma unroll
@@ -1387,13 +1271,17 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma(float *__restrict__ out, 
     l = l * corr + ps;
     m = m_new;
 #pragma unroll
-    for (int b = 0; b < DB; b++)
+    for (int b = 0; b < DB; b++) {  // a tile's products by themselves
+      v16f_t p4[4];
 #pragma unroll
-      for (int r = 0; r < 16; r++) o[b][r] *= corr;
+      for (int c = 0; c < 4; c++)
 #pragma unroll
-    for (int s = 0; s < 16; s++)
+        for (int r = 0; r < 16; r++) p4[c][r] = 0.0f;
 #pragma unroll
-      for (int b = 0; b < DB; b++) o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vreg[b][s], sacc[s], o[b], 0, 0, 0);
+      for (int s = 0; s < 16; s++) p4[s & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vreg[b][s], sacc[s], p4[s & 3], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[b][r] = fmaf(o[b][r], corr, (p4[0][r] + p4[1][r]) + (p4[2][r] + p4[3][r]));
+    }
   }
   // o[b][r] = unnormalised output element d = 32b + 8*(r/4) + 4*half + r%4 of query `col`
   Cm[wv][lane] = m;
@@ -1428,7 +1316,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma(float *__restrict__ out, 
   }
 }
 
-// The same prompt attention with bf16 matrix instructions (v_mfma_f32_32x32x16_bf16, 16 times the rate of the
+// The same for 32 rows and more with bf16 matrix instructions (v_mfma_f32_32x32x16_bf16, 16 times the rate of the
 // fp32-operand one): every operand is written as hi + lo bf16 terms and each product as hi*hi + hi*lo + lo*hi, so
 // what is dropped is below 2^-16 of a product -- the "two terms" grade of the GEMMs (gemm_precision 2).  With
 // fp32 operands the matrix instructions alone are 4096 cycles of a 32-key tile; here they are 768 and the tile is
@@ -1641,10 +1529,13 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
   if (S == 0) return 0;
   (void)max_T;
   hipStream_t st = state().stream;
-  if (S >= 32 && pos == nullptr) {  // prompt rows on the matrix cores
+  // Prompt rows on the matrix cores.  16 .. 31 rows with fp32 operands, as the kernels for fewer have them: a key tile is 4096 cycles whatever the rows, so that
+  // half a block of them is the least that pays.  Whole prompts, us, against groups of eight rows that shared their key loads: 1280-wide Q8_0, 17 rows behind 689
+  // 3276 -> 2832, 20 rows alone 2239 -> 2185; 1.1B shape, 24 rows behind 1500 3084 -> 2509.  12 rows behind 689 would go 2426 -> 2672.
+  if (S >= 16 && pos == nullptr) {
     // eight wavefronts per block where their LDS tiles fit (head_dim <= 64), four otherwise
     dim3 grid(H, (S + 31) / 32);
-    if (state().gemm_precision == 0) {  // fp32 operands asked for: the products are fp32 products
+    if (state().gemm_precision == 0 || S < 32) {  // fp32 operands asked for: the products are fp32 products
       switch (Dh) {
         case 32: hipLaunchKernelGGL((k_attn_mfma<32, 8>), grid, dim3(512), 0, st, out, q, kc, vc, S, start_pos, H, Hkv); break;
         case 64: hipLaunchKernelGGL((k_attn_mfma<64, 8>), grid, dim3(512), 0, st, out, q, kc, vc, S, start_pos, H, Hkv); break;
@@ -1658,18 +1549,6 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
         case 128: hipLaunchKernelGGL((k_attn_mfma_bf<128, 4>), grid, dim3(256), 0, st, out, q, kc, vc, S, start_pos, H, Hkv); break;
         default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
       }
-    }
-    CTHIP_LAUNCH_CHECK();
-    return 0;
-  }
-  constexpr int R = 8;
-  if (S >= 2 * R) {  // short prompts: groups of R rows share their K / V loads
-    dim3 grid(H, (S + R - 1) / R), block(256);
-    switch (Dh) {
-      case 32: hipLaunchKernelGGL((k_attn_rows<32, R>), grid, block, 0, st, out, q, kc, vc, S, start_pos, pos, H, Hkv); break;
-      case 64: hipLaunchKernelGGL((k_attn_rows<64, R>), grid, block, 0, st, out, q, kc, vc, S, start_pos, pos, H, Hkv); break;
-      case 128: hipLaunchKernelGGL((k_attn_rows<128, R>), grid, block, 0, st, out, q, kc, vc, S, start_pos, pos, H, Hkv); break;
-      default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
     }
     CTHIP_LAUNCH_CHECK();
     return 0;
