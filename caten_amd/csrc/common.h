@@ -283,6 +283,9 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
 bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in);
 // x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
+// Linear over 8 .. 64 rows that lie as operands of two terms (linear_few.hip)
+bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: there is a pass over the rows in front of it anyway
+int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route);
 bool linear_planes_ready(const WMat *w, int m, int precision);
 void weight_planes_release(const WMat *w);
 // The terms of all matrices together are kept up to this many bytes.  They are given back where memory is short, by
@@ -292,7 +295,9 @@ bool weight_planes_drop();
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
                          int precision, const GemmRoute *route, unsigned char *planes_out, bool *done);
 bool rows_planes_supported(int K);
-int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps);
+// How a pass in front of a Linear writes its rows: fp32, as two bf16 terms a row (planes.h), as matrix operands of two terms (store_operands4)
+enum { kTermsNone = 0, kTermsPlanes = 1, kTermsOperands = 2 };
+int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps, int terms);
 void wmat_drop_planes(WMat *w);
 // matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays
 bool matmul_planes_pay(int M, int N, int K, int precision);
@@ -302,7 +307,7 @@ bool reduce_norm_supported(int n, int nparts);
 // C (m, n) = sum_z ws[z] + bias + residual for partial tiles handed over through GemmDeferred
 int launch_splitk_reduce(float *C, float *ws, int ksplit, int m, int n, const float *bias, const float *residual);
 int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, int64_t part_stride, const float *bias,
-                       const float *resid, const float *g, const float *b, float eps, int64_t rows, int n, bool rms, bool terms = false);
+                       const float *resid, const float *g, const float *b, float eps, int64_t rows, int n, bool rms, int terms = kTermsNone);
 // takes the device address of the static split-K scratch of cthip_matmul_noalloc (once per device, that device current)
 int matmul_scratch_init(int device);
 // gate|up rows (m, 2*cols) -> silu(gate)*up (m, cols), or a norm, as a launch of its own

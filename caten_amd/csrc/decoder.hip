@@ -935,7 +935,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     if ((rc = (e))) goto done; \
   } while (0)
   TRY(alloc((void **)&X, sizeof(float) * (size_t)s * D));
-  TRY(alloc((void **)&XN, sizeof(float) * (size_t)s * D));
+  TRY(alloc((void **)&XN, sizeof(float) * (size_t)((s + 15) / 16 * 16) * D));  // (whole blocks of 16 rows as matrix operands)
   TRY(alloc((void **)&QKV, sizeof(float) * (size_t)s * QW));
   TRY(alloc((void **)&Q, sizeof(float) * (size_t)s * D));
   TRY(alloc((void **)&ATT, sizeof(float) * (size_t)s * D));
@@ -978,18 +978,26 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       held.push_back(w);
       return true;
     };
+    // 8 .. 64 rows: the Linears behind a norm as one launch each, no partial tiles to add up (linear_few.hip); the norm writes their operands.
+    // (fewer and larger matrices keep the launch whose inputs have all 24 bits, linear_rows.hip)
+    auto few = [&](const WMat *w) {
+      return !(planes && std::find(held.begin(), held.end(), w) != held.end()) && rows_planes_supported(D) && w->cols == D && linear_few_pays(w, R, prec, true) &&
+             !linear_rows_pays(w, XN, D, R, prec, nullptr, nullptr);
+    };
+    auto in_terms = [&](const WMat *w) { return !w ? kTermsNone : in_planes(w) ? kTermsPlanes : few(w) ? kTermsOperands : kTermsNone; };
     auto no_planes = [&](const WMat *w) {
       held.erase(std::find(held.begin(), held.end(), w));
       weight_planes_release(w);
     };
     // y = norm(x), as terms where the Linear behind it takes them
-    auto norm = [&](float *y, const float *x, const float *g, const float *b, bool terms) {
-      if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps);
+    auto norm = [&](float *y, const float *x, const float *g, const float *b, int terms) {
+      if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps, terms);
       return gpt2 ? cthip_layernorm(y, x, g, b, c.eps, R, D) : cthip_rmsnorm(y, x, g, c.eps, R, D);
     };
     // y = W.in + ..., in and y as terms where in_terms / out_terms
-    auto linear = [&](float *y, const WMat *w, const float *in, bool in_terms, const float *bias, const float *residual, int act, const GemmRoute *route,
+    auto linear = [&](float *y, const WMat *w, const float *in, int in_terms, const float *bias, const float *residual, int act, const GemmRoute *route,
                       bool out_terms, GemmDeferred *defer = nullptr) {
+      if (in_terms == kTermsOperands) return launch_linear_few(y, w, in, R, bias, residual, act, route);
       if (in_terms || (planes && linear_planes_pays(w, R, prec, false))) {
         bool taken = false;
         const int r = launch_linear_planes(out_terms ? nullptr : y, w, in_terms ? nullptr : in, in_terms ? (const unsigned char *)in : nullptr, R, bias,
@@ -1001,7 +1009,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       return prompt_linear(y, w, in, R, bias, residual, act, prec, defer, route);
     };
     // Xr += W.in + bias, then XN = norm(Xr) with (g, b), as terms or not; g == nullptr: no norm follows (after the last layer)
-    auto linear_residual_norm = [&](const WMat *w, const float *in, bool in_terms, const float *bias, const float *g, const float *b, bool out_terms) {
+    auto linear_residual_norm = [&](const WMat *w, const float *in, int in_terms, const float *bias, const float *g, const float *b, int out_terms) {
       GemmDeferred df;
       const bool fuse = g != nullptr && reduce_norm_supported(D, 1);
       int r = linear(Xr, w, in, in_terms, bias, Xr, CTHIP_ACT_NONE, nullptr, false, fuse ? &df : nullptr);
@@ -1018,7 +1026,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       }
       return g ? norm(XN, Xr, g, b, out_terms) : 0;
     };
-    bool xt = in_planes(d->layers[0].attn);
+    int xt = in_terms(d->layers[0].attn);
     TRY(norm(XN, X, d->layers[0].ln1_g, d->layers[0].ln1_b, xt));
     for (int l = 0; l < c.n_layers; l++) {
       Layer &L = d->layers[l];
@@ -1061,7 +1069,8 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         if (att && !attended) att = false, no_planes(L.proj);
       }
       if (!attended) TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
-      const bool ft = in_planes(L.fc), gt = ft && (gpt2 || L.fc_pairs) && in_planes(L.fc2);
+      const int ft = in_terms(L.fc);
+      const bool gt = ft == kTermsPlanes && (gpt2 || L.fc_pairs) && in_planes(L.fc2);
       TRY(linear_residual_norm(L.proj, ATT, att, L.proj_b, L.ln2_g, L.ln2_b, ft));
       const float *hin = Hb;
       if (!gpt2 && L.fc_pairs && (2 * F) % 4 == 0) {  // SwiGLU in the epilogue of the gate|up launch
@@ -1075,7 +1084,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
           hin = G;
         }
       }
-      xt = !last && in_planes(d->layers[l + 1].attn);
+      xt = last ? kTermsNone : in_terms(d->layers[l + 1].attn);
       TRY(linear_residual_norm(L.fc2, hin, gt, L.fc2_b, last ? nullptr : d->layers[l + 1].ln1_g, last ? nullptr : d->layers[l + 1].ln1_b, xt));
     }
   }

@@ -749,6 +749,17 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
     const int rc = launch_linear_rows(y, w, x, x_stride, m, bias, residual, act, prologue, norm_g, norm_b, eps, state().gemm_precision, nullptr, &done);
     if (rc || done) return rc;
   }
+  if (prologue != CTHIP_PRO_SWIGLU && linear_few_pays(w, m, state().gemm_precision, prologue != CTHIP_PRO_NONE) && !stream_capturing() &&
+      !(((uintptr_t)x | (uintptr_t)y | (uintptr_t)bias | (uintptr_t)residual | (uintptr_t)norm_g | (uintptr_t)norm_b) & 15)) {
+    // the pass in front writes the (normalised) rows as matrix operands
+    void *operands = nullptr;
+    if (!alloc_scratch(&operands, sizeof(float) * (size_t)((m + 15) / 16 * 16) * w->cols)) {  // fully written below, but for rows that reach no result
+      int rc = launch_rows_planes(operands, x, m, (int)w->cols, prologue, norm_g, norm_b, eps, kTermsOperands);
+      if (!rc) rc = launch_linear_few(y, w, operands, m, bias, residual, act, nullptr);
+      const int rf = cthip_free(operands);  // stream-ordered: handed out again only to later work on this stream
+      return rc ? rc : rf;
+    }
+  }
   if (m >= 8) {
     // several input rows: the MFMA tile path reads the weights once instead of once per row
     const float *xin = x;

@@ -1,0 +1,205 @@
+// Linear over 8 .. 64 rows that lie in memory as operands of two bf16 terms (store_operands4 in planes.h), on packed weights of up to 2048 columns: the
+// projections of a short prompt, or of the next turn of a conversation.
+//
+// The tiles of matmul.hip give such a product to a whole chip only by splitting K, which leaves partial tiles in memory and a
+// second launch that adds them up.  Here a workgroup owns 16 NB output columns and ALL of K: its eight wavefronts take an eighth of K each,
+// fetch their pieces of the weights and of the rows straight into operand registers (v_mfma_f32_16x16x32_bf16, lane l: row l % 16, k = 8 (l / 16) .. + 7 of a
+// block of 32), BATCH blocks asked for together, and meet once in LDS.  A workgroup reads nothing twice; the rows are read by all of them, out of L2,
+// and lie as the wavefronts hold them, whole cache lines to a request (as rows of terms, 16 half lines a request: 9.2 us for 37 rows of 1024 x 4096 fp16, 7.6 this
+// way; by tiles 7.9 and 3.3 for their sums).  What bounds it: a launch, one round trip for a batch, and what a compute unit pulls out of
+// L2 (all rows and its columns: 220 KB there).
+// Products as in the tiles: the integers of a quantised weight are exact in bf16, their block's scale is applied to the block's
+// sum; an fp16 weight is two terms, and the product of both lower terms is left out.  Error against 64 bits the same (2.5e-6, fp16 3.7e-6).
+#include "common.h"
+#include "planes.h"
+
+namespace cthip {
+
+struct FewArgs {
+  const unsigned char *A;    // the rows as operands of two terms (store_operands4)
+  const unsigned char *W;    // N rows of packed weights, wpitch bytes apart
+  const unsigned short *wd;  // scales, nkb a row
+  int wpitch;
+  int nkb;                   // blocks of 32 k
+  PlaneGemmArgs e;           // M, N and what happens to the result
+};
+
+enum { FW_Q8 = 0, FW_Q4 = 1, FW_F16 = 2 };
+typedef float v4f_few __attribute__((ext_vector_type(4)));
+constexpr int kFewWaves = 8;
+
+template <int SRC, int MB, int NB, int BATCH>
+__global__ __launch_bounds__(64 * kFewWaves, MB * NB <= 2 && BATCH <= 5 ? 4 : 2) void k_linear_few(FewArgs a) {
+  constexpr int NPB = SRC == FW_F16 ? 2 : 1, ROWS = 16 * MB, COLS = 16 * NB;
+  extern __shared__ __align__(16) float red[];  // [wavefront][row][column]
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, col = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * COLS, M = a.e.M, N = a.e.N;
+  const int per = (a.nkb + kFewWaves - 1) / kFewWaves, kb0 = wv * per, kb1 = min(a.nkb, kb0 + per);
+  const unsigned char *ap = a.A + lane * 16;
+  const unsigned char *wp[NB];
+  const unsigned short *dp[NB];
+  v4f_few acc[MB][NB];
+#pragma unroll
+  for (int j = 0; j < NB; j++) {
+    const int n = min(n0 + 16 * j + col, N - 1);  // columns past the end repeat the last one
+    // 8 k of a block: 8 bytes of Q8_0; the low (k < 16) or high nibbles of 8 bytes of Q4_0; 16 bytes of fp16
+    wp[j] = a.W + (int64_t)n * a.wpitch + (SRC == FW_Q8 ? 8 * g : SRC == FW_Q4 ? 8 * (g & 1) : 16 * g);
+    dp[j] = SRC == FW_F16 ? nullptr : a.wd + (int64_t)n * a.nkb;
+#pragma unroll
+    for (int i = 0; i < MB; i++) acc[i][j] = v4f_few{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  for (int b0 = kb0; b0 < kb1; b0 += BATCH) {
+    // every request of the batch, none behind a branch: blocks past the share repeat its last one and are not multiplied
+    uint4 w[BATCH][NB];
+    unsigned d[BATCH][NB];
+    v8bf af[BATCH][MB][2];
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) {
+      const int kb = min(b0 + b, kb1 - 1);
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        if constexpr (SRC == FW_F16) {
+          w[b][j] = *(const uint4 *)(wp[j] + kb * 64);
+        } else {
+          const uint2 t = *(const uint2 *)(wp[j] + kb * (SRC == FW_Q8 ? 32 : 16));
+          w[b][j].x = t.x, w[b][j].y = t.y;
+          d[b][j] = dp[j][kb];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int i = 0; i < MB; i++) af[b][i][q] = __builtin_bit_cast(v8bf, *(const uint4 *)(ap + ((kb * 2 + q) * MB + i) * 1024));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) {
+      if (b0 + b >= kb1) break;  // (uniform)
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        v8bf bf[NPB];
+        const uint4 v = w[b][j];
+        if constexpr (SRC == FW_F16) {
+          const unsigned h[4] = {v.x, v.y, v.z, v.w};
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 4; e++) x[2 * e] = half_bits_to_float((unsigned short)(h[e] & 0xffff)), x[2 * e + 1] = half_bits_to_float((unsigned short)(h[e] >> 16));
+          uint4 pl[2];
+          split8_planes<2>(x, pl);
+          bf[0] = __builtin_bit_cast(v8bf, pl[0]);
+          bf[NPB - 1] = __builtin_bit_cast(v8bf, pl[1]);
+        } else if constexpr (SRC == FW_Q8) {
+          bf[0] = bf_of_q8(v.x, v.y);
+        } else {
+          const int sh = 4 * (g >> 1);
+          const unsigned lo = (((v.x >> sh) & 0x0f0f0f0fu) + 0x78787878u) ^ 0x80808080u, hi = (((v.y >> sh) & 0x0f0f0f0fu) + 0x78787878u) ^ 0x80808080u;  // nibble - 8 as int8
+          bf[0] = bf_of_q8(lo, hi);
+        }
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+          if constexpr (SRC == FW_F16) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][1], bf[0], acc[i][j], 0, 0, 0);  // smallest products first
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][0], bf[NPB - 1], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][0], bf[0], acc[i][j], 0, 0, 0);
+          } else {
+            v4f_few t = {0.0f, 0.0f, 0.0f, 0.0f};
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][1], bf[0], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][0], bf[0], t, 0, 0, 0);
+            const float dd = half_bits_to_float((unsigned short)d[b][j]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(dd, t[r], acc[i][j][r]);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) red[(wv * ROWS + 16 * i + 4 * g + r) * COLS + 16 * j + col] = acc[i][j][r];
+  __syncthreads();
+  for (int f = tid; f < M * (COLS / 4); f += 64 * kFewWaves) {
+    const int m = f / (COLS / 4), c = 4 * (f % (COLS / 4));
+    float4 t[kFewWaves], v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int w = 0; w < kFewWaves; w++) t[w] = *(const float4 *)(red + (w * ROWS + m) * COLS + c);
+#pragma unroll
+    for (int w = 0; w < kFewWaves; w++) v.x += t[w].x, v.y += t[w].y, v.z += t[w].z, v.w += t[w].w;
+    plane_gemm_store(a.e, m, n0 + c, v);
+  }
+}
+
+// Against a launch of tiles, for the most part with a second one for their sums; us, m = 8 / 17 / 40 / 64, the norm in front included:
+//   Q8_0 768 x 2304 10.9 / 11.1 / 11.7 / 12.0 -> 7.0 / 7.3 / 8.1 / 8.8, 1280 x 5120 13.0 / 13.3 / 14.9 / 16.0 -> 9.5 / 10.5 / 11.7 / 13.0; Q4_0 alike;
+//   f16 1024 x 4096 11.1 / 11.4 / 12.4 / 13.7 -> 6.8 / 7.3 / 8.5 / 9.2, 2048 x 11264 m = 17 / 40 / 64 30.9 / 31.9 / 34.8 -> 19.7 / 21.6 / 24.7.
+// Short rows of many columns and long rows of few are where it loses (256 x 8192 m = 64 8.9 -> 9.4, 2048 x 256 m = 64 12.1 -> 12.8).  Where the rows are not
+// passed over anyway its operands are a launch of their own, 2.5 us: 1024 x 4096 f16 8.5 / 8.9 / 9.8 / 10.8 -> 6.4 / 7.0 / 8.0 / 8.7, but 2048 x 768
+// 8.1 / 8.1 / 8.5 / 8.9 -> 7.7 / 9.1 / 10.7 / 12.4, 256 x 768 5.7 / 5.8 / 5.8 / 6.2 -> 5.9 / 6.2 / 6.8 / 7.3.
+bool linear_few_pays(const WMat *w, int m, int precision, bool norm) {
+  if (precision != GEMM_BF16X3 || m < 8 || m > 64 || w->cols % 32 || w->cols > 2048 || w->rows % 4 || w->rows > 48ll * state().compute_units) return false;
+  if (w->type != CTHIP_Q8_0 && w->type != CTHIP_Q4_0 && w->type != CTHIP_F16) return false;
+  if (norm) return w->cols < 512 ? w->rows <= (m > 32 ? 4096 : 8192) : !(m > 32 && w->cols > 1280 && w->rows < 512);
+  return w->cols >= 512 && w->rows <= 8192 && (w->cols <= 1280 ? m <= 32 || w->rows >= 512 : m <= 16);
+}
+
+template <int SRC, int MB, int NB>
+static int few_launch(const FewArgs &a) {
+  const dim3 grid((unsigned)((a.e.N + 16 * NB - 1) / (16 * NB))), block(64 * kFewWaves);
+  constexpr size_t lds = (size_t)kFewWaves * 16 * MB * 16 * NB * 4;
+  const int per = (a.nkb + kFewWaves - 1) / kFewWaves;  // blocks of a wavefront: in one batch where registers hold them
+  if constexpr (NB == 3) {
+    if (lds > 64 * 1024) CTHIP_CHECK(hipFuncSetAttribute((const void *)k_linear_few<SRC, MB, 3, (MB <= 2 ? 4 : 2)>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_linear_few<SRC, MB, 3, (MB <= 2 ? 4 : 2)>), grid, block, lds, state().stream, a);
+    CTHIP_LAUNCH_CHECK();
+    return 0;
+  }
+  constexpr int kLong = MB <= 2 ? 8 : 4;
+  if (per <= 4) hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, 4>), grid, block, lds, state().stream, a);
+  else if (per == 5) hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, 5>), grid, block, lds, state().stream, a);
+  else hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, kLong>), grid, block, lds, state().stream, a);
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+
+// y (m, rows) = act(x W^T + bias) + residual; act may be kActSwigluPairs, route as for launch_linear_gemm.
+// Call only where linear_few_pays; y, bias and residual on 16 bytes.
+int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route) {
+  FewArgs a = {};
+  a.nkb = (int)(w->cols / 32);
+  a.A = (const unsigned char *)operands;
+  a.W = (const unsigned char *)w->q;
+  a.wd = (const unsigned short *)w->d;
+  a.wpitch = (int)(w->type == CTHIP_Q8_0 ? w->cols : w->type == CTHIP_Q4_0 ? w->cols / 2 : 2 * w->cols);
+  a.e.C = y;
+  a.e.M = m, a.e.N = (int)w->rows;
+  a.e.bias = bias, a.e.residual = residual;
+  a.e.act = act;
+  if (act == kActSwigluPairs) {
+    if (residual || route) return fail(CTHIP_E_BAD_ARG, "launch_linear_few: paired SwiGLU epilogue with a residual or a route");
+    a.e.act = CTHIP_ACT_NONE;
+    a.e.pairs = 1;
+  }
+  if (route) {
+    a.e.routed = 1;
+    a.e.route = *route;
+  }
+  const int nb = (a.e.N + 16 * state().compute_units - 1) / (16 * state().compute_units);  // 16 columns a workgroup, 32 or 48 where that is the one round over the chip
+#define FEW2(SRC, MB) return nb == 1 ? few_launch<SRC, MB, 1>(a) : nb == 2 ? few_launch<SRC, MB, 2>(a) : few_launch<SRC, MB, 3>(a)
+#define FEW(SRC)               \
+  do {                         \
+    if (m <= 16) FEW2(SRC, 1); \
+    if (m <= 32) FEW2(SRC, 2); \
+    if (m <= 48) FEW2(SRC, 3); \
+    FEW2(SRC, 4);              \
+  } while (0)
+  if (w->type == CTHIP_Q8_0) FEW(FW_Q8);
+  if (w->type == CTHIP_Q4_0) FEW(FW_Q4);
+  FEW(FW_F16);
+#undef FEW
+#undef FEW2
+}
+
+}  // namespace cthip

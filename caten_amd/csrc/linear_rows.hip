@@ -359,6 +359,7 @@ struct RowsPlanesArgs {
   int K, kbp;
   const float *g, *b;
   float eps;
+  int row_blocks;  // not ROWS: as matrix operands of that many blocks of 16 rows (store_operands4), 0 = as planes
 };
 template <int PRO, int NP, bool ROWS, int NT, int VPL>
 __global__ __launch_bounds__(NT) void k_rows_planes(RowsPlanesArgs a) {
@@ -438,7 +439,9 @@ __global__ __launch_bounds__(NT) void k_rows_planes(RowsPlanesArgs a) {
       if (ROWS) split8_rows<NP>(t, pl);
       else split8_planes<NP>(t, pl);
 #pragma unroll
-      for (int q = 0; q < NP; q++) a.out[((int64_t)blockIdx.x * a.kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
+      for (int q = 0; q < NP; q++)
+        if (!ROWS && a.row_blocks) a.out[((int64_t)((c >> 2) * NP + q) * a.row_blocks + (blockIdx.x >> 4)) * 64 + 16 * (c & 3) + (blockIdx.x & 15)] = pl[q];
+        else a.out[((int64_t)blockIdx.x * a.kbp + (c >> 2)) * (4 * NP) + 4 * q + (c & 3)] = pl[q];
     }
   };
   emit(1.0f);
@@ -560,8 +563,8 @@ bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, in
 
 // rows with what a Linear has in front of it as bf16 planes for gemm_planes.hip (x on 16 bytes, K % 32 == 0)
 bool rows_planes_supported(int K) { return K % 32 == 0 && K <= kRowsPlanesMaxK; }
-int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps) {
-  const RowsPlanesArgs pa = {(uint4 *)planes, nullptr, x, K, K, K / 32, g, b, eps};
+int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps, int terms) {
+  const RowsPlanesArgs pa = {(uint4 *)planes, nullptr, x, K, K, K / 32, g, b, eps, terms == kTermsOperands ? (m + 15) / 16 : 0};
   if (pro == CTHIP_PRO_LAYERNORM) rows_planes_launch<CTHIP_PRO_LAYERNORM, 2, false>(pa, m);
   else if (pro == CTHIP_PRO_RMSNORM) rows_planes_launch<CTHIP_PRO_RMSNORM, 2, false>(pa, m);
   else rows_planes_launch<CTHIP_PRO_NONE, 2, false>(pa, m);
@@ -604,7 +607,7 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
   a.rscale = rscale;
   int rc = 0;
   a.A = planes;
-  const RowsPlanesArgs pa = {(uint4 *)planes, rscale, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps};
+  const RowsPlanesArgs pa = {(uint4 *)planes, rscale, x, x_stride, (int)w->cols, a.nkb, norm_g, pro == CTHIP_PRO_LAYERNORM || m >= 8 ? norm_b : nullptr, eps, 0};
 #define RP2(PRO)                                              \
   do {                                                        \
     if (terms == 3) rows_planes_launch<PRO, 3, true>(pa, m);  \

@@ -62,6 +62,17 @@ __device__ __forceinline__ void store_planes4(unsigned short *planes, int64_t ro
   *(uint2 *)(p + 32) = pl[1];
 }
 
+// The same for a handful of rows (linear_few.hip), as operands of v_mfma_f32_16x16x32_bf16 lie in a wavefront: [block of 32 k][term][16 rows][lane][8 k],
+// lane = 16 (k / 8 of the block) + row % 16, row_blocks = blocks of 16 rows
+__device__ __forceinline__ void store_operands4(unsigned short *planes, int row, int row_blocks, int col, const float *v) {
+  uint2 pl[2];
+  split4_planes<2>(v[0], v[1], v[2], v[3], pl);
+  const int lane = 16 * ((col >> 3) & 3) + (row & 15);
+  unsigned short *p = planes + (((int64_t)(col >> 5) * 2 * row_blocks + (row >> 4)) * 64 + lane) * 8 + (col & 7);
+  *(uint2 *)p = pl[0];
+  *(uint2 *)(p + row_blocks * 512) = pl[1];
+}
+
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // 16 bytes per lane from sbase + voff straight into LDS at lds + 16 * lane.  Written out because the compiler, which

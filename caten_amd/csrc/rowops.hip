@@ -139,7 +139,8 @@ struct ReduceNormArgs {
   float eps;
   int64_t rows;
   int n;
-  unsigned short *planes;  // non-null: the normalised rows go out as two bf16 terms (gemm_planes.hip) instead of y
+  unsigned short *planes;  // non-null: the normalised rows go out as two bf16 terms (gemm_planes.hip) instead of y ...
+  int row_blocks;          // ... or, when set, as matrix operands of that many blocks of 16 rows (linear_few.hip)
 };
 
 template <int MODE, int VPL, int NZ>
@@ -202,7 +203,8 @@ __global__ __launch_bounds__(256) void k_reduce_norm(ReduceNormArgs a) {
       const float4 g = a.g ? gm[j] : make_float4(1.f, 1.f, 1.f, 1.f);
       const float4 b = a.b ? bt[j] : make_float4(0.f, 0.f, 0.f, 0.f);
       const float o[4] = {v[j][0] * rstd * g.x + b.x, v[j][1] * rstd * g.y + b.y, v[j][2] * rstd * g.z + b.z, v[j][3] * rstd * g.w + b.w};
-      if (a.planes) store_planes4(a.planes, row, n >> 5, 4 * (lane + 64 * j), o);
+      if (a.planes && a.row_blocks) store_operands4(a.planes, (int)row, a.row_blocks, 4 * (lane + 64 * j), o);
+      else if (a.planes) store_planes4(a.planes, row, n >> 5, 4 * (lane + 64 * j), o);
       else ((float4 *)(a.y + row * n))[lane + 64 * j] = make_float4(o[0], o[1], o[2], o[3]);
     }
   }
@@ -277,7 +279,8 @@ __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
       const float4 g = a.g ? gm[j] : make_float4(1.f, 1.f, 1.f, 1.f);
       const float4 b = a.b ? bt[j] : make_float4(0.f, 0.f, 0.f, 0.f);
       const float o[4] = {v[j][0] * rstd * g.x + b.x, v[j][1] * rstd * g.y + b.y, v[j][2] * rstd * g.z + b.z, v[j][3] * rstd * g.w + b.w};
-      if (a.planes) store_planes4(a.planes, row, n >> 5, 4 * (tid + 256 * j), o);
+      if (a.planes && a.row_blocks) store_operands4(a.planes, (int)row, a.row_blocks, 4 * (tid + 256 * j), o);
+      else if (a.planes) store_planes4(a.planes, row, n >> 5, 4 * (tid + 256 * j), o);
       else ((float4 *)(a.y + row * n))[tid + 256 * j] = make_float4(o[0], o[1], o[2], o[3]);
     }
   }
@@ -286,11 +289,11 @@ __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
 bool reduce_norm_supported(int n, int nparts) { return reduce_norm_plan(n, nparts, 1).ok || reduce_norm_plan(n, nparts, 1 << 20).ok; }
 
 int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, int64_t part_stride, const float *bias,
-                       const float *resid, const float *g, const float *b, float eps, int64_t rows, int n, bool rms, bool terms) {
+                       const float *resid, const float *g, const float *b, float eps, int64_t rows, int n, bool rms, int terms) {
   if (rows == 0 || n == 0) return 0;
   if (terms && n % 32) return fail(CTHIP_E_BAD_ARG, "reduce + norm: rows of %d as terms", n);
   if (!reduce_norm_supported(n, nparts)) return fail(CTHIP_E_BAD_ARG, "reduce + norm: rows of %d with %d shares", n, nparts);
-  ReduceNormArgs a = {y, xout, parts, nparts, part_stride, bias, resid, g, b, eps, rows, n, terms ? (unsigned short *)y : nullptr};
+  ReduceNormArgs a = {y, xout, parts, nparts, part_stride, bias, resid, g, b, eps, rows, n, terms ? (unsigned short *)y : nullptr, terms == kTermsOperands ? (int)(rows + 15) / 16 : 0};
   hipStream_t st = state().stream;
   const ReduceNormPlan pl = reduce_norm_plan(n, nparts, rows);
   if (pl.wide) {
