@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void k_copies(CopyBatch cb) {
 }
 
 // One row of one batch: scores (bmm.hip's KC layout), softmax, values (NC layout), copy.  Sums as in k_bmm.  The row's scores stay in
-// LDS; a 12-head step at position 30: 9 us instead of six launches of 2.6 - 4.8, every one of them behind the host.
+// LDS; a 12-head step at position 30: 8 us instead of six launches of 2.6 - 4.8, every one of them behind the host.
 struct GraphAttn {
   BmmArgs s, v;
   float *probs;
@@ -80,10 +80,6 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
     const int64_t d0 = p - a.pre_out[0], d1 = p - a.pre_out[1];
     return d0 >= 0 && d0 < a.pre_n[0] ? a.pre_in[0] + d0 : d1 >= 0 && d1 < a.pre_n[1] ? a.pre_in[1] + d1 : p;
   };
-#pragma unroll
-  for (int q = 0; q < 2; q++)
-    for (int t = 4 * ((blockIdx.y * gridDim.x + blockIdx.x) * 256 + tid); t < a.pre_n[q]; t += 1024 * gridDim.x * gridDim.y)
-      *(float4 *)(a.pre_out[q] + t) = *(const float4 *)(a.pre_in[q] + t);
   float4 vw[4];
   {
     // the first keys' values are asked for ahead of the scores: they arrive behind them
@@ -201,6 +197,11 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
     }
     __syncthreads();
   }
+  // (the copies last: in front, everything else waited for their round trip to memory: 9.3 -> 8.1 us a launch of a 12-head step at position 27)
+#pragma unroll
+  for (int q = 0; q < 2; q++)
+    for (int t = 4 * ((blockIdx.y * gridDim.x + blockIdx.x) * 256 + tid); t < a.pre_n[q]; t += 1024 * gridDim.x * gridDim.y)
+      *(float4 *)(a.pre_out[q] + t) = *(const float4 *)(a.pre_in[q] + t);
 }
 
 // ---- what a chain may touch ----
