@@ -378,6 +378,13 @@ __device__ __forceinline__ float group_sum(float v) {
   if (G == 32) v += __shfl_xor(v, 16, 64);
   return v;
 }
+template <int G>
+__device__ __forceinline__ float group_max(float v) {
+  if (G == 64) return wave_max(v);
+  v = row16_max(v);
+  if (G == 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return v;
+}
 
 __device__ __forceinline__ float half_bits_to_float(unsigned short h) {
   return (float)__builtin_bit_cast(_Float16, h);

@@ -2,11 +2,10 @@
 // LayerNorm->softmax), elementwise activations, embedding gather, argmax, RoPE
 // and the KV-cached attention of batch-1 decode.
 //
-// Row ops: one wavefront owns one row and keeps it in registers (VPL float4 per
-// lane, 128-bit coalesced loads/stores), so every row is read once and written
-// once; the reductions are 64-lane shuffles, no LDS.  Rows longer than
-// 64*4*8 = 2048 floats fall back to one 256-thread block per row that re-reads
-// the row through L2.
+// Row ops: one wavefront (short rows: a part of one) owns one row and keeps it in
+// registers (VPL float4 per lane, 128-bit loads / stores), so every row is read
+// once and written once; the reductions are lane moves, no LDS.  Rows longer than
+// 64*4*8 = 2048 floats take a block per row.
 #include <type_traits>
 #include "common.h"
 #include "planes.h"
@@ -342,12 +341,108 @@ int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, in
   return 0;
 }
 
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// Rows of 4 .. 2048 floats that are short or that k_rowop cannot read: LPR lanes hold a row, VPL chunks of four floats each, at any alignment (the loads
+// are 16 bytes at 4-byte alignment).  Chunk c starts at min(4c, n - 4): the last one of a row that is no multiple of four
+// overlaps its neighbour, whose share it leaves out of the sums and stores a second time with the same values.
+// U times 64 / LPR rows per wavefront, all of their requests in flight together.  A row of 87 floats is 348 bytes: a block per row with
+// a barrier per sum took 50 us over 65 536 of them, bound by blocks to start and round trips, this 8.6 (5.3 TB/s).
+template <int MODE, int LPR, int VPL, int U>
+__global__ __launch_bounds__(256) void k_rowop_any(RowArgs a) {
+  constexpr bool NORM = MODE != ROW_SOFTMAX;
+  constexpr int RPW = 64 / LPR;
+  const int lane = threadIdx.x & 63, sub = lane & (LPR - 1), n = a.n, nc = (n + 3) >> 2;
+  const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (RPW * U) + lane / LPR;
+  f4_any t[U][VPL], gm[NORM ? VPL : 1], bt[NORM ? VPL : 1];
+  int at[VPL], own[VPL];  // a chunk's first element, and the first one that is its own (4: none)
+#pragma unroll
+  for (int j = 0; j < VPL; j++) {
+    const int c = sub + LPR * j;
+    at[j] = min(4 * c, n - 4);
+    own[j] = c < nc ? 4 * c - at[j] : 4;
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const float *xr = a.x + min(row0 + RPW * u, a.rows - 1) * n;
+#pragma unroll
+    for (int j = 0; j < VPL; j++) t[u][j] = *(const f4_any *)(xr + at[j]);
+  }
+  if (NORM) {
+    const float *gp = a.g ? a.g : a.x, *bp = a.b ? a.b : a.x;  // a.x: unused stand-in, so that no request sits behind a branch
+#pragma unroll
+    for (int j = 0; j < VPL; j++) {
+      gm[NORM ? j : 0] = *(const f4_any *)(gp + at[j]);
+      bt[NORM ? j : 0] = *(const f4_any *)(bp + at[j]);
+      if (!a.g) gm[NORM ? j : 0] = f4_any{1.0f, 1.0f, 1.0f, 1.0f};
+      if (!a.b) bt[NORM ? j : 0] = f4_any{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+  const float inv_n = 1.0f / (float)n;
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    float v[VPL][4];
+#pragma unroll
+    for (int j = 0; j < VPL; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[j][e] = t[u][j][e];
+    if (NORM) {
+      float mean = 0.0f, q = 0.0f;
+      if (MODE != ROW_RMSNORM) {
+        float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPL; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) s += e >= own[j] ? v[j][e] : 0.0f;
+        mean = group_sum<LPR>(s) * inv_n;
+      }
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          v[j][e] -= mean;
+          q += e >= own[j] ? v[j][e] * v[j][e] : 0.0f;
+        }
+      const float rstd = 1.0f / sqrtf(group_sum<LPR>(q) * inv_n + a.eps);
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[j][e] = v[j][e] * rstd * gm[NORM ? j : 0][e] + bt[NORM ? j : 0][e];
+    }
+    if (MODE == ROW_SOFTMAX || MODE == ROW_LN_SOFTMAX) {
+      float m = -INFINITY, s = 0.0f;  // (a maximum may count an element twice)
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) m = fmaxf(m, v[j][e]);
+      m = group_max<LPR>(m);
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          v[j][e] = ct_exp(v[j][e] - m);
+          s += e >= own[j] ? v[j][e] : 0.0f;
+        }
+      const float inv = 1.0f / group_sum<LPR>(s);
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[j][e] *= inv;
+    }
+    if (row0 + RPW * u < a.rows) {
+      float *yr = a.y + (row0 + RPW * u) * n;
+#pragma unroll
+      for (int j = 0; j < VPL; j++)
+        if (own[j] < 4) *(f4_any *)(yr + at[j]) = f4_any{v[j][0], v[j][1], v[j][2], v[j][3]};
+    }
+  }
+}
+
 // Softmax of rows of any length from 4 up to 4 NT VPL floats (LayerNorm -> softmax likewise), at any alignment: one block
 // per row, the row in its registers (read once, written once).  Chunk c of four floats starts at min(4c, n - 4): the last
 // one of a row that is no multiple of four overlaps its neighbour, whose share it leaves out of the sums and stores a second
 // time with the same values.  (The loads are 16 bytes at 4-byte alignment.)  What this replaces read the row three to five
 // times, a float per lane: (5402, 7011) 102 -> 51 us, 5.9 TB/s.
-typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
 template <int MODE, int NT, int VPL>
 __global__ __launch_bounds__(NT) void k_rowop_block(RowArgs a) {
   constexpr int NW = NT / 64;
@@ -575,14 +670,13 @@ template <int MODE>
 static int launch_rowop(RowArgs a) {
   if (a.rows == 0 || a.n == 0) return 0;
   hipStream_t st = state().stream;
-  if (a.n % 4 == 0 && a.n <= 2048 && ((uintptr_t)a.x % 16 == 0) && ((uintptr_t)a.y % 16 == 0) &&
+  if (a.n % 4 == 0 && a.n > 256 && a.n <= 2048 && ((uintptr_t)a.x % 16 == 0) && ((uintptr_t)a.y % 16 == 0) &&
       (!a.g || (uintptr_t)a.g % 16 == 0) && (!a.b || (uintptr_t)a.b % 16 == 0)) {
     const int n4 = a.n / 4;
     const int vpl = (n4 + 63) / 64;
     if ((a.rows + 3) / 4 > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "row op: too many rows");
     dim3 grid((unsigned)((a.rows + 3) / 4)), block(256);
     switch (vpl) {
-      case 1: hipLaunchKernelGGL((k_rowop<MODE, 1>), grid, block, 0, st, a); break;
       case 2: hipLaunchKernelGGL((k_rowop<MODE, 2>), grid, block, 0, st, a); break;
       case 3: hipLaunchKernelGGL((k_rowop<MODE, 3>), grid, block, 0, st, a); break;
       case 4: hipLaunchKernelGGL((k_rowop<MODE, 4>), grid, block, 0, st, a); break;
@@ -592,9 +686,37 @@ static int launch_rowop(RowArgs a) {
     CTHIP_LAUNCH_CHECK();
     return 0;
   }
+  const int nc = (a.n + 3) / 4;
+  // Up to 256 floats whatever their alignment (65 536 rows: LayerNorm of 40 13.5 -> 5.2 us, of 87 50 -> 8.6, LayerNorm -> softmax of 128 22.8 -> 12.6, RMSNorm of
+  // 255 43 -> 20.7; 256 aligned 21.1 -> 20.3).  Longer ones that k_rowop cannot read: norms up to its 2048 (2047: 82.6 -> 76.6, 511: 58 -> 40), softmax up to
+  // 1024 (LayerNorm -> softmax of 403 41.5 -> 31.5, of 1001 76 -> 73; of 2047 a block per row is better: 71.8, 78 this way).
+  if (a.n >= 4 && a.n <= (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM ? 2048 : 1024)) {
+    const int lpr = nc <= 16 ? 16 : nc <= 32 ? 32 : 64;
+    // two passes of rows per wavefront where that leaves every SIMD eight wavefronts (65 536 rows of 255: 26 -> 20.9 us)
+    const int64_t once = (int64_t)(64 / lpr) * 4, full = 8ll * state().compute_units;
+    const bool two = nc <= 64 && a.rows >= 2 * once * full;
+    const int64_t blocks = (a.rows + once * (two ? 2 : 1) - 1) / (once * (two ? 2 : 1));
+    if (blocks > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "row op: too many rows");
+#define ROW_ANY(LPR, VPL, U) hipLaunchKernelGGL((k_rowop_any<MODE, LPR, VPL, U>), dim3((unsigned)blocks), dim3(256), 0, st, a)
+    if (nc <= 16 && two) ROW_ANY(16, 1, 2);
+    else if (nc <= 16) ROW_ANY(16, 1, 1);
+    else if (nc <= 32 && two) ROW_ANY(32, 1, 2);
+    else if (nc <= 32) ROW_ANY(32, 1, 1);
+    else if (nc <= 64 && two) ROW_ANY(64, 1, 2);
+    else if (nc <= 64) ROW_ANY(64, 1, 1);
+    else if (nc <= 128) ROW_ANY(64, 2, 1);
+    else if (nc <= 192) ROW_ANY(64, 3, 1);
+    else if (nc <= 256) ROW_ANY(64, 4, 1);
+    else if constexpr (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM) {
+      if (nc <= 384) ROW_ANY(64, 6, 1);
+      else ROW_ANY(64, 8, 1);
+    }
+#undef ROW_ANY
+    CTHIP_LAUNCH_CHECK();
+    return 0;
+  }
   if (a.rows > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "row op: too many rows");
   const dim3 grid((unsigned)a.rows);
-  const int nc = (a.n + 3) / 4;
   // Pieces of rows where no block holds a row, or where at most a quarter of the chip would hold one: a block takes 9.7 us
   // over a row of 50 257, two launches over its pieces 6.4 up to 21 rows and as much as the blocks at 64
   const bool split = MODE == ROW_SOFTMAX && a.rows <= 65535 && (nc > 16384 || (nc > 8192 && a.rows <= 48));
@@ -612,8 +734,7 @@ static int launch_rowop(RowArgs a) {
   }
   if constexpr (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM) {
 #define NORM_BLOCK(VPL) hipLaunchKernelGGL((k_norm_block<MODE, VPL>), grid, dim3(256), 0, st, a)
-    if (a.n <= 1024) NORM_BLOCK(4);
-    else if (a.n <= 2048) NORM_BLOCK(8);
+    if (a.n < 4) hipLaunchKernelGGL((k_rowop_generic<MODE>), grid, dim3(256), 0, st, a);
     else if (a.n <= 4096) NORM_BLOCK(16);
     else if (a.n <= 8192) NORM_BLOCK(32);
     else if (a.n <= 16384) NORM_BLOCK(64);
@@ -624,8 +745,6 @@ static int launch_rowop(RowArgs a) {
   } else {
 #define ROW_BLOCK(NT, VPL) hipLaunchKernelGGL((k_rowop_block<MODE, NT, VPL>), grid, dim3(NT), 0, st, a)
   if (a.n < 4 || nc > 16384) hipLaunchKernelGGL((k_rowop_generic<MODE>), grid, dim3(256), 0, st, a);
-  else if (nc <= 64) ROW_BLOCK(64, 1);
-  else if (nc <= 256) ROW_BLOCK(64, 4);
   else if (nc <= 512) ROW_BLOCK(256, 2);
   else if (nc <= 1024) ROW_BLOCK(256, 4);
   else if (nc <= 2048) ROW_BLOCK(256, 8);
@@ -641,39 +760,20 @@ static int launch_rowop(RowArgs a) {
 
 
 // ------------------------------------------------------------------ elementwise
-// A block owns UNARY_PER_BLOCK consecutive elements; a thread takes UNARY_VEC-wide pieces 256 pieces apart, all of
-// its loads issued before the first store.  (A capped grid with a grid-stride loop, one float4 in flight per thread,
-// ran at 75 us on 50 M elements; this at what the renderer's element-wise kernels reach.)
-template <int VEC>
-__global__ __launch_bounds__(256) void k_unary(int kind, float *__restrict__ y, const float *__restrict__ x, int64_t n) {
-  constexpr int PER = 256 * 4 * VEC;  // elements per block
-  const int64_t base = (int64_t)blockIdx.x * PER;
-  if (base + PER <= n) {
-    if (VEC == 4) {
-      float4 v[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[e] = ((const float4 *)(x + base))[256 * e + threadIdx.x];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[e].x = apply_act(kind, v[e].x);
-        v[e].y = apply_act(kind, v[e].y);
-        v[e].z = apply_act(kind, v[e].z);
-        v[e].w = apply_act(kind, v[e].w);
-        ((float4 *)(y + base))[256 * e + threadIdx.x] = v[e];
-      }
-    } else {
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[e] = x[base + 256 * e + threadIdx.x];
-#pragma unroll
-      for (int e = 0; e < 4; e++) y[base + 256 * e + threadIdx.x] = apply_act(kind, v[e]);
-    }
-  } else {
-    for (int64_t k = base + threadIdx.x; k < n; k += 256) y[k] = apply_act(kind, x[k]);
+// Four elements a thread at any alignment (the loads are 16 bytes at 4-byte alignment); the up to three elements behind
+// the last piece are one more request of the last block.  Four pieces a thread gained nothing on large arrays (50 M elements 69 -> 66 us) and left
+// smaller ones to a few workgroups (900 000: SiLU 4.2 -> 2.9); a capped grid with a grid-stride loop took 75 us on 50 M.
+__global__ __launch_bounds__(256) void k_unary(int kind, float *y, const float *x, int64_t n) {
+  const int64_t nc = n >> 2, c = (int64_t)blockIdx.x * 256 + threadIdx.x, tail = 4 * nc + threadIdx.x;
+  const bool last = blockIdx.x == gridDim.x - 1 && tail < n;
+  const float vt = last ? x[tail] : 0.0f;
+  if (c < nc) {
+    const f4_any v = *(const f4_any *)(x + 4 * c);
+    *(f4_any *)(y + 4 * c) = f4_any{apply_act(kind, v.x), apply_act(kind, v.y), apply_act(kind, v.z), apply_act(kind, v.w)};
   }
+  if (last) y[tail] = apply_act(kind, vt);
 }
 
-// out[t,:] = W[idx[t],:]  (+ W2[pos0 + t,:] when W2 is given: wte + wpe of Transformer, layers.lisp:80-82)
 __global__ __launch_bounds__(256) void k_embedding(float *__restrict__ out, const float *__restrict__ W,
                                                    const float *__restrict__ idx_f, const int *__restrict__ idx_i,
                                                    int vocab, int dim, const float *__restrict__ W2,
@@ -1719,11 +1819,9 @@ int cthip_unary(int kind, float *y, const float *x, int64_t n) {
   CTHIP_ARG(n >= 0 && (n == 0 || (y && x)));
   CTHIP_ARG(kind >= CTHIP_ACT_NONE && kind <= CTHIP_ACT_TANH);
   if (n == 0) return 0;
-  const bool vec = ((uintptr_t)x % 16 == 0) && ((uintptr_t)y % 16 == 0);
-  const int64_t per = vec ? 4096 : 1024, blocks = (n + per - 1) / per;
+  const int64_t blocks = (n + 1023) / 1024;
   if (blocks > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "cthip_unary: %lld elements exceed the grid", (long long)n);
-  if (vec) hipLaunchKernelGGL(k_unary<4>, dim3((unsigned)blocks), dim3(256), 0, state().stream, kind, y, x, n);
-  else hipLaunchKernelGGL(k_unary<1>, dim3((unsigned)blocks), dim3(256), 0, state().stream, kind, y, x, n);
+  hipLaunchKernelGGL(k_unary, dim3((unsigned)blocks), dim3(256), 0, state().stream, kind, y, x, n);
   CTHIP_LAUNCH_CHECK();
   return 0;
 }

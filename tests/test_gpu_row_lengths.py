@@ -91,3 +91,69 @@ def test_layernorm_softmax_of_rows_that_are_not_finite(ops, rows, n):
         y[0, n - 1] = bad
         got = ops.layernorm_softmax(y)
         assert np.isnan(got[0]).all() and np.array_equal(got[1:], alone[1:])
+
+
+@pytest.mark.parametrize("n", [4, 5, 40, 63, 64, 65, 87, 127, 128, 129, 200, 255, 256, 258, 513, 770, 1023, 1537, 2047])
+@pytest.mark.parametrize("rows", [1, 7, 33, 40001])
+def test_rows_of_a_part_of_a_wavefront(ops, oracle, rows, n):
+    """Several rows per wavefront, one or two passes of them, at element offsets of any alignment; results may go where the input was,
+    a row that is not finite leaves its neighbours alone, and nothing is stored behind the last row."""
+    import ctypes as C
+    from caten_amd import _lib
+    lib = _lib.load()
+    if rows * n > 6_000_000:
+        rows = 6_000_000 // n
+    rng = np.random.default_rng(n)
+    x = rng.normal(0.3, 1, (rows, n)).astype(np.float32)
+    g, b = rng.normal(1, 0.02, n).astype(np.float32), rng.normal(0, 0.02, n).astype(np.float32)
+    bad = rows // 2
+    x[bad, n // 2] = np.inf
+    dev, gd, bd = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    for p, k in ((dev, rows * n + 16), (gd, n + 1), (bd, n + 1)):
+        _lib.check(lib.cthip_alloc(C.byref(p), 4 * k))
+    g1, b1 = np.concatenate([[0], g]).astype(np.float32), np.concatenate([[0], b]).astype(np.float32)
+    _lib.check(lib.cthip_h2d(gd, g1.ctypes.data_as(C.c_void_p), 4 * (n + 1)))
+    _lib.check(lib.cthip_h2d(bd, b1.ctypes.data_as(C.c_void_p), 4 * (n + 1)))
+    ok = np.arange(rows) != bad
+    for op, want, tol in (("softmax", oracle.softmax(x[ok]), (1e-4, 1e-7)), ("layernorm", oracle.layernorm(x[ok], g, b), (1e-4, 3e-5)),
+                          ("rmsnorm", oracle.rmsnorm(x[ok], g), (1e-4, 1e-5)), ("layernorm_softmax", oracle.softmax(oracle.layernorm(x[ok], g, b)), (1e-4, 1e-7))):
+        for off in (0, 1):
+            buf = np.full(rows * n + 16, 7.5, np.float32)
+            buf[off:off + rows * n] = x.ravel()
+            _lib.check(lib.cthip_h2d(dev, buf.ctypes.data_as(C.c_void_p), buf.nbytes))
+            p = C.c_void_p(dev.value + 4 * off)
+            gp, bp = C.c_void_p(gd.value + 4), C.c_void_p(bd.value + 4)
+            if op == "softmax":
+                rc = lib.cthip_softmax(p, p, rows, n)
+            elif op == "rmsnorm":
+                rc = lib.cthip_rmsnorm(p, p, gp, 1e-5, rows, n)
+            else:
+                rc = getattr(lib, "cthip_" + op)(p, p, gp, bp, 1e-5, rows, n)
+            _lib.check(rc)
+            _lib.check(lib.cthip_d2h(buf.ctypes.data_as(C.c_void_p), dev, buf.nbytes))
+            assert (buf[:off] == 7.5).all() and (buf[off + rows * n:] == 7.5).all()
+            y = buf[off:off + rows * n].reshape(rows, n)
+            close(y[ok], want, *tol)
+            assert np.isnan(y[bad, n // 2])
+    for p in (dev, gd, bd):
+        _lib.check(lib.cthip_free(p))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 1023, 1024, 1027, 4099, 100_001])
+def test_unary_of_any_length(ops, n):
+    import ctypes as C
+    from caten_amd import _lib
+    lib = _lib.load()
+    x = np.random.default_rng(n).normal(0, 2, n + 9).astype(np.float32)
+    dev = C.c_void_p()
+    _lib.check(lib.cthip_alloc(C.byref(dev), x.nbytes))
+    for off in (0, 1):
+        _lib.check(lib.cthip_h2d(dev, x.ctypes.data_as(C.c_void_p), x.nbytes))
+        p = C.c_void_p(dev.value + 4 * off)
+        _lib.check(lib.cthip_unary(3, p, p, n))
+        y = np.empty_like(x)
+        _lib.check(lib.cthip_d2h(y.ctypes.data_as(C.c_void_p), dev, x.nbytes))
+        want = x.astype(np.float64)
+        want[off:off + n] /= 1 + np.exp(-want[off:off + n])
+        close(y, want, 1e-5, 1e-6)
+    _lib.check(lib.cthip_free(dev))
