@@ -386,6 +386,8 @@ __device__ __forceinline__ float group_max(float v) {
   return v;
 }
 
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte access at 4-byte alignment
+
 __device__ __forceinline__ float half_bits_to_float(unsigned short h) {
   return (float)__builtin_bit_cast(_Float16, h);
 }

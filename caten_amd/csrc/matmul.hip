@@ -59,6 +59,9 @@ struct GemmArgs {
 // holds them k-contiguous per row in bf16, 16-byte chunks swizzled by row so that neither the operand
 // reads nor the staging writes collide on banks.  Two LDS buffers and three register sets keep the
 // global loads three K-steps ahead of the MFMAs with one barrier per step.
+// At one and two terms 80 registers per lane leave room for two workgroups on a compute unit, one multiplying while the other waits for its
+// barrier or stores (two terms with 96, one workgroup: 2048 x 2048 x 512 29.2 us, 23.6 with two; 1024^3, a tile per compute unit, 15.2 -> 14.0 by its
+// 32-bit offsets alone); the 96 KB of three terms allow one.
 enum { W_ROWMAJOR = 0, W_F32 = 1, W_F16 = 2, W_Q4 = 3, W_Q8 = 4 };  // W_Q4 / W_Q8: k_gemm_qpc only
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
@@ -91,17 +94,38 @@ __device__ __forceinline__ void split4(float r0, float r1, float r2, float r3, u
 __device__ __align__(16) unsigned g_zeros[8];  // zero-initialised, never written (not const: a load that may come from
                                                 // either here or an operand must stay a global-memory load)
 
-// Four consecutive floats at p without a branch or a dependent instruction: of the four, those past `nvalid`
-// (0..4) are read from g_zeros.  AL: the four are 16-byte aligned and all inside or all outside.  A K-step's
+// How a thread asks for four consecutive floats of an operand's row.  LD_VEC, LD_ANY: one 16-byte request inside the operand (rows of at least four floats),
+// at an offset from a uniform address: rows past the end are the last one, columns that reach past the end the row's last four.  What is past
+// the end of K becomes zero when it is staged; LD_ANY (rows of any alignment) then also moves the elements of a row's end into their place.
+// LD_ELEM: what is left (fewer than four columns, or more than 2^24).  At two terms, element by element / this way: 281^3 14.0 / 7.6 us, 587 x 1571 x 245
+// 24.6 / 9.3 (through planes), 17 x 4999 x 4999 43.5 / 27; fp32 operands 1001^3 37.6 / 30, three terms 36.8 / 24.
+enum { LD_ELEM = 0, LD_VEC = 1, LD_ANY = 2 };
+__device__ __forceinline__ float4 load4_in(const float *m, int off) {
+  const f4_any v = *(const f4_any *)((const char *)m + 4u * (unsigned)off);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+// LD_ELEM: four consecutive floats at p without a branch or a dependent instruction: of the four, those past `nvalid`
+// (0..4) are read from g_zeros.  Like the ones above a K-step's
 // requests stay one straight run of loads, so that the waits before their use count the younger requests
 // instead of draining them.
-template <bool AL>
 __device__ __forceinline__ float4 load4(const float *p, int nvalid) {
   const float *z = (const float *)g_zeros;
-  if (AL) return *(const float4 *)(nvalid > 0 ? p : z);
   return make_float4(*(nvalid > 0 ? p : z), *(nvalid > 1 ? p + 1 : z), *(nvalid > 2 ? p + 2 : z), *(nvalid > 3 ? p + 3 : z));
 }
+// the four are 16-byte aligned and all inside or all outside (k_gemm_f32pc and the kernels of packed weights: the matrix
+// instructions set their pace, and the moves into place cost them 3 - 8 %)
+__device__ __forceinline__ float4 load4_vec(const float *p, int nvalid) {
+  return *(const float4 *)(nvalid > 0 ? p : (const float *)g_zeros);
+}
 __device__ __forceinline__ int clamp04(int v) { return v < 0 ? 0 : v > 4 ? 4 : v; }
+// by = c - min(c, len - 4): elements move down by that many, zeros behind them (LD_VEC: none or all of them)
+template <int LD>
+__device__ __forceinline__ float4 shift4(float4 v, int by) {
+  if (LD == LD_ANY && (by & 1)) v = make_float4(v.y, v.z, v.w, 0.0f);
+  if (LD == LD_ANY && (by & 2)) v = make_float4(v.z, v.w, 0.0f, 0.0f);
+  if (by > 3) v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  return v;
+}
 
 struct ARegs {  // one K-step of A held by a thread: rows ar + 16 i
   float4 v0, v1, v2, v3;
@@ -137,7 +161,6 @@ __device__ __forceinline__ void store_tile(const GemmArgs &a, const float *Cs, i
     const int part = n0 >= a.route.c0[2] ? 2 : n0 >= a.route.c0[1] ? 1 : 0;  // uniform over the workgroup
     dst = a.route.dst[part], ldd = a.route.ld[part], cbase = a.route.c0[part];
   }
-  const bool vec = (N & 3) == 0 && (ldd & 3) == 0;
 #pragma unroll
   for (int j = 0; j < (BM * F4 + NT - 1) / NT; j++) {
     const int f = tid + NT * j, lr = f / F4, c4 = f % F4;
@@ -155,20 +178,20 @@ __device__ __forceinline__ void store_tile(const GemmArgs &a, const float *Cs, i
           make_float2(apply_act(CTHIP_ACT_SILU, v[0]) * v[1], apply_act(CTHIP_ACT_SILU, v[2]) * v[3]);
       continue;
     }
-    if (vec) {
+    if (col + 4 <= N) {  // (at any alignment: rows of N floats)
       if (!plain) {
         if (a.bias) {
-          const float4 bb = *(const float4 *)(a.bias + col);
+          const f4_any bb = *(const f4_any *)(a.bias + col);
           v[0] += bb.x, v[1] += bb.y, v[2] += bb.z, v[3] += bb.w;
         }
 #pragma unroll
         for (int t = 0; t < 4; t++) v[t] = apply_act(a.act, v[t]);
         if (a.residual) {
-          const float4 rr = *(const float4 *)(a.residual + (int64_t)row * N + col);
+          const f4_any rr = *(const f4_any *)(a.residual + (int64_t)row * N + col);
           v[0] += rr.x, v[1] += rr.y, v[2] += rr.z, v[3] += rr.w;
         }
       }
-      *(float4 *)o = make_float4(v[0], v[1], v[2], v[3]);
+      *(f4_any *)o = f4_any{v[0], v[1], v[2], v[3]};
     } else {
       for (int t = 0; t < 4 && col + t < N; t++) {
         float x = v[t];
@@ -182,8 +205,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &a, const float *Cs, i
   }
 }
 
-template <int BMODE, int NS, bool AL>
-__global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
+template <int BMODE, int NS, int LD>
+__global__ __launch_bounds__(768, NS == 6 ? 3 : 6) void k_gemm_split(GemmArgs a) {
   constexpr int BM = 64, BN = 64, BK = 64, LDK = BK, NP = (NS == 1) ? 1 : (NS == 3) ? 2 : 3;
   constexpr int NSET = 3;  // register sets = K-steps of global loads in flight
   constexpr int kOpBytes = 2 * NP * BM * LDK * 2, kCBytes = BM * (BN + 4) * 4;
@@ -223,7 +246,8 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
   auto fetch_a = [&](int k0, ARegs &ra) __attribute__((always_inline)) {  // k0 counts from kbeg
     auto ld = [&](int i) __attribute__((always_inline)) {
       const int row = m0 + ar + 16 * i, k = kbeg + k0 + 4 * akq;
-      return load4<AL>(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
+      if (LD != LD_ELEM) return load4_in(a.A + (int64_t)m0 * ldk, min(ar + 16 * i, M - 1 - m0) * ldk + min(k, ldk - 4));
+      return load4(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
     };
     ra.v0 = ld(0);
     ra.v1 = ld(1);
@@ -233,8 +257,9 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
   auto fetch_b = [&](int k0, BRegs<BMODE> &rb) __attribute__((always_inline)) {
     if (BMODE == W_ROWMAJOR) {
       auto ld = [&](int j) __attribute__((always_inline)) {
-        const int k = kbeg + k0 + 4 * bkq + j, n = n0 + 4 * bnq;
-        const float4 v = load4<AL>(a.B + (int64_t)k * N + n, k < K ? clamp04(N - n) : 0);
+        const int kb = min(kbeg + k0, ldk - 1), k = kbeg + k0 + 4 * bkq + j, n = n0 + 4 * bnq;
+        const float4 v = LD != LD_ELEM ? load4_in(a.B + (int64_t)kb * N, min(4 * bkq + j, ldk - 1 - kb) * N + min(n, N - 4))
+                                       : load4(a.B + (int64_t)k * N + n, k < K ? clamp04(N - n) : 0);
         return v4u{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
       };
       // constant indices only: the sets must stay in registers
@@ -261,8 +286,11 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
       }
     }
   };
-  auto stage_a = [&](const ARegs &ra, int buf) __attribute__((always_inline)) {
-    auto put = [&](int i, const float4 v) __attribute__((always_inline)) {
+  auto stage_a = [&](const ARegs &ra, int k0, int buf) __attribute__((always_inline)) {
+    const bool edge = LD != LD_ELEM && kbeg + k0 + BK > ldk && kbeg + k0 < ldk;  // uniform (a step past the end is not multiplied)
+    const int by = LD == LD_ANY ? kbeg + k0 + 4 * akq - min(kbeg + k0 + 4 * akq, ldk - 4) : kbeg + k0 + 4 * akq < ldk ? 0 : 4;
+    auto put = [&](int i, float4 v) __attribute__((always_inline)) {
+      if (edge) v = shift4<LD>(v, by);
       uint2 pl[NP];
       split4<NP>(v.x, v.y, v.z, v.w, pl);
 #pragma unroll
@@ -274,7 +302,19 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
     put(2, ra.v2);
     put(3, ra.v3);
   };
-  auto stage_b = [&](const BRegs<BMODE> &rb, int buf) __attribute__((always_inline)) {
+  auto stage_b = [&](const BRegs<BMODE> &rbi, int k0, int buf) __attribute__((always_inline)) {
+    BRegs<BMODE> rb = rbi;
+    if (BMODE == W_ROWMAJOR && LD != LD_ELEM && ((LD == LD_ANY && n0 + BN > N) || kbeg + k0 + BK > ldk) && kbeg + k0 < ldk) {  // uniform: columns into their place, zeros behind K
+      const int by = LD == LD_ANY ? n0 + 4 * bnq - min(n0 + 4 * bnq, N - 4) : 0;
+      auto fix = [&](v4u q, int j) __attribute__((always_inline)) {
+        const float4 v = shift4<LD>(make_float4(__uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z), __uint_as_float(q.w)), kbeg + k0 + 4 * bkq + j < ldk ? by : 4);
+        return v4u{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+      };
+      rb.v[0] = fix(rb.v[0], 0);
+      rb.v[BRegs<BMODE>::NV > 1 ? 1 : 0] = fix(rb.v[BRegs<BMODE>::NV > 1 ? 1 : 0], 1);
+      rb.v[BRegs<BMODE>::NV > 2 ? 2 : 0] = fix(rb.v[BRegs<BMODE>::NV > 2 ? 2 : 0], 2);
+      rb.v[BRegs<BMODE>::NV > 3 ? 3 : 0] = fix(rb.v[BRegs<BMODE>::NV > 3 ? 3 : 0], 3);
+    }
     if (BMODE == W_ROWMAJOR) {
       // column 4 bnq + i gets its 4 consecutive k: a 4x4 transpose in registers
       auto put = [&](int i, unsigned x0, unsigned x1, unsigned x2, unsigned x3) __attribute__((always_inline)) {
@@ -323,30 +363,35 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
       }
     }
   };
-  // all operand reads of a step are issued before its first matrix instruction: the matrix cores start when the
-  // first operands arrive and the rest come in behind them (read-then-use pairs each wait out an LDS round trip)
+  // operand reads are issued ahead of the matrix instructions, a whole step's (two terms: half a step's, for the registers): the matrix cores
+  // start when the first operands arrive and the rest come in behind them (read-then-use pairs each wait out an LDS round trip)
   auto mma = [&](int buf) __attribute__((always_inline)) {
     // 32x32x16: lane l holds A[i = l%32][k = 8*(l/32) .. +7] and B[k = 8*(l/32) .. +7][j = l%32]
     const int rowa = 32 * wm + (lane & 31), rowb = 32 * wn + (lane & 31);
-    v8bf av[BK / 16][NP], bv[BK / 16][NP];
+    constexpr int SL = NP == 2 ? 2 : BK / 16;  // k-slices read together
 #pragma unroll
-    for (int s = 0; s < BK / 16; s++) {
-      const int ch = 2 * s + (lane >> 5);
+    for (int s0 = 0; s0 < BK / 16; s0 += SL) {
+      v8bf av[SL][NP], bv[SL][NP];
 #pragma unroll
-      for (int p = 0; p < NP; p++) {
-        av[s][p] = __builtin_bit_cast(v8bf, *(const uint4 *)&As[buf][p][rowa][8 * (ch ^ swz(rowa))]);
-        bv[s][p] = __builtin_bit_cast(v8bf, *(const uint4 *)&Bs[buf][p][rowb][8 * (ch ^ swz(rowb))]);
+      for (int s = 0; s < SL; s++) {
+        const int ch = 2 * (s0 + s) + (lane >> 5);
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          av[s][p] = __builtin_bit_cast(v8bf, *(const uint4 *)&As[buf][p][rowa][8 * (ch ^ swz(rowa))]);
+          bv[s][p] = __builtin_bit_cast(v8bf, *(const uint4 *)&Bs[buf][p][rowb][8 * (ch ^ swz(rowb))]);
+        }
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int s = 0; s < BK / 16; s++) {
-      // every pair of planes whose product is above 2^-8(NP) of the leading one, smallest first
+      for (int s = 0; s < SL; s++) {
+        // every pair of planes whose product is above 2^-8(NP) of the leading one, smallest first
 #pragma unroll
-      for (int t = NP - 1; t >= 0; t--) {
+        for (int t = NP - 1; t >= 0; t--) {
 #pragma unroll
-        for (int p = 0; p <= t; p++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s][p], bv[s][t - p], acc, 0, 0, 0);
+          for (int p = 0; p <= t; p++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s][p], bv[s][t - p], acc, 0, 0, 0);
+        }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   const int nsteps = K > kbeg ? (K - kbeg + BK - 1) / BK : 0;
@@ -366,11 +411,11 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
       fetch_a(0, ra0);
       fetch_a(BK, ra1);
       fetch_a(2 * BK, ra2);
-      stage_a(ra0, 0);
+      stage_a(ra0, 0, 0);
       fetch_a(3 * BK, ra0);
       __syncthreads();
       auto step = [&](int i, ARegs &ran) __attribute__((always_inline)) {
-        stage_a(ran, (i + 1) & 1);
+        stage_a(ran, (i + 1) * BK, (i + 1) & 1);
         fetch_a((i + 1 + NSET) * BK, ran);
         __syncthreads();
       };
@@ -387,11 +432,11 @@ __global__ __launch_bounds__(768) void k_gemm_split(GemmArgs a) {
       fetch_b(0, rb0);
       fetch_b(BK, rb1);
       fetch_b(2 * BK, rb2);
-      stage_b(rb0, 0);
+      stage_b(rb0, 0, 0);
       fetch_b(3 * BK, rb0);
       __syncthreads();
       auto step = [&](int i, BRegs<BMODE> &rbn) __attribute__((always_inline)) {
-        stage_b(rbn, (i + 1) & 1);
+        stage_b(rbn, (i + 1) * BK, (i + 1) & 1);
         fetch_b((i + 1 + NSET) * BK, rbn);
         __syncthreads();
       };
@@ -531,7 +576,7 @@ __global__ __launch_bounds__(256 + 64 * NPW) void k_gemm_qpc(GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < NA; i++) {
       const int row = m0 + ar + (PT / 16) * i, k = kbeg + k0 + 4 * akq;
-      ra.v[i] = load4<true>(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
+      ra.v[i] = load4_vec(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
     }
     const int k = kbeg + k0 + 16 * wkc;
 #pragma unroll
@@ -725,7 +770,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs a) {
 
   auto load_a = [&](int u, int k0) {  // unit u: row u / 8, k = 4 (u % 8) .. +3
     const int row = m0 + (u >> 3), k = kbeg + k0 + 4 * (u & 7);
-    return load4<AL>(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
+    return AL ? load4_vec(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0) : load4(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
   };
   auto fetch = [&](int k0, FRegsA &ra, FRegsB &rb) {
     ra.v0 = load_a(tid, k0);
@@ -891,7 +936,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs a) {
 // offsets computed once -- no address arithmetic, bounds tests or selects on the vector unit, which the staging
 // wavefronts share with the multiplying one of their SIMD.  B is (K,N) row-major here; packed weights (N,K) keep
 // k_gemm_f32, which measured faster on the prompt shapes.
-template <bool AL, bool FULL>
+template <int LD, bool FULL>
 __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
   constexpr int BM = 64, BN = 64, BK = 32, NP = BK / 2;
   // plane pitches in floats: a multiple of 4 where the staging writes are 16 bytes (B), else 8-byte aligned
@@ -971,16 +1016,21 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const int u = t + 256 * h, row = m0 + (u >> 3), k = kbeg + k0 + 4 * (u & 7);
-          const float4 v = load4<AL>(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
+          const float4 v = LD == LD_ANY   ? load4_in(a.A + (int64_t)m0 * ldk, min(u >> 3, M - 1 - m0) * ldk + min(k, ldk - 4))
+                           : LD == LD_VEC ? load4_vec(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0)
+                                          : load4(a.A + (int64_t)row * ldk + k, row < M ? clamp04(K - k) : 0);
           if (h == 0) ra.v0 = v;
           else ra.v1 = v;
         }
       };
-      auto stage = [&](const FRegsA &ra, int buf) __attribute__((always_inline)) {
+      auto stage = [&](const FRegsA &ra, int k0, int buf) __attribute__((always_inline)) {
+        const bool edge = LD == LD_ANY && kbeg + k0 + BK > ldk && kbeg + k0 < ldk;  // uniform (a step past the end is not multiplied)
+        const int by = kbeg + k0 + 4 * (t & 7) - min(kbeg + k0 + 4 * (t & 7), ldk - 4);
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const int u = t + 256 * h, row = u >> 3, g = u & 7;
-          const float4 v = h == 0 ? ra.v0 : ra.v1;
+          float4 v = h == 0 ? ra.v0 : ra.v1;
+          if (edge) v = shift4<LD>(v, by);
           float *p = (float *)(smem + buf * kABuf) + 2 * g * PA + 2 * row;
           *(float2 *)p = make_float2(v.x, v.z);         // k = 4g, 4g + 2
           *(float2 *)(p + PA) = make_float2(v.y, v.w);  // k = 4g + 1, 4g + 3
@@ -990,14 +1040,14 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
       fetch(0, r0);
       fetch(BK, r1);
       fetch(2 * BK, r2);
-      stage(r0, 0);
+      stage(r0, 0, 0);
       fetch(3 * BK, r0);
-      stage(r1, 1);
+      stage(r1, BK, 1);
       fetch(4 * BK, r1);
       __syncthreads();
       // step i stages step i + 2 (register set and buffer (i + 2) % 3) and requests step i + 5
       auto step = [&](int i, FRegsA &rs, int buf) __attribute__((always_inline)) {
-        stage(rs, buf);
+        stage(rs, (i + 2) * BK, buf);
         fetch((i + 5) * BK, rs);
         __syncthreads();
       };
@@ -1023,12 +1073,27 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
         // thread (g, h, nq): rows k = 4g + h and 4g + 2 + h of the step, columns 4 nq .. + 3
         const int g = t >> 5, h = (t >> 4) & 1, n = n0 + 4 * (t & 15);
         const int k1 = kbeg + k0 + 4 * g + h, k2 = k1 + 2;
-        const float4 v1 = load4<AL>(a.B + (int64_t)k1 * N + n, k1 < K ? clamp04(N - n) : 0);
-        const float4 v2 = load4<AL>(a.B + (int64_t)k2 * N + n, k2 < K ? clamp04(N - n) : 0);
+        const int kb = min(kbeg + k0, ldk - 1);
+        auto row = [&](int k) __attribute__((always_inline)) {
+          return LD == LD_ANY   ? load4_in(a.B + (int64_t)kb * N, min(k - (kbeg + k0), ldk - 1 - kb) * N + min(n, N - 4))
+                 : LD == LD_VEC ? load4_vec(a.B + (int64_t)k * N + n, k < K ? clamp04(N - n) : 0)
+                                : load4(a.B + (int64_t)k * N + n, k < K ? clamp04(N - n) : 0);
+        };
+        const float4 v1 = row(k1), v2 = row(k2);
         rb.r0 = make_uint4(__float_as_uint(v1.x), __float_as_uint(v1.y), __float_as_uint(v1.z), __float_as_uint(v1.w));
         rb.r1 = make_uint4(__float_as_uint(v2.x), __float_as_uint(v2.y), __float_as_uint(v2.z), __float_as_uint(v2.w));
       };
-      auto stage = [&](const FRegsB &rb, int buf) __attribute__((always_inline)) {
+      auto stage = [&](const FRegsB &rbi, int k0, int buf) __attribute__((always_inline)) {
+        FRegsB rb = rbi;
+        if (LD == LD_ANY && (n0 + BN > N || kbeg + k0 + BK > ldk) && kbeg + k0 < ldk) {  // uniform: columns into their place, zeros behind K
+          const int n = n0 + 4 * (t & 15), by = n - min(n, N - 4), k1 = kbeg + k0 + 4 * (t >> 5) + ((t >> 4) & 1);
+          auto fix = [&](uint4 q, int k) __attribute__((always_inline)) {
+            const float4 v = shift4<LD>(make_float4(__uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z), __uint_as_float(q.w)), k < ldk ? by : 4);
+            return make_uint4(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w));
+          };
+          rb.r0 = fix(rb.r0, k1);
+          rb.r1 = fix(rb.r1, k1 + 2);
+        }
         float *p = (float *)(smem + kABytes + buf * kBBuf) + (t >> 4) * PB + 2 * 4 * (t & 15);  // plane 2g + h = t / 16
         *(uint4 *)p = make_uint4(rb.r0.x, rb.r1.x, rb.r0.y, rb.r1.y);
         *(uint4 *)(p + 4) = make_uint4(rb.r0.z, rb.r1.z, rb.r0.w, rb.r1.w);
@@ -1037,13 +1102,13 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
       fetch(0, r0);
       fetch(BK, r1);
       fetch(2 * BK, r2);
-      stage(r0, 0);
+      stage(r0, 0, 0);
       fetch(3 * BK, r0);
-      stage(r1, 1);
+      stage(r1, BK, 1);
       fetch(4 * BK, r1);
       __syncthreads();
       auto step = [&](int i, FRegsB &rs, int buf) __attribute__((always_inline)) {
-        stage(rs, buf);
+        stage(rs, (i + 2) * BK, buf);
         fetch((i + 5) * BK, rs);
         __syncthreads();
       };
@@ -1189,15 +1254,20 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
       }
     }
   }
+  // how the tiles of k_gemm_split and k_gemm_f32pc read their operands: see LD_VEC
+  const int ld = a.K < 4 || a.K > 1 << 24 || (bmode == B_ROWMAJOR && (a.N < 4 || a.N > 1 << 24)) ? LD_ELEM
+                 : a.K % 4 == 0 && (bmode != B_ROWMAJOR || a.N % 4 == 0) ? LD_VEC
+                                                                               : LD_ANY;
   if (precision == GEMM_FP32) {
     // aligned: every 4 (8 for packed weights) consecutive operand elements a thread asks for are one aligned vector
     const bool al = bmode == B_ROWMAJOR ? (a.K % 4 == 0 && a.N % 4 == 0) : (a.K % 8 == 0);
     if (bmode == B_ROWMAJOR) {
       const bool full = al && a.M % 64 == 0 && a.N % 64 == 0 && a.K % 32 == 0 && a.kper % 32 == 0 && (int64_t)a.M * a.K * 4 < (1ll << 32) &&
                         ((int64_t)64 * a.N + a.N) * 4 < (1ll << 32);
-      if (full) hipLaunchKernelGGL((k_gemm_f32pc<true, true>), grid, dim3(768), 0, st, a);
-      else if (al) hipLaunchKernelGGL((k_gemm_f32pc<true, false>), grid, dim3(768), 0, st, a);
-      else hipLaunchKernelGGL((k_gemm_f32pc<false, false>), grid, dim3(768), 0, st, a);
+      if (full) hipLaunchKernelGGL((k_gemm_f32pc<LD_VEC, true>), grid, dim3(768), 0, st, a);
+      else if (ld == LD_VEC) hipLaunchKernelGGL((k_gemm_f32pc<LD_VEC, false>), grid, dim3(768), 0, st, a);
+      else if (ld == LD_ANY) hipLaunchKernelGGL((k_gemm_f32pc<LD_ANY, false>), grid, dim3(768), 0, st, a);
+      else hipLaunchKernelGGL((k_gemm_f32pc<LD_ELEM, false>), grid, dim3(768), 0, st, a);
     } else {
       if (al) hipLaunchKernelGGL((k_gemm_f32<true>), grid, block, 0, st, a);
       else hipLaunchKernelGGL((k_gemm_f32<false>), grid, block, 0, st, a);
@@ -1222,28 +1292,20 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
 #undef QSEL
 #undef QG
   } else {
-    int wm = W_ROWMAJOR;
-    if (bmode == B_WMAT) wm = a.wtype == CTHIP_F16 ? W_F16 : W_F32;
-#define SPLIT3(MODE, AL)                                                                                      \
-  if (precision == GEMM_BF16X6) hipLaunchKernelGGL((k_gemm_split<MODE, 6, AL>), grid, dim3(768), 0, st, a);      \
-  else if (precision == GEMM_BF16X3) hipLaunchKernelGGL((k_gemm_split<MODE, 3, AL>), grid, dim3(768), 0, st, a); \
-  else hipLaunchKernelGGL((k_gemm_split<MODE, 1, AL>), grid, dim3(768), 0, st, a)
-#define SPLIT(MODE)      \
-  case MODE:             \
-    if (al) {            \
-      SPLIT3(MODE, true); \
-    } else {             \
-      SPLIT3(MODE, false); \
-    }                    \
-    break
-    // aligned: every 4 consecutive floats a thread asks for are one 16-byte vector, inside or outside as a whole
-    const bool al = a.K % 4 == 0 && (bmode != B_ROWMAJOR || a.N % 4 == 0);
-    switch (wm) {
-      SPLIT(W_ROWMAJOR);
-      SPLIT(W_F32);
-      SPLIT(W_F16);
+#define SPLIT(MODE, LD)                                                                                       \
+  if (precision == GEMM_BF16X6) hipLaunchKernelGGL((k_gemm_split<MODE, 6, LD>), grid, dim3(768), 0, st, a);      \
+  else if (precision == GEMM_BF16X3) hipLaunchKernelGGL((k_gemm_split<MODE, 3, LD>), grid, dim3(768), 0, st, a); \
+  else hipLaunchKernelGGL((k_gemm_split<MODE, 1, LD>), grid, dim3(768), 0, st, a)
+    // (packed rows are whole chunks of 16 here)
+    if (bmode == B_WMAT) {
+      if (a.wtype == CTHIP_F16 && ld == LD_VEC) { SPLIT(W_F16, LD_VEC); }
+      else if (a.wtype == CTHIP_F16) { SPLIT(W_F16, LD_ELEM); }
+      else if (ld == LD_VEC) { SPLIT(W_F32, LD_VEC); }
+      else { SPLIT(W_F32, LD_ELEM); }
     }
-#undef SPLIT3
+    else if (ld == LD_VEC) { SPLIT(W_ROWMAJOR, LD_VEC); }
+    else if (ld == LD_ANY) { SPLIT(W_ROWMAJOR, LD_ANY); }
+    else { SPLIT(W_ROWMAJOR, LD_ELEM); }
 #undef SPLIT
   }
   hipError_t le = hipGetLastError();

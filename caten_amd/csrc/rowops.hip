@@ -341,8 +341,6 @@ int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, in
   return 0;
 }
 
-typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
-
 // Rows of 4 .. 2048 floats that are short or that k_rowop cannot read: LPR lanes hold a row, VPL chunks of four floats each, at any alignment (the loads
 // are 16 bytes at 4-byte alignment).  Chunk c starts at min(4c, n - 4): the last one of a row that is no multiple of four
 // overlaps its neighbour, whose share it leaves out of the sums and stores a second time with the same values.
