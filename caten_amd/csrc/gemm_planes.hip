@@ -520,20 +520,6 @@ int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N,
   const int rf = cthip_free(pa);  // stream-ordered: handed out again only to later work on this stream
   return rc ? rc : rf;
 }
-// What the same product takes with its operands converted per 64 x 64 tile (launch_gemm): per round of tiles over an XCD 1.4 / 1.5 / 3 us and
-// 5.5 / 8.2 / 13.8 us per 1000 k at one / two / three terms, 7.9 / 10 / 15.3 where rows are not whole 16-byte pieces; short grids
-// split over K.  Within 15 % of the measured times from 500^3 to 4096^3 (but 25 % under those of an unaligned product of one round).
-static double tiles64_us(int M, int N, int K, int terms, bool aligned) {
-  const int tm = (M + 63) / 64, tn = (N + 63) / 64;
-  const int64_t tiles = (int64_t)tm * tn, cus = state().compute_units;
-  int64_t ks = (tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles, most = tiles;
-  ks = ks < K / 192 ? ks : K / 192;
-  ks = ks < 1 ? 1 : ks > 16 ? 16 : ks;
-  for (int rx = 1; rx <= 8; rx *= 2) most = std::min(most, (int64_t)((tm + rx - 1) / rx) * ((tn + 8 / rx - 1) / (8 / rx)));  // of an XCD
-  const double c = terms == 3 ? (aligned ? 13.8 : 15.3) : terms == 2 ? (aligned ? 8.2 : 10.0) : (aligned ? 5.5 : 7.9), start = terms == 3 ? 3.0 : terms == 2 ? 1.5 : 1.4;
-  const double full = (double)(most * ks) * 8.0 / cus, rounds = full <= 4.0 ? ceil(full) : 0.5 * ceil(2.0 * full);
-  return 2.0 + (ks > 1 ? 5.0 : 0.0) + rounds * (start + c * K / ks * 1e-3);
-}
 // Measured from 1000^3 to 2300^3, from (4096, 4096, 128) to (2500, 600, 4000), at one to three terms, rows of whole 16-byte pieces or not: at such sizes, which the
 // caches hold, planes_us is off by what is put right here, and the rule misses the better one by at most 12 % in 86 of 87.
 bool matmul_planes_pay(int M, int N, int K, int precision) {
@@ -541,7 +527,7 @@ bool matmul_planes_pay(int M, int N, int K, int precision) {
   const int terms = plane_terms(precision);
   const bool aligned = K % 4 == 0 && N % 4 == 0;
   const double us = planes_us(M, N, K, terms, terms, false, ((double)M + N) * K * (4 + 2 * terms)), out = 4e-6 * M * N;
-  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tiles64_us(M, N, K, terms, aligned);
+  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, false, aligned, false).us;
 }
 
 // ---- Linears over many rows ----
@@ -647,19 +633,6 @@ void weight_planes_limit(int64_t bytes) {
   if (over) weight_planes_drop();
 }
 
-// What launch_gemm takes: 64 x 128 tiles of a quantised matrix, one workgroup per compute unit.
-static double linear_tiles_us(const WMat *w, int m, int terms) {
-  const int N = (int)w->rows, K = (int)w->cols;
-  const int64_t cus = state().compute_units;
-  // (fp16 weights: half the bytes, which shows in a few rounds)
-  if (!is_quant(w)) return tiles64_us(m, N, K, terms, true) * (w->type == CTHIP_F16 && (int64_t)((m + 63) / 64) * ((N + 63) / 64) <= 4 * cus ? 0.92 : 1.0);
-  const int64_t tiles = (int64_t)((m + 63) / 64) * ((N + 127) / 128);
-  int64_t ks = cus / tiles;
-  ks = ks < K / 192 ? ks : K / 192;
-  ks = ks < 1 ? 1 : ks > 16 ? 16 : ks;
-  const double c = terms == 2 ? 13.2 : 10.0;
-  return 2.0 + (ks > 1 ? 5.0 : 0.0) + (double)((tiles * ks + cus - 1) / cus) * (1.0 + c * K / ks * 1e-3);
-}
 bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   if (precision == GEMM_FP32 || m < 64 || w->rows < 64 || w->cols < 64 || (!is_quant(w) && w->cols % 16)) return false;
   // (three terms against integers: registers for one 32-column block less per wavefront, no faster than the tiles)
@@ -668,7 +641,10 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   double bytes = 0.0;
   if (!weight_planes_kept(w, terms_b)) bytes = (double)w->q_bytes + weight_plane_bytes(w, terms_b);
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
-  return planes_us(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes) * 1.04 < linear_tiles_us(w, m, terms);
+  // (fp16 weights: half the bytes, which shows in a few rounds of tiles)
+  const bool few_half = w->type == CTHIP_F16 && (int64_t)((m + 63) / 64) * ((w->rows + 63) / 64) <= 4 * state().compute_units;
+  return planes_us(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes) * 1.04 <
+         tile_plan(m, (int)w->rows, (int)w->cols, precision, is_quant(w), true, false).us * (few_half ? 0.92 : 1.0);
 }
 // ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {

@@ -11,6 +11,9 @@
 // eight staging wavefronts.  Finished tiles leave through LDS as whole rows (store_tile).
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "common.h"
 
 namespace cthip {
@@ -1184,6 +1187,38 @@ int matmul_scratch_init(int device) {
   return 0;
 }
 
+// How many workgroups share the reduction axis of a tile, and what the launch (with the one that adds the shares up) then takes, in microseconds:
+// per round of tiles over an XCD a start and a time per step of 64, plus, where shares are added, a launch and their bytes (`deferred`: the bytes; the
+// next launch adds them on its way).  Fitted to 1 .. 8 shares of 20 shapes from (20, 232, 144) to (512, 2048, 5632), to which it keeps
+// within 15 %.  Two workgroups per compute unit of a tile, which filled the chip and was the rule before, took for 700^3 at two terms 14.0 us
+// (one share: 9.8), 512^3 9.3 (8.2), 400 x 2304 x 768 Q8_0 24 (14: shares that an XCD has no room for), 70 x 1280 x 5120 23 (15).
+TilePlan tile_plan(int M, int N, int K, int precision, bool quant, bool aligned, bool deferred) {
+  struct Cost {
+    double start, step, unaligned;            // one round
+    double start_n, step_n, unaligned_n;      // several: every compute unit at work
+  };
+  static const Cost costs[7] = {{1.0, 1.22, 1.55, 1.0, 1.30, 1.60}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64},
+                                {1.6, 0.85, 1.10, 3.0, 0.88, 0.98}, {2.0, 0.55, 0.55, 2.0, 0.66, 0.66}, {2.0, 0.72, 0.72, 2.0, 0.87, 0.87},
+                                {2.0, 0.90, 0.90, 2.0, 1.10, 1.10}};  // k_gemm_f32pc; k_gemm_split, one .. three terms; k_gemm_qpc, one .. three
+  const Cost &c = costs[precision == GEMM_FP32 ? 0 : (quant ? 3 : 0) + (precision == GEMM_BF16 ? 1 : precision == GEMM_BF16X3 ? 2 : 3)];
+  const bool two = !quant && (precision == GEMM_BF16 || precision == GEMM_BF16X3);  // workgroups on a compute unit
+  const int tm = (M + 63) / 64, tn = (N + (quant ? 127 : 63)) / (quant ? 128 : 64), nsteps = (K + 63) / 64;
+  int64_t most = (int64_t)tm * tn;  // tiles of an XCD
+  for (int rx = 1; rx <= 8; rx *= 2) most = std::min(most, (int64_t)((tm + rx - 1) / rx) * ((tn + 8 / rx - 1) / (8 / rx)));
+  TilePlan best = {1, 1e30};
+  for (int ks = 1; ks <= 16 && ks <= std::max(nsteps, 1); ks++) {
+    const int steps = (nsteps + ks - 1) / ks, shares = steps ? (nsteps + steps - 1) / steps : 1;
+    if (shares < ks) continue;  // the same steps as with fewer
+    const double n = (double)(most * shares) * 8.0 / state().compute_units;
+    const double rounds = n <= 1.0 ? 1.0 : n <= 2.0 && two ? 1.85 : n <= 4.0 ? ceil(n) : 0.5 * ceil(2.0 * n);
+    const double tile = n <= 1.0 ? c.start + (aligned ? c.step : c.unaligned) * steps : c.start_n + (aligned ? c.step_n : c.unaligned_n) * steps;
+    const double sum = shares > 1 ? (deferred ? 0.3 : 2.6) + (deferred ? 0.6e-6 : 0.85e-6) * 4.0 * shares * M * N : 0.0;
+    const double us = 2.0 + rounds * tile + sum;
+    if (us < best.us) best = {ks, us};
+  }
+  return best;
+}
+
 // static_ws: null = split-K partials come from the caching allocator; otherwise they go to this buffer of
 // static_ws_bytes bytes and nothing is allocated or freed
 int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t static_ws_bytes, GemmDeferred *defer) {
@@ -1221,18 +1256,22 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
       }
     }
     grid.x = 8u * (unsigned)a.rm * (unsigned)a.rn;
-    // too few tiles to occupy the chip and a long reduction axis: split K over several workgroups per tile
+    // too few tiles to occupy the chip and a long reduction axis: split K over several workgroups per tile.  (Paired tiles are stored by the
+    // workgroup that computed them.)
     const int nsteps = (a.K + 63) / 64;  // K-steps of 64 (two of the fp32 kernel's)
-    // workgroups aimed at: two per compute unit where the tiles fill less than half the chip (GPT-2 / Llama
-    // prefill 1.47 / 3.29 -> 1.44 / 3.18 ms against 1.5; three per unit: 1.55 / 3.18), else 1.5 (a 1024^3
-    // product, one tile per unit, loses 10-30 % when it is split in two)
-    // (the 512-thread workgroups of k_gemm_qpc sit one to a compute unit: aim at one each)
-    int ks = quant ? (int)(cus / tiles) : (int)((tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles);
-    if (ks > nsteps / 3) ks = nsteps / 3;
-    if (ks > 16) ks = 16;
-    if (a.pairs) ks = 1;  // paired tiles are stored by the workgroup that computed them
-    // routed ones go through the reduction where it shortens every workgroup's chain by more than its launch takes (500 k: 6 us)
-    if (a.routed && ks > 1 && a.K - a.K / ks < 500) ks = 1;
+    const bool aligned = a.K % 4 == 0 && (bmode == B_WMAT || a.N % 4 == 0);
+    int ks = a.pairs ? 1 : tile_plan(a.M, a.N, a.K, precision, quant, aligned, defer && !static_ws && a.act == CTHIP_ACT_NONE).ks;
+    if (static_ws) {
+      // what does not fit split two ways per compute unit is refused, what fits is split as often as it does
+      int fill = (int)((tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles);
+      fill = std::min(std::min(fill, nsteps / 3), 16);
+      const int share = fill > 1 ? (nsteps + fill - 1) / fill : nsteps, most = share > 0 ? (nsteps + share - 1) / share : 1;
+      const size_t tile_bytes = sizeof(float) * (size_t)a.M * a.N;
+      if (most > 1 && most * tile_bytes > static_ws_bytes)
+        return fail(CTHIP_E_UNSUPPORTED, "cthip_matmul_noalloc: (%d,%d,%d) splits its reduction %d ways and needs %zu bytes of partial "
+                    "tiles; the static scratch holds %zu (use cthip_matmul)", a.M, a.N, a.K, most, most * tile_bytes, static_ws_bytes);
+      ks = std::min(ks, (int)(static_ws_bytes / tile_bytes));
+    }
     if (ks > 1) {
       const int steps_per = (nsteps + ks - 1) / ks;
       a.kper = steps_per * 64;
@@ -1240,9 +1279,6 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
       if (a.ksplit > 1) {
         const size_t need = sizeof(float) * (size_t)a.ksplit * a.M * a.N;
         if (static_ws) {
-          if (need > static_ws_bytes)
-            return fail(CTHIP_E_UNSUPPORTED, "cthip_matmul_noalloc: (%d,%d,%d) splits its reduction %d ways and needs %zu bytes of partial "
-                        "tiles; the static scratch holds %zu (use cthip_matmul)", a.M, a.N, a.K, a.ksplit, need, static_ws_bytes);
           a.ws = static_ws;  // every element of every share is written before the reduction reads it
         } else {
           int rc = alloc_scratch((void **)&a.ws, need);
