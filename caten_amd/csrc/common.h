@@ -290,6 +290,8 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in);
 // x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
 // Linear over 8 .. 64 rows that lie as operands of two terms (linear_few.hip)
 bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: there is a pass over the rows in front of it anyway
+bool linear_few_shares_pays(const WMat *w, int m, int precision);
+int launch_linear_few_shares(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual, GemmDeferred *defer);
 int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route);
 bool linear_planes_ready(const WMat *w, int m, int precision);
 void weight_planes_release(const WMat *w);

@@ -1006,6 +1006,8 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         if (taken) return r;
         if (in_terms || out_terms) return fail(CTHIP_E_STATE, "prompt: a Linear of %lld x %lld over %d rows cannot take its input as terms", (long long)w->rows, (long long)w->cols, R);
       }
+      if (defer && act == CTHIP_ACT_NONE && !route && linear_few_shares_pays(w, R, prec) && !linear_rows_pays(w, in, w->cols, R, prec, nullptr, nullptr))
+        return launch_linear_few_shares(y, w, in, R, bias, residual, defer);
       return prompt_linear(y, w, in, R, bias, residual, act, prec, defer, route);
     };
     // Xr += W.in + bias, then XN = norm(Xr) with (g, b), as terms or not; g == nullptr: no norm follows (after the last layer)

@@ -10,6 +10,8 @@
 // L2 (all rows and its columns: 220 KB there).
 // Products as in the tiles: the integers of a quantised weight are exact in bf16, their block's scale is applied to the block's
 // sum; an fp16 weight is two terms, and the product of both lower terms is left out.  Error against 64 bits the same (2.5e-6, fp16 3.7e-6).
+#include <algorithm>
+
 #include "common.h"
 #include "planes.h"
 
@@ -21,6 +23,8 @@ struct FewArgs {
   const unsigned short *wd;  // scales, nkb a row
   int wpitch;
   int nkb;                   // blocks of 32 k
+  const float *X;            // the rows as they are (X32)
+  float *ws;                 // several shares of K (gridDim.y): their sums, [share][row][column]
   PlaneGemmArgs e;           // M, N and what happens to the result
 };
 
@@ -28,15 +32,21 @@ enum { FW_Q8 = 0, FW_Q4 = 1, FW_F16 = 2 };
 typedef float v4f_few __attribute__((ext_vector_type(4)));
 constexpr int kFewWaves = 8;
 
-template <int SRC, int MB, int NB, int BATCH>
+template <int SRC, int MB, int NB, int BATCH, bool X32>
 __global__ __launch_bounds__(64 * kFewWaves, MB * NB <= 2 && BATCH <= 5 ? 4 : 2) void k_linear_few(FewArgs a) {
   constexpr int NPB = SRC == FW_F16 ? 2 : 1, ROWS = 16 * MB, COLS = 16 * NB;
   extern __shared__ __align__(16) float red[];  // [wavefront][row][column]
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, col = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * COLS, M = a.e.M, N = a.e.N;
-  const int per = (a.nkb + kFewWaves - 1) / kFewWaves, kb0 = wv * per, kb1 = min(a.nkb, kb0 + per);
+  const int share = (a.nkb + gridDim.y - 1) / gridDim.y, s0 = blockIdx.y * share, s1 = min(a.nkb, s0 + share);
+  const int per = (share + kFewWaves - 1) / kFewWaves, kb0 = s0 + wv * per, kb1 = min(s1, kb0 + per);
   const unsigned char *ap = a.A + lane * 16;
+  const float *xp[MB];
+  if constexpr (X32) {
+#pragma unroll
+    for (int i = 0; i < MB; i++) xp[i] = a.X + (int64_t)min(16 * i + col, M - 1) * (32 * a.nkb) + 8 * g;  // rows past the end repeat the last one
+  }
   const unsigned char *wp[NB];
   const unsigned short *dp[NB];
   v4f_few acc[MB][NB];
@@ -53,7 +63,7 @@ __global__ __launch_bounds__(64 * kFewWaves, MB * NB <= 2 && BATCH <= 5 ? 4 : 2)
     // every request of the batch, none behind a branch: blocks past the share repeat its last one and are not multiplied
     uint4 w[BATCH][NB];
     unsigned d[BATCH][NB];
-    v8bf af[BATCH][MB][2];
+    uint4 af[BATCH][MB][2];  // two terms of 8 k, or 8 floats
 #pragma unroll
     for (int b = 0; b < BATCH; b++) {
       const int kb = min(b0 + b, kb1 - 1);
@@ -70,12 +80,23 @@ __global__ __launch_bounds__(64 * kFewWaves, MB * NB <= 2 && BATCH <= 5 ? 4 : 2)
 #pragma unroll
       for (int q = 0; q < 2; q++)
 #pragma unroll
-        for (int i = 0; i < MB; i++) af[b][i][q] = __builtin_bit_cast(v8bf, *(const uint4 *)(ap + ((kb * 2 + q) * MB + i) * 1024));
+        for (int i = 0; i < MB; i++) af[b][i][q] = X32 ? *(const uint4 *)(xp[i] + kb * 32 + 4 * q) : *(const uint4 *)(ap + ((kb * 2 + q) * MB + i) * 1024);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < BATCH; b++) {
       if (b0 + b >= kb1) break;  // (uniform)
+      v8bf at[MB][2];
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        uint4 pl[2] = {af[b][i][0], af[b][i][1]};
+        if constexpr (X32) {
+          const float4 lo = __builtin_bit_cast(float4, pl[0]), hi = __builtin_bit_cast(float4, pl[1]);
+          const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+          split8_planes<2>(x, pl);
+        }
+        at[i][0] = __builtin_bit_cast(v8bf, pl[0]), at[i][1] = __builtin_bit_cast(v8bf, pl[1]);
+      }
 #pragma unroll
       for (int j = 0; j < NB; j++) {
         v8bf bf[NPB];
@@ -99,13 +120,13 @@ __global__ __launch_bounds__(64 * kFewWaves, MB * NB <= 2 && BATCH <= 5 ? 4 : 2)
 #pragma unroll
         for (int i = 0; i < MB; i++) {
           if constexpr (SRC == FW_F16) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][1], bf[0], acc[i][j], 0, 0, 0);  // smallest products first
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][0], bf[NPB - 1], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][0], bf[0], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][1], bf[0], acc[i][j], 0, 0, 0);  // smallest products first
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][0], bf[NPB - 1], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][0], bf[0], acc[i][j], 0, 0, 0);
           } else {
             v4f_few t = {0.0f, 0.0f, 0.0f, 0.0f};
-            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][1], bf[0], t, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b][i][0], bf[0], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][1], bf[0], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[i][0], bf[0], t, 0, 0, 0);
             const float dd = half_bits_to_float((unsigned short)d[b][j]);
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(dd, t[r], acc[i][j][r]);
@@ -128,7 +149,11 @@ __global__ __launch_bounds__(64 * kFewWaves, MB * NB <= 2 && BATCH <= 5 ? 4 : 2)
     for (int w = 0; w < kFewWaves; w++) t[w] = *(const float4 *)(red + (w * ROWS + m) * COLS + c);
 #pragma unroll
     for (int w = 0; w < kFewWaves; w++) v.x += t[w].x, v.y += t[w].y, v.z += t[w].z, v.w += t[w].w;
-    plane_gemm_store(a.e, m, n0 + c, v);
+    if (a.ws) {
+      if (n0 + c < N) *(float4 *)(a.ws + ((int64_t)blockIdx.y * M + m) * N + n0 + c) = v;
+    } else {
+      plane_gemm_store(a.e, m, n0 + c, v);
+    }
   }
 }
 
@@ -151,25 +176,34 @@ static int few_launch(const FewArgs &a) {
   constexpr size_t lds = (size_t)kFewWaves * 16 * MB * 16 * NB * 4;
   const int per = (a.nkb + kFewWaves - 1) / kFewWaves;  // blocks of a wavefront: in one batch where registers hold them
   if constexpr (NB == 3) {
-    if (lds > 64 * 1024) CTHIP_CHECK(hipFuncSetAttribute((const void *)k_linear_few<SRC, MB, 3, (MB <= 2 ? 4 : 2)>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_linear_few<SRC, MB, 3, (MB <= 2 ? 4 : 2)>), grid, block, lds, state().stream, a);
+    if (lds > 64 * 1024) CTHIP_CHECK(hipFuncSetAttribute((const void *)k_linear_few<SRC, MB, 3, (MB <= 2 ? 4 : 2), false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_linear_few<SRC, MB, 3, (MB <= 2 ? 4 : 2), false>), grid, block, lds, state().stream, a);
     CTHIP_LAUNCH_CHECK();
     return 0;
   }
   constexpr int kLong = MB <= 2 ? 8 : 4;
-  if (per <= 4) hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, 4>), grid, block, lds, state().stream, a);
-  else if (per == 5) hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, 5>), grid, block, lds, state().stream, a);
-  else hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, kLong>), grid, block, lds, state().stream, a);
+  if (per <= 4) hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, 4, false>), grid, block, lds, state().stream, a);
+  else if (per == 5) hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, 5, false>), grid, block, lds, state().stream, a);
+  else hipLaunchKernelGGL((k_linear_few<SRC, MB, NB, kLong, false>), grid, block, lds, state().stream, a);
   CTHIP_LAUNCH_CHECK();
   return 0;
 }
 
-// y (m, rows) = act(x W^T + bias) + residual; act may be kActSwigluPairs, route as for launch_linear_gemm.
-// Call only where linear_few_pays; y, bias and residual on 16 bytes.
-int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route) {
+template <int SRC, int MB>
+static int few_launch32(const FewArgs &a, int shares) {
+  const dim3 grid((unsigned)((a.e.N + 15) / 16), (unsigned)shares), block(64 * kFewWaves);
+  constexpr size_t lds = (size_t)kFewWaves * 16 * MB * 16 * 4;
+  const int share = (a.nkb + shares - 1) / shares, per = (share + kFewWaves - 1) / kFewWaves;
+  if (per <= 2) hipLaunchKernelGGL((k_linear_few<SRC, MB, 1, 2, true>), grid, block, lds, state().stream, a);
+  else if (per <= 4) hipLaunchKernelGGL((k_linear_few<SRC, MB, 1, 4, true>), grid, block, lds, state().stream, a);
+  else hipLaunchKernelGGL((k_linear_few<SRC, MB, 1, 6, true>), grid, block, lds, state().stream, a);
+  CTHIP_LAUNCH_CHECK();
+  return 0;
+}
+
+static FewArgs few_args(float *y, const WMat *w, int m, const float *bias, const float *residual, int act) {
   FewArgs a = {};
   a.nkb = (int)(w->cols / 32);
-  a.A = (const unsigned char *)operands;
   a.W = (const unsigned char *)w->q;
   a.wd = (const unsigned short *)w->d;
   a.wpitch = (int)(w->type == CTHIP_Q8_0 ? w->cols : w->type == CTHIP_Q4_0 ? w->cols / 2 : 2 * w->cols);
@@ -177,6 +211,46 @@ int launch_linear_few(float *y, const WMat *w, const void *operands, int m, cons
   a.e.M = m, a.e.N = (int)w->rows;
   a.e.bias = bias, a.e.residual = residual;
   a.e.act = act;
+  return a;
+}
+
+// The Linears in front of a norm of a short prompt (projection, second of the MLP), which adds shares of K up on its way: rows as they are, which every
+// workgroup splits into their two terms (as many bytes either way), shares to fill the chip once, twice as many where a wavefront
+// would have more than four blocks.  A prompt of gpt2 q8_0, 9 / 14 rows 543 / 550 -> 486 / 493 us, q4_0 28 rows 630 -> 605, gpt2-medium q8_0 22 rows 1125 -> 1067,
+// gpt2-large f16 12 rows 1664 -> 1560, llama-1.1b f16 9 rows 1472 -> 1384; more rows are as fast in tiles (gpt2-medium 37: 1220, 1224; llama-1.1b f16 17:
+// 1496, 1517) or faster (gpt2-large 52 rows 2116, 2277 this way), and
+// so are 4096 output columns (llama-7b 12 rows 3960, 4199).
+bool linear_few_shares_pays(const WMat *w, int m, int precision) {
+  if (precision != GEMM_BF16X3 || m < 8 || w->cols % 32 || w->rows % 4 || w->rows > 8ll * state().compute_units) return false;
+  if (w->type != CTHIP_Q8_0 && w->type != CTHIP_Q4_0 && w->type != CTHIP_F16) return false;
+  return m <= 16 || (m <= 32 && w->rows <= 1024);
+}
+// y (m, rows) = x W^T + bias + residual, or defer's shares of x W^T (to be added up and freed by the caller); all on 16 bytes
+int launch_linear_few_shares(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual, GemmDeferred *defer) {
+  FewArgs a = few_args(y, w, m, bias, residual, CTHIP_ACT_NONE);
+  a.X = x;
+  int shares = std::max(1, std::min(state().compute_units / ((a.e.N + 15) / 16), a.nkb / kFewWaves));
+  if (a.nkb > 4 * kFewWaves * shares) shares *= 2;
+  shares = std::min(shares, 16);
+  const int share = (a.nkb + shares - 1) / shares;
+  shares = (a.nkb + share - 1) / share;
+  if (shares > 1) {
+    const int rc = alloc_scratch((void **)&a.ws, sizeof(float) * (size_t)shares * m * a.e.N);  // fully written
+    if (rc) return rc;
+  }
+  const int rc = w->type == CTHIP_Q8_0   ? (m <= 16 ? few_launch32<FW_Q8, 1>(a, shares) : few_launch32<FW_Q8, 2>(a, shares))
+                 : w->type == CTHIP_Q4_0 ? (m <= 16 ? few_launch32<FW_Q4, 1>(a, shares) : few_launch32<FW_Q4, 2>(a, shares))
+                                         : (m <= 16 ? few_launch32<FW_F16, 1>(a, shares) : few_launch32<FW_F16, 2>(a, shares));
+  if (rc && a.ws) cthip_free(a.ws);
+  else if (a.ws) defer->ws = a.ws, defer->ksplit = shares;
+  return rc;
+}
+
+// y (m, rows) = act(x W^T + bias) + residual; act may be kActSwigluPairs, route as for launch_linear_gemm.
+// Call only where linear_few_pays; y, bias and residual on 16 bytes.
+int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route) {
+  FewArgs a = few_args(y, w, m, bias, residual, act);
+  a.A = (const unsigned char *)operands;
   if (act == kActSwigluPairs) {
     if (residual || route) return fail(CTHIP_E_BAD_ARG, "launch_linear_few: paired SwiGLU epilogue with a residual or a route");
     a.e.act = CTHIP_ACT_NONE;
