@@ -926,9 +926,11 @@ __global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs a) {
 // One wavefront per SIMD issues an instruction every 8 cycles or so: with every wavefront staging, requesting and
 // multiplying, a step's hundred-odd other instructions did not fit behind its 16 matrix instructions (64 cycles
 // each) and a step took 1950 cycles instead of 1024.  Here a multiplying wavefront issues nothing but its matrix
-// instructions and the operand reads of the NEXT step (a second register set; the operands of an fp32 matrix
-// instruction are one register each), which needs three LDS buffers: in step i the staging wavefronts fill
-// buffer (i + 2) % 3 while the multiplying ones read buffer (i + 1) % 3 and compute from registers.
+// instructions and the operand reads of the NEXT half step (a second register set; the operands of an fp32 matrix
+// instruction are one register each), the last half's from the next step's buffer, which needs three LDS buffers: in step i the staging
+// wavefronts fill buffer (i + 2) % 3 while the multiplying ones read buffers i % 3 and (i + 1) % 3 and compute from registers.
+// Reading a whole step ahead took 86 registers a lane and left room for one workgroup on a compute unit; at 58 there are two, one multiplying
+// while the other waits or stores: 2048^3 154 -> 141 us (122 TFLOP/s), 2048 x 2048 x 512 49 -> 40, 4000 x 4000 x 100 80 -> 57, one tile a unit alike.
 //
 // LDS layout: plane p = 2 (k / 4) + (k % 2) holds, for every row, the PAIR (k, k + 2) -- what a lane (row l % 32,
 // half l / 32) feeds to the two matrix instructions 2j, 2j + 1 of a step is the 8 bytes [plane 2j + l / 32][row],
@@ -940,7 +942,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs a) {
 // wavefronts share with the multiplying one of their SIMD.  B is (K,N) row-major here; packed weights (N,K) keep
 // k_gemm_f32, which measured faster on the prompt shapes.
 template <int LD, bool FULL>
-__global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
+__global__ __launch_bounds__(768, 6) void k_gemm_f32pc(GemmArgs a) {
   constexpr int BM = 64, BN = 64, BK = 32, NP = BK / 2;
   // plane pitches in floats: a multiple of 4 where the staging writes are 16 bytes (B), else 8-byte aligned
   constexpr int PA = 2 * BM + 2, PB = 2 * BN + 4;
@@ -967,22 +969,14 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
 
   if (nsteps > 0) {  // K = 0 comes without operands
     if (role == 0) {
-      // ---- multiply: registers of step i were read during step i - 1
+      // ---- multiply: registers of a half step were read during the one before
       const unsigned abase = 4u * (unsigned)((lane >> 5) * PA + 2 * (32 * wm + (lane & 31)));
       const unsigned bbase = (unsigned)kABytes + 4u * (unsigned)((lane >> 5) * PB + 2 * (32 * wn + (lane & 31)));
-      auto rd = [&](int buf, float2(&av)[8], float2(&bv)[8]) __attribute__((always_inline)) {
-        const unsigned char *pa = smem + abase + (unsigned)buf * kABuf, *pb = smem + bbase + (unsigned)buf * kBBuf;
+      // a step's eight pairs in two halves: each half's reads lie between the pairs of matrix instructions of the half before
+      auto half = [&](int buf, int j0, const float2(&av)[4], const float2(&bv)[4], float2(&an)[4], float2(&bn)[4]) __attribute__((always_inline)) {
+        const unsigned char *pa = smem + abase + (unsigned)buf * kABuf + j0 * (2 * PA * 4), *pb = smem + bbase + (unsigned)buf * kBBuf + j0 * (2 * PB * 4);
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-          av[j] = *(const float2 *)(pa + j * (2 * PA * 4));
-          bv[j] = *(const float2 *)(pb + j * (2 * PB * 4));
-        }
-      };
-      // the next step's reads are spread between this step's pairs of matrix instructions
-      auto step = [&](int nbuf, const float2(&av)[8], const float2(&bv)[8], float2(&an)[8], float2(&bn)[8]) __attribute__((always_inline)) {
-        const unsigned char *pa = smem + abase + (unsigned)nbuf * kABuf, *pb = smem + bbase + (unsigned)nbuf * kBBuf;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < 4; j++) {
           an[j] = *(const float2 *)(pa + j * (2 * PA * 4));
           bn[j] = *(const float2 *)(pb + j * (2 * PB * 4));
           __builtin_amdgcn_sched_barrier(0);
@@ -990,20 +984,21 @@ __global__ __launch_bounds__(768) void k_gemm_f32pc(GemmArgs a) {
           acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j].y, bv[j].y, acc, 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
       };
-      float2 a0[8], b0[8], a1[8], b1[8];
+      float2 a0[4], b0[4], a1[4], b1[4];
       __syncthreads();  // steps 0 and 1 are staged
-      rd(0, a0, b0);
-      int nb = 1;  // buffer of the step after the current one
-      int i = 0;
-      for (; i + 2 <= nsteps; i += 2) {
-        step(nb, a0, b0, a1, b1);
-        nb = nb == 2 ? 0 : nb + 1;
-        step(nb, a1, b1, a0, b0);
-        nb = nb == 2 ? 0 : nb + 1;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        a0[j] = *(const float2 *)(smem + abase + j * (2 * PA * 4));
+        b0[j] = *(const float2 *)(smem + bbase + j * (2 * PB * 4));
       }
-      if (i < nsteps) step(nb, a0, b0, a1, b1);
+      int cb = 0;  // the current step's buffer
+      for (int i = 0; i < nsteps; i++) {
+        half(cb, 4, a0, b0, a1, b1);
+        cb = cb == 2 ? 0 : cb + 1;
+        half(cb, 0, a1, b1, a0, b0);
+        __syncthreads();
+      }
     } else if (role == 1) {
       // ---- stage A: units t and t + 256 of the 64 rows x 8 groups of 4 consecutive k
       unsigned aoff[2];
@@ -1197,11 +1192,11 @@ TilePlan tile_plan(int M, int N, int K, int precision, bool quant, bool aligned,
     double start, step, unaligned;            // one round
     double start_n, step_n, unaligned_n;      // several: every compute unit at work
   };
-  static const Cost costs[7] = {{1.0, 1.22, 1.55, 1.0, 1.30, 1.60}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64},
+  static const Cost costs[7] = {{1.0, 1.22, 1.55, 1.1, 1.05, 1.20}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64},
                                 {1.6, 0.85, 1.10, 3.0, 0.88, 0.98}, {2.0, 0.55, 0.55, 2.0, 0.66, 0.66}, {2.0, 0.72, 0.72, 2.0, 0.87, 0.87},
                                 {2.0, 0.90, 0.90, 2.0, 1.10, 1.10}};  // k_gemm_f32pc; k_gemm_split, one .. three terms; k_gemm_qpc, one .. three
   const Cost &c = costs[precision == GEMM_FP32 ? 0 : (quant ? 3 : 0) + (precision == GEMM_BF16 ? 1 : precision == GEMM_BF16X3 ? 2 : 3)];
-  const bool two = !quant && (precision == GEMM_BF16 || precision == GEMM_BF16X3);  // workgroups on a compute unit
+  const bool two = !quant && precision != GEMM_BF16X6;  // workgroups on a compute unit
   const int tm = (M + 63) / 64, tn = (N + (quant ? 127 : 63)) / (quant ? 128 : 64), nsteps = (K + 63) / 64;
   int64_t most = (int64_t)tm * tn;  // tiles of an XCD
   for (int rx = 1; rx <= 8; rx *= 2) most = std::min(most, (int64_t)((tm + rx - 1) / rx) * ((tn + 8 / rx - 1) / (8 / rx)));
