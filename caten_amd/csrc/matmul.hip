@@ -1205,9 +1205,9 @@ TilePlan tile_plan(int M, int N, int K, int precision, bool quant, bool aligned,
     const int steps = (nsteps + ks - 1) / ks, shares = steps ? (nsteps + steps - 1) / steps : 1;
     if (shares < ks) continue;  // the same steps as with fewer
     const double n = (double)(most * shares) * 8.0 / state().compute_units;
-    // (more tiles of a quantised matrix than compute units: shares gain 8 % at the most, 203 x 12288 x 4096 107 -> 98 us, and reorder the sums
-    // of a prompt, which a Q8_0 cache answers with other quants)
-    if (quant && shares > 1 && most * 8 > state().compute_units) break;
+    // (shares of quantised tiles only where compute units are left for them: in a second round they gain 8 % at the most, 203 x 12288 x 4096 107 -> 98 us,
+    // and reorder the sums of a prompt, which a Q8_0 cache answers with other quants)
+    if (quant && shares > 1 && n > 1.0) break;
     const double rounds = n <= 1.0 ? 1.0 : n <= 2.0 && two ? 1.85 : n <= 4.0 ? ceil(n) : 0.5 * ceil(2.0 * n);
     const double tile = n <= 1.0 ? c.start + (aligned ? c.step : c.unaligned) * steps : c.start_n + (aligned ? c.step_n : c.unaligned_n) * steps;
     const double sum = shares > 1 ? (deferred ? 0.3 : 2.6) + (deferred ? 0.6e-6 : 0.85e-6) * 4.0 * shares * M * N : 0.0;
