@@ -3,7 +3,7 @@
 // The vector kernels (gemv_kernels.h, gemv_wide.hip) spend 2.4 - 7.8 vector instructions on a weight -- a conversion, a
 // multiply-add, their share of the prologue -- which at one wavefront per SIMD is as much time as the weights take to arrive.
 // Here the input vector is written as four signed base-256 digits per element (30 bits below the largest value of its chunk, the block of 32
-// that meets 16 bytes of weights, with a power of two for each), nibbles go to v_mfma_i32_16x16x64_i8 as bytes (one or two
+// that meets 16 bytes of weights, with a power of two for each; all bits there are where fewer than 30 lie above the smallest float), nibbles go to v_mfma_i32_16x16x64_i8 as bytes (one or two
 // bit operations per four of them), and the products and their sums over a chunk are exact integers:
 //   sum q x = 2^e (((i0 256 + i1) 256 + i2) 256 + i3),  i_r = sum over the chunk of q * digit r.
 // Digits are the rows of the first operand, weight rows the columns of the second: lane l holds 16 bytes of weight row l % 16, the (l / 16)-th chunk of
@@ -24,8 +24,10 @@ namespace cthip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
+// A chunk's sums are taken times 2^-28 and its power of two times 2^28: a weight row's scale, a multiple of 2^-24, times that power is then exact down to
+// chunks of subnormal numbers, and in range as far up as the vector kernels' sums of nibble times input are.
 // four consecutive k of a chunk (eight neighbouring lanes hold one): digit words of the four elements, and what undoes the
-// chunk's power of two.  A chunk with an infinity or a NaN keeps its sign there and nothing else: 2^e becomes infinity / NaN.
+// chunk's power of two (and the 16 of a nibble).  A chunk with an infinity or a NaN keeps its sign there and nothing else: 2^e becomes infinity / NaN.
 __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   unsigned m = 0;
 #pragma unroll
@@ -33,13 +35,12 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xf, 0xf, true));   // quad_perm 1, 0, 3, 2
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xf, 0xf, true));   // quad_perm 2, 3, 0, 1
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));  // row_half_mirror
-  const unsigned E = max(m >> 23, 30u);  // nothing below the smallest normal number is kept
+  const unsigned E = max(m >> 23, 7u);  // (a unit is 2^(E - 156); at 7 the smallest subnormal number, of which every float is a multiple)
   const bool finite = m < 0x7f800000u;
-  const float up = __uint_as_float((finite ? 283u - E : 0u) << 23);
   unsigned t[4];
 #pragma unroll
   for (int e = 0; e < 4; e++) {
-    int x = (int)rintf(v[e] * up);
+    int x = (int)rintf(__builtin_amdgcn_ldexpf(v[e], 156 - (int)E));  // (the factor itself may lie past the largest float)
     if (!finite) x = (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u ? ((int)__float_as_uint(v[e]) < 0 ? -1 : 1) << 24 : 0;
     t[e] = ((unsigned)x + 0x808080u) ^ 0x808080u;  // bytes: signed digits, the highest in byte 3
   }
@@ -49,7 +50,7 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   w[1] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
   w[2] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
   w[3] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
-  return m > 0x7f800000u ? __uint_as_float(0x7fc00000u) : finite ? __uint_as_float((E - 29u) << 23) : INFINITY;
+  return m > 0x7f800000u ? __uint_as_float(0x7fc00000u) : finite ? __uint_as_float((E - 5u) << 23) : INFINITY;
 }
 
 struct GemvIntShape {
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
       }
       unsigned w[4];
       const float down = int_digits(v, w);
-      put(k, w, down * 0.0625f);  // (nibbles are multiplied as 16 (n - 8))
+      put(k, w, down);
     }
   }
   if (RMS || LAYERNORM) {
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
       }
       r = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, lo, r, 0, 0, 0);
       r = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, hi, r, 0, 0, 0);
-      const float f = fmaf((float)(r[0] * 256 + r[1]), 65536.0f, (float)(r[2] * 256 + r[3]));
+      const float f = fmaf((float)(r[0] * 256 + r[1]), 0x1p-12f, (float)(r[2] * 256 + r[3]) * 0x1p-28f);
       const float d = half_bits_to_float((unsigned short)(s ? st[p] >> 16 : st[p])) * sx[unit * 8 + 2 * g + s];
       acc = fmaf(d, f, acc);
     }
