@@ -15,7 +15,7 @@
 // is two terms, exact; an fp32 weight three.  Products of terms below 2^-24 of the leading one are left out.
 // An infinity or a NaN stands in the last term, which meets the leading term of a weight only (infinity times a lower
 // term of zero would be NaN): it comes out as it does of fp32 products.  Matrix cores take a term below 2^-126 for zero: a
-// row of nothing above 2^-32 goes in times 2^64.
+// row of nothing above 2^-32 goes in times the power of two that takes it to 2^-16.
 // Three terms per input, two where "gemm_precision" asks for operands rounded to bf16.
 //
 // K is shared among as many workgroups as fill the chip; a share leaves its partial sums in memory and draws a ticket, the
@@ -457,8 +457,10 @@ __global__ __launch_bounds__(NT) void k_rows_planes(RowsPlanesArgs a) {
 #pragma unroll
     for (int w = 0; w < NW; w++) m = fmaxf(m, red[2][w]);
     const bool small = m < 0x1p-32f;
-    if (small) emit(0x1p64f);
-    if (tid == 0) a.rscale[blockIdx.x] = small ? 0x1p-64f : 1.0f;
+    // to 2^-16: 110 bits above what the matrix cores take for zero, and 2^15 finite weights times it have a finite sum
+    const int e = small ? 111 - max((int)(__float_as_uint(m) >> 23), 1) : 0;
+    if (small) emit(__uint_as_float((unsigned)(127 + e) << 23));
+    if (tid == 0) a.rscale[blockIdx.x] = __uint_as_float((unsigned)(127 - e) << 23);
   }
 }
 constexpr int kRowsPlanesMaxK = 8 * 1024 * 4;  // widest row the largest instantiation holds

@@ -111,6 +111,21 @@ def test_inputs_that_are_not_finite_or_nearly_so(ops, kind, rows, cols, m):
     w.free()
 
 
+@pytest.mark.parametrize("rows,cols,m", [(2603, 2052, 5), (1100, 11000, 7)])
+def test_small_rows_against_large_weights(ops, rows, cols, m):
+    """fp32 weights about 1e35 and rows down to subnormal numbers: the results are ordinary floats."""
+    rng = np.random.default_rng(rows)
+    a = rng.normal(0, 1e35, (rows, cols)).astype(np.float32)
+    w = ops.WeightMatrix("f32", a, rows, cols)
+    x = rng.normal(0, 1, (m, cols)) * np.array([1.0, 2.0 ** -33, 1e-12, 1e-30, 1e-39, 1e-20, 1e-10])[:m, None]
+    x = x.astype(np.float32)
+    got, want = ops.linear(x, w), x.astype(np.float64) @ a.astype(np.float64).T
+    assert np.abs(want).max() < 2.0 ** 127  # (rows of ones: 1e35 sqrt(cols) = 1e37, and a few times that)
+    assert np.all(np.isfinite(got))
+    assert np.all(np.abs(got - want) <= tree_bound(cols) * (np.abs(x.astype(np.float64)) @ np.abs(a.astype(np.float64)).T))
+    w.free()
+
+
 @pytest.mark.parametrize("kind,rows,cols,m,precision", [
     ("f16", 2100, 28672, 27, 2), ("f16", 2100, 28672, 32, 2), ("f16", 2100, 28672, 18, 3), ("f16", 2100, 28672, 32, 3), ("f16", 2050, 29568, 25, 2),
     ("f16", 2500, 24576, 31, 2), ("q4_0", 4098 * 128, 2240, 16, 2), ("f16", 2100, 28672, 17, 2), ("f16", 2100, 28672, 16, 2), ("q8_0", 1700, 28672, 16, 3)])
