@@ -197,9 +197,36 @@ __global__ __launch_bounds__(256) void k_argmax_finish(GemvArgs a, int nparts) {
   }
 }
 
+// Element i of an input vector with its prologue.  A norm's mean and rstd are what the wavefront got from generic_stats().
+struct GenericStats {
+  float mean, rstd;
+};
+__device__ __forceinline__ GenericStats generic_stats(const GemvArgs &a, const float *x, int lane) {
+  GenericStats s = {0.0f, 1.0f};
+  if (a.pro != CTHIP_PRO_LAYERNORM && a.pro != CTHIP_PRO_RMSNORM) return s;
+  float t = 0.0f, v = 0.0f;
+  if (a.pro == CTHIP_PRO_LAYERNORM) {
+    for (int i = lane; i < a.cols; i += 64) t += x[i];
+    s.mean = wave_sum(t) / (float)a.cols;
+  }
+  for (int i = lane; i < a.cols; i += 64) v = fmaf(x[i] - s.mean, x[i] - s.mean, v);
+  s.rstd = 1.0f / sqrtf(wave_sum(v) / (float)a.cols + a.eps);
+  return s;
+}
+template <bool PRO>
+__device__ __forceinline__ float generic_input(const GemvArgs &a, const float *x, const GenericStats &s, int64_t i) {
+  if (!PRO) return x[i];
+  if (a.pro == CTHIP_PRO_SWIGLU) return ct_silu(x[i]) * x[a.cols + i];
+  float t = (x[i] - s.mean) * s.rstd;
+  if (a.norm_g) t *= a.norm_g[i];
+  if (a.norm_b) t += a.norm_b[i];
+  return t;
+}
+
 // Fallback for shapes no (G,KC) instantiation covers: one wavefront per row, the
-// input vector re-read through the cache hierarchy. `x` must already carry the prologue.
-template <int TYPE>
+// input vector re-read through the cache hierarchy.  PRO: with its prologue, applied anew for every row (where there is no memory to
+// keep the result in); else `x` must already carry it.
+template <int TYPE, bool PRO>
 __global__ __launch_bounds__(256) void k_gemv_generic(GemvArgs a) {
   constexpr int XPC = Fmt<TYPE>::XPC;
   constexpr bool QUANT = (TYPE == CTHIP_Q8_0 || TYPE == CTHIP_Q4_0);
@@ -211,6 +238,7 @@ __global__ __launch_bounds__(256) void k_gemv_generic(GemvArgs a) {
   const float *__restrict__ x = a.x + (int64_t)m * a.x_stride;
   const uint4 *__restrict__ qp = (const uint4 *)a.q;
   const int posv = a.pos ? a.pos[0] : 0;
+  const GenericStats st = PRO ? generic_stats(a, x, lane) : GenericStats{0.0f, 1.0f};
   float best_v = -INFINITY;
   int best_i = 0x7fffffff;
   for (int row = wave; row < a.rows; row += total_waves) {
@@ -221,7 +249,7 @@ __global__ __launch_bounds__(256) void k_gemv_generic(GemvArgs a) {
       float xsum = 0.0f;
 #pragma unroll
       for (int e = 0; e < XPC; e++) {
-        xl[e] = x[(int64_t)c * XPC + e];
+        xl[e] = generic_input<PRO>(a, x, st, (int64_t)c * XPC + e);
         xsum += xl[e];
       }
       float scale = 1.0f;
@@ -242,8 +270,8 @@ __global__ __launch_bounds__(256) void k_gemv_generic(GemvArgs a) {
 }
 
 // fp32 / fp16 rows whose width is no multiple of a 16-byte chunk: rows start at any element, so the lanes of a
-// wavefront stride the row element by element.  `x` must already carry the prologue.
-template <int TYPE>
+// wavefront stride the row element by element.  PRO as above.
+template <int TYPE, bool PRO>
 __global__ __launch_bounds__(256) void k_gemv_elements(GemvArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -251,6 +279,7 @@ __global__ __launch_bounds__(256) void k_gemv_elements(GemvArgs a) {
   const int m = blockIdx.y;
   const float *__restrict__ x = a.x + (int64_t)m * a.x_stride;
   const int posv = a.pos ? a.pos[0] : 0;
+  const GenericStats st = PRO ? generic_stats(a, x, lane) : GenericStats{0.0f, 1.0f};
   float best_v = -INFINITY;
   int best_i = 0x7fffffff;
   for (int row = wave; row < a.rows; row += total_waves) {
@@ -258,7 +287,7 @@ __global__ __launch_bounds__(256) void k_gemv_elements(GemvArgs a) {
     for (int c = lane; c < a.cols; c += 64) {
       const int64_t e = (int64_t)row * a.cols + c;
       const float w = TYPE == CTHIP_F16 ? half_bits_to_float(((const unsigned short *)a.q)[e]) : ((const float *)a.q)[e];
-      acc = fmaf(w, x[c], acc);
+      acc = fmaf(w, generic_input<PRO>(a, x, st, c), acc);
     }
     acc = wave_sum(acc);
     if (lane == 0) {
@@ -549,9 +578,11 @@ int launch_gemv(const WMat *w, GemvArgs a, int m) {
     }
     return 0;
   }
-  // generic path: prologue into a temporary, then wave-per-row
+  // generic path: prologue into a temporary, then wave-per-row.  (Under graph capture the launch applies it itself: a replay would find
+  // the temporary in other hands.)
   float *tmp = nullptr;
-  if (a.pro != CTHIP_PRO_NONE) {
+  const bool inside = a.pro != CTHIP_PRO_NONE && stream_capturing();
+  if (a.pro != CTHIP_PRO_NONE && !inside) {
     int rc = alloc_scratch((void **)&tmp, sizeof(float) * (size_t)a.cols * m);  // fully written below
     if (rc) return rc;
     rc = launch_prologue(tmp, a.x, a.cols, a.pro, a.norm_g, a.norm_b, a.eps, a.x_stride, m);
@@ -570,18 +601,24 @@ int launch_gemv(const WMat *w, GemvArgs a, int m) {
   // rows that are whole 16-byte chunks are read chunk by chunk; any other width (fp32 / fp16 only: quantised rows
   // are multiples of 32) element by element
   const bool chunks = a.cols % xpc_of(w->type) == 0;
+#define GENERIC(K, TYPE)                                                                        \
+  do {                                                                                          \
+    if (inside) hipLaunchKernelGGL((K<TYPE, true>), grid, block, 0, s.stream, a);                \
+    else hipLaunchKernelGGL((K<TYPE, false>), grid, block, 0, s.stream, a);                      \
+  } while (0)
   switch (w->type) {
-    case CTHIP_Q8_0: hipLaunchKernelGGL(k_gemv_generic<CTHIP_Q8_0>, grid, block, 0, s.stream, a); break;
-    case CTHIP_Q4_0: hipLaunchKernelGGL(k_gemv_generic<CTHIP_Q4_0>, grid, block, 0, s.stream, a); break;
+    case CTHIP_Q8_0: GENERIC(k_gemv_generic, CTHIP_Q8_0); break;
+    case CTHIP_Q4_0: GENERIC(k_gemv_generic, CTHIP_Q4_0); break;
     case CTHIP_F16:
-      if (chunks) hipLaunchKernelGGL(k_gemv_generic<CTHIP_F16>, grid, block, 0, s.stream, a);
-      else hipLaunchKernelGGL(k_gemv_elements<CTHIP_F16>, grid, block, 0, s.stream, a);
+      if (chunks) GENERIC(k_gemv_generic, CTHIP_F16);
+      else GENERIC(k_gemv_elements, CTHIP_F16);
       break;
     default:
-      if (chunks) hipLaunchKernelGGL(k_gemv_generic<CTHIP_F32>, grid, block, 0, s.stream, a);
-      else hipLaunchKernelGGL(k_gemv_elements<CTHIP_F32>, grid, block, 0, s.stream, a);
+      if (chunks) GENERIC(k_gemv_generic, CTHIP_F32);
+      else GENERIC(k_gemv_elements, CTHIP_F32);
       break;
   }
+#undef GENERIC
   CTHIP_LAUNCH_CHECK();
   if (a.am_val) {
     hipLaunchKernelGGL(k_argmax_finish, dim3(1), dim3(256), 0, s.stream, a, (int)(grid.x * 4));
@@ -760,8 +797,9 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
       return rc ? rc : rf;
     }
   }
-  if (m >= 8) {
-    // several input rows: the MFMA tile path reads the weights once instead of once per row
+  // several input rows: the MFMA tile path reads the weights once instead of once per row.  (Not with a prologue under graph capture: its rows go
+  // through memory that a replay would find in other hands, the single-row kernels apply it themselves.)
+  if (m >= 8 && !(prologue != CTHIP_PRO_NONE && stream_capturing())) {
     const float *xin = x;
     float *tmp = nullptr;
     int rc;

@@ -1259,6 +1259,8 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
     const int nsteps = (a.K + 63) / 64;  // K-steps of 64 (two of the fp32 kernel's)
     const bool aligned = a.K % 4 == 0 && (bmode == B_WMAT || a.N % 4 == 0);
     int ks = a.pairs ? 1 : tile_plan(a.M, a.N, a.K, precision, quant, aligned, defer && !static_ws && a.act == CTHIP_ACT_NONE).ks;
+    // (under graph capture no block is taken for shares: a replay would find it in other hands)
+    if (ks > 1 && !static_ws && stream_capturing()) ks = 1;
     if (static_ws) {
       // what does not fit split two ways per compute unit is refused, what fits is split as often as it does
       int fill = (int)((tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles);

@@ -15,10 +15,13 @@ def packed(kind, a):
 
 
 def cases(ops, _lib, lib, rng):
-    def linear(kind, rows, cols, m, tol):
+    def linear(kind, rows, cols, m, tol, pro=_lib.PRO_NONE):
         w = ops.WeightMatrix(kind, packed(kind, rng.normal(0, 0.05, (rows, cols)).astype(np.float32)), rows, cols)
-        x, y = ops.DeviceArray.from_numpy(rng.normal(0, 1, (m, cols)).astype(np.float32)), ops.DeviceArray((m, rows))
-        return y, tol, (w, x), lambda: _lib.check(lib.cthip_linear(y.ptr, w.handle, x.ptr, m, None, None, 0, 0, None, None, 1e-5))
+        x = ops.DeviceArray.from_numpy(rng.normal(0.3, 1, (m, cols * (2 if pro == _lib.PRO_SWIGLU else 1))).astype(np.float32))
+        y, g, b = ops.DeviceArray((m, rows)), *(ops.DeviceArray.from_numpy(rng.normal(1, 0.1, cols).astype(np.float32)) for _ in range(2))
+        gamma = g.ptr if pro in (_lib.PRO_LAYERNORM, _lib.PRO_RMSNORM) else None
+        beta = b.ptr if pro == _lib.PRO_LAYERNORM else None
+        return y, tol, (w, x, g, b), lambda: _lib.check(lib.cthip_linear(y.ptr, w.handle, x.ptr, m, None, None, 0, pro, gamma, beta, 1e-5))
 
     def row(n):
         x = rng.normal(0, 1, (2, n)).astype(np.float32)
@@ -35,10 +38,14 @@ def cases(ops, _lib, lib, rng):
         y = ops.DeviceArray((m, n))
         return y, 5e-5, (a, b), lambda: _lib.check(lib.cthip_matmul(y.ptr, a.ptr, b.ptr, m, n, k, 0, 2))
 
-    # few rows; many rows of a matrix that would keep its terms, and of one that makes them at every call; long rows; a large product
-    # (none of them splits its reduction on the path without scratch)
+    # few rows; many rows of a matrix that would keep its terms, and of one that makes them at every call; long rows; a large product; products and Linears
+    # that share their reduction, then Linears with a norm or SwiGLU in front: rows past and below the tiles', widths that no single-row kernel is laid out for
     return [linear("q8_0", 4100, 2048, 7, 1e-6), linear("q4_0", 12000, 2080, 5, 1e-6), linear("f16", 4100, 1008, 777, 5e-5), linear("q8_0", 11270, 2080, 391, 5e-5),
-            linear("f32", 6402, 1600, 517, 5e-5), row(50257), row(70001), best(50257), matmul(1500, 1500, 1500)]
+            linear("f32", 6402, 1600, 517, 5e-5), row(50257), row(70001), best(50257), matmul(1500, 1500, 1500),
+            matmul(130, 190, 1024), linear("f16", 300, 4096, 20, 5e-5), linear("q8_0", 640, 5120, 70, 5e-5),
+            linear("q8_0", 520, 1024, 40, 5e-5, _lib.PRO_RMSNORM), linear("f32", 333, 512, 100, 5e-5, _lib.PRO_LAYERNORM), linear("f16", 300, 1024, 9, 5e-5, _lib.PRO_SWIGLU),
+            linear("q4_0", 2600, 4096, 12, 5e-5, _lib.PRO_SWIGLU), linear("f32", 200, 1001, 12, 5e-5, _lib.PRO_LAYERNORM), linear("f32", 200, 1001, 3, 1e-6, _lib.PRO_RMSNORM),
+            linear("f16", 201, 999, 5, 1e-6, _lib.PRO_SWIGLU), linear("q8_0", 70, 40960, 3, 1e-6, _lib.PRO_LAYERNORM), linear("q4_0", 70, 40960, 9, 5e-5, _lib.PRO_RMSNORM)]
 
 
 def test_captured_calls_take_no_scratch():
