@@ -1262,14 +1262,15 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
     // (under graph capture no block is taken for shares: a replay would find it in other hands)
     if (ks > 1 && !static_ws && stream_capturing()) ks = 1;
     if (static_ws) {
-      // what does not fit split two ways per compute unit is refused, what fits is split as often as it does
+      // Refused are products for which shares that fill the chip would not fit.  The launch needs no such line (it makes fewer shares where that is faster, and
+      // never more than fit): it is the entry point's, callers have another path behind it, and it stays where it was drawn.
       int fill = (int)((tiles * 2 <= cus ? cus * 2 : cus * 3 / 2) / tiles);
       fill = std::min(std::min(fill, nsteps / 3), 16);
       const int share = fill > 1 ? (nsteps + fill - 1) / fill : nsteps, most = share > 0 ? (nsteps + share - 1) / share : 1;
       const size_t tile_bytes = sizeof(float) * (size_t)a.M * a.N;
       if (most > 1 && most * tile_bytes > static_ws_bytes)
-        return fail(CTHIP_E_UNSUPPORTED, "cthip_matmul_noalloc: (%d,%d,%d) splits its reduction %d ways and needs %zu bytes of partial "
-                    "tiles; the static scratch holds %zu (use cthip_matmul)", a.M, a.N, a.K, most, most * tile_bytes, static_ws_bytes);
+        return fail(CTHIP_E_UNSUPPORTED, "cthip_matmul_noalloc: (%d,%d,%d) is past this entry point: partial tiles to fill the chip are %d x %zu bytes, "
+                    "the static scratch holds %zu (use cthip_matmul)", a.M, a.N, a.K, most, tile_bytes, static_ws_bytes);
       ks = std::min(ks, (int)(static_ws_bytes / tile_bytes));
     }
     if (ks > 1) {

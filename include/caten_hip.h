@@ -302,10 +302,13 @@ int cthip_set_option(const char *name, int value);
  * in every mode. */
 int cthip_matmul(float *C, const float *A, const float *B, int M, int N, int K, int act, int precision);
 /* cthip_matmul for callers that cannot allocate device memory (code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc): same arguments, same kernels, same results, but the partial tiles of
+ * loops, harnesses that forbid hipMalloc): same arguments, same operand formats, but the partial tiles of
  * a split reduction go to a 4 MiB array that is part of the library's code object instead of a block of the
- * caching allocator, and no allocation or release happens during the call.  A shape whose split needs more
- * (split count x M x N x 4 bytes) returns CTHIP_E_UNSUPPORTED.  All calls on one GPU share that array: calls
+ * caching allocator, and no allocation or release happens during the call.  (cthip_matmul takes kernels over
+ * operands converted once for large products; where it does not, and its shares fit the array, the results are
+ * the same bits.)  CTHIP_E_UNSUPPORTED where partial tiles to fill the chip do not fit: with t tiles of 64 x 64,
+ * c compute units and f = min(2c / t, or 1.5c / t from 2t > c on; K / 192; 16), f > 1 and f x M x N x 4 bytes
+ * exceed the array.  The launch itself may share the reduction less.  All calls on one GPU share that array: calls
  * that overlap on one GPU (two host threads, two streams) race.  It has no counterpart in the reference. */
 int cthip_matmul_noalloc(float *C, const float *A, const float *B, int M, int N, int K, int act, int precision);
 

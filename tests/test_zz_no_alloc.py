@@ -58,3 +58,17 @@ def test_noalloc_matmul_refuses_what_the_scratch_cannot_hold():
         _lib.check(lib.cthip_matmul_noalloc(dC.ptr, dA.ptr, dB.ptr, M, N, K, 0, 0))
     _lib.check(lib.cthip_matmul(dC.ptr, dA.ptr, dB.ptr, M, N, K, 0, 0))  # the allocating entry point takes it
     _lib.check(lib.cthip_sync())
+
+
+def test_noalloc_matmul_says_where_its_line_lies():
+    """Two partial tiles of (768, 768) do not fit 4 MiB, of (704, 704) they do -- whatever share count the launch then takes."""
+    from caten_amd import _lib, HipError
+    lib = _lib.init(0)
+    rng = np.random.default_rng(8)
+    A, B = rng.uniform(-1, 1, (768, 768)).astype(np.float32), rng.uniform(-1, 1, (768, 768)).astype(np.float32)
+    with pytest.raises(HipError, match="past this entry point: partial tiles to fill the chip are 2 x 2359296 bytes"):
+        _run(lib, _lib.check, lib.cthip_matmul_noalloc, A, B, 0, 3)
+    A, B = np.ascontiguousarray(A[:704, :384]), np.ascontiguousarray(B[:384, :704])
+    got, delta = _run(lib, _lib.check, lib.cthip_matmul_noalloc, A, B, 0, 3)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    assert delta == (0, 0, 0) and np.all(np.abs(got - ref) <= ATOL + RTOL * np.abs(ref))
