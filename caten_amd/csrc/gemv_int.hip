@@ -27,7 +27,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 // A chunk's sums are taken times 2^-28 and its power of two times 2^28: a weight row's scale, a multiple of 2^-24, times that power is then exact down to
 // chunks of subnormal numbers, and in range as far up as the vector kernels' sums of nibble times input are.
 // four consecutive k of a chunk (eight neighbouring lanes hold one): digit words of the four elements, and what undoes the
-// chunk's power of two (and the 16 of a nibble).  A chunk with an infinity or a NaN keeps its sign there and nothing else: 2^e becomes infinity / NaN.
+// chunk's power of two (and the 16 of a nibble).  A chunk with one infinity keeps its sign there and nothing else, 2^e becomes infinity: the product is
+// what it is of floats.  With a NaN, or with infinities whose products would be added up before they are infinite, 2^e becomes NaN (as the vector kernels' sums do).
 __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   unsigned m = 0;
 #pragma unroll
@@ -37,6 +38,14 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));  // row_half_mirror
   const unsigned E = max(m >> 23, 7u);  // (a unit is 2^(E - 156); at 7 the smallest subnormal number, of which every float is a multiple)
   const bool finite = m < 0x7f800000u;
+  int infs = 0;
+  if (!finite) {  // (the eight lanes of a chunk together)
+#pragma unroll
+    for (int e = 0; e < 4; e++) infs += (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u ? 1 : 0;
+    infs += __builtin_amdgcn_mov_dpp(infs, 0xB1, 0xf, 0xf, true);
+    infs += __builtin_amdgcn_mov_dpp(infs, 0x4E, 0xf, 0xf, true);
+    infs += __builtin_amdgcn_mov_dpp(infs, 0x141, 0xf, 0xf, true);
+  }
   unsigned t[4];
 #pragma unroll
   for (int e = 0; e < 4; e++) {
@@ -50,7 +59,7 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   w[1] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
   w[2] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
   w[3] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
-  return m > 0x7f800000u ? __uint_as_float(0x7fc00000u) : finite ? __uint_as_float((E - 5u) << 23) : INFINITY;
+  return m > 0x7f800000u || infs > 1 ? __uint_as_float(0x7fc00000u) : finite ? __uint_as_float((E - 5u) << 23) : INFINITY;
 }
 
 struct GemvIntShape {

@@ -72,6 +72,18 @@ def test_inputs_that_are_not_finite(ops, kind, rows, cols):
     assert np.array_equal(got[with_weight], np.sign(wd[with_weight, 40]) * np.inf) and np.all(np.isnan(got[~with_weight]))
     x[40] = np.nan
     assert np.all(np.isnan(ops.linear(x, w)))
+    # several in one block of 32: never a finite number or an infinity where products of both signs (or of a zero weight) meet
+    for a, b in ((np.inf, np.inf), (np.inf, -np.inf), (-np.inf, -np.inf)):
+        x[40], x[61] = a, b
+        with np.errstate(invalid="ignore"):
+            want = wd[:, 40] * a + wd[:, 61] * b
+        got = ops.linear(x, w)
+        assert np.all(np.isnan(got[np.isnan(want)])) and not np.any(np.isfinite(got))
+    # ... and in two blocks: as of floats
+    x[61], x[64 + 61] = 1.0, -np.inf
+    with np.errstate(invalid="ignore"):
+        want = wd[:, 40] * x[40] + wd[:, 64 + 61] * x[64 + 61]
+    assert np.array_equal(ops.linear(x, w), want.astype(np.float32), equal_nan=True)
     w.free()
 
 
