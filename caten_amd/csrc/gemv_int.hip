@@ -38,21 +38,23 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));  // row_half_mirror
   const unsigned E = max(m >> 23, 7u);  // (a unit is 2^(E - 156); at 7 the smallest subnormal number, of which every float is a multiple)
   const bool finite = m < 0x7f800000u;
-  int infs = 0;
-  if (!finite) {  // (the eight lanes of a chunk together)
+  int x[4], infs = 0;
 #pragma unroll
-    for (int e = 0; e < 4; e++) infs += (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u ? 1 : 0;
+  for (int e = 0; e < 4; e++) x[e] = (int)rintf(__builtin_amdgcn_ldexpf(v[e], 156 - (int)E));  // (the factor itself may lie past the largest float)
+  if (__builtin_expect(!finite, 0)) {  // (the eight lanes of a chunk together)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const bool inf = (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u;
+      x[e] = inf ? ((int)__float_as_uint(v[e]) < 0 ? -1 : 1) << 24 : 0;
+      infs += inf ? 1 : 0;
+    }
     infs += __builtin_amdgcn_mov_dpp(infs, 0xB1, 0xf, 0xf, true);
     infs += __builtin_amdgcn_mov_dpp(infs, 0x4E, 0xf, 0xf, true);
     infs += __builtin_amdgcn_mov_dpp(infs, 0x141, 0xf, 0xf, true);
   }
   unsigned t[4];
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    int x = (int)rintf(__builtin_amdgcn_ldexpf(v[e], 156 - (int)E));  // (the factor itself may lie past the largest float)
-    if (!finite) x = (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u ? ((int)__float_as_uint(v[e]) < 0 ? -1 : 1) << 24 : 0;
-    t[e] = ((unsigned)x + 0x808080u) ^ 0x808080u;  // bytes: signed digits, the highest in byte 3
-  }
+  for (int e = 0; e < 4; e++) t[e] = ((unsigned)x[e] + 0x808080u) ^ 0x808080u;  // bytes: signed digits, the highest in byte 3
   const unsigned a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
   const unsigned b01 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u), b23 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
   w[0] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
@@ -67,7 +69,8 @@ struct GemvIntShape {
   int inv_ks, inv_rows;    // 65536 / ks, 65536 / (16 rgp), rounded up: quotients of numbers below 1024
 };
 
-template <int PRO, bool NT>
+// CENTRED: the mean of a LayerNorm comes off the vector before its digits are made, not off the sums behind them
+template <int PRO, bool CENTRED, bool NT>
 __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) {
   constexpr int PD = 2;              // units in flight per wavefront (four: no faster stream, 0.8 us more code to get through)
   constexpr bool RMS = PRO == CTHIP_PRO_RMSNORM, LAYERNORM = PRO == CTHIP_PRO_LAYERNORM;
@@ -133,6 +136,26 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
   // ---- digits ----
   float s1 = 0.0f, mu = 0.0f, rstd = 1.0f;
   if (tid < 64) ((unsigned *)smem)[tid] = 0u;
+  auto of_all = [&](const float *p, int stride, int n) __attribute__((always_inline)) {  // p[0] + p[stride] + ..., n <= 16, all asked for together
+    float t[16], v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; w++) t[w] = p[min(w, n - 1) * stride];
+#pragma unroll
+    for (int w = 0; w < 16; w++) v += w < n ? t[w] : 0.0f;
+    return v;
+  };
+  if (CENTRED) {
+    auto add = [&](const float4 &t) __attribute__((always_inline)) { s1 += (t.x + t.y) + (t.z + t.w); };
+#pragma unroll
+    for (int b = 0; b < SB; b++)
+      if (tid + nthr * b < n4) add(xv[b]);
+    for (int k = tid + nthr * SB; k < n4; k += nthr) add(x4[k]);
+    s1 = wave_sum(s1);
+    if (lane == 0) red[wv] = s1;
+    __syncthreads();
+    mu = of_all(red, 1, nw) / (float)a.cols;
+    s1 = 0.0f;
+  }
   auto put = [&](int k, const unsigned *w, float down) __attribute__((always_inline)) {  // digits of k = 4 k .. + 3: [16 k][digit][16 bytes]
     unsigned *o = (unsigned *)(dig + (size_t)(k >> 2) * 64) + (k & 3);
 #pragma unroll
@@ -153,8 +176,9 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
       const float u[4] = {uv[b].x, uv[b].y, uv[b].z, uv[b].w};
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        if (LAYERNORM) s1 += v[e];
-        if (RMS) s1 = fmaf(v[e], v[e], s1);
+        if (CENTRED) v[e] -= mu;
+        else if (LAYERNORM) s1 += v[e];
+        if (RMS || CENTRED) s1 = fmaf(v[e], v[e], s1);
         if ((RMS || LAYERNORM) && a.norm_g) v[e] *= u[e];
       }
       unsigned w[4];
@@ -164,18 +188,10 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
   }
   if (RMS || LAYERNORM) {
     s1 = wave_sum(s1);
-    if (lane == 0) red[wv] = s1;
+    if (lane == 0) red[CENTRED ? 16 + wv : wv] = s1;
   }
   __syncthreads();
-  auto of_all = [&](const float *p, int stride, int n) __attribute__((always_inline)) {  // p[0] + p[stride] + ..., n <= 16, all asked for together
-    float t[16], v = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 16; w++) t[w] = p[min(w, n - 1) * stride];
-#pragma unroll
-    for (int w = 0; w < 16; w++) v += w < n ? t[w] : 0.0f;
-    return v;
-  };
-  if (LAYERNORM) {  // the deviations from the mean: the vector once more (it is in the caches; the weights are on their way)
+  if (LAYERNORM && !CENTRED) {  // the deviations from the mean: the vector once more (it is in the caches; the weights are on their way)
     mu = of_all(red, 1, nw) / (float)a.cols;
     float q = 0.0f;
     for (int k = tid; k < n4; k += nthr) {
@@ -245,7 +261,7 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
   if (oj < iters && orow < a.rows) {
     const float *p = ps + ((size_t)oj * nw + (oi >> 4) * sh.ks) * 16 + (oi & 15);
     float v = of_all(p, 16, sh.ks);
-    if (LAYERNORM) v -= mu * of;
+    if (LAYERNORM && !CENTRED) v -= mu * of;
     if (RMS || LAYERNORM) v *= rstd;
     if (a.pair_swiglu) {  // rows 2r, 2r + 1 are a (gate, up) pair, in neighbouring threads (rows are even)
       const float full = v + ob, up = __shfl_xor(full, 1, 64);
@@ -284,13 +300,18 @@ int launch_gemv_int(const WMat *w, GemvArgs a, int m, int *am_parts) {
   a.rows = (int)w->rows;
   a.cols = (int)w->cols;
   if (a.split1 <= 0) a.split1 = a.split2 = a.rows;
+  // A LayerNorm folded through the product loses what the mean takes off behind it.  Without a bias or a residual of the launch's own (a model's head), where the
+  // vector kernels normalise their copy of the vector, the mean comes off the vector here too, one barrier ahead: error against 64 bits,
+  // 50257 x 1280, mean of 3 / 30 / 300 deviations 3.5e-7 / 3.5e-6 / 3.3e-5 -> 1.4e-7 / 1.5e-6 / 6e-6 (vector kernels 4e-7 / 1e-6 / 1.6e-5; what is left is the mean's own rounding), in as much time (10.5 us).
+  const bool centred = a.pro == CTHIP_PRO_LAYERNORM && !a.bias0 && !a.residual;
   // A line asked for with the hint is fetched a second time for its second chunk, which costs 4 - 7 % of a stream; keeping the weights from
   // pushing each other out of the cache is worth more until they are many times its size (us per step, with the hint / without: 36 layers of 1280, 0.46 GB 1040 / 1100;
   // 48 of 1600, 0.87 GB 1560 / 1560; 32 of 4096, 3.7 GB 1617 / 1549).
   const bool nt = s.gemv_stream < 0 ? w->stream && !w->stream_far : s.gemv_stream != 0;
   typedef void (*int_fn)(GemvArgs, GemvIntShape);
-#define PICK(PRO) (nt ? k_gemv_int<PRO, true> : k_gemv_int<PRO, false>)
-  int_fn fn = a.pro == CTHIP_PRO_RMSNORM ? PICK(CTHIP_PRO_RMSNORM) : a.pro == CTHIP_PRO_LAYERNORM ? PICK(CTHIP_PRO_LAYERNORM) : PICK(CTHIP_PRO_NONE);
+#define PICK(PRO, CENTRED) (nt ? k_gemv_int<PRO, CENTRED, true> : k_gemv_int<PRO, CENTRED, false>)
+  int_fn fn = a.pro == CTHIP_PRO_RMSNORM ? PICK(CTHIP_PRO_RMSNORM, false) : a.pro != CTHIP_PRO_LAYERNORM ? PICK(CTHIP_PRO_NONE, false)
+              : centred ? PICK(CTHIP_PRO_LAYERNORM, true) : PICK(CTHIP_PRO_LAYERNORM, false);
 #undef PICK
   if (p.lds > 64 * 1024) {
     CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvIntMaxLdsBytes));

@@ -53,6 +53,22 @@ def test_linear(ops, kind, rows, cols):
     w.free()
 
 
+# A folded LayerNorm with no bias of its own takes the mean off the vector: integers about a mean whose sums are exact in fp32 in any order, so that the error
+# is that of the product however many deviations the mean is (taken off behind the product: that many times as much, 1e-4 at the last).
+@pytest.mark.parametrize("kind,rows,cols", [("q4_0", 6500, 1280), ("q4_0", 20011, 1600), ("q4_0", 2600, 4096), ("q4_0", 2575, 1088)])
+def test_a_mean_of_many_deviations(ops, kind, rows, cols):
+    w, wd, rng = matrix(ops, kind, rows, cols, rows + cols)
+    g, beta = rng.normal(1, 0.1, cols).astype(np.float32), rng.normal(0, 0.1, cols).astype(np.float32)
+    w.fold_layernorm(g, beta)
+    d = rng.integers(-3, 4, cols // 2)
+    d = rng.permutation(np.concatenate([d, -d])).astype(np.float64)
+    want = wd @ (d / np.sqrt((d * d).mean() + 1e-5) * g + beta)
+    for mean in (0, -64, 2047):  # 2047 x 4096 < 2^23
+        got = w.linear_folded((mean + d).astype(np.float32))
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want), mean
+    w.free()
+
+
 @pytest.mark.parametrize("kind,rows,cols", [("q4_0", 2600, 1024)])
 @pytest.mark.parametrize("scale", [1e-38, 1e-37, 1e-35, 1e-33, 1e-30, 1e-12, 1e12, 1e30, 1e36])
 def test_inputs_of_any_magnitude(ops, kind, rows, cols, scale):
