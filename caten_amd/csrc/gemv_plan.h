@@ -256,6 +256,26 @@ inline GemvIntPlan gemv_int_plan(int type, long long rows, long long cols, int c
   p.ok = p.lds <= kGemvIntMaxLdsBytes;
   return p;
 }
+// Where that kernel is the faster one.  It goes over groups of 16 rows in rounds of one (long rows) or two to a compute unit; the vector kernels spread any number of
+// rows over their wavefronts, and multiply rows that fill their lanes at the rate that the weights arrive.  us, vector / integer, matrices out of memory:
+//   most sizes                          12288 x 4096 9.9 / 8.5, 22016 x 4096 13.9 / 12.6, 4096 x 11008 12.5 / 10.5, 50257 x 1280 13.8 / 9.3, 32000 x 8192 39.4 / 35.0
+//   rows under 5/8 of a round           2048 x 2048 4.3 / 4.3, 2048 x 4096 5.1 / 5.4, 1536 x 6144 6.4 / 6.4 (2304 x 4096 5.7 / 5.5: what lies between is not looked at)
+//   a quarter of a second round         4608 x 4096 6.5 / 7.3, 4352 x 2560 5.8 / 6.1, 4864 x 5120 7.6 / 8.0, 4608 x 8192 11.9 / 12.4 (no less at 4608 x 6656 11.0 / 9.6)
+//   3072 .. 4096 columns, while the vector kernels' rows fit one more of their rounds
+//                                       7168 x 3584 6.9 / 7.2, 9216 x 4096 8.2 / 8.6; past that 7936 x 3584 7.4 / 7.4, 9728 x 4096 9.2 / 8.8
+//   4608 .. 6144 columns (10 .. 12 wavefronts, the others' places empty), from 3584 on rows that are no whole units: a last round that is less than half full
+//                                       13312 x 5760 13.2 / 14.0, 9216 x 6144 11.3 / 12.4, 50257 x 5632 33.2 / 35.2, 9216 x 3968 8.1 / 9.1;
+//                                       full ones 12288 x 6144 13.1 / 12.3, 14336 x 5120 13.6 / 13.0
+//   9728 .. 10240 columns               14 wavefronts of 42 units for 40 against five whole steps of gemv_wide.hip: 5120 x 10240 15.3 / 16.6, 9216 x 10240 21.5 / 22.4
+inline bool gemv_int_pays(long long rows, long long cols, int compute_units) {
+  const long long round = 16ll * compute_units, last = rows % round;
+  if (8 * rows < 5 * round || cols > 16384) return false;
+  if (rows <= round) return true;
+  if (4 * rows <= 5 * round && ((cols > 2304 && cols <= 6144) || cols == 8192)) return false;
+  if (cols > 3072 && cols <= 4096 && 16 * rows <= (cols > 3584 ? 37 : 29) * round) return false;
+  if (cols > 3584 && cols <= 6144 && (cols > 4608 || cols % 256) && rows > 2 * round && last > 0 && 2 * last < round) return false;
+  return !(cols > 9728 && cols <= 10240);
+}
 
 // How the split-K reduction + norm pass (rowops.hip) lays a row out: `wide` = four wavefronts per row instead of
 // one; `vpl` = the float4-per-lane count of the kernel instantiation chosen (one of 1,2,3,4,6,8 narrow / 1,2,4,8

@@ -410,13 +410,9 @@ static bool gemv_prefers_wide(const GemvVariant *v, int type, int64_t rows) {
   const int opt = state().gemv_wide;
   return opt && (!v || heavy || opt >= 2);
 }
-// The integer kernel (gemv_int.hip), us against what was there: 12288 x 4096 10.2 -> 8.6, 22016 x 4096 14.4 -> 13.2, 4096 x 4096 6.3 -> 6.1, 4096 x 11008 12.6 -> 10.1,
-// 32000 x 4096 18.4 -> 16.6, 50257 x 1280 14.4 -> 9.6, 5120 x 1280 5.5 -> 4.7, 2560 x 2048 5.2 -> 4.4.  With fewer rows its groups of 16 leave compute
-// units idle (2048 x 5632 6.5 -> 6.7, 1280 x 1280 3.7 -> 3.9), as between one and two rounds of long rows (5120 x 5120 8.4 -> 8.7).
 static bool gemv_prefers_int(int type, int64_t rows, int64_t cols) {
-  if (state().gemv_wide != 1 || !gemv_int_plan(type, rows, cols, state().compute_units).ok) return false;
-  const int64_t round = 16ll * state().compute_units;  // rows
-  return rows >= 2560 && cols <= 16384 && !(cols > 4096 && cols <= 6144 && rows > round && rows < 2 * round);
+  const int cus = state().compute_units;
+  return state().gemv_wide == 1 && gemv_int_plan(type, rows, cols, cus).ok && gemv_int_pays(rows, cols, cus);
 }
 bool gemv_norm_out_ok(const WMat *w) {
   const GemvVariant *v = pick_variant(w->type, (int)w->cols);

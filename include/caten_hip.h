@@ -257,9 +257,11 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  *   held in registers; rows of up to 36 000 columns in any weight format, no LayerNorm prologue, no fused argmax): 0 = none
  *   (rows wider than the register-resident kernels cover go as column slices, one launch each), 1 (default) = the
  *   rows no register-resident kernel covers and those whose register-resident kernel runs one wavefront per SIMD
- *   (4-bit rows past 6144 columns, 8-bit rows past 4096) but for 4-bit matrices of 2560 rows and more, which go
- *   through integer matrix instructions (0 and 2 keep them out), 2 = every launch it supports.  Results differ between the kernel
- *   families only in summation order and rounding.
+ *   (4-bit rows past 6144 columns, 8-bit rows past 4096) but for most 4-bit matrices of 10 rows per compute unit and more
+ *   whose rows are a multiple of 64, 769 .. 16384 columns, which go through integer matrix instructions (gemv_int_pays in
+ *   caten_amd/csrc/gemv_plan.h says which; 0 and 2 keep them out), 2 = every launch it supports.  A session whose gate / up rows were laid out in
+ *   pairs for a launch that only the integer kernel has keeps that launch whatever the option says later.  Results differ between the kernel
+ *   families only in summation order and rounding; inputs with an infinity may give NaN in one family and an infinity in another.
  * "attn_split": 1 (default) = decoder sessions created afterwards that run one launch per Linear and have
  *   max_seq >= 512 share the keys of a head among (compute units / heads) workgroups, at most 16, in their decode
  *   attention (long contexts); 2 .. 16 = that many workgroups per head; 0 = one workgroup per head.  Same tokens;

@@ -29,7 +29,7 @@ def close(got, want, scale):
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("kind,rows,cols", [("q4_0", 2563, 1024), ("q4_0", 2575, 1088), ("q4_0", 4096, 4096), ("q4_0", 2560, 11008), ("q4_0", 8207, 4160), ("q4_0", 20011, 1600),
+@pytest.mark.parametrize("kind,rows,cols", [("q4_0", 2563, 1024), ("q4_0", 2575, 1088), ("q4_0", 4096, 4096), ("q4_0", 2560, 11008), ("q4_0", 8207, 4160), ("q4_0", 8207, 4352), ("q4_0", 20011, 1600),
                                             ("q4_0", 50257, 1280), ("q4_0", 2561, 1216), ("q4_0", 12288, 2048)])
 def test_linear(ops, kind, rows, cols):
     w, wd, rng = matrix(ops, kind, rows, cols, rows + cols)
