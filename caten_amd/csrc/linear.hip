@@ -659,7 +659,9 @@ int wmat_create_impl(WMat **out, int type, const void *raw, int64_t rows, int64_
     }
     CTHIP_CHECK(hipMemcpyAsync(w->q, raw, (size_t)w->q_bytes, hipMemcpyDeviceToDevice, s.stream));
   }
-  w->stream = w->q_bytes + w->d_bytes > kInfinityCacheBytes;  // cannot stay cached between two uses by itself
+  // cannot stay cached between two uses by itself, nor much of it: what the hint costs k_gemv_int is not won back (gemv_int.hip; 32000 x 16384, 295 MB, 64.2 us with
+  // it, 59.9 without, 50257 x 11008 75.7 / 67.4).  A session decides anew for its matrices together.
+  w->stream = w->stream_far = w->q_bytes + w->d_bytes > kInfinityCacheBytes;
   *out = w;
   return 0;
 }

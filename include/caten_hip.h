@@ -251,8 +251,8 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  * "gemm_bf16": 1 = shorthand for gemm_precision 1, 0 = back to the default.
  * "gemv_stream_weights": whether the single-row Linear kernels request the weights with the non-temporal
  *   hint: -1 (default) = per matrix -- a matrix larger than the 256 MB Infinity Cache, and every matrix of a
- *   decoder session whose weights together exceed three quarters of it; 0 = never; 1 = always.  Results do
- *   not depend on it.  A decoder session picks its kernels when it first runs.
+ *   decoder session whose weights together exceed three quarters of it (integer launches, "gemv_wide", only in sessions, up to
+ *   eight times that cache); 0 = never; 1 = always.  Results do not depend on it.  A decoder session picks its kernels when it first runs.
  * "gemv_wide": which single-row Linear launches take the wide-row kernel (input vector staged in LDS instead of
  *   held in registers; rows of up to 36 000 columns in any weight format, no LayerNorm prologue, no fused argmax): 0 = none
  *   (rows wider than the register-resident kernels cover go as column slices, one launch each), 1 (default) = the
