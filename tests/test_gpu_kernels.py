@@ -534,6 +534,26 @@ def test_sdpa_cached(ops, oracle, S, start, H, Hkv, Dh):
             _lib.check(lib.cthip_set_option(b"gemm_precision", 2))
 
 
+# 16 .. 31 rows of heads of 128: a row to a workgroup up to three (past 192 keys four) workgroups per compute unit, past that groups of eight rows up to 64 and over 129 .. 192
+# keys, 32 rows on the matrix cores with fp32 operands else.  Each adds up at most 128 products and T weighted values in some order, each sum within (n + 2) 2^-24 of its terms' magnitudes; scores of 128 normal products stay under 60 / sqrt(128), so that an
+# exponential is off by 130 * 2^-24 * 6 at the most.
+@pytest.mark.parametrize("S,H,Hkv", [(24, 32, 32), (31, 33, 33), (31, 34, 17), (16, 64, 8), (17, 64, 8), (16, 2, 1)])
+@pytest.mark.parametrize("start", [0, 33, 48, 120, 161, 162, 300])
+def test_sdpa_of_a_few_wide_rows(ops, S, H, Hkv, start):
+    print(f"case: sdpa_cached S={S} start={start} H={H}/{Hkv} Dh=128", flush=True)
+    rng = np.random.default_rng(S + start + H)
+    T = start + S
+    q, k, v = (rng.normal(size=(n, h, 128)).astype(np.float32) for n, h in ((S, H), (T, Hkv), (T, Hkv)))
+    k64, v64 = (np.repeat(a.astype(np.float64), H // Hkv, axis=1) for a in (k, v))
+    sc = np.einsum("shd,thd->hst", q.astype(np.float64), k64) / np.sqrt(128)
+    sc[:, np.arange(T)[None, :] > start + np.arange(S)[:, None]] = -np.inf
+    p = np.exp(sc - sc.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = np.einsum("hst,thd->shd", p, v64)
+    bound = (T + 2 + 2 * 130 * 6) * 2.0 ** -24 * np.einsum("hst,thd->shd", p, np.abs(v64))
+    assert np.all(np.abs(ops.sdpa_cached(q, k, v, start) - want) <= bound)
+
+
 # ------------------------------------------------------------------ matmul (MFMA)
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (64, 64, 32), (3, 5, 7), (65, 33, 17), (100, 768, 1024), (1, 64, 64),
                                    (128, 128, 64), (64, 128, 160), (70, 64, 128), (64, 192, 96),  # 2, 5, 4, 3 K-steps of 32
