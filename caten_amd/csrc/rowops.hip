@@ -668,13 +668,17 @@ template <int MODE>
 static int launch_rowop(RowArgs a) {
   if (a.rows == 0 || a.n == 0) return 0;
   hipStream_t st = state().stream;
-  if (a.n % 4 == 0 && a.n > 256 && a.n <= 2048 && ((uintptr_t)a.x % 16 == 0) && ((uintptr_t)a.y % 16 == 0) &&
+  // (softmax without a norm in front from 129 floats on: 200, 65 536 rows 16.3 us, 17.2 by the kernel below, 256 floats 20.1 / 20.5; of 128 14.6 / 11.3)
+  if (a.n % 4 == 0 && a.n > (MODE == ROW_SOFTMAX ? 128 : 256) && a.n <= 2048 && ((uintptr_t)a.x % 16 == 0) && ((uintptr_t)a.y % 16 == 0) &&
       (!a.g || (uintptr_t)a.g % 16 == 0) && (!a.b || (uintptr_t)a.b % 16 == 0)) {
     const int n4 = a.n / 4;
     const int vpl = (n4 + 63) / 64;
     if ((a.rows + 3) / 4 > 0x7fffffff) return fail(CTHIP_E_BAD_ARG, "row op: too many rows");
     dim3 grid((unsigned)((a.rows + 3) / 4)), block(256);
     switch (vpl) {
+      case 1:
+        if constexpr (MODE == ROW_SOFTMAX) hipLaunchKernelGGL((k_rowop<MODE, 1>), grid, block, 0, st, a);
+        break;
       case 2: hipLaunchKernelGGL((k_rowop<MODE, 2>), grid, block, 0, st, a); break;
       case 3: hipLaunchKernelGGL((k_rowop<MODE, 3>), grid, block, 0, st, a); break;
       case 4: hipLaunchKernelGGL((k_rowop<MODE, 4>), grid, block, 0, st, a); break;
@@ -688,7 +692,11 @@ static int launch_rowop(RowArgs a) {
   // Up to 256 floats whatever their alignment (65 536 rows: LayerNorm of 40 13.5 -> 5.2 us, of 87 50 -> 8.6, LayerNorm -> softmax of 128 22.8 -> 12.6, RMSNorm of
   // 255 43 -> 20.7; 256 aligned 21.1 -> 20.3).  Longer ones that k_rowop cannot read: norms up to its 2048 (2047: 82.6 -> 76.6, 511: 58 -> 40), softmax up to
   // 1024 (LayerNorm -> softmax of 403 41.5 -> 31.5, of 1001 76 -> 73; of 2047 a block per row is better: 71.8, 78 this way).
-  if (a.n >= 4 && a.n <= (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM ? 2048 : 1024)) {
+  // A block per row where norms of more than 1280 (LayerNorm: 1536) floats are few: a wavefront's eight pieces of a row come one after the other (us, wavefront / block: RMSNorm
+  // 600 x 2047 3.7 / 3.3, 1300 x 1801 4.9 / 4.5, 2000 x 2047 6.2 / 5.6, 4000 x 2047 11.0 / 11.6, 1300 x 1201 3.9 / 3.8; LayerNorm 300 x 1801 3.4 / 3.1, 1000 x 2047 4.4 / 4.3,
+  // 1600 x 1801 5.4 / 5.7, 2500 x 1201 5.3 / 6.1).
+  const bool few_norms = (MODE == ROW_RMSNORM && a.n > 1280 && a.rows < 10ll * state().compute_units) || (MODE == ROW_LAYERNORM && a.n > 1536 && a.rows < 5ll * state().compute_units);
+  if (a.n >= 4 && a.n <= (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM ? 2048 : 1024) && !few_norms) {
     const int lpr = nc <= 16 ? 16 : nc <= 32 ? 32 : 64;
     // two passes of rows per wavefront where that leaves every SIMD eight wavefronts (65 536 rows of 255: 26 -> 20.9 us)
     const int64_t once = (int64_t)(64 / lpr) * 4, full = 8ll * state().compute_units;
@@ -733,6 +741,7 @@ static int launch_rowop(RowArgs a) {
   if constexpr (MODE == ROW_LAYERNORM || MODE == ROW_RMSNORM) {
 #define NORM_BLOCK(VPL) hipLaunchKernelGGL((k_norm_block<MODE, VPL>), grid, dim3(256), 0, st, a)
     if (a.n < 4) hipLaunchKernelGGL((k_rowop_generic<MODE>), grid, dim3(256), 0, st, a);
+    else if (a.n <= 2048) NORM_BLOCK(8);
     else if (a.n <= 4096) NORM_BLOCK(16);
     else if (a.n <= 8192) NORM_BLOCK(32);
     else if (a.n <= 16384) NORM_BLOCK(64);

@@ -31,6 +31,12 @@ def test_rows_of_any_length(ops, oracle, rows, n):
     close(ops.layernorm_softmax(x, g, b), oracle.softmax(oracle.layernorm(x, g, b)), 1e-4, 1e-7)
 
 
+# where norms of more than 1280 / 1536 floats go from a block to a wavefront per row (ten / five rows to each of 256 compute units), and softmax of aligned rows to one
+@pytest.mark.parametrize("rows,n", [(1279, 1537), (1280, 1537), (1279, 1536), (2559, 1281), (2560, 1281), (2559, 2047), (2560, 2046), (7, 128), (7, 132), (7, 256), (6, 260)])
+def test_either_side_of_a_row_count(ops, oracle, rows, n):
+    test_rows_of_any_length(ops, oracle, rows, n)
+
+
 @pytest.mark.parametrize("rows,n", [(3, 1025), (2, 8193), (1, 32769), (3, 50257), (49, 32769), (1, 65541), (2, 70001)])
 @pytest.mark.parametrize("masked", [-np.inf, np.finfo(np.float32).min])
 def test_softmax_of_masked_rows(ops, oracle, rows, n, masked):
