@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/caten_hip.h"
+#include "gemm_plan.h"
 
 namespace cthip {
 
@@ -249,14 +250,6 @@ int launch_embedding(float *out, const float *W, const float *idx_f, const int *
                      const float *W2, const int *pos, int max_pos);
 int launch_argmax(int64_t *out, const float *x, int64_t rows, int n, int *tok_out, int *pos, int64_t *history,
                   int *hist_n);
-// Linear over m rows on the MFMA path (weights dequantised while staged).  precision: fp32 MFMA operands,
-// operands rounded to bf16, or operands split in two / three bf16 terms (2^-16 / fp32-grade).
-enum { GEMM_FP32 = 0, GEMM_BF16 = 1, GEMM_BF16X3 = 2, GEMM_BF16X6 = 3 };
-struct TilePlan {
-  int ks;     // workgroups that share the reduction axis
-  double us;  // estimate
-};
-TilePlan tile_plan(int M, int N, int K, int precision, bool quant, bool aligned, bool deferred);  // what launch_gemm makes of a product (matmul.hip)
 // A split-K launch whose reduction the caller takes over (launch_reduce_norm): the raw partial tiles ws[z][m][n]
 struct GemmDeferred {
   float *ws = nullptr;  // null: the launch did not split K, y is complete

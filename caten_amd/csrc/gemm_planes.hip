@@ -527,7 +527,7 @@ bool matmul_planes_pay(int M, int N, int K, int precision) {
   const int terms = plane_terms(precision);
   const bool aligned = K % 4 == 0 && N % 4 == 0;
   const double us = planes_us(M, N, K, terms, terms, false, ((double)M + N) * K * (4 + 2 * terms)), out = 4e-6 * M * N;
-  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, false, aligned, false).us;
+  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, false, false, aligned, false, state().compute_units).us;
 }
 
 // ---- Linears over many rows ----
@@ -644,7 +644,7 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   // (fp16 weights: half the bytes, which shows in a few rounds of tiles)
   const bool few_half = w->type == CTHIP_F16 && (int64_t)((m + 63) / 64) * ((w->rows + 63) / 64) <= 4 * state().compute_units;
   return planes_us(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes) * 1.04 <
-         tile_plan(m, (int)w->rows, (int)w->cols, precision, is_quant(w), true, false).us * (few_half ? 0.92 : 1.0);
+         tile_plan(m, (int)w->rows, (int)w->cols, precision, true, is_quant(w), true, false, state().compute_units).us * (few_half ? 0.92 : 1.0);
 }
 // ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {

@@ -1182,41 +1182,6 @@ int matmul_scratch_init(int device) {
   return 0;
 }
 
-// How many workgroups share the reduction axis of a tile, and what the launch (with the one that adds the shares up) then takes, in microseconds:
-// per round of tiles over an XCD a start and a time per step of 64, plus, where shares are added, a launch and their bytes (`deferred`: the bytes; the
-// next launch adds them on its way).  Fitted to 1 .. 8 shares of 20 shapes from (20, 232, 144) to (512, 2048, 5632), to which it keeps
-// within 15 %.  Two workgroups per compute unit of a tile, which filled the chip and was the rule before, took for 700^3 at two terms 14.0 us
-// (one share: 9.8), 512^3 9.3 (8.2), 400 x 2304 x 768 Q8_0 24 (14: shares that an XCD has no room for), 70 x 1280 x 5120 23 (15).
-TilePlan tile_plan(int M, int N, int K, int precision, bool quant, bool aligned, bool deferred) {
-  struct Cost {
-    double start, step, unaligned;            // one round
-    double start_n, step_n, unaligned_n;      // several: every compute unit at work
-  };
-  static const Cost costs[7] = {{1.0, 1.22, 1.55, 1.1, 1.05, 1.20}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64},
-                                {1.6, 0.85, 1.10, 3.0, 0.88, 0.98}, {2.0, 0.55, 0.55, 2.0, 0.66, 0.66}, {2.0, 0.72, 0.72, 2.0, 0.87, 0.87},
-                                {2.0, 0.90, 0.90, 2.0, 1.10, 1.10}};  // k_gemm_f32pc; k_gemm_split, one .. three terms; k_gemm_qpc, one .. three
-  const Cost &c = costs[precision == GEMM_FP32 ? 0 : (quant ? 3 : 0) + (precision == GEMM_BF16 ? 1 : precision == GEMM_BF16X3 ? 2 : 3)];
-  const bool two = !quant && precision != GEMM_BF16X6;  // workgroups on a compute unit
-  const int tm = (M + 63) / 64, tn = (N + (quant ? 127 : 63)) / (quant ? 128 : 64), nsteps = (K + 63) / 64;
-  int64_t most = (int64_t)tm * tn;  // tiles of an XCD
-  for (int rx = 1; rx <= 8; rx *= 2) most = std::min(most, (int64_t)((tm + rx - 1) / rx) * ((tn + 8 / rx - 1) / (8 / rx)));
-  TilePlan best = {1, 1e30};
-  for (int ks = 1; ks <= 16 && ks <= std::max(nsteps, 1); ks++) {
-    const int steps = (nsteps + ks - 1) / ks, shares = steps ? (nsteps + steps - 1) / steps : 1;
-    if (shares < ks) continue;  // the same steps as with fewer
-    const double n = (double)(most * shares) * 8.0 / state().compute_units;
-    // (shares of quantised tiles only where compute units are left for them: in a second round they gain 8 % at the most, 203 x 12288 x 4096 107 -> 98 us,
-    // and reorder the sums of a prompt, which a Q8_0 cache answers with other quants)
-    if (quant && shares > 1 && n > 1.0) break;
-    const double rounds = n <= 1.0 ? 1.0 : n <= 2.0 && two ? 1.85 : n <= 4.0 ? ceil(n) : 0.5 * ceil(2.0 * n);
-    const double tile = n <= 1.0 ? c.start + (aligned ? c.step : c.unaligned) * steps : c.start_n + (aligned ? c.step_n : c.unaligned_n) * steps;
-    const double sum = shares > 1 ? (deferred ? 0.3 : 2.6) + (deferred ? 0.6e-6 : 0.85e-6) * 4.0 * shares * M * N : 0.0;
-    const double us = 2.0 + rounds * tile + sum;
-    if (us < best.us) best = {ks, us};
-  }
-  return best;
-}
-
 // static_ws: null = split-K partials come from the caching allocator; otherwise they go to this buffer of
 // static_ws_bytes bytes and nothing is allocated or freed
 int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t static_ws_bytes, GemmDeferred *defer) {
@@ -1258,7 +1223,7 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
     // workgroup that computed them.)
     const int nsteps = (a.K + 63) / 64;  // K-steps of 64 (two of the fp32 kernel's)
     const bool aligned = a.K % 4 == 0 && (bmode == B_WMAT || a.N % 4 == 0);
-    int ks = a.pairs ? 1 : tile_plan(a.M, a.N, a.K, precision, quant, aligned, defer && !static_ws && a.act == CTHIP_ACT_NONE).ks;
+    int ks = a.pairs ? 1 : tile_plan(a.M, a.N, a.K, precision, bmode == B_WMAT, quant, aligned, defer && !static_ws && a.act == CTHIP_ACT_NONE, cus).ks;
     // (under graph capture no block is taken for shares: a replay would find it in other hands)
     if (ks > 1 && !static_ws && stream_capturing()) ks = 1;
     if (static_ws) {

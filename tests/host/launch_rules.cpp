@@ -1,7 +1,8 @@
-// The rules that choose between launches (caten_amd/csrc/gemv_plan.h) against times of both sides, taken on the card: where one side is 4 % faster or more the
+// The rules that choose between launches (caten_amd/csrc/gemv_plan.h, gemm_plan.h) against times of both sides, taken on the card: where one side is 4 % faster or more the
 // rule has to take it.  Exit status 1 and a line for every one that it does not.
 #include <stdio.h>
 
+#include "../../caten_amd/csrc/gemm_plan.h"
 #include "../../caten_amd/csrc/gemv_plan.h"
 
 using namespace cthip;
@@ -29,8 +30,44 @@ static void integer_gemv() {
   }
 }
 
+// shares of K of a product of packed weights on fp32 operands, us at 1, 2, 3, 4, 5, 6, 8, 10, 12, 16 of them (0: not timed): within 12 % of the best
+static void shares_of_fp32_tiles() {
+  static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
+  static const struct {
+    int m, rows, cols;
+    double us[10];
+  } t[] = {
+      {64, 11264, 2048, {73.7, 54.8, 51.7, 43.5, 48.6, 49.8, 49.1, 48.8, 53.6, 62.2}},  // f32
+      {64, 11264, 2048, {71.6, 56.5, 52.4, 43.9, 49.0, 49.3, 47.5, 47.6, 50.8, 54.1}},  // q8_0
+      {64, 4096, 4096, {133.6, 74.7, 54.9, 42.7, 42.1, 38.9, 32.4, 37.2, 34.7, 36.9}},  // f32
+      {24, 4800, 1600, {56.5, 33.7, 25.8, 22.8, 21.7, 21.5, 20.1, 21.1, 20.8, 23.8}},  // f32
+      {100, 1280, 5120, {162.9, 91.7, 65.2, 50.6, 40.7, 38.6, 37.2, 32.8, 30.4, 31.5}},  // q8_0
+      {48, 1600, 6400, {216.1, 113.3, 79.2, 60.0, 49.5, 43.3, 35.2, 36.3, 33.8, 29.0}},  // f32
+      {180, 768, 3072, {102.8, 57.7, 41.0, 32.9, 28.9, 30.2, 25.7, 24.1, 25.7, 23.4}},  // f32
+      {100, 2048, 2048, {69.7, 40.0, 30.6, 24.9, 25.3, 26.6, 21.4, 21.2, 23.6, 25.5}},  // q4_0
+      {256, 768, 768, {26.0, 17.8, 14.6, 13.6, 13.6, 14.4, 14.3, 14.3, 16.3, 0}},  // f16
+      {24, 2048, 5632, {154.3, 82.2, 58.1, 44.5, 37.4, 32.2, 25.6, 30.3, 27.8, 23.1}},  // f16
+      {700, 1024, 1024, {33.3, 32.0, 31.0, 27.4, 27.4, 31.4, 32.1, 31.9, 32.0, 37.8}},  // f32
+      {8, 1024, 4096, {125.8, 67.2, 48.1, 37.0, 31.7, 27.7, 22.2, 20.7, 19.0, 15.1}},  // q8_0
+  };
+  for (const auto &c : t) {
+    const int ks = tile_plan(c.m, c.rows, c.cols, GEMM_FP32, true, false, true, false, 256).ks, nsteps = (c.cols + 63) / 64;
+    double best = 1e30, got = 1e30;
+    for (int q = 0; q < 10; q++)
+      if (c.us[q] > 0) {
+        if (c.us[q] < best) best = c.us[q];
+        if ((nsteps + counts[q] - 1) / counts[q] == (nsteps + ks - 1) / ks && c.us[q] < got) got = c.us[q];
+      }
+    if (got == 1e30) continue;  // a count that was not timed
+    char what[96];
+    snprintf(what, sizeof(what), "%d shares of %d x %d x %d (%.1f against %.1f us)", ks, c.m, c.rows, c.cols, got, best);
+    expect(what, got <= 1.12 * best, true);
+  }
+}
+
 int main() {
   integer_gemv();
+  shares_of_fp32_tiles();
   printf("%d choices checked, %d wrong\n", g_checked, g_wrong);
   return g_wrong || !g_checked;
 }
