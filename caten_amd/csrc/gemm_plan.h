@@ -1,7 +1,11 @@
 // What launch_gemm (matmul.hip) makes of a product: kept apart from the kernels so that the CPU can check it (tests/host/launch_rules.cpp).
 #pragma once
+#include <stdint.h>
+
 #include <algorithm>
 #include <cmath>
+
+#include "../../include/caten_hip.h"
 
 namespace cthip {
 
@@ -50,6 +54,86 @@ inline TilePlan tile_plan(int M, int N, int K, int precision, bool packed, bool 
     if (us < best.us) best = {ks, us};
   }
   return best;
+}
+
+// ---- products whose operands lie in planes of bf16 terms (gemm_planes.hip) ----
+inline int plane_terms(int precision) { return precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1; }
+
+// Which tile: the one whose rounds over the chip cost least.  A compute unit holds `resident` workgroups; alone a workgroup
+// reaches `one`, together they reach `all` (TFLOP/s of results, measured at 1536^3, 2048^3 and 4096^3).
+struct PlaneTile {
+  int bm, bn, resident;
+  double one, all;
+  double idle = 1.0;  // share of a round's time that a single tile takes in the last one
+};
+inline double plane_tile_us(const PlaneTile &t, int M, int N, int nkb, int cus) {
+  const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), slots = (int64_t)cus * t.resident;
+  const double work = 2.0 * t.bm * t.bn * 32.0 * nkb * cus * 1e-6;  // MFLOP of a tile on every compute unit
+  const int64_t full = tiles / slots, left = tiles - full * slots;
+  double us = 2.0 + full * work * t.resident / t.all;
+  if (t.resident == 1) us += (double)M * N * 4e-7;  // nothing runs under the stores (4500 x 4500 x 600 at one term: 63 us in tiles of 128, 73 of 256)
+  if (left <= cus) {  // (large tiles are bound by power, the fewer of them the higher the clock; a few small ones start under the round before)
+    if (left) us += work / t.one * (full || t.resident == 1 ? t.idle + (1.0 - t.idle) * (double)left / cus : 1.0);
+  } else {  // between one tile per compute unit and a full round, steeper at the start: the shared units wait for both
+    const double one = work / t.one, all = work * t.resident / t.all;
+    us += one + (all - one) * (0.4 + 0.6 * (double)(left - cus) / (double)(slots - cus));
+  }
+  return us;
+}
+
+struct PlanePick {
+  int tile;   // of the list for the terms (planes_gemm)
+  double us;  // estimate of the launch
+};
+// nkb: blocks of 32 k; ints_b: B is one plane of integers with scales
+inline PlanePick plane_pick(int M, int N, int nkb, int terms, bool ints_b, int cus) {
+  // one term: 4096^3 in tiles of 64 x 64 .. 256 x 256 337, 265, 209, 202, 160 us, 2048^3 56, 49, 45, 46, 72, 1536^3 34, 36, 37, 39, 61
+  static const PlaneTile plane1[] = {{64, 64, 2, 330, 480, 0.5}, {128, 64, 3, 400, 650}, {128, 128, 2, 600, 880}, {128, 128, 2, 600, 922}, {256, 256, 1, 1290, 1290, 0.76}};
+  // two: 4096^3 580, 428, 376, 357, 346 us, 2048^3 81, 70, 69, 77, 137, 1536^3 45, 47, 51, 55, 109
+  static const PlaneTile plane[] = {{64, 64, 2, 200, 275, 0.5}, {128, 64, 3, 230, 365}, {128, 128, 2, 353, 438}, {128, 128, 2, 307, 469}, {256, 256, 1, 490, 490, 0.76}};
+  // three: 3000 x 4100 x 5000 883, 795, 732, 4096^3 1026, 861, 655
+  static const PlaneTile plane6[] = {{64, 64, 3, 110, 160}, {128, 64, 2, 110, 170}, {128, 256, 1, 205, 205, 0.6}};
+  static const PlaneTile ints[] = {{64, 64, 4, 240, 245}, {128, 128, 2, 370, 400}, {128, 192, 2, 368, 430}};
+  const PlaneTile *tiles = ints_b ? ints : terms == 3 ? plane6 : terms == 2 ? plane : plane1;
+  const int n = ints_b || terms == 3 ? 3 : 5;
+  PlanePick best = {0, 1e30};
+  for (int i = 0; i < n; i++) {
+    const double t = plane_tile_us(tiles[i], M, N, nkb, cus);
+    if (t < best.us) best = {i, t};
+  }
+  return best;
+}
+
+// Microseconds of a product (M, N, K) through planes: two passes over the operands (about 4.2 TB/s; none for operands that
+// lie in planes already) and a denser GEMM.
+inline double planes_us(int M, int N, int K, int terms, bool ints_b, double pass_bytes, int cus) {
+  if ((int64_t)((K + 31) / 32) * 64 * 3 * 256 >= (1ll << 31)) return INFINITY;  // 32-bit offsets within a tile's rows
+  const double us = plane_pick(M, N, (K + 31) / 32, terms, ints_b, cus).us;
+  return (ints_b ? us * terms / 2.0 + 4.0 : us + 2.0) + (pass_bytes > 0 ? pass_bytes / 4.2e6 + 5.0 : 0.0);
+}
+
+// Measured from 1000^3 to 2300^3, from (4096, 4096, 128) to (2500, 600, 4000), at one to three terms, rows of whole 16-byte pieces or not: at such sizes, which the
+// caches hold, planes_us is off by what is put right here, and the rule misses the better one by at most 12 % in 86 of 87.
+inline bool matmul_planes_faster(int M, int N, int K, int precision, int cus) {
+  if (precision == GEMM_FP32 || M < 64 || N < 64 || K < 64) return false;
+  const int terms = plane_terms(precision);
+  const bool aligned = K % 4 == 0 && N % 4 == 0;
+  const double us = planes_us(M, N, K, terms, false, ((double)M + N) * K * (4 + 2 * terms), cus), out = 4e-6 * M * N;
+  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, false, false, aligned, false, cus).us;
+}
+
+// The same for a Linear over weights (N, K).  planes_us and tile_plan are each off by what depends on the format: an integer or a half weight is fewer bytes for the tiles and one plane or
+// two for the products, an fp32 one is split by every tile.  One ratio each, and planes no faster than 2.5 TB/s (64 rows of f16 22016 x 4096 112 us, in tiles 74), fitted to both sides of
+// 2332 products (64 .. 2048 rows over (96, 4096) .. (12288, 4096), one to three terms): mean loss against the faster side 0.0 - 0.7 %, above 10 % in 0 - 13 of 240 - 730 a class.  (With 1.04 for
+// all, 0.92 of it for a few tiles of fp16, 0.4 - 7 % and up to 63 of 242: f16 2560 x 2048 over 900 rows 54 us, now 44, f32 4096 x 4096 over 900 150 / 128, Q4_0 2560 x 2048 over 900
+// 57 / 47, f16 at three terms 2048 x 2048 over 700 57 / 42.)
+inline bool linear_planes_faster(int M, int N, int K, int precision, int type, double pass_bytes, int cus) {
+  static const double ratio[3][3] = {{0.68, 1.16, 1.08}, {0.82, 0.90, 0.90}, {0.86, 0.68, 1.0}};  // terms; fp32, fp16, integers
+  const int terms = plane_terms(precision);
+  const bool ints = type == CTHIP_Q8_0 || type == CTHIP_Q4_0;
+  const double plane_bytes = (double)N * ((K + 31) / 32) * 64 * (ints ? 1 : type == CTHIP_F16 && terms > 2 ? 2 : terms);
+  const double us = std::max(planes_us(M, N, K, terms, ints, pass_bytes, cus) * ratio[terms - 1][ints ? 2 : type == CTHIP_F16 ? 1 : 0], plane_bytes / 2.5e6);
+  return us < tile_plan(M, N, K, precision, true, ints, true, false, cus).us;
 }
 
 }  // namespace cthip

@@ -352,52 +352,10 @@ static int planes_launch(PlaneGemmArgs a) {
   return 0;
 }
 
-// Which tile: the one whose rounds over the chip cost least.  A compute unit holds `resident` workgroups; alone a workgroup
-// reaches `one`, together they reach `all` (TFLOP/s of results, measured at 1536^3, 2048^3 and 4096^3).
-struct PlaneTile {
-  int bm, bn, resident;
-  double one, all;
-  double idle = 1.0;  // share of a round's time that a single tile takes in the last one
-};
-static double plane_tile_us(const PlaneTile &t, const PlaneGemmArgs &a, int cus) {
-  const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn), slots = (int64_t)cus * t.resident;
-  const double work = 2.0 * t.bm * t.bn * 32.0 * a.nkb * cus * 1e-6;  // MFLOP of a tile on every compute unit
-  const int64_t full = tiles / slots, left = tiles - full * slots;
-  double us = 2.0 + full * work * t.resident / t.all;
-  if (t.resident == 1) us += (double)a.M * a.N * 4e-7;  // nothing runs under the stores (4500 x 4500 x 600 at one term: 63 us in tiles of 128, 73 of 256)
-  if (left <= cus) {  // (large tiles are bound by power, the fewer of them the higher the clock; a few small ones start under the round before)
-    if (left) us += work / t.one * (full || t.resident == 1 ? t.idle + (1.0 - t.idle) * (double)left / cus : 1.0);
-  } else {  // between one tile per compute unit and a full round, steeper at the start: the shared units wait for both
-    const double one = work / t.one, all = work * t.resident / t.all;
-    us += one + (all - one) * (0.4 + 0.6 * (double)(left - cus) / (double)(slots - cus));
-  }
-  return us;
-}
-
 // A x B^T for operands in planes.  terms: of A; a.bd non-null: B is one plane of integers with scales, else terms_b planes.
-// Returns the estimated microseconds instead when `estimate` is set.
-static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b, double *estimate) {
-  const int cus = state().compute_units;
+static int planes_gemm(const PlaneGemmArgs &a, int terms, int terms_b) {
   const bool q = a.bd != nullptr;
-  // one term: 4096^3 in tiles of 64 x 64 .. 256 x 256 337, 265, 209, 202, 160 us, 2048^3 56, 49, 45, 46, 72, 1536^3 34, 36, 37, 39, 61
-  static const PlaneTile plane1[] = {{64, 64, 2, 330, 480, 0.5}, {128, 64, 3, 400, 650}, {128, 128, 2, 600, 880}, {128, 128, 2, 600, 922}, {256, 256, 1, 1290, 1290, 0.76}};
-  // two: 4096^3 580, 428, 376, 357, 346 us, 2048^3 81, 70, 69, 77, 137, 1536^3 45, 47, 51, 55, 109
-  static const PlaneTile plane[] = {{64, 64, 2, 200, 275, 0.5}, {128, 64, 3, 230, 365}, {128, 128, 2, 353, 438}, {128, 128, 2, 307, 469}, {256, 256, 1, 490, 490, 0.76}};
-  // three: 3000 x 4100 x 5000 883, 795, 732, 4096^3 1026, 861, 655
-  static const PlaneTile plane6[] = {{64, 64, 3, 110, 160}, {128, 64, 2, 110, 170}, {128, 256, 1, 205, 205, 0.6}};
-  static const PlaneTile ints[] = {{64, 64, 4, 240, 245}, {128, 128, 2, 370, 400}, {128, 192, 2, 368, 430}};
-  const PlaneTile *tiles = q ? ints : terms == 3 ? plane6 : terms == 2 ? plane : plane1;
-  const int n = q || terms == 3 ? 3 : 5;
-  int pick = 0;
-  double us = 1e30;
-  for (int i = 0; i < n; i++) {
-    const double t = plane_tile_us(tiles[i], a, cus);
-    if (t < us) us = t, pick = i;
-  }
-  if (estimate) {
-    *estimate = q ? us * terms / 2.0 + 4.0 : us + 2.0;
-    return 0;
-  }
+  const int pick = plane_pick(a.M, a.N, a.nkb, terms, q, state().compute_units).tile;
 #define T(NPA, SRC, NPB, MB, NB, WM, WN) return planes_launch<NPA, SRC, NPB, MB, NB, WM, WN, 2>(a)
 #define T3(NPA, SRC, NPB, MB, NB, WM, WN) return planes_launch<NPA, SRC, NPB, MB, NB, WM, WN, 3>(a)
 #define TILES(NPA)                                  \
@@ -465,21 +423,6 @@ static void planes_operands(PlaneGemmArgs &a, int K, int terms, int terms_b) {
   a.apitch = a.nkb * 64 * terms;
   a.bpitch = a.nkb * 64 * terms_b;
 }
-static int plane_terms(int precision) { return precision == GEMM_BF16X6 ? 3 : precision == GEMM_BF16X3 ? 2 : 1; }
-
-// Microseconds of a product (M, N, K) through planes: two passes over the operands (about 4.2 TB/s; none for operands that
-// lie in planes already) and a denser GEMM.
-static double planes_us(int M, int N, int K, int terms, int terms_b, bool ints, double pass_bytes) {
-  if ((int64_t)((K + 31) / 32) * 64 * 3 * 256 >= (1ll << 31)) return INFINITY;  // 32-bit offsets within a tile's rows
-  PlaneGemmArgs a = {};
-  a.M = M, a.N = N;
-  planes_operands(a, K, terms, terms_b);
-  static const unsigned short dummy = 0;
-  a.bd = ints ? &dummy : nullptr;
-  double us = 0;
-  planes_gemm(a, terms, terms_b, &us);
-  return us + (pass_bytes > 0 ? pass_bytes / 4.2e6 + 5.0 : 0.0);
-}
 
 // C = act(A . B + bias) + residual with B (K, N) row-major.  *done stays false, and the caller takes the other path, where the
 // results do not lie on 16 bytes or there is no memory for the terms.
@@ -516,19 +459,11 @@ int launch_matmul_planes(float *C, const float *A, const float *B, int M, int N,
     if (e != hipSuccess) rc = fail((int)e, "gemm planes: launch -> %s", hipGetErrorString(e));
   }
   a.A = pa, a.B = pb;
-  if (!rc) rc = planes_gemm(a, terms, terms, nullptr);
+  if (!rc) rc = planes_gemm(a, terms, terms);
   const int rf = cthip_free(pa);  // stream-ordered: handed out again only to later work on this stream
   return rc ? rc : rf;
 }
-// Measured from 1000^3 to 2300^3, from (4096, 4096, 128) to (2500, 600, 4000), at one to three terms, rows of whole 16-byte pieces or not: at such sizes, which the
-// caches hold, planes_us is off by what is put right here, and the rule misses the better one by at most 12 % in 86 of 87.
-bool matmul_planes_pay(int M, int N, int K, int precision) {
-  if (precision == GEMM_FP32 || M < 64 || N < 64 || K < 64) return false;
-  const int terms = plane_terms(precision);
-  const bool aligned = K % 4 == 0 && N % 4 == 0;
-  const double us = planes_us(M, N, K, terms, terms, false, ((double)M + N) * K * (4 + 2 * terms)), out = 4e-6 * M * N;
-  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, false, false, aligned, false, state().compute_units).us;
-}
+bool matmul_planes_pay(int M, int N, int K, int precision) { return matmul_planes_faster(M, N, K, precision, state().compute_units); }
 
 // ---- Linears over many rows ----
 // A weight matrix as planes: one of integers for a quantised matrix (2 bytes per weight), two exact terms for fp16 (4).
@@ -641,10 +576,7 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   double bytes = 0.0;
   if (!weight_planes_kept(w, terms_b)) bytes = (double)w->q_bytes + weight_plane_bytes(w, terms_b);
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
-  // (fp16 weights: half the bytes, which shows in a few rounds of tiles)
-  const bool few_half = w->type == CTHIP_F16 && (int64_t)((m + 63) / 64) * ((w->rows + 63) / 64) <= 4 * state().compute_units;
-  return planes_us(m, (int)w->rows, (int)w->cols, terms, terms_b, is_quant(w), bytes) * 1.04 <
-         tile_plan(m, (int)w->rows, (int)w->cols, precision, true, is_quant(w), true, false, state().compute_units).us * (few_half ? 0.92 : 1.0);
+  return linear_planes_faster(m, (int)w->rows, (int)w->cols, precision, w->type, bytes, state().compute_units);
 }
 // ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {
@@ -694,7 +626,7 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
   *done = true;
   int rc = xplanes ? 0 : planes_rows<float>(tmp, x, m, K, K, terms);
   a.A = xplanes ? xplanes : tmp, a.B = pb;
-  if (!rc) rc = planes_gemm(a, terms, terms_b, nullptr);
+  if (!rc) rc = planes_gemm(a, terms, terms_b);
   cthip_free(tmp);  // stream-ordered: handed out again only to later work on this stream
   if (temp_b) cthip_free(const_cast<unsigned char *>(pb));
   else weight_planes_release(w);

@@ -65,9 +65,57 @@ static void shares_of_fp32_tiles() {
   }
 }
 
+// Linears over many rows, us: tiles that convert their operands, operands in planes (rows of the planes' passes that every call makes included)
+static void linears_over_many_rows() {
+  static const struct {
+    int precision, type, m, rows, cols;
+    double tiles, planes;
+  } t[] = {
+      {2, CTHIP_F16, 900, 2560, 2048, 54.0, 44.1},
+      {2, CTHIP_F16, 512, 4800, 1600, 44.1, 35.2},
+      {2, CTHIP_F16, 200, 2304, 768, 10.3, 15.9},
+      {2, CTHIP_F16, 300, 1024, 1024, 12.0, 19.8},
+      {2, CTHIP_F16, 400, 5632, 2048, 52.9, 42.1},
+      {2, CTHIP_F16, 200, 768, 3072, 13.5, 46.8},
+      {2, CTHIP_F32, 900, 4096, 4096, 150.3, 128.5},
+      {2, CTHIP_F32, 1600, 2048, 5632, 196.8, 146.1},
+      {2, CTHIP_F32, 300, 2048, 2048, 21.3, 43.0},
+      {2, CTHIP_F32, 2048, 768, 768, 18.3, 26.0},
+      {2, CTHIP_F32, 900, 5632, 2048, 116.0, 89.9},
+      {2, CTHIP_Q8_0, 1200, 5120, 1280, 64.0, 53.8},
+      {2, CTHIP_Q8_0, 300, 6400, 1600, 44.9, 37.6},
+      {2, CTHIP_Q8_0, 512, 768, 3072, 18.2, 35.4},
+      {2, CTHIP_Q4_0, 900, 2560, 2048, 57.0, 46.5},
+      {2, CTHIP_Q4_0, 300, 12288, 4096, 108.7, 131.9},
+      {2, CTHIP_Q4_0, 300, 1024, 4096, 19.3, 41.9},
+      {2, CTHIP_Q4_0, 300, 2048, 5632, 34.7, 55.3},
+      {1, CTHIP_F16, 512, 1024, 4096, 19.6, 48.7},
+      {1, CTHIP_F32, 512, 11264, 2048, 103.4, 63.9},
+      {1, CTHIP_F32, 300, 1280, 5120, 26.4, 54.7},
+      {1, CTHIP_Q8_0, 64, 12288, 4096, 29.5, 51.9},
+      {1, CTHIP_Q8_0, 300, 1600, 6400, 31.5, 51.0},
+      {3, CTHIP_F16, 700, 2048, 2048, 57.4, 42.2},
+      {3, CTHIP_F16, 200, 768, 768, 9.9, 16.9},
+      {3, CTHIP_F32, 2048, 3072, 3072, 304.5, 228.8},
+      {3, CTHIP_F32, 200, 1280, 1280, 14.8, 34.2},
+      {2, CTHIP_F16, 64, 22016, 4096, 73.5, 111.9},
+      {2, CTHIP_F16, 64, 12288, 4096, 39.8, 95.7}};
+  for (const auto &c : t) {
+    const bool ints = c.type == CTHIP_Q8_0 || c.type == CTHIP_Q4_0;
+    const int terms = plane_terms(c.precision), terms_b = ints ? 1 : c.type == CTHIP_F16 && terms > 2 ? 2 : terms;
+    const bool stay = ints || (c.type == CTHIP_F16 && terms_b == 2);  // (gemm_planes.hip: weight_planes_stay)
+    const double weights = (double)c.rows * c.cols;
+    const double bytes = (double)c.m * c.cols * (4 + 2 * terms) + (stay ? 0.0 : weights * (c.type == CTHIP_F16 ? 2 : 4) + weights * 2 * terms_b);
+    char what[96];
+    snprintf(what, sizeof(what), "planes for %d rows of type %d %d x %d, %d terms (%.1f against %.1f us)", c.m, c.type, c.rows, c.cols, terms, c.planes, c.tiles);
+    expect(what, linear_planes_faster(c.m, c.rows, c.cols, c.precision, c.type, bytes, 256), c.planes < c.tiles);
+  }
+}
+
 int main() {
   integer_gemv();
   shares_of_fp32_tiles();
+  linears_over_many_rows();
   printf("%d choices checked, %d wrong\n", g_checked, g_wrong);
   return g_wrong || !g_checked;
 }
