@@ -279,7 +279,7 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route, bool *done);
 // A Linear over many rows from operands in memory as bf16 terms (gemm_planes.hip): x as fp32 rows or already as planes of plane_terms(precision) terms, the
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
-bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in);
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt);
 // x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
 // Linear over 8 .. 64 rows that lie as operands of two terms (linear_few.hip)
 bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: there is a pass over the rows in front of it anyway

@@ -998,7 +998,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     auto linear = [&](float *y, const WMat *w, const float *in, int in_terms, const float *bias, const float *residual, int act, const GemmRoute *route,
                       bool out_terms, GemmDeferred *defer = nullptr) {
       if (in_terms == kTermsOperands) return launch_linear_few(y, w, in, R, bias, residual, act, route);
-      if (in_terms || (planes && linear_planes_pays(w, R, prec, false))) {
+      if (in_terms || (planes && linear_planes_pays(w, R, prec, false, true))) {
         bool taken = false;
         const int r = launch_linear_planes(out_terms ? nullptr : y, w, in_terms ? nullptr : in, in_terms ? (const unsigned char *)in : nullptr, R, bias,
                                            residual, act, prec, route, out_terms ? (unsigned char *)y : nullptr, &taken);

@@ -18,24 +18,24 @@ struct TilePlan {
 
 // How many workgroups share the reduction axis of a tile, and what the launch (with the one that adds the shares up) then takes, in microseconds:
 // per round of tiles over an XCD a start and a time per step of 64, plus, where shares are added, a launch and their bytes (`deferred`: the bytes; the
-// next launch adds them on its way).  Fitted to 1 .. 8 shares of 20 shapes from (20, 232, 144) to (512, 2048, 5632), to which it keeps
-// within 15 %.  Two workgroups per compute unit of a tile, which filled the chip and was the rule before, took for 700^3 at two terms 14.0 us
+// next launch adds them on its way).  Fitted to 1 .. 16 shares of 3800 products, from (16, 16, 100) to (1024, 12288, 4096): mean loss against the best share count 0.0 - 0.7 % a kernel,
+// above 10 % in at most 3 of 217.  Two workgroups per compute unit of a tile, which filled the chip and was the rule before, took for 700^3 at two terms 14.0 us
 // (one share: 9.8), 512^3 9.3 (8.2), 400 x 2304 x 768 Q8_0 24 (14: shares that an XCD has no room for), 70 x 1280 x 5120 23 (15).
-// packed: the second operand is a weight matrix, which fp32 operands meet in k_gemm_f32 (no staging wavefronts: a step of 64 is 1.8 us, of k_gemm_f32pc 1.2).  Its row
-// is fitted to 1 .. 16 shares of 1050 products, f32 / f16 / Q8_0 / Q4_0 weights of (96, 4096) .. (12288, 4096) over 8 .. 1024 rows: mean loss against the best
-// share count 1 %, above 10 % in 4; by k_gemm_f32pc's row 7.5 %, above 10 % in 326 (64 rows f32 11264 x 2048 74 us, now 43), by shares that fill the chip 12 %.
-inline TilePlan tile_plan(int M, int N, int K, int precision, bool packed, bool quant, bool aligned, bool deferred, int compute_units) {
+// weights: the type of a weight matrix as the second operand, -1 for row-major floats.  On fp32 operands weights run k_gemm_f32 (no staging wavefronts: a step of
+// 64 is 1.8 us, of k_gemm_f32pc 1.2; by that one's row 7.5 % lost, 64 rows of f32 11264 x 2048 74 us, now 43); at one term fp32 weights are the bytes that count.
+inline TilePlan tile_plan(int M, int N, int K, int precision, int weights, bool aligned, bool deferred, int compute_units) {
   struct Cost {
     double start, step, unaligned;            // one round
     double start_n, step_n, unaligned_n;      // several: every compute unit at work
   };
-  static const Cost costs[8] = {{1.0, 1.22, 1.55, 1.1, 1.05, 1.20}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64},
-                                {1.6, 0.85, 1.10, 3.0, 0.88, 0.98}, {2.0, 0.55, 0.55, 2.0, 0.66, 0.66}, {2.0, 0.72, 0.72, 2.0, 0.87, 0.87},
-                                {2.0, 0.90, 0.90, 2.0, 1.10, 1.10},   // k_gemm_f32pc; k_gemm_split, one .. three terms; k_gemm_qpc, one .. three
-                                {1.3, 1.78, 2.26, 0.95, 1.27, 1.45}};  // k_gemm_f32
-  const bool f32 = packed && precision == GEMM_FP32;
-  const Cost &c = costs[f32 ? 7 : precision == GEMM_FP32 ? 0 : (quant ? 3 : 0) + (precision == GEMM_BF16 ? 1 : precision == GEMM_BF16X3 ? 2 : 3)];
-  const bool two = !quant && precision != GEMM_BF16X6 && !f32;  // a second workgroup on a compute unit is that much of a round cheaper
+  static const Cost costs[9] = {{1.0, 1.22, 1.55, 1.1, 1.05, 1.20}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64}, {1.6, 0.85, 1.10, 3.0, 0.88, 0.98},
+                                {0.6, 0.70, 0.70, 3.6, 0.60, 0.60}, {2.0, 0.72, 0.72, 2.0, 0.87, 0.87}, {2.0, 0.90, 0.90, 2.0, 1.10, 1.10},
+                                {1.3, 1.78, 2.26, 0.95, 1.27, 1.45}, {0.8, 0.47, 0.47, 0.1, 0.48, 0.48}};
+  // k_gemm_f32pc; k_gemm_split, one .. three terms; k_gemm_qpc, one .. three; k_gemm_f32; k_gemm_split, one term, fp32 weights
+  const bool f32 = weights >= 0 && precision == GEMM_FP32, quant = !f32 && (weights == CTHIP_Q8_0 || weights == CTHIP_Q4_0);
+  const int terms = precision == GEMM_FP32 ? 0 : precision == GEMM_BF16 ? 1 : precision == GEMM_BF16X3 ? 2 : 3;
+  const Cost &c = costs[f32 ? 7 : quant ? 3 + terms : weights == CTHIP_F32 && terms == 1 ? 8 : terms];
+  const bool two = !quant && terms != 3 && !f32;  // a second workgroup on a compute unit is that much of a round cheaper
   const int tm = (M + 63) / 64, tn = (N + (quant ? 127 : 63)) / (quant ? 128 : 64), nsteps = (K + 63) / 64;
   int64_t most = (int64_t)tm * tn;  // tiles of an XCD
   for (int rx = 1; rx <= 8; rx *= 2) most = std::min(most, (int64_t)((tm + rx - 1) / rx) * ((tn + 8 / rx - 1) / (8 / rx)));
@@ -44,8 +44,8 @@ inline TilePlan tile_plan(int M, int N, int K, int precision, bool packed, bool 
     const int steps = (nsteps + ks - 1) / ks, shares = steps ? (nsteps + steps - 1) / steps : 1;
     if (shares < ks) continue;  // the same steps as with fewer
     const double n = (double)(most * shares) * 8.0 / compute_units;
-    // (shares of quantised tiles only where compute units are left for them: in a second round they gain 8 % at the most, 203 x 12288 x 4096 107 -> 98 us,
-    // and reorder the sums of a prompt, which a Q8_0 cache answers with other quants)
+    // (Quantised tiles: no shares past one round.  Over 868 products that loses nothing, mean loss 0.6 % with them and without, at single ones up to 8 %, 203 x 12288 x 4096 107 us / 98;
+    // and another order of a prompt's sums puts other quants into a Q8_0 cache, tokens a few steps on included.)
     if (quant && shares > 1 && n > 1.0) break;
     const double rounds = n <= 1.0 ? 1.0 : n <= 2.0 && two ? 1.85 : n <= 4.0 ? ceil(n) : 0.5 * ceil(2.0 * n);
     const double tile = n <= 1.0 ? c.start + (aligned ? c.step : c.unaligned) * steps : c.start_n + (aligned ? c.step_n : c.unaligned_n) * steps;
@@ -119,21 +119,29 @@ inline bool matmul_planes_faster(int M, int N, int K, int precision, int cus) {
   const int terms = plane_terms(precision);
   const bool aligned = K % 4 == 0 && N % 4 == 0;
   const double us = planes_us(M, N, K, terms, false, ((double)M + N) * K * (4 + 2 * terms), cus), out = 4e-6 * M * N;
-  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, false, false, aligned, false, cus).us;
+  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, -1, aligned, false, cus).us;
 }
 
 // The same for a Linear over weights (N, K).  planes_us and tile_plan are each off by what depends on the format: an integer or a half weight is fewer bytes for the tiles and one plane or
 // two for the products, an fp32 one is split by every tile.  One ratio each, and planes no faster than 2.5 TB/s (64 rows of f16 22016 x 4096 112 us, in tiles 74), fitted to both sides of
-// 2332 products (64 .. 2048 rows over (96, 4096) .. (12288, 4096), one to three terms): mean loss against the faster side 0.0 - 0.7 %, above 10 % in 0 - 13 of 240 - 730 a class.  (With 1.04 for
-// all, 0.92 of it for a few tiles of fp16, 0.4 - 7 % and up to 63 of 242: f16 2560 x 2048 over 900 rows 54 us, now 44, f32 4096 x 4096 over 900 150 / 128, Q4_0 2560 x 2048 over 900
-// 57 / 47, f16 at three terms 2048 x 2048 over 700 57 / 42.)
-inline bool linear_planes_faster(int M, int N, int K, int precision, int type, double pass_bytes, int cus) {
-  static const double ratio[3][3] = {{0.68, 1.16, 1.08}, {0.82, 0.90, 0.90}, {0.86, 0.68, 1.0}};  // terms; fp32, fp16, integers
+// 3220 products (64 .. 2048 rows over (96, 4096) .. (22016, 4096), one to three terms, matrices out of the cache and out of memory): mean loss against the faster side 0.0 - 1.1 % a class.
+// (With 1.04 for all, 0.92 of it for a few tiles of fp16, up to 7 %: fp32 4096 x 4096 over 900 rows 150 us, now 128, Q4_0 2560 x 2048 over 900 57 / 47, f16 at three terms
+// 2048 x 2048 over 700 57 / 42.)  fp16 at two terms is where cache and memory part, 4 bytes a weight against 2: 1280 x 5120 over 900 rows, tiles / planes, 65 / 78 us out of the
+// cache, 64 / 111 out of memory, 4800 x 1600 over 512 44 / 35 and 44 / 46; the ratio is right out of memory.
+// prompt: in a session's prompt the weights come out of memory, what is in front writes planes, and behind tiles a norm adds the shares up: the older ratios, which were
+// fitted there (by the others llama-1.1b f16 640 rows 5.4 -> 7.0 ms, q4_0 64 rows 1.63 -> 1.83, gpt2-medium q4_0 128 rows 1.50 -> 1.68).
+inline bool linear_planes_faster(int M, int N, int K, int precision, int type, double pass_bytes, bool prompt, int cus) {
+  static const double ratio[3][3] = {{0.84, 1.12, 1.20}, {0.84, 1.00, 0.88}, {0.84, 0.68, 1.0}};  // terms; fp32, fp16, integers
   const int terms = plane_terms(precision);
   const bool ints = type == CTHIP_Q8_0 || type == CTHIP_Q4_0;
-  const double plane_bytes = (double)N * ((K + 31) / 32) * 64 * (ints ? 1 : type == CTHIP_F16 && terms > 2 ? 2 : terms);
-  const double us = std::max(planes_us(M, N, K, terms, ints, pass_bytes, cus) * ratio[terms - 1][ints ? 2 : type == CTHIP_F16 ? 1 : 0], plane_bytes / 2.5e6);
-  return us < tile_plan(M, N, K, precision, true, ints, true, false, cus).us;
+  double us = planes_us(M, N, K, terms, ints, pass_bytes, cus);
+  if (prompt) {
+    us *= type == CTHIP_F16 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 4 * cus ? 1.13 : 1.04;
+  } else {
+    const double plane_bytes = (double)N * ((K + 31) / 32) * 64 * (ints ? 1 : type == CTHIP_F16 && terms > 2 ? 2 : terms);
+    us = std::max(us * ratio[terms - 1][ints ? 2 : type == CTHIP_F16 ? 1 : 0], plane_bytes / 2.5e6);
+  }
+  return us < tile_plan(M, N, K, precision, type, true, false, cus).us;
 }
 
 }  // namespace cthip

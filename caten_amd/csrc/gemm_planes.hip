@@ -568,7 +568,7 @@ void weight_planes_limit(int64_t bytes) {
   if (over) weight_planes_drop();
 }
 
-bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt) {
   if (precision == GEMM_FP32 || m < 64 || w->rows < 64 || w->cols < 64 || (!is_quant(w) && w->cols % 16)) return false;
   // (three terms against integers: registers for one 32-column block less per wavefront, no faster than the tiles)
   if (is_quant(w) && precision == GEMM_BF16X6) return false;
@@ -576,11 +576,11 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in) {
   double bytes = 0.0;
   if (!weight_planes_kept(w, terms_b)) bytes = (double)w->q_bytes + weight_plane_bytes(w, terms_b);
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
-  return linear_planes_faster(m, (int)w->rows, (int)w->cols, precision, w->type, bytes, state().compute_units);
+  return linear_planes_faster(m, (int)w->rows, (int)w->cols, precision, w->type, bytes, prompt, state().compute_units);
 }
 // ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {
-  return linear_planes_pays(w, m, precision, true) && weight_planes(w, weight_terms(w, plane_terms(precision)), nullptr);
+  return linear_planes_pays(w, m, precision, true, true) && weight_planes(w, weight_terms(w, plane_terms(precision)), nullptr);
 }
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
                          int precision, const GemmRoute *route, unsigned char *planes_out, bool *done) {

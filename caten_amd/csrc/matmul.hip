@@ -1223,7 +1223,7 @@ int launch_gemm(GemmArgs a, int bmode, int precision, float *static_ws, size_t s
     // workgroup that computed them.)
     const int nsteps = (a.K + 63) / 64;  // K-steps of 64 (two of the fp32 kernel's)
     const bool aligned = a.K % 4 == 0 && (bmode == B_WMAT || a.N % 4 == 0);
-    int ks = a.pairs ? 1 : tile_plan(a.M, a.N, a.K, precision, bmode == B_WMAT, quant, aligned, defer && !static_ws && a.act == CTHIP_ACT_NONE, cus).ks;
+    int ks = a.pairs ? 1 : tile_plan(a.M, a.N, a.K, precision, bmode == B_WMAT ? a.wtype : -1, aligned, defer && !static_ws && a.act == CTHIP_ACT_NONE, cus).ks;
     // (under graph capture no block is taken for shares: a replay would find it in other hands)
     if (ks > 1 && !static_ws && stream_capturing()) ks = 1;
     if (static_ws) {

@@ -30,28 +30,40 @@ static void integer_gemv() {
   }
 }
 
-// shares of K of a product of packed weights on fp32 operands, us at 1, 2, 3, 4, 5, 6, 8, 10, 12, 16 of them (0: not timed): within 12 % of the best
-static void shares_of_fp32_tiles() {
+// shares of K of a product of packed weights, us at 1, 2, 3, 4, 5, 6, 8, 10, 12, 16 of them (0: not timed): within 12 % of the best
+static void shares_of_tiles() {
   static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
   static const struct {
-    int m, rows, cols;
+    int precision, type, m, rows, cols;
     double us[10];
   } t[] = {
-      {64, 11264, 2048, {73.7, 54.8, 51.7, 43.5, 48.6, 49.8, 49.1, 48.8, 53.6, 62.2}},  // f32
-      {64, 11264, 2048, {71.6, 56.5, 52.4, 43.9, 49.0, 49.3, 47.5, 47.6, 50.8, 54.1}},  // q8_0
-      {64, 4096, 4096, {133.6, 74.7, 54.9, 42.7, 42.1, 38.9, 32.4, 37.2, 34.7, 36.9}},  // f32
-      {24, 4800, 1600, {56.5, 33.7, 25.8, 22.8, 21.7, 21.5, 20.1, 21.1, 20.8, 23.8}},  // f32
-      {100, 1280, 5120, {162.9, 91.7, 65.2, 50.6, 40.7, 38.6, 37.2, 32.8, 30.4, 31.5}},  // q8_0
-      {48, 1600, 6400, {216.1, 113.3, 79.2, 60.0, 49.5, 43.3, 35.2, 36.3, 33.8, 29.0}},  // f32
-      {180, 768, 3072, {102.8, 57.7, 41.0, 32.9, 28.9, 30.2, 25.7, 24.1, 25.7, 23.4}},  // f32
-      {100, 2048, 2048, {69.7, 40.0, 30.6, 24.9, 25.3, 26.6, 21.4, 21.2, 23.6, 25.5}},  // q4_0
-      {256, 768, 768, {26.0, 17.8, 14.6, 13.6, 13.6, 14.4, 14.3, 14.3, 16.3, 0}},  // f16
-      {24, 2048, 5632, {154.3, 82.2, 58.1, 44.5, 37.4, 32.2, 25.6, 30.3, 27.8, 23.1}},  // f16
-      {700, 1024, 1024, {33.3, 32.0, 31.0, 27.4, 27.4, 31.4, 32.1, 31.9, 32.0, 37.8}},  // f32
-      {8, 1024, 4096, {125.8, 67.2, 48.1, 37.0, 31.7, 27.7, 22.2, 20.7, 19.0, 15.1}},  // q8_0
+      {0, CTHIP_F32, 64, 11264, 2048, {73.7, 54.8, 51.7, 43.5, 48.6, 49.8, 49.1, 48.8, 53.6, 62.2}},
+      {0, CTHIP_Q8_0, 64, 11264, 2048, {71.6, 56.5, 52.4, 43.9, 49.0, 49.3, 47.5, 47.6, 50.8, 54.1}},
+      {0, CTHIP_F32, 64, 4096, 4096, {133.6, 74.7, 54.9, 42.7, 42.1, 38.9, 32.4, 37.2, 34.7, 36.9}},
+      {0, CTHIP_F32, 24, 4800, 1600, {56.5, 33.7, 25.8, 22.8, 21.7, 21.5, 20.1, 21.1, 20.8, 23.8}},
+      {0, CTHIP_Q8_0, 100, 1280, 5120, {162.9, 91.7, 65.2, 50.6, 40.7, 38.6, 37.2, 32.8, 30.4, 31.5}},
+      {0, CTHIP_F32, 48, 1600, 6400, {216.1, 113.3, 79.2, 60.0, 49.5, 43.3, 35.2, 36.3, 33.8, 29.0}},
+      {0, CTHIP_F32, 180, 768, 3072, {102.8, 57.7, 41.0, 32.9, 28.9, 30.2, 25.7, 24.1, 25.7, 23.4}},
+      {0, CTHIP_Q4_0, 100, 2048, 2048, {69.7, 40.0, 30.6, 24.9, 25.3, 26.6, 21.4, 21.2, 23.6, 25.5}},
+      {0, CTHIP_F16, 256, 768, 768, {26.0, 17.8, 14.6, 13.6, 13.6, 14.4, 14.3, 14.3, 16.3, 0}},
+      {0, CTHIP_F16, 24, 2048, 5632, {154.3, 82.2, 58.1, 44.5, 37.4, 32.2, 25.6, 30.3, 27.8, 23.1}},
+      {0, CTHIP_F32, 700, 1024, 1024, {33.3, 32.0, 31.0, 27.4, 27.4, 31.4, 32.1, 31.9, 32.0, 37.8}},
+      {0, CTHIP_Q8_0, 8, 1024, 4096, {125.8, 67.2, 48.1, 37.0, 31.7, 27.7, 22.2, 20.7, 19.0, 15.1}},
+      {1, CTHIP_Q4_0, 100, 3072, 1024, {14.2, 12.3, 12.2, 11.7, 11.7, 15.4, 16.1, 16.0, 16.1, 22.2}},
+      {1, CTHIP_Q4_0, 150, 2048, 1024, {14.2, 11.7, 11.0, 10.1, 10.1, 12.7, 13.1, 13.0, 13.0, 16.7}},
+      {1, CTHIP_Q4_0, 300, 1024, 1024, {14.2, 12.4, 12.2, 11.8, 11.8, 12.7, 16.5, 16.5, 16.5, 20.6}},
+      {1, CTHIP_Q4_0, 66, 12288, 4096, {44.6, 51.3, 53.3, 45.3, 49.9, 53.5, 54.9, 63.4, 69.0, 78.8}},
+      {2, CTHIP_Q8_0, 100, 1280, 5120, {57.6, 34.0, 25.9, 21.5, 19.5, 18.3, 16.3, 16.1, 23.6, 20.7}},
+      {2, CTHIP_Q8_0, 512, 768, 768, {11.7, 12.1, 11.6, 11.8, 11.8, 16.5, 16.4, 16.4, 21.7, 0}},
+      {2, CTHIP_F16, 100, 1024, 4096, {33.6, 21.1, 16.8, 14.2, 13.1, 12.5, 12.0, 15.1, 14.6, 14.1}},
+      {2, CTHIP_F16, 300, 2048, 2048, {19.2, 21.9, 19.1, 21.0, 22.0, 22.4, 23.2, 23.3, 28.1, 31.9}},
+      {1, CTHIP_F32, 200, 1280, 1280, {13.9, 12.0, 11.4, 13.0, 13.2, 13.2, 15.1, 16.4, 16.4, 16.4}},
+      {1, CTHIP_F32, 80, 2048, 1024, {9.7, 9.0, 8.6, 8.1, 8.2, 9.9, 8.9, 9.0, 8.9, 12.7}},
+      {3, CTHIP_F32, 150, 2048, 5632, {69.1, 41.4, 54.2, 44.6, 39.4, 46.8, 40.5, 46.5, 50.4, 50.0}},
+      {3, CTHIP_Q4_0, 100, 2048, 1024, {18.5, 14.1, 12.8, 11.5, 11.5, 11.2, 10.6, 10.6, 10.5, 15.9}},
   };
   for (const auto &c : t) {
-    const int ks = tile_plan(c.m, c.rows, c.cols, GEMM_FP32, true, false, true, false, 256).ks, nsteps = (c.cols + 63) / 64;
+    const int ks = tile_plan(c.m, c.rows, c.cols, c.precision, c.type, true, false, 256).ks, nsteps = (c.cols + 63) / 64;
     double best = 1e30, got = 1e30;
     for (int q = 0; q < 10; q++)
       if (c.us[q] > 0) {
@@ -59,23 +71,20 @@ static void shares_of_fp32_tiles() {
         if ((nsteps + counts[q] - 1) / counts[q] == (nsteps + ks - 1) / ks && c.us[q] < got) got = c.us[q];
       }
     if (got == 1e30) continue;  // a count that was not timed
-    char what[96];
-    snprintf(what, sizeof(what), "%d shares of %d x %d x %d (%.1f against %.1f us)", ks, c.m, c.rows, c.cols, got, best);
+    char what[128];
+    snprintf(what, sizeof(what), "%d shares of %d x %d x %d, type %d, operands %d (%.1f against %.1f us)", ks, c.m, c.rows, c.cols, c.type, c.precision, got, best);
     expect(what, got <= 1.12 * best, true);
   }
 }
 
-// Linears over many rows, us: tiles that convert their operands, operands in planes (rows of the planes' passes that every call makes included)
+// Linears over many rows (fp16 at two terms: out of memory), us: tiles that convert their operands, operands in planes (rows of the planes' passes that every call makes included)
 static void linears_over_many_rows() {
   static const struct {
     int precision, type, m, rows, cols;
     double tiles, planes;
   } t[] = {
-      {2, CTHIP_F16, 900, 2560, 2048, 54.0, 44.1},
-      {2, CTHIP_F16, 512, 4800, 1600, 44.1, 35.2},
       {2, CTHIP_F16, 200, 2304, 768, 10.3, 15.9},
       {2, CTHIP_F16, 300, 1024, 1024, 12.0, 19.8},
-      {2, CTHIP_F16, 400, 5632, 2048, 52.9, 42.1},
       {2, CTHIP_F16, 200, 768, 3072, 13.5, 46.8},
       {2, CTHIP_F32, 900, 4096, 4096, 150.3, 128.5},
       {2, CTHIP_F32, 1600, 2048, 5632, 196.8, 146.1},
@@ -99,7 +108,12 @@ static void linears_over_many_rows() {
       {3, CTHIP_F32, 2048, 3072, 3072, 304.5, 228.8},
       {3, CTHIP_F32, 200, 1280, 1280, 14.8, 34.2},
       {2, CTHIP_F16, 64, 22016, 4096, 73.5, 111.9},
-      {2, CTHIP_F16, 64, 12288, 4096, 39.8, 95.7}};
+      {2, CTHIP_F16, 64, 12288, 4096, 39.8, 95.7},
+      {2, CTHIP_F16, 900, 1280, 5120, 64.0, 111.0},
+      {2, CTHIP_F16, 640, 2048, 5632, 74.0, 122.0},
+      {2, CTHIP_F16, 640, 11264, 2048, 123.1, 87.4},
+      {2, CTHIP_F16, 1500, 4800, 1600, 107.1, 73.7},
+      {2, CTHIP_F16, 640, 4800, 1600, 45.4, 51.9}};
   for (const auto &c : t) {
     const bool ints = c.type == CTHIP_Q8_0 || c.type == CTHIP_Q4_0;
     const int terms = plane_terms(c.precision), terms_b = ints ? 1 : c.type == CTHIP_F16 && terms > 2 ? 2 : terms;
@@ -108,13 +122,13 @@ static void linears_over_many_rows() {
     const double bytes = (double)c.m * c.cols * (4 + 2 * terms) + (stay ? 0.0 : weights * (c.type == CTHIP_F16 ? 2 : 4) + weights * 2 * terms_b);
     char what[96];
     snprintf(what, sizeof(what), "planes for %d rows of type %d %d x %d, %d terms (%.1f against %.1f us)", c.m, c.type, c.rows, c.cols, terms, c.planes, c.tiles);
-    expect(what, linear_planes_faster(c.m, c.rows, c.cols, c.precision, c.type, bytes, 256), c.planes < c.tiles);
+    expect(what, linear_planes_faster(c.m, c.rows, c.cols, c.precision, c.type, bytes, false, 256), c.planes < c.tiles);
   }
 }
 
 int main() {
   integer_gemv();
-  shares_of_fp32_tiles();
+  shares_of_tiles();
   linears_over_many_rows();
   printf("%d choices checked, %d wrong\n", g_checked, g_wrong);
   return g_wrong || !g_checked;
