@@ -30,7 +30,7 @@ inline TilePlan tile_plan(int M, int N, int K, int precision, int weights, bool 
   };
   static const Cost costs[9] = {{1.0, 1.22, 1.55, 1.1, 1.05, 1.20}, {1.7, 0.37, 0.73, 1.15, 0.37, 0.50}, {1.2, 0.57, 0.86, 1.2, 0.53, 0.64}, {1.6, 0.85, 1.10, 3.0, 0.88, 0.98},
                                 {0.6, 0.70, 0.70, 3.6, 0.60, 0.60}, {2.0, 0.72, 0.72, 2.0, 0.87, 0.87}, {2.0, 0.90, 0.90, 2.0, 1.10, 1.10},
-                                {1.3, 1.78, 2.26, 0.95, 1.27, 1.45}, {0.8, 0.47, 0.47, 0.1, 0.48, 0.48}};
+                                {1.3, 1.78, 2.26, 0.95, 1.27, 1.45}, {0.55, 0.48, 0.48, 0.1, 0.48, 0.48}};
   // k_gemm_f32pc; k_gemm_split, one .. three terms; k_gemm_qpc, one .. three; k_gemm_f32; k_gemm_split, one term, fp32 weights
   const bool f32 = weights >= 0 && precision == GEMM_FP32, quant = !f32 && (weights == CTHIP_Q8_0 || weights == CTHIP_Q4_0);
   const int terms = precision == GEMM_FP32 ? 0 : precision == GEMM_BF16 ? 1 : precision == GEMM_BF16X3 ? 2 : 3;
@@ -112,14 +112,16 @@ inline double planes_us(int M, int N, int K, int terms, bool ints_b, double pass
   return (ints_b ? us * terms / 2.0 + 4.0 : us + 2.0) + (pass_bytes > 0 ? pass_bytes / 4.2e6 + 5.0 : 0.0);
 }
 
-// Measured from 1000^3 to 2300^3, from (4096, 4096, 128) to (2500, 600, 4000), at one to three terms, rows of whole 16-byte pieces or not: at such sizes, which the
-// caches hold, planes_us is off by what is put right here, and the rule misses the better one by at most 12 % in 86 of 87.
+// At sizes that the caches hold planes_us is off by what is put right here: fitted to both sides of 2280 products, a third of them with fewer than 500 k, from (200, 200, 64) to
+// (5000, 5000, 5000), at one to three terms, rows of whole 16-byte pieces or not: mean loss against the faster side 0.5 - 0.7 %, above 10 % in 55.  (0.8 us + 8 and a sixth of the time that the
+// result's bytes take, 4 % on top, whatever the terms: 0.5 - 1.8 %, 103; 3338 x 3584 x 116 at one term 27 us, now 21, 4452 x 2292 x 292 at three 83, now 70.)
 inline bool matmul_planes_faster(int M, int N, int K, int precision, int cus) {
   if (precision == GEMM_FP32 || M < 64 || N < 64 || K < 64) return false;
   const int terms = plane_terms(precision);
   const bool aligned = K % 4 == 0 && N % 4 == 0;
   const double us = planes_us(M, N, K, terms, false, ((double)M + N) * K * (4 + 2 * terms), cus), out = 4e-6 * M * N;
-  return (aligned ? 0.8 * us + 8.0 + out / 6.0 : 0.9 * us + 10.0 + out / 4.2) * 1.04 < tile_plan(M, N, K, precision, -1, aligned, false, cus).us;
+  const double planes = aligned ? 0.83 * us + 8.0 : terms == 3 ? 0.95 * us + 8.0 : 0.94 * us + 10.4 + out / 4.0;
+  return planes < tile_plan(M, N, K, precision, -1, aligned, false, cus).us;
 }
 
 // The same for a Linear over weights (N, K).  planes_us and tile_plan are each off by what depends on the format: an integer or a half weight is fewer bytes for the tiles and one plane or

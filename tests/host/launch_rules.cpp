@@ -126,10 +126,46 @@ static void linears_over_many_rows() {
   }
 }
 
+// matrix products, us: tiles that convert their operands, operands in planes with the passes that make them
+static void matrix_products() {
+  static const struct {
+    int precision, m, n, k;
+    double tiles, planes;
+  } t[] = {
+      {1, 3338, 3584, 116, 28.5, 23.2},
+      {1, 4124, 2716, 88, 27.2, 20.6},
+      {2, 4124, 2716, 88, 31.5, 25.3},
+      {2, 1992, 356, 480, 9.1, 17.8},
+      {1, 4476, 1924, 1328, 85.4, 59.4},
+      {3, 665, 933, 120, 7.2, 13.0},
+      {3, 1317, 232, 221, 8.7, 13.7},
+      {3, 4452, 2292, 292, 82.6, 70.0},
+      {2, 2232, 1795, 459, 28.9, 41.0},
+      {3, 1124, 1644, 476, 21.3, 27.7},
+      {3, 1814, 885, 446, 22.0, 27.1},
+      {1, 2988, 1092, 100, 11.1, 13.7},
+      {2, 563, 461, 164, 7.1, 12.9},
+      {2, 892, 761, 475, 10.9, 18.9},
+      {1, 1789, 2401, 201, 18.6, 22.7},
+      {1, 367, 251, 281, 8.4, 13.0},
+      {1, 255, 397, 1685, 9.4, 30.0},
+      {2, 2016, 1984, 4728, 160.5, 133.3},
+      {3, 3792, 1168, 88, 25.9, 19.6},
+      {2, 1084, 804, 3672, 57.4, 66.8},
+      {2, 1740, 980, 1128, 25.3, 35.5},
+      {2, 408, 536, 1968, 13.6, 41.7}};
+  for (const auto &c : t) {
+    char what[96];
+    snprintf(what, sizeof(what), "planes for %d x %d x %d, operands %d (%.1f against %.1f us)", c.m, c.n, c.k, c.precision, c.planes, c.tiles);
+    expect(what, matmul_planes_faster(c.m, c.n, c.k, c.precision, 256), c.planes < c.tiles);
+  }
+}
+
 int main() {
   integer_gemv();
   shares_of_tiles();
   linears_over_many_rows();
+  matrix_products();
   printf("%d choices checked, %d wrong\n", g_checked, g_wrong);
   return g_wrong || !g_checked;
 }
