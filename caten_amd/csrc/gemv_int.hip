@@ -38,16 +38,14 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));  // row_half_mirror
   const unsigned E = max(m >> 23, 7u);  // (a unit is 2^(E - 156); at 7 the smallest subnormal number, of which every float is a multiple)
   const bool finite = m < 0x7f800000u;
+  // (the factor itself may lie past the largest float; 30 bits and a sign, an infinity stays one of 2^30 and what is beside it becomes nothing)
+  const int up = finite ? 156 - (int)E : -512;
   int x[4], infs = 0;
 #pragma unroll
-  for (int e = 0; e < 4; e++) x[e] = (int)rintf(__builtin_amdgcn_ldexpf(v[e], 156 - (int)E));  // (the factor itself may lie past the largest float)
-  if (__builtin_expect(!finite, 0)) {  // (the eight lanes of a chunk together)
+  for (int e = 0; e < 4; e++) x[e] = (int)__builtin_amdgcn_fmed3f(rintf(__builtin_amdgcn_ldexpf(v[e], up)), -0x1p30f, 0x1p30f);
+  if (__any(!finite)) {  // (uniform: the eight lanes of a chunk are together)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const bool inf = (__float_as_uint(v[e]) & 0x7fffffffu) == 0x7f800000u;
-      x[e] = inf ? ((int)__float_as_uint(v[e]) < 0 ? -1 : 1) << 24 : 0;
-      infs += inf ? 1 : 0;
-    }
+    for (int e = 0; e < 4; e++) infs += abs(x[e]) >> 30;
     infs += __builtin_amdgcn_mov_dpp(infs, 0xB1, 0xf, 0xf, true);
     infs += __builtin_amdgcn_mov_dpp(infs, 0x4E, 0xf, 0xf, true);
     infs += __builtin_amdgcn_mov_dpp(infs, 0x141, 0xf, 0xf, true);
@@ -171,19 +169,20 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
 #pragma unroll
     for (int b = 0; b < SB; b++) {
       const int k = i0 + nthr * b;
-      if (k >= n4) break;
-      float v[4] = {xv[b].x, xv[b].y, xv[b].z, xv[b].w};
-      const float u[4] = {uv[b].x, uv[b].y, uv[b].z, uv[b].w};
+      if (k < n4) {  // (not a break: three ways out of a loop are ten scalar registers, and past 80 a compute unit holds one workgroup of sixteen wavefronts)
+        float v[4] = {xv[b].x, xv[b].y, xv[b].z, xv[b].w};
+        const float u[4] = {uv[b].x, uv[b].y, uv[b].z, uv[b].w};
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        if (CENTRED) v[e] -= mu;
-        else if (LAYERNORM) s1 += v[e];
-        if (RMS || CENTRED) s1 = fmaf(v[e], v[e], s1);
-        if ((RMS || LAYERNORM) && a.norm_g) v[e] *= u[e];
+        for (int e = 0; e < 4; e++) {
+          if (CENTRED) v[e] -= mu;
+          else if (LAYERNORM) s1 += v[e];
+          if (RMS || CENTRED) s1 = fmaf(v[e], v[e], s1);
+          if ((RMS || LAYERNORM) && a.norm_g) v[e] *= u[e];
+        }
+        unsigned w[4];
+        const float down = int_digits(v, w);
+        put(k, w, down);
       }
-      unsigned w[4];
-      const float down = int_digits(v, w);
-      put(k, w, down);
     }
   }
   if (RMS || LAYERNORM) {

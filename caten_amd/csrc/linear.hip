@@ -410,9 +410,12 @@ static bool gemv_prefers_wide(const GemvVariant *v, int type, int64_t rows) {
   const int opt = state().gemv_wide;
   return opt && (!v || heavy || opt >= 2);
 }
-static bool gemv_prefers_int(int type, int64_t rows, int64_t cols) {
+// Several input rows are as many workgroups again.  With a norm in front a lane holds more than 64 registers, and of workgroups of more than twelve wavefronts a compute unit
+// holds one: 4096 x 4096, RMSNorm, 2 / 3 rows 8.0 / 11.8 us by the vector kernels, 10.2 / 14.1 this way (2560 x 2048 6.7 / 9.1 and 6.0 / 6.1; without a norm 7.4 / 11.1 and 7.4 / 10.3).
+static bool gemv_prefers_int(int type, int64_t rows, int64_t cols, int m = 1, int pro = CTHIP_PRO_NONE) {
   const int cus = state().compute_units;
-  return state().gemv_wide == 1 && gemv_int_plan(type, rows, cols, cus).ok && gemv_int_pays(rows, cols, cus);
+  const GemvIntPlan p = gemv_int_plan(type, rows, cols, cus);
+  return state().gemv_wide == 1 && p.ok && gemv_int_pays(rows, cols, cus) && !(m > 1 && pro != CTHIP_PRO_NONE && p.ks * p.rgp > 12);
 }
 bool gemv_norm_out_ok(const WMat *w) {
   const GemvVariant *v = pick_variant(w->type, (int)w->cols);
@@ -531,7 +534,7 @@ int launch_gemv(const WMat *w, GemvArgs a, int m) {
   if (a.split1 <= 0) a.split1 = a.split2 = a.rows;
   if (a.am_val && m != 1) return fail(CTHIP_E_BAD_ARG, "gemv: the fused argmax needs m == 1");
   // (rows laid out in pairs for a launch that only the integer kernel is: it stays with it whatever the options say now)
-  if ((gemv_prefers_int(w->type, w->rows, w->cols) || (a.pair_swiglu && !vector_pair_swiglu_ok(w->type, w->rows, w->cols))) && gemv_int_supported(w, a)) {
+  if ((gemv_prefers_int(w->type, w->rows, w->cols, m, a.pro) || (a.pair_swiglu && !vector_pair_swiglu_ok(w->type, w->rows, w->cols))) && gemv_int_supported(w, a)) {
     int parts = 0;
     const int rc = launch_gemv_int(w, a, m, &parts);
     if (rc || !a.am_val) return rc;
