@@ -279,13 +279,14 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route, bool *done);
 // A Linear over many rows from operands in memory as bf16 terms (gemm_planes.hip): x as fp32 rows or already as planes of plane_terms(precision) terms, the
 // result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
+// planes_in: x lies in planes already; prompt: one of a session's prompt (linear_planes_faster in gemm_plan.h)
 bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt);
-// x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
 // Linear over 8 .. 64 rows that lie as operands of two terms (linear_few.hip)
 bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: there is a pass over the rows in front of it anyway
-bool linear_few_shares_pays(const WMat *w, int m, int precision);
+bool linear_few_shares_pays(const WMat *w, int m, int precision);  // rows as they are, shares of K left to the norm behind (any number of columns)
 int launch_linear_few_shares(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual, GemmDeferred *defer);
 int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route);
+// x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
 bool linear_planes_ready(const WMat *w, int m, int precision);
 void weight_planes_release(const WMat *w);
 // The terms of all matrices together are kept up to this many bytes.  They are given back where memory is short, by

@@ -970,8 +970,8 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // over the rows does all three (launch_reduce_norm) instead of a reduction launch and a norm launch.
     // Many rows: a Linear takes its input as two bf16 terms (gemm_planes.hip) and what produces that input writes it so;
     // a row of terms is as long as the fp32 row whose buffer it takes.  (Sessions with a quantised cache stay
-    // with the tiles here, for want of a measurement: no order of summation is kept for their sake, fewer rows go through
-    // the same launches in every session.)
+    // with the tiles here, for want of a measurement; fewer rows go through the same launches in every session.  The one order of summation
+    // that is kept for their sake, at no cost that was found, is that of quantised tiles: tile_plan.)
     const bool planes = !d->kvq && prec == GEMM_BF16X3_DEFAULT && s >= 64 && rows_planes_supported(D) && F % 32 == 0;
     auto in_planes = [&](const WMat *w) {
       if (!planes || !w || !linear_planes_ready(w, R, prec)) return false;

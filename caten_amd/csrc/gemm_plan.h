@@ -72,7 +72,7 @@ inline double plane_tile_us(const PlaneTile &t, int M, int N, int nkb, int cus) 
   const int64_t full = tiles / slots, left = tiles - full * slots;
   double us = 2.0 + full * work * t.resident / t.all;
   if (t.resident == 1) us += (double)M * N * 4e-7;  // nothing runs under the stores (4500 x 4500 x 600 at one term: 63 us in tiles of 128, 73 of 256)
-  if (left <= cus) {  // (large tiles are bound by power, the fewer of them the higher the clock; a few small ones start under the round before)
+  if (left <= cus) {  // (a few tiles in the last round take less than a full round of them: `idle`)
     if (left) us += work / t.one * (full || t.resident == 1 ? t.idle + (1.0 - t.idle) * (double)left / cus : 1.0);
   } else {  // between one tile per compute unit and a full round, steeper at the start: the shared units wait for both
     const double one = work / t.one, all = work * t.resident / t.all;

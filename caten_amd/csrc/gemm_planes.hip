@@ -38,8 +38,8 @@ __device__ __forceinline__ int swz(int r) {
 // large (64 x 64: 16 reads for 24 instructions at two terms); two workgroups of four wavefronts per compute unit fill each
 // other's waits (reading a step's operands under the step before it instead, two sets of registers, measured the same or
 // slower; so did deeper rings than the launcher's).  4096^3, two terms: 284 us without the passes in front = 484 TFLOP/s of
-// results, 1.45 PFLOP/s of matrix instructions (the library's bf16 product reaches 1.2 - 1.5 on the card: the clock falls to 1.6 GHz under
-// them), against 180 with the operands converted per tile.  Integers need two products instead of three but 16 multiply-adds per lane and block for
+// results, 1.45 PFLOP/s of matrix instructions (the library's bf16 product reaches 1.2 - 1.5 on the card), against 180 with the operands converted per tile.
+// (3000 x 4100 x 5000, 256 x 256 tiles: matrix cores busy 54 % of the cycles that the counters show, 1.9 GHz.)  Integers need two products instead of three but 16 multiply-adds per lane and block for
 // the scales: 1900 x 11264 x 2048 194 us (operands converted per tile: 340), 1900 x 2048 x 5632 117 us (149).
 template <int NPA, int SRC, int NPB, int MB, int NB, int WM, int WN, int NBUF>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a) {

@@ -1,8 +1,11 @@
-// Linear over 8 .. 64 rows that lie in memory as operands of two bf16 terms (store_operands4 in planes.h), on packed weights of up to 2048 columns: the
-// projections of a short prompt, or of the next turn of a conversation.
+// Linear over a handful of rows: the projections of a short prompt, or of the next turn of a conversation.  Two ways:
+//  - 8 .. 64 rows that lie in memory as operands of two bf16 terms (store_operands4 in planes.h), packed weights of up to 2048 columns, ALL of K in a
+//    workgroup, the result finished here (launch_linear_few);
+//  - X32: 8 .. 32 rows as they are, split by every workgroup, packed weights of any number of columns; K is shared among gridDim.y workgroups, whose partial sums go to memory
+//    for the pass behind that adds up and normalises (launch_linear_few_shares; one share is finished here).
 //
 // The tiles of matmul.hip give such a product to a whole chip only by splitting K, which leaves partial tiles in memory and a
-// second launch that adds them up.  Here a workgroup owns 16 NB output columns and ALL of K: its eight wavefronts take an eighth of K each,
+// second launch that adds them up.  Here a workgroup owns 16 NB output columns and all of K (or its share): its eight wavefronts take an eighth of it each,
 // fetch their pieces of the weights and of the rows straight into operand registers (v_mfma_f32_16x16x32_bf16, lane l: row l % 16, k = 8 (l / 16) .. + 7 of a
 // block of 32), BATCH blocks asked for together, and meet once in LDS.  A workgroup reads nothing twice; the rows are read by all of them, out of L2,
 // and lie as the wavefronts hold them, whole cache lines to a request (as rows of terms, 16 half lines a request: 9.2 us for 37 rows of 1024 x 4096 fp16, 7.6 this

@@ -781,6 +781,7 @@ __global__ __launch_bounds__(256) void k_unary(int kind, float *y, const float *
   if (last) y[tail] = apply_act(kind, vt);
 }
 
+// out[t,:] = W[idx[t],:]  (+ W2[pos0 + t,:] when W2 is given: wte + wpe of Transformer, layers.lisp:80-82)
 __global__ __launch_bounds__(256) void k_embedding(float *__restrict__ out, const float *__restrict__ W,
                                                    const float *__restrict__ idx_f, const int *__restrict__ idx_i,
                                                    int vocab, int dim, const float *__restrict__ W2,
@@ -1376,7 +1377,7 @@ __global__ __launch_bounds__(256) void k_attn_rows(float *__restrict__ out, cons
   }
 }
 
-// Prompt rows on the matrix cores (16 rows and more): one block per (head, 32 consecutive query rows); its
+// Prompt rows on the matrix cores (32 rows and more; 16 .. 31 unless launch_attn has a better use for them): one block per (head, 32 consecutive query rows); its
 // NW wavefronts take the 32-key tiles of the visible cache round-robin, each with its own online softmax
 // for all 32 rows, and meet once in LDS.  fp32 MFMA operands (v_mfma_f32_32x32x2_f32): the products are the
 // reference's fp32 products, only the summation order differs.

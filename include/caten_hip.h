@@ -340,7 +340,7 @@ int cthip_rope(float *out, const float *x, int B, int S, int H, int Dh, float ba
  * (max_len, Hkv, Dh) (layers.lisp:19-33) holding T = start_pos+S rows, with the
  * causal mask of layers.lisp:83 applied.  out (S,H,Dh).  From 32 rows on the products run on the matrix cores:
  * with two bf16 terms per operand (2^-16 of a product dropped), or with fp32 operands when option
- * "gemm_precision" is 0. */
+ * "gemm_precision" is 0.  16 to 31 rows have fp32 products, on the matrix cores or (heads of 128, few heads or few keys) off them. */
 int cthip_sdpa_cached(float *out, const float *q, const float *k_cache, const float *v_cache,
                       int S, int start_pos, int H, int Hkv, int Dh);
 /* The same cache as GGUF-Q8_0 rows (the reference's cache is dense fp32, layers.lisp:19-33; its Q8_0 block is
