@@ -396,8 +396,6 @@ bool gemv_is_direct(const WMat *w) {
   return pick_variant(w->type, (int)w->cols) != nullptr || gemv_slices(w->type, (long long)w->cols, &width) > 0 ||
          gemv_wide_plan(w->type, w->rows, w->cols, state().compute_units).ok;
 }
-// true when a single-row launch over a (rows, cols) matrix of gate / up rows in turn can apply SwiGLU in its epilogue:
-// the launch it will be holds a row pair per wavefront (the routing of launch_gemv, repeated)
 // The wide-row kernel takes the rows no variant covers, and those whose variant holds so much of the input vector
 // per lane (128 floats: 4-bit rows past 6144 columns, 8-bit rows past 4096) that it needs more than 256 registers
 // and runs one wavefront per SIMD (Llama-70B shape, 8192-wide 4-bit rows: 12.3 -> 11.8 ms per step; narrower
@@ -434,6 +432,8 @@ static bool vector_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
   // has (enough rows for every wavefront to loop at any occupancy)
   return (gemv_ring_depth(type, v->KC) & 1) == 0 && rows >= 32ll * s.compute_units;
 }
+// true when a single-row launch over a (rows, cols) matrix of gate / up rows in turn can apply SwiGLU in its epilogue:
+// the launch it will be holds a row pair per wavefront, or is the integer kernel (the routing of launch_gemv, repeated)
 bool gemv_pair_swiglu_ok(int type, int64_t rows, int64_t cols) {
   if (rows <= 0 || (rows & 1) || cols <= 0 || cols > 0x7fffffff) return false;
   return gemv_prefers_int(type, rows, cols) || vector_pair_swiglu_ok(type, rows, cols);
