@@ -13,7 +13,7 @@
 // early, and more or fewer wavefronts per SIMD all measured the same or slower.
 // With the launch that splits: 1900 rows, 32 heads on 4 key / value heads of 64: 130 -> 66 us; 32 heads of 128: 234 -> 118 us.
 #include "common.h"
-#include "planes.h"
+#include "digits.h"
 
 namespace cthip {
 
@@ -56,6 +56,7 @@ __global__ __launch_bounds__(256) void k_attn_split(unsigned short *__restrict__
 struct AttnPlanesArgs {
   float *out;                  // (S, H, DH), or null:
   unsigned short *out_planes;  // rows of two terms for gemm_planes.hip
+  unsigned char *out_digits;   // rows for gemm_digits.hip
   const float *q;              // (S, H, DH)
   const unsigned char *kp, *vp;
   int S, start, H, Hkv, nkb;   // nkb: blocks of 32 keys
@@ -222,6 +223,20 @@ __global__ __launch_bounds__(128 * NW) void k_attn_planes(AttnPlanesArgs a) {
   }
   if (i0 + col >= a.S) return;
   const float inv = 1.0f / l;
+  if (a.out_digits) {
+    // a lane's halves of two blocks of 32 -> one whole block: lanes 0 .. 31 the even one, lanes 32 .. 63 the odd one
+#pragma unroll
+    for (int d = 0; d < DB; d += 2) {
+      float v[32];
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[d][r] * inv), __float_as_uint(o[d + 1][r] * inv), false, false);
+        v[8 * (r >> 2) + (r & 3)] = __uint_as_float(s[0]), v[8 * (r >> 2) + 4 + (r & 3)] = __uint_as_float(s[1]);
+      }
+      store_digits32(a.out_digits, (int64_t)(a.S + 31) / 32 * 32, a.H * DH / 32, i0 + col, (h * DH >> 5) + d + half, v);
+    }
+    return;
+  }
 #pragma unroll
   for (int d = 0; d < DB; d++)
 #pragma unroll
@@ -243,11 +258,12 @@ bool attn_planes_pays(int S, int start, int H, int Hkv, int DH) {
   const double each = 0.75 * tiles / (4.0 * state().compute_units), chain = 0.75 * longest;
   return 10.0 + f * (each > chain ? each : chain) < before;
 }
-int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH, bool *done) {
+int launch_attn_planes(float *out, void *out_terms, int terms, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH, bool *done) {
   if ((DH != 64 && DH != 128) || S < 1 || Hkv < 1 || H % Hkv) return fail(CTHIP_E_UNSUPPORTED, "attention: %d rows, %d heads on %d of %d", S, H, Hkv, DH);
   AttnPlanesArgs a = {};
   a.out = out;
-  a.out_planes = (unsigned short *)out_planes;
+  a.out_planes = terms == kTermsPlanes ? (unsigned short *)out_terms : nullptr;
+  a.out_digits = terms == kTermsDigits ? (unsigned char *)out_terms : nullptr;
   a.q = q;
   a.S = S, a.start = start, a.H = H, a.Hkv = Hkv;
   const int T = start + S, group = H / Hkv;

@@ -95,8 +95,9 @@ struct WMat {
   // valid for exactly these gamma / beta / bias vectors
   const float *fold_g = nullptr, *fold_b = nullptr, *fold_bias = nullptr;
   float *fold_s = nullptr, *fold_c = nullptr;
-  // the matrix as bf16 terms, made by the first Linear over many rows that wants them (gemm_planes.hip)
+  // the matrix as bf16 terms, made by the first Linear over many rows that wants them (gemm_planes.hip), or as digits (gemm_digits.hip)
   void *planes = nullptr;
+  int planes_terms = 0;  // how many terms, kDigits
   int64_t planes_bytes = 0;
   int planes_users = 0;  // launches being put together from them; they are not given back meanwhile
 };
@@ -241,11 +242,13 @@ __device__ __forceinline__ int attn_head_of_block(int b, int H, int Hkv) {
 }
 #endif
 int launch_attn(float *out, const float *q, const float *kc, const float *vc, int S, int start_pos, const int *pos,
-                int max_T, int H, int Hkv, int Dh, const AttnSplit *split = nullptr);
-// attention of many prompt rows with keys and values split once (attn_planes.hip); out as fp32 rows or as rows of two terms
+                int max_T, int H, int Hkv, int Dh, const AttnSplit *split = nullptr, void *digits = nullptr);
+// digits: non-null = the result goes there as digits (gemm_digits.hip) instead of out, where that is supported
+inline bool attn_digits_supported(int S, int Dh) { return S >= 32 && (Dh == 32 || Dh == 64 || Dh == 128) && state().gemm_precision != 0; }
+// attention of many prompt rows with keys and values split once (attn_planes.hip); out as fp32 rows, as rows of two terms or as digits
 bool attn_planes_pays(int S, int start, int H, int Hkv, int DH);
 // (*done stays false where there is no memory for the terms)
-int launch_attn_planes(float *out, void *out_planes, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH, bool *done);
+int launch_attn_planes(float *out, void *out_terms, int terms, const float *q, const float *kc, const float *vc, int S, int start, int H, int Hkv, int DH, bool *done);
 int launch_embedding(float *out, const float *W, const float *idx_f, const int *idx_i, int ntok, int vocab, int dim,
                      const float *W2, const int *pos, int max_pos);
 int launch_argmax(int64_t *out, const float *x, int64_t rows, int n, int *tok_out, int *pos, int64_t *history,
@@ -277,9 +280,10 @@ int launch_linear_gemm(float *y, const WMat *w, const float *x, int m, const flo
 bool linear_rows_pays(const WMat *w, const float *x, int64_t x_stride, int m, int precision, const float *g, const float *b);
 int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride, int m, const float *bias, const float *residual, int act,
                        int pro, const float *norm_g, const float *norm_b, float eps, int precision, const GemmRoute *route, bool *done);
-// A Linear over many rows from operands in memory as bf16 terms (gemm_planes.hip): x as fp32 rows or already as planes of plane_terms(precision) terms, the
-// result to y / the route or (two terms, rows of whole blocks) as planes.  *done stays false where this path does not apply.
-// planes_in: x lies in planes already; prompt: one of a session's prompt (linear_planes_faster in gemm_plan.h)
+// A Linear over many rows from operands in memory as bf16 terms (gemm_planes.hip) or, over 4-bit weights at two terms' precision, as digits (gemm_digits.hip):
+// x as fp32 rows or already as the matrix takes it (linear_terms), the result to y / the route or (two terms, rows of whole blocks) as out_terms says.
+// *done stays false where this path does not apply.  planes_in: x lies in planes or digits already; prompt: one of a session's prompt (linear_planes_faster in
+// gemm_plan.h); defer: as for launch_linear_gemm, shares of K only with digits.
 bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt);
 // Linear over 8 .. 64 rows that lie as operands of two terms (linear_few.hip)
 bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: there is a pass over the rows in front of it anyway
@@ -288,16 +292,26 @@ int launch_linear_few_shares(float *y, const WMat *w, const float *x, int m, con
 int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route);
 // x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
 bool linear_planes_ready(const WMat *w, int m, int precision);
+int linear_terms(const WMat *w, int precision);  // kTermsPlanes or kTermsDigits
 void weight_planes_release(const WMat *w);
 // The terms of all matrices together are kept up to this many bytes.  They are given back where memory is short, by
 // cthip_cache_trim and by a lower limit; weight_planes_drop returns whether there were any.
 void weight_planes_limit(int64_t bytes);
 bool weight_planes_drop();
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
-                         int precision, const GemmRoute *route, unsigned char *planes_out, bool *done);
+                         int precision, const GemmRoute *route, unsigned char *planes_out, int out_terms, bool prompt, GemmDeferred *defer, bool *done);
 bool rows_planes_supported(int K);
-// How a pass in front of a Linear writes its rows: fp32, as two bf16 terms a row (planes.h), as matrix operands of two terms (store_operands4)
-enum { kTermsNone = 0, kTermsPlanes = 1, kTermsOperands = 2 };
+// How a pass in front of a Linear writes its rows: fp32, as two bf16 terms a row (planes.h), as matrix operands of two terms (store_operands4), as digits (digits.h)
+enum { kTermsNone = 0, kTermsPlanes = 1, kTermsOperands = 2, kTermsDigits = 3 };
+// ---- 6-bit digits (gemm_digits.hip) ----
+constexpr int kDigits = -1;  // in the place of a number of terms
+int64_t digit_weight_bytes(const WMat *w);
+int make_weight_digits(unsigned char *out, const WMat *w);
+inline bool rows_digits_supported(int K) { return K % 32 == 0 && K <= 8192; }  // behind a norm
+int launch_rows_digits(void *digits, const float *x, int m, int K, int pro, const float *g, const float *b, float eps);
+struct DigitGemmArgs;
+struct DigitsPick;
+int digits_gemm(const DigitGemmArgs &a, const DigitsPick &pick);
 int launch_rows_planes(void *planes, const float *x, int m, int K, int pro, const float *g, const float *b, float eps, int terms);
 void wmat_drop_planes(WMat *w);
 // matmul over operands split into bf16 terms once (gemm_planes.hip), B (K, N) row-major; call only where it pays

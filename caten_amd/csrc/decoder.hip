@@ -919,6 +919,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   const int D = c.dim, F = c.ffn, V = c.vocab, KD = kv_dim(c), Dh = c.dim / c.n_heads;
   const int QW = D + 2 * KD, HW = gpt2 ? F : 2 * F;
   const int prec = state().gemm_precision;
+  const size_t s32 = (size_t)(s + 31) / 32 * 32;  // rows that may go as digits: whole blocks of 32
   int rc = 0;
   float *X = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *Hb = nullptr, *G = nullptr, *KF = nullptr, *VF = nullptr;
   int *ids_dev = nullptr;
@@ -935,12 +936,12 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     if ((rc = (e))) goto done; \
   } while (0)
   TRY(alloc((void **)&X, sizeof(float) * (size_t)s * D));
-  TRY(alloc((void **)&XN, sizeof(float) * (size_t)((s + 15) / 16 * 16) * D));  // (whole blocks of 16 rows as matrix operands)
+  TRY(alloc((void **)&XN, sizeof(float) * (s >= 64 ? s32 : (size_t)(s + 15) / 16 * 16) * D));  // (whole blocks of 16 rows as matrix operands)
   TRY(alloc((void **)&QKV, sizeof(float) * (size_t)s * QW));
   TRY(alloc((void **)&Q, sizeof(float) * (size_t)s * D));
-  TRY(alloc((void **)&ATT, sizeof(float) * (size_t)s * D));
-  TRY(alloc((void **)&Hb, sizeof(float) * (size_t)s * HW));
-  if (!gpt2) TRY(alloc((void **)&G, sizeof(float) * (size_t)s * F));
+  TRY(alloc((void **)&ATT, sizeof(float) * (s >= 64 ? s32 : (size_t)s) * D));
+  TRY(alloc((void **)&Hb, sizeof(float) * (s >= 64 ? s32 : (size_t)s) * HW));
+  if (!gpt2) TRY(alloc((void **)&G, sizeof(float) * (s >= 64 ? s32 : (size_t)s) * F));
   if (d->kvq || d->kvp) {
     TRY(alloc((void **)&KF, sizeof(float) * (size_t)(n + s) * KD));
     TRY(alloc((void **)&VF, sizeof(float) * (size_t)(n + s) * KD));
@@ -968,15 +969,17 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // A row-split Linear (attention projection, second MLP Linear) whose reduction axis was shared among several
     // workgroups per tile leaves partial tiles; what follows it is the residual add and the next norm, so one pass
     // over the rows does all three (launch_reduce_norm) instead of a reduction launch and a norm launch.
-    // Many rows: a Linear takes its input as two bf16 terms (gemm_planes.hip) and what produces that input writes it so;
-    // a row of terms is as long as the fp32 row whose buffer it takes.  (Sessions with a quantised cache stay
+    // Many rows: a Linear takes its input as two bf16 terms (gemm_planes.hip), or over 4-bit weights as digits (gemm_digits.hip), and what produces that
+    // input writes it so; a row of terms is as long as the fp32 row whose buffer it takes, one of digits no longer.  (Sessions with a quantised cache stay
     // with the tiles here, for want of a measurement; fewer rows go through the same launches in every session.  The one order of summation
     // that is kept for their sake, at no cost that was found, is that of quantised tiles: tile_plan.)
     const bool planes = !d->kvq && prec == GEMM_BF16X3_DEFAULT && s >= 64 && rows_planes_supported(D) && F % 32 == 0;
-    auto in_planes = [&](const WMat *w) {
-      if (!planes || !w || !linear_planes_ready(w, R, prec)) return false;
+    auto in_planes = [&](const WMat *w) -> int {
+      if (!planes || !w) return kTermsNone;
+      const int terms = linear_terms(w, prec);
+      if ((terms == kTermsDigits && !rows_digits_supported(D)) || !linear_planes_ready(w, R, prec)) return kTermsNone;
       held.push_back(w);
-      return true;
+      return terms;
     };
     // 8 .. 64 rows: the Linears behind a norm as one launch each, no partial tiles to add up (linear_few.hip); the norm writes their operands.
     // (fewer and larger matrices keep the launch whose inputs have all 24 bits, linear_rows.hip)
@@ -984,24 +987,29 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       return !(planes && std::find(held.begin(), held.end(), w) != held.end()) && rows_planes_supported(D) && w->cols == D && linear_few_pays(w, R, prec, true) &&
              !linear_rows_pays(w, XN, D, R, prec, nullptr, nullptr);
     };
-    auto in_terms = [&](const WMat *w) { return !w ? kTermsNone : in_planes(w) ? kTermsPlanes : few(w) ? kTermsOperands : kTermsNone; };
+    auto in_terms = [&](const WMat *w) -> int {
+      if (w && linear_terms(w, prec) == kTermsDigits && few(w)) return kTermsOperands;  // (64 rows, GPT-2 medium: 1140 us, as digits 1360)
+      const int terms = in_planes(w);
+      return terms || !w ? terms : few(w) ? kTermsOperands : kTermsNone;
+    };
     auto no_planes = [&](const WMat *w) {
       held.erase(std::find(held.begin(), held.end(), w));
       weight_planes_release(w);
     };
     // y = norm(x), as terms where the Linear behind it takes them
     auto norm = [&](float *y, const float *x, const float *g, const float *b, int terms) {
+      if (terms == kTermsDigits) return launch_rows_digits(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps);
       if (terms) return launch_rows_planes(y, x, R, D, gpt2 ? CTHIP_PRO_LAYERNORM : CTHIP_PRO_RMSNORM, g, gpt2 ? b : nullptr, c.eps, terms);
       return gpt2 ? cthip_layernorm(y, x, g, b, c.eps, R, D) : cthip_rmsnorm(y, x, g, c.eps, R, D);
     };
-    // y = W.in + ..., in and y as terms where in_terms / out_terms
+    // y = W.in + ..., in and y as terms as in_terms / out_terms say
     auto linear = [&](float *y, const WMat *w, const float *in, int in_terms, const float *bias, const float *residual, int act, const GemmRoute *route,
-                      bool out_terms, GemmDeferred *defer = nullptr) {
+                      int out_terms, GemmDeferred *defer = nullptr) {
       if (in_terms == kTermsOperands) return launch_linear_few(y, w, in, R, bias, residual, act, route);
       if (in_terms || (planes && linear_planes_pays(w, R, prec, false, true))) {
         bool taken = false;
         const int r = launch_linear_planes(out_terms ? nullptr : y, w, in_terms ? nullptr : in, in_terms ? (const unsigned char *)in : nullptr, R, bias,
-                                           residual, act, prec, route, out_terms ? (unsigned char *)y : nullptr, &taken);
+                                           residual, act, prec, route, out_terms ? (unsigned char *)y : nullptr, out_terms, true, defer, &taken);
         if (in_terms) no_planes(w);  // no more than a layer's matrices are held at a time
         if (taken) return r;
         if (in_terms || out_terms) return fail(CTHIP_E_STATE, "prompt: a Linear of %lld x %lld over %d rows cannot take its input as terms", (long long)w->rows, (long long)w->cols, R);
@@ -1014,7 +1022,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     auto linear_residual_norm = [&](const WMat *w, const float *in, int in_terms, const float *bias, const float *g, const float *b, int out_terms) {
       GemmDeferred df;
       const bool fuse = g != nullptr && reduce_norm_supported(D, 1);
-      int r = linear(Xr, w, in, in_terms, bias, Xr, CTHIP_ACT_NONE, nullptr, false, fuse ? &df : nullptr);
+      int r = linear(Xr, w, in, in_terms, bias, Xr, CTHIP_ACT_NONE, nullptr, kTermsNone, fuse ? &df : nullptr);
       if (r) return r;
       if (df.ws) {
         if (reduce_norm_supported(D, df.ksplit)) {
@@ -1039,7 +1047,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         // batch's rows [n, n + s) join them (rotated where the model rotates) and are quantised into the cache
         TRY(launch_kvq_dequant(KF, L.kq, L.kdq, n, KD));
         TRY(launch_kvq_dequant(VF, L.vq, L.vdq, n, KD));
-        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, false));
+        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, kTermsNone));
         TRY(launch_qkv_split(Q, KF, VF, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
         TRY(launch_kvq_append(L.kq, L.kdq, KF + (int64_t)n * KD, KD, s, n, nullptr, KD));
         TRY(launch_kvq_append(L.vq, L.vdq, VF + (int64_t)n * KD, KD, s, n, nullptr, KD));
@@ -1049,7 +1057,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
         // batch's rows [n, n + s) join them (rotated where the model rotates) and are copied into their pages
         TRY(launch_kvp_gather(KF, L.k_pages, n, KD));
         TRY(launch_kvp_gather(VF, L.v_pages, n, KD));
-        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, false));
+        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, kTermsNone));
         TRY(launch_qkv_split(Q, KF, VF, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
         TRY(launch_kvp_append(L.k_pages, L.v_pages, KF + (int64_t)n * KD, VF + (int64_t)n * KD, KD, s, n, nullptr, KD));
         K = KF, V = VF;
@@ -1057,22 +1065,27 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
       if (gpt2 && D % 128 == 0 && KD % 128 == 0) {
         // no rotation: the thirds of the fused projection go straight to the query rows and the cache rows
         const GemmRoute rt = {{Q, L.k_cache + (int64_t)n * KD, L.v_cache + (int64_t)n * KD}, {0, D, D + KD}, {D, KD, KD}};
-        TRY(linear(nullptr, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, &rt, false));
+        TRY(linear(nullptr, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, &rt, kTermsNone));
       } else {
-        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, false));
+        TRY(linear(QKV, L.attn, XN, xt, L.attn_b, nullptr, CTHIP_ACT_NONE, nullptr, kTermsNone));
         TRY(launch_qkv_split(Q, L.k_cache, L.v_cache, QKV, s, n, c.n_heads, c.n_kv_heads, Dh, gpt2 ? 0.0f : c.rope_base));
       }
       }
       if (last) R = 1, Xr = X + (int64_t)(s - 1) * D;
-      bool att = false, attended = false;
+      int att = kTermsNone;
+      bool attended = false;
       if (!last && planes && attn_planes_pays(R, n, c.n_heads, c.n_kv_heads, Dh)) {
         att = in_planes(L.proj);
-        TRY(launch_attn_planes(att ? nullptr : ATT, att ? ATT : nullptr, Q, K, V, R, n, c.n_heads, c.n_kv_heads, Dh, &attended));
-        if (att && !attended) att = false, no_planes(L.proj);
+        TRY(launch_attn_planes(att ? nullptr : ATT, att ? ATT : nullptr, att, Q, K, V, R, n, c.n_heads, c.n_kv_heads, Dh, &attended));
+        if (att && !attended) att = kTermsNone, no_planes(L.proj);
       }
-      if (!attended) TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split));
+      if (!attended) {
+        if (!last && planes && linear_terms(L.proj, prec) == kTermsDigits && attn_digits_supported(R, Dh)) att = in_planes(L.proj);
+        TRY(launch_attn(ATT, last ? Q + (int64_t)(s - 1) * D : Q, K, V, R, n + s - R, nullptr, n + s, c.n_heads, c.n_kv_heads, Dh, last ? &last_split : &split, att ? ATT : nullptr));
+      }
       const int ft = in_terms(L.fc);
-      const bool gt = ft == kTermsPlanes && (gpt2 || L.fc_pairs) && in_planes(L.fc2);
+      // (what writes planes does not write digits)
+      const int gt = (ft == kTermsDigits || (ft == kTermsPlanes && L.fc2 && linear_terms(L.fc2, prec) == kTermsPlanes)) && (gpt2 || L.fc_pairs) ? in_planes(L.fc2) : kTermsNone;
       TRY(linear_residual_norm(L.proj, ATT, att, L.proj_b, L.ln2_g, L.ln2_b, ft));
       const float *hin = Hb;
       if (!gpt2 && L.fc_pairs && (2 * F) % 4 == 0) {  // SwiGLU in the epilogue of the gate|up launch

@@ -104,6 +104,36 @@ inline PlanePick plane_pick(int M, int N, int nkb, int terms, bool ints_b, int c
   return best;
 }
 
+// ---- Linears whose operands lie as 6-bit digits (gemm_digits.hip): tile and shares of K ----
+struct DigitsPick {
+  int tile, ks, fullest;  // tile: of the list; fullest: tiles of the fullest compute unit
+  double us;              // of the launch, and with shares of what adds them up
+};
+// What the result is: rows of floats, rows as digits, SwiGLU of (gate, up) columns as digits (a wavefront's columns have to be whole blocks of results), or raw sums of a share of K
+enum { kDigitsPlain = 0, kDigitsOut = 1, kDigitsOutPairs = 2, kDigitsShares = 3 };
+// shares: whether K may be split (deferred: the launch behind adds the shares up on its way).  A launch is its ends and a time per block of 32 k of the fullest compute unit, us:
+// `first`, and `more` (`many` past two) for each further tile.  Fitted to weights out of memory: 64 x 64 / 64 x 128 / 128 x 128 for 100 x 3072 x 1024 10.0 / 12.3 / 18.5,
+// 300 x 2560 x 2048 15.7 / 19.4 / 29.6, 200 x 11264 x 2048 34 / 28 / 33, 280 x 4096 x 4096 40 / 35 / 52, 1900 x 2048 x 5632 98 / 71 / 80, 1900 x 11264 x 2048 195 / 133 / 128.
+inline DigitsPick digits_pick(int M, int N, int nkb, int out, bool shares, bool deferred, int cus) {
+  static const struct {
+    int bm, bn;
+    double ends, first, more, many;
+  } tiles[] = {{64, 64, 4.4, 0.175, 0.095, 0.14}, {64, 128, 5.0, 0.235, 0.14, 0.18}, {128, 128, 7.6, 0.35, 0.26, 0.30}};
+  DigitsPick best = {1, 1, 1, 1e30};
+  for (int ks = 1; ks <= (shares ? 8 : 1); ks++) {
+    const int per = (nkb + ks - 1) / ks;
+    if ((nkb + per - 1) / per != ks || (ks > 1 && per < 8)) continue;
+    for (int t = out == kDigitsOutPairs ? 1 : 0; t < 3; t++) {
+      const int64_t of_xcd = ((int64_t)((M + tiles[t].bm - 1) / tiles[t].bm) * ((N + tiles[t].bn - 1) / tiles[t].bn) + 7) / 8 * ks;
+      const int fullest = (int)((of_xcd * 8 + cus - 1) / cus);
+      const double us = tiles[t].ends + (out ? 2.5 : 0.0) + per * (tiles[t].first + (fullest <= 2 ? tiles[t].more : tiles[t].many) * (fullest - 1)) +
+                        (ks > 1 ? (deferred ? 0.3 : 2.6) + (deferred ? 0.6e-6 : 0.85e-6) * 4.0 * ks * M * N : 0.0);
+      if (us < best.us) best = {t, ks, fullest, us};
+    }
+  }
+  return best;
+}
+
 // Microseconds of a product (M, N, K) through planes: two passes over the operands (about 4.2 TB/s; none for operands that
 // lie in planes already) and a denser GEMM.
 inline double planes_us(int M, int N, int K, int terms, bool ints_b, double pass_bytes, int cus) {
@@ -122,6 +152,14 @@ inline bool matmul_planes_faster(int M, int N, int K, int precision, int cus) {
   const double us = planes_us(M, N, K, terms, false, ((double)M + N) * K * (4 + 2 * terms), cus), out = 4e-6 * M * N;
   const double planes = aligned ? 0.83 * us + 8.0 : terms == 3 ? 0.95 * us + 8.0 : 0.94 * us + 10.4 + out / 4.0;
   return planes < tile_plan(M, N, K, precision, -1, aligned, false, cus).us;
+}
+
+// Linears over 4-bit weights at two terms: digits against tiles that convert their operands.
+inline bool linear_digits_faster(int M, int N, int K, int type, double pass_bytes, bool prompt, int cus) {
+  if ((int64_t)(K / 32) * 4096 * 8 >= (1ll << 31)) return false;  // 32-bit offsets within a tile's rows
+  // (in a prompt, behind other launches, 1.5 - 2 us more than by itself)
+  const double us = digits_pick(M, N, K / 32, kDigitsPlain, true, prompt, cus).us + (prompt ? 1.5 : 0.0) + (pass_bytes > 0 ? pass_bytes / 4.2e6 + 5.0 : 0.0);
+  return us < tile_plan(M, N, K, GEMM_BF16X3, type, true, false, cus).us;
 }
 
 // The same for a Linear over weights (N, K).  planes_us and tile_plan are each off by what depends on the format: an integer or a half weight is fewer bytes for the tiles and one plane or

@@ -14,7 +14,8 @@
 #include <unordered_set>
 
 #include "common.h"
-#include "planes.h"
+#include "digits.h"
+#include "gemm_plan.h"
 
 namespace cthip {
 
@@ -476,12 +477,19 @@ static int64_t g_planes_limit = 32ll << 30, g_planes_bytes = 0;
 static std::unordered_set<WMat *> g_planes_of;
 
 static bool is_quant(const WMat *w) { return w->type == CTHIP_Q8_0 || w->type == CTHIP_Q4_0; }
-static int weight_terms(const WMat *w, int terms) { return is_quant(w) ? 1 : w->type == CTHIP_F16 && terms > 2 ? 2 : terms; }
-static int64_t weight_plane_bytes(const WMat *w, int terms_b) { return w->rows * ((w->cols + 31) / 32) * 64 * terms_b; }
+static int weight_terms(const WMat *w, int terms) {
+  if (w->type == CTHIP_Q4_0 && terms == 2) return kDigits;
+  return is_quant(w) ? 1 : w->type == CTHIP_F16 && terms > 2 ? 2 : terms;
+}
+int linear_terms(const WMat *w, int precision) { return weight_terms(w, plane_terms(precision)) == kDigits ? kTermsDigits : kTermsPlanes; }
+static int64_t weight_plane_bytes(const WMat *w, int terms_b) {
+  return terms_b == kDigits ? digit_weight_bytes(w) : w->rows * ((w->cols + 31) / 32) * 64 * terms_b;
+}
 static bool weight_planes_stay(const WMat *w, int terms_b) { return is_quant(w) || (w->type == CTHIP_F16 && terms_b == 2); }
 
 static int make_weight_planes(unsigned char *out, const WMat *w, int terms_b) {
   const int K = (int)w->cols;
+  if (terms_b == kDigits) return make_weight_digits(out, w);
   if (w->type == CTHIP_F16) return planes_rows<_Float16>(out, (const _Float16 *)w->q, w->rows, K, K, terms_b);
   if (w->type == CTHIP_F32) return planes_rows<float>(out, (const float *)w->q, w->rows, K, K, terms_b);
   const int64_t n8 = w->rows * K / 8;
@@ -494,7 +502,7 @@ static int make_weight_planes(unsigned char *out, const WMat *w, int terms_b) {
 }
 // Whether they are there or the next call's stay (with g_planes_mu held)
 static bool weight_planes_room(const WMat *w, int terms_b) {
-  return weight_planes_stay(w, terms_b) && (w->planes || g_planes_bytes + weight_plane_bytes(w, terms_b) <= g_planes_limit);
+  return weight_planes_stay(w, terms_b) && (w->planes ? w->planes_terms == terms_b : g_planes_bytes + weight_plane_bytes(w, terms_b) <= g_planes_limit);
 }
 static bool weight_planes_kept(const WMat *w, int terms_b) {
   std::lock_guard<std::mutex> lk(g_planes_mu);
@@ -521,6 +529,7 @@ static const unsigned char *weight_planes(const WMat *w, int terms_b, bool *temp
   }
   if (stay) {
     m->planes = p;
+    m->planes_terms = terms_b;
     m->planes_bytes = bytes;
     m->planes_users = 1;
     g_planes_bytes += bytes;
@@ -576,6 +585,9 @@ bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, boo
   double bytes = 0.0;
   if (!weight_planes_kept(w, terms_b)) bytes = (double)w->q_bytes + weight_plane_bytes(w, terms_b);
   if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
+  // (a prompt past the limit: memory that is only lent for a launch, where that is long)
+  if (terms_b == kDigits && prompt && m < 512 && !weight_planes_kept(w, terms_b)) return false;
+  if (terms_b == kDigits) return linear_digits_faster(m, (int)w->rows, (int)w->cols, w->type, bytes, prompt, state().compute_units);
   return linear_planes_faster(m, (int)w->rows, (int)w->cols, precision, w->type, bytes, prompt, state().compute_units);
 }
 // ... and nothing can be in the way of it
@@ -583,9 +595,11 @@ bool linear_planes_ready(const WMat *w, int m, int precision) {
   return linear_planes_pays(w, m, precision, true, true) && weight_planes(w, weight_terms(w, plane_terms(precision)), nullptr);
 }
 int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned char *xplanes, int m, const float *bias, const float *residual, int act,
-                         int precision, const GemmRoute *route, unsigned char *planes_out, bool *done) {
+                         int precision, const GemmRoute *route, unsigned char *planes_out, int out_terms, bool prompt, GemmDeferred *defer, bool *done) {
   const int K = (int)w->cols, terms = plane_terms(precision), terms_b = weight_terms(w, terms);
-  PlaneGemmArgs a = {};
+  const bool digits = terms_b == kDigits;
+  if (digits && ((uintptr_t)x & 15)) return 0;  // (the pass that makes digits reads 16 bytes at a time)
+  DigitGemmArgs a = {};
   a.C = y;
   a.M = m, a.N = (int)w->rows;
   a.bias = bias, a.residual = residual;
@@ -606,17 +620,19 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
   if (a.N % 4 == 0 && (at & 15)) return 0;
   if (planes_out) {
     const int width = a.pairs ? a.N / 2 : a.N;
-    if (terms != 2 || a.N % 4 || width % 32) return 0;
-    a.planes = (unsigned short *)planes_out;
+    if (terms != 2 || a.N % 4 || width % 32 || (out_terms == kTermsDigits && !digits)) return 0;
+    if (out_terms == kTermsDigits) a.digits = planes_out;
+    else a.planes = (unsigned short *)planes_out;
     a.pkb = width / 32;
   }
   planes_operands(a, K, terms, terms_b);
-  if (is_quant(w)) {
+  if (is_quant(w) && !digits) {
     a.bd = (const unsigned short *)w->d;
     a.dpitch = a.nkb;
   }
   unsigned char *tmp = nullptr;
-  if (stream_capturing() || (!xplanes && alloc_scratch((void **)&tmp, (size_t)m * a.apitch))) return 0;  // fully written by the pass in front
+  if (stream_capturing() || (!xplanes && alloc_scratch((void **)&tmp, digits ? (size_t)digit_row_bytes(m, a.nkb) : (size_t)m * a.apitch)))
+    return 0;  // written by the pass in front, but for rows that reach no result
   bool temp_b = false;
   const unsigned char *pb = weight_planes(w, terms_b, &temp_b);
   if (!pb) {
@@ -624,9 +640,27 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
     return 0;
   }
   *done = true;
-  int rc = xplanes ? 0 : planes_rows<float>(tmp, x, m, K, K, terms);
+  int rc = xplanes ? 0 : digits ? launch_rows_digits(tmp, x, m, K, CTHIP_PRO_NONE, nullptr, nullptr, 0.0f) : planes_rows<float>(tmp, x, m, K, K, terms);
   a.A = xplanes ? xplanes : tmp, a.B = pb;
-  if (!rc) rc = planes_gemm(a, terms, terms_b);
+  if (!rc && digits) {
+    // Shares of K: left to the caller, or added up (with bias and residual) by a launch of their own
+    const bool plain = a.act == CTHIP_ACT_NONE && !a.pairs && !a.routed && !planes_out;
+    const int out = !a.digits ? kDigitsPlain : a.pairs ? kDigitsOutPairs : kDigitsOut;
+    DigitsPick pick = digits_pick(m, a.N, a.nkb, out, plain, defer != nullptr, state().compute_units);
+    float *ws = nullptr;
+    if (pick.ks > 1 && alloc_scratch((void **)&ws, sizeof(float) * (size_t)pick.ks * m * a.N)) pick = digits_pick(m, a.N, a.nkb, out, false, false, state().compute_units);
+    if (ws) a.C = ws, a.bias = a.residual = nullptr;
+    rc = digits_gemm(a, pick);
+    if (ws && defer && !rc) {
+      defer->ws = ws;
+      defer->ksplit = pick.ks;
+    } else if (ws) {
+      if (!rc) rc = launch_splitk_reduce(y, ws, pick.ks, m, a.N, bias, residual);
+      cthip_free(ws);  // stream-ordered: handed out again only to later work on this stream
+    }
+  } else if (!rc) {
+    rc = planes_gemm(a, terms, terms_b);
+  }
   cthip_free(tmp);  // stream-ordered: handed out again only to later work on this stream
   if (temp_b) cthip_free(const_cast<unsigned char *>(pb));
   else weight_planes_release(w);

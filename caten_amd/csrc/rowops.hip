@@ -8,7 +8,7 @@
 // 64*4*8 = 2048 floats take a block per row.
 #include <type_traits>
 #include "common.h"
-#include "planes.h"
+#include "digits.h"
 #include "gemv_plan.h"
 
 namespace cthip {
@@ -140,6 +140,7 @@ struct ReduceNormArgs {
   int n;
   unsigned short *planes;  // non-null: the normalised rows go out as two bf16 terms (gemm_planes.hip) instead of y ...
   int row_blocks;          // ... or, when set, as matrix operands of that many blocks of 16 rows (linear_few.hip)
+  unsigned char *digits;   // non-null: ... as digits (gemm_digits.hip)
 };
 
 template <int MODE, int VPL, int NZ>
@@ -215,6 +216,7 @@ __global__ __launch_bounds__(256) void k_reduce_norm(ReduceNormArgs a) {
 template <int MODE, int VPL, int NZ>
 __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
   __shared__ float red[2][4];
+  __shared__ __align__(16) float turn[VPL * 32 * 36];  // digits: a thread's four values -> blocks of 32, 36 apart (no bank twice)
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t row = blockIdx.x;
   const int n = a.n, n4 = n >> 2;
@@ -278,9 +280,22 @@ __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
       const float4 g = a.g ? gm[j] : make_float4(1.f, 1.f, 1.f, 1.f);
       const float4 b = a.b ? bt[j] : make_float4(0.f, 0.f, 0.f, 0.f);
       const float o[4] = {v[j][0] * rstd * g.x + b.x, v[j][1] * rstd * g.y + b.y, v[j][2] * rstd * g.z + b.z, v[j][3] * rstd * g.w + b.w};
-      if (a.planes && a.row_blocks) store_operands4(a.planes, (int)row, a.row_blocks, 4 * (tid + 256 * j), o);
+      if (a.digits) *(float4 *)&turn[(tid / 8 + 32 * j) * 36 + 4 * (tid % 8)] = make_float4(o[0], o[1], o[2], o[3]);
+      else if (a.planes && a.row_blocks) store_operands4(a.planes, (int)row, a.row_blocks, 4 * (tid + 256 * j), o);
       else if (a.planes) store_planes4(a.planes, row, n >> 5, 4 * (tid + 256 * j), o);
       else ((float4 *)(a.y + row * n))[tid + 256 * j] = make_float4(o[0], o[1], o[2], o[3]);
+    }
+  }
+  if (a.digits) {
+    __syncthreads();
+    if (tid < n >> 5) {  // (at most 32 VPL <= 256 blocks)
+      float f[32];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const float4 u = *(const float4 *)&turn[tid * 36 + 4 * q];
+        f[4 * q] = u.x, f[4 * q + 1] = u.y, f[4 * q + 2] = u.z, f[4 * q + 3] = u.w;
+      }
+      store_digits32(a.digits, (a.rows + 31) / 32 * 32, n >> 5, row, tid, f);
     }
   }
 }
@@ -292,9 +307,15 @@ int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, in
   if (rows == 0 || n == 0) return 0;
   if (terms && n % 32) return fail(CTHIP_E_BAD_ARG, "reduce + norm: rows of %d as terms", n);
   if (!reduce_norm_supported(n, nparts)) return fail(CTHIP_E_BAD_ARG, "reduce + norm: rows of %d with %d shares", n, nparts);
-  ReduceNormArgs a = {y, xout, parts, nparts, part_stride, bias, resid, g, b, eps, rows, n, terms ? (unsigned short *)y : nullptr, terms == kTermsOperands ? (int)(rows + 15) / 16 : 0};
+  ReduceNormArgs a = {y, xout, parts, nparts, part_stride, bias, resid, g, b, eps, rows, n, terms == kTermsPlanes || terms == kTermsOperands ? (unsigned short *)y : nullptr,
+                      terms == kTermsOperands ? (int)(rows + 15) / 16 : 0, terms == kTermsDigits ? (unsigned char *)y : nullptr};
   hipStream_t st = state().stream;
-  const ReduceNormPlan pl = reduce_norm_plan(n, nparts, rows);
+  ReduceNormPlan pl = reduce_norm_plan(n, nparts, rows);
+  if (a.digits && !pl.wide) {  // digits take a workgroup per row (whose registers hold whatever one wavefront's would)
+    const int v4 = (n / 4 + 255) / 256;
+    pl.wide = true;
+    pl.vpl = v4 <= 1 ? 1 : v4 <= 2 ? 2 : v4 <= 4 ? 4 : 8;
+  }
   if (pl.wide) {
     const int vplw = pl.vpl;
     dim3 gridw((unsigned)rows), blockw(256);
@@ -1586,7 +1607,7 @@ __device__ __forceinline__ void split8(const float *x, v8bf_t &hi, v8bf_t &lo) {
 template <int DH, int NW>
 __global__ __launch_bounds__(64 * NW) void k_attn_mfma_bf(float *__restrict__ out, const float *__restrict__ q,
                                                       const float *__restrict__ kc, const float *__restrict__ vc, int S,
-                                                      int start_pos, int H, int Hkv) {
+                                                      int start_pos, int H, int Hkv, unsigned char *__restrict__ digits) {
   constexpr int NSL = DH / 16;  // 16-wide slices of the head dimension in K Q^T
   constexpr int DB = DH / 32;   // 32-wide blocks of the head dimension
   constexpr int KP = DH + 8;    // row pitch of the bf16 key tile: 16-byte reads of 8 consecutive rows hit all banks
@@ -1733,16 +1754,39 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma_bf(float *__restrict__ ou
     L = fmaf(e[w], Cl[w][lane], L);
   }
   const float inv = 1.0f / L;
-  if (i0 + col < S) {
-    float *orow = out + ((int64_t)(i0 + col) * H + h) * DH;
-    constexpr int RPW = DB * 16 / NW;  // wavefront wv finishes registers wv * RPW .. of every lane
+  constexpr int RPW = DB * 16 / NW;  // wavefront wv finishes registers wv * RPW .. of every lane
+  float res[RPW];
+#pragma unroll
+  for (int k = 0; k < RPW; k++) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) v = fmaf(e[w], W[w].Co[wv * RPW + k][lane], v);
+    res[k] = v * inv;
+  }
+  if (digits) {  // for gemm_digits.hip: a block of 32 of a row to a thread, through the memory of the query rows
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < RPW; k++) {
       const int R = wv * RPW + k, b = R >> 4, r = R & 15;
-      float v = 0.0f;
+      Qs[col][32 * b + 8 * (r >> 2) + 4 * half + (r & 3)] = res[k];
+    }
+    __syncthreads();
+    const int row = tid & 31, b = tid >> 5;
+    if (b < DB && i0 + row < S) {
+      float v[32];
 #pragma unroll
-      for (int w = 0; w < NW; w++) v = fmaf(e[w], W[w].Co[R][lane], v);
-      orow[32 * b + 8 * (r >> 2) + 4 * half + (r & 3)] = v * inv;
+      for (int q4 = 0; q4 < 8; q4++) {
+        const float4 t = *(const float4 *)&Qs[row][32 * b + 4 * q4];
+        v[4 * q4] = t.x, v[4 * q4 + 1] = t.y, v[4 * q4 + 2] = t.z, v[4 * q4 + 3] = t.w;
+      }
+      store_digits32(digits, (int64_t)(S + 31) / 32 * 32, H * DH / 32, i0 + row, (h * DH >> 5) + b, v);
+    }
+  } else if (i0 + col < S) {
+    float *orow = out + ((int64_t)(i0 + col) * H + h) * DH;
+#pragma unroll
+    for (int k = 0; k < RPW; k++) {
+      const int R = wv * RPW + k, b = R >> 4, r = R & 15;
+      orow[32 * b + 8 * (r >> 2) + 4 * half + (r & 3)] = res[k];
     }
   }
 }
@@ -1762,8 +1806,9 @@ int launch_attn_parts(const float *q, const float *kc, const float *vc, const in
 }
 
 int launch_attn(float *out, const float *q, const float *kc, const float *vc, int S, int start_pos, const int *pos,
-                int max_T, int H, int Hkv, int Dh, const AttnSplit *split) {
+                int max_T, int H, int Hkv, int Dh, const AttnSplit *split, void *digits) {
   if (S == 0) return 0;
+  if (digits && !attn_digits_supported(S, Dh)) return fail(CTHIP_E_STATE, "attention: %d rows, heads of %d as digits", S, Dh);
   (void)max_T;
   hipStream_t st = state().stream;
   // Prompt rows on the matrix cores.  16 .. 31 rows with fp32 operands, as the kernels for fewer have them: a key tile is 4096 cycles whatever the rows, so that
@@ -1793,9 +1838,9 @@ int launch_attn(float *out, const float *q, const float *kc, const float *vc, in
       }
     } else {  // two bf16 terms per operand, whatever the GEMMs use
       switch (Dh) {
-        case 32: hipLaunchKernelGGL((k_attn_mfma_bf<32, 8>), grid, dim3(512), 0, st, out, q, kc, vc, S, start_pos, H, Hkv); break;
-        case 64: hipLaunchKernelGGL((k_attn_mfma_bf<64, 8>), grid, dim3(512), 0, st, out, q, kc, vc, S, start_pos, H, Hkv); break;
-        case 128: hipLaunchKernelGGL((k_attn_mfma_bf<128, 4>), grid, dim3(256), 0, st, out, q, kc, vc, S, start_pos, H, Hkv); break;
+        case 32: hipLaunchKernelGGL((k_attn_mfma_bf<32, 8>), grid, dim3(512), 0, st, out, q, kc, vc, S, start_pos, H, Hkv, (unsigned char *)digits); break;
+        case 64: hipLaunchKernelGGL((k_attn_mfma_bf<64, 8>), grid, dim3(512), 0, st, out, q, kc, vc, S, start_pos, H, Hkv, (unsigned char *)digits); break;
+        case 128: hipLaunchKernelGGL((k_attn_mfma_bf<128, 4>), grid, dim3(256), 0, st, out, q, kc, vc, S, start_pos, H, Hkv, (unsigned char *)digits); break;
         default: return fail(CTHIP_E_UNSUPPORTED, "attention: head_dim %d (supported: 32, 64, 128)", Dh);
       }
     }

@@ -1,0 +1,95 @@
+"""Linears over many rows on 4-bit weights, whose operands lie as 6-bit digits (csrc/gemm_digits.hip): every tile, with one share of K and several, at edges that
+no tile divides and odd numbers of blocks; rows of any magnitude and rows that are not finite; prompts, whose norms, attention and GELU / SwiGLU write digits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from caten_amd import _lib, ops as o
+    _lib.init(0)
+    return o
+
+
+def weights(ops, rows, cols, rng):
+    from caten_amd.llm import Tensor
+    return ops.WeightMatrix("q4_0", Tensor.from_f32(rng.normal(0, 0.05, (rows, cols)).astype(np.float32), "q4_0").raw, rows, cols)
+
+
+def bound(x, w):
+    """2^-19 of the largest value of a block of 32 goes with every value of it (csrc/digits.h), and fp32 sums of at most K terms, here in runs of 32, round K / 32 + 32 times."""
+    xb, wb = np.abs(x).reshape(len(x), -1, 32), np.abs(w).reshape(len(w), -1, 32)
+    return 2.0 ** -19 * xb.max(-1) @ wb.sum(-1).T + (x.shape[1] / 32 + 32) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
+
+
+# tile 64 x 64 with 1, 3, 5 shares; 64 x 128 with few workgroups (1, 2, 4, 7 shares) and many; 128 x 128 with 1, 2, 5 shares
+@pytest.mark.parametrize("rows,cols,m", [(3001, 64, 2049), (9001, 64, 701), (1026, 4128, 513), (514, 8224, 577),
+                                         (6401, 96, 577), (2051, 288, 1025), (4100, 4128, 129), (6401, 4128, 65), (4100, 8224, 97), (6401, 64, 1537),
+                                         (12001, 288, 1537), (3001, 544, 2049), (2051, 8224, 701), (2051, 8224, 577)])
+def test_linear_digits(ops, rows, cols, m):
+    rng = np.random.default_rng(rows + m)
+    w = weights(ops, rows, cols, rng)
+    x = rng.normal(0, 1, (m, cols)).astype(np.float32) * np.exp2(rng.integers(-20, 20, (m, 1))).astype(np.float32)
+    x[:, ::37] *= 50.0
+    at, rs = np.unique(np.r_[0:40, rows - 40:rows, rng.integers(0, rows, 60)]), np.unique(np.r_[0:9, m - 9:m, rng.integers(0, m, 40)])
+    x64, w64 = x[rs].astype(np.float64), w.dequantize()[at].astype(np.float64)
+    want, most = x64 @ w64.T, bound(x64, w64)
+    for _ in range(2):  # with the matrix's digits made, and as they are kept
+        got = ops.linear(x, w)[np.ix_(rs, at)]
+        assert np.all(np.abs(got - want) <= most)
+    bias, res = rng.normal(0, 1, rows).astype(np.float32), rng.normal(0, 1, (m, rows)).astype(np.float32)
+    ends = 4 * 2.0 ** -24 * (np.abs(want) + np.abs(bias[at]) + np.abs(res[rs][:, at]))
+    got = ops.linear(x, w, bias, res)[np.ix_(rs, at)]
+    assert np.all(np.abs(got - (want + bias[at] + res[rs][:, at])) <= most + ends)
+    got = ops.linear(x, w, bias, act="relu")[np.ix_(rs, at)]
+    assert np.all(np.abs(got - np.maximum(want + bias[at], 0.0)) <= most + ends)
+    w.free()
+
+
+def test_rows_of_any_magnitude_and_rows_that_are_not_finite(ops):
+    rng = np.random.default_rng(5)
+    w = weights(ops, 4100, 4128, rng)
+    w64 = w.dequantize().astype(np.float64)
+    x = rng.normal(0, 1, (129, 4128)).astype(np.float32)
+    scale = np.array([1e-25, 1e-20, 1e-10, 1.0, 1e10, 1e30, 1e33] * 19)[:129]  # (1e-25: every digit of a block is a normal power of two)
+    x = (x * scale[:, None]).astype(np.float32)
+    x[7] = 0.0
+    x[8, 100:] = 0.0
+    x[40, 5], x[41, 4127], x[42, 64] = np.inf, -np.inf, np.nan
+    got = ops.linear(x, w)
+    odd = np.arange(129)[~np.isfinite(x).all(1)]
+    assert list(odd) == [40, 41, 42]
+    assert np.isnan(got[odd]).all()
+    fine = np.setdiff1d(np.arange(129), odd)
+    x64 = x[fine].astype(np.float64)
+    assert np.all(np.abs(got[fine] - x64 @ w64.T) <= bound(x64, w64))
+    assert not got[7].any()
+    w.free()
+
+
+@pytest.mark.parametrize("arch,kinds,rows", [("gpt2", ("q4_0", "q4_0"), 65), ("gpt2", ("q4_0", "q4_0"), 223), ("gpt2", ("q4_0", "q4_0"), 897), ("gpt2", ("q4_0", "q8_0"), 700),
+                                             ("gpt2", ("q8_0", "q4_0"), 700), ("llama", ("q4_0", "q4_0"), 96), ("llama", ("q4_0", "q4_0"), 333), ("llama", ("q4_0", "q8_0"), 1300)])
+def test_prompt_equals_short_pieces(ops, arch, kinds, rows):
+    """kinds: of the Linears behind a norm, and of the attention projection and the second MLP Linear; pieces of 63 rows take other kernels."""
+    from caten_amd import llm, synth
+    if arch == "llama":
+        cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=1024, n_heads=16, n_kv_heads=4, ffn=2816, n_layers=3, vocab=500, max_seq=2048)
+        w = synth.llama_weights(cfg, seed=3)
+        make, dicts = llm.make_llama, [llm.llama_state_dict(w, k) for k in kinds]
+    else:
+        cfg = dict(synth.GPT2_CONFIGS["gpt2"], dim=1024, n_heads=16, n_layers=3, vocab=500, max_seq=2048)
+        w = synth.gpt2_weights(cfg, seed=3)
+        make, dicts = llm.make_gpt2, [llm.gpt2_state_dict(w, k) for k in kinds]
+    behind = ("attn.c_proj.weight", "mlp.c_proj.weight", "attention.wo.weight", "feed_forward.w2.weight")
+    model = make(cfg, {k: dicts[1][k] if k.endswith(behind) else dicts[0][k] for k in dicts[0]})
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], rows + 1, seed=3)]
+    got = [model.forward(ids[:rows], rows, 0, return_logits=True), model.forward(ids[rows:], 1, rows, return_logits=True)]
+    for n in range(0, rows, 63):
+        want = [model.forward(ids[n:min(n + 63, rows)], min(63, rows - n), n, return_logits=True)]
+    want.append(model.forward(ids[rows:], 1, rows, return_logits=True))
+    for (t0, l0), (t1, l1) in zip(got, want):
+        assert t0 == t1
+        assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
+    model.close()
