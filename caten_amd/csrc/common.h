@@ -401,6 +401,12 @@ __device__ __forceinline__ float group_max(float v) {
   return v;
 }
 
+// An argument that a kernel's end needs, loaded where this stands: left alone each is loaded right in front of its use, and an epilogue is a chain of scalar loads.
+template <typename T>
+__device__ __forceinline__ T early(T x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
 typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte access at 4-byte alignment
 
 __device__ __forceinline__ float half_bits_to_float(unsigned short h) {

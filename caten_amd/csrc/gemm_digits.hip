@@ -38,6 +38,8 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
   const int b0 = tile / (a.band * a.tn), inb = tile - b0 * a.band * a.tn, height = min(a.band, a.tm - b0 * a.band);
   const int mi = b0 * a.band + inb % height, ni = inb / height;
   const int m0 = mi * BM, n0 = ni * BN;
+  const PlaneStore store(a);
+  unsigned char *const digits = early(a.digits);
   const int nkb = a.nkb, k0 = blockIdx.y * a.kper, nsteps = min(a.kper, nkb - k0);  // of this share (none is empty)
 
   // where this lane's pieces of a step lie, as offsets from the step's bases; groups of rows past the end repeat the last one
@@ -179,15 +181,9 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
   constexpr int LDC = 32 * NB + 4, C4 = 8 * NB;
   float *Cs = (float *)smem + wave * 32 * LDC;
   const int col0 = n0 + 32 * NB * wn, c4 = lane % C4, at = col0 + 4 * c4;  // a lane stores the same four columns of every 64 / C4-th row
-  const bool rows4 = a.N % 4 == 0 && a.act == CTHIP_ACT_NONE && !a.pairs && !a.planes && !a.routed;  // rows of whole pieces of four floats, with a residual or without
 #pragma unroll
   for (int i = 0; i < MB; i++) {
     const int row0 = m0 + 32 * (MB * wm + i);
-    constexpr int NU = OUT == kDigitsPlain ? 32 * C4 / 64 : 1;
-    float4 rr[NU];
-    if (OUT == kDigitsPlain && rows4 && a.residual)  // (asked for in front of the turn: piece by piece each is a round trip to memory)
-#pragma unroll
-      for (int u = 0; u < NU; u++) rr[u] = *(const float4 *)(a.residual + (int64_t)min(row0 + lane / C4 + u * (64 / C4), a.M - 1) * a.N + min(at, a.N - 4));
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
@@ -199,7 +195,7 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
 #pragma unroll 1
       for (int u = lane; u < 32 * NB / PER; u += 64) {
         const int c = (u >> 5) * 32 * PER, row = row0 + col;
-        if (row >= a.M || col0 + c >= a.N) continue;
+        if (row >= store.M || col0 + c >= store.N) continue;
         const float *p = Cs + col * LDC + c;
         float v[32];
 #pragma unroll
@@ -208,38 +204,28 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
           if (PER == 2) v[2 * q] = ct_silu(t.x) * t.y, v[2 * q + 1] = ct_silu(t.z) * t.w;
           else v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
         }
-        if (PER == 1 && a.act == CTHIP_ACT_GELU) {
+        if (PER == 1 && store.act == CTHIP_ACT_GELU) {
 #pragma unroll
           for (int q = 0; q < 32; q++) v[q] = ct_gelu(v[q]);
         }
-        store_digits32(a.digits, (int64_t)mg * 32, a.pkb, row, (col0 + c) / (32 * PER), v);
+        store_digits32(digits, (int64_t)mg * 32, store.pkb, row, (col0 + c) / (32 * PER), v);
       }
-    } else if (OUT == kDigitsPlain && rows4) {
-#pragma unroll
-      for (int u = 0; u < NU; u++) {
-        const int r = lane / C4 + u * (64 / C4);
-        float4 v = *(const float4 *)(Cs + r * LDC + 4 * c4);
-        if (a.residual) v.x += rr[u].x, v.y += rr[u].y, v.z += rr[u].z, v.w += rr[u].w;
-        if (row0 + r < a.M && at < a.N) *(float4 *)(a.C + (int64_t)(row0 + r) * a.N + at) = v;
-      }
+    } else if constexpr (OUT == kDigitsPlain) {
+      plane_gemm_store_rows<NB>(store, Cs, row0, col0, lane, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     } else {
 #pragma unroll 1
       for (int r = lane / C4; r < 32; r += 64 / C4) {
         const int row = row0 + r;
         const float4 v = *(const float4 *)(Cs + r * LDC + 4 * c4);
-        if (row >= a.M || at >= a.N) continue;
-        if (OUT == kDigitsPlain) {
-          plane_gemm_store(a, row, at, v);
+        if (row >= store.M || at >= store.N) continue;
+        float *p = store.C + ((int64_t)blockIdx.y * store.M + row) * store.N + at;
+        if (store.N % 4 == 0) {
+          *(float4 *)p = v;
         } else {
-          float *p = a.C + ((int64_t)blockIdx.y * a.M + row) * a.N + at;
-          if (a.N % 4 == 0) {
-            *(float4 *)p = v;
-          } else {
-            p[0] = v.x;
-            if (at + 1 < a.N) p[1] = v.y;
-            if (at + 2 < a.N) p[2] = v.z;
-            if (at + 3 < a.N) p[3] = v.w;
-          }
+          p[0] = v.x;
+          if (at + 1 < store.N) p[1] = v.y;
+          if (at + 2 < store.N) p[2] = v.z;
+          if (at + 3 < store.N) p[3] = v.w;
         }
       }
     }

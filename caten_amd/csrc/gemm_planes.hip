@@ -67,6 +67,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
   const int mi = b0 * a.band + inb % height, ni = inb / height;
   const int m0 = mi * BM, n0 = ni * BN;
   const int nsteps = a.nkb;
+  const PlaneStore store(a);
 
   // where this lane's pieces of a step lie, as offsets from the step's bases; rows past the end repeat the last one
   unsigned avo[IA], bvo[IB], svo[IS > 0 ? IS : 1];
@@ -85,19 +86,26 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
     const int s = ((j * NW + wave) * 64 + lane) % BN;
     svo[j] = (unsigned)(min(s, a.N - 1 - n0) * a.dpitch) * 2u;
   }
-  const unsigned char *ab = a.A + (int64_t)m0 * a.apitch;
+  const unsigned char *ab = a.A + (int64_t)m0 * a.apitch;  // of the next step to ask for
   const unsigned char *bb = a.B + (int64_t)n0 * a.bpitch;
   const unsigned char *sb = SRC == PL_PLANES ? nullptr : (const unsigned char *)(a.bd + (int64_t)n0 * a.dpitch);
-  auto issue = [&](int step, int buf) __attribute__((always_inline)) {
-    step = min(step, nsteps - 1);  // past the end: the last step again, so that the counts stay the same
-    const unsigned base = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)buf * BUF);
-    const unsigned char *as = uniform(ab + (int64_t)step * (CA * 16)), *bs = uniform(bb + (int64_t)step * (CB * 16));
+  unsigned al[IA], bl[IB], sl[IS > 0 ? IS : 1];  // where its pieces go, in the first buffer
 #pragma unroll
-    for (int j = 0; j < IA; j++) dma16(as, avo[j], base + ((j * NW + wave) * 1024) % ABYTES);
+  for (int j = 0; j < IA; j++) al[j] = lds0 + ((j * NW + wave) * 1024) % ABYTES;
 #pragma unroll
-    for (int j = 0; j < IB; j++) dma16(bs, bvo[j], base + ABYTES + ((j * NW + wave) * 1024) % BBYTES);
+  for (int j = 0; j < IB; j++) bl[j] = lds0 + ABYTES + ((j * NW + wave) * 1024) % BBYTES;
 #pragma unroll
-    for (int j = 0; j < IS; j++) dma2(uniform(sb + (int64_t)step * 2), svo[j], base + ABYTES + BBYTES + ((j * NW + wave) * 256) % (SBYTES ? SBYTES : 1));
+  for (int j = 0; j < IS; j++) sl[j] = lds0 + ABYTES + BBYTES + ((j * NW + wave) * 256) % (SBYTES ? SBYTES : 1);
+  int left = nsteps;  // steps to ask for
+  auto issue = [&](int buf) __attribute__((always_inline)) {
+    const unsigned char *as = uniform(ab), *bs = uniform(bb);
+#pragma unroll
+    for (int j = 0; j < IA; j++) dma16(as, avo[j], al[j] + buf * BUF);
+#pragma unroll
+    for (int j = 0; j < IB; j++) dma16(bs, bvo[j], bl[j] + buf * BUF);
+#pragma unroll
+    for (int j = 0; j < IS; j++) dma2(uniform(sb), svo[j], sl[j] + buf * BUF);
+    if (--left > 0) ab += CA * 16, bb += CB * 16, sb += 2;  // past the end: the last step again, so that the counts stay the same
   };
 
   v16f acc[MB][NB];
@@ -109,6 +117,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
       for (int r = 0; r < 16; r++) acc[i][b][r] = 0.0f;
 
   const int half = lane >> 5, col = lane & 31;
+  constexpr bool EARLY = MB * NB < 8;  // (registers for it)
+  float4 bias;
+  if (EARLY) bias = plane_gemm_bias<NB>(store, n0 + 32 * NB * wn, lane);
   // k of the matrix instructions of a block: slice s, lane half h take k = 16 h + 8 s .. +7 (the same for A and B)
   v16f tmp[2][SRC == PL_INT ? MB : 1] = {};  // PL_INT: partial sums of a block of 32 k, unscaled
   float dlast = 0.0f;
@@ -195,14 +206,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
 
   if (nsteps > 0) {
 #pragma unroll
-    for (int s = 0; s < NBUF - 1; s++) issue(s, s);
-    int buf = 0;
-    for (int i = 0; i < nsteps; i++) {
-      wait_barrier<LOADS *(NBUF - 2)>();  // step i has landed; nobody reads the buffer of step i - 1 any more
-      issue(i + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
-      mul(buf);
-      buf = buf + 1 == NBUF ? 0 : buf + 1;
-    }
+    for (int s = 0; s < NBUF - 1; s++) issue(s);
+    // Its buffer known to the compiler, a step has fewer instructions: where an LDS instruction's offset reaches all of them (256 x 256 at two terms: 362 us rolled, 398 not).
+    constexpr bool UNROLL = NBUF * BUF <= 80 * 1024;
+    int b0 = 0;
+    for (int i = 0; i < nsteps;)
+#pragma unroll
+      for (int b1 = 0; b1 < (UNROLL ? NBUF : 1); b1++) {
+        const int buf = UNROLL ? b1 : b0;
+        wait_barrier<LOADS *(NBUF - 2)>();  // step i has landed; nobody reads the buffer of step i - 1 any more
+        issue(buf == 0 ? NBUF - 1 : buf - 1);
+        mul(buf);
+        b0 = b0 + 1 == NBUF ? 0 : b0 + 1;
+        if (++i == nsteps) break;
+      }
   }
   wait_barrier<0>();
   if (SRC == PL_INT && NB % 2 == 0)
@@ -213,7 +230,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
 
   // ---- acc[i][b][r] is row 8 (r / 4) + 4 half + r % 4, column `col` of its block.  A wavefront turns its blocks around
   // in a piece of LDS of its own (no barrier) and stores rows of 32 NB columns, 16 bytes per lane.
-  constexpr int LDC = 32 * NB + 4, C4 = 8 * NB;
+  if (!EARLY) bias = plane_gemm_bias<NB>(store, n0 + 32 * NB * wn, lane);
+  constexpr int LDC = 32 * NB + 4;
   float *Cs = (float *)smem + wave * 32 * LDC;
 #pragma unroll
   for (int i = 0; i < MB; i++) {
@@ -222,12 +240,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_planes(PlaneGemmArgs a
 #pragma unroll
       for (int r = 0; r < 16; r++) Cs[(8 * (r >> 2) + 4 * half + (r & 3)) * LDC + 32 * b + col] = acc[i][b][r];
     __builtin_amdgcn_wave_barrier();
-#pragma unroll 2  // (a body small enough that the loop over i is unrolled for certain: acc has to stay in registers)
-    for (int u = 0; u < 32 * C4 / 64; u++) {
-      const int f = lane + 64 * u, lr = f / C4, c4 = f % C4;
-      const float4 v = *(const float4 *)(Cs + lr * LDC + 4 * c4);
-      plane_gemm_store(a, m0 + 32 * (MB * wm + i) + lr, n0 + 32 * NB * wn + 4 * c4, v);
-    }
+    plane_gemm_store_rows<NB, EARLY ? 4 : 1>(store, Cs, m0 + 32 * (MB * wm + i), n0 + 32 * NB * wn, lane, bias);
     __builtin_amdgcn_wave_barrier();
   }
 }

@@ -115,8 +115,19 @@ __device__ __forceinline__ v8bf bf_of_q8(unsigned a, unsigned b) {
   return __builtin_bit_cast(v8bf, make_uint4(pack_int_bf16(sbyte0_f32(a), sbyte1_f32(a)), pack_int_bf16(sbyte2_f32(a), sbyte3_f32(a)),
                                              pack_int_bf16(sbyte0_f32(b), sbyte1_f32(b)), pack_int_bf16(sbyte2_f32(b), sbyte3_f32(b))));
 }
-// columns col .. col + 3 of one row of a finished tile, rows of whole pieces of four: bias bb (where a.bias), activation, residual rr (where a.residual), and where they go
-__device__ __forceinline__ void plane_gemm_finish(const PlaneGemmArgs &a, int N, int row, int col, float4 v4, float4 bb, float4 rr) {
+// What the end of a kernel needs of its arguments, loaded where this is made
+struct PlaneStore {
+  float *C;
+  const float *bias, *residual;
+  unsigned short *planes;
+  int M, N, act, pairs, routed, pkb;
+  const GemmRoute &route;
+  __device__ __forceinline__ PlaneStore(const PlaneGemmArgs &a)
+      : C(early(a.C)), bias(early(a.bias)), residual(early(a.residual)), planes(early(a.planes)), M(early(a.M)), N(early(a.N)), act(early(a.act)), pairs(early(a.pairs)),
+        routed(early(a.routed)), pkb(early(a.pkb)), route(a.route) {}
+};
+// columns col .. col + 3, all of them inside, of one row of a finished tile: bias bb (where a.bias), activation, residual rr (where a.residual), and where they go
+__device__ __forceinline__ void plane_gemm_finish(const PlaneStore &a, int N, int row, int col, float4 v4, float4 bb, float4 rr) {
   float v[4] = {v4.x, v4.y, v4.z, v4.w};
   if (a.bias) v[0] += bb.x, v[1] += bb.y, v[2] += bb.z, v[3] += bb.w;
   if (a.pairs) {
@@ -149,26 +160,119 @@ __device__ __forceinline__ void plane_gemm_finish(const PlaneGemmArgs &a, int N,
     ldd = p2 ? a.route.ld[2] : p1 ? a.route.ld[1] : a.route.ld[0];
     cbase = p2 ? a.route.c0[2] : p1 ? a.route.c0[1] : 0;
   }
-  *(float4 *)(dst + (int64_t)row * ldd + (col - cbase)) = make_float4(v[0], v[1], v[2], v[3]);
+  *(f4_any *)(dst + (int64_t)row * ldd + (col - cbase)) = f4_any{v[0], v[1], v[2], v[3]};
 }
-// the same for any rows, bias and residual from memory
+// the same where a row ends within them
+__device__ __forceinline__ void plane_gemm_finish_any(const PlaneStore &a, int row, int col, float4 v4) {
+  const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+  for (int t = 0; t < 4 && col + t < a.N; t++) {
+    float x = apply_act(a.act, v[t] + (a.bias ? a.bias[col + t] : 0.0f));
+    if (a.residual) x += a.residual[(int64_t)row * a.N + col + t];
+    a.C[(int64_t)row * a.N + col + t] = x;
+  }
+}
+// columns col .. col + 3 of one row: the same for the kernels of a few rows, which ask for bias and residual as they go
 __device__ __forceinline__ void plane_gemm_store(const PlaneGemmArgs &a, int row, int col, float4 v4) {
   int N = a.N;
   asm volatile("" : "+s"(N));  // read anew at every call: known to be the same, it has the caller's loop copied for each case below (3000 x 4100 x 5000: 2.4 % slower)
   if (row >= a.M || col >= N) return;
+  float v[4] = {v4.x, v4.y, v4.z, v4.w};
   if ((N & 3) == 0) {
-    float4 bb = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rr = bb;
-    if (a.bias) bb = *(const float4 *)(a.bias + col);
-    if (a.residual && !a.pairs) rr = *(const float4 *)(a.residual + (int64_t)row * N + col);
-    plane_gemm_finish(a, N, row, col, v4, bb, rr);
+    if (a.bias) {
+      const float4 bb = *(const float4 *)(a.bias + col);
+      v[0] += bb.x, v[1] += bb.y, v[2] += bb.z, v[3] += bb.w;
+    }
+    if (a.pairs) {
+      v[0] = apply_act(CTHIP_ACT_SILU, v[0]) * v[1], v[1] = apply_act(CTHIP_ACT_SILU, v[2]) * v[3];
+      if (a.planes) {  // two columns of the result: neighbours in both terms
+        const unsigned h = pack_bf16_pl(v[0], v[1]);
+        const unsigned l = pack_bf16_pl(v[0] - __uint_as_float(h << 16), v[1] - __uint_as_float(h & 0xffff0000u));
+        unsigned short *p = a.planes + ((int64_t)row * a.pkb + (col >> 6)) * 64 + ((col >> 1) & 31);
+        *(unsigned *)p = h;
+        *(unsigned *)(p + 32) = l;
+      } else {
+        *(float2 *)(a.C + (int64_t)row * (N >> 1) + (col >> 1)) = make_float2(v[0], v[1]);
+      }
+      return;
+    }
+    if (a.act != CTHIP_ACT_NONE)
+#pragma unroll
+      for (int t = 0; t < 4; t++) v[t] = apply_act(a.act, v[t]);
+    if (a.residual) {
+      const float4 rr = *(const float4 *)(a.residual + (int64_t)row * N + col);
+      v[0] += rr.x, v[1] += rr.y, v[2] += rr.z, v[3] += rr.w;
+    }
+    if (a.planes) {
+      store_planes4(a.planes, row, a.pkb, col, v);
+      return;
+    }
+    float *dst = a.C;
+    int ldd = N, cbase = 0;
+    if (a.routed) {
+      // (selected, not indexed: an index would put the arguments into scratch memory)
+      const bool p2 = col >= a.route.c0[2], p1 = col >= a.route.c0[1];
+      dst = p2 ? a.route.dst[2] : p1 ? a.route.dst[1] : a.route.dst[0];
+      ldd = p2 ? a.route.ld[2] : p1 ? a.route.ld[1] : a.route.ld[0];
+      cbase = p2 ? a.route.c0[2] : p1 ? a.route.c0[1] : 0;
+    }
+    *(float4 *)(dst + (int64_t)row * ldd + (col - cbase)) = make_float4(v[0], v[1], v[2], v[3]);
     return;
   }
-  const float v[4] = {v4.x, v4.y, v4.z, v4.w};
   for (int t = 0; t < 4 && col + t < N; t++) {
     float x = apply_act(a.act, v[t] + (a.bias ? a.bias[col + t] : 0.0f));
     if (a.residual) x += a.residual[(int64_t)row * N + col + t];
     a.C[(int64_t)row * N + col + t] = x;
   }
+}
+// A wavefront's 32 rows of 32 NB columns, which lie in LDS (pitch 32 NB + 4), to where they go.  A lane stores the same four columns of every 64 / C4-th row, so that their bias is
+// read once, by plane_gemm_bias, long before; the residual of plain rows is asked for several rows at a time.  Short code: with every row's
+// cases copied out a kernel was 14 - 50 KB, now 8 - 33, and a launch of a few steps waited for its instructions (4500 x 4500 x 600 at one term 59.7 -> 53.6 us with
+// the shorter step, Q8_0 3072 x 1024 over 900 rows 31.1 -> 27.7).
+template <int NB>
+__device__ __forceinline__ float4 plane_gemm_bias(const PlaneStore &a, int col0, int lane) {
+  if (!a.bias) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const f4_any t = *(const f4_any *)(a.bias + min(col0 + 4 * (lane % (8 * NB)), a.N - 4));
+  return make_float4(t[0], t[1], t[2], t[3]);
+}
+template <int NB, int AHEAD = 4>
+__device__ __forceinline__ void plane_gemm_store_rows(const PlaneStore &a, const float *Cs, int row0, int col0, int lane, float4 bias) {
+  constexpr int LDC = 32 * NB + 4, C4 = 8 * NB, RPI = 64 / C4, NU = 32 / RPI;  // rows per instruction
+  const int lr = lane / C4, c4 = lane % C4, at = col0 + 4 * c4;
+  const bool mine = lr < RPI && at + 4 <= a.N;  // (16-byte accesses at any alignment: rows of N floats)
+  const float *p = Cs + lr * LDC + 4 * c4;
+  if (a.act == CTHIP_ACT_NONE && !a.pairs && !a.planes && !a.routed) {
+#pragma unroll
+    for (int u0 = 0; u0 < NU; u0 += AHEAD) {
+      f4_any rr[AHEAD];
+      if (a.residual)
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) rr[u] = *(const f4_any *)(a.residual + (int64_t)min(row0 + lr + (u0 + u) * RPI, a.M - 1) * a.N + min(at, a.N - 4));
+#pragma unroll
+      for (int u = 0; u < AHEAD; u++) {
+        const int row = row0 + lr + (u0 + u) * RPI;
+        float4 v = *(const float4 *)(p + (u0 + u) * RPI * LDC);
+        if (a.bias) v.x += bias.x, v.y += bias.y, v.z += bias.z, v.w += bias.w;
+        if (a.residual) v.x += rr[u][0], v.y += rr[u][1], v.z += rr[u][2], v.w += rr[u][3];
+        if (mine && row < a.M) *(f4_any *)(a.C + (int64_t)row * a.N + at) = f4_any{v.x, v.y, v.z, v.w};
+      }
+    }
+  } else {
+#pragma unroll 1
+    for (int u = 0; u < NU; u++) {
+      const int row = row0 + lr + u * RPI;
+      const float4 v = *(const float4 *)(p + u * RPI * LDC);
+      if (!mine || row >= a.M) continue;
+      float4 rr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (a.residual && !a.pairs) {
+        const f4_any t = *(const f4_any *)(a.residual + (int64_t)row * a.N + at);
+        rr = make_float4(t[0], t[1], t[2], t[3]);
+      }
+      plane_gemm_finish(a, a.N, row, at, v, bias, rr);
+    }
+  }
+  if (a.N % 4 && lr < RPI && at < a.N && at + 4 > a.N)
+#pragma unroll 1
+    for (int r = lr; r < min(32, a.M - row0); r += RPI) plane_gemm_finish_any(a, row0 + r, at, *(const float4 *)(Cs + r * LDC + 4 * c4));
 }
 #endif
 

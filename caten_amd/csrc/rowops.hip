@@ -213,10 +213,10 @@ __global__ __launch_bounds__(256) void k_reduce_norm(ReduceNormArgs a) {
 // true if the fused pass can take this shape (otherwise the caller reduces and normalises in two launches)
 // The same with four wavefronts per row (rows too wide, or with too many shares, for one wavefront's registers):
 // thread t of the row's 256 owns float4 t + 256 j, the row statistics meet in LDS.
-template <int MODE, int VPL, int NZ>
+template <int MODE, int VPL, int NZ, bool DIGITS>
 __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
   __shared__ float red[2][4];
-  __shared__ __align__(16) float turn[VPL * 32 * 36];  // digits: a thread's four values -> blocks of 32, 36 apart (no bank twice)
+  __shared__ __align__(16) float turn[DIGITS ? VPL * 32 * 36 : 4];  // digits: a thread's four values -> blocks of 32, 36 apart (no bank twice)
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t row = blockIdx.x;
   const int n = a.n, n4 = n >> 2;
@@ -280,13 +280,13 @@ __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
       const float4 g = a.g ? gm[j] : make_float4(1.f, 1.f, 1.f, 1.f);
       const float4 b = a.b ? bt[j] : make_float4(0.f, 0.f, 0.f, 0.f);
       const float o[4] = {v[j][0] * rstd * g.x + b.x, v[j][1] * rstd * g.y + b.y, v[j][2] * rstd * g.z + b.z, v[j][3] * rstd * g.w + b.w};
-      if (a.digits) *(float4 *)&turn[(tid / 8 + 32 * j) * 36 + 4 * (tid % 8)] = make_float4(o[0], o[1], o[2], o[3]);
+      if (DIGITS) *(float4 *)&turn[(tid / 8 + 32 * j) * 36 + 4 * (tid % 8)] = make_float4(o[0], o[1], o[2], o[3]);
       else if (a.planes && a.row_blocks) store_operands4(a.planes, (int)row, a.row_blocks, 4 * (tid + 256 * j), o);
       else if (a.planes) store_planes4(a.planes, row, n >> 5, 4 * (tid + 256 * j), o);
       else ((float4 *)(a.y + row * n))[tid + 256 * j] = make_float4(o[0], o[1], o[2], o[3]);
     }
   }
-  if (a.digits) {
+  if (DIGITS) {
     __syncthreads();
     if (tid < n >> 5) {  // (at most 32 VPL <= 256 blocks)
       float f[32];
@@ -319,7 +319,11 @@ int launch_reduce_norm(float *y, float *xout, const float *parts, int nparts, in
   if (pl.wide) {
     const int vplw = pl.vpl;
     dim3 gridw((unsigned)rows), blockw(256);
-#define RW3(MODE, V, Z) hipLaunchKernelGGL((k_reduce_norm_wide<MODE, V, Z>), gridw, blockw, 0, st, a)
+#define RW3(MODE, V, Z)                                                                                     \
+    do {                                                                                                    \
+      if (a.digits) hipLaunchKernelGGL((k_reduce_norm_wide<MODE, V, Z, true>), gridw, blockw, 0, st, a);    \
+      else hipLaunchKernelGGL((k_reduce_norm_wide<MODE, V, Z, false>), gridw, blockw, 0, st, a);            \
+    } while (0)
 #define RW2(MODE, V)                       \
     if (nparts <= 2) RW3(MODE, V, 2);      \
     else if (nparts <= 4) RW3(MODE, V, 4); \
