@@ -970,9 +970,10 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // workgroups per tile leaves partial tiles; what follows it is the residual add and the next norm, so one pass
     // over the rows does all three (launch_reduce_norm) instead of a reduction launch and a norm launch.
     // Many rows: a Linear takes its input as two bf16 terms (gemm_planes.hip), or over 4-bit weights as digits (gemm_digits.hip), and what produces that
-    // input writes it so; a row of terms is as long as the fp32 row whose buffer it takes, one of digits no longer.  (Sessions with a quantised cache stay
-    // with the tiles here, for want of a measurement; fewer rows go through the same launches in every session.  The one order of summation
-    // that is kept for their sake, at no cost that was found, is that of quantised tiles: tile_plan.)
+    // input writes it so; a row of terms is as long as the fp32 row whose buffer it takes, one of digits no longer.
+    // (Sessions with a quantised cache stay with the tiles: other sums put other quants into the cache, and with them logits a token later move by 1.4e-3 and tokens change, 1 of 8
+    // of the 7B shape behind 203 rows.  It would be faster: Q4_0, 1.1B shape, 300 rows 3.40 -> 2.52 ms, 1900 rows 16.9 -> 8.5.  Fewer rows go through the same launches in every
+    // session.  The one order of summation that is kept for their sake, at no cost that was found, is that of quantised tiles: tile_plan.)
     const bool planes = !d->kvq && prec == GEMM_BF16X3_DEFAULT && s >= 64 && rows_planes_supported(D) && F % 32 == 0;
     auto in_planes = [&](const WMat *w) -> int {
       if (!planes || !w) return kTermsNone;

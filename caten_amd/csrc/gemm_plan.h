@@ -176,7 +176,10 @@ inline bool linear_planes_faster(int M, int N, int K, int precision, int type, d
   const bool ints = type == CTHIP_Q8_0 || type == CTHIP_Q4_0;
   double us = planes_us(M, N, K, terms, ints, pass_bytes, cus);
   if (prompt) {
-    us *= type == CTHIP_F16 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 4 * cus ? 1.13 : 1.04;
+    // (fp16 tiles, two to a compute unit, are at their best while that is one round: prompts with them / planes, GPT-2 medium 300 rows 1.89 / 2.03 ms, large 256 rows
+    // 3.16 / 3.48; 350 rows of the 1.1B shape 4.33 / 3.90)
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    us *= type != CTHIP_F16 ? 1.04 : tiles <= 2 * cus ? 1.4 : tiles <= 4 * cus ? 1.13 : 1.04;
   } else {
     const double plane_bytes = (double)N * ((K + 31) / 32) * 64 * (ints ? 1 : type == CTHIP_F16 && terms > 2 ? 2 : terms);
     us = std::max(us * ratio[terms - 1][ints ? 2 : type == CTHIP_F16 ? 1 : 0], plane_bytes / 2.5e6);
