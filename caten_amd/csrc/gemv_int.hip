@@ -13,8 +13,10 @@
 //
 // K is shared among the ks wavefronts of a workgroup (a unit of 128 bytes of each of 16 rows at a time, whole cache lines of
 // a row), rgp such sets work on neighbouring groups of 16 rows; a workgroup goes over its groups with PD units in flight per
-// wavefront and meets once, for the sums of them all.  What bounds it: the weights, behind 3.5 us of launch, the vector's way into LDS and the meeting at
-// the end (22016 x 4096, 50.7 MB: 13.2 us).  Errors against 64 bits, 4096 columns: 0.6 - 1.2e-7; the vector kernels, which take nibbles times
+// wavefront and meets once, for the sums of them all.  What bounds it: the weights, behind 3 us of launch, the vector's way into LDS and the meeting at
+// the end (22016 x 4096, 50.7 MB: 12.9 us, 4096 x 11008, 25.4 MB: 8.6, 4096 x 4096, 9.4 MB: 5.4).  Everything in front of the stream is instructions that sixteen wavefronts share four
+// issue slots for, and any wait there is one in front of the weights: with addresses per lane, divisions for the share of the rows and a common block of zeros whose address had to
+// be fetched for every unit, the three were 13.3, 10.4 and 6.2 us.  Errors against 64 bits, 4096 columns: 0.6 - 1.2e-7; the vector kernels, which take nibbles times
 // inputs less eight times the inputs' sum, 2 - 5e-7.
 #include "common.h"
 #include "gemv_kernels.h"
@@ -38,12 +40,15 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
   m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));  // row_half_mirror
   const unsigned E = max(m >> 23, 7u);  // (a unit is 2^(E - 156); at 7 the smallest subnormal number, of which every float is a multiple)
   const bool finite = m < 0x7f800000u;
-  // (the factor itself may lie past the largest float; 30 bits and a sign, an infinity stays one of 2^30 and what is beside it becomes nothing)
-  const int up = finite ? 156 - (int)E : -512;
+  // (the factor itself may lie past the largest float; 30 bits and a sign)
   int x[4], infs = 0;
 #pragma unroll
-  for (int e = 0; e < 4; e++) x[e] = (int)__builtin_amdgcn_fmed3f(rintf(__builtin_amdgcn_ldexpf(v[e], up)), -0x1p30f, 0x1p30f);
-  if (__any(!finite)) {  // (uniform: the eight lanes of a chunk are together)
+  for (int e = 0; e < 4; e++) x[e] = (int)rintf(__builtin_amdgcn_ldexpf(v[e], 156 - (int)E));
+  if (__builtin_expect(__any(!finite), 0)) {  // (uniform: the eight lanes of a chunk are together)
+    // an infinity stays one of 2^30 and what is beside it becomes nothing
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (!finite) x[e] = (int)__builtin_amdgcn_fmed3f(__builtin_amdgcn_ldexpf(v[e], -512), -0x1p30f, 0x1p30f);
 #pragma unroll
     for (int e = 0; e < 4; e++) infs += abs(x[e]) >> 30;
     infs += __builtin_amdgcn_mov_dpp(infs, 0xB1, 0xf, 0xf, true);
@@ -65,6 +70,7 @@ __device__ __forceinline__ float int_digits(const float *v, unsigned *w) {
 struct GemvIntShape {
   int upw, ks, rgp;        // units per wavefront and group; wavefronts sharing a group; groups a workgroup works on together
   int inv_ks, inv_rows;    // 65536 / ks, 65536 / (16 rgp), rounded up: quotients of numbers below 1024
+  int grid, full, rest;    // workgroups; every one goes over `full` groups of 16 rgp rows, the first `rest` over one more
 };
 
 // CENTRED: the mean of a LayerNorm comes off the vector before its digits are made, not off the sums behind them
@@ -74,8 +80,8 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
   constexpr bool RMS = PRO == CTHIP_PRO_RMSNORM, LAYERNORM = PRO == CTHIP_PRO_LAYERNORM;
   constexpr int CB = 128;            // bytes of digits per chunk: [half of its k][digit][16 bytes]
   extern __shared__ __align__(16) unsigned char smem[];
-  const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, g = lane >> 4, i = lane & 15;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), sub = (wv * sh.inv_ks) >> 16, wk = wv - sub * sh.ks, nw = sh.ks * sh.rgp;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, i = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), sub = (wv * sh.inv_ks) >> 16, wk = wv - sub * sh.ks, nw = sh.ks * sh.rgp, nthr = 64 * nw;
   const int nchunks = a.cols >> 5, n4 = a.cols >> 2;
   const int cpad = sh.ks * sh.upw * 8;  // chunks that the wavefronts go over: zeros past the row
   // LDS: 256 bytes of zeros, digits, a scale per chunk, reductions, the groups' partial sums
@@ -83,53 +89,51 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
   float *sx = (float *)(dig + (size_t)cpad * CB), *red = sx + cpad, *ps = red + 32;
   const int m = blockIdx.y;
   const float *__restrict__ x = a.x + (int64_t)m * a.x_stride;
-  const int rows_sg = 16 * sh.rgp, nsg = (a.rows + rows_sg - 1) / rows_sg;
-  const int iters = (nsg - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int posv = a.pos ? a.pos[0] : 0;
+  const int rows_sg = 16 * sh.rgp, iters = sh.full + ((int)blockIdx.x < sh.rest ? 1 : 0);
 
   // ---- the row this thread finishes (the plan: no more of them than threads), and what it needs for that ----
-  const int oj = (tid * sh.inv_rows) >> 16, oi = tid - oj * rows_sg, orow = ((int)blockIdx.x + oj * (int)gridDim.x) * rows_sg + oi;
-  const float *zf = (const float *)g_gemv_zeros;
+  const int oj = (tid * sh.inv_rows) >> 16, oi = tid - oj * rows_sg, orow = ((int)blockIdx.x + oj * sh.grid) * rows_sg + oi;
   const int orc = min(orow, a.rows - 1);
-  const float *pb = a.bias ? a.bias + orc : zf, *pr = a.residual ? a.residual + (int64_t)m * a.y_stride + orc : zf, *pf = a.fold_s ? a.fold_s + orc : zf;
 
   // ---- the input vector is asked for, then the first units of weights ----
   constexpr int SB = 3;
   const float4 *x4 = (const float4 *)x;
   const float4 *u4 = (RMS || LAYERNORM) && a.norm_g ? (const float4 *)a.norm_g : x4;
   float4 xv[SB], uv[SB];
-  auto ask = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < SB; b++) {
-      const int k = min(i0 + nthr * b, n4 - 1);
-      xv[b] = x4[k];
-      if (RMS || LAYERNORM) uv[b] = u4[k];
-    }
-  };
-  ask(tid);
-  const float ob = *pb, orr = *pr, of = *pf;
+  for (int b = 0; b < SB; b++) {
+    const unsigned k = 16u * (unsigned)min(tid + nthr * b, n4 - 1);
+    xv[b] = *(const float4 *)((const char *)x4 + k);
+    if (RMS || LAYERNORM) uv[b] = *(const float4 *)((const char *)u4 + k);
+  }
+  // (what is not there is read as the vector's first element and counts as nothing.  Not a block of zeros of the program's: its address comes out of memory by itself, and
+  // a wavefront that picks between that and another stands still for it -- in front of the first weights and again at every unit: see `request`)
+  typedef const __attribute__((address_space(1))) float *gfloat;  // (a flat load would be waited for with everything behind it)
+  auto opt = [&](const float *p, int64_t off) __attribute__((always_inline)) { return ((p ? (gfloat)p : (gfloat)x) + (p ? off : 0))[p ? (unsigned)orc : 0u]; };
+  const float rb = opt(a.bias, 0), rr = opt(a.residual, (int64_t)m * a.y_stride), rf = LAYERNORM ? opt(a.fold_s, 0) : 0.0f;
 
-  const uint4 *__restrict__ qp = (const uint4 *)a.q;
   uint4 wt[PD][2];
   unsigned st[PD];  // the scales of both chunks
   const int nu = iters * sh.upw;  // units of this wavefront
   int rq_j = 0, rq_u = 0;         // the next one to ask for
   auto request = [&](int p) __attribute__((always_inline)) {
-    const int row = min(((int)blockIdx.x + rq_j * (int)gridDim.x) * rows_sg + 16 * sub + i, a.rows - 1);
-    const bool past = rq_j >= iters;  // (uniform) nothing left: sixteen bytes that are there anyway, never used
+    const bool past = rq_j >= iters;  // (uniform) nothing left: the matrix's first bytes, never used
+    const int row0 = past ? 0 : min(((int)blockIdx.x + rq_j * sh.grid) * rows_sg + 16 * sub, a.rows - 1);
     // chunks 2g and 2g + 1 of the unit: both loads of a wavefront touch the same lines, the scales are one load
-    const int c0 = (wk * sh.upw + rq_u) * 8 + 2 * g;
+    // (nchunks is even; past the row: its last two chunks again, against zeros)
+    const int c0 = min((wk * sh.upw + rq_u) * 8 + 2 * g, nchunks - 2);
+    // offsets from the group's first row, which is the same for the wavefront: 16 rows of at most 2^20 columns
+    const unsigned off = past ? 0u : (unsigned)(min(i, a.rows - 1 - row0) * nchunks + c0);
+    const char *q0 = (const char *)a.q + (int64_t)row0 * nchunks * 16, *d0 = (const char *)a.d + (int64_t)row0 * nchunks * 2;
 #pragma unroll
-    for (int s = 0; s < 2; s++) {
-      const int c = min(c0 + s, nchunks - 1);  // past the row: its last chunk again, against zeros
-      wt[p][s] = load_chunk<NT>(past ? (const uint4 *)g_gemv_zeros : qp + (int64_t)row * nchunks + c);
-    }
-    st[p] = *(past ? (const unsigned *)g_gemv_zeros : (const unsigned *)(a.d + (int64_t)row * nchunks + min(c0, nchunks - 2)));
+    for (int s = 0; s < 2; s++) wt[p][s] = load_chunk<NT>((const uint4 *)(q0 + 16u * off) + s);
+    st[p] = *(const unsigned *)(d0 + 2u * off);
     if (++rq_u == sh.upw) rq_u = 0, rq_j++;
   };
 #pragma unroll
   for (int p = 0; p < PD; p++) request(p);
   __builtin_amdgcn_sched_barrier(0);
+  const int posv = a.pos ? a.pos[0] : 0;
 
   // ---- digits ----
   float s1 = 0.0f, mu = 0.0f, rstd = 1.0f;
@@ -164,26 +168,27 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
     const unsigned z[4] = {0u, 0u, 0u, 0u};
     put(k, z, 0.0f);
   }
-  for (int i0 = tid; i0 < n4; i0 += nthr * SB) {  // (a chunk's lanes stay together: n4 is a multiple of eight)
-    if (i0 != tid) ask(i0);
+  auto piece = [&](int k, const float4 &x0, const float4 &u0) __attribute__((always_inline)) {  // (a chunk's lanes stay together: n4 is a multiple of eight)
+    float v[4] = {x0.x, x0.y, x0.z, x0.w};
+    const float u[4] = {u0.x, u0.y, u0.z, u0.w};
 #pragma unroll
-    for (int b = 0; b < SB; b++) {
-      const int k = i0 + nthr * b;
-      if (k < n4) {  // (not a break: three ways out of a loop are ten scalar registers, and past 80 a compute unit holds one workgroup of sixteen wavefronts)
-        float v[4] = {xv[b].x, xv[b].y, xv[b].z, xv[b].w};
-        const float u[4] = {uv[b].x, uv[b].y, uv[b].z, uv[b].w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          if (CENTRED) v[e] -= mu;
-          else if (LAYERNORM) s1 += v[e];
-          if (RMS || CENTRED) s1 = fmaf(v[e], v[e], s1);
-          if ((RMS || LAYERNORM) && a.norm_g) v[e] *= u[e];
-        }
-        unsigned w[4];
-        const float down = int_digits(v, w);
-        put(k, w, down);
-      }
+    for (int e = 0; e < 4; e++) {
+      if (CENTRED) v[e] -= mu;
+      else if (LAYERNORM) s1 += v[e];
+      if (RMS || CENTRED) s1 = fmaf(v[e], v[e], s1);
+      if ((RMS || LAYERNORM) && a.norm_g) v[e] *= u[e];
     }
+    unsigned w[4];
+    const float down = int_digits(v, w);
+    put(k, w, down);
+  };
+  // (what has been asked for stays out of the loop over the rest: behind a way back the wait for it would be one for the weights as well)
+#pragma unroll
+  for (int b = 0; b < SB; b++)
+    if (tid + nthr * b < n4) piece(tid + nthr * b, xv[b], uv[b]);
+  for (int k = tid + nthr * SB; k < n4; k += nthr) {
+    const float4 t = x4[k];
+    piece(k, t, RMS || LAYERNORM ? u4[k] : t);
   }
   if (RMS || LAYERNORM) {
     s1 = wave_sum(s1);
@@ -254,6 +259,7 @@ __global__ __launch_bounds__(1024) void k_gemv_int(GemvArgs a, GemvIntShape sh) 
   __syncthreads();
 
   // ---- the sums of the wavefronts, in their order, and the epilogue ----
+  const float ob = a.bias ? rb : 0.0f, orr = a.residual ? rr : 0.0f, of = LAYERNORM && a.fold_s ? rf : 0.0f;
   if (RMS || LAYERNORM) rstd = 1.0f / sqrtf(of_all(LAYERNORM ? red + 16 : red, 1, nw) / (float)a.cols + a.eps);
   float best = -INFINITY;
   int besti = 0x7fffffff;
@@ -315,7 +321,8 @@ int launch_gemv_int(const WMat *w, GemvArgs a, int m, int *am_parts) {
   if (p.lds > 64 * 1024) {
     CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvIntMaxLdsBytes));
   }
-  hipLaunchKernelGGL(fn, dim3(p.grid, (unsigned)m), dim3(64 * p.ks * p.rgp), p.lds, s.stream, a, GemvIntShape{p.upw, p.ks, p.rgp, (65536 + p.ks - 1) / p.ks, (65536 + 16 * p.rgp - 1) / (16 * p.rgp)});
+  const long long nsg = (w->rows + 16 * p.rgp - 1) / (16 * p.rgp);
+  hipLaunchKernelGGL(fn, dim3(p.grid, (unsigned)m), dim3(64 * p.ks * p.rgp), p.lds, s.stream, a, GemvIntShape{p.upw, p.ks, p.rgp, (65536 + p.ks - 1) / p.ks, (65536 + 16 * p.rgp - 1) / (16 * p.rgp), (int)p.grid, (int)(nsg / p.grid), (int)(nsg % p.grid)});
   CTHIP_LAUNCH_CHECK();
   *am_parts = (int)p.grid;
   return 0;
