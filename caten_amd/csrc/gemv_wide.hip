@@ -63,18 +63,18 @@ void k_gemv_wide(GemvArgs a, int tpr) {
       const int c = (rq_grp * NC + k) * 64 + lane;
       const bool ok = c < nchunks;
       const int sidx = Q4 ? c : c >> 1;
-      wt[p][0][k] = load_chunk<NT>(ok ? qp + (int64_t)row0 * nchunks + c : (const uint4 *)g_gemv_zeros);
-      if (RW > 1) wt[p][RW - 1][k] = load_chunk<NT>(ok ? qp + (int64_t)row1 * nchunks + c : (const uint4 *)g_gemv_zeros);
+      wt[p][0][k] = load_chunk<NT>(ok ? qp + (int64_t)row0 * nchunks + c : (const uint4 *)gemv_zeros());
+      if (RW > 1) wt[p][RW - 1][k] = load_chunk<NT>(ok ? qp + (int64_t)row1 * nchunks + c : (const uint4 *)gemv_zeros());
       if (QUANT) {
-        st[p][0][k] = *(ok ? a.d + (int64_t)row0 * scales_per_row + sidx : (const unsigned short *)g_gemv_zeros);
-        if (RW > 1) st[p][RW - 1][k] = *(ok ? a.d + (int64_t)row1 * scales_per_row + sidx : (const unsigned short *)g_gemv_zeros);
+        st[p][0][k] = *(ok ? a.d + (int64_t)row0 * scales_per_row + sidx : (const unsigned short *)gemv_zeros());
+        if (RW > 1) st[p][RW - 1][k] = *(ok ? a.d + (int64_t)row1 * scales_per_row + sidx : (const unsigned short *)gemv_zeros());
       }
     }
     // the rows' bias and residual travel with their tiles: lanes 0, 1 ask for row0's, lanes 2, 3 for row1's
     const int er = (lane & 2) ? row1 : row0;
     const float *pb = a.bias ? a.bias + er : nullptr;
     const float *pr = a.residual ? a.residual + (int64_t)m * a.y_stride + er : nullptr;
-    const float *any = pb ? pb : pr ? pr : (const float *)g_gemv_zeros;
+    const float *any = pb ? pb : pr ? pr : (const float *)gemv_zeros();
     epi_t[p] = *((lane & 1) ? (pr ? pr : any) : (pb ? pb : any));
     // advance; past the last tile the last one is requested again (and never consumed)
     if (rq_left > 1) {

@@ -52,9 +52,23 @@ __global__ __launch_bounds__(256) void k_copies(CopyBatch cb) {
 
 // One row of one batch: scores (bmm.hip's KC layout), softmax, values (NC layout), copy.  Sums as in k_bmm.  The row's scores stay in
 // LDS; a 12-head step at position 30: 8 us instead of six launches of 2.6 - 4.8, every one of them behind the host.
+// (What the kernel is told is what it needs and no more: a round of scalar loads is 0.2 us in front of everything else, and two descriptions of whole products were
+// eight of them.)
+struct GraphRows {  // where an operand's row of a batch begins: elements per step of a batch axis, per row
+  int64_t at, sb[3], si;
+};
 struct GraphAttn {
-  BmmArgs s, v;
-  float *probs;
+  const float *Q, *K, *V, *M0, *M1;  // M0, M1: addends of the scores (none: the queries' first element, with strides of 0)
+  GraphRows q, k, v, m0, m1;
+  int64_t k_sj, v_sk, m0_sj, m1_sj;
+  int N, Kd, Nv;             // keys, elements of a key, of a value
+  int nb1;
+  unsigned inv_nb1;          // 2^32 / nb1, rounded up: quotients of numbers below 2^16
+  bool has0, has1;
+  float s_alpha, v_alpha;
+  float *S, *probs, *C;
+  GraphRows s, p, c;
+  int64_t c_sj;
   float *copy;               // null: no copy behind it
   int64_t cb, ci, cj;        // its strides per batch, row, column
   // copies of a contiguous row in front (a step's new key and value rows): the workgroups share them, and whoever needs a
@@ -69,62 +83,99 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
   __shared__ float4 part[16][16];
   __shared__ float red[8];
   const int tid = threadIdx.x, i = blockIdx.x, lane = tid & 63, wv = tid >> 6, c = tid & 15, g = tid >> 4;
-  int bz = blockIdx.y;
-  const int b2 = bz % a.s.nb[2];
-  bz /= a.s.nb[2];
-  const int b1 = bz % a.s.nb[1], b0 = bz / a.s.nb[1];
-  auto off = [&](const BmmOperand &o) { return o.base + (int64_t)b0 * o.sb[0] + (int64_t)b1 * o.sb[1] + (int64_t)b2 * o.sb[2]; };
-  const int N = a.s.N, K = a.s.K;
-  const float *A = a.s.A + off(a.s.a) + (int64_t)i * a.s.a.si, *KB = a.s.B + off(a.s.b), *VB = a.v.B + off(a.v.b);
-  auto at = [&](const float *p) __attribute__((always_inline)) {  // where what belongs at p can be read now
-    const int64_t d0 = p - a.pre_out[0], d1 = p - a.pre_out[1];
-    return d0 >= 0 && d0 < a.pre_n[0] ? a.pre_in[0] + d0 : d1 >= 0 && d1 < a.pre_n[1] ? a.pre_in[1] + d1 : p;
+  const int b2 = blockIdx.y, b0 = a.nb1 > 1 ? (int)__umulhi(blockIdx.z, a.inv_nb1) : (int)blockIdx.z, b1 = (int)blockIdx.z - b0 * a.nb1;
+  auto off = [&](const GraphRows &o) { return o.at + (int64_t)b0 * o.sb[0] + (int64_t)b1 * o.sb[1] + (int64_t)b2 * o.sb[2] + (int64_t)i * o.si; };
+  // (one wait for all of what the first loads' addresses are made of)
+  const float *Qp = a.Q, *Kp = a.K, *Vp = a.V;
+  GraphRows rq = a.q, rk = a.k, rv = a.v;
+  int64_t k_sj = a.k_sj, v_sk = a.v_sk;
+  int N = a.N, K = a.Kd, Nv = a.Nv;
+  asm volatile(""
+               : "+s"(Qp), "+s"(Kp), "+s"(Vp), "+s"(rq.at), "+s"(rq.sb[0]), "+s"(rq.sb[1]), "+s"(rq.sb[2]), "+s"(rq.si), "+s"(rk.at), "+s"(rk.sb[0]), "+s"(rk.sb[1]),
+                 "+s"(rk.sb[2]), "+s"(rv.at), "+s"(rv.sb[0]), "+s"(rv.sb[1]), "+s"(rv.sb[2]), "+s"(k_sj), "+s"(v_sk), "+s"(N), "+s"(K), "+s"(Nv));
+  typedef const __attribute__((address_space(1))) float *gfloat;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef const __attribute__((address_space(1))) f4 *gfloat4;
+  const gfloat A = (gfloat)(Qp + off(rq)), KB = (gfloat)(Kp + off(rk)), VB = (gfloat)(Vp + off(rv));
+  // what belongs at p, from where it can be read now.  (Selects, not branches: behind a branch every load was waited for by itself, eight round trips in front
+  // of the first score; a launch of a 12-head step at position 27, 8.5 -> 5 us.)
+  const uint64_t o0 = (uint64_t)a.pre_out[0], o1 = (uint64_t)a.pre_out[1], m0 = (uint64_t)a.pre_in[0] - o0, m1 = (uint64_t)a.pre_in[1] - o1;
+  const uint64_t n0 = 4ull * a.pre_n[0], n1 = 4ull * a.pre_n[1];
+  auto at = [&](gfloat p) __attribute__((always_inline)) {
+    const uint64_t x = (uint64_t)p;
+    const bool in0 = x - o0 < n0, in1 = x - o1 < n1;
+    const uint64_t lo = in0 ? m0 : in1 ? m1 : 0;
+    const f4 t = *(gfloat4)(x + lo);
+    return make_float4(t[0], t[1], t[2], t[3]);
   };
-  float4 vw[4];
-  {
-    // the first keys' values are asked for ahead of the scores: they arrive behind them
+  // Asked for in front of any arithmetic, in the order of use: four passes of 16 keys together (64-wide heads: one piece of each key per lane), the addends, the
+  // same keys' values, and one piece a thread of the copies in front, the workgroups in turn.
+  const gfloat p0 = (gfloat)(a.M0 + off(a.m0)), p1 = (gfloat)(a.M1 + off(a.m1));
+  float *Crow = a.S + off(a.s);
+  float4 kw[4], vw[4], cw[2];
+  float e0[4], e1[4];
+  auto addends = [&](int j0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) vw[u] = *(const float4 *)at(VB + (int64_t)min(g + 16 * u, N - 1) * a.v.b.sk + (4 * c < a.v.N ? 4 * c : 0));
-    // four passes of 16 keys asked for together (64-wide heads: one piece of each key per lane)
-    const float *p0 = a.s.pre0 ? a.s.pre0 + off(a.s.p0) + (int64_t)i * a.s.p0.si : A, *p1 = a.s.pre1 ? a.s.pre1 + off(a.s.p1) + (int64_t)i * a.s.p1.si : A;
-    const int64_t s0 = a.s.pre0 ? a.s.p0.sj : 0, s1 = a.s.pre1 ? a.s.p1.sj : 0;
-    float *Crow = a.s.C + off(a.s.c) + (int64_t)i * a.s.c.si;
-    for (int j0 = 0; j0 < N; j0 += 64) {
-      float acc[4], e0[4], e1[4];
+    for (int u = 0; u < 4; u++) {
+      const int j = min(j0 + 16 * u + g, N - 1);
+      e0[u] = p0[j * a.m0_sj];
+      e1[u] = p1[j * a.m1_sj];
+    }
+  };
+  auto keys = [&](int j0, int k0, float4 *w) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) w[u] = at(KB + (int64_t)min(j0 + 16 * u + g, N - 1) * k_sj + k0);
+  };
+  const int kc = 4 * c < K ? 4 * c : 0, nwg = gridDim.x * gridDim.y * gridDim.z, unit = tid * nwg + (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+  const f4 x0 = *(gfloat4)(A + kc);
+  keys(0, kc, kw);
+  __builtin_amdgcn_sched_barrier(0);
+  addends(0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < 4; u++) vw[u] = at(VB + (int64_t)min(g + 16 * u, N - 1) * v_sk + (4 * c < Nv ? 4 * c : 0));
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const f4 t = *(gfloat4)(4 * unit < a.pre_n[q] ? (gfloat)a.pre_in[q] + 4 * unit : A);
+    cw[q] = make_float4(t[0], t[1], t[2], t[3]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  auto pass = [&](int j0) __attribute__((always_inline)) {
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto dot = [&](const f4 &x, const float4 *w) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int j = min(j0 + 16 * u + g, N - 1);
-        e0[u] = p0[j * s0];
-        e1[u] = p1[j * s1];
+        acc[u] = fmaf(x.x, w[u].x, acc[u]);
+        acc[u] = fmaf(x.y, w[u].y, acc[u]);
+        acc[u] = fmaf(x.z, w[u].z, acc[u]);
+        acc[u] = fmaf(x.w, w[u].w, acc[u]);
       }
+    };
+    if (4 * c < K) dot(x0, kw);
+    for (int k0 = 4 * c + 64; k0 < K; k0 += 64) {
+      float4 w[4];
+      keys(j0, k0, w);
+      const f4 x = *(gfloat4)(A + k0);
+      dot(x, w);
+    }
 #pragma unroll
-      for (int u = 0; u < 4; u++) acc[u] = 0.0f;
-      for (int k0 = 4 * c; k0 < K; k0 += 64) {
-        float4 w[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) w[u] = *(const float4 *)at(KB + (int64_t)min(j0 + 16 * u + g, N - 1) * a.s.b.sj + k0);
-        const float4 x = *(const float4 *)(A + k0);
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          acc[u] = fmaf(x.x, w[u].x, acc[u]);
-          acc[u] = fmaf(x.y, w[u].y, acc[u]);
-          acc[u] = fmaf(x.z, w[u].z, acc[u]);
-          acc[u] = fmaf(x.w, w[u].w, acc[u]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int j = j0 + 16 * u + g;
-        acc[u] = row16_sum(acc[u]);
-        if (c == 0 && j < N) {
-          float v = a.s.alpha * acc[u];
-          if (a.s.pre0) v += e0[u];
-          if (a.s.pre1) v += e1[u];
-          Crow[j] = v;
-          sc[j] = v;
-        }
+    for (int u = 0; u < 4; u++) {
+      const int j = j0 + 16 * u + g;
+      acc[u] = row16_sum(acc[u]);
+      if (c == 0 && j < N) {
+        float v = a.s_alpha * acc[u];
+        if (a.has0) v += e0[u];
+        if (a.has1) v += e1[u];
+        Crow[j] = v;
+        sc[j] = v;
       }
     }
+  };
+  pass(0);  // (not in the loop: at its top the wait for the first keys would be one for everything that has been asked for)
+  for (int j0 = 64; j0 < N; j0 += 64) {
+    keys(j0, kc, kw);
+    addends(j0);
+    pass(j0);
   }
   __syncthreads();
   float m = -INFINITY;
@@ -143,18 +194,18 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
   if (lane == 0) red[4 + wv] = l;
   __syncthreads();
   const float inv = 1.0f / ((red[4] + red[5]) + (red[6] + red[7]));
-  float *P = a.probs + off(a.v.a) + (int64_t)i * a.v.a.si;
+  float *P = a.probs + off(a.p);
   for (int j = tid; j < N; j += 256) {
     const float p = sc[j] * inv;
     sc[j] = p;
     P[j] = p;
   }
   __syncthreads();
-  float *C = a.v.C + off(a.v.c) + (int64_t)i * a.v.c.si;
-  float *Y = a.copy ? a.copy + (int64_t)blockIdx.y * a.cb + (int64_t)i * a.ci : nullptr;
-  for (int d0 = 0; d0 < a.v.N; d0 += 64) {
+  float *C = a.C + off(a.c);
+  float *Y = a.copy ? a.copy + (int64_t)(blockIdx.z * gridDim.y + blockIdx.y) * a.cb + (int64_t)i * a.ci : nullptr;
+  for (int d0 = 0; d0 < Nv; d0 += 64) {
     const int j4 = d0 + 4 * c;
-    const bool live = j4 < a.v.N;
+    const bool live = j4 < Nv;
     const int jc = live ? j4 : 0;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int k0 = g; k0 < N; k0 += 64) {
@@ -164,7 +215,7 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
         for (int u = 0; u < 4; u++) w[u] = vw[u];
       } else {
 #pragma unroll
-        for (int u = 0; u < 4; u++) w[u] = *(const float4 *)at(VB + (int64_t)min(k0 + 16 * u, N - 1) * a.v.b.sk + jc);
+        for (int u = 0; u < 4; u++) w[u] = at(VB + (int64_t)min(k0 + 16 * u, N - 1) * v_sk + jc);
       }
 #pragma unroll
       for (int u = 0; u < 4; u++) {
@@ -190,18 +241,19 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
       const float o[4] = {s.x, s.y, s.z, s.w};
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        const float v = a.v.alpha * o[q];
-        C[(int64_t)(j4 + q) * a.v.c.sj] = v;
+        const float v = a.v_alpha * o[q];
+        C[(int64_t)(j4 + q) * a.c_sj] = v;
         if (Y) Y[(int64_t)(j4 + q) * a.cj] = v;
       }
     }
     __syncthreads();
   }
-  // (the copies last: in front, everything else waited for their round trip to memory: 9.3 -> 8.1 us a launch of a 12-head step at position 27)
+  // (the copies' first pieces, one to a thread and the workgroups in turn, were asked for with the first values: a round trip to memory less at the end)
 #pragma unroll
-  for (int q = 0; q < 2; q++)
-    for (int t = 4 * ((blockIdx.y * gridDim.x + blockIdx.x) * 256 + tid); t < a.pre_n[q]; t += 1024 * gridDim.x * gridDim.y)
-      *(float4 *)(a.pre_out[q] + t) = *(const float4 *)(a.pre_in[q] + t);
+  for (int q = 0; q < 2; q++) {
+    if (4 * unit < a.pre_n[q]) *(float4 *)(a.pre_out[q] + 4 * unit) = cw[q];
+    for (int t = 4 * (unit + 256 * nwg); t < a.pre_n[q]; t += 1024 * nwg) *(float4 *)(a.pre_out[q] + t) = *(const float4 *)(a.pre_in[q] + t);
+  }
 }
 
 // ---- what a chain may touch ----
@@ -277,8 +329,23 @@ static int run_attention(const GraphOp *ops, int left, int &rc) {
       if (!apart(outs[p], outs[q])) return 0;
   }
   GraphAttn a = {};
-  a.s = s;
-  a.v = v;
+  auto rows_of = [](const BmmOperand &o) { return GraphRows{o.base, {o.sb[0], o.sb[1], o.sb[2]}, o.si}; };
+  auto whole = [&](const BmmOperand &o) {  // (all rows of a batch are read)
+    GraphRows r = rows_of(o);
+    r.si = 0;
+    return r;
+  };
+  a.Q = s.A, a.K = s.B, a.V = v.B, a.S = s.C, a.C = v.C;
+  a.q = rows_of(s.a), a.k = whole(s.b), a.v = whole(v.b), a.s = rows_of(s.c), a.p = rows_of(v.a), a.c = rows_of(v.c);
+  a.k_sj = s.b.sj, a.v_sk = v.b.sk, a.c_sj = v.c.sj;
+  a.has0 = s.pre0 != nullptr, a.has1 = s.pre1 != nullptr;
+  a.M0 = a.has0 ? s.pre0 : s.A, a.M1 = a.has1 ? s.pre1 : s.A;
+  if (a.has0) a.m0 = rows_of(s.p0), a.m0_sj = s.p0.sj;
+  else a.m0.at = s.a.base;
+  if (a.has1) a.m1 = rows_of(s.p1), a.m1_sj = s.p1.sj;
+  else a.m1.at = s.a.base;
+  a.N = s.N, a.Kd = s.K, a.Nv = v.N, a.s_alpha = s.alpha, a.v_alpha = v.alpha;
+  a.nb1 = s.nb[1], a.inv_nb1 = s.nb[1] > 1 ? (unsigned)((0x100000000ull + s.nb[1] - 1) / s.nb[1]) : 0u;
   a.probs = ops[1].out - v.a.base;  // (the kernel adds v.a's offsets)
   int used = 3;
   if (left > 3 && ops[3].kind == GraphOp::COPY) {
@@ -329,7 +396,7 @@ static int run_attention(const GraphOp *ops, int left, int &rc) {
       a.pre_n[q] = c.ext[2];
     }
   }
-  hipLaunchKernelGGL(k_graph_attn, dim3(s.M, (unsigned)nb), dim3(256), 0, state().stream, a);
+  hipLaunchKernelGGL(k_graph_attn, dim3(s.M, (unsigned)s.nb[2], (unsigned)(s.nb[0] * s.nb[1])), dim3(256), 0, state().stream, a);
   const hipError_t e = hipGetLastError();
   rc = e == hipSuccess ? 0 : fail((int)e, "graph: launch -> %s", hipGetErrorString(e));
   return npre + used;

@@ -69,7 +69,10 @@ __device__ __forceinline__ v4f mma_rows(v8bf a, v8bf b, v4f c) { return __builti
 enum { RW_Q8 = 1, RW_Q4 = 2, RW_F16 = 3, RW_F32 = 4 };
 
 constexpr int kRowsMax = 32, kRowsGroups = 4096;  // input rows, column groups
-__device__ int g_rows_tickets[kRowsGroups];  // zero between launches
+__device__ __forceinline__ static int *rows_tickets() {  // zero between launches (inside a function its address is known without a trip to memory)
+  static __device__ int tickets[kRowsGroups];
+  return tickets;
+}
 
 // Bytes of a weight row in a unit, and blocks of 32 k: whole cache lines.  (Requests that cover 32 bytes of a row each, as
 // operand registers would ask for them, are bound by the tag lookups of the compute unit's cache: 2.4 TB/s of Q8_0 and
@@ -311,10 +314,10 @@ __global__ __launch_bounds__(64 * NW, 2) void k_linear_rows(RowsGemmArgs a) {
     // back and invalidate the whole L2 of the XCD); the counters are left at zero for the next launch
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) s_ticket = __hip_atomic_fetch_add(g_rows_tickets + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) s_ticket = __hip_atomic_fetch_add(rows_tickets() + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (s_ticket != (int)gridDim.y - 1) return;
-    if (tid == 0) __hip_atomic_store(g_rows_tickets + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(rows_tickets() + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
     __syncthreads();
   }

@@ -94,8 +94,11 @@ __device__ __forceinline__ void split4(float r0, float r1, float r2, float r3, u
 
 // Zeros in device memory: what a request outside an operand reads.  (A load followed by a select would make
 // the request's own thread wait for it at once; a branch around it splits the run of requests.)
-__device__ __align__(16) unsigned g_zeros[8];  // zero-initialised, never written (not const: a load that may come from
-                                                // either here or an operand must stay a global-memory load)
+// Not const: a load that may come from either here or an operand must stay a global-memory load.  Inside a function: its address is known without a trip to memory.
+__device__ __forceinline__ static unsigned *zero_block() {
+  static __device__ __align__(16) unsigned zeros[8];
+  return zeros;
+}
 
 // How a thread asks for four consecutive floats of an operand's row.  LD_VEC, LD_ANY: one 16-byte request inside the operand (rows of at least four floats),
 // at an offset from a uniform address: rows past the end are the last one, columns that reach past the end the row's last four.  What is past
@@ -108,17 +111,17 @@ __device__ __forceinline__ float4 load4_in(const float *m, int off) {
   return make_float4(v.x, v.y, v.z, v.w);
 }
 // LD_ELEM: four consecutive floats at p without a branch or a dependent instruction: of the four, those past `nvalid`
-// (0..4) are read from g_zeros.  Like the ones above a K-step's
+// (0..4) are read from zero_block().  Like the ones above a K-step's
 // requests stay one straight run of loads, so that the waits before their use count the younger requests
 // instead of draining them.
 __device__ __forceinline__ float4 load4(const float *p, int nvalid) {
-  const float *z = (const float *)g_zeros;
+  const float *z = (const float *)zero_block();
   return make_float4(*(nvalid > 0 ? p : z), *(nvalid > 1 ? p + 1 : z), *(nvalid > 2 ? p + 2 : z), *(nvalid > 3 ? p + 3 : z));
 }
 // the four are 16-byte aligned and all inside or all outside (k_gemm_f32pc and the kernels of packed weights: the matrix
 // instructions set their pace, and the moves into place cost them 3 - 8 %)
 __device__ __forceinline__ float4 load4_vec(const float *p, int nvalid) {
-  return *(const float4 *)(nvalid > 0 ? p : (const float *)g_zeros);
+  return *(const float4 *)(nvalid > 0 ? p : (const float *)zero_block());
 }
 __device__ __forceinline__ int clamp04(int v) { return v < 0 ? 0 : v > 4 ? 4 : v; }
 // by = c - min(c, len - 4): elements move down by that many, zeros behind them (LD_VEC: none or all of them)
@@ -314,14 +317,14 @@ __global__ __launch_bounds__(768, NS == 6 ? 3 : 6) void k_gemm_split(GemmArgs a)
       const bool ok = n < N && k < K;
       const int64_t e = (int64_t)n * ldk + k;  // element index of the chunk
       if (BMODE == W_F32) {
-        const v4u *src = ok ? (const v4u *)((const float *)a.wq + e) : (const v4u *)g_zeros;
+        const v4u *src = ok ? (const v4u *)((const float *)a.wq + e) : (const v4u *)zero_block();
         const int st = ok ? 1 : 0;  // the zeros are 32 bytes long
         rb.v[0] = src[0];
         rb.v[BRegs<BMODE>::NV > 1 ? 1 : 0] = src[st];
         rb.v[BRegs<BMODE>::NV > 2 ? 2 : 0] = src[2 * st];
         rb.v[BRegs<BMODE>::NV > 3 ? 3 : 0] = src[3 * st];
       } else if (BMODE == W_F16) {
-        const v4u *src = ok ? (const v4u *)((const unsigned short *)a.wq + e) : (const v4u *)g_zeros;
+        const v4u *src = ok ? (const v4u *)((const unsigned short *)a.wq + e) : (const v4u *)zero_block();
         rb.v[0] = src[0];
         rb.v[BRegs<BMODE>::NV > 1 ? 1 : 0] = src[1];
       }
@@ -627,10 +630,10 @@ __global__ __launch_bounds__(256 + 64 * NPW) void k_gemm_qpc(GemmArgs a) {
       const int n = n0 + wr + (PT / 4) * j;
       const int64_t e = (int64_t)n * ldk + k;
       const uint8_t *q = (const uint8_t *)a.wq + (WT == W_Q8 ? e : ((e >> 5) << 4));
-      rb.v[j] = *((n < N && k < K) ? (const uint4 *)q : (const uint4 *)g_zeros);
+      rb.v[j] = *((n < N && k < K) ? (const uint4 *)q : (const uint4 *)zero_block());
     }
     const int ns = n0 + sr, ks = kbeg + k0 + 32 * sb;
-    rb.d = *((ns < N && ks < K) ? a.wd + (int64_t)ns * blocks_per_row + (ks >> 5) : (const unsigned short *)g_zeros);
+    rb.d = *((ns < N && ks < K) ? a.wd + (int64_t)ns * blocks_per_row + (ks >> 5) : (const unsigned short *)zero_block());
   };
   auto stage = [&](const ARg &ra, const BRg &rb, int buf) {
 #pragma unroll
@@ -828,7 +831,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs a) {
       const int n = n0 + (tid >> 2), k = kbeg + k0 + 8 * (tid & 3);
       const bool in = n < N && k < K;
       const int64_t e = (int64_t)n * ldk + k;
-      const void *z = g_zeros;
+      const void *z = zero_block();
       if (!AL) {
         // fp32 / fp16 rows of any width: element loads, zeros past the end of the row
         unsigned x[8];

@@ -925,7 +925,10 @@ __global__ __launch_bounds__(NT) void k_argmax(ArgmaxArgs a) {
 // draw a ticket; the last one settles the row (6.3 us as two launches).  A part's result is one 8-byte device-scope store
 // that has reached memory before its ticket is drawn; the counters are left at zero for the next launch.
 constexpr int kArgmaxParts = 64, kArgmaxPartRows = 16;
-__device__ int g_argmax_tickets[kArgmaxPartRows];
+__device__ __forceinline__ static int *argmax_tickets() {  // (inside a function its address is known without a trip to memory)
+  static __device__ int tickets[kArgmaxPartRows];
+  return tickets;
+}
 __global__ __launch_bounds__(256) void k_argmax_parts(ArgmaxArgs a, unsigned long long *__restrict__ parts) {
   __shared__ int ticket;
   const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
@@ -938,7 +941,7 @@ __global__ __launch_bounds__(256) void k_argmax_parts(ArgmaxArgs a, unsigned lon
   if (tid == 0) {
     __hip_atomic_store(mine + part, ((unsigned long long)__float_as_uint(best) << 32) | (unsigned)bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    ticket = __hip_atomic_fetch_add(g_argmax_tickets + row, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    ticket = __hip_atomic_fetch_add(argmax_tickets() + row, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (ticket != kArgmaxParts - 1 || tid >= 64) return;
@@ -948,7 +951,7 @@ __global__ __launch_bounds__(256) void k_argmax_parts(ArgmaxArgs a, unsigned lon
   argmax_wave(best, bi);
   if (tid == 0) {
     argmax_store(a, row, bi);
-    __hip_atomic_store(g_argmax_tickets + row, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(argmax_tickets() + row, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 static_assert(kArgmaxParts == 64, "one part per lane of the wavefront that settles a row");
