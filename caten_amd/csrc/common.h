@@ -417,10 +417,18 @@ __device__ __forceinline__ float half_bits_to_float(unsigned short h) {
 // api/high-level-ops.lisp:112-117): exp(x) = exp2(x * 1/ln2); sigmoid = recip(1 + exp2(-x/ln2));
 // tanh(y) = 2*sigmoid(2y) - 1.
 __device__ __forceinline__ float ct_exp(float x) { return exp2f(x * 1.442695f); }
-// keys per range where at most nz workgroups share T keys in whole tiles
-__device__ __forceinline__ int attn_split_keys(int T, int nz, int tile) {
-  const int tiles = (T + tile - 1) / tile;
-  return ((tiles + nz - 1) / nz) * tile;
+// floor(x / d) of numbers that are the same in every lane, 0 <= x < 2^19, d >= 1, in six instructions where a division of integers is thirty that nothing
+// runs beside: the quotient is off by x / d * 2^-22 at most, half a part in d is what it may be.
+__device__ __forceinline__ int uniform_div(int x, int d) {
+  return __builtin_amdgcn_readfirstlane((int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)d)));
+}
+// keys per range where at most nz workgroups share T keys in whole tiles, and how many ranges that makes
+struct AttnRanges {
+  int per, n;
+};
+__device__ __forceinline__ AttnRanges attn_split_keys(int T, int nz, int tile) {
+  const int tiles = (int)((unsigned)(T + tile - 1) / (unsigned)tile), each = uniform_div(tiles + nz - 1, nz);
+  return {each * tile, uniform_div(tiles + each - 1, each)};
 }
 // The workgroup that drew a head's last ticket adds the ranges' triples up, in range order: `all` holds nranges
 // records of dh unnormalised outputs, the running maximum and the running sum.  The loads are device-scope (they do
@@ -461,9 +469,9 @@ struct AttnParts {
 };
 __device__ __forceinline__ AttnParts attn_parts_load(const float *all, int ranges, int dh, int lane) {
   AttnParts p;
-  p.ml = *(const float2 *)(all + (lane < ranges ? lane : ranges - 1) * (dh + 2) + dh);
+  p.ml = *(const float2 *)(all + (unsigned)((lane < ranges ? lane : ranges - 1) * (dh + 2) + dh));
 #pragma unroll
-  for (int r = 0; r < kAttnSplitMaxRanges; r++) p.o[r] = all[(r < ranges ? r : ranges - 1) * (dh + 2) + lane];
+  for (int r = 0; r < kAttnSplitMaxRanges; r++) p.o[r] = (all + (r < ranges ? r : ranges - 1) * (dh + 2))[(unsigned)lane];
   return p;
 }
 __device__ __forceinline__ float attn_parts_merge(const AttnParts &p, int nranges, int lane) {
@@ -473,11 +481,10 @@ __device__ __forceinline__ float attn_parts_merge(const AttnParts &p, int nrange
   float o = 0.0f, L = 0.0f;
 #pragma unroll
   for (int r = 0; r < kAttnSplitMaxRanges; r++) {
-    if (r < nranges) {
-      const float er = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), r));
-      o = fmaf(er, p.o[r], o);
-      L = fmaf(er, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.ml.y), r)), L);
-    }
+    // (selects: behind a branch, a range's record is asked for there, one more round trip.  What lies in a record that is not in use counts as nothing.)
+    const float er = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), r));
+    o = fmaf(er, r < nranges ? p.o[r] : 0.0f, o);
+    L = fmaf(er, r < nranges ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.ml.y), r)) : 0.0f, L);
   }
   return o / L;
 }

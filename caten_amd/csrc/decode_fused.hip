@@ -186,7 +186,8 @@ void k_dec_attn_proj(DecAttnArgs a) {
   const int g = lane / LPK, c = lane % LPK;
   // The projection slab of this head.  gridDim.y workgroups per head repeat the head's attention and share the
   // slab's rows: what one compute unit has to fetch bounds the launch, and the slab is most of it.
-  const int rr = D / (int)gridDim.y, rbase = (int)blockIdx.y * rr;  // this workgroup's rows of the slab
+  const int posv = a.pos[0];  // (asked for here, by all: where one wavefront alone wants it, it is one more round trip behind the records)
+  const int rr = uniform_div(D, (int)gridDim.y), rbase = (int)blockIdx.y * rr;  // this workgroup's rows of the slab
   const int pc = tid % CPR, pr0 = tid / CPR;
   uint4 pw[JR];
   unsigned ps[JR];
@@ -211,12 +212,11 @@ void k_dec_attn_proj(DecAttnArgs a) {
     static_assert(DH == 64, "a wavefront of output columns");
     if (wv == 0) {
       const AttnParts p = attn_parts_load(a.parts + (int64_t)h * a.ranges * (DH + 2), a.ranges, DH, lane);
-      const int T = a.pos[0] + 1, per = attn_split_keys(T, a.ranges, kAttnSplitTile);
-      oh[lane] = attn_parts_merge(p, (T + per - 1) / per, lane);
+      oh[lane] = attn_parts_merge(p, attn_split_keys(posv + 1, a.ranges, kAttnSplitTile).n, lane);
     }
     __syncthreads();
   } else {
-    const int T = a.pos[0] + 1;
+    const int T = posv + 1;
     const unsigned kvs4 = (unsigned)(D / 4);
     const float4 q4 = *(const float4 *)(a.q + h * DH + 4 * c);
     const float4 *__restrict__ kp = (const float4 *)(a.kc + h * DH) + c;
@@ -362,7 +362,7 @@ void k_dec_attn_proj_q8(DecAttnQ8Args a) {
   const int h = blockIdx.x, H = gridDim.x, D = H * DH, nb = D / 32;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = lane / LPK, c = lane % LPK;
-  const int rr = D / (int)gridDim.y, rbase = (int)blockIdx.y * rr;
+  const int rr = uniform_div(D, (int)gridDim.y), rbase = (int)blockIdx.y * rr;
   const int pc = tid % CPR, pr0 = tid / CPR;
   uint4 pw[JR];
   unsigned ps[JR];

@@ -197,10 +197,11 @@ void k_gqa_attn_proj(GqaAttnArgs a) {
   __shared__ __align__(16) float oh[DH];
   const int H = gridDim.x, D = a.D, KD = a.KD;
   const int h = attn_head_of_block(blockIdx.x, H, KD / DH);  // the query heads of a key / value head on one XCD
-  const int hk = h / (H / (KD / DH));
+  const int hk = uniform_div(h, uniform_div(H, KD / DH));
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = lane / LPK, c = lane % LPK;
-  const int rr = D / (int)gridDim.y, rbase = (int)blockIdx.y * rr;
+  const int posv = a.pos[0];  // (asked for here, by all: where one wavefront alone wants it, it is one more round trip behind the records)
+  const int rr = uniform_div(D, (int)gridDim.y), rbase = (int)blockIdx.y * rr;
   const int pc = tid & 1, pr0 = tid >> 1;
   uint4 pw[JR];
   unsigned ps[JR];
@@ -224,12 +225,11 @@ void k_gqa_attn_proj(GqaAttnArgs a) {
     static_assert(DH == 64, "a wavefront of output columns");
     if (wv == 0) {
       const AttnParts p = attn_parts_load(a.parts + (int64_t)h * a.ranges * (DH + 2), a.ranges, DH, lane);
-      const int T = a.pos[0] + 1, per = attn_split_keys(T, a.ranges, kAttnSplitTile);
-      oh[lane] = attn_parts_merge(p, (T + per - 1) / per, lane);
+      oh[lane] = attn_parts_merge(p, attn_split_keys(posv + 1, a.ranges, kAttnSplitTile).n, lane);
     }
     __syncthreads();
   } else {
-    const int T = a.pos[0] + 1;
+    const int T = posv + 1;
     const unsigned kvs4 = (unsigned)(KD / 4);
     const float4 q4 = *(const float4 *)(a.q + h * DH + 4 * c);
     const float4 *__restrict__ kp = (const float4 *)(a.kc + hk * DH) + c;

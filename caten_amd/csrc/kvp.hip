@@ -65,14 +65,13 @@ void k_attn_cached_paged(float *__restrict__ out, const float *__restrict__ q, c
   const int T = start_pos + (pos ? pos[0] : 0) + 1;
   int k0 = 0, k1 = T, nranges = 1;
   if (STEP) {
-    const int nz = (int)gridDim.z, tiles = (T + TILE - 1) / TILE;
-    const int per = ((tiles + nz - 1) / nz) * TILE;  // keys per range
-    nranges = (T + per - 1) / per;
-    k0 = (int)blockIdx.z * per;
+    const AttnRanges r = attn_split_keys(T, (int)gridDim.z, TILE);
+    nranges = r.n;
+    k0 = (int)blockIdx.z * r.per;
     if (k0 >= T) return;  // (uniform) no range for this workgroup
-    k1 = min(T, k0 + per);
+    k1 = min(T, k0 + r.per);
   }
-  const int hk = h / (H / Hkv);
+  const int group = uniform_div(H, Hkv), hk = uniform_div(h, group);
   const int KD = Hkv * DH;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = lane / LPK, c = lane % LPK;
@@ -109,7 +108,7 @@ void k_attn_cached_paged(float *__restrict__ out, const float *__restrict__ q, c
         q4 = rope4_apply(q4, ra);
         kn = rope4_apply(kn, ra);
       }
-      if (h % (H / Hkv) == 0 && tid < LPK && blockIdx.z == 0) {
+      if (h == hk * group && tid < LPK && blockIdx.z == 0) {
         float *kd = const_cast<float *>(kvp_row(kpages, T - 1, KD)), *vd = const_cast<float *>(kvp_row(vpages, T - 1, KD));
         ((float4 *)(kd + hk * DH))[c] = kn;
         ((float4 *)(vd + hk * DH))[c] = vn;

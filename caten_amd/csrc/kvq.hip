@@ -186,20 +186,32 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
   __shared__ float ang_s[DH / 2], ang_c[DH / 2];
   __shared__ int ticket;
   const int h = attn_head_of_block(blockIdx.x, H, Hkv);
-  const int T = pos[0] + 1;
-  int k0 = 0, k1 = T, nranges = 1;
-  {
-    const int per = attn_split_keys(T, (int)gridDim.z, TILE);
-    nranges = (T + per - 1) / per;
-    k0 = (int)blockIdx.z * per;
-    if (k0 >= T) return;  // (uniform) no range for this workgroup
-    k1 = min(T, k0 + per);
-  }
-  const int group = H / Hkv, hk = h / group;
+  const int group = uniform_div(H, Hkv), hk = uniform_div(h, group);
   const int KD = Hkv * DH, nb = KD / 32;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = lane / LPK, c = lane % LPK;
   const int col = hk * DH + 16 * c;  // first of this lane's 16 elements inside a cache row
+  auto load16 = [&](const float *src, float *x) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const float4 v = *(const float4 *)(src + 4 * e);
+      x[4 * e] = v.x, x[4 * e + 1] = v.y, x[4 * e + 2] = v.z, x[4 * e + 3] = v.w;
+    }
+  };
+  const int posv = pos[0];
+  float qr[16], kn[16], vn[16];  // the query and the new row, asked for beside the position
+  load16(qv + (int64_t)h * DH + 16 * c, qr);
+  load16(newkv + col, kn);
+  load16(newkv + KD + col, vn);
+  const int T = posv + 1;
+  int k0 = 0, k1 = T, nranges = 1;
+  {
+    const AttnRanges r = attn_split_keys(T, (int)gridDim.z, TILE);
+    nranges = r.n;
+    k0 = (int)blockIdx.z * r.per;
+    if (k0 >= T) return;  // (uniform) no range for this workgroup
+    k1 = min(T, k0 + r.per);
+  }
   // A tile's rows and scales.  The first tile is asked for as soon as the position is known, before the angles, the
   // query and the new row are worked on: its round trip to memory runs beside that arithmetic.
   uint4 kr[KPT], vr[KPT];
@@ -215,7 +227,8 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
       vs[u] = vd[(int64_t)jj * nb + (col >> 5)];
     }
   };
-  if (k0 + wv * KPT * KPW < k1) request(k0);  // (uniform per wavefront)
+  __builtin_amdgcn_sched_barrier(0);
+  request(k0);  // (every wavefront: behind a branch, whatever is waited for next would be waited for with these)
   if (rope) {
     if (tid < DH / 2) {  // theta_i = base^(-2i / DH), as k_rope spells it
       const float expo = (float)(2 * tid) / (float)DH;
@@ -227,13 +240,6 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
     }
     __syncthreads();
   }
-  auto load16 = [&](const float *src, float *x) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float4 v = *(const float4 *)(src + 4 * e);
-      x[4 * e] = v.x, x[4 * e + 1] = v.y, x[4 * e + 2] = v.z, x[4 * e + 3] = v.w;
-    }
-  };
   auto rotate16 = [&](float *x) {  // pairs 8c .. 8c + 7 of the head
 #pragma unroll
     for (int t = 0; t < 8; t++) {
@@ -242,13 +248,11 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
       x[2 * t] = o0, x[2 * t + 1] = o1;
     }
   };
-  float qr[16];
-  load16(qv + (int64_t)h * DH + 16 * c, qr);
   if (rope) rotate16(qr);
   // the new row of this key / value head: needed by the range that ends at T, and by the one that stores it
   uint4 knq = make_uint4(0u, 0u, 0u, 0u), vnq = knq;
   unsigned knd = 0, vnd = 0;
-  const bool has_new = k1 == T, stores = blockIdx.z == 0 && h % group == 0;
+  const bool has_new = k1 == T, stores = blockIdx.z == 0 && h == hk * group;
   if (has_new || stores) {  // (uniform)
     auto quantise = [&](const float *x, uint4 &qv4, unsigned &dv) {  // lanes c and c ^ 1 share a block of 32
       float amax = 0.0f;
@@ -267,12 +271,9 @@ __global__ __launch_bounds__(256) void k_attn_q8_step(float *__restrict__ out, c
       qv4 = make_uint4(w[0], w[1], w[2], w[3]);
       dv = __builtin_bit_cast(unsigned short, (_Float16)dd);
     };
-    float x[16];
-    load16(newkv + col, x);
-    if (rope) rotate16(x);
-    quantise(x, knq, knd);
-    load16(newkv + KD + col, x);
-    quantise(x, vnq, vnd);
+    if (rope) rotate16(kn);
+    quantise(kn, knq, knd);
+    quantise(vn, vnq, vnd);
     if (stores && tid < LPK) {  // the `!assign` into the cache row at pos
       *(uint4 *)(kq + (int64_t)(T - 1) * KD + col) = knq;
       *(uint4 *)(vq + (int64_t)(T - 1) * KD + col) = vnq;

@@ -1079,21 +1079,21 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
   __shared__ float pm[NW], pl[NW];
   __shared__ int ticket;
   const int h = attn_head_of_block(blockIdx.x, H, Hkv), i = blockIdx.y;
+  const int group = uniform_div(H, Hkv), hk = uniform_div(h, group);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int g = lane / LPK, c = lane % LPK;
+  float4 q4 = *(const float4 *)(q + ((int64_t)i * H + h) * DH + 4 * c);  // (in front of the position's round trip)
   const int T = start_pos + (pos ? pos[0] : 0) + i + 1;
   // this workgroup's keys [k0, k1): everything, or one of `nranges` ranges of whole tiles
   int k0 = 0, k1 = T, nranges = 1;
   if (SPLIT) {
-    const int per = attn_split_keys(T, (int)gridDim.z, TILE);
-    nranges = (T + per - 1) / per;
-    k0 = (int)blockIdx.z * per;
+    const AttnRanges r = attn_split_keys(T, (int)gridDim.z, TILE);
+    nranges = r.n;
+    k0 = (int)blockIdx.z * r.per;
     if (k0 >= T) return;  // (uniform) no range for this workgroup
-    k1 = min(T, k0 + per);
+    k1 = min(T, k0 + r.per);
   }
-  const int hk = h / (H / Hkv);
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int g = lane / LPK, c = lane % LPK;
   const unsigned kvs4 = (unsigned)(Hkv * DH / 4);
-  float4 q4 = *(const float4 *)(q + ((int64_t)i * H + h) * DH + 4 * c);
   const float4 *__restrict__ kp = (const float4 *)(kc + (int64_t)hk * DH) + c;
   const float4 *__restrict__ vp = (const float4 *)(vc + (int64_t)hk * DH) + c;
   const float scale = 1.0f / sqrtf((float)DH);
@@ -1124,7 +1124,7 @@ void k_attn_cached(float *__restrict__ out, const float *__restrict__ q,
       const Rope4 ra = rope4_angles(c, DH, log2_base, T - 1);
       q4 = rope4_apply(q4, ra);
       kn = rope4_apply(kn, ra);
-      if (h % (H / Hkv) == 0 && tid < LPK && (!SPLIT || blockIdx.z == 0)) {
+      if (h == hk * group && tid < LPK && (!SPLIT || blockIdx.z == 0)) {
         ((float4 *)(kc + (int64_t)(T - 1) * KD + hk * DH))[c] = kn;
         ((float4 *)(vc + (int64_t)(T - 1) * KD + hk * DH))[c] = vn;
       }
@@ -1432,7 +1432,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma(float *__restrict__ out, 
   const int h = blockIdx.x, i0 = (gridDim.y - 1 - blockIdx.y) * 32;  // the longest groups are dispatched first
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int half = lane >> 5, col = lane & 31;
-  const int hk = h / (H / Hkv), KD = Hkv * DH;
+  const int hk = uniform_div(h, uniform_div(H, Hkv)), KD = Hkv * DH;
   const int qrow = min(i0 + col, S - 1);  // rows past the end repeat the last one and are not stored
   const int Tq = start_pos + qrow + 1;    // keys this lane's query sees
   const int Tmax = start_pos + min(i0 + 32, S);
@@ -1627,7 +1627,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma_bf(float *__restrict__ ou
   const int h = blockIdx.x, i0 = (gridDim.y - 1 - blockIdx.y) * 32;  // the longest groups are dispatched first
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int half = lane >> 5, col = lane & 31;
-  const int hk = h / (H / Hkv), KD = Hkv * DH;
+  const int hk = uniform_div(h, uniform_div(H, Hkv)), KD = Hkv * DH;
   const int qrow = min(i0 + col, S - 1);  // rows past the end repeat the last one and are not stored
   const int Tq = start_pos + qrow + 1;    // keys this lane's query sees
   const int Tmax = start_pos + min(i0 + 32, S);
