@@ -125,6 +125,10 @@ struct PlaneStore {
   __device__ __forceinline__ PlaneStore(const PlaneGemmArgs &a)
       : C(early(a.C)), bias(early(a.bias)), residual(early(a.residual)), planes(early(a.planes)), M(early(a.M)), N(early(a.N)), act(early(a.act)), pairs(early(a.pairs)),
         routed(early(a.routed)), pkb(early(a.pkb)), route(a.route) {}
+  // left to the compiler, right in front of their use: kernels whose first loads are what a launch waits for
+  struct Late {};
+  __device__ __forceinline__ PlaneStore(const PlaneGemmArgs &a, Late)
+      : C(a.C), bias(a.bias), residual(a.residual), planes(a.planes), M(a.M), N(a.N), act(a.act), pairs(a.pairs), routed(a.routed), pkb(a.pkb), route(a.route) {}
 };
 // columns col .. col + 3, all of them inside, of one row of a finished tile: bias bb (where a.bias), activation, residual rr (where a.residual), and where they go
 __device__ __forceinline__ void plane_gemm_finish(const PlaneStore &a, int N, int row, int col, float4 v4, float4 bb, float4 rr) {
