@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemv_int.h"
 #include "gemv_kernels.h"
 #include "decode_fused.h"
 
@@ -67,9 +68,9 @@ __device__ __forceinline__ void gqa_stage_request(const GqaStage &s, GqaStageReg
   }
 }
 
-// gamma * x to LDS (swizzled), 1 / rms(x) returned; block 0 stores x to s.xout.  red holds NT / 64 floats.
-template <int NT, int NV, bool ACC>
-__device__ __forceinline__ float gqa_stage_finish(const GqaStage &s, GqaStageRegs<NV, ACC> &r, float *xs, float *red) {
+// gamma * x handed to `put` (which float4 of the vector, its value), 1 / rms(x) returned behind a barrier; block 0 stores x to s.xout.  red holds NT / 64 floats.
+template <int NT, int NV, bool ACC, class Put>
+__device__ __forceinline__ float gqa_stage_finish(const GqaStage &s, GqaStageRegs<NV, ACC> &r, float *red, Put put) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (ACC) {
 #pragma unroll
@@ -91,7 +92,7 @@ __device__ __forceinline__ float gqa_stage_finish(const GqaStage &s, GqaStageReg
   for (int k = 0; k < NV; k++) {
     const float4 v = r.v[k], g = r.g[k];
     ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
-    ((float4 *)xs)[swz(tid + NT * k)] = make_float4(v.x * g.x, v.y * g.y, v.z * g.z, v.w * g.w);
+    put(tid + NT * k, make_float4(v.x * g.x, v.y * g.y, v.z * g.z, v.w * g.w));
     if (blockIdx.x == 0 && s.xout) ((float4 *)s.xout)[tid + NT * k] = v;
   }
   ss = wave_sum(ss);
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(NT) void k_gqa_qkv(GqaQkvArgs a) {
     const uint4 zz = make_uint4(0u, 0u, 0u, 0u);
     for (int64_t k = (int64_t)blockIdx.x * NT + tid; k < a.zero_n16; k += (int64_t)gridDim.x * NT) z[k] = zz;
   }
-  const float rstd = gqa_stage_finish<NT>(a.st, sr, xs, red);
+  const float rstd = gqa_stage_finish<NT>(a.st, sr, red, [&](int k, float4 v) __attribute__((always_inline)) { ((float4 *)xs)[swz(k)] = v; });
   float acc[RW];
 #pragma unroll
   for (int u = 0; u < RW; u++) acc[u] = 0.0f;
@@ -344,34 +345,37 @@ void k_gqa_attn_proj(GqaAttnArgs a) {
 }
 
 // ---- launch 3: RMSNorm folded through 32 gate and 32 up rows, SwiGLU, one Q4_0 block per row of `down` ----
-template <int KC, int NT>
+// The 64 rows are four groups of 16 for the matrix cores (gemv_int.hip): every wavefront takes an eighth of K, 256 columns, of all of them, so that it reads its
+// digits once for four groups.  (In vector instructions, a row of 2048 to a wavefront at a time, products and sums were 2.8 us of a launch; as integers 11.1 -> 10.3 us.)
+// What is left is what a workgroup has to read: 128 KB of accumulators, 111 KB of weights, at 64 bytes a clock.
+template <int NT>
 __global__ __launch_bounds__(NT) void k_gqa_mlp(GqaMlpArgs a) {
-  constexpr int RW = 32 / (NT / 64);    // gate rows (and up rows) per wavefront
-  constexpr int PJ = 2048 * KC / NT;    // rows of the down projection per thread
-  __shared__ __align__(16) float xs[2048 * KC];
-  __shared__ float red[NT / 64];
-  __shared__ __align__(16) float hs[32];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int D = a.st.D;
+  constexpr int NW = NT / 64, D = 2048, NG = 4, PJ = D / NT;  // PJ: rows of the down projection per thread
+  static_assert(NW == D / 256 && NT == D / 4, "a unit of 256 columns to a wavefront, four floats of the vector to a thread");
+  constexpr int CB = 128;  // bytes of digits per chunk
+  __shared__ __align__(16) unsigned char dig[256 + D / 32 * CB];  // 256 bytes of zeros in front
+  __shared__ float sx[D / 32], red[NW];
+  __shared__ float part[NW][16 * NG];
+  __shared__ __align__(16) float hs[NW][32];
+  __shared__ __align__(16) unsigned char hd[NW][CB];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, i = lane & 15;
   const int slab = blockIdx.x;
-  GqaStageRegs<512 * KC / NT, true> sr;
+  GqaStageRegs<1, true> sr;
   gqa_stage_request<NT>(a.st, sr);
   __builtin_amdgcn_sched_barrier(0);
-  uint4 wg[RW][KC], wu[RW][KC];
-  unsigned sg[RW][KC], su[RW][KC];
+  // groups 0, 1: the slab's gate rows, 2, 3: its up rows; chunks 2g and 2g + 1 of the wavefront's unit
+  uint4 wt[NG][2];
+  unsigned st[NG];
 #pragma unroll
-  for (int u = 0; u < RW; u++) {
-    const int64_t gr = (int64_t)(slab * 32 + wv * RW + u) * a.gate_stride, ur = gr + a.up_off;
-#pragma unroll
-    for (int j = 0; j < KC; j++) {
-      const int64_t gi = gr * (64 * KC) + lane + 64 * j, ui = ur * (64 * KC) + lane + 64 * j;
-      wg[u][j] = ((const uint4 *)a.wq)[gi];
-      wu[u][j] = ((const uint4 *)a.wq)[ui];
-      sg[u][j] = a.wd[gi];
-      su[u][j] = a.wd[ui];
-    }
+  for (int q = 0; q < NG; q++) {
+    const int64_t row0 = (int64_t)(slab * 32 + 16 * (q & 1)) * a.gate_stride + (q < 2 ? 0 : a.up_off);  // (the same for the wavefront)
+    const unsigned off = (unsigned)(i * a.gate_stride * (D / 32) + wv * 8 + 2 * g);
+    const uint4 *wq = (const uint4 *)((const char *)a.wq + row0 * (D / 2) + 16u * off);
+    wt[q][0] = wq[0];
+    wt[q][1] = wq[1];
+    st[q] = *(const unsigned *)((const char *)a.wd + row0 * (D / 16) + 2u * off);
   }
-  // this slab's block of every row of the down projection: row r = tid + NT j (D = 2048 * KC)
+  // this slab's block of every row of the down projection: row r = tid + NT j
   uint4 pw[PJ];
   unsigned ps[PJ];
 #pragma unroll
@@ -381,48 +385,59 @@ __global__ __launch_bounds__(NT) void k_gqa_mlp(GqaMlpArgs a) {
     ps[j] = a.pd[idx];
   }
   __builtin_amdgcn_sched_barrier(0);
-  const float rstd = gqa_stage_finish<NT>(a.st, sr, xs, red);
-  float ag[RW], au[RW];
+  if (tid < 64) ((unsigned *)dig)[tid] = 0u;
+  const float rstd = gqa_stage_finish<NT>(a.st, sr, red, [&](int k, float4 v) __attribute__((always_inline)) {
+    const float x[4] = {v.x, v.y, v.z, v.w};
+    unsigned w[4];
+    const float down = int_digits(x, w);
+    int_digits_put(dig + 256, sx, k, w, down);
+  });
+  {
+    const bool act = (i >> 2) == g;  // this lane's row of the first operand belongs to its own chunk of k
+    const unsigned char *dl = act ? dig + 256 + (wv * 8 + 2 * g) * CB + (i & 3) * 16 : dig + (lane < 32 ? 192 : 64);
+    float acc[NG] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int u = 0; u < RW; u++) ag[u] = au[u] = 0.0f;
+    for (int s = 0; s < 2; s++) {
+      const v4i a0 = *(const v4i *)(dl + (act ? s * CB : 0)), a1 = *(const v4i *)(dl + (act ? s * CB + 64 : 0));
+      const float sc = sx[wv * 8 + 2 * g + s];
 #pragma unroll
-  for (int j = 0; j < KC; j++) {
-    float xr[32];
-    const float xsum = read_block(xs, lane + 64 * j, xr);
-#pragma unroll
-    for (int u = 0; u < RW; u++) {
-      ag[u] += chunk_dot<CTHIP_Q4_0>(wg[u][j], half_bits_to_float((unsigned short)sg[u][j]), xr, xsum);
-      au[u] += chunk_dot<CTHIP_Q4_0>(wu[u][j], half_bits_to_float((unsigned short)su[u][j]), xr, xsum);
+      for (int q = 0; q < NG; q++) acc[q] = fmaf(half_bits_to_float((unsigned short)(s ? st[q] >> 16 : st[q])) * sc, int_chunk(wt[q][s], a0, a1), acc[q]);
     }
-  }
 #pragma unroll
-  for (int u = 0; u < RW; u++) {
-    ag[u] = wave_sum(ag[u]);
-    au[u] = wave_sum(au[u]);
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int u = 0; u < RW; u++) hs[wv * RW + u] = ct_silu(rstd * ag[u]) * (rstd * au[u]);
+    for (int q = 0; q < NG; q++) {
+      acc[q] += __shfl_xor(acc[q], 16, 64);
+      acc[q] += __shfl_xor(acc[q], 32, 64);
+    }
+    part[wv][lane] = g == 0 ? acc[0] : g == 1 ? acc[1] : g == 2 ? acc[2] : acc[3];
   }
   __syncthreads();
-  float hr[32], hsum;
-  {
-    float p8[8];
+  {  // every wavefront for itself: lanes 0 .. 31 the gates, 32 .. 63 the ups
+    float v = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-      const float4 v = *(const float4 *)(hs + 4 * t);
-      hr[4 * t + 0] = v.x;
-      hr[4 * t + 1] = v.y;
-      hr[4 * t + 2] = v.z;
-      hr[4 * t + 3] = v.w;
-      p8[t] = (v.x + v.y) + (v.z + v.w);
-    }
-    hsum = ((p8[0] + p8[1]) + (p8[2] + p8[3])) + ((p8[4] + p8[5]) + (p8[6] + p8[7]));
+    for (int w = 0; w < NW; w++) v += part[w][lane];
+    v *= rstd;
+    const float up = __shfl_xor(v, 32, 64);
+    if (lane < 32) hs[wv][lane] = ct_silu(v) * up;
+    __builtin_amdgcn_wave_barrier();
   }
+  // the 32 hidden units are one chunk of every row of the down projection: a lane's own row takes the place of its own chunk
+  const float4 h4 = *(const float4 *)(hs[wv] + 4 * (lane & 7));
+  const float hx[4] = {h4.x, h4.y, h4.z, h4.w};
+  unsigned hw[4];
+  const float down = int_digits(hx, hw);  // (the same in every lane)
+  if (lane < 8) {
+    unsigned *o = (unsigned *)(hd[wv] + (lane >> 2) * 64) + (lane & 3);
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[4 * r] = hw[r];
+  }
+  __builtin_amdgcn_wave_barrier();
+  const bool act = (i >> 2) == g;
+  const unsigned char *hl = act ? hd[wv] + (i & 3) * 16 : dig + (lane < 32 ? 192 : 64);
+  const v4i h0 = *(const v4i *)hl, h1 = *(const v4i *)(hl + (act ? 64 : 0));
   long long *accum = a.accum + (int64_t)xcd_id() * D;
 #pragma unroll
   for (int j = 0; j < PJ; j++) {
-    const float s = chunk_dot<CTHIP_Q4_0>(pw[j], half_bits_to_float((unsigned short)ps[j]), hr, hsum);
+    const float s = half_bits_to_float((unsigned short)ps[j]) * down * int_chunk(pw[j], h0, h1);
     __hip_atomic_fetch_add(accum + tid + NT * j, to_fix(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
 }
@@ -512,7 +527,7 @@ int launch_gqa_mlp(const GqaMlpArgs &a, int F, int HKV) {
   if (D != 2048 || F % 32) return fail(CTHIP_E_BAD_ARG, "decoder: fused SwiGLU launch with D = %d, F = %d", D, F);
   dim3 grid(F / 32), block(512);
   hipStream_t st = state().stream;
-  hipLaunchKernelGGL((k_gqa_mlp<1, 512>), grid, block, 0, st, a);
+  hipLaunchKernelGGL((k_gqa_mlp<512>), grid, block, 0, st, a);
   CTHIP_LAUNCH_CHECK();
   return 0;
 }

@@ -129,3 +129,26 @@ def test_sessions_match_the_vector_kernels(ops, arch, kind):
     assert runs[0][0] == runs[1][0]
     for a, b in zip(runs[0][1], runs[1][1]):
         assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
+
+
+# The three-launch layer's MLP: a workgroup to 32 hidden units, one of them, an odd number, whole rounds and a last one.  Against a launch per Linear: hidden units and
+# down projection are sums of 2048 and ffn products, off by at most (n + 2) 2^-24 of their terms' magnitudes on either side, which are a few times the sums here; two layers and the head.
+@pytest.mark.parametrize("ffn", [32, 96, 1120])
+def test_layers_of_slabs_match_a_launch_per_linear(ffn):
+    print(f"case: three-launch layer, {ffn} hidden units", flush=True)
+    from caten_amd import _lib, llm, synth
+    lib = _lib.load()
+    cfg = dict(synth.LLAMA_CONFIGS["llama-1.1b"], ffn=ffn, n_layers=2, vocab=1003, max_seq=64)
+    sd = llm.llama_state_dict(synth.llama_weights(cfg, seed=17), "q4_0")
+    prompt, runs = synth.prompt(cfg["vocab"], 7, seed=17), []
+    try:
+        for fused in (1, 0):
+            _lib.check(lib.cthip_set_option(b"decode_fused", fused))
+            model = llm.make_llama(cfg, sd)
+            runs.append(llm.gpt2_generate(model, prompt, 8, on_device=False, keep_logits=True))
+            model.close()
+    finally:
+        _lib.check(lib.cthip_set_option(b"decode_fused", 1))
+    assert runs[0][0] == runs[1][0]
+    for a, b in zip(runs[0][1], runs[1][1]):
+        assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
