@@ -126,6 +126,36 @@ def test_small_rows_against_large_weights(ops, rows, cols, m):
     w.free()
 
 
+@pytest.mark.parametrize("prologue", [None, "swiglu"])
+@pytest.mark.parametrize("rows,cols", [(4096, 2052), (1100, 11000)])
+def test_rows_small_in_part_or_whole(ops, rows, cols, prologue):
+    """Several blocks share an input row without a norm, 2048 columns each: ordinary rows, rows that only one block can tell from small ones, small ones, one of zeros.  With SwiGLU
+    at gates of 16, silu(g) = g (1 - 1e-7): its own error, a few 2^-24 of a value, adds to the sums'."""
+    rng = np.random.default_rng(rows)
+    a = rng.normal(0, 1e30, (rows, cols)).astype(np.float32)
+    w = ops.WeightMatrix("f32", a, rows, cols)
+    v = rng.normal(0, 1, (7, cols))
+    v[1, :2048] *= 1e-20
+    v[2, 2048:] *= 1e-20
+    v[3] *= 1e-15
+    v[4] *= 1e-30
+    v[4, -1] = 2.0 ** -20
+    v[5] *= 2.0 ** -40
+    v[5, :2048] = 0.0
+    v[6] = 0.0
+    x = v.astype(np.float32)
+    if prologue:
+        gate = np.full_like(x, 16.0)
+        x64 = 16.0 / (1 + np.exp(-16.0)) * (x / 16.0).astype(np.float64)
+        x = np.concatenate([gate, x / np.float32(16.0)], 1)
+    else:
+        x64 = x.astype(np.float64)
+    got, want = ops.linear(x, w, prologue=prologue), x64 @ a.astype(np.float64).T
+    bound = (tree_bound(cols) + (8 * 2.0 ** -24 if prologue else 0)) * (np.abs(x64) @ np.abs(a.astype(np.float64)).T)
+    assert np.all(np.abs(got - want) <= bound)
+    w.free()
+
+
 @pytest.mark.parametrize("kind,rows,cols,m,precision", [
     ("f16", 2100, 28672, 27, 2), ("f16", 2100, 28672, 32, 2), ("f16", 2100, 28672, 18, 3), ("f16", 2100, 28672, 32, 3), ("f16", 2050, 29568, 25, 2),
     ("f16", 2500, 24576, 31, 2), ("q4_0", 4098 * 128, 2240, 16, 2), ("f16", 2100, 28672, 17, 2), ("f16", 2100, 28672, 16, 2), ("q8_0", 1700, 28672, 16, 3)])
