@@ -112,13 +112,14 @@ struct DigitsPick {
 // What the result is: rows of floats, rows as digits, SwiGLU of (gate, up) columns as digits (a wavefront's columns have to be whole blocks of results), or raw sums of a share of K
 enum { kDigitsPlain = 0, kDigitsOut = 1, kDigitsOutPairs = 2, kDigitsShares = 3 };
 // shares: whether K may be split (deferred: the launch behind adds the shares up on its way).  A launch is its ends and a time per block of 32 k of the fullest compute unit, us:
-// `first`, and `more` (`many` past two) for each further tile.  Fitted to weights out of memory: 64 x 64 / 64 x 128 / 128 x 128 for 100 x 3072 x 1024 10.0 / 12.3 / 18.5,
+// `first` (and `filled` times the share of the compute units that have a tile: a step of 128 x 128 takes 0.34 us on 60 of them, 0.41 on 240), and `more` (`many` past two) for each
+// further tile.  Fitted to weights out of memory: 64 x 64 / 64 x 128 / 128 x 128 for 100 x 3072 x 1024 10.0 / 12.3 / 18.5,
 // 300 x 2560 x 2048 15.7 / 19.4 / 29.6, 200 x 11264 x 2048 34 / 28 / 33, 280 x 4096 x 4096 40 / 35 / 52, 1900 x 2048 x 5632 98 / 71 / 80, 1900 x 11264 x 2048 195 / 133 / 128.
 inline DigitsPick digits_pick(int M, int N, int nkb, int out, bool shares, bool deferred, int cus) {
   static const struct {
     int bm, bn;
-    double ends, first, more, many;
-  } tiles[] = {{64, 64, 4.4, 0.175, 0.095, 0.14}, {64, 128, 5.0, 0.235, 0.14, 0.18}, {128, 128, 7.6, 0.35, 0.26, 0.30}};
+    double ends, first, filled, more, many;
+  } tiles[] = {{64, 64, 4.4, 0.175, 0.0, 0.095, 0.14}, {64, 128, 5.0, 0.235, 0.0, 0.14, 0.18}, {128, 128, 7.6, 0.32, 0.10, 0.26, 0.30}};
   DigitsPick best = {1, 1, 1, 1e30};
   for (int ks = 1; ks <= (shares ? 8 : 1); ks++) {
     const int per = (nkb + ks - 1) / ks;
@@ -126,7 +127,7 @@ inline DigitsPick digits_pick(int M, int N, int nkb, int out, bool shares, bool 
     for (int t = out == kDigitsOutPairs ? 1 : 0; t < 3; t++) {
       const int64_t of_xcd = ((int64_t)((M + tiles[t].bm - 1) / tiles[t].bm) * ((N + tiles[t].bn - 1) / tiles[t].bn) + 7) / 8 * ks;
       const int fullest = (int)((of_xcd * 8 + cus - 1) / cus);
-      const double us = tiles[t].ends + (out ? 2.5 : 0.0) + per * (tiles[t].first + (fullest <= 2 ? tiles[t].more : tiles[t].many) * (fullest - 1)) +
+      const double us = tiles[t].ends + (out ? 2.5 : 0.0) + per * (tiles[t].first + tiles[t].filled * std::min(1.0, of_xcd * 8.0 / cus) + (fullest <= 2 ? tiles[t].more : tiles[t].many) * (fullest - 1)) +
                         (ks > 1 ? (deferred ? 0.3 : 2.6) + (deferred ? 0.6e-6 : 0.85e-6) * 4.0 * ks * M * N : 0.0);
       if (us < best.us) best = {t, ks, fullest, us};
     }
