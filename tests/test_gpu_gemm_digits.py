@@ -24,10 +24,11 @@ def bound(x, w):
     return 2.0 ** -19 * xb.max(-1) @ wb.sum(-1).T + (x.shape[1] / 32 + 32) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
 
 
-# tile 64 x 64 with 1, 3, 5 shares; 64 x 128 with few workgroups (1, 2, 4, 7 shares) and many; 128 x 128 with 1, 2, 5 shares
+# tile 64 x 64 with 1, 3, 5 shares; 64 x 128 with few workgroups (1, 2, 4, 7 shares) and many (the line behind them too); 128 x 128 with 1 and 3 shares (the last line)
 @pytest.mark.parametrize("rows,cols,m", [(3001, 64, 2049), (9001, 64, 701), (1026, 4128, 513), (514, 8224, 577),
                                          (6401, 96, 577), (2051, 288, 1025), (4100, 4128, 129), (6401, 4128, 65), (4100, 8224, 97), (6401, 64, 1537),
-                                         (12001, 288, 1537), (3001, 544, 2049), (2051, 8224, 701), (2051, 8224, 577)])
+                                         (12001, 288, 1537), (3001, 544, 2049), (2051, 8224, 701), (2051, 8224, 577),
+                                         (9001, 1056, 641), (12001, 544, 1537), (9001, 8224, 193)])
 def test_linear_digits(ops, rows, cols, m):
     rng = np.random.default_rng(rows + m)
     w = weights(ops, rows, cols, rng)
