@@ -161,8 +161,28 @@ static void matrix_products() {
   }
 }
 
+// Linears on 4-bit weights through 6-bit digits, one share of K, us with tiles of 64 x 64, 64 x 128, 128 x 128
+static void tiles_of_digits() {
+  static const struct {
+    int m, n, k;
+    double us[3];
+  } t[] = {{100, 3072, 1024, {10.0, 12.3, 18.5}},
+           {300, 2560, 2048, {15.7, 19.4, 29.6}},
+           {200, 11264, 2048, {34.0, 28.0, 33.0}},
+           {280, 4096, 4096, {40.0, 35.0, 52.0}},
+           {1900, 2048, 5632, {98.0, 71.0, 80.0}},
+           {1900, 11264, 2048, {195.0, 133.0, 128.0}}};
+  for (const auto &c : t) {
+    const int tile = digits_pick(c.m, c.n, c.k / 32, kDigitsPlain, false, false, 256).tile;
+    char what[96];
+    snprintf(what, sizeof(what), "digits of %d x %d x %d: tile %d takes %.1f us", c.m, c.n, c.k, tile, c.us[tile]);
+    expect(what, c.us[tile] <= std::min(c.us[0], std::min(c.us[1], c.us[2])), true);
+  }
+}
+
 int main() {
   integer_gemv();
+  tiles_of_digits();
   shares_of_tiles();
   linears_over_many_rows();
   matrix_products();
