@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "graph_ops.h"
+#include "graph_plan.h"
 
 namespace cthip {
 
@@ -78,7 +79,7 @@ struct GraphAttn {
   int pre_n[2];
 };
 constexpr int kGraphAttnMaxKeys = 2048;
-__global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
+__global__ __launch_bounds__(kGraphAttnThreads) void k_graph_attn(GraphAttn a) {
   __shared__ float sc[kGraphAttnMaxKeys];
   __shared__ float4 part[16][16];
   __shared__ float red[8];
@@ -126,7 +127,8 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
 #pragma unroll
     for (int u = 0; u < 4; u++) w[u] = at(KB + (int64_t)min(j0 + 16 * u + g, N - 1) * k_sj + k0);
   };
-  const int kc = 4 * c < K ? 4 * c : 0, nwg = gridDim.x * gridDim.y * gridDim.z, unit = tid * nwg + (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+  const int kc = 4 * c < K ? 4 * c : 0;
+  const GraphShare mine = graph_share(((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, (int64_t)gridDim.x * gridDim.y * gridDim.z, tid);
   const f4 x0 = *(gfloat4)(A + kc);
   keys(0, kc, kw);
   __builtin_amdgcn_sched_barrier(0);
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
   for (int u = 0; u < 4; u++) vw[u] = at(VB + (int64_t)min(g + 16 * u, N - 1) * v_sk + (4 * c < Nv ? 4 * c : 0));
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    const f4 t = *(gfloat4)(4 * unit < a.pre_n[q] ? (gfloat)a.pre_in[q] + 4 * unit : A);
+    const f4 t = *(gfloat4)(mine.first < a.pre_n[q] ? (gfloat)a.pre_in[q] + mine.first : A);
     cw[q] = make_float4(t[0], t[1], t[2], t[3]);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -251,8 +253,8 @@ __global__ __launch_bounds__(256) void k_graph_attn(GraphAttn a) {
   // (the copies' first pieces, one to a thread and the workgroups in turn, were asked for with the first values: a round trip to memory less at the end)
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    if (4 * unit < a.pre_n[q]) *(float4 *)(a.pre_out[q] + 4 * unit) = cw[q];
-    for (int t = 4 * (unit + 256 * nwg); t < a.pre_n[q]; t += 1024 * nwg) *(float4 *)(a.pre_out[q] + t) = *(const float4 *)(a.pre_in[q] + t);
+    if (mine.first < a.pre_n[q]) *(float4 *)(a.pre_out[q] + mine.first) = cw[q];
+    for (int64_t t = mine.first + mine.step; t < a.pre_n[q]; t += mine.step) *(float4 *)(a.pre_out[q] + t) = *(const float4 *)(a.pre_in[q] + t);
   }
 }
 
@@ -396,7 +398,7 @@ static int run_attention(const GraphOp *ops, int left, int &rc) {
       a.pre_n[q] = c.ext[2];
     }
   }
-  hipLaunchKernelGGL(k_graph_attn, dim3(s.M, (unsigned)s.nb[2], (unsigned)(s.nb[0] * s.nb[1])), dim3(256), 0, state().stream, a);
+  hipLaunchKernelGGL(k_graph_attn, dim3(s.M, (unsigned)s.nb[2], (unsigned)(s.nb[0] * s.nb[1])), dim3(kGraphAttnThreads), 0, state().stream, a);
   const hipError_t e = hipGetLastError();
   rc = e == hipSuccess ? 0 : fail((int)e, "graph: launch -> %s", hipGetErrorString(e));
   return npre + used;

@@ -58,3 +58,73 @@ def test_a_failing_node_leaves_what_ran_before_it(oracle):
     assert np.allclose(dz.numpy(), oracle.softmax(want), rtol=1e-5, atol=1e-6)
     _lib.check(lib.cthip_vm_destroy(vm))
     _lib.check(lib.cthip_program_destroy(program))
+
+
+@pytest.mark.parametrize("batches,h,s,t,dh", [((3,), 2, 5, 9, 64), ((3, 2), 5, 4, 70, 64), ((1, 7), 3, 2, 33, 128), ((5, 1), 2, 3, 65, 32)])
+def test_attention_over_batches_and_heads(batches, h, s, t, dh):
+    """Copies of the last batch's new key and value rows, scores, softmax, values and the copy that puts the heads side by side, as one launch over every batch axis: each buffer
+    against 64 bits.  Sums of at most `t` or `dh` products of fp32 numbers; exp2's argument, scores below 16 in magnitude, is off by their own error."""
+    import ctypes as C
+    from caten_amd import _lib, blueprints as bp, ops
+    from caten_amd.renderer import item_sexp
+    lib = _lib.init(0)
+    nb, rng, row = int(np.prod(batches)), np.random.default_rng(h * t), h * dh
+    print(f"case: batches {batches}, {h} heads, {s} rows, {t} keys of {dh}", flush=True)
+    add, mul, A = bp._add, bp._mul, bp._A
+
+    def index(*terms):  # (stride, axis) pairs and constants
+        e = 0
+        for x in terms:
+            x = mul(*x) if isinstance(x, tuple) else x
+            e = x if e == 0 else add(e, x)
+        return e
+
+    def nest(name, ext, red, out, body):
+        g = [f"_gid{q}" for q in range(len(ext))]
+        head = [bp._for(x, e) for x, e in zip(g, ext)]
+        mid = [bp._decl("acc", 0.0), bp._for("_gid9", red), bp._red("acc", add("acc", body(g, "_gid9"))), bp._end("_gid9")] if red else []
+        return {"name": name, "blueprint": [bp._glob("val_o", "output", 1)] + [bp._glob(f"val_{x}", "input", 1) for x in ("a", "b")[:2 if red else 1]] + head + mid +
+                [bp._store("val_o", out(g), mul("acc", 0.125) if name == "it_scores" else "acc" if red else body(g, None))] + [bp._end(x) for x in reversed(g)]}
+
+    nax = len(batches)
+    strides = [int(np.prod(batches[q + 1:])) for q in range(nax)]
+    bt = lambda g, k: [(k * strides[q], g[q]) for q in range(nax)]  # noqa: E731
+    copy = nest("it_copy", (row,), None, lambda g: g[0], lambda g, _: A("val_a", g[0]))
+    scores = nest("it_scores", (*batches, h, s, t), dh, lambda g: index(*bt(g, h * s * t), (s * t, g[nax]), (t, g[nax + 1]), g[nax + 2]),
+                  lambda g, k: mul(A("val_a", index(*bt(g, s * row), (dh, g[nax]), (row, g[nax + 1]), k)), A("val_b", index(*bt(g, t * row), (dh, g[nax]), (row, g[nax + 2]), k))))
+    values = nest("it_values", (*batches, h, s, dh), t, lambda g: index(*bt(g, s * row), (s * dh, g[nax]), (dh, g[nax + 1]), g[nax + 2]),
+                  lambda g, k: mul(A("val_a", index(*bt(g, h * s * t), (s * t, g[nax]), (t, g[nax + 1]), k)), A("val_b", index(*bt(g, t * row), (dh, g[nax]), (row, k), g[nax + 2]))))
+    softmax = bp.softmax_rows(rows=nb * h * s, n=t)
+    q, k, v, nk, nv = (rng.normal(0, 1, shape).astype(np.float32) for shape in ((nb, s, h, dh), (nb, t, h, dh), (nb, t, h, dh), (row,), (row,)))
+    d = {n: ops.DeviceArray.from_numpy(x) for n, x in dict(q=q, k=k, v=v, nk=nk, nv=nv).items()}
+    d.update(sc=ops.DeviceArray((nb, h, s, t)), pr=ops.DeviceArray((nb, h, s, t)), o=ops.DeviceArray((nb, h, s, dh)))
+    slots = list(d) + ["k_new", "v_new"]
+    vm, programs = C.c_void_p(), []
+    _lib.check(lib.cthip_vm_create(C.byref(vm), len(slots)))
+    try:
+        for item, args in ((copy, ("k_new", "nk")), (copy, ("v_new", "nv")), (scores, ("sc", "q", "k")), (softmax, ("pr", "sc")), (values, ("o", "pr", "v"))):
+            program, n = C.c_void_p(), len(args)
+            _lib.check(lib.cthip_program_create(C.byref(program), item_sexp(item).encode()))
+            programs.append(program)
+            at = [slots.index(x) for x in args]
+            _lib.check(lib.cthip_vm_add_kernel(vm, program, n, (C.c_int * n)(*[2] * n), (C.c_longlong * n)(*at), (C.c_double * n)(), (C.c_int * n)(), 1, (C.c_int * 1)(0), (C.c_int * 1)(at[0])))
+        new = (nb * t - 1) * row * 4  # the last row of the last batch
+        for slot, x in enumerate(slots):
+            _lib.check(lib.cthip_vm_set_buffer(vm, slot, d[x].ptr if x in d else d[x[0]].ptr + new))
+        for _ in range(2):
+            _lib.check(lib.cthip_vm_run(vm))
+        got = {x: d[x].numpy().astype(np.float64) for x in ("k", "v", "sc", "pr", "o")}
+    finally:
+        _lib.check(lib.cthip_vm_destroy(vm))
+        for program in programs:
+            _lib.check(lib.cthip_program_destroy(program))
+    k.reshape(-1)[-row:], v.reshape(-1)[-row:] = nk, nv
+    assert np.array_equal(got["k"], k) and np.array_equal(got["v"], v)
+    q, k, v = (x.astype(np.float64).transpose(0, 2, 1, 3) for x in (q, k, v))
+    want, eps = q @ k.transpose(0, 1, 3, 2) * 0.125, 2.0 ** -24
+    assert np.all(np.abs(got["sc"] - want) <= dh * eps * (np.abs(q) @ np.abs(k).transpose(0, 1, 3, 2)))
+    assert np.abs(want).max() < 16
+    e = np.exp(got["sc"] - got["sc"].max(-1, keepdims=True))
+    pr = e / e.sum(-1, keepdims=True)
+    assert np.all(np.abs(got["pr"] - pr) <= (t + 64) * eps * pr)  # (16 log2(e) 2^-24 in the argument, twice, and the sum's)
+    assert np.all(np.abs(got["o"] - got["pr"] @ v) <= t * eps * (got["pr"] @ np.abs(v)))
