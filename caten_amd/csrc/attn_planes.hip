@@ -221,7 +221,6 @@ __global__ __launch_bounds__(128 * NW) void k_attn_planes(AttnPlanesArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; r++) o[d][r] = o[d][r] * e0 + mine[(2 + 16 * d + r) * 64] * e1;
   }
-  if (i0 + col >= a.S) return;
   const float inv = 1.0f / l;
   if (a.out_digits) {
     // a lane's halves of two blocks of 32 -> one whole block: lanes 0 .. 31 the even one, lanes 32 .. 63 the odd one
@@ -233,10 +232,13 @@ __global__ __launch_bounds__(128 * NW) void k_attn_planes(AttnPlanesArgs a) {
         const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[d][r] * inv), __float_as_uint(o[d + 1][r] * inv), false, false);
         v[8 * (r >> 2) + (r & 3)] = __uint_as_float(s[0]), v[8 * (r >> 2) + 4 + (r & 3)] = __uint_as_float(s[1]);
       }
-      store_digits32(a.out_digits, (int64_t)(a.S + 31) / 32 * 32, a.H * DH / 32, i0 + col, (h * DH >> 5) + d + half, v);
+      const float m = digits_top(v);
+      const bool rest = digits_uneven_columns(v, m, i0 + col < a.S) || digits_one_large(v, m);
+      if (i0 + col < a.S) store_digits32(a.out_digits, (int64_t)(a.S + 31) / 32 * 32, a.H * DH / 32, i0 + col, (h * DH >> 5) + d + half, v, m, rest);
     }
     return;
   }
+  if (i0 + col >= a.S) return;
 #pragma unroll
   for (int d = 0; d < DB; d++)
 #pragma unroll

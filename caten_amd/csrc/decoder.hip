@@ -31,6 +31,7 @@
 
 #include "common.h"
 #include "decode_fused.h"
+#include "digits.h"
 
 namespace cthip {
 
@@ -919,7 +920,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   const int D = c.dim, F = c.ffn, V = c.vocab, KD = kv_dim(c), Dh = c.dim / c.n_heads;
   const int QW = D + 2 * KD, HW = gpt2 ? F : 2 * F;
   const int prec = state().gemm_precision;
-  const size_t s32 = (size_t)(s + 31) / 32 * 32;  // rows that may go as digits: whole blocks of 32
+  const size_t s32 = (size_t)(s + 31) / 32 * 32;
   int rc = 0;
   float *X = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *Hb = nullptr, *G = nullptr, *KF = nullptr, *VF = nullptr;
   int *ids_dev = nullptr;
@@ -935,13 +936,23 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   do {                        \
     if ((rc = (e))) goto done; \
   } while (0)
+  // rows that may go as terms: whole blocks of 16 rows as matrix operands, of 32 as digits, which take more room than floats (a block may have its rest beside them); whether any do is
+  // settled here, so that no row finds its buffer too small for them later
+  bool digits = false;
+  for (const Layer &L : d->layers)
+    for (const WMat *w : {L.attn, L.proj, L.fc, L.fc2})
+      digits = digits || (w && !d->kvq && prec == GEMM_BF16X3_DEFAULT && linear_terms(w, prec) == kTermsDigits && linear_planes_pays(w, s, prec, true, true));
+  auto terms_bytes = [&](int width) {
+    const size_t floats = sizeof(float) * (s >= 64 ? s32 : (size_t)(s + 15) / 16 * 16) * width;
+    return digits ? std::max(floats, (size_t)digit_row_bytes(s, (width + 31) / 32)) : floats;
+  };
   TRY(alloc((void **)&X, sizeof(float) * (size_t)s * D));
-  TRY(alloc((void **)&XN, sizeof(float) * (s >= 64 ? s32 : (size_t)(s + 15) / 16 * 16) * D));  // (whole blocks of 16 rows as matrix operands)
+  TRY(alloc((void **)&XN, terms_bytes(D)));
   TRY(alloc((void **)&QKV, sizeof(float) * (size_t)s * QW));
   TRY(alloc((void **)&Q, sizeof(float) * (size_t)s * D));
-  TRY(alloc((void **)&ATT, sizeof(float) * (s >= 64 ? s32 : (size_t)s) * D));
-  TRY(alloc((void **)&Hb, sizeof(float) * (s >= 64 ? s32 : (size_t)s) * HW));
-  if (!gpt2) TRY(alloc((void **)&G, sizeof(float) * (s >= 64 ? s32 : (size_t)s) * F));
+  TRY(alloc((void **)&ATT, terms_bytes(D)));
+  TRY(alloc((void **)&Hb, gpt2 ? terms_bytes(F) : sizeof(float) * (s >= 64 ? s32 : (size_t)s) * HW));
+  if (!gpt2) TRY(alloc((void **)&G, terms_bytes(F)));
   if (d->kvq || d->kvp) {
     TRY(alloc((void **)&KF, sizeof(float) * (size_t)(n + s) * KD));
     TRY(alloc((void **)&VF, sizeof(float) * (size_t)(n + s) * KD));
@@ -970,7 +981,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     // workgroups per tile leaves partial tiles; what follows it is the residual add and the next norm, so one pass
     // over the rows does all three (launch_reduce_norm) instead of a reduction launch and a norm launch.
     // Many rows: a Linear takes its input as two bf16 terms (gemm_planes.hip), or over 4-bit weights as digits (gemm_digits.hip), and what produces that
-    // input writes it so; a row of terms is as long as the fp32 row whose buffer it takes, one of digits no longer.
+    // input writes it so; a row of terms is as long as the fp32 row whose buffer it takes.
     // (Sessions with a quantised cache stay with the tiles: other sums put other quants into the cache, and with them logits a token later move by 1.4e-3 and tokens change, 1 of 8
     // of the 7B shape behind 203 rows.  It would be faster: Q4_0, 1.1B shape, 300 rows 3.40 -> 2.52 ms, 1900 rows 16.9 -> 8.5.  Fewer rows go through the same launches in every
     // session.  The one order of summation that is kept for their sake, at no cost that was found, is that of quantised tiles: tile_plan.)
@@ -978,7 +989,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     auto in_planes = [&](const WMat *w) -> int {
       if (!planes || !w) return kTermsNone;
       const int terms = linear_terms(w, prec);
-      if ((terms == kTermsDigits && !rows_digits_supported(D)) || !linear_planes_ready(w, R, prec)) return kTermsNone;
+      if ((terms == kTermsDigits && (!digits || !rows_digits_supported(D))) || !linear_planes_ready(w, R, prec)) return kTermsNone;
       held.push_back(w);
       return terms;
     };

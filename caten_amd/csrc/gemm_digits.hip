@@ -5,7 +5,8 @@
 // multiplies them at four times the rate, K = 64 holding two digits of a block against the same weights twice, and applies the powers of two itself: two instructions
 // of 38 cycles per block, 96 bytes per row and block instead of 128, 24 per column instead of 64.  The block's scale is one multiply-add per result, as there.
 // What is lost: 2^-19 of a block's largest value, where two bf16 terms lose 2^-18 of each value.  Measured against 64 bits over rows of normal values 1.03e-6 (two terms:
-// 2.46e-6), with every 37th column 100 times as large 2.1e-6 (2.3e-6), values of wide range, exp(2 x), 2.2 - 2.35e-6 (2.1 - 2.4e-6).
+// 2.46e-6), with every 37th column 100 times as large 2.1e-6 (2.3e-6), values of wide range, exp(2 x), 2.2 - 2.35e-6 (2.1 - 2.4e-6).  Results that the largest values do not reach would
+// lose more: blocks with values far above the others have what three digits leave as two bf16 terms besides (digits.h: which, and what that leaves of the loss).
 //
 // us, operands in place / planes: 1900 x 11264 x 2048 134 / 194, 1900 x 2048 x 5632 71 / 117, 1900 x 2560 x 2048 38 / 70; prompt of 1900 rows, 1.1B shape, 10.9 -> 7.7 ms, of 300, 7B shape,
 // 16.2 -> 8.7.  What bounds it: large products the power limit (a card at 1.5 - 1.8 GHz there; a step of two workgroups of 128 x 256 was 2550 cycles, of which the matrix
@@ -94,6 +95,9 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
 
   v16f tmp[2] = {};  // sums over a block of 32 k, unscaled
   float dlast = 0.0f;
+  unsigned least[MB];  // of this lane's pairs of exponents: below 256 where the upper one is 0
+#pragma unroll
+  for (int i = 0; i < MB; i++) least[i] = 0xffffu;
   // both: the step has all of its KB blocks (an odd number of blocks: the last one's second half counts for nothing)
   auto mul = [&](int buf, bool both) __attribute__((always_inline)) {
     uint4 a16[KB][MB][2], b16[KB][NB];
@@ -126,6 +130,8 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
       for (int i = 1; i < MB; i++) lda(i);
 #pragma unroll
       for (int b = 1; b < NB; b++) ldb(b);
+#pragma unroll
+      for (int i = 0; i < MB; i++) least[i] = min(least[i], (unsigned)sc[k][i]);
     }
     if (KB == 1) issue((buf + NBUF - 1) % NBUF);  // while they are on their way
     __builtin_amdgcn_sched_barrier(0);
@@ -175,6 +181,65 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[MB - 1][NB - 1][r] = fmaf(dlast, even ? tmp[0][r] : tmp[1][r], acc[MB - 1][NB - 1][r]);
 
+  // ---- what three digits left of blocks that have it as terms (digits.h), of this wavefront's own rows.  Rare: one look at a wavefront's exponents, and where one is 0 all of the
+  // share's again, 32 blocks of k at a time; a block is the four instructions of two bf16 terms against the same weights, its loads waited for.  (us with the pass that makes the
+  // digits, no such block / a column of all of K / every block: 1900 x 11264 x 2048 147 / 164 / 490, 1900 x 2048 x 5632 92 / 97 / 285, 280 x 12288 x 4096 62 / 64 / 186; two bf16 terms in
+  // place, without their pass: 194 and 117 for the first two.)
+#pragma unroll
+  for (int i = 0; i < MB; i++) {
+    const int group = min(m0 / 32 + MB * wm + i, mg - 1);  // (past the end: not this wavefront's)
+    const bool mine = m0 + 32 * (MB * wm + i) + col < a.M;
+    if (!__any(mine && least[i] < 256u)) continue;
+    const unsigned char *words = a.A + (int64_t)mg * nkb * kDigitRecord + ((int64_t)k0 * mg + group) * 128;
+    const unsigned char *rests = a.A + (int64_t)mg * nkb * (kDigitRecord + kDigitScales) + ((int64_t)group * nkb + k0) * kDigitRests + lane * 16;
+    const unsigned upper = half ? ~0u : 0u;
+    const int rows = a.M - 32 * group - 4 * (lane & 7);  // of the four whose exponents this lane looks at
+#pragma unroll 1
+    for (int c = 0; c < nsteps; c += 32) {
+      unsigned any = 0;
+      uint4 word[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) word[u] = *(const uint4 *)(words + (int64_t)min(c + 8 * u + (lane >> 3), nsteps - 1) * mg * 128 + (lane & 7) * 16);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const bool has = ((word[u].x < 0x1000000u) & (rows > 0)) | ((word[u].y < 0x1000000u) & (rows > 1)) | ((word[u].z < 0x1000000u) & (rows > 2)) | ((word[u].w < 0x1000000u) & (rows > 3));
+        uint64_t t = __ballot(has & (c + 8 * u + (lane >> 3) < nsteps));  // eight lanes to a block of k
+        t |= t >> 4, t |= t >> 2, t |= t >> 1;
+        any |= (unsigned)((t & 0x0101010101010101ull) * 0x0102040810204080ull >> 56) << (8 * u);
+      }
+#pragma unroll 1
+      while (any) {
+        const int kb = c + __builtin_ctz(any);
+        any &= any - 1;
+        const unsigned has = mine & (*(const unsigned *)(words + (int64_t)kb * mg * 128 + col * 4) < 0x1000000u) ? ~0u : 0u;  // (else nothing was written there)
+        const uint4 *r = (const uint4 *)(rests + (int64_t)kb * kDigitRests);
+        uint4 t[4] = {r[128], r[192], r[0], r[64]};  // the small term first
+#pragma unroll
+        for (int q = 0; q < 4; q++) t[q].x &= has, t[q].y &= has, t[q].z &= has, t[q].w &= has;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+          const unsigned char *w = a.B + ((int64_t)min(n0 / 32 + NB * wn + b, ng - 1) * nkb + k0 + kb) * kDigitWRecord;
+          const uint4 w16 = *(const uint4 *)(w + col * 16);
+          const uint2 w8 = *(const uint2 *)(w + 512 + col * 8);
+          const float dw = *(const float *)(w + 768 + col * 4);
+          const v6u_dg six = {w16.x, w16.y, w16.z, w16.w, w8.x, w8.y};
+          const auto all = __builtin_bit_cast(v16u_dg, __builtin_amdgcn_cvt_scalef32_pk32_bf16_fp6(six, 1.0f));
+          unsigned mid[8];  // k 16 half .. + 15  (not a choice of two elements, which is made one of sixteen)
+#pragma unroll
+          for (int e = 0; e < 8; e++) mid[e] = all[e] ^ ((all[e] ^ all[8 + e]) & upper);
+          const uint4 k8[2] = {make_uint4(mid[0], mid[1], mid[2], mid[3]), make_uint4(mid[4], mid[5], mid[6], mid[7])};
+          v16f p;
+#pragma unroll
+          for (int e = 0; e < 16; e++) p[e] = 0.0f;
+#pragma unroll
+          for (int q = 0; q < 4; q++) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, t[q]), __builtin_bit_cast(v8bf, k8[q & 1]), p, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[i][b][e] = fmaf(dw, p[e], acc[i][b][e]);
+        }
+      }
+    }
+  }
+
   // ---- acc[i][b][r] is row 8 (r / 4) + 4 half + r % 4, column `col` of its block.  A wavefront turns its blocks around in a piece of LDS of its own
   // (no barrier) and stores rows of 32 NB columns, 16 bytes per lane, or a block of 32 columns of a row per lane as digits.
   // (Small code: a launch of a few steps waits for its own instructions.)
@@ -195,7 +260,7 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
 #pragma unroll 1
       for (int u = lane; u < 32 * NB / PER; u += 64) {
         const int c = (u >> 5) * 32 * PER, row = row0 + col;
-        if (row >= store.M || col0 + c >= store.N) continue;
+        if (col0 + c >= store.N) continue;  // (the same for a block's 32 lanes)
         const float *p = Cs + col * LDC + c;
         float v[32];
 #pragma unroll
@@ -208,7 +273,9 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
 #pragma unroll
           for (int q = 0; q < 32; q++) v[q] = ct_gelu(v[q]);
         }
-        store_digits32(digits, (int64_t)mg * 32, store.pkb, row, (col0 + c) / (32 * PER), v);
+        const float m = digits_top(v);
+        const bool rest = digits_uneven_columns(v, m, row < store.M) || digits_one_large(v, m);
+        if (row < store.M) store_digits32(digits, (int64_t)mg * 32, store.pkb, row, (col0 + c) / (32 * PER), v, m, rest);
       }
     } else if constexpr (OUT == kDigitsPlain) {
       plane_gemm_store_rows<NB>(store, Cs, row0, col0, lane, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
@@ -270,10 +337,36 @@ int make_weight_digits(unsigned char *out, const WMat *w) {
   return 0;
 }
 
-// ---- rows -> digits, with the norm that a Linear has in front ----
-// Four rows to a workgroup, a wavefront per row while it is normalised (V4 float4 per lane), then 64 blocks of the four rows at a time through LDS, so that neighbouring
-// lanes hold the same block of neighbouring rows, whose 16-byte pieces of a digit lie side by side.  (A row's blocks in its own wavefront's lanes, 16 bytes
-// stored every 3072: 1900 rows of 2048 13.4 us.)
+// ---- rows -> digits ----
+// A workgroup takes eight blocks of 32 rows, a block of a row per thread, through LDS: a wavefront reads 1024 bytes of a row at a time, and neighbouring lanes hold the same block of
+// neighbouring rows, whose 16-byte pieces of a digit lie side by side.
+__global__ __launch_bounds__(256) void k_digits_rows(unsigned char *__restrict__ out, const float *__restrict__ x, int64_t rows, int K) {
+  constexpr int PITCH = 36, BLOCK = 32 * PITCH + 32;  // floats between rows and blocks: no two of the 16 lanes of a 16-byte access meet in a bank
+  __shared__ __align__(16) float turn[8 * BLOCK];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nkb = K >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * 32;
+  const int kb0 = blockIdx.y * 8, at = min(kb0 * 32 + 4 * lane, K - 4);
+  float4 v4[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) v4[j] = *(const float4 *)(x + min(row0 + wave + 4 * j, rows - 1) * K + at);
+#pragma unroll
+  for (int j = 0; j < 8; j++) *(float4 *)&turn[(lane >> 3) * BLOCK + (wave + 4 * j) * PITCH + 4 * (lane & 7)] = v4[j];
+  __syncthreads();
+  const int r = tid & 31, kb = kb0 + (tid >> 5);
+  if (kb >= nkb) return;  // (the same for a block's 32 lanes)
+  float v[32];
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const float4 f = *(const float4 *)&turn[(tid >> 5) * BLOCK + r * PITCH + 4 * q];
+    v[4 * q] = f.x, v[4 * q + 1] = f.y, v[4 * q + 2] = f.z, v[4 * q + 3] = f.w;
+  }
+  const float m = digits_top(v);
+  const bool rest = digits_uneven_columns(v, m, row0 + r < rows) || digits_one_large(v, m);
+  if (row0 + r < rows) store_digits32(out, (rows + 31) / 32 * 32, nkb, row0 + r, kb, v, m, rest);
+}
+
+// The same behind a norm, a wavefront per row (V4 float4 per lane) while it is normalised, four rows to a workgroup; then 64 blocks of the four rows at a time through LDS.
+// (A row's blocks in its own wavefront's lanes, 16 bytes stored every 3072: 1900 rows of 2048 13.4 us.)
 template <int PRO, int V4>
 __global__ __launch_bounds__(256) void k_rows_digits(unsigned char *__restrict__ out, const float *__restrict__ x, int64_t rows, int K, const float *__restrict__ g,
                                                      const float *__restrict__ b, float eps) {
@@ -281,58 +374,53 @@ __global__ __launch_bounds__(256) void k_rows_digits(unsigned char *__restrict__
   __shared__ __align__(16) float turn[4 * RS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n4 = K >> 2, nkb = K >> 5;
   const int64_t row0 = (int64_t)blockIdx.x * 4;
-  constexpr bool NORM = PRO != CTHIP_PRO_NONE;
   const float4 *xr = (const float4 *)(x + min(row0 + wave, rows - 1) * K);
   const int crow = threadIdx.x & 3, cblk = threadIdx.x >> 2;  // what this thread converts
-  // (a row without a norm may be longer than the registers: piece by piece)
-  for (int at = 0; at < n4; at += 64 * V4) {
-    float4 v[V4], gm[NORM ? V4 : 1], bt[PRO == CTHIP_PRO_LAYERNORM ? V4 : 1];
+  float4 v[V4], gm[V4], bt[PRO == CTHIP_PRO_LAYERNORM ? V4 : 1];
 #pragma unroll
-    for (int j = 0; j < V4; j++) v[j] = xr[min(at + lane + 64 * j, n4 - 1)];
-    if (NORM) {
+  for (int j = 0; j < V4; j++) v[j] = xr[min(lane + 64 * j, n4 - 1)];
 #pragma unroll
-      for (int j = 0; j < V4; j++) {
-        gm[j] = ((const float4 *)(g ? g : x))[min(lane + 64 * j, n4 - 1)];
-        if (PRO == CTHIP_PRO_LAYERNORM) bt[j] = ((const float4 *)(b ? b : x))[min(lane + 64 * j, n4 - 1)];
+  for (int j = 0; j < V4; j++) {
+    gm[j] = ((const float4 *)(g ? g : x))[min(lane + 64 * j, n4 - 1)];
+    if (PRO == CTHIP_PRO_LAYERNORM) bt[j] = ((const float4 *)(b ? b : x))[min(lane + 64 * j, n4 - 1)];
+  }
+  const float inv_n = 1.0f / (float)K;
+  float mean = 0.0f, q = 0.0f;
+  if (PRO == CTHIP_PRO_LAYERNORM) {
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < V4; j++) s += lane + 64 * j < n4 ? (v[j].x + v[j].y) + (v[j].z + v[j].w) : 0.0f;
+    mean = wave_sum(s) * inv_n;
+  }
+#pragma unroll
+  for (int j = 0; j < V4; j++) {
+    v[j].x -= mean, v[j].y -= mean, v[j].z -= mean, v[j].w -= mean;
+    q += lane + 64 * j < n4 ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.0f;
+  }
+  const float rstd = 1.0f / sqrtf(wave_sum(q) * inv_n + eps);
+#pragma unroll
+  for (int j = 0; j < V4; j++) {
+    v[j].x *= rstd, v[j].y *= rstd, v[j].z *= rstd, v[j].w *= rstd;
+    if (g) v[j].x *= gm[j].x, v[j].y *= gm[j].y, v[j].z *= gm[j].z, v[j].w *= gm[j].w;
+    if (PRO == CTHIP_PRO_LAYERNORM && b) v[j].x += bt[j].x, v[j].y += bt[j].y, v[j].z += bt[j].z, v[j].w += bt[j].w;
+  }
+#pragma unroll
+  for (int c = 0; c < V4; c += 8) {
+    const int kb0 = 8 * c;
+    if (kb0 >= nkb) break;
+    if (c) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 8 && j < V4; j++) *(float4 *)&turn[wave * RS + (lane / 8 + 8 * j) * 36 + 4 * (lane % 8)] = make_float4(v[c + j].x, v[c + j].y, v[c + j].z, v[c + j].w);
+    __syncthreads();
+    if (kb0 + cblk < nkb && cblk < 8 * V4 && row0 + crow < rows) {
+      float t[32];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float4 f = *(const float4 *)&turn[crow * RS + cblk * 36 + 4 * i];
+        t[4 * i] = f.x, t[4 * i + 1] = f.y, t[4 * i + 2] = f.z, t[4 * i + 3] = f.w;
       }
-      const float inv_n = 1.0f / (float)K;
-      float mean = 0.0f, q = 0.0f;
-      if (PRO == CTHIP_PRO_LAYERNORM) {
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < V4; j++) s += lane + 64 * j < n4 ? (v[j].x + v[j].y) + (v[j].z + v[j].w) : 0.0f;
-        mean = wave_sum(s) * inv_n;
-      }
-#pragma unroll
-      for (int j = 0; j < V4; j++) {
-        v[j].x -= mean, v[j].y -= mean, v[j].z -= mean, v[j].w -= mean;
-        q += lane + 64 * j < n4 ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.0f;
-      }
-      const float rstd = 1.0f / sqrtf(wave_sum(q) * inv_n + eps);
-#pragma unroll
-      for (int j = 0; j < V4; j++) {
-        v[j].x *= rstd, v[j].y *= rstd, v[j].z *= rstd, v[j].w *= rstd;
-        if (g) v[j].x *= gm[j].x, v[j].y *= gm[j].y, v[j].z *= gm[j].z, v[j].w *= gm[j].w;
-        if (PRO == CTHIP_PRO_LAYERNORM && b) v[j].x += bt[j].x, v[j].y += bt[j].y, v[j].z += bt[j].z, v[j].w += bt[j].w;
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < V4; c += 8) {
-      const int kb0 = (at + 64 * c) >> 3;
-      if (kb0 >= nkb) break;
-      if (at || c) __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 8 && j < V4; j++) *(float4 *)&turn[wave * RS + (lane / 8 + 8 * j) * 36 + 4 * (lane % 8)] = make_float4(v[c + j].x, v[c + j].y, v[c + j].z, v[c + j].w);
-      __syncthreads();
-      if (kb0 + cblk < nkb && cblk < 8 * V4 && row0 + crow < rows) {
-        float t[32];
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-          const float4 f = *(const float4 *)&turn[crow * RS + cblk * 36 + 4 * q];
-          t[4 * q] = f.x, t[4 * q + 1] = f.y, t[4 * q + 2] = f.z, t[4 * q + 3] = f.w;
-        }
-        store_digits32(out, (rows + 31) / 32 * 32, nkb, row0 + crow, kb0 + cblk, t);
-      }
+      const float m = digits_top(t);
+      store_digits32(out, (rows + 31) / 32 * 32, nkb, row0 + crow, kb0 + cblk, t, m, digits_uneven(t, m) || digits_one_large(t, m));
     }
   }
 }
@@ -350,7 +438,7 @@ int launch_rows_digits(void *digits, const float *x, int m, int K, int pro, cons
   } while (0)
   if (pro == CTHIP_PRO_LAYERNORM) RDN(CTHIP_PRO_LAYERNORM);
   else if (pro == CTHIP_PRO_RMSNORM) RDN(CTHIP_PRO_RMSNORM);
-  else RD(CTHIP_PRO_NONE, 8);
+  else hipLaunchKernelGGL(k_digits_rows, dim3((m + 31) / 32, (K / 32 + 7) / 8), dim3(256), 0, state().stream, (unsigned char *)digits, x, (int64_t)m, K);
 #undef RDN
 #undef RD
   CTHIP_LAUNCH_CHECK();

@@ -295,7 +295,8 @@ __global__ __launch_bounds__(256) void k_reduce_norm_wide(ReduceNormArgs a) {
         const float4 u = *(const float4 *)&turn[tid * 36 + 4 * q];
         f[4 * q] = u.x, f[4 * q + 1] = u.y, f[4 * q + 2] = u.z, f[4 * q + 3] = u.w;
       }
-      store_digits32(a.digits, (a.rows + 31) / 32 * 32, n >> 5, row, tid, f);
+      const float m = digits_top(f);
+      store_digits32(a.digits, (a.rows + 31) / 32 * 32, n >> 5, row, tid, f, m, digits_uneven(f, m) || digits_one_large(f, m));
     }
   }
 }
@@ -1779,14 +1780,16 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma_bf(float *__restrict__ ou
     }
     __syncthreads();
     const int row = tid & 31, b = tid >> 5;
-    if (b < DB && i0 + row < S) {
+    if (b < DB) {  // (the same for a block's 32 lanes)
       float v[32];
 #pragma unroll
       for (int q4 = 0; q4 < 8; q4++) {
         const float4 t = *(const float4 *)&Qs[row][32 * b + 4 * q4];
         v[4 * q4] = t.x, v[4 * q4 + 1] = t.y, v[4 * q4 + 2] = t.z, v[4 * q4 + 3] = t.w;
       }
-      store_digits32(digits, (int64_t)(S + 31) / 32 * 32, H * DH / 32, i0 + row, (h * DH >> 5) + b, v);
+      const float m = digits_top(v);
+      const bool rest = digits_uneven_columns(v, m, i0 + row < S) || digits_one_large(v, m);
+      if (i0 + row < S) store_digits32(digits, (int64_t)(S + 31) / 32 * 32, H * DH / 32, i0 + row, (h * DH >> 5) + b, v, m, rest);
     }
   } else if (i0 + col < S) {
     float *orow = out + ((int64_t)(i0 + col) * H + h) * DH;

@@ -1,5 +1,5 @@
 """Linears over many rows on 4-bit weights, whose operands lie as 6-bit digits (csrc/gemm_digits.hip): every tile, with one share of K and several, at edges that
-no tile divides and odd numbers of blocks; rows of any magnitude and rows that are not finite; prompts, whose norms, attention and GELU / SwiGLU write digits."""
+no tile divides and odd numbers of blocks; rows of any magnitude and rows that are not finite; prompts, whose norms, attention and GELU / SwiGLU write digits; values that are small beside others of their block."""
 import numpy as np
 import pytest
 
@@ -93,4 +93,94 @@ def test_prompt_equals_short_pieces(ops, arch, kinds, rows):
     for (t0, l0), (t1, l1) in zip(got, want):
         assert t0 == t1
         assert np.linalg.norm(l0 - l1) < 1e-4 * np.linalg.norm(l1)
+    model.close()
+
+
+def terms_bound(x, w):
+    """What two bf16 terms of every value leave: 2^-18 of each, and fp32 sums as in bound(); values whose terms end below 2^-126, where the matrix cores have zero."""
+    return (2.0 ** -18 + (x.shape[1] / 32 + 32) * 2.0 ** -24) * (np.abs(x) @ np.abs(w).T) + 2.0 ** -124 * np.abs(w).sum(-1)
+
+
+# columns of a block of 32 that are larger, by how much, in which rows; 2^18 (digits of a small value all zero) and what a model's own largest channels are
+@pytest.mark.parametrize("cols_large,factor,rows_large", [(1, 1e3, "all"), (4, 700.0, "all"), (16, 1e3, "all"), (24, 2.0 ** 18, "all"), (31, 2.0 ** 16, "all"), (1, 1e3, "one"), (1, 2.0 ** 26, "few"), (0, 1.0, "wide")])
+@pytest.mark.parametrize("rows,cols,m", [(3001, 288, 577), (2051, 4128, 129), (4100, 1056, 65), (9001, 544, 1537)])
+def test_results_that_the_large_values_do_not_reach(ops, rows, cols, m, cols_large, factor, rows_large):
+    """Weights of zero at the large columns: the results are sums of small values alone, and as near as two terms of every value make them.  "wide": values of exp(6 x)."""
+    from caten_amd.llm import Tensor
+    print(f"case: {rows} x {cols}, {m} rows, {cols_large} columns of 32, {factor}, {rows_large}", flush=True)
+    rng = np.random.default_rng(rows + cols_large)
+    a = rng.normal(0, 0.05, (rows, cols)).astype(np.float32)
+    large = np.zeros(cols, bool)
+    for b in range(cols // 32):
+        large[32 * b + rng.permutation(32)[:cols_large]] = True
+    a[:, large] = 0.0
+    w = ops.WeightMatrix("q4_0", Tensor.from_f32(a, "q4_0").raw, rows, cols)
+    x = rng.uniform(0.5, 1.0, (m, cols)) * rng.choice([-1.0, 1.0], (m, cols))
+    at_rows = np.ones(m, bool) if rows_large == "all" else np.arange(m) % 32 == 5 if rows_large == "one" else np.arange(m) % 7 == 3
+    x[np.ix_(at_rows, large)] *= factor
+    if rows_large == "wide":
+        x = np.exp(6.0 * rng.normal(0, 1, (m, cols))) * np.sign(x)
+        x[:, ::2] = 0.0
+    x = x.astype(np.float32)
+    at, rs = np.unique(np.r_[0:20, rows - 20:rows, rng.integers(0, rows, 40)]), np.unique(np.r_[0:9, m - 9:m, rng.integers(0, m, 60), np.flatnonzero(at_rows)[:9]])
+    x64, w64 = x[rs].astype(np.float64), w.dequantize()[at].astype(np.float64)
+    assert not w64[:, large].any()
+    got = ops.linear(x, w)[np.ix_(rs, at)]
+    most = terms_bound(x64, w64) if rows_large != "wide" else bound(x64, w64)
+    assert np.all(np.abs(got - x64 @ w64.T) <= most)
+    if rows_large == "wide":  # blocks that have no terms lose less than twice what those that have them keep
+        assert np.linalg.norm((got - x64 @ w64.T) / (np.abs(x64) @ np.abs(w64).T)) <= 2.0 * 2.0 ** -18 * np.sqrt(got.size)
+    w.free()
+
+
+def test_rows_of_the_smallest_magnitudes(ops):
+    """Below 2^-110 a digit's power of two would end past the smallest: what is left goes as terms."""
+    rng = np.random.default_rng(8)
+    w = weights(ops, 4100, 1056, rng)
+    w64 = w.dequantize().astype(np.float64)
+    x = rng.normal(0, 1, (129, 1056)) * np.array([1e-32, 1e-33, 1e-34, 1e-35, 1e-36, 1e-37, 1.0])[np.arange(129) % 7][:, None]
+    x = x.astype(np.float32)
+    x64 = x.astype(np.float64)
+    got = ops.linear(x, w)
+    assert np.all(np.abs(got - x64 @ w64.T) <= np.maximum(bound(x64, w64), terms_bound(x64, w64)))
+    w.free()
+
+
+@pytest.mark.parametrize("arch,rows", [("gpt2", 97), ("gpt2", 700), ("llama", 96), ("llama", 1300)])
+def test_prompt_with_large_channels(arch, rows):
+    """A model whose norms, attention and MLP each have a few channels a thousand times as large that the Linears behind do not read (weights of zero there): what norms, attention and the
+    GELU / SwiGLU launches write carries the others as well as pieces of 63 rows do, whose inputs are two terms or fp32."""
+    print(f"case: {arch}, {rows} rows", flush=True)
+    from caten_amd import llm, synth
+    cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=1024, n_heads=16, n_kv_heads=4, ffn=2816) if arch == "llama" else dict(synth.GPT2_CONFIGS["gpt2"], dim=1024, n_heads=16)
+    cfg.update(n_layers=3, vocab=500, max_seq=2048)
+    w = (synth.llama_weights if arch == "llama" else synth.gpt2_weights)(cfg, seed=3)
+    rng = np.random.default_rng(1)
+    D, F, H, HK = cfg["dim"], cfg["ffn"], cfg["n_heads"], cfg.get("n_kv_heads", cfg["n_heads"])
+    Dh = D // H
+    pick = lambda n: np.arange(0, n, 32) + rng.integers(0, 32, n // 32)  # noqa: E731  (one of every 32)
+    ch, ff, vh = pick(D), pick(F), pick(HK * Dh)
+    oh = np.concatenate([h * Dh + vh[vh // Dh == h // (H // HK)] % Dh for h in range(H)])  # where the attention's result has them
+    keys = dict(n1="attn_norm", n2="ffn_norm", qkv=("wq", "wk", "wv"), v="wv", o="wo", fc=("w_gate", "w_up"), up="w_up", down="w_down") if arch == "llama" else \
+        dict(n1="ln1_g", n2="ln2_g", qkv=("attn_w",), v="attn_w", o="proj_w", fc=("fc_w",), up="fc_w", down="fc2_w")
+    for l in range(3):
+        for norm, behind in ((keys["n1"], keys["qkv"]), (keys["n2"], keys["fc"])):
+            w[norm][l][ch] *= 1000.0
+            for k in behind:
+                w[k][l][:, ch] = 0.0
+        w[keys["v"]][l][(0 if arch == "llama" else 2 * D) + vh] *= 1000.0
+        w[keys["o"]][l][:, oh] = 0.0
+        w[keys["up"]][l][ff] *= 1000.0
+        w[keys["down"]][l][:, ff] = 0.0
+    sd = (llm.llama_state_dict if arch == "llama" else llm.gpt2_state_dict)(w, "q4_0")
+    make = llm.make_llama if arch == "llama" else llm.make_gpt2
+    model = make(cfg, sd)
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], rows + 1, seed=3)]
+    got = [model.forward(ids[:rows], rows, 0, return_logits=True), model.forward(ids[rows:], 1, rows, return_logits=True)]
+    for n in range(0, rows, 63):
+        want = [model.forward(ids[n:min(n + 63, rows)], min(63, rows - n), n, return_logits=True)]
+    want.append(model.forward(ids[rows:], 1, rows, return_logits=True))
+    # the last row's single-row Linears, which take nibbles times inputs less eight times the inputs' sum, are off by up to 1e-4 of these logits on either side
+    for (t0, l0), (t1, l1) in zip(got, want):
+        assert np.linalg.norm(l0 - l1) < 2e-4 * np.linalg.norm(l1)
     model.close()
