@@ -95,11 +95,12 @@ struct WMat {
   // valid for exactly these gamma / beta / bias vectors
   const float *fold_g = nullptr, *fold_b = nullptr, *fold_bias = nullptr;
   float *fold_s = nullptr, *fold_c = nullptr;
-  // the matrix as bf16 terms, made by the first Linear over many rows that wants them (gemm_planes.hip), or as digits (gemm_digits.hip)
-  void *planes = nullptr;
-  int planes_terms = 0;  // how many terms, kDigits
-  int64_t planes_bytes = 0;
-  int planes_users = 0;  // launches being put together from them; they are not given back meanwhile
+  // the matrix as bf16 terms (gemm_planes.hip) and as digits (gemm_digits.hip), each made by the first Linear over many rows that wants it
+  struct Form {
+    void *p = nullptr;
+    int64_t bytes = 0;
+    int users = 0;  // launches being put together from it; it is not given back meanwhile
+  } forms[2];
 };
 // gfx950: 256 MB of Infinity Cache in front of HBM
 static const int64_t kInfinityCacheBytes = 256ll << 20;
@@ -290,10 +291,10 @@ bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: 
 bool linear_few_shares_pays(const WMat *w, int m, int precision);  // rows as they are, shares of K left to the norm behind (any number of columns)
 int launch_linear_few_shares(float *y, const WMat *w, const float *x, int m, const float *bias, const float *residual, GemmDeferred *defer);
 int launch_linear_few(float *y, const WMat *w, const void *operands, int m, const float *bias, const float *residual, int act, const GemmRoute *route);
-// x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release
+// x in planes certainly runs: the matrix has its terms (made here if need be), held until weight_planes_release at the same precision
 bool linear_planes_ready(const WMat *w, int m, int precision);
 int linear_terms(const WMat *w, int precision);  // kTermsPlanes or kTermsDigits
-void weight_planes_release(const WMat *w);
+void weight_planes_release(const WMat *w, int precision);
 // The terms of all matrices together are kept up to this many bytes.  They are given back where memory is short, by
 // cthip_cache_trim and by a lower limit; weight_planes_drop returns whether there were any.
 void weight_planes_limit(int64_t bytes);

@@ -1006,7 +1006,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
     };
     auto no_planes = [&](const WMat *w) {
       held.erase(std::find(held.begin(), held.end(), w));
-      weight_planes_release(w);
+      weight_planes_release(w, prec);
     };
     // y = norm(x), as terms where the Linear behind it takes them
     auto norm = [&](float *y, const float *x, const float *g, const float *b, int terms) {
@@ -1124,7 +1124,7 @@ static int prefill(Decoder *d, const int *ids, int s, int n) {
   TRY(queue_head(d));
 #undef TRY
 done:
-  for (const WMat *w : held) weight_planes_release(w);
+  for (const WMat *w : held) weight_planes_release(w, prec);
   for (void *p : tmp) cthip_free(p);
   return rc;
 }

@@ -513,27 +513,39 @@ static int make_weight_planes(unsigned char *out, const WMat *w, int terms_b) {
   CTHIP_LAUNCH_CHECK();
   return 0;
 }
+// A matrix of 4 bits is held in both of its forms where both are asked for (one term in bf16, two as digits); where there is room for one alone, the one that nobody uses goes.
+static WMat::Form &form_of(const WMat *w, int terms_b) { return const_cast<WMat *>(w)->forms[terms_b == kDigits]; }
+static int64_t form_spare(const WMat *w, int terms_b) {  // (with g_planes_mu held) bytes of the other form that can go
+  const WMat::Form &o = w->forms[terms_b != kDigits];
+  return o.p && !o.users ? o.bytes : 0;
+}
 // Whether they are there or the next call's stay (with g_planes_mu held)
 static bool weight_planes_room(const WMat *w, int terms_b) {
-  return weight_planes_stay(w, terms_b) && (w->planes ? w->planes_terms == terms_b : g_planes_bytes + weight_plane_bytes(w, terms_b) <= g_planes_limit);
+  return weight_planes_stay(w, terms_b) && (form_of(w, terms_b).p || g_planes_bytes - form_spare(w, terms_b) + weight_plane_bytes(w, terms_b) <= g_planes_limit);
 }
 static bool weight_planes_kept(const WMat *w, int terms_b) {
   std::lock_guard<std::mutex> lk(g_planes_mu);
   return weight_planes_room(w, terms_b);
 }
+static void form_give_back(WMat::Form &f) {  // (stream-ordered: the block goes to later work on this stream only)
+  cthip_free(f.p);
+  g_planes_bytes -= f.bytes;
+  f = {};
+}
 // The terms for one launch, null where there is no memory for them (or for terms that stay, where temp is null).  *temp:
 // the caller frees them after its launch, else it calls weight_planes_release.
 static const unsigned char *weight_planes(const WMat *w, int terms_b, bool *temp) {
   std::lock_guard<std::mutex> lk(g_planes_mu);
-  WMat *m = const_cast<WMat *>(w);
+  WMat::Form &f = form_of(w, terms_b);
   const int64_t bytes = weight_plane_bytes(w, terms_b);
   const bool stay = weight_planes_room(w, terms_b);
-  if (stay && w->planes) {
-    m->planes_users++;
+  if (stay && f.p) {
+    f.users++;
     if (temp) *temp = false;
-    return (const unsigned char *)w->planes;
+    return (const unsigned char *)f.p;
   }
   if (!stay && !temp) return nullptr;
+  if (stay && g_planes_bytes + bytes > g_planes_limit) form_give_back(const_cast<WMat *>(w)->forms[terms_b != kDigits]);
   unsigned char *p = nullptr;
   if (alloc_spare((void **)&p, (size_t)bytes)) return nullptr;
   if (make_weight_planes(p, w, terms_b)) {
@@ -541,42 +553,35 @@ static const unsigned char *weight_planes(const WMat *w, int terms_b, bool *temp
     return nullptr;
   }
   if (stay) {
-    m->planes = p;
-    m->planes_terms = terms_b;
-    m->planes_bytes = bytes;
-    m->planes_users = 1;
+    f.p = p;
+    f.bytes = bytes;
+    f.users = 1;
     g_planes_bytes += bytes;
-    g_planes_of.insert(m);
+    g_planes_of.insert(const_cast<WMat *>(w));
   }
   if (temp) *temp = !stay;
   return p;
 }
-void weight_planes_release(const WMat *w) {
+void weight_planes_release(const WMat *w, int precision) {
   std::lock_guard<std::mutex> lk(g_planes_mu);
-  const_cast<WMat *>(w)->planes_users--;
-}
-static void planes_give_back(WMat *w) {  // (stream-ordered: the block goes to later work on this stream only)
-  cthip_free(w->planes);
-  g_planes_bytes -= w->planes_bytes;
-  w->planes = nullptr;
+  form_of(w, weight_terms(w, plane_terms(precision))).users--;
 }
 void wmat_drop_planes(WMat *w) {
   std::lock_guard<std::mutex> lk(g_planes_mu);
-  if (!w->planes) return;
-  planes_give_back(w);
+  for (WMat::Form &f : w->forms)
+    if (f.p) form_give_back(f);
   g_planes_of.erase(w);
 }
 bool weight_planes_drop() {
   std::lock_guard<std::mutex> lk(g_planes_mu);
   bool any = false;
   for (auto it = g_planes_of.begin(); it != g_planes_of.end();) {
-    if ((*it)->planes_users) {
-      ++it;
-      continue;
+    bool left = false;
+    for (WMat::Form &f : (*it)->forms) {
+      if (f.p && !f.users) form_give_back(f), any = true;
+      left = left || f.p;
     }
-    planes_give_back(*it);
-    it = g_planes_of.erase(it);
-    any = true;
+    it = left ? std::next(it) : g_planes_of.erase(it);
   }
   return any;
 }
@@ -676,7 +681,7 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
   }
   cthip_free(tmp);  // stream-ordered: handed out again only to later work on this stream
   if (temp_b) cthip_free(const_cast<unsigned char *>(pb));
-  else weight_planes_release(w);
+  else weight_planes_release(w, precision);
   return rc;
 }
 

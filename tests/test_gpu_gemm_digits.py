@@ -184,3 +184,40 @@ def test_prompt_with_large_channels(arch, rows):
     for (t0, l0), (t1, l1) in zip(got, want):
         assert np.linalg.norm(l0 - l1) < 2e-4 * np.linalg.norm(l1)
     model.close()
+
+
+def test_both_forms_of_a_matrix_are_kept(ops):
+    """A 4-bit matrix is integers in bf16 to Linears at one term and digits at two: each form is made once and stays; with room for one of them alone, the one in use takes the other's."""
+    import ctypes as C
+    from caten_amd import _lib
+    lib = _lib.init(0)
+    rows, cols = 5001, 2048
+    form = {1: rows * cols // 32 * 64, 2: (rows + 31) // 32 * (cols // 32) * 1024}  # 20.5 and 10.3 MB
+    w = weights(ops, rows, cols, np.random.default_rng(1))
+    x = np.random.default_rng(2).normal(0, 1, (3000, cols)).astype(np.float32)  # (rows that pay for the form at every call)
+
+    def live():
+        a, b, c = C.c_size_t(), C.c_size_t(), C.c_size_t()
+        _lib.check(lib.cthip_cache_stats(C.byref(a), C.byref(b), C.byref(c)))
+        return a.value
+
+    def run(precision):
+        _lib.check(lib.cthip_set_option(b"gemm_precision", precision))
+        return ops.linear(x, w)
+
+    try:
+        _lib.check(lib.cthip_set_option(b"weight_planes", 0))
+        none, want = live(), {p: run(p) for p in (1, 2)}
+        assert live() == none
+        for limit, both in ((256, True), (24, False)):
+            _lib.check(lib.cthip_cache_trim())
+            _lib.check(lib.cthip_set_option(b"weight_planes", limit))
+            held = {1: 0, 2: 0}
+            for p in (2, 1, 2, 1, 1, 2):
+                assert np.array_equal(run(p), want[p])
+                held = {q: form[q] if q == p or (both and held[q]) else 0 for q in held}
+                assert sum(held.values()) <= live() - none <= sum(held.values()) * 1.25, (limit, p)  # (blocks come in size classes)
+    finally:
+        _lib.check(lib.cthip_set_option(b"gemm_precision", 2))
+        _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
+    w.free()
