@@ -346,11 +346,11 @@ __global__ __launch_bounds__(256) void k_digits_rows(unsigned char *__restrict__
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nkb = K >> 5;
   const int64_t row0 = (int64_t)blockIdx.x * 32;
   const int kb0 = blockIdx.y * 8, at = min(kb0 * 32 + 4 * lane, K - 4);
-  float4 v4[8];
+  f4_any v4[8];  // (rows at any alignment)
 #pragma unroll
-  for (int j = 0; j < 8; j++) v4[j] = *(const float4 *)(x + min(row0 + wave + 4 * j, rows - 1) * K + at);
+  for (int j = 0; j < 8; j++) v4[j] = *(const f4_any *)(x + min(row0 + wave + 4 * j, rows - 1) * K + at);
 #pragma unroll
-  for (int j = 0; j < 8; j++) *(float4 *)&turn[(lane >> 3) * BLOCK + (wave + 4 * j) * PITCH + 4 * (lane & 7)] = v4[j];
+  for (int j = 0; j < 8; j++) *(f4_any *)&turn[(lane >> 3) * BLOCK + (wave + 4 * j) * PITCH + 4 * (lane & 7)] = v4[j];
   __syncthreads();
   const int r = tid & 31, kb = kb0 + (tid >> 5);
   if (kb >= nkb) return;  // (the same for a block's 32 lanes)
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void k_rows_digits(unsigned char *__restrict__
     }
   }
 }
-// (x, g and b on 16 bytes, K a multiple of 32; a norm: K <= 8192)
+// (K a multiple of 32; a norm: x, g and b on 16 bytes, K <= 8192)
 int launch_rows_digits(void *digits, const float *x, int m, int K, int pro, const float *g, const float *b, float eps) {
   if (K % 32 || (pro != CTHIP_PRO_NONE && !rows_digits_supported(K))) return fail(CTHIP_E_BAD_ARG, "rows of %d as digits", K);
   const dim3 grid((m + 3) / 4);

@@ -616,7 +616,6 @@ int launch_linear_planes(float *y, const WMat *w, const float *x, const unsigned
                          int precision, const GemmRoute *route, unsigned char *planes_out, int out_terms, bool prompt, GemmDeferred *defer, bool *done) {
   const int K = (int)w->cols, terms = plane_terms(precision), terms_b = weight_terms(w, terms);
   const bool digits = terms_b == kDigits;
-  if (digits && ((uintptr_t)x & 15)) return 0;  // (the pass that makes digits reads 16 bytes at a time)
   DigitGemmArgs a = {};
   a.C = y;
   a.M = m, a.N = (int)w->rows;

@@ -221,3 +221,19 @@ def test_both_forms_of_a_matrix_are_kept(ops):
         _lib.check(lib.cthip_set_option(b"gemm_precision", 2))
         _lib.check(lib.cthip_set_option(b"weight_planes", 32768))
     w.free()
+
+
+@pytest.mark.parametrize("rows,cols,m", [(1026, 4128, 513), (6401, 96, 577)])
+def test_rows_at_any_alignment(ops, rows, cols, m):
+    """Input rows that do not lie on 16 bytes take the same launches as rows that do: the same results."""
+    from caten_amd import _lib
+    lib = _lib.init(0)
+    rng = np.random.default_rng(4)
+    w, x = weights(ops, rows, cols, rng), rng.normal(0, 1, (m, cols)).astype(np.float32)
+    dx, dy = ops.DeviceArray((m * cols + 4,)), ops.DeviceArray((m, rows))
+    want = ops.linear(x, w)
+    for off in (4, 8, 12):
+        _lib.check(lib.cthip_h2d(dx.ptr + off, x.ctypes.data, x.nbytes))
+        _lib.check(lib.cthip_linear(dy.ptr, w.handle, dx.ptr + off, m, None, None, 0, 0, None, None, 0.0))
+        assert np.array_equal(dy.numpy(), want), off
+    w.free()
