@@ -284,8 +284,8 @@ int launch_linear_rows(float *y, const WMat *w, const float *x, int64_t x_stride
 // A Linear over many rows from operands in memory as bf16 terms (gemm_planes.hip) or, over 4-bit weights at two terms' precision, as digits (gemm_digits.hip):
 // x as fp32 rows or already as the matrix takes it (linear_terms), the result to y / the route or (two terms, rows of whole blocks) as out_terms says.
 // *done stays false where this path does not apply.  planes_in: x lies in planes or digits already; prompt: one of a session's prompt (linear_planes_faster in
-// gemm_plan.h); defer: as for launch_linear_gemm, shares of K only with digits.
-bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt);
+// gemm_plan.h); shares: K may be split (no activation); defer: as for launch_linear_gemm, shares of K only with digits.
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt, bool shares = true);
 // Linear over 8 .. 64 rows that lie as operands of two terms (linear_few.hip)
 bool linear_few_pays(const WMat *w, int m, int precision, bool norm);  // norm: there is a pass over the rows in front of it anyway
 bool linear_few_shares_pays(const WMat *w, int m, int precision);  // rows as they are, shares of K left to the norm behind (any number of columns)

@@ -155,11 +155,13 @@ inline bool matmul_planes_faster(int M, int N, int K, int precision, int cus) {
   return planes < tile_plan(M, N, K, precision, -1, aligned, false, cus).us;
 }
 
-// Linears over 4-bit weights at two terms: digits against tiles that convert their operands.
-inline bool linear_digits_faster(int M, int N, int K, int type, double pass_bytes, bool prompt, int cus) {
-  if ((int64_t)(K / 32) * 4096 * 8 >= (1ll << 31)) return false;  // 32-bit offsets within a tile's rows
-  // (in a prompt, behind other launches, 1.5 - 2 us more than by itself)
-  const double us = digits_pick(M, N, K / 32, kDigitsPlain, true, prompt, cus).us + (prompt ? 1.5 : 0.0) + (pass_bytes > 0 ? pass_bytes / 4.2e6 + 5.0 : 0.0);
+// Linears over 4-bit weights at two terms: digits against tiles that convert their operands; shares: whether K may be split (no activation behind the sums).  x_bytes, w_bytes: what the
+// passes move that write the rows' and the weights' digits (0: there already).  Over 17 matrices (768 x 768 .. 22016 x 4096), 64 .. 2000 rows, weights out of memory, with and without an
+// activation: 0.5 % behind the faster side on average (shares taken for granted and a pass at 5 us + 4.2 TB/s: 2 %, and 1.5 times as long for 72 x 4096 x 11008 with an activation, 71 us
+// for 48).
+inline bool digits_fit(int K) { return (int64_t)(K / 32) * 4096 * 8 < (1ll << 31); }  // 32-bit offsets within a tile's rows
+inline bool linear_digits_faster(int M, int N, int K, int type, double x_bytes, double w_bytes, bool shares, int cus) {
+  const double us = digits_pick(M, N, K / 32, kDigitsPlain, shares, false, cus).us + (x_bytes > 0 ? x_bytes / 6e6 + 3.0 : 0.0) + (w_bytes > 0 ? w_bytes / 4.2e6 + 5.0 : 0.0);
   return us < tile_plan(M, N, K, GEMM_BF16X3, type, true, false, cus).us;
 }
 

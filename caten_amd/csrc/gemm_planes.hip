@@ -595,18 +595,24 @@ void weight_planes_limit(int64_t bytes) {
   if (over) weight_planes_drop();
 }
 
-bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt) {
+bool linear_planes_pays(const WMat *w, int m, int precision, bool planes_in, bool prompt, bool shares) {
   if (precision == GEMM_FP32 || m < 64 || w->rows < 64 || w->cols < 64 || (!is_quant(w) && w->cols % 16)) return false;
   // (three terms against integers: registers for one 32-column block less per wavefront, no faster than the tiles)
   if (is_quant(w) && precision == GEMM_BF16X6) return false;
   const int terms = plane_terms(precision), terms_b = weight_terms(w, terms);
-  double bytes = 0.0;
-  if (!weight_planes_kept(w, terms_b)) bytes = (double)w->q_bytes + weight_plane_bytes(w, terms_b);
-  if (!planes_in) bytes += (double)m * w->cols * (4 + 2 * terms);
-  // (a prompt past the limit: memory that is only lent for a launch, where that is long)
-  if (terms_b == kDigits && prompt && m < 512 && !weight_planes_kept(w, terms_b)) return false;
-  if (terms_b == kDigits) return linear_digits_faster(m, (int)w->rows, (int)w->cols, w->type, bytes, prompt, state().compute_units);
-  return linear_planes_faster(m, (int)w->rows, (int)w->cols, precision, w->type, bytes, prompt, state().compute_units);
+  const double w_bytes = weight_planes_kept(w, terms_b) ? 0.0 : (double)w->q_bytes + weight_plane_bytes(w, terms_b);
+  const double x_bytes = planes_in ? 0.0 : (double)m * w->cols * (4 + 2 * terms);
+  if (terms_b == kDigits) {
+    if (!digits_fit((int)w->cols)) return false;
+    // A prompt whose digits stay: always.  (Six layers, 65 / 256 / 950 rows, tiles alone and digits alone: 384 wide 347 / 364 / 434 and 307 / 325 / 419 us, GPT-2 small 403 / 405 / 701 and
+    // 355 / 375 / 544, 1.1B shape 600 / 747 / 2032 and 528 / 615 / 1243, 7B shape 1452 / 2106 / 7201 and 1019 / 1384 / 3607; nowhere between 65 and 1900 rows are tiles the faster ones, and
+    // chosen Linear by Linear the small models were up to 15 % slower than digits alone.)
+    // Past the limit: memory that is only lent for a launch, where that is long.
+    if (prompt && w_bytes == 0.0) return true;
+    if (prompt && m < 512) return false;
+    return linear_digits_faster(m, (int)w->rows, (int)w->cols, w->type, x_bytes, w_bytes, shares, state().compute_units);
+  }
+  return linear_planes_faster(m, (int)w->rows, (int)w->cols, precision, w->type, w_bytes + x_bytes, prompt, state().compute_units);
 }
 // ... and nothing can be in the way of it
 bool linear_planes_ready(const WMat *w, int m, int precision) {

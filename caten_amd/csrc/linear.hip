@@ -816,7 +816,7 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
     }
     bool done = false;
     rc = 0;
-    if (linear_planes_pays(w, m, state().gemm_precision, false, false))
+    if (linear_planes_pays(w, m, state().gemm_precision, false, false, act == CTHIP_ACT_NONE))
       rc = launch_linear_planes(y, w, xin, nullptr, m, bias, residual, act, state().gemm_precision, nullptr, nullptr, kTermsNone, false, nullptr, &done);
     if (!done) rc = launch_linear_gemm(y, w, xin, m, bias, residual, act, state().gemm_precision);
     if (tmp) cthip_free(tmp);

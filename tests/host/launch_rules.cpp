@@ -94,10 +94,6 @@ static void linears_over_many_rows() {
       {2, CTHIP_Q8_0, 1200, 5120, 1280, 64.0, 53.8},
       {2, CTHIP_Q8_0, 300, 6400, 1600, 44.9, 37.6},
       {2, CTHIP_Q8_0, 512, 768, 3072, 18.2, 35.4},
-      {2, CTHIP_Q4_0, 900, 2560, 2048, 57.0, 46.5},
-      {2, CTHIP_Q4_0, 300, 12288, 4096, 108.7, 131.9},
-      {2, CTHIP_Q4_0, 300, 1024, 4096, 19.3, 41.9},
-      {2, CTHIP_Q4_0, 300, 2048, 5632, 34.7, 55.3},
       {1, CTHIP_F16, 512, 1024, 4096, 19.6, 48.7},
       {1, CTHIP_F32, 512, 11264, 2048, 103.4, 63.9},
       {1, CTHIP_F32, 300, 1280, 5120, 26.4, 54.7},
@@ -161,28 +157,99 @@ static void matrix_products() {
   }
 }
 
-// Linears on 4-bit weights through 6-bit digits, one share of K, us with tiles of 64 x 64, 64 x 128, 128 x 128
+// Linears on 4-bit weights at two terms, us: tiles that convert their operands, 6-bit digits (the pass that writes the rows' included); shares of K where nothing but a bias follows, none
+// behind an activation.  Sizes that the rule was not fitted to, but for the last: the side that it takes is within 9 % of the other.
+static void digits_or_tiles() {
+  static const struct {
+    int m, n, k;
+    bool shares;
+    double tiles, digits;
+  } t[] = {{80, 1536, 512, true, 8.9, 9.5}, {80, 1536, 512, false, 8.9, 11.9}, {170, 1536, 512, true, 10.5, 9.7}, {170, 1536, 512, false, 11.9, 12.2},
+           {370, 1536, 512, true, 10.7, 10.1}, {370, 1536, 512, false, 12.1, 12.8}, {800, 1536, 512, true, 11.8, 12.8}, {800, 1536, 512, false, 13.2, 15.4},
+           {1700, 1536, 512, true, 22.2, 16.2}, {1700, 1536, 512, false, 24.8, 21.2}, {80, 704, 2816, true, 12.0, 13.0}, {80, 704, 2816, false, 12.1, 23.9},
+           {170, 704, 2816, true, 13.8, 15.1}, {170, 704, 2816, false, 14.0, 24.7}, {370, 704, 2816, true, 18.4, 19.1}, {370, 704, 2816, false, 18.5, 26.1},
+           {800, 704, 2816, true, 28.6, 26.8}, {800, 704, 2816, false, 28.8, 29.4}, {1700, 704, 2816, true, 41.2, 35.6}, {1700, 704, 2816, false, 42.6, 40.0},
+           {80, 2880, 960, true, 12.7, 12.0}, {80, 2880, 960, false, 12.8, 14.4}, {170, 2880, 960, true, 16.1, 12.6}, {170, 2880, 960, false, 17.4, 15.1},
+           {370, 2880, 960, true, 17.2, 16.2}, {370, 2880, 960, false, 18.7, 21.1}, {800, 2880, 960, true, 32.8, 20.1}, {800, 2880, 960, false, 35.4, 25.0},
+           {1700, 2880, 960, true, 53.4, 30.4}, {1700, 2880, 960, false, 57.8, 35.9}, {80, 3840, 1536, true, 15.2, 15.2}, {80, 3840, 1536, false, 15.4, 17.6},
+           {170, 3840, 1536, true, 20.7, 16.4}, {170, 3840, 1536, false, 21.1, 19.1}, {370, 3840, 1536, true, 25.4, 21.6}, {370, 3840, 1536, false, 26.8, 26.6},
+           {800, 3840, 1536, true, 50.3, 28.8}, {800, 3840, 1536, false, 53.8, 33.2}, {1700, 3840, 1536, true, 95.3, 49.9}, {1700, 3840, 1536, false, 99.4, 58.9},
+           {80, 5376, 1344, true, 18.6, 14.5}, {80, 5376, 1344, false, 18.7, 17.0}, {170, 5376, 1344, true, 21.7, 15.8}, {170, 5376, 1344, false, 22.9, 18.5},
+           {370, 5376, 1344, true, 42.1, 21.1}, {370, 5376, 1344, false, 45.0, 26.1}, {800, 5376, 1344, true, 63.4, 34.4}, {800, 5376, 1344, false, 67.3, 40.2},
+           {1700, 5376, 1344, true, 107.3, 57.3}, {1700, 5376, 1344, false, 113.2, 66.2}, {80, 1792, 7168, true, 21.8, 20.8}, {80, 1792, 7168, false, 21.8, 49.1},
+           {170, 1792, 7168, true, 29.0, 26.2}, {170, 1792, 7168, false, 29.4, 50.1}, {370, 1792, 7168, true, 56.8, 41.1}, {370, 1792, 7168, false, 55.4, 53.0},
+           {800, 1792, 7168, true, 98.9, 68.8}, {800, 1792, 7168, false, 99.5, 73.9}, {1700, 1792, 7168, true, 182.5, 98.8}, {1700, 1792, 7168, false, 183.1, 101.7},
+           {80, 6144, 2304, true, 25.2, 21.1}, {80, 6144, 2304, false, 25.4, 23.6}, {170, 6144, 2304, true, 33.4, 26.3}, {170, 6144, 2304, false, 34.7, 31.3},
+           {370, 6144, 2304, true, 65.1, 33.4}, {370, 6144, 2304, false, 68.2, 37.9}, {800, 6144, 2304, true, 103.5, 56.4}, {800, 6144, 2304, false, 107.1, 60.1},
+           {1700, 6144, 2304, true, 199.4, 94.3}, {1700, 6144, 2304, false, 207.1, 103.8}, {80, 8192, 3072, true, 31.7, 26.2}, {80, 8192, 3072, false, 31.8, 28.8},
+           {170, 8192, 3072, true, 45.4, 33.3}, {170, 8192, 3072, false, 47.0, 38.3}, {370, 8192, 3072, true, 90.5, 45.5}, {370, 8192, 3072, false, 92.9, 50.3},
+           {800, 8192, 3072, true, 178.1, 89.9}, {800, 8192, 3072, false, 182.4, 98.3}, {1700, 8192, 3072, true, 324.1, 166.2}, {1700, 8192, 3072, false, 328.4, 174.9}, {72, 4096, 11008, false, 48.0, 71.1}};
+  for (const auto &c : t) {
+    const bool digits = linear_digits_faster(c.m, c.n, c.k, CTHIP_Q4_0, (double)c.m * c.k * 8, 0.0, c.shares, 256);
+    char what[128];
+    snprintf(what, sizeof(what), "digits for %d rows of 4 bits %d x %d%s (%.1f against %.1f us)", c.m, c.n, c.k, c.shares ? "" : ", activation", c.digits, c.tiles);
+    if (c.digits > 1.09 * c.tiles || c.tiles > 1.09 * c.digits) expect(what, digits, c.digits < c.tiles);
+  }
+}
+
+// Their tiles, one share of K, us with 64 x 64, 64 x 128, 128 x 128: within 6 % of the best
 static void tiles_of_digits() {
   static const struct {
     int m, n, k;
     double us[3];
-  } t[] = {{100, 3072, 1024, {10.0, 12.3, 18.5}},
-           {300, 2560, 2048, {15.7, 19.4, 29.6}},
-           {200, 11264, 2048, {34.0, 28.0, 33.0}},
-           {280, 4096, 4096, {40.0, 35.0, 52.0}},
-           {1900, 2048, 5632, {98.0, 71.0, 80.0}},
-           {1900, 11264, 2048, {195.0, 133.0, 128.0}}};
+  } t[] = {{80, 1536, 512, {9.5, 10.8, 14.0}}, {260, 1536, 512, {10.2, 11.5, 14.9}}, {520, 1536, 512, {10.7, 12.0, 15.3}}, {800, 1536, 512, {12.8, 12.7, 15.9}},
+           {1100, 1536, 512, {13.7, 13.5, 16.5}}, {1700, 1536, 512, {17.6, 16.2, 18.0}}, {80, 704, 2816, {21.6, 26.3, 39.6}}, {260, 704, 2816, {23.3, 27.9, 41.1}},
+           {520, 704, 2816, {24.4, 29.5, 42.3}}, {800, 704, 2816, {26.8, 32.3, 44.2}}, {1100, 704, 2816, {28.0, 32.9, 45.6}}, {1700, 704, 2816, {34.4, 35.5, 48.0}},
+           {80, 2880, 960, {11.9, 14.0, 19.1}}, {260, 2880, 960, {13.3, 15.3, 20.7}}, {520, 2880, 960, {17.5, 17.5, 22.6}}, {800, 2880, 960, {23.2, 20.0, 24.9}},
+           {1100, 2880, 960, {28.3, 22.6, 25.6}}, {1700, 2880, 960, {36.6, 30.2, 33.1}}, {80, 3840, 1536, {15.2, 18.1, 25.6}}, {260, 3840, 1536, {20.1, 20.6, 28.4}},
+           {520, 3840, 1536, {30.0, 25.6, 31.3}}, {800, 3840, 1536, {37.7, 28.5, 34.0}}, {1100, 3840, 1536, {47.1, 38.7, 42.2}}, {1700, 3840, 1536, {66.0, 50.8, 49.8}},
+           {80, 5376, 1344, {14.5, 17.1, 23.7}}, {260, 5376, 1344, {19.6, 19.7, 26.9}}, {520, 5376, 1344, {29.3, 25.7, 30.1}}, {800, 5376, 1344, {41.5, 34.5, 38.8}},
+           {1100, 5376, 1344, {51.6, 39.6, 42.7}}, {1700, 5376, 1344, {74.8, 57.6, 58.4}}, {80, 1792, 7168, {47.0, 56.5, 90.7}}, {260, 1792, 7168, {49.5, 58.9, 91.4}},
+           {520, 1792, 7168, {55.9, 63.1, 94.7}}, {800, 1792, 7168, {70.6, 69.1, 97.9}}, {1100, 1792, 7168, {84.8, 78.2, 100.3}}, {1700, 1792, 7168, {120.3, 98.3, 112.0}},
+           {80, 6144, 2304, {21.1, 24.3, 35.4}}, {260, 6144, 2304, {31.1, 28.9, 39.7}}, {520, 6144, 2304, {54.2, 39.5, 46.3}}, {800, 6144, 2304, {68.5, 56.7, 59.6}},
+           {1100, 6144, 2304, {92.1, 68.9, 68.0}}, {1700, 6144, 2304, {129.8, 99.5, 94.4}}, {80, 8192, 3072, {26.5, 31.0, 45.0}}, {260, 8192, 3072, {53.1, 43.0, 52.0}},
+           {520, 8192, 3072, {85.1, 69.3, 76.0}}, {800, 8192, 3072, {115.8, 90.5, 89.8}}, {1100, 8192, 3072, {153.1, 117.3, 111.8}}, {1700, 8192, 3072, {224.0, 165.8, 161.5}}};
   for (const auto &c : t) {
     const int tile = digits_pick(c.m, c.n, c.k / 32, kDigitsPlain, false, false, 256).tile;
     char what[96];
     snprintf(what, sizeof(what), "digits of %d x %d x %d: tile %d takes %.1f us", c.m, c.n, c.k, tile, c.us[tile]);
-    expect(what, c.us[tile] <= std::min(c.us[0], std::min(c.us[1], c.us[2])), true);
+    expect(what, c.us[tile] <= 1.06 * std::min(c.us[0], std::min(c.us[1], c.us[2])), true);
+  }
+}
+
+// Their shares of K, us at 1, 2, 3, 4, 6, 8 of them: within 12 % of the best; a count that was not timed lies between two that are
+static void shares_of_digits() {
+  static const int counts[] = {1, 2, 3, 4, 6, 8};
+  static const struct {
+    int m, n, k;
+    double us[6];
+  } t[] = {{80, 704, 2816, {21.6, 17.3, 15.2, 14.0, 13.3, 12.9}}, {170, 704, 2816, {22.3, 18.3, 16.4, 15.3, 15.1, 16.2}}, {370, 704, 2816, {23.5, 20.9, 19.1, 20.3, 19.7, 21.6}},
+           {800, 704, 2816, {26.8, 28.3, 25.7, 26.4, 26.2, 26.9}}, {80, 3840, 1536, {15.2, 15.8, 16.4, 16.5, 18.1, 18.3}},
+           {170, 3840, 1536, {16.4, 20.9, 21.9, 22.6, 25.2, 19.2}}, {370, 3840, 1536, {20.5, 28.4, 29.1, 27.5, 31.5, 21.7}},
+           {800, 3840, 1536, {28.5, 40.3, 42.4, 46.3, 52.1, 28.8}}, {80, 1792, 7168, {47.0, 31.8, 25.9, 23.1, 22.5, 20.7}},
+           {170, 1792, 7168, {47.9, 33.3, 31.9, 28.0, 27.7, 26.8}}, {370, 1792, 7168, {50.7, 44.3, 40.7, 39.3, 44.3, 38.9}},
+           {800, 1792, 7168, {69.1, 61.9, 66.8, 62.0, 65.7, 67.1}}, {80, 6144, 2304, {21.1, 23.1, 23.2, 23.3, 25.3, 25.4}},
+           {170, 6144, 2304, {26.1, 30.5, 27.9, 29.3, 31.4, 35.8}}, {370, 6144, 2304, {33.4, 41.2, 42.7, 44.8, 50.3, 56.4}},
+           {800, 6144, 2304, {56.7, 70.3, 75.1, 80.8, 91.7, 106.0}}};
+  for (const auto &c : t) {
+    const int ks = digits_pick(c.m, c.n, c.k / 32, kDigitsPlain, true, false, 256).ks;
+    double best = 1e30, got = 0.0;
+    for (int q = 0; q < 6; q++) {
+      best = std::min(best, c.us[q]);
+      if (counts[q] <= ks) got = c.us[q];
+      if (counts[q] >= ks && (q == 0 || counts[q - 1] < ks)) got = std::max(got, c.us[q]);
+    }
+    char what[96];
+    snprintf(what, sizeof(what), "%d shares of digits of %d x %d x %d (%.1f against %.1f us)", ks, c.m, c.n, c.k, got, best);
+    expect(what, got <= 1.12 * best, true);
   }
 }
 
 int main() {
   integer_gemv();
+  digits_or_tiles();
   tiles_of_digits();
+  shares_of_digits();
   shares_of_tiles();
   linears_over_many_rows();
   matrix_products();
