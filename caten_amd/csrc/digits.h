@@ -64,11 +64,12 @@ __device__ __forceinline__ float digits_top(const float *v) {
 __device__ __forceinline__ bool digits_uneven_columns(const float *v, float m, bool in) {
   const int lane = threadIdx.x & 63;
   const bool ok = in && m > 0.0f && m < INFINITY;
-  const int up = 128 - (int)(__float_as_uint(m) >> 23);
+  // (a row with an infinity or a NaN makes every sum a NaN, and no column is small)
+  const float up = ok ? __uint_as_float((254u - max(__float_as_uint(m) >> 23, 1u)) << 23) : 0.0f;
   float s[32];
 #pragma unroll
   for (int i = 0; i < 32; i++) {
-    const float t = ok ? __builtin_amdgcn_ldexpf(v[i], up) : 0.0f;
+    const float t = v[i] * up;
     s[i] = t * t;
   }
   // a column's sum to each lane: half of the columns a step, to the lanes that keep them
@@ -98,7 +99,7 @@ __device__ __forceinline__ bool digits_uneven_columns(const float *v, float m, b
     const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
     return __uint_as_float(p[0]) + __uint_as_float(p[1]);
   };
-  const float top = ok ? __builtin_amdgcn_ldexpf(m, up) : 0.0f;
+  const float top = ok ? m * up : 0.0f;
   const float all = half_sum(top * top);
   const unsigned long long rows = __ballot(ok);
   const float n = (float)__popc((unsigned)(lane & 32 ? rows >> 32 : rows));

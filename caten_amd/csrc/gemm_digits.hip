@@ -130,8 +130,6 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
       for (int i = 1; i < MB; i++) lda(i);
 #pragma unroll
       for (int b = 1; b < NB; b++) ldb(b);
-#pragma unroll
-      for (int i = 0; i < MB; i++) least[i] = min(least[i], (unsigned)sc[k][i]);
     }
     if (KB == 1) issue((buf + NBUF - 1) % NBUF);  // while they are on their way
     __builtin_amdgcn_sched_barrier(0);
@@ -164,6 +162,10 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
       __builtin_amdgcn_sched_barrier(0);
     }
     dlast = d[KB - 1][NB - 1];
+#pragma unroll
+    for (int k = 0; k < KB; k++)
+#pragma unroll
+      for (int i = 0; i < MB; i++) least[i] = min(least[i], (unsigned)sc[k][i]);
   };
 
 #pragma unroll
