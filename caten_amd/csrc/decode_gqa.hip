@@ -16,10 +16,10 @@
 // attention launch adds into is cleared by the next layer's qkv launch, the set the MLP launch adds into by the
 // attention launch: in both cases the last reader has finished and the next writer has not started.
 //
-// A row of D = 2048 * KC columns is 64 * KC blocks of 32 (KC = 1 is what is built): lane l of a wavefront owns blocks l + 64 j of every
+// k_gqa_qkv: a row of D = 2048 * KC columns is 64 * KC blocks of 32 (KC = 1 is what is built): lane l of a wavefront owns blocks l + 64 j of every
 // row the wavefront handles, so the 32 input floats of a block are read from LDS once and multiply several rows.
 // The staged vector is stored with the 16-byte slot index xor-ed by the block index: lanes read whole blocks
-// (128 bytes apart), which would otherwise all fall on the same LDS banks.
+// (128 bytes apart), which would otherwise all fall on the same LDS banks.  k_gqa_mlp takes its rows in groups of 16 against digits of the vector instead.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -347,7 +347,9 @@ void k_gqa_attn_proj(GqaAttnArgs a) {
 // ---- launch 3: RMSNorm folded through 32 gate and 32 up rows, SwiGLU, one Q4_0 block per row of `down` ----
 // The 64 rows are four groups of 16 for the matrix cores (gemv_int.hip): every wavefront takes an eighth of K, 256 columns, of all of them, so that it reads its
 // digits once for four groups.  (In vector instructions, a row of 2048 to a wavefront at a time, products and sums were 2.8 us of a launch; as integers 11.1 -> 10.3 us.)
-// What is left is what a workgroup has to read: 128 KB of accumulators, 111 KB of weights, at 64 bytes a clock.
+// What a workgroup has to read, 128 KB of accumulators and 111 KB of weights, is 1.7 us at 64 bytes a clock; what bounds the rest of the launch is not known.
+// Digits hold 30 bits below a chunk's largest value.  The vector instructions held each input's 24, but summed nibbles times inputs less eight times the inputs' sum, which has 24 below the
+// largest: normal inputs 3.9e-7 -> 0.3e-7 off 64 bits, one of 32 a thousand times as large at a weight of zero 8.7e-5 -> 4e-7.
 template <int NT>
 __global__ __launch_bounds__(NT) void k_gqa_mlp(GqaMlpArgs a) {
   constexpr int NW = NT / 64, D = 2048, NG = 4, PJ = D / NT;  // PJ: rows of the down projection per thread

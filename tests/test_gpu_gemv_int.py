@@ -152,3 +152,34 @@ def test_layers_of_slabs_match_a_launch_per_linear(ffn):
     assert runs[0][0] == runs[1][0]
     for a, b in zip(runs[0][1], runs[1][1]):
         assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
+
+
+def test_slabs_whose_large_values_meet_weights_of_zero(ops):
+    """A layer of slabs whose MLP has channels a thousand times as large that gate, up and down do not read: its digits, 30 bits below a chunk's largest value, against the
+    same model in fp32.  The launch per Linear takes nibbles times inputs less eight times the inputs' sum, which has 24 bits below the largest."""
+    print("case: three-launch layer, large channels", flush=True)
+    from caten_amd import _lib, llm, synth
+    lib = _lib.load()
+    cfg = dict(synth.LLAMA_CONFIGS["llama-1.1b"], ffn=1120, n_layers=2, vocab=1003, max_seq=64)
+    w, rng = synth.llama_weights(cfg, seed=17), np.random.default_rng(2)
+    ch, ff = (np.arange(0, n, 32) + rng.integers(0, 32, n // 32) for n in (cfg["dim"], cfg["ffn"]))
+    for l in range(2):
+        w["ffn_norm"][l][ch] *= 1000.0
+        w["w_up"][l][ff] *= 1000.0
+        w["w_gate"][l][:, ch] = w["w_up"][l][:, ch] = 0.0
+        w["w_down"][l][:, ff] = 0.0
+    sd = llm.llama_state_dict(w, "q4_0")
+    exact = {k: llm.Tensor.from_f32(ops.WeightMatrix(t.kind, t.raw, t.rows, t.cols).dequantize()) if t.kind == "q4_0" else t for k, t in sd.items()}
+    prompt, last = synth.prompt(cfg["vocab"], 2, seed=17), []
+    try:
+        for fused, d in ((1, sd), (0, sd), (0, exact)):
+            _lib.check(lib.cthip_set_option(b"decode_fused", fused))
+            model = llm.make_llama(cfg, d)
+            model.forward(prompt[:1], 1, 0)
+            last.append(model.forward(prompt[1:], 1, 1, return_logits=True)[1].astype(np.float64))
+            model.close()
+    finally:
+        _lib.check(lib.cthip_set_option(b"decode_fused", 1))
+    digits, vector = (np.linalg.norm(x - last[2]) / np.linalg.norm(last[2]) for x in last[:2])
+    print("digits", digits, "vector kernels", vector, flush=True)
+    assert digits <= vector and digits <= 1e-5
