@@ -23,7 +23,7 @@ namespace cthip {
 template <int MB, int NB, int WM, int WN, int KB, int NBUF, int OUT>
 __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 ? 3 : 2) void k_gemm_digits(DigitGemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN, NBLK = MB * NB;
-  static_assert(NBLK * KB * NBUF % 2 == 0, "the sums of a step's last block wait for the next step's first: two sets in turn");
+  static_assert(NBLK * KB % 2 == 0, "the sums of a step's last block wait for the next step's first: two sets in turn");
   constexpr int ABYTES = BM * 96, BBYTES = BN * 32, SBYTES = BM * 4;
   constexpr int PART = ABYTES + BBYTES + SBYTES, BUF = KB * PART;
   constexpr int NA = ABYTES / 1024, NBL = BBYTES / 1024, NS = BM / 64;  // load instructions of a step
@@ -150,10 +150,9 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
         const v8i_dg av = {(int)a16[k][i][j].x, (int)a16[k][i][j].y, (int)a16[k][i][j].z, (int)a16[k][i][j].w, (int)a8[k][i][j].x, (int)a8[k][i][j].y, 0, 0};
         t = j ? __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, t, 2, 2, 1, sc[k][i], 0, 127) : __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, t, 2, 2, 0, sc[k][i], 0, 127);
       }
-      const int set = buf * KB * NBLK + q;
-      tmp[set & 1] = t;
+      tmp[q & 1] = t;
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[pi][pb][r] = fmaf(dp, tmp[(set & 1) ^ 1][r], acc[pi][pb][r]);
+      for (int r = 0; r < 16; r++) acc[pi][pb][r] = fmaf(dp, tmp[(q & 1) ^ 1][r], acc[pi][pb][r]);
 #pragma unroll
       for (int g = 0; g < 2; g++) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -179,9 +178,8 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
       if ((i += KB) >= nsteps) break;
     }
   wait_barrier<0>();
-  const bool even = NBLK * KB % 2 && nsteps % 2;  // which set the last block went to
 #pragma unroll
-  for (int r = 0; r < 16; r++) acc[MB - 1][NB - 1][r] = fmaf(dlast, even ? tmp[0][r] : tmp[1][r], acc[MB - 1][NB - 1][r]);
+  for (int r = 0; r < 16; r++) acc[MB - 1][NB - 1][r] = fmaf(dlast, tmp[1][r], acc[MB - 1][NB - 1][r]);
 
   // ---- what three digits left of blocks that have it as terms (digits.h), of this wavefront's own rows.  Rare: one look at a wavefront's exponents, and where one is 0 all of the
   // share's again, 32 blocks of k at a time; a block is the four instructions of two bf16 terms against the same weights, its loads waited for.  (us with the pass that makes the
@@ -452,7 +450,7 @@ static int digits_launch_as(DigitGemmArgs a, int ks) {
   constexpr int BM = 32 * MB * WM, BN = 32 * NB * WN;
   constexpr size_t buf = KB * ((size_t)BM * 100 + (size_t)BN * 32), turn = (size_t)WM * WN * 32 * (32 * NB + 4) * 4;
   constexpr size_t lds = NBUF * buf > turn ? NBUF * buf : turn;
-  static_assert(lds <= 80 * 1024, "two workgroups to a compute unit and more");
+  static_assert(lds <= 64 * 1024, "what a launch may ask for without an attribute, and two workgroups to a compute unit and more");
   a.col_bias = a.bias, a.bias = nullptr;
   a.tm = (a.M + BM - 1) / BM;
   a.tn = (a.N + BN - 1) / BN;
@@ -465,11 +463,6 @@ static int digits_launch_as(DigitGemmArgs a, int ks) {
     if (best < 0 || score < best) best = score, a.band = h;
   }
   auto fn = k_gemm_digits<MB, NB, WM, WN, KB, NBUF, OUT>;
-  static bool big_lds = false;
-  if (!big_lds && lds > 64 * 1024) {
-    CTHIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    big_lds = true;
-  }
   hipLaunchKernelGGL(fn, dim3(8u * a.chunk, (a.nkb + a.kper - 1) / a.kper), dim3(64 * WM * WN), lds, state().stream, a);
   CTHIP_LAUNCH_CHECK();
   return 0;

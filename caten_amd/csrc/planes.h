@@ -175,58 +175,18 @@ __device__ __forceinline__ void plane_gemm_finish_any(const PlaneStore &a, int r
     a.C[(int64_t)row * a.N + col + t] = x;
   }
 }
-// columns col .. col + 3 of one row: the same for the kernels of a few rows, which ask for bias and residual as they go
-__device__ __forceinline__ void plane_gemm_store(const PlaneGemmArgs &a, int row, int col, float4 v4) {
-  int N = a.N;
-  asm volatile("" : "+s"(N));  // read anew at every call: known to be the same, it has the caller's loop copied for each case below (3000 x 4100 x 5000: 2.4 % slower)
-  if (row >= a.M || col >= N) return;
-  float v[4] = {v4.x, v4.y, v4.z, v4.w};
-  if ((N & 3) == 0) {
-    if (a.bias) {
-      const float4 bb = *(const float4 *)(a.bias + col);
-      v[0] += bb.x, v[1] += bb.y, v[2] += bb.z, v[3] += bb.w;
-    }
-    if (a.pairs) {
-      v[0] = apply_act(CTHIP_ACT_SILU, v[0]) * v[1], v[1] = apply_act(CTHIP_ACT_SILU, v[2]) * v[3];
-      if (a.planes) {  // two columns of the result: neighbours in both terms
-        const unsigned h = pack_bf16_pl(v[0], v[1]);
-        const unsigned l = pack_bf16_pl(v[0] - __uint_as_float(h << 16), v[1] - __uint_as_float(h & 0xffff0000u));
-        unsigned short *p = a.planes + ((int64_t)row * a.pkb + (col >> 6)) * 64 + ((col >> 1) & 31);
-        *(unsigned *)p = h;
-        *(unsigned *)(p + 32) = l;
-      } else {
-        *(float2 *)(a.C + (int64_t)row * (N >> 1) + (col >> 1)) = make_float2(v[0], v[1]);
-      }
-      return;
-    }
-    if (a.act != CTHIP_ACT_NONE)
-#pragma unroll
-      for (int t = 0; t < 4; t++) v[t] = apply_act(a.act, v[t]);
-    if (a.residual) {
-      const float4 rr = *(const float4 *)(a.residual + (int64_t)row * N + col);
-      v[0] += rr.x, v[1] += rr.y, v[2] += rr.z, v[3] += rr.w;
-    }
-    if (a.planes) {
-      store_planes4(a.planes, row, a.pkb, col, v);
-      return;
-    }
-    float *dst = a.C;
-    int ldd = N, cbase = 0;
-    if (a.routed) {
-      // (selected, not indexed: an index would put the arguments into scratch memory)
-      const bool p2 = col >= a.route.c0[2], p1 = col >= a.route.c0[1];
-      dst = p2 ? a.route.dst[2] : p1 ? a.route.dst[1] : a.route.dst[0];
-      ldd = p2 ? a.route.ld[2] : p1 ? a.route.ld[1] : a.route.ld[0];
-      cbase = p2 ? a.route.c0[2] : p1 ? a.route.c0[1] : 0;
-    }
-    *(float4 *)(dst + (int64_t)row * ldd + (col - cbase)) = make_float4(v[0], v[1], v[2], v[3]);
+// columns col .. col + 3 of one row: the same where bias and residual are asked for as a thread goes (linear_rows.hip)
+__device__ __forceinline__ void plane_gemm_store(const PlaneGemmArgs &args, int row, int col, float4 v4) {
+  const PlaneStore a(args, PlaneStore::Late());
+  if (row >= a.M || col >= a.N) return;
+  if (a.N & 3) {
+    plane_gemm_finish_any(a, row, col, v4);
     return;
   }
-  for (int t = 0; t < 4 && col + t < N; t++) {
-    float x = apply_act(a.act, v[t] + (a.bias ? a.bias[col + t] : 0.0f));
-    if (a.residual) x += a.residual[(int64_t)row * N + col + t];
-    a.C[(int64_t)row * N + col + t] = x;
-  }
+  float4 bb = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rr = bb;
+  if (a.bias) bb = *(const float4 *)(a.bias + col);
+  if (a.residual && !a.pairs) rr = *(const float4 *)(a.residual + (int64_t)row * a.N + col);
+  plane_gemm_finish(a, a.N, row, col, v4, bb, rr);
 }
 // A wavefront's 32 rows of 32 NB columns, which lie in LDS (pitch 32 NB + 4), to where they go.  A lane stores the same four columns of every 64 / C4-th row, so that their bias is
 // read once, by plane_gemm_bias, long before; the residual of plain rows is asked for several rows at a time.  Short code: with every row's
