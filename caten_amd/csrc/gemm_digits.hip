@@ -182,59 +182,117 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB * KB <= 2 ? 4 : MB * NB <= 4 
   for (int r = 0; r < 16; r++) acc[MB - 1][NB - 1][r] = fmaf(dlast, tmp[1][r], acc[MB - 1][NB - 1][r]);
 
   // ---- what three digits left of blocks that have it as terms (digits.h), of this wavefront's own rows.  Rare: one look at a wavefront's exponents, and where one is 0 all of the
-  // share's again, 32 blocks of k at a time; a block is the four instructions of two bf16 terms against the same weights, its loads waited for.  (us with the pass that makes the
-  // digits, no such block / a column of all of K / every block: 1900 x 11264 x 2048 147 / 164 / 490, 1900 x 2048 x 5632 92 / 97 / 285, 280 x 12288 x 4096 62 / 64 / 186; two bf16 terms in
-  // place, without their pass: 194 and 117 for the first two.)
+  // share's again, 32 blocks of k at a time; a block is the four instructions of two bf16 terms against the same weights.  (us with the pass that makes the digits, no such block / a
+  // column of all of K / every block: 1900 x 11264 x 2048 150 / 158 / 400, 1900 x 2048 x 5632 92 / 95 / 235, 280 x 12288 x 4096 62 / 65 / 162; two bf16 terms in place, without their pass:
+  // 194 and 117 for the first two.  Every block is 128 bytes a row for every tile of columns, by every wavefront for itself.)
+  bool look = false, mine[MB];
 #pragma unroll
   for (int i = 0; i < MB; i++) {
-    const int group = min(m0 / 32 + MB * wm + i, mg - 1);  // (past the end: not this wavefront's)
-    const bool mine = m0 + 32 * (MB * wm + i) + col < a.M;
-    if (!__any(mine && least[i] < 256u)) continue;
-    const unsigned char *words = a.A + (int64_t)mg * nkb * kDigitRecord + ((int64_t)k0 * mg + group) * 128;
-    const unsigned char *rests = a.A + (int64_t)mg * nkb * (kDigitRecord + kDigitScales) + ((int64_t)group * nkb + k0) * kDigitRests + lane * 16;
+    mine[i] = m0 + 32 * (MB * wm + i) + col < a.M;
+    look = look || __any(mine[i] && least[i] < 256u);
+  }
+  if (look) {
+    const unsigned char *words = a.A + (int64_t)mg * nkb * kDigitRecord + (int64_t)k0 * mg * 128;
+    const unsigned char *rests = a.A + (int64_t)mg * nkb * (kDigitRecord + kDigitScales) + (int64_t)k0 * kDigitRests + lane * 16;
+    int group[MB];  // (past the end: not this wavefront's)
+#pragma unroll
+    for (int i = 0; i < MB; i++) group[i] = min(m0 / 32 + MB * wm + i, mg - 1);
     const unsigned upper = half ? ~0u : 0u;
-    const int rows = a.M - 32 * group - 4 * (lane & 7);  // of the four whose exponents this lane looks at
+    auto word_of = [&](int i, int kb) __attribute__((always_inline)) { return *(const unsigned *)(words + ((int64_t)kb * mg + group[i]) * 128 + col * 4); };
+    auto terms_of = [&](int i, int kb, uint4 *t) __attribute__((always_inline)) {  // the small term first
+      const uint4 *r = (const uint4 *)(rests + ((int64_t)group[i] * nkb + kb) * kDigitRests);
+      t[0] = r[128], t[1] = r[192], t[2] = r[0], t[3] = r[64];
+    };
+    auto weights_of = [&](int b, int kb, uint4 &w16, uint2 &w8, float &dw) __attribute__((always_inline)) {
+      const unsigned char *w = a.B + ((int64_t)min(n0 / 32 + NB * wn + b, ng - 1) * nkb + k0 + kb) * kDigitWRecord;
+      w16 = *(const uint4 *)(w + col * 16);
+      w8 = *(const uint2 *)(w + 512 + col * 8);
+      dw = *(const float *)(w + 768 + col * 4);
+    };
+    auto own = [&](int i, unsigned word, uint4 *t) __attribute__((always_inline)) {  // (rows that have none: nothing was written there)
+      const unsigned has = mine[i] & (word < 0x1000000u) ? ~0u : 0u;
+#pragma unroll
+      for (int q = 0; q < 4; q++) t[q].x &= has, t[q].y &= has, t[q].z &= has, t[q].w &= has;
+    };
+    auto add = [&](int b, const uint4 (*t)[4], uint4 w16, uint2 w8, float dw) __attribute__((always_inline)) {
+      const v6u_dg six = {w16.x, w16.y, w16.z, w16.w, w8.x, w8.y};
+      const auto all = __builtin_bit_cast(v16u_dg, __builtin_amdgcn_cvt_scalef32_pk32_bf16_fp6(six, 1.0f));
+      unsigned mid[8];  // k 16 half .. + 15  (not a choice of two elements, which is made one of sixteen)
+#pragma unroll
+      for (int e = 0; e < 8; e++) mid[e] = all[e] ^ ((all[e] ^ all[8 + e]) & upper);
+      const uint4 k8[2] = {make_uint4(mid[0], mid[1], mid[2], mid[3]), make_uint4(mid[4], mid[5], mid[6], mid[7])};
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        v16f p;
+#pragma unroll
+        for (int e = 0; e < 16; e++) p[e] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, t[i][q]), __builtin_bit_cast(v8bf, k8[q & 1]), p, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][b][e] = fmaf(dw, p[e], acc[i][b][e]);
+      }
+    };
 #pragma unroll 1
     for (int c = 0; c < nsteps; c += 32) {
       unsigned any = 0;
-      uint4 word[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) word[u] = *(const uint4 *)(words + (int64_t)min(c + 8 * u + (lane >> 3), nsteps - 1) * mg * 128 + (lane & 7) * 16);
+      for (int i = 0; i < MB; i++) {
+        const int rows = a.M - 32 * (m0 / 32 + MB * wm + i) - 4 * (lane & 7);  // of the four whose exponents this lane looks at
+        uint4 word[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const bool has = ((word[u].x < 0x1000000u) & (rows > 0)) | ((word[u].y < 0x1000000u) & (rows > 1)) | ((word[u].z < 0x1000000u) & (rows > 2)) | ((word[u].w < 0x1000000u) & (rows > 3));
-        uint64_t t = __ballot(has & (c + 8 * u + (lane >> 3) < nsteps));  // eight lanes to a block of k
-        t |= t >> 4, t |= t >> 2, t |= t >> 1;
-        any |= (unsigned)((t & 0x0101010101010101ull) * 0x0102040810204080ull >> 56) << (8 * u);
+        for (int u = 0; u < 4; u++) word[u] = *(const uint4 *)(words + ((int64_t)min(c + 8 * u + (lane >> 3), nsteps - 1) * mg + group[i]) * 128 + (lane & 7) * 16);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const bool has = ((word[u].x < 0x1000000u) & (rows > 0)) | ((word[u].y < 0x1000000u) & (rows > 1)) | ((word[u].z < 0x1000000u) & (rows > 2)) | ((word[u].w < 0x1000000u) & (rows > 3));
+          uint64_t t = __ballot(has & (c + 8 * u + (lane >> 3) < nsteps));  // eight lanes to a block of k
+          t |= t >> 4, t |= t >> 2, t |= t >> 1;
+          any |= (unsigned)((t & 0x0101010101010101ull) * 0x0102040810204080ull >> 56) << (8 * u);
+        }
       }
+      if constexpr (KB == 2) {
+        // a block's loads asked for under the one before it, where there are registers for both (1900 x 2048 x 5632, every block, 285 -> 235 us)
+        struct {
+          unsigned word[MB];
+          uint4 t[MB][4], w16[NB];
+          uint2 w8[NB];
+          float dw[NB];
+        } now, next;
+        auto ask = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+          for (int i = 0; i < MB; i++) next.word[i] = word_of(i, kb), terms_of(i, kb, next.t[i]);
+#pragma unroll
+          for (int b = 0; b < NB; b++) weights_of(b, kb, next.w16[b], next.w8[b], next.dw[b]);
+        };
+        if (any) ask(c + __builtin_ctz(any));
 #pragma unroll 1
-      while (any) {
-        const int kb = c + __builtin_ctz(any);
-        any &= any - 1;
-        const unsigned has = mine & (*(const unsigned *)(words + (int64_t)kb * mg * 128 + col * 4) < 0x1000000u) ? ~0u : 0u;  // (else nothing was written there)
-        const uint4 *r = (const uint4 *)(rests + (int64_t)kb * kDigitRests);
-        uint4 t[4] = {r[128], r[192], r[0], r[64]};  // the small term first
+        while (any) {
+          now = next;
+          any &= any - 1;
+          if (any) ask(c + __builtin_ctz(any));
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < 4; q++) t[q].x &= has, t[q].y &= has, t[q].z &= has, t[q].w &= has;
+          for (int i = 0; i < MB; i++) own(i, now.word[i], now.t[i]);
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-          const unsigned char *w = a.B + ((int64_t)min(n0 / 32 + NB * wn + b, ng - 1) * nkb + k0 + kb) * kDigitWRecord;
-          const uint4 w16 = *(const uint4 *)(w + col * 16);
-          const uint2 w8 = *(const uint2 *)(w + 512 + col * 8);
-          const float dw = *(const float *)(w + 768 + col * 4);
-          const v6u_dg six = {w16.x, w16.y, w16.z, w16.w, w8.x, w8.y};
-          const auto all = __builtin_bit_cast(v16u_dg, __builtin_amdgcn_cvt_scalef32_pk32_bf16_fp6(six, 1.0f));
-          unsigned mid[8];  // k 16 half .. + 15  (not a choice of two elements, which is made one of sixteen)
+          for (int b = 0; b < NB; b++) add(b, now.t, now.w16[b], now.w8[b], now.dw[b]);
+        }
+      } else {
+#pragma unroll 1
+        for (; any; any &= any - 1) {
+          const int kb = c + __builtin_ctz(any);
+          unsigned word[MB];
+          uint4 t[MB][4];
 #pragma unroll
-          for (int e = 0; e < 8; e++) mid[e] = all[e] ^ ((all[e] ^ all[8 + e]) & upper);
-          const uint4 k8[2] = {make_uint4(mid[0], mid[1], mid[2], mid[3]), make_uint4(mid[4], mid[5], mid[6], mid[7])};
-          v16f p;
+          for (int i = 0; i < MB; i++) word[i] = word_of(i, kb), terms_of(i, kb, t[i]);
 #pragma unroll
-          for (int e = 0; e < 16; e++) p[e] = 0.0f;
+          for (int i = 0; i < MB; i++) own(i, word[i], t[i]);
 #pragma unroll
-          for (int q = 0; q < 4; q++) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, t[q]), __builtin_bit_cast(v8bf, k8[q & 1]), p, 0, 0, 0);
-#pragma unroll
-          for (int e = 0; e < 16; e++) acc[i][b][e] = fmaf(dw, p[e], acc[i][b][e]);
+          for (int b = 0; b < NB; b++) {
+            uint4 w16;
+            uint2 w8;
+            float dw;
+            weights_of(b, kb, w16, w8, dw);
+            add(b, t, w16, w8, dw);
+          }
         }
       }
     }
