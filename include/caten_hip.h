@@ -279,9 +279,10 @@ int cthip_linear(float *y, const void *wmat, const float *x, int m, const float 
  *   (a session then holds the rows it has used instead of max_seq rows); such a session runs one launch per
  *   Linear; tokens and logits are those of the dense cache.
  * "weight_planes": MiB (default 32768).  A Linear over 64 rows and more, a long prompt's among them, may take its
- *   weights as bf16 terms; a quantised matrix (2 bytes per weight, beside its 1.06 or 0.56) and an fp16 one (4 bytes)
- *   keep theirs from the first such call on, up to this limit for all matrices of the process together and as long as
- *   a sixteenth of the device memory stays free: a 7B model of 4 bits holds 4 GB before its first long prompt and 17 behind it.
+ *   weights as matrix operands; an 8-bit matrix (2 bytes per weight, beside its 1.06), an fp16 one (4 bytes) and a 4-bit one
+ *   (1 byte, beside its 0.56; 2 more for Linears at one bf16 term) keep theirs from the first such call on, up to this limit for all
+ *   matrices of the process together and as long as a sixteenth of the device memory stays free: a 7B model of 4 bits holds 4 GB before
+ *   its first long prompt and 10.5 behind it.
  *   They are given back when a matrix is destroyed, by cthip_cache_trim, by an allocation here that finds no memory,
  *   and by a lower limit; 0 = none are kept.  Results do not depend on it where the same launch is chosen; past the
  *   limit the terms are made by every call that still pays with them.
