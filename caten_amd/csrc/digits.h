@@ -64,13 +64,14 @@ __device__ __forceinline__ float digits_top(const float *v) {
 __device__ __forceinline__ bool digits_uneven_columns(const float *v, float m, bool in) {
   const int lane = threadIdx.x & 63;
   const bool ok = in && m > 0.0f && m < INFINITY;
-  // (a row with an infinity or a NaN makes every sum a NaN, and no column is small)
-  const float up = ok ? __uint_as_float((254u - max(__float_as_uint(m) >> 23, 1u)) << 23) : 0.0f;
+  // (the largest value comes to 0.5 .. 1, past 2^126 to less than 4, so that squares may be held to 0 .. 1, a bit of their instruction that makes a NaN 0: a row that is not finite counts as
+  // nothing, and the others are looked at without it)
+  const float up = ok ? __uint_as_float((253u - min(max(__float_as_uint(m) >> 23, 1u), 252u)) << 23) : 0.0f;
   float s[32];
 #pragma unroll
   for (int i = 0; i < 32; i++) {
     const float t = v[i] * up;
-    s[i] = t * t;
+    s[i] = __builtin_amdgcn_fmed3f(t * t, 0.0f, 1.0f);
   }
   // a column's sum to each lane: half of the columns a step, to the lanes that keep them
 #pragma unroll

@@ -133,6 +133,27 @@ def test_results_that_the_large_values_do_not_reach(ops, rows, cols, m, cols_lar
     w.free()
 
 
+def test_rows_beside_rows_that_are_not_finite(ops):
+    """One row of every 32 is infinities or NaNs, one is past 2^127: the others' small values are as near as without them."""
+    from caten_amd.llm import Tensor
+    rng = np.random.default_rng(9)
+    rows, cols, m = 4100, 1056, 129
+    a = rng.normal(0, 0.05, (rows, cols)).astype(np.float32)
+    a[:, 7::8] = 0.0
+    w = ops.WeightMatrix("q4_0", Tensor.from_f32(a, "q4_0").raw, rows, cols)
+    x = (rng.uniform(0.5, 1.0, (m, cols)) * rng.choice([-1.0, 1.0], (m, cols))).astype(np.float32)
+    x[:, 7::8] *= 1000.0  # (one in a block would be found by its row alone)
+    x[3::32], x[3::64, 9:] = np.nan, np.inf
+    x[11::32] *= np.float32(2.0 ** 117)
+    assert np.abs(x[11]).max() >= 2.0 ** 126
+    fine = np.setdiff1d(np.arange(m), np.arange(3, m, 32))
+    x64, w64 = x[fine].astype(np.float64), w.dequantize().astype(np.float64)
+    got = ops.linear(x, w)
+    assert np.isnan(got[3::32]).all()
+    assert np.all(np.abs(got[fine] - x64 @ w64.T) <= terms_bound(x64, w64))
+    w.free()
+
+
 def test_rows_of_the_smallest_magnitudes(ops):
     """Below 2^-110 a digit's power of two would end past the smallest: what is left goes as terms."""
     rng = np.random.default_rng(8)
