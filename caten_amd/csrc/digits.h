@@ -54,9 +54,10 @@ __device__ __forceinline__ float digits_top(const float *v) {
 //   k, r                        1, 8  1, 32  1, 64  1, 256  1, 1000   4, 8  4, 32  4, 256   16, 32  16, 256   24, 32  24, 256   one row of 32, k = 1, r = 16  32   64
 //   digits alone                1.3   5.3    10     42      165       2.1   8.4    67       12      93        13      100       3.6                            7.2  14
 //   uneven columns, one large   1.3   3.8    3.3    1.3     1.0       2.1   1.3    1.0      11      1.0       13      1.0       3.6                            7.2  2.2
-//   uneven row, one large       1.3   1.7    1.4    1.1     1.0       2.0   1.7    1.0      8       1.0       13      59        3.3                            1.5  1.0
-// Blocks that have a rest without need, of 100000: columns: normal values, Laplace's, GELU(x) 0, x SiLU(y) 1; row: normal values 0, Laplace's 10, scaled by exp(y / 2) a column 10
-// (of x SiLU(y), which no norm leaves, 9000).
+//   uneven row, one large       1.3   1.5    1.2    1.0     1.0       1.9   1.2    1.0      3.2     1.0       12      1.8       (a row by itself: as on the left)
+//     (28 columns of 32 and more: as digits alone up to 256, 240 at 1000; 31 of 32: as digits alone at any, for a single value that is small says nothing)
+// Blocks that have a rest without need, of 100000: columns: normal values, Laplace's, GELU(x) 0, x SiLU(y) 1; row: normal values 0.1, Laplace's 60, scaled by exp(y / 2) a column 70
+// (of x SiLU(y), which no norm leaves, 16000).
 //
 // Of a column of a group's rows, how far it is below the largest values: half of log2(the rows' largest values' squares / its squares); past 18 in the mean square of the columns
 // (fewer rows: more, for chance makes columns of a few rows small), or 2^13 and more in any.  Lanes 0 .. 31 (32 .. 63) hold the rows, all of them active; `in`: this lane's row counts.  A row is taken
@@ -115,17 +116,14 @@ __device__ __forceinline__ bool digits_one_large(const float *v, float m) {
   for (int i = 0; i < 32; i++) s += fabsf(v[i]);
   return s < 1.5f * m;
 }
-// Where a thread has a row by itself, and rows are what a norm leaves, of one magnitude but for a few values: the mean square of log2(largest / value) past 30 (normal values
-// 7, off by 2.1; the logarithm's fraction taken as linear; zeros lose nothing)
+// Where a thread has a row by itself, and rows are what a norm leaves, of one magnitude but for a few values: what log2(largest / value) has past 4.5, summed, past 32 (normal values
+// 3.8, off by 3.3; the logarithm's fraction taken as linear; zeros lose nothing).  (Its mean square past 30 in that place took 24 of 32 columns 256 times as large for even in half of the rows.)
 __device__ __forceinline__ bool digits_uneven(const float *v, float m) {
-  const unsigned top = __float_as_uint(m) << 1;
+  const unsigned top = max(__float_as_uint(m) << 1, 9u << 23) - (9u << 23);
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 32; i++) {
-    const float d = (float)(top - min((__float_as_uint(v[i]) << 1) - 1u, top)) * 0x1p-24f;
-    s = fmaf(d, d, s);
-  }
-  return s > 32.0f * 30.0f;
+  for (int i = 0; i < 32; i++) s += (float)(top - min((__float_as_uint(v[i]) << 1) - 1u, top));
+  return s > 32.0f * 0x1p24f;
 }
 
 // A block of 32 values of row `row` (k = 32 kb ..) as digits, into an operand of rows32 rows (a multiple of 32) and nkb blocks; m: their largest magnitude, rest: what the last

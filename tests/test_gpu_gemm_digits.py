@@ -207,6 +207,35 @@ def test_prompt_with_large_channels(arch, rows):
     model.close()
 
 
+@pytest.mark.parametrize("arch,rows", [("gpt2", 97), ("gpt2", 700), ("llama", 96), ("llama", 1300)])
+def test_prompt_behind_a_norm_with_most_channels_large(arch, rows):
+    """Norms in front of the attention that leave 24 of 32 channels 256 times as large, which q, k and v do not read: rows by themselves say which blocks have the rest as terms.  Against the
+    pieces of 63 rows of test_prompt_with_large_channels: two terms are off by 2.5e-6 a Linear, twelve on either side by 1.2e-5, and as much again
+    for scores of some size."""
+    print(f"case: {arch}, {rows} rows", flush=True)
+    from caten_amd import llm, synth
+    cfg = dict(synth.LLAMA_CONFIGS["llama-tiny"], dim=1024, n_heads=16, n_kv_heads=4, ffn=2816) if arch == "llama" else dict(synth.GPT2_CONFIGS["gpt2"], dim=1024, n_heads=16)
+    cfg.update(n_layers=3, vocab=500, max_seq=2048)
+    w = (synth.llama_weights if arch == "llama" else synth.gpt2_weights)(cfg, seed=3)
+    rng = np.random.default_rng(1)
+    large = np.concatenate([32 * b + rng.permutation(32)[:24] for b in range(cfg["dim"] // 32)])
+    norm, behind = ("attn_norm", ("wq", "wk", "wv")) if arch == "llama" else ("ln1_g", ("attn_w",))
+    for l in range(3):
+        w[norm][l][large] *= 256.0
+        for k in behind:
+            w[k][l] *= 2.0  # (a quarter of the columns is left)
+            w[k][l][:, large] = 0.0
+    model = (llm.make_llama if arch == "llama" else llm.make_gpt2)(cfg, (llm.llama_state_dict if arch == "llama" else llm.gpt2_state_dict)(w, "q4_0"))
+    ids = [float(t) for t in synth.prompt(cfg["vocab"], rows, seed=3)]
+    got = model.forward(ids, rows, 0, return_logits=True)[1]
+    for n in range(0, rows, 63):
+        want = model.forward(ids[n:n + 63], min(63, rows - n), n, return_logits=True)[1]
+    off = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print("off by", off, flush=True)
+    assert off < 2.5e-5
+    model.close()
+
+
 def test_both_forms_of_a_matrix_are_kept(ops):
     """A 4-bit matrix is integers in bf16 to Linears at one term and digits at two: each form is made once and stays; with room for one of them alone, the one in use takes the other's."""
     import ctypes as C
